@@ -90,44 +90,35 @@ class MoEMLP(nn.Module):
 
     def forward(self, x: torch.Tensor, decode: bool = False) -> torch.Tensor:
         T, H = x.shape
+        w13, w2 = (self.w13_q, self.w2_q) if self.fp8 else (self.w13, self.w2)
+        s13, s2 = (self.w13_s, self.w2_s) if self.fp8 else (None, None)
+        if not self._force_loop and ops.moe_route_ok(x, self.router_w, self.top_k):
+            # static shapes, no host sync: such a step can be captured. A loop
+            # over the experts measured 25.0 ms for 512 tokens x 4 layers (64
+            # experts of 1408, top 6) against 1.9 ms, most of it launches and the
+            # host's wait for the counts.
+            P = T * self.top_k
+            few = T <= 64 or (decode and P <= 2048)      # the pair kernels' range
+            tiles = ops.moe_sorted_ok(x, w13, w2)
+            if few or tiles:
+                idx, wts, tok = ops.moe_route(x, self.router_w, self.top_k)
+                local = self.shared is not None and get_tp_size() == 1
+                shared = self.shared(x) if local else None
+                if tiles and not (few and not ops.moe_sorted_wins(P, self.num_experts, self.fp8)):
+                    out = ops.moe_sorted_mlp(x, w13, s13, w2, s2, idx, wts, more=shared)
+                else:
+                    y = ops.moe_grouped_mlp(x, w13, s13, w2, s2, idx.view(-1), tok.view(-1),
+                                            wts.view(-1), self.i_local, self.fp8,
+                                            num_experts=self.num_experts)
+                    out = ops.moe_combine(y, self.top_k, shared)
+                if local or self.shared is None:
+                    return tp_all_reduce(out)
+                return tp_all_reduce(out) + self.shared(x)
+
         router_logits = F.linear(x.float(), self.router_w)  # [T, E]
         probs = torch.softmax(router_logits, dim=-1)
         topw, topi = probs.topk(self.top_k, dim=-1)           # [T, K]
         topw = (topw / topw.sum(dim=-1, keepdim=True)).to(x.dtype)
-
-        # grouped path: pair-major kernels for tiny T; for DECODE batches
-        # past 64 the expert-major kernels keep the stage in one
-        # static-shaped launch pair (graph-capturable to batch 256).
-        # Prefill-sized T stays on the sorted per-expert hipBLASLt loop —
-        # extending the GEMV-style grouped path to 65..341-token prefill
-        # chunks measured -18% on the moe-small c=4 turn.
-        grouped_ok = T <= 64 or (decode and T * self.top_k <= 2048)
-        if x.is_cuda and grouped_ok and not self._force_loop:
-            # grouped-kernel path: one launch per stage for all pairs, no
-            # host sync, shape-static -> hipGraph-capturable decode
-            flat_e = topi.reshape(-1).to(torch.int32).contiguous()
-            # NOTE: for T=1 expand().reshape(-1) is a stride-0 VIEW whose
-            # data_ptr covers one element — must materialize contiguously
-            flat_t = (
-                torch.arange(T, device=x.device, dtype=torch.int32)
-                .repeat_interleave(self.top_k)
-                .contiguous()
-            )
-            flat_w = topw.reshape(-1).float().contiguous()
-            y = ops.moe_grouped_mlp(
-                x.contiguous(),
-                self.w13_q if self.fp8 else self.w13,
-                self.w13_s if self.fp8 else None,
-                self.w2_q if self.fp8 else self.w2,
-                self.w2_s if self.fp8 else None,
-                flat_e, flat_t, flat_w, self.i_local, self.fp8,
-                num_experts=self.num_experts,
-            )
-            out = torch.zeros_like(x)
-            out.index_add_(0, flat_t.long(), y)
-            if self.shared is not None:
-                return tp_all_reduce(out) + self.shared(x)
-            return tp_all_reduce(out)
 
         out = torch.zeros_like(x)
         # token gather per expert (sorted dispatch)
@@ -280,12 +271,15 @@ class RoutedExperts(nn.Module):
         if (x.is_cuda and x.dtype == torch.bfloat16 and fast_act
                 and C % 16 == 0 and I % 16 == 0 and self.force_path is None):
             # the framework's grouped expert GEMV kernels (pair- or expert-major)
+            if (ops.moe_sorted_ok(x, self.w13, self.w2, self.act)
+                    and ops.moe_sorted_wins(T * top, self.r.experts, False)):
+                return ops.moe_sorted_mlp(x, self.w13, None, self.w2, None, idx, wts, self.act)
             flat_t = torch.arange(T, device=x.device, dtype=torch.int32).repeat_interleave(top)
             y = ops.moe_grouped_mlp(x.contiguous(), self.w13, None, self.w2, None,
                                     idx.reshape(-1), flat_t.contiguous(),
                                     wts.reshape(-1).contiguous(), I, False,
                                     num_experts=self.r.experts, act=self.act)
-            return y.view(T, top, C).float().sum(1).to(x.dtype)
+            return ops.moe_combine(y, top)
         if not self.gated:
             return mx.moe_pairs_plain(x.contiguous(), self.w13, self.w2, idx, wts, self.act)
         return mx.moe_pairs_mlp(x.contiguous(), self.w13, self.w2, idx, wts, self.act)
@@ -295,6 +289,8 @@ class RoutedExperts(nn.Module):
 
         T, C = x.shape
         top, I = self.r.top, self.r.ff
+        if ops.moe_sorted_ok(x, self.w13, self.w2, self.act) and self.gated == (self.act != "relu2"):
+            return ops.moe_sorted_mlp(x, self.w13, None, self.w2, None, idx, wts, self.act)
         flat_e = idx.reshape(-1).long()
         order = torch.argsort(flat_e, stable=True)
         tok = torch.div(order, top, rounding_mode="floor")

@@ -333,6 +333,130 @@ def gateup_silu_norm(
     return gateup_silu(rms_norm(x, norm_w, eps), gate_up_w, i_local)
 
 
+def _moe_act(act):
+    """(kernel's activation number, limit, alpha) of an expert activation, None
+    if the kernels have no such activation."""
+    if isinstance(act, tuple) and act[0] == "clamp_swish":
+        return 2, float(act[1]), float(act[2])
+    if act == "relu2":
+        return 3, 0.0, 0.0
+    return (0, 0.0, 0.0) if act in (None, "silu") else None
+
+
+def moe_route_ok(x: torch.Tensor, router_w: torch.Tensor, top: int) -> bool:
+    """Whether moe_route takes this router: a row of activations and logits in
+    LDS, eight-channel rows for moe_combine."""
+    E, K = router_w.shape
+    return (
+        x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
+        and router_w.dtype == torch.float32 and router_w.is_contiguous()
+        and K % 8 == 0 and E <= 1024 and top <= min(E, 64) and (K + E) * 4 <= 65536
+        and x.data_ptr() % 16 == 0 and router_w.data_ptr() % 16 == 0
+    )
+
+
+def moe_route(x: torch.Tensor, router_w: torch.Tensor, top: int):
+    """Softmax routing of bf16 rows x [T, K] by float32 router_w [E, K]: experts
+    int32, weights float32 (normalised over the chosen) and tokens int32, each
+    [T, top]."""
+    T, K = x.shape
+    E = router_w.shape[0]
+    lib, hip = _lib()
+    idx, tok = torch.empty(2, T, top, dtype=torch.int32, device=x.device)
+    wts = torch.empty(T, top, dtype=torch.float32, device=x.device)
+    hip.check(lib.oa_moe_route(hip.current_stream_ptr(), x.data_ptr(), router_w.data_ptr(),
+                               idx.data_ptr(), wts.data_ptr(), tok.data_ptr(), T, E, K, top),
+              "oa_moe_route")
+    return idx, wts, tok
+
+
+def moe_combine(y: torch.Tensor, top: int, more: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """out[t] = sum of rows t * top .. + top of y [T * top, H] (+ more[t]), bf16
+    with float32 sums in one order."""
+    T, H = y.shape[0] // top, y.shape[1]
+    assert y.is_cuda and y.dtype == torch.bfloat16 and y.is_contiguous()
+    assert more is None or (more.shape == (T, H) and more.dtype == y.dtype
+                            and more.is_contiguous())
+    lib, hip = _lib()
+    out = torch.empty(T, H, dtype=y.dtype, device=y.device)
+    hip.check(lib.oa_moe_combine(hip.current_stream_ptr(), y.data_ptr(),
+                                 more.data_ptr() if more is not None else None, out.data_ptr(),
+                                 T, top, H), "oa_moe_combine")
+    return out
+
+
+def moe_sorted_wins(pairs: int, experts: int, fp8: bool) -> bool:
+    """Sorted tiles against a weight stream per pair, measured in graphs (both
+    products and the sort, us): 64 experts of 1408 x 2048, fp8: 24 pairs 47 to
+    49, 48 pairs 82 to 91, 78 pairs 102 to 144; bf16: 48 pairs 148 to 130, 78
+    pairs 181 to 204. 16 experts of 1024 x 2048, fp8: 16 pairs 34 to 25, 32
+    pairs 35 to 47; bf16: 32 pairs 62 to 65, 52 pairs 64 to 100."""
+    return pairs >= (max(24, experts // 2) if fp8 else max(32, experts))
+
+
+def moe_sorted_ok(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, act=None) -> bool:
+    """Whether moe_sorted_mlp takes these experts: both products run over
+    128-column steps, a gate strip holds 64 rows."""
+    return (
+        x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
+        and w13.is_contiguous() and w2.is_contiguous() and w13.dtype == w2.dtype
+        and w13.dtype in (torch.bfloat16, torch.uint8) and _moe_act(act) is not None
+        and x.shape[1] % 128 == 0 and w2.shape[2] % 128 == 0 and w13.shape[0] <= 1024
+        and all(t.data_ptr() % 16 == 0 for t in (x, w13, w2))
+    )
+
+
+def moe_sorted_mlp(
+    x: torch.Tensor,
+    w13: torch.Tensor,
+    w13_scale: Optional[torch.Tensor],
+    w2: torch.Tensor,
+    w2_scale: Optional[torch.Tensor],
+    expert_ids: torch.Tensor,
+    pair_weights: torch.Tensor,
+    act=None,
+    more: Optional[torch.Tensor] = None,
+) -> torch.Tensor:
+    """Routed experts of a prompt-sized batch (GPU): out[t] = sum over token t's
+    choices j of weight_tj * W2[e_tj] act(W13[e_tj] x_t), plus more[t] if given.
+    x [T, H] bf16; expert_ids int32 and pair_weights float32 [T, top]; experts as
+    in moe_grouped_mlp, bf16 or fp8 with row scales. Pairs are sorted by expert
+    on the GPU and every expert's rows run as matrix-core tiles: no host sync,
+    static shapes."""
+    T, H = x.shape
+    top = expert_ids.shape[1]
+    E, I = w13.shape[0], w2.shape[2]
+    actk, limit, alpha = _moe_act(act)
+    assert w13.shape[1] == (I if actk == 3 else 2 * I) and w13.shape[2] == H and w2.shape[1] == H
+    assert expert_ids.dtype == torch.int32 and expert_ids.is_contiguous()
+    assert pair_weights.dtype == torch.float32 and pair_weights.is_contiguous()
+    assert expert_ids.shape == pair_weights.shape == (T, top)
+    assert (w13.dtype == torch.uint8) == (w13_scale is not None) == (w2_scale is not None)
+    P = T * top
+    # rows of a tile, by the rows that an expert has on average (64 experts of
+    # 1408 x 2048, both products, bf16, us): 1.5 rows 193 with 16 to 182 with 64
+    # (fp8 99 to 112), 3.8 rows 206 to 203 (106 to 116), 6 rows 231 to 214; 48 rows
+    # 307 with 64 to 297 with 128, 96 rows 378 to 385, 192 rows 582 to 501
+    bm = 16 if P <= 4 * E else 64 if P < 128 * E else 128
+    max_tiles = P // bm + min(E, P)
+    lib, hip = _lib()
+    stream, dev = hip.current_stream_ptr(), x.device
+    ints = torch.empty(2 * E + 2 + max_tiles + P, dtype=torch.int32, device=dev)
+    off, pre, tile_e, perm = ints.split([E + 1, E + 1, max_tiles, P])
+    lists = (off.data_ptr(), pre.data_ptr(), tile_e.data_ptr(), perm.data_ptr())
+    hip.check(lib.oa_moe_sort(stream, expert_ids.data_ptr(), P, E, bm, *lists), "oa_moe_sort")
+    mid = torch.empty(P, I, dtype=x.dtype, device=dev)
+    y = torch.empty(P, H, dtype=x.dtype, device=dev)
+    ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
+    hip.check(lib.oa_moe_grouped(stream, x.data_ptr(), w13.data_ptr(), ptr(w13_scale), *lists, None,
+                                 mid.data_ptr(), E, I, H, top, bm, max_tiles,
+                                 2 if actk == 3 else 1, actk, limit, alpha), "oa_moe_grouped(up)")
+    hip.check(lib.oa_moe_grouped(stream, mid.data_ptr(), w2.data_ptr(), ptr(w2_scale), *lists,
+                                 pair_weights.data_ptr(), y.data_ptr(), E, H, I, top, bm, max_tiles,
+                                 0, 0, 0.0, 0.0), "oa_moe_grouped(down)")
+    return moe_combine(y, top, more)
+
+
 def moe_grouped_mlp(
     x: torch.Tensor,
     w13: torch.Tensor,
@@ -363,15 +487,8 @@ def moe_grouped_mlp(
     or "relu2" for UNGATED experts: w13 is [E, I, K] (up rows alone) and the
     middle activation is relu(up x)^2.
     """
-    if isinstance(act, tuple):
-        assert act[0] == "clamp_swish"
-        actk, limit, alpha = 2, float(act[1]), float(act[2])
-    elif act == "relu2":
-        assert w13.shape[1] == i_local
-        actk, limit, alpha = 3, 0.0, 0.0
-    else:
-        assert act in (None, "silu")
-        actk, limit, alpha = 0, 0.0, 0.0
+    actk, limit, alpha = _moe_act(act)
+    assert actk != 3 or w13.shape[1] == i_local
     assert x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous()
     # stride-0 expand views have a data_ptr that covers ONE element — the
     # kernels index these linearly, so contiguity is load-bearing

@@ -25,6 +25,7 @@ SOURCES = [
     "attention_prefill.hip",
     "fp8_moe.hip",
     "moe_gemv.hip",
+    "moe_grouped.hip",
 ]
 
 # the sequence-mixer kernels of hybrid decoders live in a library of their

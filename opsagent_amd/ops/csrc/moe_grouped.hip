@@ -1,0 +1,501 @@
+// Routed experts of prompt-sized batches on the matrix cores: five launches for
+// a layer, static shapes, no host synchronisation (a per-expert loop of library
+// products needs a device-to-host copy of the counts and about eight launches
+// per used expert).
+//
+//   oa_moe_sort           pairs (token, choice) in expert order, expert offsets,
+//                         the list of row tiles
+//   oa_moe_grouped        MODE 1: mid[s] = act(gate) * up of the pair at sorted
+//                         place s, its activation row gathered from x;
+//                         MODE 2: mid[s] = relu(up)^2 (ungated experts);
+//                         MODE 0: y[p] = pair_weight * (W2 mid[s]), scattered
+//                         back to the pair's own row p
+//   oa_moe_combine        out[t] = sum over a token's pairs, in their own order
+//                         (+ another row, the shared expert's)
+//
+// A pair's result depends on no other pair, and a token's pairs are added in
+// one order: the output does not depend on how pairs are placed in an expert.
+// Activations are bf16; weights bf16, or fp8 (e4m3, one float32 scale per row)
+// widened exactly to bf16 in registers. Sums are float32.
+#include <type_traits>
+
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(4))) unsigned int mgu4;
+typedef __attribute__((ext_vector_type(8))) short mgs8;
+typedef __attribute__((ext_vector_type(8))) __bf16 mgb8;
+typedef __attribute__((ext_vector_type(2))) __bf16 mgb2;
+typedef __attribute__((ext_vector_type(4))) float mgf4;
+
+#define MG_MAX_E 1024
+
+// ---- routing ----------------------------------------------------------------
+// Router logits (float32 weights and sums on bf16 rows), softmax and the `top`
+// best experts of TT tokens per block, weights normalised over the chosen: one
+// launch instead of a cast, a float32 library product, softmax, top-k (two
+// launches), sum, division and casts (61 us for 13 tokens and 64 experts of 2048
+// columns, about 5 us each). 11.3 us there, 6.6 us for 16 experts: bound by what
+// one CU draws (the matrix of 64 experts is 512 KiB, 47 GB/s). Logits spread over
+// blocks and chosen in a second launch measured 13.1 us. A wave takes an expert's
+// row in 1 KiB pieces and keeps TT sums; ties go to the lower expert.
+template <int TT>
+__global__ __launch_bounds__(1024) void moe_route_kernel(const uint16_t* __restrict__ x,
+                                                         const float* __restrict__ rw,
+                                                         int* __restrict__ idx,
+                                                         float* __restrict__ wout,
+                                                         int* __restrict__ tok, int T, int E, int K,
+                                                         int top) {
+    extern __shared__ __attribute__((aligned(16))) float rl[];
+    float* xs = rl;                     // [TT][K]
+    float* lg = rl + TT * K;            // [TT][E]
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int t0 = blockIdx.x * TT;
+    for (int i = tid; i < TT * (K / 4); i += 1024) {
+        const int t = i / (K / 4), c = i - t * (K / 4);
+        const uint2 v = *reinterpret_cast<const uint2*>(x + (size_t)min(t0 + t, T - 1) * K + c * 4);
+        *reinterpret_cast<float4*>(xs + t * K + c * 4) =
+            make_float4(bf16_lo(v.x), bf16_hi(v.x), bf16_lo(v.y), bf16_hi(v.y));
+    }
+    __syncthreads();
+    for (int e = wid; e < E; e += 16) {
+        const float* wr = rw + (size_t)e * K;
+        float a[TT];
+#pragma unroll
+        for (int t = 0; t < TT; ++t) a[t] = 0.0f;
+        for (int k = lane * 4; k < K; k += 256) {
+            const float4 w = *reinterpret_cast<const float4*>(wr + k);
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                const float4 v = *reinterpret_cast<const float4*>(xs + t * K + k);
+                a[t] = fmaf(w.x, v.x, a[t]);
+                a[t] = fmaf(w.y, v.y, a[t]);
+                a[t] = fmaf(w.z, v.z, a[t]);
+                a[t] = fmaf(w.w, v.w, a[t]);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+            a[t] = wave_reduce_sum(a[t]);
+            if (lane == 0) lg[t * E + e] = a[t];
+        }
+    }
+    __syncthreads();
+    if (wid >= TT || t0 + wid >= T) return;
+    float* z = lg + wid * E;            // one wave per token from here on
+    const size_t o = (size_t)(t0 + wid) * top;
+    float mx = -INFINITY;
+    for (int e = lane; e < E; e += 64) mx = fmaxf(mx, z[e]);
+    mx = wave_reduce_max(mx);
+    float sum = 0.0f;
+    for (int e = lane; e < E; e += 64) sum += expf(z[e] - mx);
+    sum = wave_reduce_sum(sum);
+    for (int e = lane; e < E; e += 64) z[e] = expf(z[e] - mx) / sum;
+    float mine = 0.0f, total = 0.0f;    // lane r keeps the r-th choice's score
+    int who = 0;
+    for (int r = 0; r < top; ++r) {
+        float bv = -INFINITY;
+        int bi = 0x7fffffff;
+        for (int e = lane; e < E; e += 64)
+            if (z[e] > bv) {
+                bv = z[e];
+                bi = e;
+            }
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            const float ov = __shfl_xor(bv, d, 64);
+            const int oi = __shfl_xor(bi, d, 64);
+            if (ov > bv || (ov == bv && oi < bi)) {
+                bv = ov;
+                bi = oi;
+            }
+        }
+        if (bi == 0x7fffffff) {         // no score left that compares (NaN logits)
+            bi = 0;
+            bv = 0.0f;
+        }
+        total += bv;
+        if (lane == r) {
+            mine = bv;
+            who = bi;
+        }
+        if (lane == (bi & 63)) z[bi] = -INFINITY;   // the lane that reads it next
+    }
+    if (lane < top) {
+        idx[o + lane] = who;
+        wout[o + lane] = mine / (total + 1e-20f);
+        tok[o + lane] = t0 + wid;
+    }
+}
+
+// ---- sorting ----------------------------------------------------------------
+// One block: counts per expert, offsets, tiles of `bm` rows, then the places.
+// off [E + 1]; pre [E + 1]: first tile of every expert; tile_e: expert of every
+// tile; perm [P]: pair at every sorted place.
+__global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ expert_ids, int P,
+                                                        int E, int bm, int* __restrict__ off,
+                                                        int* __restrict__ pre,
+                                                        int* __restrict__ tile_e,
+                                                        int* __restrict__ perm) {
+    __shared__ int cnt[MG_MAX_E], cur[MG_MAX_E], wsum[2][16];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    for (int e = tid; e < E; e += 1024) cnt[e] = 0;
+    __syncthreads();
+    for (int p = tid; p < P; p += 1024) {
+        const int e = expert_ids[p];
+        if ((unsigned)e < (unsigned)E) atomicAdd(&cnt[e], 1);
+    }
+    __syncthreads();
+    // inclusive scans of rows and tiles, one expert per thread (E <= 1024)
+    const int c = tid < E ? cnt[tid] : 0;
+    const int nt = (c + bm - 1) / bm;
+    int a = c, b = nt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int x = __shfl_up(a, o, 64), y = __shfl_up(b, o, 64);
+        if (lane >= o) {
+            a += x;
+            b += y;
+        }
+    }
+    if (lane == 63) {
+        wsum[0][wid] = a;
+        wsum[1][wid] = b;
+    }
+    __syncthreads();
+    for (int w = 0; w < wid; ++w) {
+        a += wsum[0][w];
+        b += wsum[1][w];
+    }
+    if (tid < E) {
+        off[tid + 1] = a;
+        pre[tid + 1] = b;
+        cur[tid] = a - c;
+        for (int i = b - nt; i < b; ++i) tile_e[i] = tid;
+    }
+    if (tid == 0) off[0] = pre[0] = 0;
+    __syncthreads();
+    for (int p = tid; p < P; p += 1024) {
+        const int e = expert_ids[p];
+        if ((unsigned)e < (unsigned)E) perm[atomicAdd(&cur[e], 1)] = p;
+    }
+}
+
+// ---- grouped products ---------------------------------------------------------
+__device__ __forceinline__ float mg_gate_act(float g, float u, int act, float limit, float alpha) {
+    if (act == 2) {
+        g = fminf(g, limit);
+        u = fminf(fmaxf(u, -limit), limit);
+        return g / (1.0f + __expf(-alpha * g)) * (u + 1.0f);
+    }
+    return g / (1.0f + __expf(-g)) * u;
+}
+
+// 8 fp8 (two words) to 8 bf16, exactly
+__device__ __forceinline__ mgs8 mg_widen(uint32_t lo, uint32_t hi) {
+    union {
+        mgb2 h[4];
+        mgs8 v;
+    } r;
+    r.h[0] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false);
+    r.h[1] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
+    r.h[2] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false);
+    r.h[3] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
+    return r.v;
+}
+
+// A block of four waves takes BM sorted rows of one expert and 128 of its weight
+// rows (64 gate and the 64 up rows beside them). Weight rows go from memory
+// straight into the A fragments of v_mfma_f32_16x16x32_bf16, one 128-column step
+// ahead: 16 rows x 64 bytes per load reach 6.0 TB/s with plain loads (5.2 with
+// non-temporal ones, 6.4 for whole contiguous rows) and need no LDS. The
+// activation rows, which all four waves read, are staged in LDS in two buffers
+// with one barrier per step; 16-byte chunks are XORed with the row so that a
+// fragment read touches every bank once. Grid: work items in an order that puts
+// the row tiles of one expert and weight strip next to each other on ONE die
+// (block ids go round the eight dies), so the strip is read from memory once.
+template <int BM, bool FP8, int MODE>
+__global__ __launch_bounds__(256, BM > 64 ? 2 : 3) void moe_grouped_kernel(
+    const uint16_t* __restrict__ x, const char* __restrict__ w, const float* __restrict__ wscale,
+    const int* __restrict__ off, const int* __restrict__ pre, const int* __restrict__ tile_e,
+    const int* __restrict__ perm, const float* __restrict__ pair_w, uint16_t* __restrict__ out,
+    int E, int N, int K, int top, int strips, int act, float limit, float alpha) {
+    constexpr int FM = BM / 16;                  // activation fragments
+    constexpr int XL = BM * 16 / 256;            // 16-byte chunks per thread and step
+    constexpr int WL = FP8 ? 2 : 4;              // weight loads per fragment and step
+    __shared__ __attribute__((aligned(16))) char xs[2][BM * 256];
+    __shared__ int rows_s[BM];
+
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int r = lane & 15, q = lane >> 4;
+    const int per = gridDim.x >> 3;              // work items per die
+    const int item = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    const int tiles = pre[E];
+    if (item >= tiles * strips) return;
+    const int e = tile_e[item / strips];
+    const int t0 = pre[e], mt = pre[e + 1] - t0;
+    const int in = item - t0 * strips;
+    const int strip = in / mt, mtile = in - strip * mt;
+    const int s0 = off[e] + mtile * BM;
+    const int m = min(BM, off[e + 1] - s0);
+
+    // source row of every activation row (rows past the end repeat the last one)
+    if (tid < BM) {
+        const int s = s0 + min(tid, m - 1);
+        rows_s[tid] = MODE == 0 ? s : perm[s] / top;
+    }
+    __syncthreads();
+    const uint16_t* xp[XL];
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+        const int c = tid + i * 256;
+        xp[i] = x + (size_t)rows_s[c >> 4] * K + (c & 15) * 8;
+    }
+    // weight rows of this wave: two fragments of 16
+    const size_t rb = FP8 ? (size_t)K : (size_t)K * 2;
+    const int n0 = MODE == 1 ? strip * 64 + wid * 16 : strip * 128 + wid * 32;
+    const char* we = w + (size_t)e * (MODE == 1 ? 2 * N : N) * rb;
+    const char* wp[2];
+    wp[0] = we + (size_t)min(n0 + r, N - 1) * rb + q * 16;
+    wp[1] = we + (size_t)(MODE == 1 ? N + min(n0 + r, N - 1) : min(n0 + 16 + r, N - 1)) * rb + q * 16;
+
+    mgf4 acc[2][FM];
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int j = 0; j < FM; ++j) acc[f][j] = mgf4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    mgu4 xr[XL], wb[2][2][WL];
+    const int ns = K / 128;
+#pragma unroll
+    for (int i = 0; i < XL; ++i) xr[i] = *reinterpret_cast<const mgu4*>(xp[i]);
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int j = 0; j < WL; ++j) wb[0][f][j] = *reinterpret_cast<const mgu4*>(wp[f] + j * 64);
+
+    // `more` is a compile-time constant: the loads of the next step are counted
+    // exactly, so a wait never drains them
+    auto step = [&](int s, mgu4 (&cur)[2][WL], mgu4 (&nxt)[2][WL], char* buf, auto more) {
+#pragma unroll
+        for (int i = 0; i < XL; ++i) {
+            const int c = tid + i * 256, row = c >> 4;
+            *reinterpret_cast<mgu4*>(buf + row * 256 + (((c & 15) ^ (row & 15)) << 4)) = xr[i];
+        }
+        __syncthreads();
+        if (decltype(more)::value) {
+#pragma unroll
+            for (int i = 0; i < XL; ++i)
+                xr[i] = *reinterpret_cast<const mgu4*>(xp[i] + (size_t)(s + 1) * 128);
+#pragma unroll
+            for (int f = 0; f < 2; ++f)
+#pragma unroll
+                for (int j = 0; j < WL; ++j)
+                    nxt[f][j] = *reinterpret_cast<const mgu4*>(wp[f] + (size_t)(s + 1) * (FP8 ? 128 : 256) + j * 64);
+            __builtin_amdgcn_sched_barrier(0);   // the loads are issued before the products
+        }
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            // fp8: one 16-byte load holds the lane's columns of two products
+            const int chunk = FP8 ? (ks >> 1) * 8 + q * 2 + (ks & 1) : ks * 4 + q;
+            mgs8 a[2];
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                if (FP8) {
+                    const mgu4 v = cur[f][ks >> 1];
+                    a[f] = (ks & 1) ? mg_widen(v[2], v[3]) : mg_widen(v[0], v[1]);
+                } else {
+                    a[f] = *reinterpret_cast<const mgs8*>(&cur[f][FP8 ? 0 : ks]);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < FM; ++j) {
+                const mgs8 b = *reinterpret_cast<const mgs8*>(buf + (j * 16 + r) * 256 + ((chunk ^ r) << 4));
+#pragma unroll
+                for (int f = 0; f < 2; ++f)
+                    acc[f][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        __builtin_bit_cast(mgb8, a[f]), __builtin_bit_cast(mgb8, b), acc[f][j], 0, 0, 0);
+            }
+        }
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    int s = 0;
+    for (; s + 2 < ns; s += 2) {
+        step(s, wb[0], wb[1], xs[0], yes);
+        step(s + 1, wb[1], wb[0], xs[1], yes);
+    }
+    if (s + 2 == ns) {
+        step(s, wb[0], wb[1], xs[0], yes);
+        step(s + 1, wb[1], wb[0], xs[1], no);
+    } else {
+        step(s, wb[0], wb[1], xs[0], no);
+    }
+
+    // lane: sorted row r of a fragment, weight rows q * 4 .. + 3
+    float sc[2][4];
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (!FP8) {
+                sc[f][i] = 1.0f;
+                continue;
+            }
+            const int n = min(n0 + (MODE == 1 ? 0 : f * 16) + q * 4 + i, N - 1);
+            sc[f][i] = wscale[(size_t)e * (MODE == 1 ? 2 * N : N) + (MODE == 1 && f ? N + n : n)];
+        }
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+        const int row = j * 16 + r;
+        if (row >= m) continue;
+        if (MODE == 1) {
+            uint32_t o[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float v0 = mg_gate_act(acc[0][j][2 * h] * sc[0][2 * h],
+                                             acc[1][j][2 * h] * sc[1][2 * h], act, limit, alpha);
+                const float v1 = mg_gate_act(acc[0][j][2 * h + 1] * sc[0][2 * h + 1],
+                                             acc[1][j][2 * h + 1] * sc[1][2 * h + 1], act, limit, alpha);
+                o[h] = pack_bf16x2(v0, v1);
+            }
+            *reinterpret_cast<uint2*>(out + (size_t)(s0 + row) * N + n0 + q * 4) = make_uint2(o[0], o[1]);
+        } else {
+            const int pair = MODE == 0 ? perm[s0 + row] : 0;
+            const float pw = MODE == 0 ? pair_w[pair] : 1.0f;
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                const int n = n0 + f * 16 + q * 4;
+                if (n >= N) continue;              // N is a multiple of 16
+                float v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    v[i] = acc[f][j][i] * sc[f][i];
+                    if (MODE == 2) {
+                        v[i] = fmaxf(v[i], 0.0f);
+                        v[i] *= v[i];
+                    } else {
+                        v[i] *= pw;
+                    }
+                }
+                *reinterpret_cast<uint2*>(out + (size_t)(MODE == 0 ? pair : s0 + row) * N + n) =
+                    make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+            }
+        }
+    }
+}
+
+// ---- sum over a token's pairs ---------------------------------------------------
+// eight channels per thread; `more` (optional) is added as one more row
+__global__ __launch_bounds__(256) void moe_combine_kernel(const uint16_t* __restrict__ y,
+                                                          const uint16_t* __restrict__ more,
+                                                          uint16_t* __restrict__ out, int top,
+                                                          int H8, int64_t n) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        const int64_t t = i / H8, c = i - t * H8;
+        const uint4* yr = reinterpret_cast<const uint4*>(y) + t * top * H8 + c;
+        float s[8] = {};
+        for (int k = 0; k < top; ++k) {
+            const uint4 v = yr[(int64_t)k * H8];
+            const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                s[2 * j] += bf16_lo(u[j]);
+                s[2 * j + 1] += bf16_hi(u[j]);
+            }
+        }
+        if (more) {
+            const uint4 v = reinterpret_cast<const uint4*>(more)[i];
+            const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                s[2 * j] += bf16_lo(u[j]);
+                s[2 * j + 1] += bf16_hi(u[j]);
+            }
+        }
+        reinterpret_cast<uint4*>(out)[i] = make_uint4(pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]),
+                                                      pack_bf16x2(s[4], s[5]), pack_bf16x2(s[6], s[7]));
+    }
+}
+
+// idx, w, tok [T, top]: expert, weight and token of every pair
+extern "C" int oa_moe_route(void* stream, const void* x, const void* rw, void* idx, void* w, void* tok,
+                            int T, int E, int K, int top) {
+    if (T < 1 || E < 1 || E > MG_MAX_E || top < 1 || top > E || top > 64 || K < 4 || K % 4 != 0)
+        return -100;
+    // four tokens per block once the blocks fill the chip, LDS allowing
+    const bool four = T >= 1024 && (size_t)4 * (K + E) * 4 <= 65536;
+    const size_t lds = (size_t)(four ? 4 : 1) * (K + E) * 4;
+    if (lds > 65536) return -101;
+    if (four)
+        hipLaunchKernelGGL(moe_route_kernel<4>, dim3(CEIL_DIV(T, 4)), dim3(1024), lds, (hipStream_t)stream,
+                           (const uint16_t*)x, (const float*)rw, (int*)idx, (float*)w, (int*)tok, T, E, K, top);
+    else
+        hipLaunchKernelGGL(moe_route_kernel<1>, dim3(T), dim3(1024), lds, (hipStream_t)stream,
+                           (const uint16_t*)x, (const float*)rw, (int*)idx, (float*)w, (int*)tok, T, E, K, top);
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
+extern "C" int oa_moe_sort(void* stream, const void* expert_ids, int P, int E, int bm, void* off,
+                           void* pre, void* tile_e, void* perm) {
+    if (P < 1 || E < 1 || E > MG_MAX_E || (bm != 16 && bm != 64 && bm != 128)) return -100;
+    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream,
+                       (const int*)expert_ids, P, E, bm, (int*)off, (int*)pre, (int*)tile_e, (int*)perm);
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
+// mode 0: x = mid [P, K], w [E, N, K], out = y [P, N]; mode 1: x [T, K],
+// w [E, 2N, K], out = mid [P, N]; mode 2: x [T, K], w [E, N, K], out = mid.
+// max_tiles: no fewer than the tiles that oa_moe_sort can make of P pairs.
+extern "C" int oa_moe_grouped(void* stream, const void* x, const void* w, const void* wscale,
+                              const void* off, const void* pre, const void* tile_e, const void* perm,
+                              const void* pair_w, void* out, int E, int N, int K, int top, int bm,
+                              int max_tiles, int mode, int act, float limit, float alpha) {
+    if (K < 128 || K % 128 != 0 || N < 16 || N % 16 != 0 || (mode == 1 && N % 64 != 0) || top < 1 ||
+        max_tiles < 1 || E < 1 || mode < 0 || mode > 2)
+        return -100;
+    const int strips = mode == 1 ? N / 64 : CEIL_DIV(N, 128);
+    const int64_t items = (int64_t)strips * max_tiles;
+    if (items > (1 << 28)) return -101;
+    const dim3 grid((unsigned)(CEIL_DIV(items, 8) * 8)), block(256);
+#define MG(BMV, F, MO)                                                                              \
+    hipLaunchKernelGGL((moe_grouped_kernel<BMV, F, MO>), grid, block, 0, (hipStream_t)stream,      \
+                       (const uint16_t*)x, (const char*)w, (const float*)wscale, (const int*)off,  \
+                       (const int*)pre, (const int*)tile_e, (const int*)perm, (const float*)pair_w, \
+                       (uint16_t*)out, E, N, K, top, strips, act, limit, alpha)
+#define MGM(BMV, F)                    \
+    do {                               \
+        if (mode == 0) MG(BMV, F, 0);  \
+        else if (mode == 1) MG(BMV, F, 1); \
+        else MG(BMV, F, 2);            \
+    } while (0)
+#define MGF(BMV)                   \
+    do {                           \
+        if (wscale) MGM(BMV, true); \
+        else MGM(BMV, false);      \
+    } while (0)
+    switch (bm) {
+        case 16: MGF(16); break;
+        case 64: MGF(64); break;
+        case 128: MGF(128); break;
+        default: return -102;
+    }
+#undef MGF
+#undef MGM
+#undef MG
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
+extern "C" int oa_moe_combine(void* stream, const void* y, const void* more, void* out, int T,
+                              int top, int H) {
+    if (T < 1 || top < 1 || H < 8 || H % 8 != 0) return -100;
+    const int64_t n = (int64_t)T * (H / 8);
+    const int64_t blocks = CEIL_DIV(n, 256);
+    hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0,
+                       (hipStream_t)stream, (const uint16_t*)y, (const uint16_t*)more, (uint16_t*)out,
+                       top, H / 8, n);
+    HIP_CHECK_LAUNCH();
+    return 0;
+}

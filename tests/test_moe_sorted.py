@@ -1,0 +1,110 @@
+"""Sorted expert tiles (ops.moe_sorted_mlp) against the float64 sum over a
+token's experts, at the edges of row tiles, weight strips and expert counts."""
+
+import pytest
+import torch
+
+from opsagent_amd import ops
+from opsagent_amd.ops import torch_ref
+
+
+def _reference(x, w13, w2, idx, wts, act, more):
+    x = x.double()
+    out = torch.zeros(x.shape[0], w2.shape[1], dtype=torch.float64, device=x.device)
+    for e in range(w13.shape[0]):
+        rows, place = (idx == e).nonzero(as_tuple=True)
+        if not rows.numel():
+            continue
+        h = x[rows] @ w13[e].double().T
+        if act == "relu2":
+            a = torch.relu(h) ** 2
+        else:
+            g, u = h.chunk(2, -1)
+            if isinstance(act, tuple):
+                _, limit, alpha = act
+                g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+                a = g * torch.sigmoid(alpha * g) * (u + 1.0)
+            else:
+                a = g * torch.sigmoid(g) * u
+        out.index_add_(0, rows, wts[rows, place, None].double() * (a @ w2[e].double().T))
+    return out if more is None else out + more.double()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E,top,K", [(1, 16, 4, 2048), (13, 64, 6, 2048), (3, 5, 5, 200),
+                                       (65, 130, 8, 1000), (1025, 64, 6, 2048), (1027, 8, 1, 8192)])
+def test_route(T, E, top, K):
+    """Against float64: weights to float32 rounding of K products (the chosen
+    scores lie in 0..1, so 1e-5 holds at K = 8192 with logits of a few units),
+    experts wherever the choice is clearer than that."""
+    gen = torch.Generator(device="cuda").manual_seed(T + E)
+    x = torch.randn(T, K, generator=gen, device="cuda").bfloat16()
+    rw = torch.randn(E, K, generator=gen, device="cuda") * (2.0 * K ** -0.5)
+    assert ops.moe_route_ok(x, rw, top)
+    idx, wts, tok = ops.moe_route(x, rw, top)
+    score = torch.softmax(x.double() @ rw.double().T, -1)
+    want = score.topk(min(top + 1, E), -1)
+    clear = torch.ones(T, dtype=torch.bool, device="cuda")
+    if E > top:
+        clear = want.values[:, top - 1] - want.values[:, top] > 1e-5
+    assert clear.float().mean() > 0.9
+    assert torch.equal(idx[clear].sort(-1).values, want.indices[clear, :top].int().sort(-1).values)
+    picked = score.gather(1, idx.long())
+    assert (wts - picked / picked.sum(-1, keepdim=True)).abs().max() < 1e-5
+    assert torch.equal(tok, torch.arange(T, device="cuda", dtype=torch.int32)[:, None].expand(T, top))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("T,E,top,H,I,act,spread", [
+    (65, 8, 2, 128, 128, None, "even"),             # one K step, one strip
+    (64, 4, 1, 256, 128, None, "one"),              # every row in one expert: a full tile
+    (65, 4, 1, 256, 384, None, "one"),              # ... and one row more
+    (300, 64, 6, 512, 256, None, "even"),           # many small experts
+    (5, 16, 2, 256, 256, None, "even"),             # 16-row tiles, experts without rows
+    (17, 4, 1, 256, 128, None, "one"),              # ... one row past a 16-row tile
+    (700, 5, 3, 384, 640, "relu2", "skew"),         # odd step counts, ungated
+    (1100, 4, 3, 256, 256, ("clamp_swish", 7.0, 1.702), "skew"),   # 128-row tiles
+    (129, 3, 1, 128, 128, None, "one"),             # an expert without rows on each side
+])
+def test_sorted_experts(fp8, T, E, top, H, I, act, spread):
+    gen = torch.Generator(device="cuda").manual_seed(T * 7 + I)
+    rn = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    x = rn(T, H).bfloat16()
+    w13 = (rn(E, I if act == "relu2" else 2 * I, H) * H ** -0.5).bfloat16()
+    w2 = (rn(E, H, I) * I ** -0.5).bfloat16()
+    score = rn(T, E)
+    if spread == "skew":
+        score += torch.linspace(3, 0, E, device="cuda")
+    elif spread == "one":
+        score[:, E // 2] += 100.0
+    idx = score.topk(top, -1).indices.to(torch.int32)
+    wts = torch.softmax(score, -1).gather(1, idx.long()).contiguous()
+    more = rn(T, H).bfloat16() if T % 2 else None
+    s13 = s2 = None
+    d13, d2 = w13, w2
+    if fp8:
+        w13, s13 = ops.quant_fp8(w13)
+        w2, s2 = ops.quant_fp8(w2)
+        s13, s2 = s13.view(E, -1), s2.view(E, -1)
+        d13, d2 = torch_ref.dequant_fp8(w13, s13), torch_ref.dequant_fp8(w2, s2)
+    assert ops.moe_sorted_ok(x, w13, w2, act)
+    got = ops.moe_sorted_mlp(x, w13, s13, w2, s2, idx, wts, act, more)
+    again = ops.moe_sorted_mlp(x, w13, s13, w2, s2, idx, wts, act, more)
+    assert torch.equal(got, again)                  # no sum depends on placement
+    want = _reference(x, d13, d2, idx, wts, act, more)
+    # bf16 rounds the middle activation, a pair's row and the sum: three
+    # independent errors of 2^-9 / sqrt(3) of a value (0.0011 each), 0.002 together
+    err = (got.double() - want).norm() / want.norm()
+    assert err < 4e-3, float(err)
+
+
+
+def test_sorted_experts_refuse():
+    """CPU tensors and activations that the kernels do not have stay on the
+    general path."""
+    x = torch.zeros(4, 128, dtype=torch.bfloat16)
+    w13 = torch.zeros(2, 256, 128, dtype=torch.bfloat16)
+    w2 = torch.zeros(2, 128, 128, dtype=torch.bfloat16)
+    assert not ops.moe_sorted_ok(x, w13, w2)
+    assert ops._moe_act("gelu_tanh") is None and ops._moe_act(None) == (0, 0.0, 0.0)
