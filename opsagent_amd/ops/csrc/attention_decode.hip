@@ -16,41 +16,75 @@
 //   o_part   [B*Hk*NSPLIT, G, 128] f32, ml_part [B*Hk*NSPLIT, G, 2] f32
 //   out      [B, Hq, 128] bf16
 //
-// Wave layout: 16 lanes per key row (16 x 8 dims = 128), 4 keys in flight per
-// wave, 4 waves per workgroup each owning a quarter of the split's key range.
+// A split is `chunk` keys, a multiple of 64 (decode_chunk), and at most nsplit
+// splits cover a sequence; blocks past its last key end at once and the combine
+// reads the splits that exist.
 
 #include "common.h"
 
 #define DHEAD 128
 
-// FUSED = true folds the split-combine into this launch with the CDNA guide's
-// Guideline-16 in-launch split-K hand-off (plain-store form): each split
-// block publishes its partial with an agent-scope release and bumps a ticket
-// counter; the LAST arriver for (b, h) acquires, reads every split's slab
-// and writes the final output — saving the second kernel launch per layer.
-// `cnt` must be zeroed before every launch by a hipMemsetAsync on the stream
-// (a memset node under graph capture, replayed first — guide G16).
-// ROPE = true additionally fuses the per-token RoPE + paged-KV scatter that
-// the separate rope_kv kernel did (4.7 us/layer of pure launch latency at
-// decode): every block ropes its G q heads IN REGISTERS (rotate-half partner
-// dims live in lane dl^8 — one __shfl_xor), the main loop covers only the
-// CACHED keys [0, n-1), and the split that owns key n-1 ropes the new k from
-// the raw GEMV output, scatters roped-k and v to the cache slot, and folds
-// the new key into its online softmax. kin/vin/cs/sn/slots/kcw/vcw are only
-// read when ROPE.
-template <int G, bool FUSED, bool ROPE, bool DEEP = true>
+typedef __attribute__((ext_vector_type(8))) __bf16 da_b8;
+typedef __attribute__((ext_vector_type(4))) float da_f4;
+
+// Keys of a split: few splits of 64 keys leave the chip idle, many of them pay the
+// per-block latency (tables, partial results) over and over. `base` comes from
+// the launch (decode_chunk_base).
+__device__ __forceinline__ int decode_chunk(int n, int nsplit, int base) {
+    const int c = (CEIL_DIV(n, nsplit) + 63) & ~63;
+    return c > base ? c : base;
+}
+
+// value of lane `N` of the own 16 lanes, and rotations within them
+template <int N>
+__device__ __forceinline__ float row_bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + N, 0xf, 0xf, true));
+}
+template <int N>
+__device__ __forceinline__ float row_ror(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, 0xf, 0xf, true));
+}
+
+// Scores on the matrix cores, values on the vector units, all in 32 bits.
+//
+// 16 keys x 128 channels go from the cache straight into A fragments of
+// v_mfma_f32_16x16x32_bf16. A query is an exact sum of three bf16 numbers (its
+// rotation is done in float32), which take three groups of the sixteen columns:
+// four heads leave room for them, eight heads need a second product for the third
+// part. A product of 16 keys thus costs 4 or 8 matrix instructions where dot
+// products by lanes cost 4 heads x (32 multiply-adds + a 16-lane reduction) and
+// bound the kernel (1.4 TB/s at batch 47). Adding the column groups is two
+// rotations within 16 lanes; the lane of column c then keeps head c % GP and one
+// key (two for eight heads) of its own 16-lane row, so a weight is one exponential
+// per lane, and all four keys' weights of a row reach its lanes, which hold 8
+// value channels each, by row broadcasts. Softmax weights, their sums and the
+// value sums never leave float32. Each row keeps its own running maximum; rows,
+// waves and splits are merged at the end.
+//
+// FUSED = true folds the split-combine into this launch with an in-launch split-K
+// hand-off (plain-store form): each split block publishes its partial with an
+// agent-scope release and bumps a ticket counter; the LAST arriver for (b, h)
+// acquires, reads every split's slab and writes the final output. `cnt` must be
+// zeroed before every launch. ROPE = true takes the raw projection outputs: the
+// queries are rotated while they are split, the loop covers the CACHED keys
+// [0, n-1), and the split that owns key n-1 rotates the new key, stores it and its
+// value in the cache and starts its softmax with them. kin/vin/cs/sn/slots/kcw/vcw
+// are only read when ROPE.
+template <int G, bool FUSED, bool ROPE>
 __global__ __launch_bounds__(256) void decode_attn_kernel(
     const uint32_t* __restrict__ q, const uint32_t* __restrict__ kc,
     const uint32_t* __restrict__ vc, const int* __restrict__ block_table,
     const int* __restrict__ seq_lens, float* __restrict__ o_part,
     float* __restrict__ ml_part, unsigned* __restrict__ cnt,
     uint32_t* __restrict__ out, int B, int Hk, int max_blocks,
-    int block_shift /* log2(block_size) */, int nsplit, float scale,
+    int block_shift /* log2(block_size) */, int nsplit, int chunk_base, float scale,
     int qs2 /* q batch-row stride in words */,
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
     const float* __restrict__ cs, const float* __restrict__ sn,
     const int* __restrict__ slots, uint32_t* __restrict__ kcw,
     uint32_t* __restrict__ vcw, int ks2, int vs2) {
+    constexpr int GP = G > 4 ? 8 : 4;            // columns of one part of the queries
+    constexpr int KL = GP / 4;                   // keys per lane and tile
     const int bh = blockIdx.x;
     const int b = bh / Hk;
     const int h = bh % Hk;
@@ -58,8 +92,9 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
     const int Hq = Hk * G;
 
     const int n = seq_lens[b];
-    const int chunk = CEIL_DIV(n, nsplit);
+    const int chunk = decode_chunk(n, nsplit, chunk_base);
     const int kstart = split * chunk;
+    if (!FUSED && kstart >= n) return;
     const int kend = min(n, kstart + chunk);
     // ROPE: the new key (index n-1) is handled from registers, not cache
     const int n_cached = ROPE ? (n - 1) : n;
@@ -67,237 +102,276 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
 
     const int lane = threadIdx.x & (WAVE - 1);
     const int wid = threadIdx.x / WAVE;
-    const int g16 = lane >> 4;   // key slot within the wave's 4-key window
-    const int dl = lane & 15;    // owns dims dl*8 .. dl*8+7
+    const int g16 = lane >> 4;   // row of 16 lanes: keys g16 * 4 .. + 3 of a tile
+    const int dl = lane & 15;    // column; owns value channels dl*8 .. dl*8+7
 
     const int part_idx = (bh * nsplit + split);
     float* opart_row = o_part + ((size_t)part_idx * G) * DHEAD;
     float* mlpart_row = ml_part + ((size_t)part_idx * G) * 2;
 
-    // per-wave sub-range (over CACHED keys only)
-    const int span = kend_c - kstart;
-    const int wchunk = CEIL_DIV(max(span, 0), 4);
+    // per-wave sub-range (over CACHED keys only), whole tiles of 16
+    const int span = max(kend_c - kstart, 0);
+    const int wchunk = ((span + 63) >> 6) << 4;
     const int wstart = kstart + wid * wchunk;
     const int wend = min(kend_c, wstart + wchunk);
+    const int nt = wend > wstart ? (wend - wstart + 15) >> 4 : 0;
 
-    // load q fragments: [G][8] floats per lane (all lane groups redundant)
-    float qreg[G][8];
+    const int* btrow = block_table + (size_t)b * max_blocks;
+    const int bmask = (1 << block_shift) - 1;
+    auto slot_of = [&](int kk) {
+        return (int64_t)btrow[kk >> block_shift] << block_shift | (kk & bmask);
+    };
+    uint4 kr_[2][4], vr_[2][4];
+    auto load_tile = [&](int t, uint4 (&kw)[4], uint4 (&vw)[4]) {
+        const int k0 = wstart + t * 16;
+        // keys past the end repeat the last one; their weights are zero
+        const uint32_t* kp = kc + ((size_t)slot_of(min(k0 + dl, wend - 1)) * Hk + h) * (DHEAD / 2) + g16 * 4;
 #pragma unroll
-    for (int gh = 0; gh < G; ++gh) {
-        const uint32_t* qp = q + (size_t)b * qs2 + ((size_t)(h * G + gh) * DHEAD + dl * 8) / 2;
-        uint4 w = *reinterpret_cast<const uint4*>(qp);
+        for (int s = 0; s < 4; ++s) kw[s] = *reinterpret_cast<const uint4*>(kp + s * 16);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            vw[i] = *reinterpret_cast<const uint4*>(
+                vc + ((size_t)slot_of(min(k0 + g16 * 4 + i, wend - 1)) * Hk + h) * (DHEAD / 2) + dl * 4);
+    };
+    if (nt > 0) load_tile(0, kr_[0], vr_[0]);
+
+    // queries: lane (column dl, channels s*32 + g16*8 .. + 7 of step s)
+    const int head = dl % GP, part = dl / GP;
+    const bool have = head < G;
+    float qf[4][8];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const uint4 w = *reinterpret_cast<const uint4*>(
+            q + (size_t)b * qs2 + ((size_t)(h * G + (have ? head : 0)) * DHEAD + s * 32 + g16 * 8) / 2);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            qreg[gh][j * 2] = bf16_lo((&w.x)[j]);
-            qreg[gh][j * 2 + 1] = bf16_hi((&w.x)[j]);
+            qf[s][j * 2] = have ? bf16_lo((&w.x)[j]) : 0.0f;
+            qf[s][j * 2 + 1] = have ? bf16_hi((&w.x)[j]) : 0.0f;
         }
     }
-
-    // ROPE: rotate-half q in registers. Lane dl owns dims dl*8..dl*8+7; the
-    // partner half (d +/- 64) lives in lane dl^8 of the same 16-lane group.
-    float c8[8], s8[8];
+    // ROPE: channel d pairs with d + 64, two steps on in the same lane
+    float c8[2][8], s8[2][8];
     if (ROPE) {
-        const int pos = n - 1;
-        const float* crow = cs + (size_t)pos * (DHEAD / 2) + (dl & 7) * 8;
-        const float* srow = sn + (size_t)pos * (DHEAD / 2) + (dl & 7) * 8;
+        const int pos = max(n - 1, 0);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            c8[j] = crow[j];
-            s8[j] = srow[j];
+        for (int s = 0; s < 2; ++s) {
+            const float* crow = cs + (size_t)pos * (DHEAD / 2) + s * 32 + g16 * 8;
+            const float* srow = sn + (size_t)pos * (DHEAD / 2) + s * 32 + g16 * 8;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                c8[s][j] = crow[j];
+                s8[s][j] = srow[j];
+            }
         }
 #pragma unroll
-        for (int gh = 0; gh < G; ++gh) {
-            float part[8];
+        for (int s = 0; s < 2; ++s)
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                part[j] = __shfl_xor(qreg[gh][j], 8, WAVE);
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                qreg[gh][j] = (dl < 8)
-                                  ? qreg[gh][j] * c8[j] - part[j] * s8[j]
-                                  : qreg[gh][j] * c8[j] + part[j] * s8[j];
-        }
+            for (int j = 0; j < 8; ++j) {
+                const float x1 = qf[s][j], x2 = qf[s + 2][j];
+                qf[s][j] = x1 * c8[s][j] - x2 * s8[s][j];
+                qf[s + 2][j] = x2 * c8[s][j] + x1 * s8[s][j];
+            }
     }
 
-    float m[G], lsum[G], o[G][8];
+    // running maximum of the lane's head over its row's keys, the lane's share of
+    // the sum of weights, value sums of all heads
+    float m = -INFINITY, lsum = 0.0f, o[G][8];
 #pragma unroll
-    for (int gh = 0; gh < G; ++gh) {
-        m[gh] = -INFINITY;
-        lsum[gh] = 0.0f;
+    for (int gh = 0; gh < G; ++gh)
 #pragma unroll
         for (int j = 0; j < 8; ++j) o[gh][j] = 0.0f;
-    }
 
-    const int bmask = (1 << block_shift) - 1;
-    const int* btrow = block_table + (size_t)b * max_blocks;
-
-    // 2-deep key-quad pipeline: issue the raw 16-B K/V loads for quad i+1
-    // before the softmax/accumulate work of quad i — the online-softmax
-    // update is loop-carried but the loads are not, and one quad in flight
-    // (2 x 16 B/lane) is far too little to cover HBM latency at 8 waves/CU.
-    auto issue_loads = [&](int kk0, uint4& kw, uint4& vw, bool& valid, int64_t&) {
-        const int kk = kk0 + g16;
-        valid = (kk0 < wend) && (kk < wend);
-        if (valid) {
-            const int64_t slot =
-                (int64_t)btrow[kk >> block_shift] << block_shift | (kk & bmask);
-            kw = *reinterpret_cast<const uint4*>(
-                kc + ((size_t)slot * Hk + h) * (DHEAD / 2) + dl * 4);
-            vw = *reinterpret_cast<const uint4*>(
-                vc + ((size_t)slot * Hk + h) * (DHEAD / 2) + dl * 4);
-        }
-    };
-    auto process = [&](const uint4& kw, const uint4& vw, bool valid) {
-        float kv_k[8], kv_v[8];
-        if (valid) {
+    if (ROPE && n - 1 >= kstart && n - 1 < kend && wid == 3) {
+        uint4 vw = *reinterpret_cast<const uint4*>(
+            vin + (size_t)b * vs2 + ((size_t)h * DHEAD + dl * 8) / 2);
+        float kf[4][8];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const uint4 w = *reinterpret_cast<const uint4*>(
+                kin + (size_t)b * ks2 + ((size_t)h * DHEAD + s * 32 + g16 * 8) / 2);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                kv_k[j * 2] = bf16_lo((&kw.x)[j]);
-                kv_k[j * 2 + 1] = bf16_hi((&kw.x)[j]);
-                kv_v[j * 2] = bf16_lo((&vw.x)[j]);
-                kv_v[j * 2 + 1] = bf16_hi((&vw.x)[j]);
+                kf[s][j * 2] = bf16_lo((&w.x)[j]);
+                kf[s][j * 2 + 1] = bf16_hi((&w.x)[j]);
             }
         }
+        float dot = 0.0f;
 #pragma unroll
-        for (int gh = 0; gh < G; ++gh) {
-            float s = 0.0f;
-            if (valid) {
+        for (int s = 0; s < 2; ++s)
 #pragma unroll
-                for (int j = 0; j < 8; ++j) s += qreg[gh][j] * kv_k[j];
+            for (int j = 0; j < 8; ++j) {
+                const float x1 = kf[s][j], x2 = kf[s + 2][j];
+                kf[s][j] = x1 * c8[s][j] - x2 * s8[s][j];
+                kf[s + 2][j] = x2 * c8[s][j] + x1 * s8[s][j];
+                dot = fmaf(qf[s][j], kf[s][j], dot);
+                dot = fmaf(qf[s + 2][j], kf[s + 2][j], dot);
             }
-            s = group16_reduce_sum(s);  // all 16 lanes of the group get the dot
-            if (valid) {
-                s *= scale;
-                const float mn = fmaxf(m[gh], s);
-                const float alpha = __expf(m[gh] - mn);
-                const float p = __expf(s - mn);
+        dot += __shfl_xor(dot, 16, WAVE);
+        dot += __shfl_xor(dot, 32, WAVE);
+        const int64_t slot = slots[b];
+        if (dl == 0) {
 #pragma unroll
-                for (int j = 0; j < 8; ++j) o[gh][j] = o[gh][j] * alpha + p * kv_v[j];
-                lsum[gh] = lsum[gh] * alpha + p;
-                m[gh] = mn;
+            for (int s = 0; s < 4; ++s)
+                *reinterpret_cast<uint4*>(kcw + ((size_t)slot * Hk + h) * (DHEAD / 2) + s * 16 + g16 * 4) =
+                    make_uint4(pack_bf16x2(kf[s][0], kf[s][1]), pack_bf16x2(kf[s][2], kf[s][3]),
+                               pack_bf16x2(kf[s][4], kf[s][5]), pack_bf16x2(kf[s][6], kf[s][7]));
+        }
+        if (g16 == 0) {
+            *reinterpret_cast<uint4*>(vcw + ((size_t)slot * Hk + h) * (DHEAD / 2) + dl * 4) = vw;
+            m = dot * scale;
+            lsum = part == 0 ? 1.0f : 0.0f;
+#pragma unroll
+            for (int gh = 0; gh < G; ++gh)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    o[gh][j * 2] = bf16_lo((&vw.x)[j]);
+                    o[gh][j * 2 + 1] = bf16_hi((&vw.x)[j]);
+                }
+        }
+    }
+
+    // the lane's part of its query, and the third parts for a second product
+    da_b8 qb[4], qb2[GP == 8 ? 4 : 1];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float hi = bf16_to_f32(f32_to_bf16(qf[s][j]));
+            const float r1 = qf[s][j] - hi;
+            const float mid = bf16_to_f32(f32_to_bf16(r1));
+            const float lo = r1 - mid;
+            if (GP == 8) {
+                qb[s][j] = (__bf16)(part == 0 ? hi : mid);
+                qb2[GP == 8 ? s : 0][j] = (__bf16)(part == 0 ? lo : 0.0f);
+            } else {
+                qb[s][j] = (__bf16)(part == 0 ? hi : part == 1 ? mid : part == 2 ? lo : 0.0f);
             }
         }
-    };
-    {
-        // 4-deep key-quad pipeline (modulo-scheduled with NAMED slots —
-        // a runtime-indexed ring would go to scratch, guide rule 20):
-        // 2-deep left most of the ~900-cycle HBM latency exposed at small
-        // batch, where one quad is only 32 B/lane in flight. DEEP is
-        // dispatched for B<=4 only: the extra slots cost ~34 VGPRs
-        // (G4: 140->174 -> one fewer wave/SIMD) — right when latency-
-        // bound, an occupancy tax once a big batch saturates HBM.
-        // G8 keeps depth 2 (qreg+o already hold 128 VGPRs).
-        int64_t dummy = 0;
-        if (G <= 4 && DEEP) {
-            uint4 kA{}, vA4{}, kB{}, vB4{}, kC{}, vC4{}, kD{}, vD4{};
-            bool va = false, vb = false, vc2 = false, vd = false;
-            issue_loads(wstart, kA, vA4, va, dummy);
-            issue_loads(wstart + 4, kB, vB4, vb, dummy);
-            issue_loads(wstart + 8, kC, vC4, vc2, dummy);
-            for (int kk0 = wstart; kk0 < wend; kk0 += 16) {
-                issue_loads(kk0 + 12, kD, vD4, vd, dummy);
-                process(kA, vA4, va);
-                issue_loads(kk0 + 16, kA, vA4, va, dummy);
-                process(kB, vB4, vb);
-                issue_loads(kk0 + 20, kB, vB4, vb, dummy);
-                process(kC, vC4, vc2);
-                issue_loads(kk0 + 24, kC, vC4, vc2, dummy);
-                process(kD, vD4, vd);
-            }
+
+    auto process = [&](int t, const uint4 (&kw)[4], const uint4 (&vw)[4]) {
+        da_f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(da_b8, kw[s]), qb[s], acc, 0, 0, 0);
+        if (GP == 8) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(da_b8, kw[s]),
+                                                              qb2[GP == 8 ? s : 0], acc, 0, 0, 0);
+        }
+        float x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            x[i] = acc[i];
+            if (GP == 4) x[i] += row_ror<4>(x[i]);
+            x[i] += row_ror<8>(x[i]);
+        }
+        // the lane's own keys of its row
+        float sc[KL], p[KL];
+        const int key = wstart + t * 16 + g16 * 4 + part * KL;
+        if (GP == 4) {
+            sc[0] = part & 2 ? (part & 1 ? x[3] : x[2]) : (part & 1 ? x[1] : x[0]);
         } else {
-            uint4 kwA{}, vwA{}, kwB{}, vwB{};
-            bool va = false, vb = false;
-            issue_loads(wstart, kwA, vwA, va, dummy);
-            for (int kk0 = wstart; kk0 < wend; kk0 += 4) {
-                issue_loads(kk0 + 4, kwB, vwB, vb, dummy);
-                process(kwA, vwA, va);
-                kwA = kwB; vwA = vwB; va = vb;
-            }
+            sc[0] = part ? x[2] : x[0];
+            sc[KL - 1] = part ? x[3] : x[1];
+        }
+        float mx = m;
+#pragma unroll
+        for (int i = 0; i < KL; ++i) {
+            sc[i] = key + i < wend ? sc[i] * scale : -INFINITY;
+            mx = fmaxf(mx, sc[i]);
+        }
+        if (GP == 4) mx = fmaxf(mx, row_ror<4>(mx));
+        mx = fmaxf(mx, row_ror<8>(mx));
+        const float ref = mx == -INFINITY ? 0.0f : mx;
+        const float alpha = __expf(m - ref);
+        m = mx;
+        lsum *= alpha;
+#pragma unroll
+        for (int i = 0; i < KL; ++i) {
+            p[i] = __expf(sc[i] - ref);
+            lsum += p[i];
+        }
+        // rescale the value sums only where some row's maximum moved
+        if (__any(alpha != 1.0f)) {
+            float al[8];
+            al[0] = row_bcast<0>(alpha); al[1] = row_bcast<1>(alpha);
+            al[2] = row_bcast<2>(alpha); al[3] = row_bcast<3>(alpha);
+            al[4] = row_bcast<4>(alpha); al[5] = row_bcast<5>(alpha);
+            al[6] = row_bcast<6>(alpha); al[7] = row_bcast<7>(alpha);
+#pragma unroll
+            for (int gh = 0; gh < G; ++gh)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) o[gh][j] *= al[gh];
+        }
+#define DA_KEY(I)                                                                              \
+    {                                                                                          \
+        float vf[8], pb[8];                                                                    \
+        _Pragma("unroll") for (int j = 0; j < 4; ++j) {                                        \
+            vf[j * 2] = bf16_lo((&vw[I].x)[j]);                                                \
+            vf[j * 2 + 1] = bf16_hi((&vw[I].x)[j]);                                            \
+        }                                                                                      \
+        const float pv = p[GP == 4 ? 0 : ((I) & 1)];                                           \
+        constexpr int c0 = GP == 4 ? (I) * 4 : ((I) >> 1) * 8;                                 \
+        pb[0] = row_bcast<c0 + 0>(pv);                                                         \
+        if (G > 1) pb[1] = row_bcast<c0 + 1>(pv);                                              \
+        if (G > 2) {                                                                           \
+            pb[2] = row_bcast<c0 + 2>(pv);                                                     \
+            pb[3] = row_bcast<c0 + 3>(pv);                                                     \
+        }                                                                                      \
+        if (G > 4) {                                                                           \
+            pb[4] = row_bcast<(c0 + 4) & 15>(pv);                                              \
+            pb[5] = row_bcast<(c0 + 5) & 15>(pv);                                              \
+            pb[6] = row_bcast<(c0 + 6) & 15>(pv);                                              \
+            pb[7] = row_bcast<(c0 + 7) & 15>(pv);                                              \
+        }                                                                                      \
+        _Pragma("unroll") for (int gh = 0; gh < G; ++gh)                                       \
+            _Pragma("unroll") for (int j = 0; j < 8; ++j)                                      \
+                o[gh][j] = fmaf(pb[gh], vf[j], o[gh][j]);                                      \
+    }
+        DA_KEY(0) DA_KEY(1) DA_KEY(2) DA_KEY(3)
+#undef DA_KEY
+    };
+    // one tile in flight behind the one in work; the last load repeats its tile, so
+    // that waits count exactly
+    for (int t = 0; t < nt; t += 2) {
+        load_tile(min(t + 1, nt - 1), kr_[1], vr_[1]);
+        __builtin_amdgcn_sched_barrier(0);
+        process(t, kr_[0], vr_[0]);
+        if (t + 1 < nt) {
+            load_tile(min(t + 2, nt - 1), kr_[0], vr_[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            process(t + 1, kr_[1], vr_[1]);
         }
     }
 
-    // ROPE: the owning split ropes the NEW key from the raw GEMV output,
-    // scatters roped-k and v to the cache slot, and folds it into wave 3's
-    // online softmax (the cross-wave LDS merge below absorbs it).
-    if (ROPE) {
-        const int pos = n - 1;
-        if (pos >= kstart && pos < kend && wid == 3) {
-            const bool nv = (g16 == 0);
-            uint4 kw{}, vw{};
-            if (nv) {
-                kw = *reinterpret_cast<const uint4*>(
-                    kin + (size_t)b * ks2 + ((size_t)h * DHEAD + dl * 8) / 2);
-                vw = *reinterpret_cast<const uint4*>(
-                    vin + (size_t)b * vs2 + ((size_t)h * DHEAD + dl * 8) / 2);
-            }
-            float kf[8], vf[8];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                kf[j * 2] = bf16_lo((&kw.x)[j]);
-                kf[j * 2 + 1] = bf16_hi((&kw.x)[j]);
-                vf[j * 2] = bf16_lo((&vw.x)[j]);
-                vf[j * 2 + 1] = bf16_hi((&vw.x)[j]);
-            }
-            float kp[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) kp[j] = __shfl_xor(kf[j], 8, WAVE);
-            float kr[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                kr[j] = (dl < 8) ? kf[j] * c8[j] - kp[j] * s8[j]
-                                 : kf[j] * c8[j] + kp[j] * s8[j];
-            if (nv) {
-                const int64_t slot = slots[b];
-                uint4 kout;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    (&kout.x)[j] = pack_bf16x2(kr[j * 2], kr[j * 2 + 1]);
-                *reinterpret_cast<uint4*>(
-                    kcw + ((size_t)slot * Hk + h) * (DHEAD / 2) + dl * 4) = kout;
-                *reinterpret_cast<uint4*>(
-                    vcw + ((size_t)slot * Hk + h) * (DHEAD / 2) + dl * 4) = vw;
-            }
-#pragma unroll
-            for (int gh = 0; gh < G; ++gh) {
-                float s = 0.0f;
-                if (nv) {
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) s += qreg[gh][j] * kr[j];
-                }
-                s = group16_reduce_sum(s);
-                if (nv) {
-                    s *= scale;
-                    const float mn = fmaxf(m[gh], s);
-                    const float alpha = __expf(m[gh] - mn);
-                    const float p = __expf(s - mn);
-#pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        o[gh][j] = o[gh][j] * alpha + p * vf[j];
-                    lsum[gh] = lsum[gh] * alpha + p;
-                    m[gh] = mn;
-                }
-            }
-        }
-    }
+    // sums and maxima of every head to all lanes of a row
+    if (GP == 4) lsum += row_ror<4>(lsum);
+    lsum += row_ror<8>(lsum);
+    float mh[8], lh[8];
+    mh[0] = row_bcast<0>(m); mh[1] = row_bcast<1>(m); mh[2] = row_bcast<2>(m); mh[3] = row_bcast<3>(m);
+    mh[4] = row_bcast<4>(m); mh[5] = row_bcast<5>(m); mh[6] = row_bcast<6>(m); mh[7] = row_bcast<7>(m);
+    lh[0] = row_bcast<0>(lsum); lh[1] = row_bcast<1>(lsum); lh[2] = row_bcast<2>(lsum); lh[3] = row_bcast<3>(lsum);
+    lh[4] = row_bcast<4>(lsum); lh[5] = row_bcast<5>(lsum); lh[6] = row_bcast<6>(lsum); lh[7] = row_bcast<7>(lsum);
 
     // merge the wave's 4 key-groups (lanes l, l^16, l^32 hold same dims)
 #pragma unroll
     for (int off = 16; off <= 32; off <<= 1) {
 #pragma unroll
         for (int gh = 0; gh < G; ++gh) {
-            const float m2 = __shfl_xor(m[gh], off, WAVE);
-            const float l2 = __shfl_xor(lsum[gh], off, WAVE);
+            const float m2 = __shfl_xor(mh[gh], off, WAVE);
+            const float l2 = __shfl_xor(lh[gh], off, WAVE);
             float o2[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) o2[j] = __shfl_xor(o[gh][j], off, WAVE);
-            const float mn = fmaxf(m[gh], m2);
+            const float mn = fmaxf(mh[gh], m2);
             // guard: empty partial (l == 0, m == -inf) must not produce NaN
-            const float a1 = (lsum[gh] > 0.0f) ? __expf(m[gh] - mn) : 0.0f;
+            const float a1 = (lh[gh] > 0.0f) ? __expf(mh[gh] - mn) : 0.0f;
             const float a2 = (l2 > 0.0f) ? __expf(m2 - mn) : 0.0f;
 #pragma unroll
             for (int j = 0; j < 8; ++j) o[gh][j] = o[gh][j] * a1 + o2[j] * a2;
-            lsum[gh] = lsum[gh] * a1 + l2 * a2;
-            m[gh] = (lsum[gh] > 0.0f) ? mn : -INFINITY;
+            lh[gh] = lh[gh] * a1 + l2 * a2;
+            mh[gh] = (lh[gh] > 0.0f) ? mn : -INFINITY;
         }
     }
 
@@ -310,8 +384,8 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
 #pragma unroll
             for (int j = 0; j < 8; ++j) lds_o[wid][gh][dl * 8 + j] = o[gh][j];
             if (dl == 0) {
-                lds_ml[wid][gh][0] = m[gh];
-                lds_ml[wid][gh][1] = lsum[gh];
+                lds_ml[wid][gh][0] = mh[gh];
+                lds_ml[wid][gh][1] = lh[gh];
             }
         }
     }
@@ -400,7 +474,8 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
 template <int G>
 __global__ __launch_bounds__(512) void decode_combine_kernel(
     const float* __restrict__ o_part, const float* __restrict__ ml_part,
-    uint32_t* __restrict__ out, int B, int Hk, int nsplit) {
+    const int* __restrict__ seq_lens, uint32_t* __restrict__ out, int B, int Hk, int nsplit,
+    int chunk_base) {
     const int bq = blockIdx.x;
     const int Hq = Hk * G;
     const int b = bq / Hq;
@@ -412,7 +487,9 @@ __global__ __launch_bounds__(512) void decode_combine_kernel(
 
     extern __shared__ __attribute__((aligned(16))) float sml[];  // [nsplit][2]
     const int base = (b * Hk + h) * nsplit;
-    for (int s = threadIdx.x; s < nsplit; s += blockDim.x) {
+    const int n = seq_lens[b];
+    const int ns = CEIL_DIV(n, decode_chunk(n, nsplit, chunk_base));
+    for (int s = threadIdx.x; s < ns; s += blockDim.x) {
         const float2 ml = *reinterpret_cast<const float2*>(
             ml_part + ((size_t)(base + s) * G + gh) * 2);
         sml[s * 2] = ml.x;
@@ -421,10 +498,10 @@ __global__ __launch_bounds__(512) void decode_combine_kernel(
     __syncthreads();
 
     float mt = -INFINITY;
-    for (int s = sh; s < nsplit; s += 4)
+    for (int s = sh; s < ns; s += 4)
         if (sml[s * 2 + 1] > 0.0f) mt = fmaxf(mt, sml[s * 2]);
     float lt = 0.0f, ot = 0.0f;
-    for (int s = sh; s < nsplit; s += 4) {
+    for (int s = sh; s < ns; s += 4) {
         const float lw = sml[s * 2 + 1];
         if (lw > 0.0f) {
             const float sc = __expf(sml[s * 2] - mt);
@@ -455,6 +532,16 @@ __global__ __launch_bounds__(512) void decode_combine_kernel(
     }
 }
 
+// Keys of the smallest split, by the (sequence, key head) pairs of the launch. Both
+// launches, 8 key heads, us with 64 / 128 / 256 / 512 keys: one sequence of 1151
+// tokens 14.4 / 14.5 / 15.9 / 19.3 (16.8 before scores ran on the matrix cores),
+// 8 of up to 1500 29.3 / 20.6 / 20.6 / 21.2 (38.5), 16 43.3 / 32.0 / 27.8 / 30.4
+// (64.3), 32 of up to 3000 104 / 86 / 72 / 69 (146), 64 180 / 153 / 129 / 117 (266;
+// its cache rows alone take 89 at 5.5 TB/s), 64 of up to 300 39 / 31 / 27 / 26 (152).
+static int decode_chunk_base(int pairs) {
+    return pairs <= 8 ? 64 : pairs <= 64 ? 128 : pairs <= 128 ? 256 : 512;
+}
+
 // fused: cnt_ws must be a zero-initialized... no — zeroed HERE each call via
 // hipMemsetAsync (graph-capturable memset node). fused=0 keeps the two-kernel
 // path (A/B reference and fallback).
@@ -481,41 +568,37 @@ extern "C" int oa_attention_decode(void* stream, const void* q, const void* kc,
         if (e != hipSuccess) return (int)e;
     }
 
-    const bool deep = B <= 4;
+    const int cb = decode_chunk_base(B * Hk);
 #define LAUNCH_G(GV)                                                                \
     do {                                                                            \
-        auto kf = deep ? decode_attn_kernel<GV, true, false, true>                  \
-                       : decode_attn_kernel<GV, true, false, false>;                \
-        auto ku = deep ? decode_attn_kernel<GV, false, false, true>                 \
-                       : decode_attn_kernel<GV, false, false, false>;               \
         if (fused) {                                                                \
-            hipLaunchKernelGGL(kf, grid, block,                                     \
+            hipLaunchKernelGGL((decode_attn_kernel<GV, true, false>), grid, block,         \
                                0, (hipStream_t)stream, (const uint32_t*)q,          \
                                (const uint32_t*)kc, (const uint32_t*)vc,            \
                                (const int*)block_table, (const int*)seq_lens,       \
                                (float*)o_part, (float*)ml_part, (unsigned*)cnt_ws,  \
                                (uint32_t*)out, B, Hk, max_blocks, block_shift,      \
-                               nsplit, scale, qs2, (const uint32_t*)nullptr,        \
+                               nsplit, cb, scale, qs2, (const uint32_t*)nullptr,        \
                                (const uint32_t*)nullptr, (const float*)nullptr,     \
                                (const float*)nullptr, (const int*)nullptr,          \
                                (uint32_t*)nullptr, (uint32_t*)nullptr, 0, 0);       \
             HIP_CHECK_LAUNCH();                                                     \
         } else {                                                                    \
-            hipLaunchKernelGGL(ku, grid, block,                                     \
+            hipLaunchKernelGGL((decode_attn_kernel<GV, false, false>), grid, block,        \
                                0, (hipStream_t)stream, (const uint32_t*)q,          \
                                (const uint32_t*)kc, (const uint32_t*)vc,            \
                                (const int*)block_table, (const int*)seq_lens,       \
                                (float*)o_part, (float*)ml_part, (unsigned*)cnt_ws,  \
                                (uint32_t*)out, B, Hk, max_blocks, block_shift,      \
-                               nsplit, scale, qs2, (const uint32_t*)nullptr,        \
+                               nsplit, cb, scale, qs2, (const uint32_t*)nullptr,        \
                                (const uint32_t*)nullptr, (const float*)nullptr,     \
                                (const float*)nullptr, (const int*)nullptr,          \
                                (uint32_t*)nullptr, (uint32_t*)nullptr, 0, 0);       \
             HIP_CHECK_LAUNCH();                                                     \
             hipLaunchKernelGGL((decode_combine_kernel<GV>), cgrid, cblock, clds,    \
                                (hipStream_t)stream, (const float*)o_part,           \
-                               (const float*)ml_part, (uint32_t*)out, B, Hk,        \
-                               nsplit);                                             \
+                               (const float*)ml_part, (const int*)seq_lens,         \
+                               (uint32_t*)out, B, Hk, nsplit, cb);                                             \
             HIP_CHECK_LAUNCH();                                                     \
         }                                                                           \
     } while (0)
@@ -551,25 +634,24 @@ extern "C" int oa_attention_decode_rope(
     dim3 cgrid(B * Hq), cblock(512);
     const int clds = nsplit * 2 * (int)sizeof(float);
 
-    const bool deep = B <= 4;
+    const int cb = decode_chunk_base(B * Hk);
 #define LAUNCH_GR(GV)                                                              \
     do {                                                                            \
-        auto kr = deep ? decode_attn_kernel<GV, false, true, true>                  \
-                       : decode_attn_kernel<GV, false, true, false>;                \
-        hipLaunchKernelGGL(kr, grid, block, 0,   \
+        hipLaunchKernelGGL((decode_attn_kernel<GV, false, true>), grid, block, 0,   \
                            (hipStream_t)stream, (const uint32_t*)q,                 \
                            (const uint32_t*)kc, (const uint32_t*)vc,                \
                            (const int*)block_table, (const int*)seq_lens,           \
                            (float*)o_part, (float*)ml_part, (unsigned*)nullptr,     \
                            (uint32_t*)out, B, Hk, max_blocks, block_shift, nsplit,  \
-                           scale, q_stride / 2, (const uint32_t*)kin,               \
+                           cb, scale, q_stride / 2, (const uint32_t*)kin,               \
                            (const uint32_t*)vin, (const float*)cos_t,               \
                            (const float*)sin_t, (const int*)slots, (uint32_t*)kc,   \
                            (uint32_t*)vc, k_stride / 2, v_stride / 2);              \
         HIP_CHECK_LAUNCH();                                                         \
         hipLaunchKernelGGL((decode_combine_kernel<GV>), cgrid, cblock, clds,        \
                            (hipStream_t)stream, (const float*)o_part,               \
-                           (const float*)ml_part, (uint32_t*)out, B, Hk, nsplit);   \
+                           (const float*)ml_part, (const int*)seq_lens,             \
+                           (uint32_t*)out, B, Hk, nsplit, cb);                      \
         HIP_CHECK_LAUNCH();                                                         \
     } while (0)
 

@@ -1,0 +1,109 @@
+"""Paged decode attention at the edges of tiles (16 keys), waves (64), splits and
+cache blocks, against float64."""
+
+import pytest
+import torch
+
+from opsagent_amd import ops
+
+D = 128
+
+
+def _case(lens, Hk, G, bs, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    rn = lambda *s: torch.randn(*s, generator=gen, device="cuda").bfloat16()  # noqa: E731
+    need = [(n + bs - 1) // bs for n in lens]
+    order = torch.randperm(sum(need), generator=torch.Generator().manual_seed(seed)).tolist()
+    table = torch.zeros(len(lens), max(need) + 1, dtype=torch.int32)
+    at = 0
+    for b, k in enumerate(need):
+        table[b, :k] = torch.tensor(order[at : at + k])
+        at += k
+    kc, vc = rn(at, bs, Hk, D), rn(at, bs, Hk, D)
+    qkv = rn(len(lens), (Hk * G + 2 * Hk) * D)
+    q, k, v = (t.view(len(lens), -1, D) for t in qkv.split([Hk * G * D, Hk * D, Hk * D], -1))
+    slots = [int(table[b, (n - 1) // bs]) * bs + (n - 1) % bs for b, n in enumerate(lens)]
+    return (q, k, v, kc, vc, table.cuda(), torch.tensor(lens, dtype=torch.int32, device="cuda"),
+            torch.tensor(slots, dtype=torch.int32, device="cuda"))
+
+
+def _attend(q, ks, vs, G):
+    """q [Hq, D], ks/vs [n, Hk, D], float64."""
+    s = torch.einsum("hgd,nhd->hgn", q.view(-1, G, D), ks) * D ** -0.5
+    return torch.einsum("hgn,nhd->hgd", torch.softmax(s, -1), vs).reshape(-1, D)
+
+
+def _rotate(x, pos, cos, sin):
+    c, s = cos[pos].double(), sin[pos].double()
+    a, b = x[..., : D // 2], x[..., D // 2 :]
+    return torch.cat([a * c - b * s, b * c + a * s], -1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("G", [1, 2, 4, 8])
+@pytest.mark.parametrize("lens,bs,nsplit", [
+    ([1], 32, 32),                                   # the new key alone
+    ([2, 16, 17, 18, 64, 65, 66], 32, 32),           # a tile and a wave more or less
+    ([127, 128, 129, 130, 257, 513, 1025], 16, 32),  # a split more or less
+    ([900, 3, 700], 8, 3),                           # blocks smaller than a tile, few splits
+    ([200] * 20 + [1, 65], 32, 1),                   # one split, many sequences
+    ([1500 - 61 * i for i in range(24)], 64, 4),     # large splits, ragged
+])
+def test_decode_attention(G, lens, bs, nsplit):
+    Hk = 4
+    q, k, v, kc, vc, table, lens_t, slots = _case(lens, Hk, G, bs, seed=sum(lens) + G)
+    cos, sin = (t.cuda() for t in ops.rope_cos_sin(2048, D))
+    flat_k, flat_v = kc.view(-1, Hk, D), vc.view(-1, Hk, D)
+    rows = lambda b, n: (table[b, torch.arange(n, device="cuda") // bs].long() * bs  # noqa: E731
+                         + torch.arange(n, device="cuda") % bs)
+    plain, roped, new_k = [], [], []
+    for b, n in enumerate(lens):
+        r = rows(b, n)
+        ks, vs = flat_k[r].double(), flat_v[r].double()
+        plain.append(_attend(q[b].double(), ks, vs, G))
+        new_k.append(_rotate(k[b].double(), n - 1, cos, sin))
+        ks, vs = torch.cat([ks[:-1], new_k[-1][None]]), torch.cat([vs[:-1], v[b].double()[None]])
+        roped.append(_attend(_rotate(q[b].double(), n - 1, cos, sin), ks, vs, G))
+
+    # the result is one bf16 rounding (2^-9 / sqrt(3) of a value = 0.0011 in norm)
+    # of a float32 sum
+    def check(got, want):
+        want = torch.stack(want)
+        err = (got.double() - want).norm() / want.norm()
+        assert err < 2e-3, float(err)
+
+    check(ops.attention_decode_paged(q, kc, vc, table, lens_t, nsplit=nsplit), plain)
+    check(ops.attention_decode_paged(q, kc, vc, table, lens_t, nsplit=nsplit, fused_combine=True),
+          plain)
+    check(ops.attention_decode_rope(q, k, v, kc, vc, table, lens_t, cos, sin, slots,
+                                    nsplit=nsplit), roped)
+    check(flat_k[slots.long()], new_k)               # the new key and value are cached
+    assert torch.equal(flat_v[slots.long()], v)
+
+
+@pytest.mark.gpu
+def test_decode_scores_in_32_bits():
+    """Scores far beyond what 16-bit queries would keep apart: two keys differ by
+    2^-12 of a query of 64, and the softmax is steep."""
+    Hk, G, n = 1, 4, 33
+    q = torch.zeros(1, G, D, device="cuda", dtype=torch.bfloat16)
+    k = torch.zeros(1, Hk, D, device="cuda", dtype=torch.bfloat16)
+    v = torch.zeros_like(k)
+    q[0, :, 3] = 1.0
+    cos = torch.full((64, D // 2), 0.7071067811865476, device="cuda")
+    sin = cos.clone()                                # rotated queries are no bf16 values
+    kc = torch.zeros(2, 32, Hk, D, device="cuda", dtype=torch.bfloat16)
+    kc[:, :, 0, 3] = 4096.0
+    kc[0, 7, 0, 3 + D // 2] = 64.0                   # 64 * 0.7071 above the others
+    vc = torch.randn(2, 32, Hk, D, device="cuda").bfloat16()
+    table = torch.tensor([[0, 1]], dtype=torch.int32, device="cuda")
+    lens = torch.tensor([n], dtype=torch.int32, device="cuda")
+    slots = torch.tensor([32], dtype=torch.int32, device="cuda")
+    got = ops.attention_decode_rope(q, k, v, kc, vc, table, lens, cos, sin, slots, scale=0.25)
+    qr = _rotate(q[0].double(), 0, cos, sin)
+    ks = torch.cat([kc[0, :, :].double(), _rotate(k.double(), 0, cos, sin)])
+    vs = torch.cat([vc[0].double(), v.double()])
+    s = torch.einsum("hd,nd->hn", qr, ks[:, 0]) * 0.25
+    want = torch.softmax(s, -1) @ vs[:, 0]
+    # scores are near 724, float32 keeps 6e-5 of them: weights to 1e-4, then bf16
+    assert ((got[0].double() - want).norm() / want.norm()) < 2e-3
