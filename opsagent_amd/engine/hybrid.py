@@ -954,11 +954,10 @@ class GatedMLP(nn.Module):
         self.down_w = _param(_rand(gen, hidden, ff, std=1.0 / math.sqrt(ff), dtype=dtype))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        M, K = x.shape
+        K = x.shape[1]
         if (
-            x.is_cuda and x.dtype == torch.bfloat16 and K % 8 == 0 and self.ff % 8 == 0
-            and isinstance(self.act, str)
-            and (ops._gemv_m_ok(M) or ops._bf16_mfma_ok(M, K, gateup=True))
+            K % 8 == 0 and self.ff % 8 == 0 and isinstance(self.act, str)
+            and ops.gateup_fused(x, self.gate_up_w, self.ff)
         ):
             act = ops.gateup_act(x, self.gate_up_w, self.ff, self.act)   # fused decode GEMV
         else:

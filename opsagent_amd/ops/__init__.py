@@ -72,16 +72,59 @@ def _gemv_m_ok(M: int) -> bool:
     return M in _GEMV_MS and M <= cap
 
 
+def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
+    """Which form of the skinny product (skinny.hip; figures there) takes M rows
+    of K columns against N (gate-up: 2N) weight rows: 0 none, 1 strips, 2
+    persistent.
+
+    The persistent form pays where a block goes over several strips: gate-up and
+    N >= 6144 up to 16 rows, N >= 16384 up to 32. A strip block reads all of x from
+    the L2, which costs 0.6 of the time that so many weight bytes take; the library
+    starts 3.5 us later and streams 0.87 as fast, so strips win while their x
+    traffic is under 35 MB + a quarter of the weight (25 MB + a fifth from 17 rows
+    on, whose fragments are two)."""
+    if M < 1 or M > 32 or K % 32 != 0:
+        return 0
+    if K == 4096 and (M <= 16 if gateup or N < 16384 else True) and (gateup or N >= 6144):
+        return 2
+    weight = (2 if gateup else 1) * N * K * 2e-6
+    traffic = ((N + 15) // 16) * M * K * 2e-6
+    return int(traffic < (35 + 0.25 * weight if M <= 16 else 25 + 0.2 * weight))
+
+
+def _skinny_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """16-byte loads of the rows of both operands."""
+    return (
+        x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+        and w.dim() == 2 and w.is_contiguous() and x.dim() >= 1 and x.shape[-1] == w.shape[1]
+        and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1
+                                   and x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0))
+        and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+    )
+
+
+def _skinny(x: torch.Tensor, w: torch.Tensor, form: int, gateup: bool = False,
+            act: int = 0) -> torch.Tensor:
+    lib, hip = _lib()
+    K = x.shape[-1]
+    M, N = x.numel() // K, w.shape[0] // (2 if gateup else 1)
+    out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
+    hip.check(lib.oa_skinny(hip.current_stream_ptr(), x.data_ptr(),
+                            K if x.is_contiguous() else x.stride(0), w.data_ptr(), out.data_ptr(),
+                            M, N, K, int(gateup), act, form), "oa_skinny")
+    return out
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """F.linear with custom HIP fast paths for decode shapes: the VALU
-    skinny GEMV at M <= 2 (hipBLASLt's M=1 kernels run ~2.5x off the HBM
-    roofline on gfx950) and the MFMA batched GEMV at M 3..8 / K <= 6144
-    (_bf16_mfma_ok); everything else goes to hipBLASLt."""
+    """F.linear with custom HIP paths for decode shapes: the VALU GEMV at M <= 2
+    (hipBLASLt's M=1 kernels run ~2.5x off the HBM roofline on gfx950) and the
+    skinny matrix-core products up to 32 rows where they win (_skinny_form);
+    everything else goes to hipBLASLt."""
     M = x.numel() // x.shape[-1]
     if (
         x.is_cuda
         and x.dtype == torch.bfloat16
-        and (_gemv_m_ok(M) or _bf16_mfma_ok(M, x.shape[-1]))
+        and _gemv_m_ok(M)
         and x.shape[-1] % 8 == 0
         and w.stride(1) == 1
         and x.is_contiguous()
@@ -102,6 +145,10 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         )
         hip_lib.check(rc, "oa_gemv")
         return out
+    if M <= 32 and _skinny_ok(x, w):
+        form = _skinny_form(M, w.shape[0], w.shape[1])
+        if form:
+            return _skinny(x, w, form)
     return torch.nn.functional.linear(x, w)
 
 
@@ -580,46 +627,44 @@ def rope_kv_fused(
 def gateup_silu(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> torch.Tensor:
     """silu(x @ gate^T) * (x @ up^T) with gate_up_w = [gate; up] rows.
 
-    GPU decode (M <= 8): one fused HIP kernel, no [*, 2I] intermediate.
-    Otherwise: library GEMM + the silu_mul kernel."""
-    M = x.numel() // x.shape[-1]
-    if (
-        x.is_cuda
-        and x.dtype == torch.bfloat16
-        and (_gemv_m_ok(M) or _bf16_mfma_ok(M, x.shape[-1], gateup=True))
-        and x.shape[-1] % 8 == 0
-        and x.is_contiguous()
-    ):
-        from opsagent_amd.ops import hip_lib
-
-        lib = hip_lib.get_lib()
-        out = torch.empty(*x.shape[:-1], i_local, dtype=x.dtype, device=x.device)
-        rc = lib.oa_gemv_gateup(
-            hip_lib.current_stream_ptr(), x.data_ptr(), gate_up_w.data_ptr(),
-            out.data_ptr(), M, i_local, x.shape[-1],
-        )
-        hip_lib.check(rc, "oa_gemv_gateup")
-        return out
+    GPU decode: one fused HIP kernel, no [*, 2I] intermediate, where gateup_fused
+    says so. Otherwise: library GEMM + the silu_mul kernel."""
+    if gateup_fused(x, gate_up_w, i_local):
+        return gateup_act(x, gate_up_w, i_local)
     gu = linear(x, gate_up_w)
     gate, up = gu.split([i_local, i_local], dim=-1)
     return silu_mul(gate.contiguous(), up.contiguous())
 
 
+def gateup_fused(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> bool:
+    """Whether gateup_act takes this product in one launch: the VALU GEMV at M <= 2,
+    the skinny matrix-core product up to 32 rows where it wins."""
+    M = x.numel() // x.shape[-1]
+    return (
+        x.is_cuda and x.dtype == torch.bfloat16 and x.shape[-1] % 8 == 0 and x.is_contiguous()
+        and (_gemv_m_ok(M) or (_skinny_ok(x, gate_up_w)
+                               and _skinny_form(M, i_local, x.shape[-1], gateup=True) > 0))
+    )
+
+
 def gateup_act(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int,
                act: str = "silu") -> torch.Tensor:
     """act(x @ gate^T) * (x @ up^T), act "silu" | "gelu_tanh", for decode-sized
-    bf16 batches: one fused GEMV launch."""
-    if act == "silu":
-        return gateup_silu(x, gate_up_w, i_local)
+    bf16 batches that gateup_fused names: one launch."""
     from opsagent_amd.ops import hip_lib
 
     M = x.numel() // x.shape[-1]
-    assert x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and act == "gelu_tanh"
+    assert x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous()
+    assert act in ("silu", "gelu_tanh")
+    if not _gemv_m_ok(M) and _skinny_ok(x, gate_up_w):
+        form = _skinny_form(M, i_local, x.shape[-1], gateup=True)
+        if form:
+            return _skinny(x, gate_up_w, form, gateup=True, act=int(act == "gelu_tanh"))
     lib = hip_lib.get_lib()
     out = torch.empty(*x.shape[:-1], i_local, dtype=x.dtype, device=x.device)
     rc = lib.oa_gemv_gateup_act(
         hip_lib.current_stream_ptr(), x.data_ptr(), gate_up_w.data_ptr(),
-        out.data_ptr(), M, i_local, x.shape[-1], 1,
+        out.data_ptr(), M, i_local, x.shape[-1], int(act == "gelu_tanh"),
     )
     hip_lib.check(rc, "oa_gemv_gateup_act")
     return out

@@ -26,6 +26,7 @@ SOURCES = [
     "fp8_moe.hip",
     "moe_gemv.hip",
     "moe_grouped.hip",
+    "skinny.hip",
 ]
 
 # the sequence-mixer kernels of hybrid decoders live in a library of their

@@ -1,0 +1,79 @@
+"""Skinny products (skinny.hip) against float64 at the edges of strips, fragments
+and steps, in both forms, and what the rule sends where."""
+
+import pytest
+import torch
+
+from opsagent_amd import ops
+
+
+def _err(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+# one bf16 rounding of a float32 sum: half a unit in the last of 8 bits, at most 2^-8
+# of a value (0.0016 in the mean), and float32 sums far below that
+TOL = 2.0 ** -8 + 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 3, 8, 16, 17, 32])
+@pytest.mark.parametrize("N,K,form", [
+    (16, 32, 1),              # one strip, one step: most waves have none
+    (40, 96, 1),              # a strip of eight rows
+    (100, 1408, 1),           # 44 steps over eight waves
+    (2048, 2816, 1),          # 88 steps: rounds and a remainder
+    (48, 14336, 1),           # deep K on four waves
+    (16, 4096, 2),            # one strip for one block
+    (4104, 4096, 2),          # one strip more than there are blocks, half empty
+    (24592, 4096, 2),         # blocks with unequal numbers of strips
+])
+def test_skinny(M, N, K, form):
+    gen = torch.Generator(device="cuda").manual_seed(M * 131 + N)
+    rn = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    wide = rn(M, K + 24).bfloat16()
+    w = (rn(N, K) * K ** -0.5).bfloat16()
+    for x in (wide[:, :K].contiguous(), wide[:, 8 : 8 + K]):
+        assert ops._skinny_ok(x, w)
+        assert _err(ops._skinny(x, w, form), x.double() @ w.double().T) < TOL
+    assert not ops._skinny_ok(wide[:, 3 : 3 + K], w)          # rows start off 16 bytes
+    if form == 2 and M > 16:
+        return
+    x = wide[:, :K].contiguous()
+    up = (rn(N, K) * K ** -0.5).bfloat16()
+    g, u = x.double() @ w.double().T, x.double() @ up.double().T
+    both = torch.cat([w, up])
+    assert _err(ops._skinny(x, both, form, gateup=True), g * torch.sigmoid(g) * u) < TOL
+    want = torch.nn.functional.gelu(g, approximate="tanh") * u
+    assert _err(ops._skinny(x, both, form, gateup=True, act=1), want) < TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [2, 3, 13, 16, 31, 33])
+@pytest.mark.parametrize("N,K", [(6144, 4096), (4096, 4096), (4096, 14336), (1008, 264)])
+def test_linear_routes_agree(M, N, K):
+    """Whatever the rule says, linear and gateup_silu give the product."""
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K, generator=gen, device="cuda").bfloat16()
+    w = (torch.randn(N, K, generator=gen, device="cuda") * K ** -0.5).bfloat16()
+    want = x.double() @ w.double().T
+    assert _err(ops.linear(x, w), want) < TOL
+    assert _err(ops.linear(x.view(M, 1, K), w).view(M, N), want) < TOL
+    g, u = want.chunk(2, -1)
+    # the unfused form rounds gate and up to bf16 before their product (the gate's
+    # error grows up to twofold in silu): 0.0016 * sqrt(1 + 2^2 + 1) in the mean
+    assert _err(ops.gateup_silu(x, w, N // 2), g * torch.sigmoid(g) * u) < 6e-3
+
+
+def test_rule():
+    """The lines as stated at _skinny_form."""
+    form = ops._skinny_form
+    assert form(8, 14336, 4096, gateup=True) == 2 and form(17, 14336, 4096, gateup=True) == 0
+    assert form(8, 6144, 4096) == 2 and form(17, 6144, 4096) == 0
+    assert form(32, 32000, 4096) == 2 and form(33, 32000, 4096) == 0
+    assert form(13, 4096, 4096) == 1 and form(32, 4096, 4096) == 0
+    assert form(3, 4096, 14336) == 1 and form(16, 4096, 14336) == 0
+    assert form(13, 2816, 2048, gateup=True) == 1
+    assert form(8, 64, 1000) == 0                             # K not a multiple of 32
+    x, w = torch.zeros(4, 64, dtype=torch.bfloat16), torch.zeros(8, 64, dtype=torch.bfloat16)
+    assert not ops._skinny_ok(x, w)                           # CPU tensors: the general path
