@@ -116,11 +116,15 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, form: int, gateup: bool = False,
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """F.linear with custom HIP paths for decode shapes: the VALU GEMV at M <= 2
-    (hipBLASLt's M=1 kernels run ~2.5x off the HBM roofline on gfx950) and the
-    skinny matrix-core products up to 32 rows where they win (_skinny_form);
-    everything else goes to hipBLASLt."""
+    """F.linear with custom HIP paths for decode shapes: the VALU GEMV at M = 1
+    (hipBLASLt's M=1 kernels run ~2.5x off the HBM roofline on gfx950), the skinny
+    matrix-core products up to 32 rows where they win (_skinny_form), the VALU GEMV
+    for what two rows are left; everything else goes to hipBLASLt."""
     M = x.numel() // x.shape[-1]
+    if 1 < M <= 32 and _skinny_ok(x, w):
+        form = _skinny_form(M, w.shape[0], w.shape[1])
+        if form:
+            return _skinny(x, w, form)
     if (
         x.is_cuda
         and x.dtype == torch.bfloat16
@@ -145,10 +149,6 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         )
         hip_lib.check(rc, "oa_gemv")
         return out
-    if M <= 32 and _skinny_ok(x, w):
-        form = _skinny_form(M, w.shape[0], w.shape[1])
-        if form:
-            return _skinny(x, w, form)
     return torch.nn.functional.linear(x, w)
 
 
@@ -637,8 +637,8 @@ def gateup_silu(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> torch
 
 
 def gateup_fused(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> bool:
-    """Whether gateup_act takes this product in one launch: the VALU GEMV at M <= 2,
-    the skinny matrix-core product up to 32 rows where it wins."""
+    """Whether gateup_act takes this product in one launch: the VALU GEMV up to
+    two rows, the skinny matrix-core product up to 32 where it wins."""
     M = x.numel() // x.shape[-1]
     return (
         x.is_cuda and x.dtype == torch.bfloat16 and x.shape[-1] % 8 == 0 and x.is_contiguous()
@@ -656,7 +656,7 @@ def gateup_act(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int,
     M = x.numel() // x.shape[-1]
     assert x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous()
     assert act in ("silu", "gelu_tanh")
-    if not _gemv_m_ok(M) and _skinny_ok(x, gate_up_w):
+    if M > 1 and _skinny_ok(x, gate_up_w):
         form = _skinny_form(M, i_local, x.shape[-1], gateup=True)
         if form:
             return _skinny(x, gate_up_w, form, gateup=True, act=int(act == "gelu_tanh"))

@@ -191,6 +191,190 @@ __global__ __launch_bounds__(256) void gemv_gateup_kernel(
     }
 }
 
+// One activation row (M = 1), K a multiple of 2048. gemv_kernel keeps one 1 KiB load
+// per row in flight and, with NORM, normalises the activations again for every row;
+// here the block's (normalised) activations are a float32 image in LDS, made while the
+// first weight loads are under way, and a wave goes over its rows as one stream of
+// GR-chunk groups (512 columns each): the next group, also the next row's, is loaded
+// before the current one is used. The image keeps columns 0-3 and 4-7 of every eight
+// apart, so that 16-byte LDS reads of a wave are contiguous. RT = 2: gate and up rows.
+// us before and now, weights of 1 GiB in turn: 28672 x 4096 gate-up with norm 43.3 and
+// 38.4, 4096 x 14336 24.9 and 20.6, 6144 x 4096 with norm 12.9 and 11.0, 4096 x 4096
+// 8.9 and 8.5, 128256 x 4096 168 and 163, 2048 x 8192 12.0 and 8.4, 16384 x 2048 gate-up
+// 14.8 and 12.9, 2048 x 2048 4.7 and 4.2 (contiguous reads alone run at 6.4 to 6.9 TB/s).
+template <bool NORM, bool ADDRES, int RT, int GR>
+__global__ __launch_bounds__(512) void gemv1_kernel(const uint32_t* __restrict__ x,
+                                                    const uint32_t* __restrict__ w,
+                                                    uint16_t* __restrict__ out,
+                                                    const uint32_t* __restrict__ wn,
+                                                    const uint16_t* __restrict__ res, int N, int K,
+                                                    int per, float eps, int act) {
+    extern __shared__ __attribute__((aligned(16))) float xl[];   // [2][K / 2]
+    __shared__ float part[8];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = blockIdx.x * 8 + wid;
+    const int r0 = wave * per, r1 = min(r0 + per, N);       // the wave's rows
+    const int k2 = K / 2, groups = K / (512 * GR);
+    const int total = max(r1 - r0, 0) * groups;
+    auto at = [&](int row, int t) { return w + (size_t)(row + (t ? N : 0)) * k2 + lane * 4; };
+    u32x4 a[GR][RT], b[GR][RT];
+    int row = min(r0, N - 1), g = 0;                        // of the group loaded last
+    auto load = [&](u32x4 (&v)[GR][RT]) {
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int i = 0; i < GR; ++i) v[i][t] = nt_load4(at(row, t) + (g * GR + i) * 256);
+    };
+    auto next = [&](u32x4 (&v)[GR][RT]) {
+        if (++g == groups) {
+            g = 0;
+            ++row;
+        }
+        load(v);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    load(a);
+
+    // activations, eight columns per thread and turn
+    float rstd = 1.0f;
+    if (NORM) {
+        float ss = 0.0f;
+        for (int i = tid; i < K / 8; i += 512) {
+            const uint4 v = reinterpret_cast<const uint4*>(x)[i];
+            const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                ss = fmaf(bf16_lo(u[j]), bf16_lo(u[j]), ss);
+                ss = fmaf(bf16_hi(u[j]), bf16_hi(u[j]), ss);
+            }
+        }
+        ss = wave_reduce_sum(ss);
+        if (lane == 0) part[wid] = ss;
+        __syncthreads();
+        ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ss += part[i];
+        rstd = rsqrtf(ss / (float)K + eps);
+    }
+    for (int i = tid; i < K / 8; i += 512) {
+        const uint4 v = reinterpret_cast<const uint4*>(x)[i];
+        const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+        float f[8];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            f[2 * j] = bf16_lo(u[j]);
+            f[2 * j + 1] = bf16_hi(u[j]);
+        }
+        if (NORM) {
+            const uint4 nv = reinterpret_cast<const uint4*>(wn)[i];
+            const uint32_t n4[4] = {nv.x, nv.y, nv.z, nv.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                f[2 * j] *= rstd * bf16_lo(n4[j]);
+                f[2 * j + 1] *= rstd * bf16_hi(n4[j]);
+            }
+        }
+        reinterpret_cast<float4*>(xl)[i] = make_float4(f[0], f[1], f[2], f[3]);
+        reinterpret_cast<float4*>(xl + k2)[i] = make_float4(f[4], f[5], f[6], f[7]);
+    }
+    __syncthreads();
+
+    float acc[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) acc[t] = 0.0f;
+    int ur = r0, ug = 0;                                    // of the group in use
+    auto use = [&](u32x4 (&v)[GR][RT]) {
+#pragma unroll
+        for (int i = 0; i < GR; ++i) {
+            const int c = (ug * GR + i) * 64 + lane;
+            const float4 lo = reinterpret_cast<const float4*>(xl)[c];
+            const float4 hi = reinterpret_cast<const float4*>(xl + k2)[c];
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                float s = acc[t];
+                s = fmaf(lo.x, bf16_lo(v[i][t][0]), s);
+                s = fmaf(lo.y, bf16_hi(v[i][t][0]), s);
+                s = fmaf(lo.z, bf16_lo(v[i][t][1]), s);
+                s = fmaf(lo.w, bf16_hi(v[i][t][1]), s);
+                s = fmaf(hi.x, bf16_lo(v[i][t][2]), s);
+                s = fmaf(hi.y, bf16_hi(v[i][t][2]), s);
+                s = fmaf(hi.z, bf16_lo(v[i][t][3]), s);
+                acc[t] = fmaf(hi.w, bf16_hi(v[i][t][3]), s);
+            }
+        }
+        if (++ug == groups) {
+            float v0 = wave_reduce_sum(acc[0]);
+            if (RT == 2) v0 = gate_act(v0, act) * wave_reduce_sum(acc[RT - 1]);
+            if (lane == 0) {
+                if (ADDRES) v0 += bf16_to_f32(res[ur]);
+                out[ur] = f32_to_bf16(v0);
+            }
+#pragma unroll
+            for (int t = 0; t < RT; ++t) acc[t] = 0.0f;
+            ug = 0;
+            ++ur;
+        }
+    };
+    // the last groups are apart, so that every wait counts the loads behind it exactly
+    int n = 0;
+    for (; n + 2 < total; n += 2) {
+        next(b);
+        use(a);
+        next(a);
+        use(b);
+    }
+    if (n + 2 == total) {
+        next(b);
+        use(a);
+        use(b);
+    } else if (n < total) {
+        use(a);
+    }
+}
+
+// mode as in oa_gemv_ex; gateup > 0: N gate and N up rows, activation gateup - 1
+static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const void* wn,
+                 const void* res, int N, int K, float eps, int mode, int gateup) {
+    // Rows per wave: as many blocks of eight waves as stay resident (two per CU by
+    // registers, four with short rows), fewer and fuller ones where that evens out the
+    // CUs by more than a fifth (6144 x 4096: 2 rows on 384 blocks 12.1 us, 3 on 256 11.0).
+    const int resident = K == 2048 && !gateup ? 4 : 2;
+    auto rounds = [&](int p) { return CEIL_DIV(CEIL_DIV(CEIL_DIV(N, p), 8), 256) * p; };
+    int per = CEIL_DIV(N, 2048 * resident);
+    for (int p = per + 1, p1 = 2 * per + 1; p <= p1; ++p)
+        if (rounds(p) * 5 < rounds(per) * 4) per = p;
+    const int blocks = CEIL_DIV(CEIL_DIV(N, per), 8);
+    const size_t lds = (size_t)K * 4;
+#define G1(NV, RV, RT, GR)                                                                            \
+    hipLaunchKernelGGL((gemv1_kernel<NV, RV, RT, GR>), dim3(blocks), dim3(512), lds, st,              \
+                       (const uint32_t*)x, (const uint32_t*)w, (uint16_t*)out, (const uint32_t*)wn,   \
+                       (const uint16_t*)res, N, K, per, eps, gateup - 1)
+    if (gateup) {
+        if (mode & 1) G1(true, false, 2, 4);
+        else G1(false, false, 2, 4);
+    } else if (K % 4096 == 0) {
+        switch (mode) {
+            case 0: G1(false, false, 1, 8); break;
+            case 1: G1(true, false, 1, 8); break;
+            case 2: G1(false, true, 1, 8); break;
+            default: G1(true, true, 1, 8); break;
+        }
+    } else {
+        switch (mode) {
+            case 0: G1(false, false, 1, 4); break;
+            case 1: G1(true, false, 1, 4); break;
+            case 2: G1(false, true, 1, 4); break;
+            default: G1(true, true, 1, 4); break;
+        }
+    }
+#undef G1
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+// the float32 image of the activations fits the LDS of two blocks per CU
+static bool gemv1_ok(int M, int K) { return M == 1 && K % 2048 == 0 && K <= 16384; }
+
 static bool gemv_bf16_use_mfma(int M, int K, int gateup);
 extern "C" int oa_gemv_bf16_mfma(void* stream, const void* x, const void* w,
                                  void* out, const void* wn, const void* res,
@@ -201,6 +385,8 @@ static int gemv_gateup_impl(void* stream, const void* x, const void* w,
                             void* out, const void* wn, int M, int I, int K,
                             float eps, int norm, int act) {
     if (K % 8 != 0) return -100;
+    if (gemv1_ok(M, K))
+        return gemv1((hipStream_t)stream, x, w, out, wn, nullptr, I, K, eps, norm ? 1 : 0, 1 + act);
     if (gemv_bf16_use_mfma(M, K, 1))
         return oa_gemv_bf16_mfma(stream, x, w, out, wn, nullptr, M, 2 * I, K,
                                  eps, norm ? 1 : 0, 1 + act);
@@ -260,6 +446,8 @@ extern "C" int oa_gemv_ex(void* stream, const void* x, const void* w, void* out,
                           const void* wn, const void* res, int M, int N, int K,
                           float eps, int mode) {
     if (K % 8 != 0) return -100;
+    if (mode < 0 || mode > 3) return -102;
+    if (gemv1_ok(M, K)) return gemv1((hipStream_t)stream, x, w, out, wn, res, N, K, eps, mode, 0);
     if (gemv_bf16_use_mfma(M, K, 0))
         return oa_gemv_bf16_mfma(stream, x, w, out, wn, res, M, N, K, eps,
                                  mode, 0);

@@ -1,0 +1,37 @@
+"""The one-row GEMV of long rows (K a multiple of 2048) against float64: rows that
+do not divide among waves, short and long K, norm prologue, residual, gate-up."""
+
+import pytest
+import torch
+
+from opsagent_amd import ops
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [8, 16, 4097, 6144, 9001])
+@pytest.mark.parametrize("K", [2048, 4096, 6144, 14336])
+def test_one_row(N, K):
+    gen = torch.Generator(device="cuda").manual_seed(N + K)
+    rn = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    x, res = rn(1, K).bfloat16(), rn(1, N).bfloat16()
+    w = (rn(N, K) * K ** -0.5).bfloat16()
+    nw = (1.0 + 0.1 * rn(K)).bfloat16()
+    xd, wd = x.double(), w.double()
+    normed = xd / torch.sqrt((xd * xd).mean() + 1e-5) * nw.double()
+
+    def check(got, want):
+        # one bf16 rounding of a float32 sum: at most 2^-8 of a value
+        assert float((got.double() - want).norm() / want.norm()) < 2.0 ** -8 + 1e-5
+
+    check(ops.linear(x, w), xd @ wd.T)
+    check(ops.linear_norm(x, nw, 1e-5, w), normed @ wd.T)
+    # the sum is rounded once, after the residual
+    check(ops.linear_addres(x, w, res), xd @ wd.T + res.double())
+    if N % 2 == 0:
+        h = N // 2
+        g, u = (normed @ wd.T).chunk(2, -1)
+        check(ops.gateup_silu_norm(x, nw, 1e-5, w, h), g * torch.sigmoid(g) * u)
+        g, u = (xd @ wd.T).chunk(2, -1)
+        check(ops.gateup_act(x, w, h, "silu"), g * torch.sigmoid(g) * u)
+        check(ops.gateup_act(x, w, h, "gelu_tanh"),
+              torch.nn.functional.gelu(g, approximate="tanh") * u)
