@@ -692,6 +692,27 @@ def kv_cache_write(
     hip.check(rc, "oa_kv_write")
 
 
+def _prefill_splits(B: int, Hq: int, Hk: int, Sq: int, Skv: int) -> Tuple[int, bool]:
+    """(key splits, merged form) of prefill attention; (1, False): not split.
+
+    Few queries over many keys leave most CUs idle. Up to 128 queries: blocks of a
+    head, from three tiles of 128 keys on (32 heads on 8, us before / split: 3 over
+    300 14.4 / 11.1, 16 over 2000 64 / 21, 77 over 1264 40.4 / 20.9). More: blocks
+    of a key head, from twelve tiles on (300 over 4000 142 / 54, 1024 over 5000 171 /
+    116; 1024 over 1024 would take 44 instead of 38.5)."""
+    if Hk < 1 or Hq % Hk:
+        return 1, False
+    tiles = (Skv + 127) // 128
+    if Sq <= 128:
+        splits = min(tiles, 256 // max(1, B * Hq)) if tiles >= 3 else 1
+        return max(1, splits), False
+    group = Hq // Hk
+    if group not in (2, 4, 8) or tiles < 12:
+        return 1, False
+    blocks = -(-Sq // (256 // group)) * B * Hk
+    return max(1, min(tiles, 256 // max(1, blocks))), True
+
+
 def attention_prefill(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -716,6 +737,17 @@ def attention_prefill(
     scale = scale if scale is not None else D ** -0.5
     lib, hip = _lib()
     out = torch.empty(B, Sq, Hq, D, dtype=q.dtype, device=q.device)
+    splits, merged = _prefill_splits(B, Hq, Hk, Sq, Skv)
+    if splits > 1 and D == 128 and "OPSAGENT_PREFILL_VARIANT" not in os.environ:
+        part = torch.empty(splits, B, Sq, Hq, D + 2, dtype=torch.float32, device=q.device)
+        sums = splits * B * Sq * Hq * D * 4
+        rc = lib.oa_attention_prefill_split(
+            hip.current_stream_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+            out.data_ptr(), part.data_ptr(), part.data_ptr() + sums, B, Hq, Hk, Sq, Skv, D,
+            scale, q.stride(1), k.stride(1), v.stride(1), splits, int(merged),
+        )
+        hip.check(rc, "oa_attention_prefill_split")
+        return out
     rc = lib.oa_attention_prefill(
         hip.current_stream_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
         out.data_ptr(), B, Hq, Hk, Sq, Skv, D, scale,

@@ -64,11 +64,15 @@ __device__ __forceinline__ int v_img_row_inv(int r) {
 // DMA-bound at ~11 GB/s/CU). The tr16 reads then address (row, d-quad)
 // pieces of the row-major image directly; the same (key&15)<<4 XOR that
 // decollides the K reads spreads the tr read's bank pattern.
-template <int RB, bool PIPE, bool VRM = false, int KB = KVBLK>
+// SPLIT: blockIdx.z takes a run of the q-tile's key tiles and leaves its unnormalised
+// float32 sums with their maximum (scaled scores) and weight sum for
+// prefill_combine_kernel: few queries over many keys fill the chip this way.
+template <int RB, bool PIPE, bool VRM = false, int KB = KVBLK, bool SPLIT = false>
 __global__ __launch_bounds__(512, 1) void attn_prefill_v2(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, uint16_t* __restrict__ out, int B, int Hq,
-    int Hk, int Sq, int Skv, float scale, int qs, int ks, int vs) {
+    int Hk, int Sq, int Skv, float scale, int qs, int ks, int vs,
+    float* __restrict__ po, float* __restrict__ pml) {
     constexpr int QROWS = 16 * RB;
     constexpr int QTILE = QROWS * NWAVE;
     constexpr int P_BYTES = QROWS * KB * 2;
@@ -126,7 +130,10 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v2(
         for (int nb = 0; nb < 8; ++nb) o_acc[rb][nb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 
     const int kv_needed = min(Skv, offset + qtile * QTILE + QTILE);
-    const int ntiles = CEIL_DIV(max(kv_needed, 0), KB);
+    const int all_tiles = CEIL_DIV(max(kv_needed, 0), KB);
+    const int run = SPLIT ? CEIL_DIV(all_tiles, (int)gridDim.z) : all_tiles;
+    const int tile0 = SPLIT ? (int)blockIdx.z * run : 0;
+    const int ntiles = SPLIT ? min(all_tiles, tile0 + run) : all_tiles;
 
     const char* kbase = reinterpret_cast<const char*>(k) +
                         ((size_t)b * Skv * ks + (size_t)hk * DHEAD) * 2;
@@ -258,11 +265,13 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v2(
 #pragma unroll
             for (int r = 0; r < 4; ++r) rowmax[r] = group16_reduce_max(rowmax[r]);
 
-            float alpha[4], psum[4];
+            float alpha[4], psum[4], mref[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float mn = fmaxf(m[rb][r], rowmax[r]);
-                alpha[r] = __expf(m[rb][r] - mn);
+                // a split may show a row none of its keys
+                mref[r] = SPLIT && mn == -INFINITY ? 0.0f : mn;
+                alpha[r] = __expf(m[rb][r] - mref[r]);
                 m[rb][r] = mn;
                 psum[r] = 0.0f;
             }
@@ -272,7 +281,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v2(
             for (int kb = 0; kb < NKB; ++kb) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float p = __expf(s[kb][r] - m[rb][r]);
+                    const float p = __expf(s[kb][r] - mref[r]);
                     s[kb][r] = p;
                     psum[r] += p;
                     *reinterpret_cast<uint16_t*>(
@@ -373,8 +382,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v2(
                          : "memory");
         }
     };
-    if (ntiles > 0) {
-        set_tile(0, 0);
+    if (ntiles > tile0) {
+        set_tile(tile0, 0);
         stage();
     }
     // static priority for the second-dispatched half (guide T5 static
@@ -386,8 +395,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v2(
         __builtin_amdgcn_s_setprio(1);
     drain();
     __syncthreads();
-    for (int t = 0; t < ntiles; ++t) {
-        const int cur = t & 1;
+    for (int t = tile0; t < ntiles; ++t) {
+        const int cur = (t - tile0) & 1;
         if (t + 1 < ntiles) set_tile(t + 1, cur ^ 1);
         if (PIPE && t + 1 < ntiles) stage();
         compute(t, smem + cur * KBYTES, smem + voff + cur * KBYTES);
@@ -403,6 +412,13 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v2(
         for (int r = 0; r < 4; ++r) {
             const int row = qrow0 + rb * 16 + fs * 4 + r;
             if (row >= Sq) continue;
+            if (SPLIT) {
+                const size_t at = ((size_t)blockIdx.z * B * Sq + (size_t)b * Sq + row) * Hq + h;
+#pragma unroll
+                for (int nb = 0; nb < 8; ++nb) po[at * DHEAD + nb * 16 + fr] = o_acc[rb][nb][r];
+                if (fr == 0) *reinterpret_cast<float2*>(pml + at * 2) = make_float2(m[rb][r], lsum[rb][r]);
+                continue;
+            }
             const float inv_l = (lsum[rb][r] > 0.0f) ? 1.0f / lsum[rb][r] : 0.0f;
             uint16_t* op = out + ((size_t)(b * Sq + row) * Hq + h) * DHEAD;
 #pragma unroll
@@ -451,11 +467,15 @@ __device__ __forceinline__ float xor32_f32(float v, int lh) {
 // all GQ heads, cutting the kernel's total KV DMA by GQ: the v3 PMC put
 // the residual WAIT at the staged-KV demand of the co-resident
 // workgroups (~9.6 TB/s against L2+HBM), which this divides by 4.
-template <int KB = 128, int GQ = 1>
+// SPLIT: blockIdx.z takes a run of the q-tile's key tiles and leaves its unnormalised
+// float32 sums with their maximum (raw scores) and weight sum for
+// prefill_combine_kernel: few queries over many keys fill the chip this way.
+template <int KB = 128, int GQ = 1, bool SPLIT = false>
 __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, uint16_t* __restrict__ out, int B, int Hq,
-    int Hk, int Sq, int Skv, float scale, int qs, int ks, int vs) {
+    int Hk, int Sq, int Skv, float scale, int qs, int ks, int vs,
+    float* __restrict__ po, float* __restrict__ pml) {
     constexpr int QROWS = 32;                // per wave
     constexpr int QTILE = QROWS * NWAVE;     // 256 across the WG
     constexpr int QTILE_H = QTILE / GQ;      // rows per head per WG
@@ -498,7 +518,10 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
     for (int db = 0; db < 4; ++db) oa[db] = (f32x16_t)(0.0f);
 
     const int kv_needed = min(Skv, offset + qtile * QTILE_H + QTILE_H);
-    const int ntiles = CEIL_DIV(max(kv_needed, 0), KB);
+    const int all_tiles = CEIL_DIV(max(kv_needed, 0), KB);
+    const int run = SPLIT ? CEIL_DIV(all_tiles, (int)gridDim.z) : all_tiles;
+    const int tile0 = SPLIT ? (int)blockIdx.z * run : 0;
+    const int ntiles = SPLIT ? min(all_tiles, tile0 + run) : all_tiles;
 
     const char* kbase = reinterpret_cast<const char*>(k) +
                         ((size_t)b * Skv * ks + (size_t)hk * DHEAD) * 2;
@@ -629,7 +652,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
         const float m_old = m;
         const float mn = fmaxf(m_old, rowmax);
         m = mn;
-        const float mnb = mn * scale2;
+        // a split may show a row none of its keys
+        const float mnb = SPLIT && mn == -INFINITY ? 0.0f : mn * scale2;
         float psum = 0.0f;
 
         // ---- exp + pack to bf16 quads: pk[kb][g] = keys kb*32+g*8+4*lh+{0..3}
@@ -657,7 +681,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
         // the first few tiles most tiles leave every row max unchanged and
         // the 64 accumulator multiplies + lsum scale are skipped outright
         if (__any(rowmax > m_old)) {
-            const float alpha = __builtin_amdgcn_exp2f((m_old - mn) * scale2);
+            const float alpha = SPLIT && mn == -INFINITY
+                                    ? 1.0f : __builtin_amdgcn_exp2f((m_old - mn) * scale2);
             lsum *= alpha;
 #pragma unroll
             for (int db = 0; db < 4; ++db)
@@ -713,16 +738,16 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
         }
     };
 
-    if (ntiles > 0) {
-        set_tile(0, 0);
+    if (ntiles > tile0) {
+        set_tile(tile0, 0);
         stage();
     }
     if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256)
         __builtin_amdgcn_s_setprio(1);
     drain();
     __syncthreads();
-    for (int t = 0; t < ntiles; ++t) {
-        const int cur = t & 1;
+    for (int t = tile0; t < ntiles; ++t) {
+        const int cur = (t - tile0) & 1;
         const int kv0 = t * KB;
         if (t + 1 < ntiles) set_tile(t + 1, cur ^ 1);
         if (t + 1 < ntiles) stage();
@@ -737,6 +762,19 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
         __syncthreads();
     }
 
+    if (SPLIT) {
+        if (qrow < Sq) {
+            const size_t row = ((size_t)blockIdx.z * B * Sq + (size_t)b * Sq + qrow) * Hq + h;
+#pragma unroll
+            for (int db = 0; db < 4; ++db)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *reinterpret_cast<float4*>(po + row * DHEAD + db * 32 + g * 8 + 4 * lh) =
+                        make_float4(oa[db][g * 4], oa[db][g * 4 + 1], oa[db][g * 4 + 2], oa[db][g * 4 + 3]);
+            if (lh == 0) *reinterpret_cast<float2*>(pml + row * 2) = make_float2(m, lsum);
+        }
+        return;
+    }
     // ---- epilogue: out[q-row][d] = o/l; lane holds dims (i&3)+8*(i>>2)+4*lh
     if (qrow < Sq) {
         const float inv_l = (lsum > 0.0f) ? 1.0f / lsum : 0.0f;
@@ -756,6 +794,73 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
     }
 }
 
+// Splits added up: one wave per (query, head) row, two channels per lane. rows = B * Sq
+// * Hq; scale2 turns a difference of maxima into a power of two.
+__global__ __launch_bounds__(256) void prefill_combine_kernel(const float* __restrict__ po,
+                                                              const float* __restrict__ pml,
+                                                              uint32_t* __restrict__ out, int rows,
+                                                              int nsplit, float scale2) {
+    const int row = blockIdx.x * 4 + threadIdx.x / WAVE, lane = threadIdx.x & (WAVE - 1);
+    if (row >= rows) return;
+    float mx = -INFINITY;
+    for (int s = 0; s < nsplit; ++s) {
+        const float2 ml = *reinterpret_cast<const float2*>(pml + ((size_t)s * rows + row) * 2);
+        if (ml.y > 0.0f) mx = fmaxf(mx, ml.x);
+    }
+    float l = 0.0f, a = 0.0f, b = 0.0f;
+    for (int s = 0; s < nsplit; ++s) {
+        const size_t r = (size_t)s * rows + row;
+        const float2 ml = *reinterpret_cast<const float2*>(pml + r * 2);
+        if (ml.y > 0.0f) {
+            const float w = __builtin_amdgcn_exp2f((ml.x - mx) * scale2);
+            const float2 o = *reinterpret_cast<const float2*>(po + r * DHEAD + lane * 2);
+            l = fmaf(ml.y, w, l);
+            a = fmaf(o.x, w, a);
+            b = fmaf(o.y, w, b);
+        }
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    out[(size_t)row * (DHEAD / 2) + lane] = pack_bf16x2(a * inv, b * inv);
+}
+
+// Key-split forms: merged = 0, a block per head and 128 queries (variant 7); 1, a block
+// per key head and 256 / (Hq / Hk) queries (variant 9; Hq / Hk of 2, 4 or 8).
+// po [nsplit, B, Sq, Hq, 128] and pml [nsplit, B, Sq, Hq, 2]: float32 scratch.
+extern "C" int oa_attention_prefill_split(
+    void* stream, const void* q, const void* k, const void* v, void* out, void* po, void* pml,
+    int B, int Hq, int Hk, int Sq, int Skv, int D, float scale, int q_stride, int k_stride,
+    int v_stride, int nsplit, int merged) {
+    if (D != DHEAD) return -100;
+    if (Hk < 1 || Hq % Hk != 0) return -101;
+    if ((q_stride | k_stride | v_stride) % 8 != 0) return -102;
+    if (nsplit < 1 || nsplit > 65535 || (int64_t)B * Sq * Hq > (1 << 30)) return -105;
+    const int gq = Hq / Hk, rows = B * Sq * Hq;
+    if (rows < 1) return 0;
+#define LAUNCH_SPLIT(KERN, QT, Y)                                                                  \
+    hipLaunchKernelGGL((KERN), dim3(CEIL_DIV(Sq, QT), Y, nsplit), dim3(512), 0,                    \
+                       (hipStream_t)stream, (const uint16_t*)q, (const uint16_t*)k,                \
+                       (const uint16_t*)v, (uint16_t*)out, B, Hq, Hk, Sq, Skv, scale, q_stride,    \
+                       k_stride, v_stride, (float*)po, (float*)pml)
+    // the maxima of the merged form are unscaled scores
+    float scale2 = 1.4426950408889634f;
+    if (!merged) {
+        LAUNCH_SPLIT((attn_prefill_v2<1, true, false, 128, true>), 128, B * Hq);
+    } else {
+        scale2 *= scale;
+        if (gq == 2) LAUNCH_SPLIT((attn_prefill_v3<128, 2, true>), 128, B * Hk);
+        else if (gq == 4) LAUNCH_SPLIT((attn_prefill_v3<128, 4, true>), 64, B * Hk);
+        else if (gq == 8) LAUNCH_SPLIT((attn_prefill_v3<128, 8, true>), 32, B * Hk);
+        else return -104;
+    }
+#undef LAUNCH_SPLIT
+    HIP_CHECK_LAUNCH();
+    hipLaunchKernelGGL(prefill_combine_kernel, dim3(CEIL_DIV(rows, 4)), dim3(256), 0,
+                       (hipStream_t)stream, (const float*)po, (const float*)pml, (uint32_t*)out, rows,
+                       nsplit, scale2);
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
 extern "C" int oa_attention_prefill_variant(
     void* stream, const void* q, const void* k, const void* v, void* out,
     int B, int Hq, int Hk, int Sq, int Skv, int D, float scale,
@@ -770,7 +875,14 @@ extern "C" int oa_attention_prefill_variant(
     hipLaunchKernelGGL(KERN, GRID, block, 0, (hipStream_t)stream,               \
                        (const uint16_t*)q, (const uint16_t*)k,                  \
                        (const uint16_t*)v, (uint16_t*)out, B, Hq, Hk, Sq, Skv,  \
-                       scale, q_stride, k_stride, v_stride)
+                       scale, q_stride, k_stride, v_stride, (float*)nullptr,    \
+                       (float*)nullptr)
+#define LAUNCH3(GQV, GRID)                                                      \
+    hipLaunchKernelGGL((attn_prefill_v3<128, GQV, false>), GRID, block, 0,      \
+                       (hipStream_t)stream, (const uint16_t*)q,                 \
+                       (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)out,  \
+                       B, Hq, Hk, Sq, Skv, scale, q_stride, k_stride, v_stride, \
+                       (float*)nullptr, (float*)nullptr)
     // RB=2 (256-row q-tile) instantiations were REMOVED: every form spilled
     // 25-43 VGPRs past the 256 cap and lost all A/Bs to the RB1 kernels.
     (void)grid2;
@@ -790,18 +902,15 @@ extern "C" int oa_attention_prefill_variant(
             LAUNCH((attn_prefill_v2<1, true, false, 128>), grid1);
             break;
         case 8:  // v3: swapped-QK^T 32x32 MFMAs, in-register P (256-row tile)
-            LAUNCH((attn_prefill_v3<128>), dim3(CEIL_DIV(Sq, 256), B * Hq));
+            LAUNCH3(1, dim3(CEIL_DIV(Sq, 256), B * Hq));
             break;
         case 9:  // v4: GQA-merged v3 — GQ q-heads share each staged KV tile
             if (Hq == 2 * Hk)
-                LAUNCH((attn_prefill_v3<128, 2>),
-                       dim3(CEIL_DIV(Sq, 128), B * (Hq / 2)));
+                LAUNCH3(2, dim3(CEIL_DIV(Sq, 128), B * (Hq / 2)));
             else if (Hq == 4 * Hk)
-                LAUNCH((attn_prefill_v3<128, 4>),
-                       dim3(CEIL_DIV(Sq, 64), B * (Hq / 4)));
+                LAUNCH3(4, dim3(CEIL_DIV(Sq, 64), B * (Hq / 4)));
             else if (Hq == 8 * Hk)
-                LAUNCH((attn_prefill_v3<128, 8>),
-                       dim3(CEIL_DIV(Sq, 32), B * (Hq / 8)));
+                LAUNCH3(8, dim3(CEIL_DIV(Sq, 32), B * (Hq / 8)));
             else
                 return -104;
             break;
@@ -809,6 +918,7 @@ extern "C" int oa_attention_prefill_variant(
             return -103;
     }
 #undef LAUNCH
+#undef LAUNCH3
     HIP_CHECK_LAUNCH();
     return 0;
 }
@@ -826,11 +936,15 @@ extern "C" int oa_attention_prefill(void* stream, const void* q, const void* k,
     // and wins whenever it applies (S8192 721 vs 556 vs 350 TF; S2048 439;
     // B16/S1024 426): the v3 PMC put the residual WAIT at staged-KV DMA
     // pressure, which merging divides by GQ. v3 covers non-4/8 GQA
-    // ratios; below ~256 workgroups the 128-row v2 keeps more CUs busy.
+    // ratios; while its blocks fit one round the 128-row v2 keeps more CUs busy.
     if (variant <= 0) {
         const int gq = (Hk > 0 && Hq % Hk == 0) ? Hq / Hk : 1;
         const int64_t grid256 = (int64_t)CEIL_DIV(Sq, 256) * B * Hq;
-        if ((gq == 2 || gq == 4 || gq == 8) && grid256 >= 256)
+        // a second round of 128-row blocks costs more than the merged form's idle
+        // CUs (32 heads on 8: 1500 tokens 85 us in 384 blocks, 58 merged in 192;
+        // 1024 tokens 38.5 in 256 blocks, 42.6 merged in 128)
+        const int64_t grid128 = (int64_t)CEIL_DIV(Sq, 128) * B * Hq;
+        if ((gq == 2 || gq == 4 || gq == 8) && grid128 > 256)
             variant = 9;
         else if (grid256 >= 256)
             variant = 8;

@@ -65,6 +65,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_masked_argmax_f32.restype = i
     lib.oa_attention_prefill.argtypes = [p, p, p, p, p, i, i, i, i, i, i, f, i, i, i]
     lib.oa_attention_prefill.restype = i
+    lib.oa_attention_prefill_split.argtypes = [p] * 7 + [i] * 6 + [f, i, i, i, i, i]
+    lib.oa_attention_prefill_split.restype = i
     lib.oa_attention_decode.argtypes = [p, p, p, p, p, p, p, p, p, p, i, i, i, i, i, i, i, f, i, i]
     lib.oa_attention_decode.restype = i
     lib.oa_attention_decode_rope.argtypes = [
