@@ -583,19 +583,17 @@ extern "C" int oa_gemv_gateup_fp8(void* stream, const void* x, const void* w8,
 // ---- fp8 MFMA tile GEMM (prefill path) -------------------------------------
 // C[M, N] = (A8[M, K] @ B8[N, K]^T) * a_scale[m] * b_scale[n], bf16 out.
 //
-// v2: 128x128 tile, 4 waves (2x2 of
-// 64x64), K-step 128 fp8 bytes (2x the old unroll -> half the barriers), A/B
-// staged by 16-B global_load_lds into a DOUBLE-BUFFERED ring (the guide's
-// step-3 '+67%' lever over register staging, and its verified 2-buffer
-// "glds + vmcnt(0) + __syncthreads" form). The XOR swizzle moves to the DMA
-// source address (glds writes lane-linear): byte ^= (row&7)<<4 spreads the
-// 16-lane fragment-read groups over the banks at 16-B granularity.
-// v_mfma_f32_16x16x32_fp8_fp8: A lane l holds row l&15, k (l>>4)*8..+8
-// (8 fp8 = 2 VGPRs); same C/D layout as the bf16 form (dtype-independent).
-// Tail rows (M or N not multiple of 128) CLAMP the DMA source row and the
-// epilogue masks the store — garbage products are never written.
+// 128x128 tile, 4 waves (2x2 of 64x64), K-steps of 128 fp8 bytes, A and B staged by
+// 16-byte global_load_lds. XOR swizzle on the DMA source address (the LDS write is
+// lane-linear): byte ^= (row & 7) << 4 spreads the 16-lane fragment-read groups over
+// the banks at 16-byte granularity. Tail rows (M or N not a multiple of 128) clamp the
+// DMA source row and the epilogue masks the store.
+//
+// The products are v_mfma_scale_f32_32x32x64_f8f6f4 with identity E8M0 scales (0x7f =
+// 2^0): the large-K scaled forms are the only fp8 MFMAs past the bf16 rate on gfx950;
+// with unit scales the numerics are plain fp8 products with float32 accumulation.
+// Fragment maps: A lane l & 31 = row, l >> 5 = 32-byte k-half; B the same over columns.
 
-typedef __attribute__((ext_vector_type(2))) int fp8_frag;   // 8 fp8
 typedef __attribute__((ext_vector_type(8))) int i32x8_f8;   // 32 fp8 (MX operand)
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;  // 32x32 C/D
 
@@ -607,122 +605,73 @@ __device__ __forceinline__ uint32_t g8_swz(int row, int byte_in_row) {
     return (uint32_t)(row * GK2 + (byte_in_row ^ ((row & 7) << 4)));
 }
 
-// GLDS=true: LDS-DMA staging (fastest when the operands are L3-resident).
-// GLDS=false: register staging (plain loads -> regs under the MFMAs ->
-// ds_write after the barrier, T14 form): the LDS-DMA gather path collapses
-// to ~0.9 TB/s chip-wide when the streamed operand MISSES the L3 (measured
-// 119 TF at M1024 N8192 K28672 where B alone is 235 MB), while plain loads
-// stream HBM at full rate.
-template <bool GLDS>
-__global__ __launch_bounds__(256, 1) void gemm_fp8_kernel_v2(
-    const uint32_t* __restrict__ a8,  // [M, K/4]
-    const uint32_t* __restrict__ b8,  // [N, K/4]
-    const float* __restrict__ ascale, // [M]
-    const float* __restrict__ bscale, // [N]
-    uint32_t* __restrict__ c,         // [M, N/2] bf16x2
-    int M, int N, int K) {
-    // ring layout: [buf][A|B] 16 KiB quadrants
-    __shared__ __attribute__((aligned(16))) char smem[4 * GTILE_B];
-
-    // N-tiles on x: the dispatcher places block b on XCD b%8, so an M-major
-    // x axis pins each M-tile's 224-block column to ONE XCD (measured 9x
-    // slowdown at N=28672 where B exceeds the L3); N-major spreads the
-    // B stream across XCDs and co-resident blocks share the small A tiles.
-    const int tm = blockIdx.y * GT;
-    const int tn = blockIdx.x * GT;
+// A ring of STAGES K-steps: STAGES - 1 are under way while one is in use. A wait
+// leaves the younger steps' transfers in flight (vmcnt counts them in order: eight per
+// wave and step); the barrier after it says both that step t has landed for every wave
+// and that step t - 1 is no longer read, so its buffer can be filled. The transfers are
+// inline asm because hipcc's wait inserter drains builtin ones before the first LDS
+// read. Work items go to the dies in runs, with the row tiles of a column strip next to
+// each other: a strip is read into one die's L2 once.
+//
+// What bounds it is what a CU draws from the L2, about 55 GB/s in every shape: two
+// blocks of two steps per CU reach 1.6 to 1.9 PFLOP/s, one block of four steps is the
+// faster form while there are no more blocks than CUs. us, the former kernel (two
+// buffers, row tiles far apart; register staging at K = 28672) / here: 28672 x 4096,
+// M = 77 53.7 / 39.3, 700 142 / 126, 2048 342 / 303; 4096 x 14336, 77 124 / 74, 700 127 /
+// 75, 2048 145 / 132; 6144 x 4096, 700 44 / 35; 4096 x 4096, 700 39 / 30; 8192 x 28672,
+// 700 583 / 217, 2048 1201 / 502. Reading the next half-step's fragments under the
+// products made it slower (4096 x 14336, 700: 93).
+template <int STAGES>
+__global__ __launch_bounds__(256, 1) void gemm_fp8_ring_kernel(
+    const uint32_t* __restrict__ a8, const uint32_t* __restrict__ b8,
+    const float* __restrict__ ascale, const float* __restrict__ bscale,
+    uint16_t* __restrict__ c, int M, int N, int K, int mtiles, int items) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int per = gridDim.x >> 3;
+    const int item = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (item >= items) return;
+    const int nt = item / mtiles;
+    const int tm = (item - nt * mtiles) * GT, tn = nt * GT;
     const int lane = threadIdx.x & (WAVE - 1);
-    const int wid = threadIdx.x / WAVE;
-    const int wr = wid >> 1;   // wave row 0..1 (owns 64 rows)
-    const int wc = wid & 1;    // wave col 0..1 (owns 64 cols)
-    const int fr = lane & 15;
-    const int fs = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int wr = wid >> 1, wc = wid & 1;
 
     f32x16_t accw[2][2] = {};
-
-    // staging: per K-step each operand moves 16 KiB = 1024 16-B pieces;
-    // 4 waves x 4 chunks x 64 lanes. Chunk c covers rows c*8..c*8+7
-    // (8 rows x 128 B); lane l -> row c*8 + l/8, byte (l%8)*16 ^ swz.
-    // Same asm-glds + persistent-operand discipline as attention_prefill
-    // (see the comment there: the builtin form's DMA gets drained at the
-    // first ds_read of every K-step by the wait inserter).
-    const int arow_l = lane >> 3;           // row within chunk
+    const int arow_l = lane >> 3;
     const int abyte_l = ((lane & 7) * 16) ^ ((arow_l & 7) << 4);
-    const char* abase = reinterpret_cast<const char*>(a8);
-    const char* bbase = reinterpret_cast<const char*>(b8);
-
-    uint32_t m0a[2][4], m0b[2][4];
-    if constexpr (GLDS) {
-#pragma unroll
-        for (int buf = 0; buf < 2; ++buf)
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const int ch = wid * 4 + p;  // chunk 0..15
-                m0a[buf][p] = __builtin_amdgcn_readfirstlane(
-                    (uint32_t)(uintptr_t)smem + buf * 2 * GTILE_B + ch * 1024);
-                m0b[buf][p] = __builtin_amdgcn_readfirstlane(
-                    (uint32_t)(uintptr_t)smem + buf * 2 * GTILE_B + GTILE_B +
-                    ch * 1024);
-            }
-    }
     const char* asrc[4];
     const char* bsrc[4];
-    uint32_t m0a_cur[4], m0b_cur[4];
-    auto set_step = [&](int k0, int buf) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const int ch = wid * 4 + p;
+        asrc[p] = reinterpret_cast<const char*>(a8) + (size_t)min(tm + ch * 8 + arow_l, M - 1) * K + abyte_l;
+        bsrc[p] = reinterpret_cast<const char*>(b8) + (size_t)min(tn + ch * 8 + arow_l, N - 1) * K + abyte_l;
+    }
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + wid * 4096);
+    auto stage = [&](int buf) {
+        const uint32_t at = lds0 + buf * 2 * GTILE_B;
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-            const int ch = wid * 4 + p;
-            const int ar = min(tm + ch * 8 + arow_l, M - 1);
-            const int br = min(tn + ch * 8 + arow_l, N - 1);
-            asrc[p] = abase + (size_t)ar * (K) + k0 + abyte_l;
-            bsrc[p] = bbase + (size_t)br * (K) + k0 + abyte_l;
-            m0a_cur[p] = m0a[buf][p];
-            m0b_cur[p] = m0b[buf][p];
+            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off"
+                         : : "s"(at + p * 1024), "v"(asrc[p]) : "memory");
+            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off"
+                         : : "s"(at + GTILE_B + p * 1024), "v"(bsrc[p]) : "memory");
         }
-    };
-    auto stage = [&]() {
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-            asm volatile(
-                "s_mov_b32 m0, %0\n\t"
-                "global_load_lds_dwordx4 %1, off"
-                :
-                : "s"(m0a_cur[p]), "v"(asrc[p]));
-            asm volatile(
-                "s_mov_b32 m0, %0\n\t"
-                "global_load_lds_dwordx4 %1, off"
-                :
-                : "s"(m0b_cur[p]), "v"(bsrc[p]));
+            asrc[p] += GK2;
+            bsrc[p] += GK2;
         }
     };
-    auto drain = [&]() {
-        asm volatile("s_waitcnt vmcnt(0)"
-                     :
-                     : "v"(asrc[0]), "v"(asrc[1]), "v"(asrc[2]), "v"(asrc[3]),
-                       "v"(bsrc[0]), "v"(bsrc[1]), "v"(bsrc[2]), "v"(bsrc[3]),
-                       "s"(m0a_cur[0]), "s"(m0a_cur[1]), "s"(m0a_cur[2]),
-                       "s"(m0a_cur[3]), "s"(m0b_cur[0]), "s"(m0b_cur[1]),
-                       "s"(m0b_cur[2]), "s"(m0b_cur[3])
-                     : "memory");
-    };
-
-    // Inner product on v_mfma_scale_f32_32x32x64_f8f6f4 with IDENTITY E8M0
-    // scales (0x7f = 2^0): the large-K scaled forms are the ONLY fp8 MFMAs
-    // past the bf16 rate on gfx950 (~4.6 PF vs ~2.1 PF for 16x16x32 fp8 —
-    // guide §3); with unit scales the numerics are exactly the plain-fp8
-    // kernel's (fp8 products, f32 accumulation; per-row float scales stay
-    // in the epilogue). Fragment maps: A lane l&31 = row, (l>>5) = 32-byte
-    // k-half; B symmetric over columns; C/D is the standard 32x32 map.
     auto compute = [&](const char* abuf, const char* bbuf) {
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {          // two K=64 steps per tile
-            const int kb = kk * 64 + (lane >> 5) * 32;  // this lane's 32 B
+        for (int kk = 0; kk < 2; ++kk) {
+            const int kb = kk * 64 + (lane >> 5) * 32;
             i32x8_f8 afrag[2], bfrag[2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int arow = wr * 64 + i * 32 + (lane & 31);
                 const int brow = wc * 64 + i * 32 + (lane & 31);
-                // 32 contiguous k-bytes under the 16-B-granular XOR swizzle
-                // = two independent 16-B reads
                 *reinterpret_cast<uint4*>(&afrag[i]) =
                     *reinterpret_cast<const uint4*>(abuf + g8_swz(arow, kb));
                 *(reinterpret_cast<uint4*>(&afrag[i]) + 1) =
@@ -737,116 +686,69 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_kernel_v2(
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
                     accw[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                        afrag[i], bfrag[j], accw[i][j],
-                        0 /*cbsz: fp8*/, 0 /*blgp: fp8*/,
-                        0, 0x7f, 0, 0x7f);
+                        afrag[i], bfrag[j], accw[i][j], 0, 0, 0, 0x7f, 0, 0x7f);
         }
     };
-
-    // register-staging state (GLDS=false): one set, T14 write-after-barrier
-    uint4 areg[4], breg[4];
-    auto load_step = [&](int k0) {
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const int ch = wid * 4 + p;
-            const int ar = min(tm + ch * 8 + arow_l, M - 1);
-            const int br = min(tn + ch * 8 + arow_l, N - 1);
-            areg[p] = *reinterpret_cast<const uint4*>(
-                abase + (size_t)ar * K + k0 + abyte_l);
-            breg[p] = *reinterpret_cast<const uint4*>(
-                bbase + (size_t)br * K + k0 + abyte_l);
-        }
-    };
-    auto write_step = [&](int buf) {
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const int ch = wid * 4 + p;
-            char* dst = smem + buf * 2 * GTILE_B + ch * 1024 + lane * 16;
-            *reinterpret_cast<uint4*>(dst) = areg[p];
-            *reinterpret_cast<uint4*>(dst + GTILE_B) = breg[p];
-        }
-    };
-
     const int nsteps = K / GK2;
-    if constexpr (GLDS) {
-        set_step(0, 0);
-        stage();
-        drain();
-        __syncthreads();
-        for (int t = 0; t < nsteps; ++t) {
-            const int cur = t & 1;
-            if (t + 1 < nsteps) {
-                set_step((t + 1) * GK2, cur ^ 1);
-                stage();
-            }
-            compute(smem + cur * 2 * GTILE_B, smem + cur * 2 * GTILE_B + GTILE_B);
-            drain();
-            __syncthreads();
-        }
-    } else {
-        load_step(0);
-        write_step(0);
-        __syncthreads();
-        for (int t = 0; t < nsteps; ++t) {
-            const int cur = t & 1;
-            if (t + 1 < nsteps) load_step((t + 1) * GK2);  // HBM hides under MFMAs
-            compute(smem + cur * 2 * GTILE_B, smem + cur * 2 * GTILE_B + GTILE_B);
-            if (t + 1 < nsteps) write_step(cur ^ 1);       // other buffer: no wait on readers
-            __syncthreads();
-        }
+#pragma unroll
+    for (int t = 0; t < STAGES - 1; ++t)
+        if (t < nsteps) stage(t);
+    int buf = 0;
+    for (int t = 0; t < nsteps; ++t) {
+        // steps behind t that are under way: up to STAGES - 2
+        const int behind = min(STAGES - 2, nsteps - 1 - t);
+        if (behind >= 2) asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)\n\ts_barrier" : : : "memory");
+        else if (behind == 1) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" : : : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
+        if (t + STAGES - 1 < nsteps) stage(buf == 0 ? STAGES - 1 : buf - 1);
+        compute(smem + buf * 2 * GTILE_B, smem + buf * 2 * GTILE_B + GTILE_B);
+        buf = buf + 1 == STAGES ? 0 : buf + 1;
     }
 
-    // epilogue: C[row][col] = acc * ascale[row] * bscale[col]
-    // 32x32 C/D map: col = lane&31, row = (r&3) + 8*(r>>2) + 4*(lane>>5)
+    // 32x32 C/D map: col = lane & 31, row = (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5).
+    // Row scales are read together (rows past the end repeat the last), not one by one
+    // behind a branch each.
+    float as[2][16], bs[2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int r = 0; r < 16; ++r)
+            as[i][r] = ascale[min(tm + wr * 64 + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5), M - 1)];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) bs[j] = bscale[min(tn + wc * 64 + j * 32 + (lane & 31), N - 1)];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int col = tn + wc * 64 + j * 32 + (lane & 31);
+        if (col >= N) continue;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int row = tm + wr * 64 + i * 32 + (r & 3) + 8 * (r >> 2) +
-                                4 * (lane >> 5);
-                const int col = tn + wc * 64 + j * 32 + (lane & 31);
-                if (row < M && col < N) {
-                    const float v = accw[i][j][r] * ascale[row] * bscale[col];
-                    reinterpret_cast<uint16_t*>(c)[(size_t)row * N + col] = f32_to_bf16(v);
-                }
+                const int row = tm + wr * 64 + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
+                if (row < M) c[(size_t)row * N + col] = f32_to_bf16(accw[i][j][r] * as[i][r] * bs[j]);
             }
-        }
     }
 }
 
 extern "C" int oa_gemm_fp8(void* stream, const void* a8, const void* b8,
                            const void* ascale, const void* bscale, void* c,
                            int M, int N, int K) {
-    if (K % GK2 != 0) return -100;
-    dim3 grid(CEIL_DIV(N, GT), CEIL_DIV(M, GT)), block(256);
-    // Staging choice (3-run A/B on MI355X): glds staging wins at every
-    // shape (1083-1551 TF vs registers' 541-764) EXCEPT deep-K (K=28672:
-    // reproducible 119-129 TF collapse of the DMA gather — both operands
-    // at 28 KiB row stride with the B panel re-read per M-tile; register
-    // staging holds 735-764 TF there). A separate SPORADIC ~4.2 ms mode
-    // was observed hitting hipBLASLt itself on the same boxes — box
-    // throttling, not kernel-attributable. OPSAGENT_FP8_STAGE=glds|reg
-    // forces a path (A/B).
-    const char* fs_env = getenv("OPSAGENT_FP8_STAGE");
-    bool use_glds = K <= 16384;
-    if (fs_env && fs_env[0] == 'g') use_glds = true;
-    if (fs_env && fs_env[0] == 'r') use_glds = false;
-    if (use_glds)
-        hipLaunchKernelGGL((gemm_fp8_kernel_v2<true>), grid, block, 0,
-                           (hipStream_t)stream, (const uint32_t*)a8,
-                           (const uint32_t*)b8, (const float*)ascale,
-                           (const float*)bscale, (uint32_t*)c, M, N, K);
-    else
-        hipLaunchKernelGGL((gemm_fp8_kernel_v2<false>), grid, block, 0,
-                           (hipStream_t)stream, (const uint32_t*)a8,
-                           (const uint32_t*)b8, (const float*)ascale,
-                           (const float*)bscale, (uint32_t*)c, M, N, K);
+    if (K % GK2 != 0 || M < 1 || N < 1) return -100;
+    const int mt = CEIL_DIV(M, GT);
+    const int64_t items = (int64_t)CEIL_DIV(N, GT) * mt;
+    if (items > (1 << 28)) return -101;
+    const dim3 grid((unsigned)(CEIL_DIV(items, 8) * 8)), block(256);
+#define RING(STAGES)                                                                              \
+    hipLaunchKernelGGL((gemm_fp8_ring_kernel<STAGES>), grid, block, (STAGES) * 2 * GTILE_B,       \
+                       (hipStream_t)stream, (const uint32_t*)a8, (const uint32_t*)b8,             \
+                       (const float*)ascale, (const float*)bscale, (uint16_t*)c, M, N, K, mt,     \
+                       (int)items)
+    if (items <= 256) RING(4);
+    else RING(2);
+#undef RING
     HIP_CHECK_LAUNCH();
     return 0;
 }
-
 
 // ---- MFMA fp8 GEMV v2 (decode path) ----------------------------------------
 // The VALU dequant stream tops out at ~4.5-4.7 TB/s (~40 VALU ops per 16 W
