@@ -213,10 +213,9 @@ class DenseMLP(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.fp8:
-            act = ops.gateup_silu_fp8(
-                x, self.gate_up_q, self.gate_up_s, self.i_local
-            )
-            return tp_all_reduce(ops.linear_fp8(act, self.down_q, self.down_s))
+            return tp_all_reduce(ops.mlp_fp8(
+                x, self.gate_up_q, self.gate_up_s, self.i_local, self.down_q, self.down_s
+            ))
         act = ops.gateup_silu(x, self.gate_up_w, self.i_local)
         return tp_all_reduce(ops.linear(act, self.down_w))
 

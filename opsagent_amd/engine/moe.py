@@ -143,13 +143,11 @@ class MoEMLP(nn.Module):
             xe = x[toks].contiguous()
             if self.fp8:
                 gu = ops.linear_fp8(xe, self.w13_q[e], self.w13_s[e])
-                gate, up = gu.split([self.i_local, self.i_local], dim=-1)
-                act = ops.silu_mul(gate.contiguous(), up.contiguous())
+                act = ops.silu_halves(gu, self.i_local)
                 ye = ops.linear_fp8(act.contiguous(), self.w2_q[e], self.w2_s[e])
             else:
                 gu = ops.linear(xe, self.w13[e])
-                gate, up = gu.split([self.i_local, self.i_local], dim=-1)
-                act = ops.silu_mul(gate.contiguous(), up.contiguous())
+                act = ops.silu_halves(gu, self.i_local)
                 ye = ops.linear(act, self.w2[e])
             out.index_add_(0, toks, ye * wts)
         if self.shared is not None:

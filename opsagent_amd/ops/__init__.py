@@ -233,6 +233,22 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def silu_halves(gu: torch.Tensor, i_local: int) -> torch.Tensor:
+    """silu(gu[..., :I]) * gu[..., I:]; on the GPU the halves are read in place where
+    their rows keep 16-byte alignment."""
+    if (
+        _is_gpu(gu) and gu.dtype == torch.bfloat16 and gu.is_contiguous() and gu.numel()
+        and i_local % 8 == 0 and gu.shape[-1] == 2 * i_local and gu.data_ptr() % 16 == 0
+    ):
+        lib, hip = _lib()
+        out = torch.empty(*gu.shape[:-1], i_local, dtype=gu.dtype, device=gu.device)
+        hip.check(lib.oa_silu_halves(hip.current_stream_ptr(), gu.data_ptr(), out.data_ptr(),
+                                     out.numel() // i_local, i_local), "oa_silu_halves")
+        return out
+    gate, up = gu.split([i_local, i_local], dim=-1)
+    return silu_mul(gate.contiguous(), up.contiguous())
+
+
 def quant_fp8(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """Per-row OCP e4m3 quantization: bf16 [T, K] -> (uint8 [T, K], f32 [T])."""
     T = x.numel() // x.shape[-1]
@@ -293,14 +309,44 @@ def linear_fp8(
             for m0 in range(0, M, 8)
         ]
         return torch.cat(parts, dim=0).reshape(*x.shape[:-1], N)
-    out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
     a8, a_scale = quant_fp8(x.reshape(M, K))
+    return _gemm_fp8(a8, a_scale, w8, w_scale).view(*x.shape[:-1], N)
+
+
+def _gemm_fp8(a8: torch.Tensor, a_scale: torch.Tensor, w8: torch.Tensor,
+              w_scale: torch.Tensor) -> torch.Tensor:
+    """The fp8 tile product of quantized rows a8 [M, K] (K % 128 == 0), bf16 [M, N]."""
+    (M, K), N = a8.shape, w8.shape[0]
+    lib, hip = _lib()
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=a8.device)
     rc = lib.oa_gemm_fp8(
         hip.current_stream_ptr(), a8.data_ptr(), w8.data_ptr(),
         a_scale.data_ptr(), w_scale.data_ptr(), out.data_ptr(), M, N, K,
     )
     hip.check(rc, "oa_gemm_fp8")
     return out
+
+
+def mlp_fp8(
+    x: torch.Tensor, gate_up_q: torch.Tensor, gate_up_s: torch.Tensor, i_local: int,
+    down_q: torch.Tensor, down_s: torch.Tensor,
+) -> torch.Tensor:
+    """(silu(x @ gate8^T) * (x @ up8^T)) @ down8^T. Where both products are tile
+    products (prefill rows), the activation is quantized as it is made: the same bf16
+    values, rows and scales as quantizing it afterwards."""
+    M, K = x.numel() // x.shape[-1], x.shape[-1]
+    if not (
+        _is_gpu(x) and M > 8 and K % 128 == 0 and i_local % 128 == 0
+        and not _fp8_mfma_ok(M, K) and not _fp8_mfma_ok(M, i_local)
+    ):
+        return linear_fp8(gateup_silu_fp8(x, gate_up_q, gate_up_s, i_local), down_q, down_s)
+    gu = linear_fp8(x, gate_up_q, gate_up_s)
+    lib, hip = _lib()
+    a8 = torch.empty(M, i_local, dtype=torch.uint8, device=x.device)
+    a_scale = torch.empty(M, dtype=torch.float32, device=x.device)
+    hip.check(lib.oa_silu_quant_fp8(hip.current_stream_ptr(), gu.data_ptr(), a8.data_ptr(),
+                                    a_scale.data_ptr(), M, i_local), "oa_silu_quant_fp8")
+    return _gemm_fp8(a8, a_scale, down_q, down_s).view(*x.shape[:-1], down_q.shape[0])
 
 
 def linear_norm(
@@ -631,9 +677,7 @@ def gateup_silu(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> torch
     says so. Otherwise: library GEMM + the silu_mul kernel."""
     if gateup_fused(x, gate_up_w, i_local):
         return gateup_act(x, gate_up_w, i_local)
-    gu = linear(x, gate_up_w)
-    gate, up = gu.split([i_local, i_local], dim=-1)
-    return silu_mul(gate.contiguous(), up.contiguous())
+    return silu_halves(linear(x, gate_up_w), i_local)
 
 
 def gateup_fused(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> bool:
@@ -907,9 +951,7 @@ def gateup_silu_fp8(
         _Mgu in (5, 7) and not _fp8_mfma_ok(_Mgu, x.shape[-1], gateup=True)
     ):
         xin = rms_norm(x, norm_w, eps) if use_norm else x
-        gu = linear_fp8(xin, w8, w_scale)
-        g, u = gu.split([i_local, i_local], dim=-1)
-        return silu_mul(g.contiguous(), u.contiguous())
+        return silu_halves(linear_fp8(xin, w8, w_scale), i_local)
     lib, hip = _lib()
     M = x.numel() // x.shape[-1]
     if use_norm and M == 1:  # see linear_norm_fp8: prenorm beats in-loop norm

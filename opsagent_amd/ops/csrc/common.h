@@ -52,6 +52,13 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     return (uint32_t)f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);
 }
 
+// silu(g) * u of two bf16 pairs, float32 inside
+__device__ __forceinline__ uint32_t silu_mul_bf16x2(uint32_t g, uint32_t u) {
+    const float lo = bf16_lo(g), hi = bf16_hi(g);
+    return pack_bf16x2(lo / (1.0f + __expf(-lo)) * bf16_lo(u),
+                       hi / (1.0f + __expf(-hi)) * bf16_hi(u));
+}
+
 // ---- wave reductions --------------------------------------------------------
 __device__ __forceinline__ float wave_reduce_sum(float v) {
 #pragma unroll

@@ -14,11 +14,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(
         uint4 o;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            uint32_t gw = (&g.x)[j], uw = (&u.x)[j];
-            float glo = bf16_lo(gw), ghi = bf16_hi(gw);
-            float lo = glo / (1.0f + __expf(-glo)) * bf16_lo(uw);
-            float hi = ghi / (1.0f + __expf(-ghi)) * bf16_hi(uw);
-            (&o.x)[j] = pack_bf16x2(lo, hi);
+            (&o.x)[j] = silu_mul_bf16x2((&g.x)[j], (&u.x)[j]);
         }
         *reinterpret_cast<uint4*>(out + i) = o;
     }
@@ -32,6 +28,34 @@ extern "C" int oa_silu_mul(void* stream, const void* gate, const void* up,
     hipLaunchKernelGGL(silu_mul_kernel, dim3(grid), dim3(256), 0,
                        (hipStream_t)stream, (const uint32_t*)gate,
                        (const uint32_t*)up, (uint32_t*)out, n2);
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
+// silu(gu[m, :I]) * gu[m, I:] of rows [M, 2 I], I % 8 == 0: the halves are read where
+// the product left them. Bound by memory (176 MB at [2048, 2 x 14336]); without the two
+// copies that the flat kernel above needs, a layer takes 45 us less at 2048 rows (78 us
+// for the three launches before), 10 less at 77 and 5 less at 47.
+__global__ __launch_bounds__(256) void silu_halves_kernel(
+    const uint4* __restrict__ gu, uint4* __restrict__ out, int64_t M, int iv /* I / 8 */) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= iv) return;
+    for (int64_t m = blockIdx.y; m < M; m += gridDim.y) {
+        const uint4 g = gu[m * 2 * iv + c], u = gu[m * 2 * iv + iv + c];
+        uint4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) (&o.x)[j] = silu_mul_bf16x2((&g.x)[j], (&u.x)[j]);
+        out[m * iv + c] = o;
+    }
+}
+
+extern "C" int oa_silu_halves(void* stream, const void* gu, void* out, int64_t M, int I) {
+    if (I % 8 != 0 || I < 8) return -100;
+    if (((uintptr_t)gu | (uintptr_t)out) % 16 != 0) return -101;
+    if (M <= 0) return 0;
+    const int iv = I / 8;
+    hipLaunchKernelGGL(silu_halves_kernel, dim3(CEIL_DIV(iv, 256), (unsigned)min(M, (int64_t)65535)),
+                       dim3(256), 0, (hipStream_t)stream, (const uint4*)gu, (uint4*)out, M, iv);
     HIP_CHECK_LAUNCH();
     return 0;
 }

@@ -39,6 +39,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_rope.restype = i
     lib.oa_silu_mul.argtypes = [p, p, p, p, i64]
     lib.oa_silu_mul.restype = i
+    lib.oa_silu_halves.argtypes = [p, p, p, i64, i]
+    lib.oa_silu_halves.restype = i
     lib.oa_kv_write.argtypes = [p, p, p, p, p, p, i, i, i]
     lib.oa_kv_write.restype = i
     lib.oa_rope_kv.argtypes = [p, p, p, p, p, p, p, p, p, p, i, i, i, i, i, i, i]
@@ -76,6 +78,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_attention_decode_rope.restype = i
     lib.oa_quant_fp8.argtypes = [p, p, p, p, i, i]
     lib.oa_quant_fp8.restype = i
+    lib.oa_silu_quant_fp8.argtypes = [p, p, p, p, i, i]
+    lib.oa_silu_quant_fp8.restype = i
     lib.oa_gemv_fp8.argtypes = [p, p, p, p, p, i, i, i]
     lib.oa_gemv_fp8.restype = i
     lib.oa_gemv_fp8_ex.argtypes = [p, p, p, p, p, p, p, i, i, i, f, i]
