@@ -437,13 +437,12 @@ def _moe_act(act):
 
 
 def moe_route_ok(x: torch.Tensor, router_w: torch.Tensor, top: int) -> bool:
-    """Whether moe_route takes this router: a row of activations and logits in
-    LDS, eight-channel rows for moe_combine."""
+    """Whether moe_route takes this router: eight-channel rows for moe_combine."""
     E, K = router_w.shape
     return (
         x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
         and router_w.dtype == torch.float32 and router_w.is_contiguous()
-        and K % 8 == 0 and E <= 1024 and top <= min(E, 64) and (K + E) * 4 <= 65536
+        and K % 8 == 0 and E <= 1024 and top <= min(E, 64)
         and x.data_ptr() % 16 == 0 and router_w.data_ptr() % 16 == 0
     )
 
@@ -457,9 +456,10 @@ def moe_route(x: torch.Tensor, router_w: torch.Tensor, top: int):
     lib, hip = _lib()
     idx, tok = torch.empty(2, T, top, dtype=torch.int32, device=x.device)
     wts = torch.empty(T, top, dtype=torch.float32, device=x.device)
+    scratch = torch.empty(lib.oa_moe_route_scratch(T, E, K), dtype=torch.float32, device=x.device)
     hip.check(lib.oa_moe_route(hip.current_stream_ptr(), x.data_ptr(), router_w.data_ptr(),
-                               idx.data_ptr(), wts.data_ptr(), tok.data_ptr(), T, E, K, top),
-              "oa_moe_route")
+                               scratch.data_ptr(), idx.data_ptr(), wts.data_ptr(), tok.data_ptr(),
+                               T, E, K, top), "oa_moe_route")
     return idx, wts, tok
 
 

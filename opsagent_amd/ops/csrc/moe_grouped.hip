@@ -30,68 +30,109 @@ typedef __attribute__((ext_vector_type(4))) float mgf4;
 #define MG_MAX_E 1024
 
 // ---- routing ----------------------------------------------------------------
-// Router logits (float32 weights and sums on bf16 rows), softmax and the `top`
-// best experts of TT tokens per block, weights normalised over the chosen: one
-// launch instead of a cast, a float32 library product, softmax, top-k (two
-// launches), sum, division and casts (61 us for 13 tokens and 64 experts of 2048
-// columns, about 5 us each). 11.3 us there, 6.6 us for 16 experts: bound by what
-// one CU draws (the matrix of 64 experts is 512 KiB, 47 GB/s). Logits spread over
-// blocks and chosen in a second launch measured 13.1 us. A wave takes an expert's
-// row in 1 KiB pieces and keeps TT sums; ties go to the lower expert.
-template <int TT>
-__global__ __launch_bounds__(1024) void moe_route_kernel(const uint16_t* __restrict__ x,
+// Router logits: float32 weights, products and sums on bf16 rows, on
+// v_mfma_f32_16x16x4_f32. A block takes 16 experts, 16 tokens and one of `splits` parts
+// of the columns, its four waves 16-column steps in turn, four steps' loads at a time;
+// parts [splits, T, E] are added up in order by the choice below. Short loops on
+// purpose: a step's other kernels leave neither the matrix nor this code in cache, and
+// straight-line code that runs once waits for its own fetch. Us inside a step, both
+// launches, 13 tokens x 64 experts x 2048: 9.9, 512 tokens 11.0 (22.2); before, logits and choice in one
+// launch with a token per block, which drew the whole matrix through every block's CU:
+// 20.9 (11.3 with it in cache), as unrolled vector code over the blocks 16.3.
+__global__ __launch_bounds__(256) void moe_logits_kernel(const uint16_t* __restrict__ x,
                                                          const float* __restrict__ rw,
+                                                         float* __restrict__ part, int T, int E,
+                                                         int K) {
+    __shared__ mgf4 red[4][64];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
+    const int t0 = blockIdx.x * 16, e0 = blockIdx.y * 16;
+    const float* wr = rw + (size_t)min(e0 + r, E - 1) * K;
+    const uint16_t* xr = x + (size_t)min(t0 + r, T - 1) * K;
+    const int stride = gridDim.z * 64;  // columns between two steps of a wave
+    mgf4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+    for (int k0 = (blockIdx.z * 4 + wid) * 16 + q * 4; k0 < K; k0 += 4 * stride) {
+        mgf4 w[4];
+        uint2 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {   // K % 4 == 0: a lane's four columns are all in or out
+            const int k = min(k0 + i * stride, K - 4);
+            w[i] = *reinterpret_cast<const mgf4*>(wr + k);
+            v[i] = *reinterpret_cast<const uint2*>(xr + k);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool in = k0 + i * stride < K;
+            const mgf4 f = {bf16_lo(v[i].x), bf16_hi(v[i].x), bf16_lo(v[i].y), bf16_hi(v[i].y)};
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? w[i][j] : 0.0f, in ? f[j] : 0.0f,
+                                                           acc, 0, 0, 0);
+        }
+    }
+    red[wid][lane] = acc;
+    __syncthreads();
+    if (wid) return;
+    acc = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+    // D: column (token) lane & 15, rows (experts) (lane >> 4) * 4 and up
+    if (t0 + r < T)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (e0 + q * 4 + j < E)
+                part[((size_t)blockIdx.z * T + t0 + r) * E + e0 + q * 4 + j] = acc[j];
+}
+
+// a op (a of the lane that DPP names); lanes without a source keep their value
+template <int CTRL, typename F>
+__device__ __forceinline__ int mg_dpp(int a, F op) {
+    return op(a, __builtin_amdgcn_update_dpp(a, a, CTRL, 0xf, 0xf, false));
+}
+// over the wave by row shifts and row broadcasts: idempotent ops only
+template <typename F>
+__device__ __forceinline__ int mg_wave_all(int a, F op) {
+    a = mg_dpp<0x111>(a, op);
+    a = mg_dpp<0x112>(a, op);
+    a = mg_dpp<0x114>(a, op);
+    a = mg_dpp<0x118>(a, op);
+    a = mg_dpp<0x142>(a, op);
+    a = mg_dpp<0x143>(a, op);
+    return __builtin_amdgcn_readlane(a, 63);
+}
+__device__ __forceinline__ float mg_wave_max(float v) {
+    return __int_as_float(mg_wave_all(__float_as_int(v), [](int a, int b) {
+        return __float_as_int(fmaxf(__int_as_float(a), __int_as_float(b)));
+    }));
+}
+
+// Softmax and the `top` best experts, a wave per token; weights normalised over the
+// chosen, ties go to the lower expert.
+__global__ __launch_bounds__(256) void moe_choose_kernel(const float* __restrict__ part,
                                                          int* __restrict__ idx,
                                                          float* __restrict__ wout,
-                                                         int* __restrict__ tok, int T, int E, int K,
-                                                         int top) {
-    extern __shared__ __attribute__((aligned(16))) float rl[];
-    float* xs = rl;                     // [TT][K]
-    float* lg = rl + TT * K;            // [TT][E]
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int t0 = blockIdx.x * TT;
-    for (int i = tid; i < TT * (K / 4); i += 1024) {
-        const int t = i / (K / 4), c = i - t * (K / 4);
-        const uint2 v = *reinterpret_cast<const uint2*>(x + (size_t)min(t0 + t, T - 1) * K + c * 4);
-        *reinterpret_cast<float4*>(xs + t * K + c * 4) =
-            make_float4(bf16_lo(v.x), bf16_hi(v.x), bf16_lo(v.y), bf16_hi(v.y));
-    }
-    __syncthreads();
-    for (int e = wid; e < E; e += 16) {
-        const float* wr = rw + (size_t)e * K;
-        float a[TT];
-#pragma unroll
-        for (int t = 0; t < TT; ++t) a[t] = 0.0f;
-        for (int k = lane * 4; k < K; k += 256) {
-            const float4 w = *reinterpret_cast<const float4*>(wr + k);
-#pragma unroll
-            for (int t = 0; t < TT; ++t) {
-                const float4 v = *reinterpret_cast<const float4*>(xs + t * K + k);
-                a[t] = fmaf(w.x, v.x, a[t]);
-                a[t] = fmaf(w.y, v.y, a[t]);
-                a[t] = fmaf(w.z, v.z, a[t]);
-                a[t] = fmaf(w.w, v.w, a[t]);
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < TT; ++t) {
-            a[t] = wave_reduce_sum(a[t]);
-            if (lane == 0) lg[t * E + e] = a[t];
-        }
-    }
-    __syncthreads();
-    if (wid >= TT || t0 + wid >= T) return;
-    float* z = lg + wid * E;            // one wave per token from here on
-    const size_t o = (size_t)(t0 + wid) * top;
+                                                         int* __restrict__ tok, int T, int E,
+                                                         int top, int splits) {
+    __shared__ float zs[4][MG_MAX_E];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int t = blockIdx.x * 4 + wid;
+    if (t >= T) return;
+    float* z = zs[wid];                 // a lane touches its own columns only
+    const size_t o = (size_t)t * top;
     float mx = -INFINITY;
-    for (int e = lane; e < E; e += 64) mx = fmaxf(mx, z[e]);
-    mx = wave_reduce_max(mx);
+    for (int e = lane; e < E; e += 64) {
+        float a = 0.0f;
+#pragma unroll 8
+        for (int s = 0; s < splits; ++s) a += part[((size_t)s * T + t) * E + e];
+        z[e] = a;
+        mx = fmaxf(mx, a);
+    }
+    mx = mg_wave_max(mx);
     float sum = 0.0f;
-    for (int e = lane; e < E; e += 64) sum += expf(z[e] - mx);
+    for (int e = lane; e < E; e += 64) sum += z[e] = expf(z[e] - mx);
     sum = wave_reduce_sum(sum);
-    for (int e = lane; e < E; e += 64) z[e] = expf(z[e] - mx) / sum;
+    for (int e = lane; e < E; e += 64) z[e] = z[e] / sum;
     float mine = 0.0f, total = 0.0f;    // lane r keeps the r-th choice's score
     int who = 0;
+#pragma unroll 1
     for (int r = 0; r < top; ++r) {
         float bv = -INFINITY;
         int bi = 0x7fffffff;
@@ -100,15 +141,9 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const uint16_t* __restr
                 bv = z[e];
                 bi = e;
             }
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) {
-            const float ov = __shfl_xor(bv, d, 64);
-            const int oi = __shfl_xor(bi, d, 64);
-            if (ov > bv || (ov == bv && oi < bi)) {
-                bv = ov;
-                bi = oi;
-            }
-        }
+        const float best = mg_wave_max(bv);
+        bi = mg_wave_all(bv == best ? bi : 0x7fffffff, [](int a, int b) { return min(a, b); });
+        bv = best;
         if (bi == 0x7fffffff) {         // no score left that compares (NaN logits)
             bi = 0;
             bv = 0.0f;
@@ -123,7 +158,7 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const uint16_t* __restr
     if (lane < top) {
         idx[o + lane] = who;
         wout[o + lane] = mine / (total + 1e-20f);
-        tok[o + lane] = t0 + wid;
+        tok[o + lane] = t;
     }
 }
 
@@ -417,21 +452,28 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const uint16_t* __rest
     }
 }
 
+// Parts of the columns: enough blocks for the chip, no fewer than four steps a wave.
+static int moe_route_splits(int T, int E, int K) {
+    const int64_t tiles = (int64_t)CEIL_DIV(T, 16) * CEIL_DIV(E, 16);
+    return (int)max((int64_t)1, min(min((int64_t)16, 1024 / tiles), (int64_t)CEIL_DIV(K, 256)));
+}
+
+// floats of oa_moe_route's scratch
+extern "C" int64_t oa_moe_route_scratch(int T, int E, int K) {
+    return (int64_t)moe_route_splits(T, E, K) * T * E;
+}
+
 // idx, w, tok [T, top]: expert, weight and token of every pair
-extern "C" int oa_moe_route(void* stream, const void* x, const void* rw, void* idx, void* w, void* tok,
-                            int T, int E, int K, int top) {
+extern "C" int oa_moe_route(void* stream, const void* x, const void* rw, void* scratch, void* idx,
+                            void* w, void* tok, int T, int E, int K, int top) {
     if (T < 1 || E < 1 || E > MG_MAX_E || top < 1 || top > E || top > 64 || K < 4 || K % 4 != 0)
         return -100;
-    // four tokens per block once the blocks fill the chip, LDS allowing
-    const bool four = T >= 1024 && (size_t)4 * (K + E) * 4 <= 65536;
-    const size_t lds = (size_t)(four ? 4 : 1) * (K + E) * 4;
-    if (lds > 65536) return -101;
-    if (four)
-        hipLaunchKernelGGL(moe_route_kernel<4>, dim3(CEIL_DIV(T, 4)), dim3(1024), lds, (hipStream_t)stream,
-                           (const uint16_t*)x, (const float*)rw, (int*)idx, (float*)w, (int*)tok, T, E, K, top);
-    else
-        hipLaunchKernelGGL(moe_route_kernel<1>, dim3(T), dim3(1024), lds, (hipStream_t)stream,
-                           (const uint16_t*)x, (const float*)rw, (int*)idx, (float*)w, (int*)tok, T, E, K, top);
+    const int splits = moe_route_splits(T, E, K);
+    hipLaunchKernelGGL(moe_logits_kernel, dim3(CEIL_DIV(T, 16), CEIL_DIV(E, 16), splits), dim3(256),
+                       0, (hipStream_t)stream, (const uint16_t*)x, (const float*)rw,
+                       (float*)scratch, T, E, K);
+    hipLaunchKernelGGL(moe_choose_kernel, dim3(CEIL_DIV(T, 4)), dim3(256), 0, (hipStream_t)stream,
+                       (const float*)scratch, (int*)idx, (float*)w, (int*)tok, T, E, top, splits);
     HIP_CHECK_LAUNCH();
     return 0;
 }

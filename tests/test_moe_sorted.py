@@ -32,7 +32,9 @@ def _reference(x, w13, w2, idx, wts, act, more):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,E,top,K", [(1, 16, 4, 2048), (13, 64, 6, 2048), (3, 5, 5, 200),
-                                       (65, 130, 8, 1000), (1025, 64, 6, 2048), (1027, 8, 1, 8192)])
+                                       (65, 130, 8, 1000), (1025, 64, 6, 2048), (1027, 8, 1, 8192),
+                                       (4, 3, 1, 8), (17, 257, 6, 1032), (128, 64, 6, 2048),
+                                       (129, 66, 6, 2048), (2, 1024, 6, 16512)])
 def test_route(T, E, top, K):
     """Against float64: weights to float32 rounding of K products (the chosen
     scores lie in 0..1, so 1e-5 holds at K = 8192 with logits of a few units),
