@@ -115,13 +115,71 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, form: int, gateup: bool = False,
     return out
 
 
+def _ring_plan(M: int, N: int, K: int, gateup: bool = False) -> Optional[Tuple[int, int]]:
+    """(rows of a tile, column splits) of the product on the transfer ring
+    (ring_gemm.hip; figures there) of M rows of K columns against N (gate-up: 2N)
+    weight rows, None where the other forms are faster.
+
+    The lines, measured at 2 to 128 rows over 12 weights, 2 GB of them in turn (us,
+    other / ring): light weights end before the ring pays for its start (4096 x 4096,
+    M = 8 10.3 / 10.9, 24 13.4 / 11.7; gate-up 2 x 2816 x 2048, 24 10.6 / 10.7, 47
+    15.4 / 12.8), short rows at few rows too (2 x 8192 x 2048, 8 15.1 / 15.3, 24 20.4
+    / 14.9), long ones less (2048 x 8192, 8 15.2 / 11.7). Column splits fill the CUs;
+    less than 0.8 of the last round filled loses (12288 x 4096, 24 22.7 / 25.0), and
+    at two or three rows so does adding up many splits (4096 x 14336, 2 21.8 / 23.0).
+    Up to 16 rows of 4096 the persistent skinny form is the better one where no
+    split is needed (2 x 14336, 8 45.1 / 46.3), under eight shorter rows the strips
+    (32000 x 2048, 4 26.6 / 29.4). Two tiles of 64 rows beat a tile of 96 or 128
+    under 64 MB of weights (2048 x 8192, 128 20.7 / 16.1; 2 x 8192 x 2048, 77 18.7 in
+    one, 19.8 in two); from there on a tile of 128 pays only with splits (2 x 14336 x
+    4096, 58.0 / 59.5)."""
+    if not 1 < M <= 128 or K % 64 or K < 256 or N % 8:
+        return None
+    weights = (2 if gateup else 1) * N * K
+    if M <= 16:
+        ok = (weights >= (2 ** 24 if K >= 8192 else 24e6 if K >= 4096 else 60e6))
+    else:
+        ok = weights >= (10e6 if gateup and M > 32 else 2 ** 24)
+    if not ok:
+        return None
+    strips = -(-N // (64 if gateup else 128))
+    for tile in (64, 32 * -(-M // 32)) if M > 64 and weights < 2 ** 25 else (32 * -(-M // 32),):
+        tiles = strips * -(-M // tile)
+        splits = max(1, min(256 // tiles, K // 256))
+        blocks = tiles * splits
+        if (blocks >= 0.8 * 256 * -(-blocks // 256) and (M >= 4 or splits <= 5)
+                and not (splits == 1 and (tile == 128 or M <= 16 and K == 4096 or M < 8 and K < 4096))):
+            return tile, splits
+    return None
+
+
+def _ring(x: torch.Tensor, w: torch.Tensor, plan: Tuple[int, int], act: int = 0) -> torch.Tensor:
+    """x @ w^T, or act 1 (silu), 2 (tanh gelu) of the gate rows times the up rows."""
+    lib, hip = _lib()
+    K, (tile, splits) = x.shape[-1], plan
+    M, N = x.numel() // K, w.shape[0] // (2 if act else 1)
+    out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
+    # at most 256 tiles of 128 x 128 float32 (gate and up): 17 MB
+    part = None if splits == 1 else torch.empty(splits * M * w.shape[0], dtype=torch.float32,
+                                                device=x.device)
+    hip.check(lib.oa_ring_gemm(hip.current_stream_ptr(), x.data_ptr(),
+                               K if x.is_contiguous() else x.stride(0), w.data_ptr(),
+                               out.data_ptr(), None if part is None else part.data_ptr(),
+                               M, N, K, tile, splits, act), "oa_ring_gemm")
+    return out
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear with custom HIP paths for decode shapes: the VALU GEMV at M = 1
-    (hipBLASLt's M=1 kernels run ~2.5x off the HBM roofline on gfx950), the skinny
-    matrix-core products up to 32 rows where they win (_skinny_form), the VALU GEMV
-    for what two rows are left; everything else goes to hipBLASLt."""
+    (hipBLASLt's M=1 kernels run ~2.5x off the HBM roofline on gfx950), the transfer
+    ring up to 128 rows and the skinny matrix-core products up to 32 where they win
+    (_ring_plan, _skinny_form), the VALU GEMV for what two rows are left; everything
+    else goes to hipBLASLt."""
     M = x.numel() // x.shape[-1]
-    if 1 < M <= 32 and _skinny_ok(x, w):
+    if 1 < M <= 128 and _skinny_ok(x, w):
+        plan = _ring_plan(M, w.shape[0], w.shape[1])
+        if plan:
+            return _ring(x, w, plan)
         form = _skinny_form(M, w.shape[0], w.shape[1])
         if form:
             return _skinny(x, w, form)
@@ -682,12 +740,13 @@ def gateup_silu(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> torch
 
 def gateup_fused(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> bool:
     """Whether gateup_act takes this product in one launch: the VALU GEMV up to
-    two rows, the skinny matrix-core product up to 32 where it wins."""
-    M = x.numel() // x.shape[-1]
+    two rows, the transfer ring and the skinny matrix-core product where they win."""
+    M, K = x.numel() // x.shape[-1], x.shape[-1]
     return (
         x.is_cuda and x.dtype == torch.bfloat16 and x.shape[-1] % 8 == 0 and x.is_contiguous()
         and (_gemv_m_ok(M) or (_skinny_ok(x, gate_up_w)
-                               and _skinny_form(M, i_local, x.shape[-1], gateup=True) > 0))
+                               and (_ring_plan(M, i_local, K, gateup=True) is not None
+                                    or _skinny_form(M, i_local, K, gateup=True) > 0)))
     )
 
 
@@ -701,6 +760,9 @@ def gateup_act(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int,
     assert x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous()
     assert act in ("silu", "gelu_tanh")
     if M > 1 and _skinny_ok(x, gate_up_w):
+        plan = _ring_plan(M, i_local, x.shape[-1], gateup=True)
+        if plan:
+            return _ring(x, gate_up_w, plan, act=1 + int(act == "gelu_tanh"))
         form = _skinny_form(M, i_local, x.shape[-1], gateup=True)
         if form:
             return _skinny(x, gate_up_w, form, gateup=True, act=int(act == "gelu_tanh"))

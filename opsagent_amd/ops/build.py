@@ -27,6 +27,7 @@ SOURCES = [
     "moe_gemv.hip",
     "moe_grouped.hip",
     "skinny.hip",
+    "ring_gemm.hip",
 ]
 
 # the sequence-mixer kernels of hybrid decoders live in a library of their

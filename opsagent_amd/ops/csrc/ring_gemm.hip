@@ -1,0 +1,233 @@
+// Products of 2 to 128 rows with large weights: C[M, N] = x[M, K] W[N, K]^T in bf16, plain
+// or gate-up with its activation. What bounds them is the weight stream, so everything
+// serves to keep enough of it under way on every CU: both operands by direct transfers
+// into a deep ring in LDS (no registers held by loads in flight), one block per CU, columns
+// split where the strips alone would leave CUs idle, and weights read without being kept
+// (nt) where they pass once: 5.9 TB/s, plain transfers of the same pieces reach 5.3. Us in
+// graphs over 2 GB of weights, before (skinny.hip up to 32 rows, the library and the
+// activation kernel above) / here: gate-up 2 x 14336 x 4096, M = 32 56.5 / 47.6, 47 55.7 /
+// 49.5, 77 59.0 / 52.9; 4096 x 14336, M = 8 29.7 / 23.3, 47 40.0 / 27.1, 77 49.1 / 30.7, 128
+// 75.4 / 33.5; 6144 x 4096, M = 8 17.4 / 13.2, 47 18.0 / 16.4, 77 22.7 / 18.0; 32000 x 4096,
+// M = 32 57.8 / 48.5, 77 56.3 / 53.7; 8192 x 28672, M = 8 89.3 / 75.4, 47 140 / 81.0, 77
+// 194 / 88.9. (The same over 0.5 GB reads up to a fifth better than inside a model.)
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(4))) float rgf4;
+typedef __attribute__((ext_vector_type(8))) short rgs8;
+
+#define RG_N 128                        // weight rows of a strip
+#define RG_K 64                         // columns of a step: 128 bytes
+
+template <int V>
+__device__ __forceinline__ void rg_wait() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(V) : "memory");
+}
+
+__device__ __forceinline__ float rg_gate(float g, float u, int act) {
+    if (act == 2) {
+        const float t = 0.7978845608028654f * fmaf(0.044715f * g * g, g, g);
+        return 0.5f * g * (1.0f + tanhf(t)) * u;
+    }
+    return g / (1.0f + __expf(-g)) * u;
+}
+
+// A block of four waves takes BM rows, a strip of 128 weight rows (GU: 64 gate rows and
+// the 64 up rows beside them) and one of `splits` runs of 64-column steps; a wave takes
+// all rows by 32 of the strip on v_mfma_f32_16x16x32_bf16, weights as the first operand,
+// so that a lane ends with four neighbouring outputs of one row. Both operands come by
+// 16-byte global_load_lds into a ring of STAGES steps: STAGES - 1 under way while one
+// is in use, waits that leave the younger ones in flight (inline asm: hipcc's own waits
+// drain builtin transfers before the first LDS read), one barrier per step, which says
+// that the step has landed for every wave and that the one before is no longer read.
+// 16-byte chunk c of row r lies at c ^ (r >> 1 & 7): the 16 rows of a fragment read
+// touch every bank once. Weight rows past N and rows past M repeat the last one.
+template <int BM, int STAGES, bool GU, bool NT>
+__global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
+    const uint16_t* __restrict__ x, int64_t xs, const uint16_t* __restrict__ w,
+    uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int K, int mtiles,
+    int splits, int items, int act) {
+    constexpr int MT = BM / 16, LPS = 4 + BM / 32, STEP = (RG_N + BM) * 128;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int per = gridDim.x >> 3;
+    const int item = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (item >= items) return;
+    const int strip = item / (splits * mtiles), rest = item - strip * splits * mtiles;
+    const int sp = rest / mtiles, m0 = (rest - sp * mtiles) * BM;
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int steps = K / RG_K;
+    const int s0 = (int)((int64_t)steps * sp / splits), s1 = (int)((int64_t)steps * (sp + 1) / splits);
+
+    // a transfer takes eight rows; this lane's row of it and its chunk
+    const int lr = lane >> 3;
+    const char* src[LPS];
+    uint32_t dst[LPS];
+#pragma unroll
+    for (int p = 0; p < LPS; ++p) {
+        const bool isw = p < 4;
+        const int r = (isw ? wid * 4 + p : (p - 4) * 4 + wid) * 8 + lr;
+        const int chunk = (lane & 7) ^ (r >> 1 & 7);
+        int64_t at;
+        if (!isw) at = min(m0 + r, M - 1) * xs;
+        else if (GU) at = (int64_t)(min(strip * 64 + (r >> 5) * 16 + (r & 15), N - 1) + (r & 16 ? N : 0)) * K;
+        else at = (int64_t)min(strip * RG_N + r, N - 1) * K;
+        src[p] = reinterpret_cast<const char*>((isw ? w : x) + at) + (int64_t)s0 * 128 + chunk * 16;
+        dst[p] = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + (isw ? 0 : RG_N * 128) +
+                                                (r - lr) * 128);
+    }
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int p = 0; p < LPS; ++p) {
+            if (NT && p < 4)
+                asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off nt"
+                             : : "s"(dst[p] + buf * STEP), "v"(src[p]) : "memory");
+            else
+                asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off"
+                             : : "s"(dst[p] + buf * STEP), "v"(src[p]) : "memory");
+            src[p] += 128;
+        }
+    };
+    rgf4 acc[2][MT] = {};
+    const int n = s1 - s0;
+#pragma unroll
+    for (int t = 0; t < STAGES - 1; ++t)
+        if (t < n) stage(t);
+    int buf = 0;
+    for (int t = 0; t < n; ++t) {
+        const int behind = min(STAGES - 2, n - 1 - t);    // younger steps under way
+        if (STAGES > 5 && behind >= 4) rg_wait<4 * LPS>();
+        else if (STAGES > 4 && behind >= 3) rg_wait<3 * LPS>();
+        else if (behind == 2) rg_wait<2 * LPS>();
+        else if (behind == 1) rg_wait<LPS>();
+        else rg_wait<0>();
+        if (t + STAGES - 1 < n) stage(buf == 0 ? STAGES - 1 : buf - 1);
+        const char* b = smem + buf * STEP;
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            const int r = lane & 15, c = kk * 4 + (lane >> 4);
+            const int at = r * 128 + ((c ^ (r >> 1)) << 4);         // rows step by 16: r >> 1 & 7 stays
+            rgs8 wf[2], xf[MT];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                wf[j] = *reinterpret_cast<const rgs8*>(b + (wid * 32 + j * 16) * 128 + at);
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+                xf[m] = *reinterpret_cast<const rgs8*>(b + (RG_N + m * 16) * 128 + at);
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[j][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[m], acc[j][m], 0, 0, 0);
+        }
+        buf = buf + 1 == STAGES ? 0 : buf + 1;
+    }
+    // D: column (row of x) lane & 15, rows (weight rows) (lane >> 4) * 4 and up
+    const int q = (lane >> 4) * 4;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int row = m0 + m * 16 + (lane & 15);
+        if (row >= M) continue;
+        if (GU) {
+            const int col = strip * 64 + wid * 16 + q;
+            if (col >= N) continue;
+            if (part) {
+                float* p = part + ((size_t)sp * M + row) * 2 * N + col;
+                *reinterpret_cast<rgf4*>(p) = acc[0][m];
+                *reinterpret_cast<rgf4*>(p + N) = acc[1][m];
+            } else {
+                float o[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = rg_gate(acc[0][m][i], acc[1][m][i], act);
+                *reinterpret_cast<uint2*>(out + (size_t)row * N + col) =
+                    make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int col = strip * RG_N + wid * 32 + j * 16 + q;
+                if (col >= N) continue;
+                if (part)
+                    *reinterpret_cast<rgf4*>(part + ((size_t)sp * M + row) * N + col) = acc[j][m];
+                else
+                    *reinterpret_cast<uint2*>(out + (size_t)row * N + col) =
+                        make_uint2(pack_bf16x2(acc[j][m][0], acc[j][m][1]),
+                                   pack_bf16x2(acc[j][m][2], acc[j][m][3]));
+            }
+        }
+    }
+}
+
+// parts [splits, M, N] (GU: [splits, M, 2 N]) added up in order
+template <bool GU>
+__global__ __launch_bounds__(256) void ring_sum_kernel(const float* __restrict__ part,
+                                                       uint16_t* __restrict__ out, int M, int N,
+                                                       int splits, int act) {
+    const int n4 = N / 4;
+    const int c = blockIdx.x * blockDim.x + threadIdx.x, row = blockIdx.y;
+    if (c >= n4) return;
+    const size_t w = (GU ? 2 : 1) * (size_t)n4;
+    const rgf4* p = reinterpret_cast<const rgf4*>(part) + row * w + c;
+    rgf4 a = {}, u = {};
+#pragma unroll 4
+    for (int s = 0; s < splits; ++s) {
+        a += p[(size_t)s * M * w];
+        if (GU) u += p[(size_t)s * M * w + n4];
+    }
+    if (GU)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[i] = rg_gate(a[i], u[i], act);
+    reinterpret_cast<uint2*>(out)[(size_t)row * n4 + c] =
+        make_uint2(pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]));
+}
+
+// out [M, N] = x [M, K] w [N, K]^T, x rows xs elements apart. act 1 (silu), 2 (tanh gelu):
+// out = act(x w[:N]^T) * (x w[N:]^T), w [2 N, K]. bm: rows of a tile, 32, 64, 96 or 128.
+// scratch: splits * M * N floats (act: twice that), unused at splits 1.
+extern "C" int oa_ring_gemm(void* stream, const void* x, int64_t xs, const void* w, void* out,
+                            void* scratch, int M, int N, int K, int bm, int splits, int act) {
+    if (M < 1 || M > 65535 || N < 4 || N % 4 != 0 || K < RG_K || K % RG_K != 0) return -100;
+    if (splits < 1 || splits > K / RG_K || (splits > 1 && !scratch)) return -101;
+    if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)scratch) % 16 != 0 || xs % 8 != 0)
+        return -102;
+    if (act < 0 || act > 2 || (bm != 32 && bm != 64 && bm != 96 && bm != 128)) return -104;
+    const bool gateup = act != 0;
+    const int mtiles = CEIL_DIV(M, bm);
+    const int64_t items = (int64_t)(gateup ? CEIL_DIV(N, 64) : CEIL_DIV(N, RG_N)) * mtiles * splits;
+    if (items > (1 << 28)) return -103;
+    hipStream_t s = (hipStream_t)stream;
+    const dim3 grid((unsigned)(CEIL_DIV(items, 8) * 8)), block(256);
+    float* part = splits > 1 ? (float*)scratch : nullptr;
+#define RG(BMV, ST, G, NT)                                                                         \
+    hipLaunchKernelGGL((ring_gemm_kernel<BMV, ST, G, NT>), grid, block, (ST) * (RG_N + (BMV)) * 128, s, \
+                       (const uint16_t*)x, xs, (const uint16_t*)w, (uint16_t*)out, part, M, N, K,  \
+                       mtiles, splits, (int)items, act)
+#define RGB(BMV, ST, NT)               \
+    do {                               \
+        if (gateup) RG(BMV, ST, true, NT); \
+        else RG(BMV, ST, false, NT);   \
+    } while (0)
+    // read without being kept: weights no other row tile reads, unless there are many rows
+    // and few weights (us kept / not, 6144 x 4096, M = 8 14.3 / 13.2, 77 18.2 / 20.2; 2 x 8192
+    // x 2048, 47 18.5 / 16.4; 8192 x 28672, 77 98.9 / 88.6)
+    const bool nt = mtiles == 1 && (bm == 32 || (int64_t)N * K * (gateup ? 2 : 1) >= 32000000);
+    if (bm == 32) RGB(32, 6, true);
+    else if (bm == 64 && nt) RGB(64, 5, true);
+    else if (bm == 64) RGB(64, 5, false);
+    else if (bm == 96 && nt) RGB(96, 5, true);
+    else if (bm == 96) RGB(96, 5, false);
+    else if (nt) RGB(128, 4, true);
+    else RGB(128, 4, false);
+#undef RGB
+#undef RG
+    if (splits > 1) {
+        const dim3 g(CEIL_DIV(N / 4, 256), M);
+        if (gateup)
+            hipLaunchKernelGGL(ring_sum_kernel<true>, g, block, 0, s, part, (uint16_t*)out, M, N,
+                               splits, act);
+        else
+            hipLaunchKernelGGL(ring_sum_kernel<false>, g, block, 0, s, part, (uint16_t*)out, M, N,
+                               splits, 0);
+    }
+    HIP_CHECK_LAUNCH();
+    return 0;
+}

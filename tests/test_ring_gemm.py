@@ -1,0 +1,77 @@
+"""Products on the transfer ring against float64: row tiles, strip and row remainders,
+fewer steps than the ring holds, column splits, both activations, rows apart; and which
+products take it."""
+
+import pytest
+import torch
+
+from opsagent_amd import ops
+
+# M, N, K, rows of a tile, splits
+FORMS = [
+    (2, 8, 64, 32, 1), (32, 128, 192, 32, 2), (17, 264, 320, 32, 5),
+    (33, 136, 384, 64, 1), (64, 256, 448, 64, 7), (65, 72, 640, 64, 3), (127, 384, 1024, 64, 16),
+    (66, 200, 256, 96, 2), (96, 128, 1088, 96, 1), (97, 392, 512, 128, 1), (128, 1000, 4096, 128, 5),
+    (200, 128, 256, 64, 2), (47, 4096, 1024, 64, 4),
+]
+
+
+def _whole(rows, cols, scale=1.0):
+    """Whole numbers up to 2 times a power of two: every product and sum is exact."""
+    return (torch.randint(-2, 3, (rows, cols), device="cuda") * scale).to(torch.bfloat16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,tile,splits", FORMS)
+def test_plain(M, N, K, tile, splits):
+    torch.manual_seed(M + N + K)
+    wide = _whole(M, K + 8)
+    w = _whole(N, K)
+    for x in (wide[:, :K].contiguous(), wide[:, :K]):      # rows apart as well
+        got = ops._ring(x, w, (tile, splits))
+        assert torch.equal(got, (x.double() @ w.double().T).to(torch.bfloat16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", [1, 2])
+@pytest.mark.parametrize("M,N,K,tile,splits", FORMS)
+def test_gateup(M, N, K, tile, splits, act):
+    torch.manual_seed(M + N + K)
+    x, w = _whole(M, K), _whole(2 * N, K, 2.0 ** -5)
+    got = ops._ring(x, w, (tile, splits), act).double()
+    g, u = (x.double() @ w.double().T).split(N, 1)
+    f = torch.nn.functional.silu(g) if act == 1 else torch.nn.functional.gelu(g, approximate="tanh")
+    # one rounding to bf16, and some float32 roundings (exp of up to |g| / ln 2 scaled
+    # bits, 1 + tanh near -1) of the exact halves
+    bound = 2.0 ** -8 * (f * u).abs() + 2.0 ** -20 * (1 + g.abs()) * (g * u).abs()
+    assert ((got - f * u).abs() <= bound).all()
+
+
+def test_plans_stay_in_range():
+    """Tiles cover the rows, splits have steps of their own, parts stay small."""
+    for gateup in (False, True):
+        for K in (256, 512, 2048, 4096, 7168, 14336, 28672):
+            for N in (8, 1024, 2048, 4096, 6144, 8192, 12288, 14336, 32000, 128256):
+                for M in range(1, 130):
+                    plan = ops._ring_plan(M, N, K, gateup)
+                    if plan is None:
+                        continue
+                    tile, splits = plan
+                    assert 1 < M <= 128 and tile in (32, 64, 96, 128)
+                    assert 1 <= splits <= K // 64
+                    assert -(-M // tile) == 1 or tile == 64
+                    if splits > 1:
+                        assert splits * M * N * (2 if gateup else 1) * 4 <= 64 << 20
+
+
+def test_plans_at_the_lines():
+    assert ops._ring_plan(1, 4096, 14336) is None
+    assert ops._ring_plan(8, 4096, 14336) == (32, 8)
+    assert ops._ring_plan(2, 4096, 14336) is None
+    assert ops._ring_plan(47, 14336, 4096, True) == (64, 1)
+    assert ops._ring_plan(128, 14336, 4096, True) is None
+    assert ops._ring_plan(8, 14336, 4096, True) is None
+    assert ops._ring_plan(96, 4096, 4096) == (64, 4)
+    assert ops._ring_plan(8, 4096, 4096) is None
+    assert ops._ring_plan(32, 12288, 4096) is None
+    assert ops._ring_plan(129, 4096, 14336) is None
