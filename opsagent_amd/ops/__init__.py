@@ -955,20 +955,26 @@ def _fp8_gemv_ok(x: torch.Tensor) -> bool:
     )
 
 
+def _fp8_gemv1_ok(x: torch.Tensor, N: int) -> bool:
+    """Mirror of fp8_moe.hip's gemv1_fp8_ok for one row x and N weight rows."""
+    return x.shape[-1] % 2048 == 0 and x.shape[-1] <= 16384 and N % 2 == 0 and x.data_ptr() % 16 == 0
+
+
 def linear_norm_fp8(
     x: torch.Tensor, norm_w: torch.Tensor, eps: float,
     w8: torch.Tensor, w_scale: torch.Tensor,
 ) -> torch.Tensor:
     """rmsnorm(x) @ dequant(W8)^T with the norm fused into the fp8 GEMV
-    prologue (fp8 decode fast path). At M=1 the VALU stream kernel runs the
-    norm per ELEMENT inside the weight loop (measured 2.7 vs 5.1 TB/s on the
-    70B qkv shape), so a single rmsnorm pass + the plain kernel wins; the
-    M>=2 MFMA path fuses the norm into its one-shot x-quant instead."""
+    prologue (fp8 decode fast path): at M=1 where the one-row kernel takes the
+    shape (once per block; _fp8_gemv1_ok). Elsewhere at M=1 the VALU stream
+    kernel would run the norm per ELEMENT inside the weight loop (measured 2.7 vs
+    5.1 TB/s on the 70B qkv shape), so a rmsnorm pass + the plain kernel wins;
+    the M>=2 MFMA path fuses the norm into its one-shot x-quant instead."""
     if not _fp8_gemv_ok(x):
         return linear_fp8(rms_norm(x, norm_w, eps), w8, w_scale)
     lib, hip = _lib()
     M = x.numel() // x.shape[-1]
-    if M == 1:
+    if M == 1 and not _fp8_gemv1_ok(x, w8.shape[0]):
         return linear_fp8(rms_norm(x, norm_w, eps), w8, w_scale)
     N, K4 = w8.shape[0], x.shape[-1]
     out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
@@ -1016,7 +1022,7 @@ def gateup_silu_fp8(
         return silu_halves(linear_fp8(xin, w8, w_scale), i_local)
     lib, hip = _lib()
     M = x.numel() // x.shape[-1]
-    if use_norm and M == 1:  # see linear_norm_fp8: prenorm beats in-loop norm
+    if use_norm and M == 1 and not _fp8_gemv1_ok(x, 2):  # see linear_norm_fp8
         x = rms_norm(x, norm_w, eps)
         norm_w = None
         use_norm = False

@@ -488,6 +488,210 @@ static bool gemv_fp8_use_mfma(int M, int rows, int K, int gateup) {
     return (size_t)M * K <= 128 * 1024;
 }
 
+// One activation row, K a multiple of 2048 up to 16384: the scheme of the bf16 one-row
+// kernel (gemv.hip) on fp8 weights. The block's activations, normalised there with NORM,
+// are a float32 image in LDS, made once while the first weights are under way, four
+// planes of four columns in sixteen so that a wave's 16-byte reads are contiguous; a wave
+// streams the rows of its units two at a time (GU: a gate row and its up row) in groups
+// of GR 1024-column chunks, the next group under way while one is in use. us inside a
+// decode step, the forms above with their normalisation in a launch of its own / here:
+// gate-up 2 x 14336 x 4096 27.4 / 21.9, 6144 x 4096 11.1 / 7.8, 4096 x 14336 13.5 / 12.1;
+// asking for the activations before the weights is 3 us of the normalised ones. A third
+// group under way from the start cost more in waits than it hid (gate-up 27.6), seven
+// chunks a group too (4096 x 14336 14.0).
+template <bool NORM, bool ADDRES, bool GU, int GR, int XV>
+__global__ __launch_bounds__(512) void gemv1_fp8_kernel(
+    const uint4* __restrict__ x, const uint32_t* __restrict__ w8, const float* __restrict__ wscale,
+    uint16_t* __restrict__ out, const uint4* __restrict__ wn, const uint16_t* __restrict__ res,
+    int N, int K, int per, float eps) {
+    extern __shared__ __attribute__((aligned(16))) float xl[];   // [4][K / 4]
+    __shared__ float part[8];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int units = GU ? N : N / 2;
+    const int u0 = (blockIdx.x * 8 + wid) * per, u1 = min(u0 + per, units);
+    const int k4 = K / 4, groups = K / (1024 * GR);
+    const int total = max(u1 - u0, 0) * groups;
+    auto row_of = [&](int u, int t) { return GU ? u + t * N : u * 2 + t; };
+    u32x4 a[GR][2], b[GR][2];
+    int u = min(u0, units - 1), g = 0;                      // of the group loaded last
+    auto load = [&](u32x4 (&v)[GR][2]) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < GR; ++i)
+                v[i][t] = nt_load4f(w8 + (size_t)row_of(u, t) * k4 + (g * GR + i) * 256 + lane * 4);
+    };
+    auto next = [&](u32x4 (&v)[GR][2]) {
+        if (++g == groups) {
+            g = 0;
+            ++u;
+        }
+        load(v);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Loads return in order: the activations and lane i's scale and residual of the wave's
+    // unit i (per <= 64) are asked for before the weights, so that the image below waits
+    // for them alone.
+    uint4 xv[XV], nv[XV];
+#pragma unroll
+    for (int j = 0; j < XV; ++j) {
+        const int i = min(j * 512 + tid, K / 8 - 1);
+        xv[j] = x[i];
+        if (NORM) nv[j] = wn[i];
+    }
+    float sc[2], rs[2] = {0.0f, 0.0f};
+    {
+        const int mine = min(u0 + lane, units - 1);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            sc[t] = wscale[row_of(mine, t)];
+            if (ADDRES) rs[t] = bf16_to_f32(res[row_of(mine, t)]);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    load(a);
+    __builtin_amdgcn_sched_barrier(0);
+
+    float rstd = 1.0f;
+    if (NORM) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int j = 0; j < XV; ++j)
+            if (j * 512 + tid < K / 8)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float lo = bf16_lo((&xv[j].x)[e]), hi = bf16_hi((&xv[j].x)[e]);
+                    ss = fmaf(lo, lo, ss);
+                    ss = fmaf(hi, hi, ss);
+                }
+        ss = wave_reduce_sum(ss);
+        if (lane == 0) part[wid] = ss;
+        __syncthreads();
+        ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ss += part[i];
+        rstd = rsqrtf(ss / (float)K + eps);
+    }
+#pragma unroll
+    for (int j = 0; j < XV; ++j) {
+        const int i = j * 512 + tid;                        // columns i * 8 .. + 7
+        if (i >= K / 8) continue;
+        float f[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            f[2 * e] = bf16_lo((&xv[j].x)[e]);
+            f[2 * e + 1] = bf16_hi((&xv[j].x)[e]);
+            if (NORM) {
+                f[2 * e] *= rstd * bf16_lo((&nv[j].x)[e]);
+                f[2 * e + 1] *= rstd * bf16_hi((&nv[j].x)[e]);
+            }
+        }
+        float* at = xl + (i & 1) * 2 * k4 + (i >> 1) * 4;
+        *reinterpret_cast<float4*>(at) = make_float4(f[0], f[1], f[2], f[3]);
+        *reinterpret_cast<float4*>(at + k4) = make_float4(f[4], f[5], f[6], f[7]);
+    }
+    __syncthreads();
+
+    float acc[2] = {0.0f, 0.0f};
+    int uu = 0, ug = 0;                                     // unit of the wave, group in use
+    auto use = [&](u32x4 (&v)[GR][2]) {
+#pragma unroll
+        for (int i = 0; i < GR; ++i) {
+            const int c = (ug * GR + i) * 64 + lane;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 f = reinterpret_cast<const float4*>(xl + q * k4)[c];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const f32x2 lo = fp8x2_to_f32<false>(v[i][t][q]), hi = fp8x2_to_f32<true>(v[i][t][q]);
+                    float d = acc[t];
+                    d = fmaf(f.x, lo[0], d);
+                    d = fmaf(f.y, lo[1], d);
+                    d = fmaf(f.z, hi[0], d);
+                    acc[t] = fmaf(f.w, hi[1], d);
+                }
+            }
+        }
+        if (++ug == groups) {
+            float r[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                r[t] = wave_reduce_sum(acc[t]) * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc[t]), uu));
+                if (ADDRES) r[t] += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rs[t]), uu));
+                acc[t] = 0.0f;
+            }
+            if (lane == 0) {
+                if (GU) out[u0 + uu] = f32_to_bf16(r[0] / (1.0f + __expf(-r[0])) * r[1]);
+                else reinterpret_cast<uint32_t*>(out)[u0 + uu] = pack_bf16x2(r[0], r[1]);
+            }
+            ug = 0;
+            ++uu;
+        }
+    };
+    // the last groups are apart, so that every wait counts the loads behind it exactly
+    int n = 0;
+    for (; n + 2 < total; n += 2) {
+        next(b);
+        use(a);
+        next(a);
+        use(b);
+    }
+    if (n + 2 == total) {
+        next(b);
+        use(a);
+        use(b);
+    } else if (n < total) {
+        use(a);
+    }
+}
+
+static bool gemv1_fp8_ok(const void* x, const void* w8, const void* wn, const void* out, int M, int N,
+                         int K, bool gateup) {
+    return M == 1 && K % 2048 == 0 && K >= 2048 && K <= 16384 && N >= 1 && (gateup || N % 2 == 0) &&
+           ((uintptr_t)x | (uintptr_t)w8 | (uintptr_t)wn) % 16 == 0 && (uintptr_t)out % 4 == 0;
+}
+
+// mode: 1 normalise x first, 2 add res
+static int gemv1_fp8(hipStream_t st, const void* x, const void* w8, const void* wscale, void* out,
+                     const void* wn, const void* res, int N, int K, float eps, int mode, bool gateup) {
+    const int units = gateup ? N : N / 2;
+    // as many blocks of eight waves as stay resident (two per CU), fewer and fuller ones
+    // where that evens out the CUs by more than a fifth
+    auto rounds = [&](int p) { return CEIL_DIV(CEIL_DIV(CEIL_DIV(units, p), 8), 256) * p; };
+    int per = CEIL_DIV(units, 4096);
+    for (int p = per + 1, p1 = 2 * per + 1; p <= p1; ++p)
+        if (rounds(p) * 5 < rounds(per) * 4) per = p;
+    if (per > 64) per = 64;
+    const int blocks = CEIL_DIV(CEIL_DIV(units, per), 8);
+#define G1F(NV, RV, GV, GR, XV)                                                                       \
+    hipLaunchKernelGGL((gemv1_fp8_kernel<NV, RV, GV, GR, XV>), dim3(blocks), dim3(512), (size_t)K * 4, \
+                       st, (const uint4*)x, (const uint32_t*)w8, (const float*)wscale,                \
+                       (uint16_t*)out, (const uint4*)wn, (const uint16_t*)res, N, K, per, eps)
+#define G1FK(NV, RV, GV)                                \
+    do {                                                \
+        if (K == 4096) G1F(NV, RV, GV, 4, 1);           \
+        else if (K < 4096) G1F(NV, RV, GV, 2, 1);       \
+        else G1F(NV, RV, GV, 2, 4);                     \
+    } while (0)
+    if (gateup) {
+        if (mode & 1) G1FK(true, false, true);
+        else G1FK(false, false, true);
+    } else {
+        switch (mode) {
+            case 0: G1FK(false, false, false); break;
+            case 1: G1FK(true, false, false); break;
+            case 2: G1FK(false, true, false); break;
+            case 3: G1FK(true, true, false); break;
+            default: return -102;
+        }
+    }
+#undef G1FK
+#undef G1F
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
 extern "C" int oa_gemv_fp8_ex(void* stream, const void* x, const void* w8,
                               const void* wscale, void* out, const void* wn,
                               const void* res, int M, int N, int K, float eps,
@@ -496,6 +700,8 @@ extern "C" int oa_gemv_fp8_ex(void* stream, const void* x, const void* w8,
     if (gemv_fp8_use_mfma(M, N, K, 0))
         return oa_gemv_fp8_mfma(stream, x, w8, wscale, out, wn, res, M, N, K,
                                 eps, mode, 0);
+    if (gemv1_fp8_ok(x, w8, mode & 1 ? wn : nullptr, out, M, N, K, false))
+        return gemv1_fp8((hipStream_t)stream, x, w8, wscale, out, wn, res, N, K, eps, mode, false);
     // M=1 runs the RW=2 two-stream form (x unpack amortized — the gateup
     // structure measured 5.96 vs 5.1 TB/s); OPSAGENT_FP8_GEMV_RW=1 forces
     // the single-stream form for A/B.
@@ -576,6 +782,9 @@ extern "C" int oa_gemv_gateup_fp8(void* stream, const void* x, const void* w8,
     if (gemv_fp8_use_mfma(M, I, K, 1))
         return oa_gemv_fp8_mfma(stream, x, w8, wscale, out, wn, nullptr, M,
                                 2 * I, K, eps, norm ? 1 : 0, 1);
+    if (gemv1_fp8_ok(x, w8, norm ? wn : nullptr, out, M, I, K, true))
+        return gemv1_fp8((hipStream_t)stream, x, w8, wscale, out, wn, nullptr, I, K, eps, norm ? 1 : 0,
+                         true);
     // M=1 instantiates RW=2 row-pairs (4 streams/wave)
     const int grid = min(4096, CEIL_DIV(I, M == 1 ? 8 : 4));
     const size_t xs_bytes = (size_t)M * K * 4;

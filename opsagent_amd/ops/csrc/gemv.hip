@@ -201,8 +201,9 @@ __global__ __launch_bounds__(256) void gemv_gateup_kernel(
 // us before and now, weights of 1 GiB in turn: 28672 x 4096 gate-up with norm 43.3 and
 // 38.4, 4096 x 14336 24.9 and 20.6, 6144 x 4096 with norm 12.9 and 11.0, 4096 x 4096
 // 8.9 and 8.5, 128256 x 4096 168 and 163, 2048 x 8192 12.0 and 8.4, 16384 x 2048 gate-up
-// 14.8 and 12.9, 2048 x 2048 4.7 and 4.2 (contiguous reads alone run at 6.4 to 6.9 TB/s).
-template <bool NORM, bool ADDRES, int RT, int GR>
+// 14.8 and 12.9, 2048 x 2048 4.7 and 4.2 (contiguous reads alone run at 6.4 to 6.9 TB/s);
+// asking for the activations before the weights takes another half a microsecond each.
+template <bool NORM, bool ADDRES, int RT, int GR, int XV>
 __global__ __launch_bounds__(512) void gemv1_kernel(const uint32_t* __restrict__ x,
                                                     const uint32_t* __restrict__ w,
                                                     uint16_t* __restrict__ out,
@@ -234,21 +235,33 @@ __global__ __launch_bounds__(512) void gemv1_kernel(const uint32_t* __restrict__
         load(v);
         __builtin_amdgcn_sched_barrier(0);
     };
+    // Loads return in order: the activations, eight columns per thread and turn, and lane
+    // i's residual of the wave's row i (per <= 64) are asked for before the weights, so
+    // that the image below waits for them alone.
+    uint4 xv[XV], nv[XV];
+#pragma unroll
+    for (int j = 0; j < XV; ++j) {
+        const int i = min(j * 512 + tid, K / 8 - 1);
+        xv[j] = reinterpret_cast<const uint4*>(x)[i];
+        if (NORM) nv[j] = reinterpret_cast<const uint4*>(wn)[i];
+    }
+    const float rs = ADDRES ? bf16_to_f32(res[min(r0 + lane, N - 1)]) : 0.0f;
+    __builtin_amdgcn_sched_barrier(0);
     load(a);
+    __builtin_amdgcn_sched_barrier(0);
 
-    // activations, eight columns per thread and turn
     float rstd = 1.0f;
     if (NORM) {
         float ss = 0.0f;
-        for (int i = tid; i < K / 8; i += 512) {
-            const uint4 v = reinterpret_cast<const uint4*>(x)[i];
-            const uint32_t u[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                ss = fmaf(bf16_lo(u[j]), bf16_lo(u[j]), ss);
-                ss = fmaf(bf16_hi(u[j]), bf16_hi(u[j]), ss);
-            }
-        }
+        for (int j = 0; j < XV; ++j)
+            if (j * 512 + tid < K / 8)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float lo = bf16_lo((&xv[j].x)[e]), hi = bf16_hi((&xv[j].x)[e]);
+                    ss = fmaf(lo, lo, ss);
+                    ss = fmaf(hi, hi, ss);
+                }
         ss = wave_reduce_sum(ss);
         if (lane == 0) part[wid] = ss;
         __syncthreads();
@@ -257,22 +270,18 @@ __global__ __launch_bounds__(512) void gemv1_kernel(const uint32_t* __restrict__
         for (int i = 0; i < 8; ++i) ss += part[i];
         rstd = rsqrtf(ss / (float)K + eps);
     }
-    for (int i = tid; i < K / 8; i += 512) {
-        const uint4 v = reinterpret_cast<const uint4*>(x)[i];
-        const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int j = 0; j < XV; ++j) {
+        const int i = j * 512 + tid;
+        if (i >= K / 8) continue;
         float f[8];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            f[2 * j] = bf16_lo(u[j]);
-            f[2 * j + 1] = bf16_hi(u[j]);
-        }
-        if (NORM) {
-            const uint4 nv = reinterpret_cast<const uint4*>(wn)[i];
-            const uint32_t n4[4] = {nv.x, nv.y, nv.z, nv.w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                f[2 * j] *= rstd * bf16_lo(n4[j]);
-                f[2 * j + 1] *= rstd * bf16_hi(n4[j]);
+        for (int e = 0; e < 4; ++e) {
+            f[2 * e] = bf16_lo((&xv[j].x)[e]);
+            f[2 * e + 1] = bf16_hi((&xv[j].x)[e]);
+            if (NORM) {
+                f[2 * e] *= rstd * bf16_lo((&nv[j].x)[e]);
+                f[2 * e + 1] *= rstd * bf16_hi((&nv[j].x)[e]);
             }
         }
         reinterpret_cast<float4*>(xl)[i] = make_float4(f[0], f[1], f[2], f[3]);
@@ -306,10 +315,9 @@ __global__ __launch_bounds__(512) void gemv1_kernel(const uint32_t* __restrict__
         if (++ug == groups) {
             float v0 = wave_reduce_sum(acc[0]);
             if (RT == 2) v0 = gate_act(v0, act) * wave_reduce_sum(acc[RT - 1]);
-            if (lane == 0) {
-                if (ADDRES) v0 += bf16_to_f32(res[ur]);
-                out[ur] = f32_to_bf16(v0);
-            }
+            if (ADDRES)
+                v0 += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rs), ur - r0));
+            if (lane == 0) out[ur] = f32_to_bf16(v0);
 #pragma unroll
             for (int t = 0; t < RT; ++t) acc[t] = 0.0f;
             ug = 0;
@@ -344,12 +352,18 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
     int per = CEIL_DIV(N, 2048 * resident);
     for (int p = per + 1, p1 = 2 * per + 1; p <= p1; ++p)
         if (rounds(p) * 5 < rounds(per) * 4) per = p;
+    if (per > 64) per = 64;
     const int blocks = CEIL_DIV(CEIL_DIV(N, per), 8);
     const size_t lds = (size_t)K * 4;
-#define G1(NV, RV, RT, GR)                                                                            \
-    hipLaunchKernelGGL((gemv1_kernel<NV, RV, RT, GR>), dim3(blocks), dim3(512), lds, st,              \
+#define G1X(NV, RV, RT, GR, XV)                                                                       \
+    hipLaunchKernelGGL((gemv1_kernel<NV, RV, RT, GR, XV>), dim3(blocks), dim3(512), lds, st,          \
                        (const uint32_t*)x, (const uint32_t*)w, (uint16_t*)out, (const uint32_t*)wn,   \
                        (const uint16_t*)res, N, K, per, eps, gateup - 1)
+#define G1(NV, RV, RT, GR)                   \
+    do {                                     \
+        if (K <= 4096) G1X(NV, RV, RT, GR, 1); \
+        else G1X(NV, RV, RT, GR, 4);         \
+    } while (0)
     if (gateup) {
         if (mode & 1) G1(true, false, 2, 4);
         else G1(false, false, 2, 4);
@@ -369,6 +383,7 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
         }
     }
 #undef G1
+#undef G1X
     HIP_CHECK_LAUNCH();
     return 0;
 }
