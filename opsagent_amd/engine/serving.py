@@ -39,6 +39,7 @@ class EngineLoop:
         self._futures: Dict[int, Future] = {}
         self._wake = threading.Event()
         self._stop = False
+        self._stopped = threading.Event()
         # TP>1 followers never accept requests: rank 0's EngineLoop drives
         # them through the engine's step broadcast (engine.follower_loop
         # is their run loop — see cli serve / bench). No threads here.
@@ -63,7 +64,8 @@ class EngineLoop:
                         self.watchdog_s,
                     )
                 self.healthy = False
-            _t.sleep(min(5.0, self.watchdog_s / 4))
+            if self._stopped.wait(min(5.0, self.watchdog_s / 4)):
+                return
 
     def submit(self, prompt_ids: List[int], params: Optional[SamplingParams] = None) -> Future:
         """Thread-safe. Future resolves to (output_ids, finish_reason)."""
@@ -101,7 +103,12 @@ class EngineLoop:
         if self.is_follower:
             return
         self._wake.set()
+        self._stopped.set()
         self._thread.join(timeout=30)
+        # A thread that outlives this call holds the engine; were it the last to let go,
+        # graphs and caches would be destroyed under whatever another thread captures,
+        # which aborts the process.
+        self._watchdog.join(timeout=30)
         try:
             self.engine.shutdown_followers()
         except Exception:  # noqa: BLE001 — best effort; followers may be gone
