@@ -82,8 +82,9 @@ def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
     the L2, which costs 0.6 of the time that so many weight bytes take; the library
     starts 3.5 us later and streams 0.87 as fast, so strips win while their x
     traffic is under 35 MB + a quarter of the weight (25 MB + a fifth from 17 rows
-    on, whose fragments are two)."""
-    if M < 1 or M > 32 or K % 32 != 0:
+    on, whose fragments are two). Under 2^18 weights every form is its launch and the
+    library keeps them."""
+    if M < 1 or M > 32 or K % 32 != 0 or (2 if gateup else 1) * N * K < 2 ** 18:
         return 0
     if K == 4096 and (M <= 16 if gateup or N < 16384 else True) and (gateup or N >= 6144):
         return 2
