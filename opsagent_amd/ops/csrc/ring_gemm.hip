@@ -14,9 +14,10 @@
 
 typedef __attribute__((ext_vector_type(4))) float rgf4;
 typedef __attribute__((ext_vector_type(8))) short rgs8;
+typedef __attribute__((ext_vector_type(8))) int rgi8;
 
 #define RG_N 128                        // weight rows of a strip
-#define RG_K 64                         // columns of a step: 128 bytes
+#define RG_K 64                         // bf16 columns of a step: 128 bytes; fp8: 128
 
 template <int V>
 __device__ __forceinline__ void rg_wait() {
@@ -41,9 +42,17 @@ __device__ __forceinline__ float rg_gate(float g, float u, int act) {
 // that the step has landed for every wave and that the one before is no longer read.
 // 16-byte chunk c of row r lies at c ^ (r >> 1 & 7): the 16 rows of a fragment read
 // touch every bank once. Weight rows past N and rows past M repeat the last one.
-template <int BM, int STAGES, bool GU, bool NT>
+//
+// F8: e4m3 rows on v_mfma_scale_f32_16x16x128_f8f6f4 with unit block scales (the tile
+// product's arithmetic), a float32 scale per row of x and of w in the epilogue. us over 2 GB
+// of weights, the tile product (fp8_moe.hip) / here: 28672 x 4096, M = 9 31.4 / 26.0, 77
+// 37.5 / 31.1; 4096 x 14336, 9 66.3 / 14.9, 47 71.4 / 18.2, 128 78.9 / 26.5; 6144 x 4096, 47
+// 26.9 / 13.2; 4096 x 4096, 77 28.6 / 14.9; 8192 x 28672, 77 140 / 46.8; 2048 x 2816, 33 20.0
+// / 8.7.
+template <int BM, int STAGES, bool GU, bool NT, bool F8>
 __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
-    const uint16_t* __restrict__ x, int64_t xs, const uint16_t* __restrict__ w,
+    const char* __restrict__ x, int64_t xs, const char* __restrict__ w,
+    const float* __restrict__ xscale, const float* __restrict__ wscale,
     uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int K, int mtiles,
     int splits, int items, int act) {
     constexpr int MT = BM / 16, LPS = 4 + BM / 32, STEP = (RG_N + BM) * 128;
@@ -55,7 +64,8 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
     const int sp = rest / mtiles, m0 = (rest - sp * mtiles) * BM;
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int steps = K / RG_K;
+    const int64_t kb = F8 ? K : 2 * (int64_t)K;     // bytes of a weight row
+    const int steps = (int)(kb / 128);
     const int s0 = (int)((int64_t)steps * sp / splits), s1 = (int)((int64_t)steps * (sp + 1) / splits);
 
     // a transfer takes eight rows; this lane's row of it and its chunk
@@ -68,10 +78,10 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
         const int r = (isw ? wid * 4 + p : (p - 4) * 4 + wid) * 8 + lr;
         const int chunk = (lane & 7) ^ (r >> 1 & 7);
         int64_t at;
-        if (!isw) at = min(m0 + r, M - 1) * xs;
-        else if (GU) at = (int64_t)(min(strip * 64 + (r >> 5) * 16 + (r & 15), N - 1) + (r & 16 ? N : 0)) * K;
-        else at = (int64_t)min(strip * RG_N + r, N - 1) * K;
-        src[p] = reinterpret_cast<const char*>((isw ? w : x) + at) + (int64_t)s0 * 128 + chunk * 16;
+        if (!isw) at = min(m0 + r, M - 1) * xs * (F8 ? 1 : 2);
+        else if (GU) at = (min(strip * 64 + (r >> 5) * 16 + (r & 15), N - 1) + (r & 16 ? N : 0)) * kb;
+        else at = min(strip * RG_N + r, N - 1) * kb;
+        src[p] = (isw ? w : x) + at + (int64_t)s0 * 128 + chunk * 16;
         dst[p] = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + (isw ? 0 : RG_N * 128) +
                                                 (r - lr) * 128);
     }
@@ -102,22 +112,47 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
         else rg_wait<0>();
         if (t + STAGES - 1 < n) stage(buf == 0 ? STAGES - 1 : buf - 1);
         const char* b = smem + buf * STEP;
+        if constexpr (F8) {
+            const int r = lane & 15, c = (lane >> 4) * 2;
+            const int at = r * 128 + ((c ^ (r >> 1)) << 4), at2 = r * 128 + (((c + 1) ^ (r >> 1)) << 4);
+            auto frag = [&](const char* rows) {
+                union {
+                    uint4 h[2];
+                    rgi8 v;
+                } f;
+                f.h[0] = *reinterpret_cast<const uint4*>(rows + at);
+                f.h[1] = *reinterpret_cast<const uint4*>(rows + at2);
+                return f.v;
+            };
+            rgi8 wf[2], xf[MT];
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            const int r = lane & 15, c = kk * 4 + (lane >> 4);
-            const int at = r * 128 + ((c ^ (r >> 1)) << 4);         // rows step by 16: r >> 1 & 7 stays
-            rgs8 wf[2], xf[MT];
+            for (int j = 0; j < 2; ++j) wf[j] = frag(b + (wid * 32 + j * 16) * 128);
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-                wf[j] = *reinterpret_cast<const rgs8*>(b + (wid * 32 + j * 16) * 128 + at);
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-                xf[m] = *reinterpret_cast<const rgs8*>(b + (RG_N + m * 16) * 128 + at);
+            for (int m = 0; m < MT; ++m) xf[m] = frag(b + (RG_N + m * 16) * 128);
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
-                    acc[j][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[m], acc[j][m], 0, 0, 0);
+                    acc[j][m] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                        wf[j], xf[m], acc[j][m], 0, 0, 0, 0x7f, 0, 0x7f);
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+                const int r = lane & 15, c = kk * 4 + (lane >> 4);
+                const int at = r * 128 + ((c ^ (r >> 1)) << 4);         // rows step by 16: r >> 1 & 7 stays
+                rgs8 wf[2], xf[MT];
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    wf[j] = *reinterpret_cast<const rgs8*>(b + (wid * 32 + j * 16) * 128 + at);
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+                    xf[m] = *reinterpret_cast<const rgs8*>(b + (RG_N + m * 16) * 128 + at);
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[j][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[m], acc[j][m], 0, 0, 0);
+            }
         }
         buf = buf + 1 == STAGES ? 0 : buf + 1;
     }
@@ -146,20 +181,28 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
             for (int j = 0; j < 2; ++j) {
                 const int col = strip * RG_N + wid * 32 + j * 16 + q;
                 if (col >= N) continue;
-                if (part)
+                if (part) {
                     *reinterpret_cast<rgf4*>(part + ((size_t)sp * M + row) * N + col) = acc[j][m];
-                else
-                    *reinterpret_cast<uint2*>(out + (size_t)row * N + col) =
-                        make_uint2(pack_bf16x2(acc[j][m][0], acc[j][m][1]),
-                                   pack_bf16x2(acc[j][m][2], acc[j][m][3]));
+                    continue;
+                }
+                if (F8) {
+                    const float sx = xscale[row];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[j][m][i] = acc[j][m][i] * sx * wscale[col + i];
+                }
+                *reinterpret_cast<uint2*>(out + (size_t)row * N + col) =
+                    make_uint2(pack_bf16x2(acc[j][m][0], acc[j][m][1]),
+                               pack_bf16x2(acc[j][m][2], acc[j][m][3]));
             }
         }
     }
 }
 
 // parts [splits, M, N] (GU: [splits, M, 2 N]) added up in order
-template <bool GU>
+template <bool GU, bool F8>
 __global__ __launch_bounds__(256) void ring_sum_kernel(const float* __restrict__ part,
+                                                       const float* __restrict__ xscale,
+                                                       const float* __restrict__ wscale,
                                                        uint16_t* __restrict__ out, int M, int N,
                                                        int splits, int act) {
     const int n4 = N / 4;
@@ -176,6 +219,11 @@ __global__ __launch_bounds__(256) void ring_sum_kernel(const float* __restrict__
     if (GU)
 #pragma unroll
         for (int i = 0; i < 4; ++i) a[i] = rg_gate(a[i], u[i], act);
+    if (F8) {
+        const float sx = xscale[row];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[i] = a[i] * sx * wscale[c * 4 + i];
+    }
     reinterpret_cast<uint2*>(out)[(size_t)row * n4 + c] =
         make_uint2(pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]));
 }
@@ -198,9 +246,10 @@ extern "C" int oa_ring_gemm(void* stream, const void* x, int64_t xs, const void*
     const dim3 grid((unsigned)(CEIL_DIV(items, 8) * 8)), block(256);
     float* part = splits > 1 ? (float*)scratch : nullptr;
 #define RG(BMV, ST, G, NT)                                                                         \
-    hipLaunchKernelGGL((ring_gemm_kernel<BMV, ST, G, NT>), grid, block, (ST) * (RG_N + (BMV)) * 128, s, \
-                       (const uint16_t*)x, xs, (const uint16_t*)w, (uint16_t*)out, part, M, N, K,  \
-                       mtiles, splits, (int)items, act)
+    hipLaunchKernelGGL((ring_gemm_kernel<BMV, ST, G, NT, false>), grid, block, (ST) * (RG_N + (BMV)) * 128, s, \
+                       (const char*)x, xs, (const char*)w, (const float*)nullptr,                  \
+                       (const float*)nullptr, (uint16_t*)out, part, M, N, K, mtiles, splits,       \
+                       (int)items, act)
 #define RGB(BMV, ST, NT)               \
     do {                               \
         if (gateup) RG(BMV, ST, true, NT); \
@@ -222,12 +271,48 @@ extern "C" int oa_ring_gemm(void* stream, const void* x, int64_t xs, const void*
     if (splits > 1) {
         const dim3 g(CEIL_DIV(N / 4, 256), M);
         if (gateup)
-            hipLaunchKernelGGL(ring_sum_kernel<true>, g, block, 0, s, part, (uint16_t*)out, M, N,
+            hipLaunchKernelGGL((ring_sum_kernel<true, false>), g, block, 0, s, part,
+                               (const float*)nullptr, (const float*)nullptr, (uint16_t*)out, M, N,
                                splits, act);
         else
-            hipLaunchKernelGGL(ring_sum_kernel<false>, g, block, 0, s, part, (uint16_t*)out, M, N,
+            hipLaunchKernelGGL((ring_sum_kernel<false, false>), g, block, 0, s, part,
+                               (const float*)nullptr, (const float*)nullptr, (uint16_t*)out, M, N,
                                splits, 0);
     }
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
+// out [M, N] = (x8 [M, K] w8 [N, K]^T) * xscale[m] * wscale[n]; bm as above (several row
+// tiles: 128), scratch as above
+extern "C" int oa_ring_gemm_fp8(void* stream, const void* x8, const void* xscale, const void* w8,
+                                const void* wscale, void* out, void* scratch, int M, int N, int K,
+                                int bm, int splits) {
+    if (M < 1 || M > 65535 || N < 4 || N % 4 != 0 || K < 128 || K % 128 != 0) return -100;
+    if (splits < 1 || splits > K / 128 || (splits > 1 && !scratch)) return -101;
+    if (((uintptr_t)x8 | (uintptr_t)w8 | (uintptr_t)out | (uintptr_t)scratch) % 16 != 0) return -102;
+    if ((bm != 32 && bm != 64 && bm != 96 && bm != 128) || (M > bm && bm != 128)) return -104;
+    const int mtiles = CEIL_DIV(M, bm);
+    const int64_t items = (int64_t)CEIL_DIV(N, RG_N) * mtiles * splits;
+    if (items > (1 << 28)) return -103;
+    hipStream_t s = (hipStream_t)stream;
+    float* part = splits > 1 ? (float*)scratch : nullptr;
+#define RG8(BMV, ST, NT)                                                                           \
+    hipLaunchKernelGGL((ring_gemm_kernel<BMV, ST, false, NT, true>),                               \
+                       dim3((unsigned)(CEIL_DIV(items, 8) * 8)), dim3(256),                        \
+                       (ST) * (RG_N + (BMV)) * 128, s, (const char*)x8, (int64_t)K, (const char*)w8, \
+                       (const float*)xscale, (const float*)wscale, (uint16_t*)out, part, M, N, K,  \
+                       mtiles, splits, (int)items, 0)
+    if (bm == 32) RG8(32, 6, true);
+    else if (bm == 64) RG8(64, 5, true);
+    else if (bm == 96) RG8(96, 5, true);
+    else if (mtiles == 1) RG8(128, 4, true);
+    else RG8(128, 4, false);
+#undef RG8
+    if (splits > 1)
+        hipLaunchKernelGGL((ring_sum_kernel<false, true>), dim3(CEIL_DIV(N / 4, 256), M), dim3(256), 0, s,
+                           part, (const float*)xscale, (const float*)wscale, (uint16_t*)out, M, N,
+                           splits, 0);
     HIP_CHECK_LAUNCH();
     return 0;
 }

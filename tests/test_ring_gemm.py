@@ -47,6 +47,43 @@ def test_gateup(M, N, K, tile, splits, act):
     assert ((got - f * u).abs() <= bound).all()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (9, 8, 128), (17, 132, 256), (33, 264, 1024), (64, 128, 1536), (65, 2048, 2816),
+    (128, 1000, 640), (129, 256, 2048), (200, 4096, 4096), (300, 520, 1152),
+])
+def test_fp8(M, N, K):
+    """Whole numbers and scales that are powers of two: exact sums, one rounding."""
+    torch.manual_seed(M + N + K)
+
+    def operand(rows):
+        v = torch.randint(-2, 3, (rows, K), device="cuda").float().to(torch.float8_e4m3fn)
+        return v.view(torch.uint8), torch.exp2(torch.randint(-3, 4, (rows,), device="cuda").float())
+
+    (xq, xs), (wq, ws) = operand(M), operand(N)
+    assert ops._ring_plan_fp8(M, N, K) is not None
+    got = ops._gemm_fp8(xq, xs, wq, ws)
+    xd = xq.view(torch.float8_e4m3fn).double() * xs.double()[:, None]
+    wd = wq.view(torch.float8_e4m3fn).double() * ws.double()[:, None]
+    assert torch.equal(got, (xd @ wd.T).to(torch.bfloat16))
+
+
+def test_fp8_plans():
+    for M in list(range(1, 140)) + [256, 257, 384, 700, 2048]:
+        for N in (4, 1024, 4096, 6144, 14336, 28672):
+            for K in (128, 2048, 4096, 14336):
+                plan = ops._ring_plan_fp8(M, N, K)
+                if plan:
+                    tile, splits = plan
+                    assert tile in (32, 64, 96, 128) and (M <= tile or tile == 128)
+                    assert 1 <= splits <= K // 128 and splits * M * N * 4 <= 64 << 20
+    assert ops._ring_plan_fp8(128, 4096, 14336) == (128, 8)
+    assert ops._ring_plan_fp8(512, 4096, 14336) == (128, 2)
+    assert ops._ring_plan_fp8(513, 4096, 14336) is None
+    assert ops._ring_plan_fp8(129, 28672, 4096) is None
+    assert ops._ring_plan_fp8(77, 6, 4096) is None
+
+
 def test_plans_stay_in_range():
     """Tiles cover the rows, splits have steps of their own, parts stay small."""
     for gateup in (False, True):
