@@ -332,8 +332,8 @@ def linear_fp8(
 
     GPU: M <= 8 -> fp8 weight-streaming GEMV (half the bytes of bf16);
     M <= 16 -> the same GEMV padded to the next instantiation (catch-up /
-    speculative verify passes); larger M (real prefill) -> quantize x per
-    token and run the fp8 MFMA tile GEMM. (A dequant-to-bf16 + hipBLASLt
+    speculative verify passes); larger M -> quantize x per token and run the
+    fp8 product on the transfer ring or in MFMA tiles (_gemm_fp8). (A dequant-to-bf16 + hipBLASLt
     variant was measured and REVERTED: 70B fp8 turn 723 ms vs 573 with the
     tile GEMM — the per-call dequant round-trip costs more than the GEMM's
     tile-pipeline inefficiency.)

@@ -856,11 +856,11 @@ __device__ __forceinline__ uint32_t g8_swz(int row, int byte_in_row) {
 //
 // What bounds it is what a CU draws from the L2, about 55 GB/s in every shape: two
 // blocks of two steps per CU reach 1.6 to 1.9 PFLOP/s, one block of four steps is the
-// faster form while there are no more blocks than CUs. us, the former kernel (two
-// buffers, row tiles far apart; register staging at K = 28672) / here: 28672 x 4096,
-// M = 77 53.7 / 39.3, 700 142 / 126, 2048 342 / 303; 4096 x 14336, 77 124 / 74, 700 127 /
-// 75, 2048 145 / 132; 6144 x 4096, 700 44 / 35; 4096 x 4096, 700 39 / 30; 8192 x 28672,
-// 700 583 / 217, 2048 1201 / 502. Reading the next half-step's fragments under the
+// faster form while there are no more blocks than CUs. Few tiles take the column-split
+// ring instead (ring_gemm.hip). us, the former kernel (two buffers, row tiles far apart;
+// register staging at K = 28672) / here: 28672 x 4096, M = 700 142 / 126, 2048 342 / 303;
+// 4096 x 14336, 700 127 / 75, 2048 145 / 132; 6144 x 4096, 700 44 / 35; 4096 x 4096, 700 39 /
+// 30; 8192 x 28672, 700 583 / 217, 2048 1201 / 502. Reading the next half-step's fragments under the
 // products made it slower (4096 x 14336, 700: 93).
 template <int STAGES>
 __global__ __launch_bounds__(256, 1) void gemm_fp8_ring_kernel(
