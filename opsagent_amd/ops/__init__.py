@@ -72,6 +72,14 @@ def _gemv_m_ok(M: int) -> bool:
     return M in _GEMV_MS and M <= cap
 
 
+def _two_rows_valu(M: int, N: int, K: int, gateup: bool) -> bool:
+    """Two rows that the VALU GEMV takes better than the matrix-core forms (us, VALU /
+    best of those, 2 GB of weights in turn: gate-up 2 x 14336 x 4096 39.5 / 44.0, 6144 x
+    4096 11.3 / 13.1, 32000 x 2048 25.0 / 28.5, 2048 x 2048 4.9 / 5.1), long rows (4096 x
+    14336 26.8 / 23.1) and small weights (512 x 2048 4.5 / 4.2) apart."""
+    return (M == 2 and K <= 8192 and (2 if gateup else 1) * N * K > 2 ** 20 and _gemv_m_ok(M))
+
+
 def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
     """Which form of the skinny product (skinny.hip; figures there) takes M rows
     of K columns against N (gate-up: 2N) weight rows: 0 none, 1 strips, 2
@@ -85,6 +93,8 @@ def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
     on, whose fragments are two). Under 2^18 weights every form is its launch and the
     library keeps them."""
     if M < 1 or M > 32 or K % 32 != 0 or (2 if gateup else 1) * N * K < 2 ** 18:
+        return 0
+    if _two_rows_valu(M, N, K, gateup):
         return 0
     if K == 4096 and (M <= 16 if gateup or N < 16384 else True) and (gateup or N >= 6144):
         return 2
@@ -134,7 +144,7 @@ def _ring_plan(M: int, N: int, K: int, gateup: bool = False) -> Optional[Tuple[i
     under 64 MB of weights (2048 x 8192, 128 20.7 / 16.1; 2 x 8192 x 2048, 77 18.7 in
     one, 19.8 in two); from there on a tile of 128 pays only with splits (2 x 14336 x
     4096, 58.0 / 59.5)."""
-    if not 1 < M <= 128 or K % 64 or K < 256 or N % 8:
+    if not 1 < M <= 128 or K % 64 or K < 256 or N % 8 or _two_rows_valu(M, N, K, gateup):
         return None
     weights = (2 if gateup else 1) * N * K
     if M <= 16:

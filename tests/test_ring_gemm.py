@@ -105,6 +105,8 @@ def test_plans_at_the_lines():
     assert ops._ring_plan(1, 4096, 14336) is None
     assert ops._ring_plan(8, 4096, 14336) == (32, 8)
     assert ops._ring_plan(2, 4096, 14336) is None
+    assert ops._ring_plan(2, 6144, 4096) is None and ops._skinny_form(2, 6144, 4096) == 0
+    assert ops._ring_plan(3, 6144, 4096) == (32, 5) and ops._skinny_form(2, 4096, 14336) == 1
     assert ops._ring_plan(47, 14336, 4096, True) == (64, 1)
     assert ops._ring_plan(128, 14336, 4096, True) is None
     assert ops._ring_plan(8, 14336, 4096, True) is None
