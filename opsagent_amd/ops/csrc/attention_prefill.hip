@@ -212,16 +212,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v2(
     auto stage = [&]() {
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
-            asm volatile(
-                "s_mov_b32 m0, %0\n\t"
-                "global_load_lds_dwordx4 %1, off"
-                :
-                : "s"(m0k_cur[p]), "v"(ksrc[p]));
-            asm volatile(
-                "s_mov_b32 m0, %0\n\t"
-                "global_load_lds_dwordx4 %1, off"
-                :
-                : "s"(m0v_cur[p]), "v"(vsrc[p]));
+            lds_transfer16(m0k_cur[p], ksrc[p]);
+            lds_transfer16(m0v_cur[p], vsrc[p]);
         }
     };
 
@@ -573,16 +565,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
     auto stage = [&]() {
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
-            asm volatile(
-                "s_mov_b32 m0, %0\n\t"
-                "global_load_lds_dwordx4 %1, off"
-                :
-                : "s"(m0k_cur[p]), "v"(ksrc[p]));
-            asm volatile(
-                "s_mov_b32 m0, %0\n\t"
-                "global_load_lds_dwordx4 %1, off"
-                :
-                : "s"(m0v_cur[p]), "v"(vsrc[p]));
+            lds_transfer16(m0k_cur[p], ksrc[p]);
+            lds_transfer16(m0v_cur[p], vsrc[p]);
         }
     };
     auto drain = [&]() {

@@ -59,6 +59,22 @@ __device__ __forceinline__ uint32_t silu_mul_bf16x2(uint32_t g, uint32_t u) {
                        hi / (1.0f + __expf(-hi)) * bf16_hi(u));
 }
 
+// ---- transfers into LDS -----------------------------------------------------
+// 16 bytes per lane from memory straight into LDS, at lds + 16 * lane (lds is uniform). The
+// transfer takes its address from m0, which a scalar write must precede by one wait
+// state; the compiler inserts that for its own transfers, not inside an asm string. m0
+// stays off the clobber list: the compiler keeps no value in it and warns about the name.
+// NT: read without being kept.
+template <bool NT = false>
+__device__ __forceinline__ void lds_transfer16(uint32_t lds, const char* src) {
+    if (NT)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt"
+                     : : "s"(lds), "v"(src) : "memory");
+    else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                     : : "s"(lds), "v"(src) : "memory");
+}
+
 // ---- wave reductions --------------------------------------------------------
 __device__ __forceinline__ float wave_reduce_sum(float v) {
 #pragma unroll

@@ -893,10 +893,8 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_ring_kernel(
         const uint32_t at = lds0 + buf * 2 * GTILE_B;
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off"
-                         : : "s"(at + p * 1024), "v"(asrc[p]) : "memory");
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off"
-                         : : "s"(at + GTILE_B + p * 1024), "v"(bsrc[p]) : "memory");
+            lds_transfer16(at + p * 1024, asrc[p]);
+            lds_transfer16(at + GTILE_B + p * 1024, bsrc[p]);
         }
 #pragma unroll
         for (int p = 0; p < 4; ++p) {

@@ -88,12 +88,8 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
     auto stage = [&](int buf) {
 #pragma unroll
         for (int p = 0; p < LPS; ++p) {
-            if (NT && p < 4)
-                asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off nt"
-                             : : "s"(dst[p] + buf * STEP), "v"(src[p]) : "memory");
-            else
-                asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off"
-                             : : "s"(dst[p] + buf * STEP), "v"(src[p]) : "memory");
+            if (NT && p < 4) lds_transfer16<true>(dst[p] + buf * STEP, src[p]);
+            else lds_transfer16(dst[p] + buf * STEP, src[p]);
             src[p] += 128;
         }
     };
