@@ -144,9 +144,9 @@ __global__ __launch_bounds__(256) void moe_choose_kernel(const float* __restrict
         const float best = mg_wave_max(bv);
         bi = mg_wave_all(bv == best ? bi : 0x7fffffff, [](int a, int b) { return min(a, b); });
         bv = best;
-        if (bi == 0x7fffffff) {         // no score left that compares (NaN logits)
-            bi = 0;
-            bv = 0.0f;
+        if (bi == 0x7fffffff) {         // no score left that compares: a NaN or an infinite
+            bi = 0;                     // logit makes all of a row NaN, and its weights too
+            bv = NAN;
         }
         total += bv;
         if (lane == r) {

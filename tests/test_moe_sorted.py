@@ -57,6 +57,31 @@ def test_route(T, E, top, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("E,top", [(64, 6), (5, 5), (130, 1)])
+def test_route_of_odd_rows(E, top):
+    """A NaN, an infinite or no finite logit makes a row's weights NaN, as softmax does,
+    with experts that exist; equal logits go to the lower experts."""
+    K = 256
+    gen = torch.Generator(device="cuda").manual_seed(E)
+    x = torch.randn(6, K, generator=gen, device="cuda").bfloat16()
+    rw = torch.randn(E, K, generator=gen, device="cuda") * K ** -0.5
+    rw[:, 0], rw[2, 1], x[:, :2] = 0.0, 0.0, 0.0
+    rw[2, 0], rw[3, 1] = float("nan"), float("inf")
+    bad = ops.moe_route(x, rw, top)                  # 0 * NaN: one logit of every row
+    assert torch.isnan(bad[1]).all() and (bad[0] >= 0).all() and (bad[0] < E).all()
+    rw[2, 0] = 0.0
+    x[1, 1] = 1.0                                    # one infinite logit; others 0 * inf
+    idx, wts, _ = ops.moe_route(x, rw, top)
+    assert torch.isnan(wts).all() and (idx >= 0).all() and (idx < E).all()
+    rw[3, 1] = 0.0
+    x[4], x[5, 5] = 0.0, float("nan")                # equal logits; a NaN activation
+    idx, wts, _ = ops.moe_route(x, rw, top)
+    assert torch.isfinite(wts[:5]).all() and torch.isnan(wts[5]).all()
+    assert torch.equal(idx[4].cpu(), torch.arange(top, dtype=torch.int32))
+    assert (wts[4] - 1.0 / top).abs().max() < 1e-6
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("T,E,top,H,I,act,spread", [
     (65, 8, 2, 128, 128, None, "even"),             # one K step, one strip
