@@ -779,7 +779,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
 }
 
 // Splits added up: one wave per (query, head) row, two channels per lane. rows = B * Sq
-// * Hq; scale2 turns a difference of maxima into a power of two.
+// * Hq; scale2 turns a difference of maxima into a power of two. A split without a visible
+// key has weight sum 0; one with a NaN or an infinite score has a NaN sum, and counts.
 __global__ __launch_bounds__(256) void prefill_combine_kernel(const float* __restrict__ po,
                                                               const float* __restrict__ pml,
                                                               uint32_t* __restrict__ out, int rows,
@@ -789,13 +790,13 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const float* __res
     float mx = -INFINITY;
     for (int s = 0; s < nsplit; ++s) {
         const float2 ml = *reinterpret_cast<const float2*>(pml + ((size_t)s * rows + row) * 2);
-        if (ml.y > 0.0f) mx = fmaxf(mx, ml.x);
+        if (ml.y != 0.0f) mx = fmaxf(mx, ml.x);
     }
     float l = 0.0f, a = 0.0f, b = 0.0f;
     for (int s = 0; s < nsplit; ++s) {
         const size_t r = (size_t)s * rows + row;
         const float2 ml = *reinterpret_cast<const float2*>(pml + r * 2);
-        if (ml.y > 0.0f) {
+        if (ml.y != 0.0f) {
             const float w = __builtin_amdgcn_exp2f((ml.x - mx) * scale2);
             const float2 o = *reinterpret_cast<const float2*>(po + r * DHEAD + lane * 2);
             l = fmaf(ml.y, w, l);

@@ -45,6 +45,25 @@ def test_split_prefill(B, Hq, Hk, Sq, Skv):
             assert err < 6e-3, (b, h, float(err))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hk,Sq,Skv", [(8, 2, 40, 900), (8, 2, 300, 1600), (8, 4, 300, 1600)])
+def test_scores_that_do_not_compare(Hq, Hk, Sq, Skv):
+    """A row with a NaN or a positive infinite score is NaN, as softmax makes it, in
+    whichever split the score lies; a negative infinite score is a weight of zero."""
+    assert ops._prefill_splits(1, Hq, Hk, Sq, Skv)[0] > 1
+    gen = torch.Generator(device="cuda").manual_seed(Sq)
+    q = torch.randn(1, Sq, Hq, D, generator=gen, device="cuda").bfloat16()
+    k, v = (torch.randn(1, Skv, Hk, D, generator=gen, device="cuda").bfloat16() for _ in range(2))
+    q[0, 3, 1, 5] = float("nan")
+    k[0, 200, 0, 7] = float("inf")                   # every row sees key 200 of key head 0
+    v[0, 500, 1, 9] = float("nan")                   # one channel, of key head 1's rows
+    bad = torch.zeros(1, Sq, Hq, D, dtype=torch.bool, device="cuda")
+    bad[0, 3, 1] = True
+    bad[0, :, : Hq // Hk] |= (q[0, :, : Hq // Hk, 7] > 0)[..., None]
+    bad[0, :, Hq // Hk : 2 * (Hq // Hk), 9] = True
+    assert torch.equal(torch.isnan(ops.attention_prefill(q, k, v)), bad)
+
+
 def test_rule():
     split = ops._prefill_splits
     assert split(1, 32, 8, 77, 1264) == (8, False) and split(1, 32, 8, 128, 256) == (1, False)
