@@ -92,11 +92,14 @@ class MoEMLP(nn.Module):
         T, H = x.shape
         w13, w2 = (self.w13_q, self.w2_q) if self.fp8 else (self.w13, self.w2)
         s13, s2 = (self.w13_s, self.w2_s) if self.fp8 else (None, None)
-        if not self._force_loop and ops.moe_route_ok(x, self.router_w, self.top_k):
+        if x.is_cuda and x.dtype == torch.bfloat16 and not self._force_loop:
             # static shapes, no host sync: such a step can be captured. A loop
             # over the experts measured 25.0 ms for 512 tokens x 4 layers (64
             # experts of 1408, top 6) against 1.9 ms, most of it launches and the
             # host's wait for the counts.
+            x = x.contiguous()
+            if x.data_ptr() % 16:                        # whole 16-byte pieces are read
+                x = x.clone()
             P = T * self.top_k
             few = T <= 64 or (decode and P <= 2048)      # the pair kernels' range
             tiles = ops.moe_sorted_ok(x, w13, w2)

@@ -534,7 +534,7 @@ def _moe_act(act):
 
 
 def moe_route_ok(x: torch.Tensor, router_w: torch.Tensor, top: int) -> bool:
-    """Whether moe_route takes this router: eight-channel rows for moe_combine."""
+    """Whether the routing kernels take this router."""
     E, K = router_w.shape
     return (
         x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
@@ -547,9 +547,15 @@ def moe_route_ok(x: torch.Tensor, router_w: torch.Tensor, top: int) -> bool:
 def moe_route(x: torch.Tensor, router_w: torch.Tensor, top: int):
     """Softmax routing of bf16 rows x [T, K] by float32 router_w [E, K]: experts
     int32, weights float32 (normalised over the chosen) and tokens int32, each
-    [T, top]."""
+    [T, top]. Static shapes and no host sync in either form: routers that the kernels do
+    not take go through the library."""
     T, K = x.shape
     E = router_w.shape[0]
+    if not moe_route_ok(x, router_w, top):
+        probs = torch.softmax(torch.nn.functional.linear(x.float(), router_w), dim=-1)
+        wts, idx = probs.topk(top, dim=-1)
+        tok = torch.arange(T, device=x.device, dtype=torch.int32)[:, None].expand(T, top)
+        return idx.int(), wts / wts.sum(dim=-1, keepdim=True), tok.contiguous()
     lib, hip = _lib()
     idx, tok = torch.empty(2, T, top, dtype=torch.int32, device=x.device)
     wts = torch.empty(T, top, dtype=torch.float32, device=x.device)

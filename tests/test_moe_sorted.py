@@ -127,6 +127,49 @@ def test_sorted_experts(fp8, T, E, top, H, I, act, spread):
 
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,top,T,form", [
+    (1030, 6, 3, "plain"),        # more experts than the routing kernels hold
+    (96, 65, 2, "plain"),         # more choices than a wave has lanes
+    (16, 4, 5, "strided"), (16, 4, 70, "strided"),
+    (16, 4, 5, "offset"),         # rows that start off 16 bytes
+])
+def test_layer_without_host_waits(E, top, T, form):
+    """What a decode step may hold runs without waiting for the GPU, as a captured step
+    has to, whatever the input's strides and the router's size."""
+    from opsagent_amd.engine.config import ModelSpec
+    from opsagent_amd.engine.moe import MoEMLP
+    from opsagent_amd.parallel import state
+
+    state.set_tp_state(0, 1, None)
+    H, I = 256, 128
+    spec = ModelSpec(name="moe", max_seq_len=64, hidden_size=H, num_heads=2, num_kv_heads=2,
+                     head_dim=128, intermediate_size=256, num_layers=1, vocab_size=64,
+                     moe_num_experts=E, moe_top_k=top, moe_intermediate_size=I,
+                     moe_shared_experts=0, moe_dtype="bf16")
+    moe = MoEMLP(spec, torch.bfloat16, torch.Generator(device="cuda").manual_seed(E)).to("cuda")
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(T, 2 * H, generator=gen, device="cuda").bfloat16()
+    if form == "strided":
+        x = x[:, H:]
+    elif form == "offset":
+        x = x.flatten()[1 : 1 + T * H].view(T, H)
+    else:
+        x = x[:, :H].contiguous()
+    moe(x)
+    torch.cuda.synchronize()
+    torch.cuda.set_sync_debug_mode("error")
+    try:
+        got = moe(x, decode=True)
+    finally:
+        torch.cuda.set_sync_debug_mode("default")
+    score, idx = torch.softmax(x.double() @ moe.router_w.double().T, -1).topk(top, -1)
+    wts = score / score.sum(-1, keepdim=True)
+    want = _reference(x, moe.w13, moe.w2, idx, wts, None, None)
+    # the roundings of test_sorted_experts
+    assert float((got.double() - want).norm() / want.norm()) < 4e-3
+
+
 def test_sorted_experts_refuse():
     """CPU tensors and activations that the kernels do not have stay on the
     general path."""
