@@ -35,8 +35,7 @@ __all__ = [
 rope_cos_sin = torch_ref.rope_cos_sin
 
 # VALU-gemv M instantiations (the dot-per-lane form; measured crossover
-# notes below). Batched decode M 3..8 rides the MFMA gemv instead
-# (_bf16_mfma_ok); M > 8 bf16 stays on hipBLASLt.
+# notes below). More rows go to the matrix-core forms (linear).
 _GEMV_MS = frozenset(range(1, 9))
 
 # Measured crossover vs hipBLASLt (concurrent bench, within-box A/B):
@@ -72,12 +71,12 @@ def _gemv_m_ok(M: int) -> bool:
     return M in _GEMV_MS and M <= cap
 
 
-def _two_rows_valu(M: int, N: int, K: int, gateup: bool) -> bool:
+def _two_rows_valu(M: int, K: int) -> bool:
     """Two rows that the VALU GEMV takes better than the matrix-core forms (us, VALU /
-    best of those, 2 GB of weights in turn: gate-up 2 x 14336 x 4096 39.5 / 44.0, 6144 x
-    4096 11.3 / 13.1, 32000 x 2048 25.0 / 28.5, 2048 x 2048 4.9 / 5.1), long rows (4096 x
-    14336 26.8 / 23.1) and small weights (512 x 2048 4.5 / 4.2) apart."""
-    return (M == 2 and K <= 8192 and (2 if gateup else 1) * N * K > 2 ** 20 and _gemv_m_ok(M))
+    best of those, 2 GB of weights in turn: gate-up 2 x 14336 x 4096 41.1 / 45.3, 6144 x
+    4096 10.7 / 12.7, 5120 x 5120 10.7 / 13.5, 32000 x 2048 25.1 / 26.0, 4096 x 4096 8.5 /
+    8.2), long rows (4096 x 14336 26.6 / 23.0) apart."""
+    return M == 2 and K <= 8192 and _gemv_m_ok(M)
 
 
 def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
@@ -85,22 +84,41 @@ def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
     of K columns against N (gate-up: 2N) weight rows: 0 none, 1 strips, 2
     persistent.
 
-    The persistent form pays where a block goes over several strips: gate-up and
-    N >= 6144 up to 16 rows, N >= 16384 up to 32. A strip block reads all of x from
-    the L2, which costs 0.6 of the time that so many weight bytes take; the library
-    starts 3.5 us later and streams 0.87 as fast, so strips win while their x
-    traffic is under 35 MB + a quarter of the weight (25 MB + a fifth from 17 rows
-    on, whose fragments are two). Under 2^18 weights every form is its launch and the
-    library keeps them."""
-    if M < 1 or M > 32 or K % 32 != 0 or (2 if gateup else 1) * N * K < 2 ** 18:
+    Strips: a block of 16 weight rows (gate-up: 32) takes a time of its own per column
+    and row of x, blocks of one CU add up, and past 4.75 TB/s memory bounds all of them;
+    measured over 64 weights this holds to a tenth. The library's best times over the same
+    weights are 5 us + its bytes at 5.9 TB/s (gate-up with its activation 7.3 and 5.4), and
+    no less than `least`, which falls where its kernels split K. Strips take what
+    they finish sooner: 4096 x 4096, M = 16 10.6 against 15.5 and 32 15.2 against 13.3;
+    1024 x 4096, 32 14.4 / 11.8; 5120 x 13824, 3 39.1 / 28.4. Up to eight rows the staged
+    GEMV is the other form where it runs, and strips are the faster one (12288 x 6144, 8
+    35.0 / 41.2), except for rows too short to pipeline, four steps a wave, in more than
+    one round (32000 x 1024, 8 19.9 / 16.0; the library 17.2). The persistent form is for
+    blocks that go over several strips: gate-up from N = 8192 on (2 x 11008, 8 36.2 / 38.4;
+    2 x 3584 16.5 / 13.8) and N >= 6144 up to 16 rows, N >= 16384 up to 32. Under 2^18
+    weights every form is one launch of 3 to 5 us and the library keeps them."""
+    R = 2 if gateup else 1
+    if M < 1 or M > 32 or K % 32 != 0 or R * N * K < 2 ** 18 or _two_rows_valu(M, K):
         return 0
-    if _two_rows_valu(M, N, K, gateup):
-        return 0
-    if K == 4096 and (M <= 16 if gateup or N < 16384 else True) and (gateup or N >= 6144):
+    if K == 4096 and (M <= 16 and N >= 8192 if gateup else N >= (6144 if M <= 16 else 16384)):
         return 2
-    weight = (2 if gateup else 1) * N * K * 2e-6
-    traffic = ((N + 15) // 16) * M * K * 2e-6
-    return int(traffic < (35 + 0.25 * weight if M <= 16 else 25 + 0.2 * weight))
+    blocks = -(-N // 16)
+    if K < 2048 and not gateup and blocks > (256 if M <= 8 else 512):
+        return 0
+    if M > 2 and _bf16_mfma_ok(M, K, gateup):
+        return 1
+    if M <= 16:
+        col = (2.5 + 0.06 * M) if gateup else (1.3 + 0.05 * M)
+    else:
+        col = (2.9 + 0.06 * M) if gateup else (1.6 + 0.045 * M)
+    mb = R * N * K * 2e-6
+    strips = max(1.8 + -(-blocks // 256) * K / 1024 * col, mb / (5.0 if M > 2 else 4.75))
+    if gateup:
+        library = max(17.6 if K >= 4096 and M <= 24 else 13.5, 7.3 + mb / 5.4)
+    else:
+        least = 10.4 if M <= 16 else 8.4 if M > 24 else 12.6 if K >= 4096 else 11.5
+        library = max(least, 5 + mb / 5.9)
+    return int(strips < library)
 
 
 def _skinny_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -131,36 +149,63 @@ def _ring_plan(M: int, N: int, K: int, gateup: bool = False) -> Optional[Tuple[i
     (ring_gemm.hip; figures there) of M rows of K columns against N (gate-up: 2N)
     weight rows, None where the other forms are faster.
 
-    The lines, measured at 2 to 128 rows over 12 weights, 2 GB of them in turn (us,
+    The lines, measured at 2 to 128 rows over 64 weights, 2 GB of them in turn (us,
     other / ring): light weights end before the ring pays for its start (4096 x 4096,
-    M = 8 10.3 / 10.9, 24 13.4 / 11.7; gate-up 2 x 2816 x 2048, 24 10.6 / 10.7, 47
-    15.4 / 12.8), short rows at few rows too (2 x 8192 x 2048, 8 15.1 / 15.3, 24 20.4
-    / 14.9), long ones less (2048 x 8192, 8 15.2 / 11.7). Column splits fill the CUs;
-    less than 0.8 of the last round filled loses (12288 x 4096, 24 22.7 / 25.0), and
-    at two or three rows so does adding up many splits (4096 x 14336, 2 21.8 / 23.0).
+    M = 8 9.1 / 10.8, 24 13.4 / 11.7; gate-up 2 x 2816 x 2048, 24 10.6 / 10.7, 47
+    15.4 / 12.8, 112 16.7 / 17.8), short rows at few rows too (2 x 8192 x 2048, 8 14.5 /
+    14.7; 2 x 8192 x 3072 23.0 / 20.3), long ones less (2048 x 8192, 8 12.6 / 11.3).
+    Column splits fill the CUs; less than 0.8 of the last round filled loses (12288 x
+    4096, 24 22.7 / 25.0), and at two or three rows so does adding up many splits (4096 x
+    14336, 2 21.8 / 23.0). Runs of a multiple of 2048 columns, 4 KiB, keep all blocks on
+    the same channels: twice as many splits mend it up to 32 rows (16384 x 4096, M = 8, the
+    library 31.5, two splits 32.9, four 26.4; 8192 x 8192 29.3, 31.5, 25.8); above and for
+    gate-up the library is faster on weights of no fewer rows than columns (2 x 4096 x
+    8192, 8 31.6 / 33.0, four or eight splits; 8192 x 8192, 64 32.8 / 35.2; but 128 48.2 /
+    41.2, 4096 x 16384, 64 41.7 / 38.1). It also is for many rows on short wide weights
+    that need splits (8192 x 2048, 48 14.0 / 14.2; 8192 x 3072, 48 18.8 / 17.1, 80 19.7 /
+    20.9).
     Up to 16 rows of 4096 the persistent skinny form is the better one where no
-    split is needed (2 x 14336, 8 45.1 / 46.3), under eight shorter rows the strips
-    (32000 x 2048, 4 26.6 / 29.4). Two tiles of 64 rows beat a tile of 96 or 128
-    under 64 MB of weights (2048 x 8192, 128 20.7 / 16.1; 2 x 8192 x 2048, 77 18.7 in
-    one, 19.8 in two); from there on a tile of 128 pays only with splits (2 x 14336 x
-    4096, 58.0 / 59.5)."""
-    if not 1 < M <= 128 or K % 64 or K < 256 or N % 8 or _two_rows_valu(M, N, K, gateup):
+    split is needed (2 x 14336, 8 45.2 / 45.4), under eight shorter rows the strips
+    (32000 x 2048, 4 26.6 / 29.4). Two tiles of 64 rows beat a tile of 128 under 64 MB of
+    weights and one of 96 under 32 MB (2048 x 8192, 80 16.7 / 15.9, 128 20.7 / 16.1; 2 x
+    3584 x 4096, 80 21.0 in one, 23.0 in two), as long as both read a strip in the same
+    round (32000 x 1024, 112 24.2 / 25.4). Without splits tiles of 96 pay in one round or
+    from rows of 4096 on (128256 x 2048, 96 130 / 132, 32000 x 2048 32.5 / 30.8, 128256 x
+    4096 228 / 225), tiles of 128 not at all (2 x 14336 x 4096, 58.0 / 59.5)."""
+    if not 1 < M <= 128 or K % 64 or K < 256 or N % 8 or _two_rows_valu(M, K):
         return None
     weights = (2 if gateup else 1) * N * K
     if M <= 16:
-        ok = (weights >= (2 ** 24 if K >= 8192 else 24e6 if K >= 4096 else 60e6))
+        ok = weights >= (2 ** 24 if K >= 8192 else 24e6 if K >= 4096 else 40e6 if K >= 3072 else 60e6)
     else:
-        ok = weights >= (10e6 if gateup and M > 32 else 2 ** 24)
+        ok = weights >= (10e6 if gateup and 32 < M <= 80 else 2 ** 24)
     if not ok:
         return None
     strips = -(-N // (64 if gateup else 128))
-    for tile in (64, 32 * -(-M // 32)) if M > 64 and weights < 2 ** 25 else (32 * -(-M // 32),):
+    one = 32 * -(-M // 32)
+    two = M > 64 and weights < (2 ** 25 if M > 96 else 2 ** 24 + 1)
+    for tile in (64, one) if two else (one,):
         tiles = strips * -(-M // tile)
         splits = max(1, min(256 // tiles, K // 256))
         blocks = tiles * splits
-        if (blocks >= 0.8 * 256 * -(-blocks // 256) and (M >= 4 or splits <= 5)
-                and not (splits == 1 and (tile == 128 or M <= 16 and K == 4096 or M < 8 and K < 4096))):
-            return tile, splits
+        if blocks < 0.8 * 256 * -(-blocks // 256):
+            continue
+        if splits == 1:
+            if tile == 128 or M <= 16 and K == 4096 or M < 8 and K < 4096:
+                continue
+            if blocks > 256 and M > 64 and (K < 4096 or tile == 64):
+                continue
+        else:
+            if not gateup and (M > 64 and 2 * K < N or M > 40 and 3 * K < N):
+                continue
+            if K % (splits * 2048) == 0:
+                if M <= 32 and not gateup:
+                    splits *= 2
+                elif weights >= K * K and M < (113 if gateup else 96):
+                    continue
+            if M < 4 and splits > 5:
+                continue
+        return tile, splits
     return None
 
 
@@ -184,8 +229,8 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear with custom HIP paths for decode shapes: the VALU GEMV at M = 1
     (hipBLASLt's M=1 kernels run ~2.5x off the HBM roofline on gfx950), the transfer
     ring up to 128 rows and the skinny matrix-core products up to 32 where they win
-    (_ring_plan, _skinny_form), the VALU GEMV for what two rows are left; everything
-    else goes to hipBLASLt."""
+    (_ring_plan, _skinny_form), the VALU GEMV for what two rows are left and the
+    matrix-core GEMV for what 3 to 8 are; everything else goes to hipBLASLt."""
     M = x.numel() // x.shape[-1]
     if 1 < M <= 128 and _skinny_ok(x, w):
         plan = _ring_plan(M, w.shape[0], w.shape[1])
@@ -197,7 +242,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if (
         x.is_cuda
         and x.dtype == torch.bfloat16
-        and _gemv_m_ok(M)
+        and (_gemv_m_ok(M) or _bf16_mfma_ok(M, x.shape[-1]))
         and x.shape[-1] % 8 == 0
         and w.stride(1) == 1
         and x.is_contiguous()

@@ -114,3 +114,48 @@ def test_plans_at_the_lines():
     assert ops._ring_plan(8, 4096, 4096) is None
     assert ops._ring_plan(32, 12288, 4096) is None
     assert ops._ring_plan(129, 4096, 14336) is None
+
+
+def test_lines_between_the_forms():
+    """Shapes on both sides of the lines at _ring_plan and _skinny_form, among them those
+    where a form would be slower than the one it replaced."""
+    def forms(M, N, K, gateup=False):
+        return ops._ring_plan(M, N, K, gateup), ops._skinny_form(M, N, K, gateup)
+
+    # runs of a multiple of 4 KiB: twice the splits, or the library
+    assert ops._ring_plan(8, 16384, 4096) == (32, 4) and ops._ring_plan(8, 8192, 8192) == (32, 8)
+    assert ops._ring_plan(64, 8192, 8192) is None and ops._ring_plan(128, 8192, 8192) == (128, 4)
+    assert ops._ring_plan(64, 4096, 16384) == (64, 8)
+    assert ops._ring_plan(24, 4096, 8192, True) is None and forms(8, 4096, 8192, True) == (None, 1)
+    # short wide weights and many rows
+    assert ops._ring_plan(48, 8192, 2048) is None and ops._ring_plan(48, 8192, 3072) == (64, 4)
+    assert ops._ring_plan(80, 8192, 3072) is None and ops._ring_plan(80, 16384, 1024) == (64, 1)
+    assert ops._ring_plan(96, 32000, 1024) == (96, 1) and ops._ring_plan(112, 32000, 1024) is None
+    assert ops._ring_plan(96, 128256, 2048) is None and ops._ring_plan(96, 128256, 4096) == (96, 1)
+    assert ops._ring_plan(80, 5120, 5120) == (96, 6) and ops._ring_plan(112, 5120, 5120) == (64, 3)
+    assert ops._ring_plan(80, 2816, 2048, True) == (96, 5)
+    assert ops._ring_plan(112, 2816, 2048, True) is None
+    # few strips or long ones: the library; short rows in many rounds: the staged GEMV
+    assert forms(3, 5120, 13824) == (None, 0) and forms(2, 5120, 13824) == (None, 0)
+    assert forms(32, 1024, 4096) == (None, 0) and forms(16, 2048, 5632) == (None, 0)
+    assert forms(32, 1024, 4096, True) == (None, 0) and forms(4, 1024, 4096, True) == (None, 1)
+    assert forms(8, 32000, 1024) == (None, 0) and ops._bf16_mfma_ok(8, 1024)
+    assert forms(9, 16384, 1024) == (None, 0) and forms(9, 8192, 1024) == (None, 1)
+    # three to eight rows that found no form
+    assert forms(8, 12288, 6144) == forms(8, 18432, 5120) == (None, 1)
+    assert forms(7, 128256, 2048) == (None, 1)
+    assert forms(8, 18432, 7168, True) == (None, 0)
+    for N, K, gateup in ((512, 1024, True), (18432, 5120, False), (256, 2048, False)):
+        assert forms(2, N, K, gateup) == (None, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(3, 16384, 1024), (8, 16400, 1024), (8, 8192, 8192),
+                                   (32, 4096, 16384), (8, 18432, 5120), (64, 4096, 16384)])
+def test_lines_agree(M, N, K):
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K, generator=gen, device="cuda").bfloat16()
+    w = (torch.randn(N, K, generator=gen, device="cuda") * K ** -0.5).bfloat16()
+    want = x.double() @ w.double().T
+    # one bf16 rounding of a float32 sum: 0.0016 in the mean
+    assert float((ops.linear(x, w).double() - want).norm() / want.norm()) < 2e-3
