@@ -244,13 +244,12 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         and x.dtype == torch.bfloat16
         and (_gemv_m_ok(M) or _bf16_mfma_ok(M, x.shape[-1]))
         and x.shape[-1] % 8 == 0
-        and w.stride(1) == 1
+        # the kernels read whole rows one after the other, 16 bytes at a time: a
+        # column slice of a wider buffer has gaps and may start anywhere
+        and w.is_contiguous()
         and x.is_contiguous()
-        # the kernels read 16 bytes at a time: a column slice of a wider
-        # buffer may start anywhere
         and x.data_ptr() % 16 == 0
         and w.data_ptr() % 16 == 0
-        and w.stride(0) % 8 == 0
     ):
         from opsagent_amd.ops import hip_lib
 
@@ -504,7 +503,7 @@ def linear_norm(
     if (
         x.is_cuda and x.dtype == torch.bfloat16
         and (_gemv_m_ok(M) or _bf16_mfma_ok(M, x.shape[-1]))
-        and x.shape[-1] % 8 == 0 and x.is_contiguous()
+        and x.shape[-1] % 8 == 0 and x.is_contiguous() and w.is_contiguous()
     ):
         from opsagent_amd.ops import hip_lib
 
@@ -526,7 +525,8 @@ def linear_addres(x: torch.Tensor, w: torch.Tensor, res: torch.Tensor) -> torch.
     if (
         x.is_cuda and x.dtype == torch.bfloat16
         and (_gemv_m_ok(M) or _bf16_mfma_ok(M, x.shape[-1]))
-        and x.shape[-1] % 8 == 0 and x.is_contiguous() and res.is_contiguous()
+        and x.shape[-1] % 8 == 0 and x.is_contiguous() and w.is_contiguous()
+        and res.is_contiguous()
     ):
         from opsagent_amd.ops import hip_lib
 
@@ -553,7 +553,7 @@ def gateup_silu_norm(
     if (
         x.is_cuda and x.dtype == torch.bfloat16
         and (_gemv_m_ok(M) or _bf16_mfma_ok(M, x.shape[-1]))
-        and x.shape[-1] % 8 == 0 and x.is_contiguous()
+        and x.shape[-1] % 8 == 0 and x.is_contiguous() and gate_up_w.is_contiguous()
     ):
         from opsagent_amd.ops import hip_lib
 
@@ -833,7 +833,8 @@ def gateup_fused(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> bool
     two rows, the transfer ring and the skinny matrix-core product where they win."""
     M, K = x.numel() // x.shape[-1], x.shape[-1]
     return (
-        x.is_cuda and x.dtype == torch.bfloat16 and x.shape[-1] % 8 == 0 and x.is_contiguous()
+        x.is_cuda and x.dtype == torch.bfloat16 and K % 8 == 0 and x.is_contiguous()
+        and gate_up_w.is_contiguous()
         and (_gemv_m_ok(M) or (_skinny_ok(x, gate_up_w)
                                and (_ring_plan(M, i_local, K, gateup=True) is not None
                                     or _skinny_form(M, i_local, K, gateup=True) > 0)))

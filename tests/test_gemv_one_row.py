@@ -35,3 +35,31 @@ def test_one_row(N, K):
         check(ops.gateup_act(x, w, h, "silu"), g * torch.sigmoid(g) * u)
         check(ops.gateup_act(x, w, h, "gelu_tanh"),
               torch.nn.functional.gelu(g, approximate="tanh") * u)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 4])
+@pytest.mark.parametrize("N,K", [(96, 512), (96, 2048)])
+def test_weights_with_gaps(M, N, K):
+    """Weight rows that lie further apart than they are long, in every entry point."""
+    gen = torch.Generator(device="cuda").manual_seed(M + K)
+    rn = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    x, res = rn(M, K).bfloat16(), rn(M, N).bfloat16()
+    w = (rn(N, K + 64) * K ** -0.5).bfloat16()[:, :K]
+    nw = (1.0 + 0.1 * rn(K)).bfloat16()
+    xd, wd = x.double(), w.double()
+    normed = xd / torch.sqrt((xd * xd).mean(-1, keepdim=True) + 1e-5) * nw.double()
+
+    def check(got, want):
+        # roundings of the normed row, of both halves (twofold in silu) and of the result
+        assert float((got.double() - want).norm() / want.norm()) < 8e-3
+
+    def silu_halves(y):
+        g, u = y.chunk(2, -1)
+        return g * torch.sigmoid(g) * u
+
+    check(ops.linear(x, w), xd @ wd.T)
+    check(ops.linear_norm(x, nw, 1e-5, w), normed @ wd.T)
+    check(ops.linear_addres(x, w, res), xd @ wd.T + res.double())
+    check(ops.gateup_silu(x, w, N // 2), silu_halves(xd @ wd.T))
+    check(ops.gateup_silu_norm(x, nw, 1e-5, w, N // 2), silu_halves(normed @ wd.T))
