@@ -71,6 +71,12 @@ def _gemv_m_ok(M: int) -> bool:
     return M in _GEMV_MS and M <= cap
 
 
+def _gemv_switched() -> bool:
+    """OPSAGENT_BF16_GEMV_MFMA or OPSAGENT_GEMV_MAX_M is set: the two choose between the
+    staged GEMVs and the library, and the newer forms step aside for both."""
+    return "OPSAGENT_BF16_GEMV_MFMA" in os.environ or "OPSAGENT_GEMV_MAX_M" in os.environ
+
+
 def _two_rows_valu(M: int, K: int) -> bool:
     """Two rows that the VALU GEMV takes better than the matrix-core forms (us, VALU /
     best of those, 2 GB of weights in turn: gate-up 2 x 14336 x 4096 41.1 / 45.3, 6144 x
@@ -122,13 +128,14 @@ def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
 
 
 def _skinny_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """16-byte loads of the rows of both operands."""
+    """16-byte loads of the rows of both operands, and no switch that asks for other
+    forms."""
     return (
         x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
         and w.dim() == 2 and w.is_contiguous() and x.dim() >= 1 and x.shape[-1] == w.shape[1]
         and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1
                                    and x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0))
-        and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+        and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and not _gemv_switched()
     )
 
 
@@ -830,14 +837,16 @@ def gateup_silu(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> torch
 
 def gateup_fused(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> bool:
     """Whether gateup_act takes this product in one launch: the VALU GEMV up to
-    two rows, the transfer ring and the skinny matrix-core product where they win."""
+    two rows, the transfer ring and the skinny matrix-core product where they win, the
+    staged matrix-core GEMV for what 3 to 8 rows are left."""
     M, K = x.numel() // x.shape[-1], x.shape[-1]
     return (
         x.is_cuda and x.dtype == torch.bfloat16 and K % 8 == 0 and x.is_contiguous()
         and gate_up_w.is_contiguous()
-        and (_gemv_m_ok(M) or (_skinny_ok(x, gate_up_w)
-                               and (_ring_plan(M, i_local, K, gateup=True) is not None
-                                    or _skinny_form(M, i_local, K, gateup=True) > 0)))
+        and (_gemv_m_ok(M) or _bf16_mfma_ok(M, K, gateup=True)
+             or (_skinny_ok(x, gate_up_w)
+                 and (_ring_plan(M, i_local, K, gateup=True) is not None
+                      or _skinny_form(M, i_local, K, gateup=True) > 0)))
     )
 
 

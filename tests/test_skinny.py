@@ -77,3 +77,27 @@ def test_rule():
     assert form(8, 64, 1000) == 0                             # K not a multiple of 32
     x, w = torch.zeros(4, 64, dtype=torch.bfloat16), torch.zeros(8, 64, dtype=torch.bfloat16)
     assert not ops._skinny_ok(x, w)                           # CPU tensors: the general path
+
+
+@pytest.mark.gpu
+def test_switches(monkeypatch):
+    """The two switches choose between the staged GEMVs and the library, whatever the
+    newer forms would take."""
+    from opsagent_amd.ops import hip_lib
+
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(8, 4096, generator=gen, device="cuda").bfloat16()
+    w = (torch.randn(6144, 4096, generator=gen, device="cuda") * 2.0 ** -6).bfloat16()
+    assert ops._ring_plan(8, 6144, 4096) and ops._skinny_ok(x, w)
+    staged = torch.empty(8, 6144, dtype=x.dtype, device="cuda")
+    hip_lib.check(hip_lib.get_lib().oa_gemv_ex(hip_lib.current_stream_ptr(), x.data_ptr(), w.data_ptr(),
+                                               staged.data_ptr(), None, None, 8, 6144, 4096, 0.0, 0), "")
+    library = torch.nn.functional.linear(x, w)
+    monkeypatch.setenv("OPSAGENT_BF16_GEMV_MFMA", "m2")
+    assert not ops._skinny_ok(x, w) and torch.equal(ops.linear(x, w), staged)
+    assert ops.gateup_fused(x, w, 3072)
+    monkeypatch.setenv("OPSAGENT_BF16_GEMV_MFMA", "0")
+    assert torch.equal(ops.linear(x, w), library) and not ops.gateup_fused(x, w, 3072)
+    monkeypatch.delenv("OPSAGENT_BF16_GEMV_MFMA")
+    monkeypatch.setenv("OPSAGENT_GEMV_MAX_M", "1")
+    assert torch.equal(ops.linear(x[:2], w), torch.nn.functional.linear(x[:2], w))
