@@ -492,26 +492,27 @@ static bool gemv_fp8_use_mfma(int M, int rows, int K, int gateup) {
 // kernel (gemv.hip) on fp8 weights. The block's activations, normalised there with NORM,
 // are a float32 image in LDS, made once while the first weights are under way, four
 // planes of four columns in sixteen so that a wave's 16-byte reads are contiguous; a wave
-// streams the rows of its units two at a time (GU: a gate row and its up row) in groups
+// streams the rows of its units, every waves-th of the weight, two at a time (GU: a gate
+// row and its up row) in groups
 // of GR 1024-column chunks, the next group under way while one is in use. us inside a
 // decode step, the forms above with their normalisation in a launch of its own / here:
 // gate-up 2 x 14336 x 4096 27.4 / 21.9, 6144 x 4096 11.1 / 7.8, 4096 x 14336 13.5 / 12.1;
 // asking for the activations before the weights is 3 us of the normalised ones. A third
 // group under way from the start cost more in waits than it hid (gate-up 27.6), seven
 // chunks a group too (4096 x 14336 14.0).
-template <bool NORM, bool ADDRES, bool GU, int GR, int XV>
-__global__ __launch_bounds__(512) void gemv1_fp8_kernel(
+template <bool NORM, bool ADDRES, bool GU, int GR, int XV, int WV>
+__global__ __launch_bounds__(WV * 64) void gemv1_fp8_kernel(
     const uint4* __restrict__ x, const uint32_t* __restrict__ w8, const float* __restrict__ wscale,
     uint16_t* __restrict__ out, const uint4* __restrict__ wn, const uint16_t* __restrict__ res,
-    int N, int K, int per, float eps) {
+    int N, int K, int waves, int full, int extra, float eps) {
     extern __shared__ __attribute__((aligned(16))) float xl[];   // [4][K / 4]
     __shared__ float part[8];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int units = GU ? N : N / 2;
-    const int u0 = (blockIdx.x * 8 + wid) * per, u1 = min(u0 + per, units);
+    const int u0 = blockIdx.x * WV + wid;
     const int k4 = K / 4, groups = K / (1024 * GR);
-    const int total = max(u1 - u0, 0) * groups;
+    const int total = (full + (u0 < extra)) * groups;       // of every waves-th unit
     auto row_of = [&](int u, int t) { return GU ? u + t * N : u * 2 + t; };
     u32x4 a[GR][2], b[GR][2];
     int u = min(u0, units - 1), g = 0;                      // of the group loaded last
@@ -525,7 +526,7 @@ __global__ __launch_bounds__(512) void gemv1_fp8_kernel(
     auto next = [&](u32x4 (&v)[GR][2]) {
         if (++g == groups) {
             g = 0;
-            ++u;
+            u += waves;
         }
         load(v);
         __builtin_amdgcn_sched_barrier(0);
@@ -536,13 +537,13 @@ __global__ __launch_bounds__(512) void gemv1_fp8_kernel(
     uint4 xv[XV], nv[XV];
 #pragma unroll
     for (int j = 0; j < XV; ++j) {
-        const int i = min(j * 512 + tid, K / 8 - 1);
+        const int i = min(j * WV * 64 + tid, K / 8 - 1);
         xv[j] = x[i];
         if (NORM) nv[j] = wn[i];
     }
     float sc[2], rs[2] = {0.0f, 0.0f};
     {
-        const int mine = min(u0 + lane, units - 1);
+        const int mine = (int)min(u0 + lane * (int64_t)waves, units - (int64_t)1);
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             sc[t] = wscale[row_of(mine, t)];
@@ -555,27 +556,32 @@ __global__ __launch_bounds__(512) void gemv1_fp8_kernel(
 
     float rstd = 1.0f;
     if (NORM) {
+        // the sum of squares in one order however many waves share a row of 4096
+        constexpr int SP = WV == 4 ? XV : 1;
+#pragma unroll
+        for (int p = 0; p < SP; ++p) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int j = p; j < (SP == 1 ? XV : p + 1); ++j)
+                if (j * WV * 64 + tid < K / 8)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float lo = bf16_lo((&xv[j].x)[e]), hi = bf16_hi((&xv[j].x)[e]);
+                        ss = fmaf(lo, lo, ss);
+                        ss = fmaf(hi, hi, ss);
+                    }
+            ss = wave_reduce_sum(ss);
+            if (lane == 0) part[p * WV + wid] = ss;
+        }
+        __syncthreads();
         float ss = 0.0f;
 #pragma unroll
-        for (int j = 0; j < XV; ++j)
-            if (j * 512 + tid < K / 8)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float lo = bf16_lo((&xv[j].x)[e]), hi = bf16_hi((&xv[j].x)[e]);
-                    ss = fmaf(lo, lo, ss);
-                    ss = fmaf(hi, hi, ss);
-                }
-        ss = wave_reduce_sum(ss);
-        if (lane == 0) part[wid] = ss;
-        __syncthreads();
-        ss = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) ss += part[i];
+        for (int i = 0; i < SP * WV; ++i) ss += part[i];
         rstd = rsqrtf(ss / (float)K + eps);
     }
 #pragma unroll
     for (int j = 0; j < XV; ++j) {
-        const int i = j * 512 + tid;                        // columns i * 8 .. + 7
+        const int i = j * WV * 64 + tid;                        // columns i * 8 .. + 7
         if (i >= K / 8) continue;
         float f[8];
 #pragma unroll
@@ -622,8 +628,8 @@ __global__ __launch_bounds__(512) void gemv1_fp8_kernel(
                 acc[t] = 0.0f;
             }
             if (lane == 0) {
-                if (GU) out[u0 + uu] = f32_to_bf16(r[0] / (1.0f + __expf(-r[0])) * r[1]);
-                else reinterpret_cast<uint32_t*>(out)[u0 + uu] = pack_bf16x2(r[0], r[1]);
+                if (GU) out[u0 + uu * waves] = f32_to_bf16(r[0] / (1.0f + __expf(-r[0])) * r[1]);
+                else reinterpret_cast<uint32_t*>(out)[u0 + uu * waves] = pack_bf16x2(r[0], r[1]);
             }
             ug = 0;
             ++uu;
@@ -656,23 +662,31 @@ static bool gemv1_fp8_ok(const void* x, const void* w8, const void* wn, const vo
 static int gemv1_fp8(hipStream_t st, const void* x, const void* w8, const void* wscale, void* out,
                      const void* wn, const void* res, int N, int K, float eps, int mode, bool gateup) {
     const int units = gateup ? N : N / 2;
-    // as many blocks of eight waves as stay resident (two per CU), fewer and fuller ones
-    // where that evens out the CUs by more than a fifth
-    auto rounds = [&](int p) { return CEIL_DIV(CEIL_DIV(CEIL_DIV(units, p), 8), 256) * p; };
-    int per = CEIL_DIV(units, 4096);
-    for (int p = per + 1, p1 = 2 * per + 1; p <= p1; ++p)
-        if (rounds(p) * 5 < rounds(per) * 4) per = p;
+    // As in gemv.hip: up to K = 4096 blocks of four waves of a unit each, no more than 32
+    // blocks per CU (us, blocks of eight / this: 6144 x 4096 8.2 / 7.1, 4096 x 4096 6.5 / 5.8,
+    // 28672 x 4096 22.2 / 21.1, 2 x 14336 x 4096 22.3 / 20.8, 5632 x 2048 4.9 / 4.9). Above: as
+    // many blocks of eight waves as stay resident (two per CU), fewer and fuller ones where
+    // that evens out the CUs by more than a fifth.
+    const int wv = K <= 4096 ? 4 : 8;
+    int per = CEIL_DIV(units, wv == 4 ? 256 * 4 * 32 : 256 * 8 * 2);
+    if (wv == 8) {
+        auto rounds = [&](int p) { return CEIL_DIV(CEIL_DIV(CEIL_DIV(units, p), 8), 256) * p; };
+        for (int p = per + 1, p1 = 2 * per + 1; p <= p1; ++p)
+            if (rounds(p) * 5 < rounds(per) * 4) per = p;
+    }
     if (per > 64) per = 64;
-    const int blocks = CEIL_DIV(CEIL_DIV(units, per), 8);
-#define G1F(NV, RV, GV, GR, XV)                                                                       \
-    hipLaunchKernelGGL((gemv1_fp8_kernel<NV, RV, GV, GR, XV>), dim3(blocks), dim3(512), (size_t)K * 4, \
+    const int blocks = CEIL_DIV(CEIL_DIV(units, per), wv);
+    const int waves = blocks * wv;
+#define G1F(NV, RV, GV, GR, XV, WV)                                                                   \
+    hipLaunchKernelGGL((gemv1_fp8_kernel<NV, RV, GV, GR, XV, WV>), dim3(blocks), dim3(WV * 64), (size_t)K * 4, \
                        st, (const uint4*)x, (const uint32_t*)w8, (const float*)wscale,                \
-                       (uint16_t*)out, (const uint4*)wn, (const uint16_t*)res, N, K, per, eps)
+                       (uint16_t*)out, (const uint4*)wn, (const uint16_t*)res, N, K, waves,           \
+                       units / waves, units % waves, eps)
 #define G1FK(NV, RV, GV)                                \
     do {                                                \
-        if (K == 4096) G1F(NV, RV, GV, 4, 1);           \
-        else if (K < 4096) G1F(NV, RV, GV, 2, 1);       \
-        else G1F(NV, RV, GV, 2, 4);                     \
+        if (K == 4096) G1F(NV, RV, GV, 4, 2, 4);        \
+        else if (K < 4096) G1F(NV, RV, GV, 2, 1, 4);    \
+        else G1F(NV, RV, GV, 2, 4, 8);                  \
     } while (0)
     if (gateup) {
         if (mode & 1) G1FK(true, false, true);

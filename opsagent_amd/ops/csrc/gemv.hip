@@ -194,33 +194,35 @@ __global__ __launch_bounds__(256) void gemv_gateup_kernel(
 // One activation row (M = 1), K a multiple of 2048. gemv_kernel keeps one 1 KiB load
 // per row in flight and, with NORM, normalises the activations again for every row;
 // here the block's (normalised) activations are a float32 image in LDS, made while the
-// first weight loads are under way, and a wave goes over its rows as one stream of
-// GR-chunk groups (512 columns each): the next group, also the next row's, is loaded
-// before the current one is used. The image keeps columns 0-3 and 4-7 of every eight
-// apart, so that 16-byte LDS reads of a wave are contiguous. RT = 2: gate and up rows.
-// us before and now, weights of 1 GiB in turn: 28672 x 4096 gate-up with norm 43.3 and
-// 38.4, 4096 x 14336 24.9 and 20.6, 6144 x 4096 with norm 12.9 and 11.0, 4096 x 4096
-// 8.9 and 8.5, 128256 x 4096 168 and 163, 2048 x 8192 12.0 and 8.4, 16384 x 2048 gate-up
-// 14.8 and 12.9, 2048 x 2048 4.7 and 4.2 (contiguous reads alone run at 6.4 to 6.9 TB/s);
-// asking for the activations before the weights takes another half a microsecond each.
-template <bool NORM, bool ADDRES, int RT, int GR, int XV>
-__global__ __launch_bounds__(512) void gemv1_kernel(const uint32_t* __restrict__ x,
+// first weight loads are under way, and a wave goes over its rows, every waves-th of the
+// weight so that all waves read one window of it (runs of rows instead: 128256 x 2048 93.9
+// us, 83.7), as one stream of GR-chunk groups (512 columns each): the next group, also the
+// next row's, is loaded before the current one is used. The image keeps columns 0-3 and
+// 4-7 of every eight apart, so that 16-byte LDS reads of a wave are contiguous. RT = 2:
+// gate and up rows.
+// us, gemv_kernel / here, weights of 2 GB in turn: 28672 x 4096 gate-up with norm 43.3 /
+// 37.1, 4096 x 14336 25.1 / 20.4, 6144 x 4096 9.6 / 9.9, with norm 12.9 / 10.4, 4096 x 4096
+// 8.1 / 7.3, 128256 x 2048 85.3 / 81.2, 2048 x 8192 11.7 / 8.3, 16384 x 2048 gate-up 13.4 /
+// 12.7, 2048 x 2048 4.4 / 4.0 (contiguous reads alone run at 6.4 to 6.9 TB/s); asking for
+// the activations before the weights takes another half a microsecond each.
+template <bool NORM, bool ADDRES, int RT, int GR, int XV, int WV>
+__global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restrict__ x,
                                                     const uint32_t* __restrict__ w,
                                                     uint16_t* __restrict__ out,
                                                     const uint32_t* __restrict__ wn,
                                                     const uint16_t* __restrict__ res, int N, int K,
-                                                    int per, float eps, int act) {
+                                                    int waves, int full, int extra, float eps,
+                                                    int act) {
     extern __shared__ __attribute__((aligned(16))) float xl[];   // [2][K / 2]
     __shared__ float part[8];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wave = blockIdx.x * 8 + wid;
-    const int r0 = wave * per, r1 = min(r0 + per, N);       // the wave's rows
+    const int wave = blockIdx.x * WV + wid;
     const int k2 = K / 2, groups = K / (512 * GR);
-    const int total = max(r1 - r0, 0) * groups;
+    const int total = (full + (wave < extra)) * groups;     // of the wave's rows: every waves-th
     auto at = [&](int row, int t) { return w + (size_t)(row + (t ? N : 0)) * k2 + lane * 4; };
     u32x4 a[GR][RT], b[GR][RT];
-    int row = min(r0, N - 1), g = 0;                        // of the group loaded last
+    int row = min(wave, N - 1), g = 0;                      // of the group loaded last
     auto load = [&](u32x4 (&v)[GR][RT]) {
 #pragma unroll
         for (int t = 0; t < RT; ++t)
@@ -230,49 +232,54 @@ __global__ __launch_bounds__(512) void gemv1_kernel(const uint32_t* __restrict__
     auto next = [&](u32x4 (&v)[GR][RT]) {
         if (++g == groups) {
             g = 0;
-            ++row;
+            row += waves;
         }
         load(v);
         __builtin_amdgcn_sched_barrier(0);
     };
     // Loads return in order: the activations, eight columns per thread and turn, and lane
-    // i's residual of the wave's row i (per <= 64) are asked for before the weights, so
+    // i's residual of the wave's row i (at most 64) are asked for before the weights, so
     // that the image below waits for them alone.
     uint4 xv[XV], nv[XV];
 #pragma unroll
     for (int j = 0; j < XV; ++j) {
-        const int i = min(j * 512 + tid, K / 8 - 1);
+        const int i = min(j * WV * 64 + tid, K / 8 - 1);
         xv[j] = reinterpret_cast<const uint4*>(x)[i];
         if (NORM) nv[j] = reinterpret_cast<const uint4*>(wn)[i];
     }
-    const float rs = ADDRES ? bf16_to_f32(res[min(r0 + lane, N - 1)]) : 0.0f;
+    const float rs = ADDRES ? bf16_to_f32(res[min(wave + lane * (int64_t)waves, N - (int64_t)1)]) : 0.0f;
     __builtin_amdgcn_sched_barrier(0);
     load(a);
     __builtin_amdgcn_sched_barrier(0);
 
     float rstd = 1.0f;
     if (NORM) {
+        // the sum of squares in one order however many waves share a row of 4096
+        constexpr int SP = WV == 4 ? XV : 1;
+#pragma unroll
+        for (int p = 0; p < SP; ++p) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int j = p; j < (SP == 1 ? XV : p + 1); ++j)
+                if (j * WV * 64 + tid < K / 8)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float lo = bf16_lo((&xv[j].x)[e]), hi = bf16_hi((&xv[j].x)[e]);
+                        ss = fmaf(lo, lo, ss);
+                        ss = fmaf(hi, hi, ss);
+                    }
+            ss = wave_reduce_sum(ss);
+            if (lane == 0) part[p * WV + wid] = ss;
+        }
+        __syncthreads();
         float ss = 0.0f;
 #pragma unroll
-        for (int j = 0; j < XV; ++j)
-            if (j * 512 + tid < K / 8)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float lo = bf16_lo((&xv[j].x)[e]), hi = bf16_hi((&xv[j].x)[e]);
-                    ss = fmaf(lo, lo, ss);
-                    ss = fmaf(hi, hi, ss);
-                }
-        ss = wave_reduce_sum(ss);
-        if (lane == 0) part[wid] = ss;
-        __syncthreads();
-        ss = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) ss += part[i];
+        for (int i = 0; i < SP * WV; ++i) ss += part[i];
         rstd = rsqrtf(ss / (float)K + eps);
     }
 #pragma unroll
     for (int j = 0; j < XV; ++j) {
-        const int i = j * 512 + tid;
+        const int i = j * WV * 64 + tid;
         if (i >= K / 8) continue;
         float f[8];
 #pragma unroll
@@ -292,7 +299,7 @@ __global__ __launch_bounds__(512) void gemv1_kernel(const uint32_t* __restrict__
     float acc[RT];
 #pragma unroll
     for (int t = 0; t < RT; ++t) acc[t] = 0.0f;
-    int ur = r0, ug = 0;                                    // of the group in use
+    int ur = wave, un = 0, ug = 0;                          // of the group in use
     auto use = [&](u32x4 (&v)[GR][RT]) {
 #pragma unroll
         for (int i = 0; i < GR; ++i) {
@@ -316,12 +323,13 @@ __global__ __launch_bounds__(512) void gemv1_kernel(const uint32_t* __restrict__
             float v0 = wave_reduce_sum(acc[0]);
             if (RT == 2) v0 = gate_act(v0, act) * wave_reduce_sum(acc[RT - 1]);
             if (ADDRES)
-                v0 += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rs), ur - r0));
+                v0 += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rs), un));
             if (lane == 0) out[ur] = f32_to_bf16(v0);
 #pragma unroll
             for (int t = 0; t < RT; ++t) acc[t] = 0.0f;
             ug = 0;
-            ++ur;
+            ++un;
+            ur += waves;
         }
     };
     // the last groups are apart, so that every wait counts the loads behind it exactly
@@ -344,25 +352,39 @@ __global__ __launch_bounds__(512) void gemv1_kernel(const uint32_t* __restrict__
 // mode as in oa_gemv_ex; gateup > 0: N gate and N up rows, activation gateup - 1
 static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const void* wn,
                  const void* res, int N, int K, float eps, int mode, int gateup) {
-    // Rows per wave: as many blocks of eight waves as stay resident (two per CU by
-    // registers, four with short rows), fewer and fuller ones where that evens out the
-    // CUs by more than a fifth (6144 x 4096: 2 rows on 384 blocks 12.1 us, 3 on 256 11.0).
-    const int resident = K == 2048 && !gateup ? 4 : 2;
-    auto rounds = [&](int p) { return CEIL_DIV(CEIL_DIV(CEIL_DIV(N, p), 8), 256) * p; };
-    int per = CEIL_DIV(N, 2048 * resident);
-    for (int p = per + 1, p1 = 2 * per + 1; p <= p1; ++p)
-        if (rounds(p) * 5 < rounds(per) * 4) per = p;
+    // Rows of 4096, and many of 2048: blocks of four waves, of two rows a wave (gate-up one
+    // pair), so that CUs even out; the image of a block is quickly made. No more than 32
+    // blocks per CU. Us, blocks of eight waves and up to 64 rows a wave / this: 6144 x 4096
+    // 10.4 / 9.9, 4096 x 4096 8.5 / 7.3, 32000 x 4096 43.5 / 40.8, 2 x 14336 x 4096 38.4 /
+    // 36.4, 128256 x 2048 83.4 / 78.2, 2 x 2816 x 2048 6.6 / 6.3, but 2048 x 2048 3.9 / 4.2, 2
+    // x 1408 x 2048 4.5 / 5.0, 2 x 8192 x 2048 12.7 / 12.9.
+    // Else: as many blocks of eight waves as stay resident (two per CU by registers, four
+    // with short rows), fewer and fuller ones where that evens out the CUs by more than a
+    // fifth.
+    const int wv = K == 4096 || (K == 2048 && (gateup ? N > 2048 && N <= 4096 : N > 4096)) ? 4 : 8;
+    int per;
+    if (wv == 4) {
+        per = CEIL_DIV(N, 256 * 4 * 32);
+        if (!gateup && per < 2) per = 2;
+    } else {
+        auto rounds = [&](int p) { return CEIL_DIV(CEIL_DIV(CEIL_DIV(N, p), 8), 256) * p; };
+        per = CEIL_DIV(N, 2048 * (K == 2048 && !gateup ? 4 : 2));
+        for (int p = per + 1, p1 = 2 * per + 1; p <= p1; ++p)
+            if (rounds(p) * 5 < rounds(per) * 4) per = p;
+    }
     if (per > 64) per = 64;
-    const int blocks = CEIL_DIV(CEIL_DIV(N, per), 8);
+    const int blocks = CEIL_DIV(CEIL_DIV(N, per), wv);
+    const int waves = blocks * wv;
     const size_t lds = (size_t)K * 4;
-#define G1X(NV, RV, RT, GR, XV)                                                                       \
-    hipLaunchKernelGGL((gemv1_kernel<NV, RV, RT, GR, XV>), dim3(blocks), dim3(512), lds, st,          \
+#define G1X(NV, RV, RT, GR, XV, WV)                                                                   \
+    hipLaunchKernelGGL((gemv1_kernel<NV, RV, RT, GR, XV, WV>), dim3(blocks), dim3(WV * 64), lds, st,  \
                        (const uint32_t*)x, (const uint32_t*)w, (uint16_t*)out, (const uint32_t*)wn,   \
-                       (const uint16_t*)res, N, K, per, eps, gateup - 1)
+                       (const uint16_t*)res, N, K, waves, N / waves, N % waves, eps, gateup - 1)
 #define G1(NV, RV, RT, GR)                   \
     do {                                     \
-        if (K <= 4096) G1X(NV, RV, RT, GR, 1); \
-        else G1X(NV, RV, RT, GR, 4);         \
+        if (wv == 4) G1X(NV, RV, RT, GR, 2, 4);         \
+        else if (K <= 4096) G1X(NV, RV, RT, GR, 1, 8);  \
+        else G1X(NV, RV, RT, GR, 4, 8);                 \
     } while (0)
     if (gateup) {
         if (mode & 1) G1(true, false, 2, 4);

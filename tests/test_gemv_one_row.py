@@ -63,3 +63,21 @@ def test_weights_with_gaps(M, N, K):
     check(ops.linear_addres(x, w, res), xd @ wd.T + res.double())
     check(ops.gateup_silu(x, w, N // 2), silu_halves(xd @ wd.T))
     check(ops.gateup_silu_norm(x, nw, 1e-5, w, N // 2), silu_halves(normed @ wd.T))
+
+
+@pytest.mark.gpu
+def test_three_rows_a_wave():
+    """More rows than 32 blocks of four waves per CU take two at a time, some waves with
+    one row less: every row once, with its own residual and scale."""
+    N, K = 65536 + 70, 2048
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    rn = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    x, res = rn(1, K).bfloat16(), (10 * rn(1, N)).bfloat16()
+    w = (rn(N, K) * K ** -0.5).bfloat16()
+    wq, ws = ops.quant_fp8(w)
+    want = (x.float() @ w.float().T + res.float())
+    want8 = x.float() @ (wq.view(torch.float8_e4m3fn).float() * ws[:, None]).T + res.float()
+    # one bf16 rounding of the value and float32 sums of 2048 products of about 1 / sqrt(K)
+    for got, ref in ((ops.linear_addres(x, w, res), want),
+                     (ops.linear_addres_fp8(x, wq, ws, res), want8)):
+        assert ((got.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4).all()
