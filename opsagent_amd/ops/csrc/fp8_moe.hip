@@ -41,21 +41,23 @@ __device__ __forceinline__ unsigned int f32x2_to_fp8(float a, float b,
 }
 
 // ---- per-token quantization -------------------------------------------------
-// q[t] = x[t] / scale, scale = max |x[t]| / 448, one block per row. SILU: the row is
-// silu(g) * u of the two halves of x [T, 2 K], rounded to bf16 as the plain activation
-// kernel's result is. Columns up to 16384 stay in registers between the two passes, the
-// rest are read again. Bound by the launch up to some MB, by memory above; us, a wave
+// q[t] = x[t] / scale, scale = max |x[t]| / 448, TPR threads per row: a block or a wave. SILU:
+// the row is silu(g) * u of the two halves of x [T, 2 K], rounded to bf16 as the plain
+// activation kernel's result is. A thread's first 64 columns stay in registers between the
+// two passes, the rest are read again. Bound by the launch up to some MB, by memory above; us, a wave
 // per row reading twice / here: [700, 14336] 14.9 / 7.4, [3, 28672] 18.0 / 7.5, [700, 4096]
 // in a run of products 9 / 5. SILU with it takes 48 us from a layer's 401 at 700 rows
 // (two copies, the activation and a second pass over 20 MB).
-template <bool SILU>
+template <bool SILU, int TPR>
 __global__ __launch_bounds__(256) void quant_fp8_kernel(
     const uint4* __restrict__ x,     // [T, K/8] bf16x8 (SILU: [T, 2 K/8])
     uint2* __restrict__ q,           // [T, K/8] fp8x8
     float* __restrict__ scales,      // [T]
-    int kv /* K / 8 */) {
+    int T, int kv /* K / 8 */) {
     constexpr int NV = 8;
-    const size_t row = blockIdx.x;
+    const int tid = threadIdx.x & (TPR - 1);
+    const size_t row = blockIdx.x * (size_t)(256 / TPR) + threadIdx.x / TPR;
+    if (TPR < 256 && row >= T) return;
     const uint4* xr = x + row * kv * (SILU ? 2 : 1);
     uint2* qr = q + row * kv;
     auto load = [&](int c) {
@@ -76,17 +78,19 @@ __global__ __launch_bounds__(256) void quant_fp8_kernel(
     uint4 w[NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        const int c = v * 256 + threadIdx.x;
+        const int c = v * TPR + tid;
         if (c < kv) widen(w[v] = load(c));
     }
-    for (int c = NV * 256 + threadIdx.x; c < kv; c += 256) widen(load(c));
-    __shared__ float red[4];
+    for (int c = NV * TPR + tid; c < kv; c += TPR) widen(load(c));
     amax = wave_reduce_max(amax);
-    if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = amax;
-    __syncthreads();
-    amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    if (TPR == 256) {
+        __shared__ float red[4];
+        if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = amax;
+        __syncthreads();
+        amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    }
     const float inv = FP8_MAX / amax;
-    if (threadIdx.x == 0) scales[row] = amax / FP8_MAX;
+    if (tid == 0) scales[row] = amax / FP8_MAX;
     auto store = [&](int c, const uint4& w) {
         uint2 o;
 #pragma unroll
@@ -100,17 +104,30 @@ __global__ __launch_bounds__(256) void quant_fp8_kernel(
     };
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        const int c = v * 256 + threadIdx.x;
+        const int c = v * TPR + tid;
         if (c < kv) store(c, w[v]);
     }
-    for (int c = NV * 256 + threadIdx.x; c < kv; c += 256) store(c, load(c));
+    for (int c = NV * TPR + tid; c < kv; c += TPR) store(c, load(c));
+}
+
+// Short rows leave most of a block idle, many of them cost a block's start each: a wave
+// per row up to 512 columns, and below 2048 from 4096 rows on (us, block / wave: [65536, 512]
+// 52.4 / 23.0, [700, 512] 2.75 / 2.59, [8192, 1024] 10.9 / 8.1, [2048, 1024] 4.0 / 4.05,
+// [8192, 1408] 11.9 / 10.5, [8192, 2048] 13.4 / 13.9).
+template <bool SILU>
+static void quant_fp8(hipStream_t st, const void* x, void* q, void* scales, int T, int K) {
+#define QUANT(TPR)                                                                                  \
+    hipLaunchKernelGGL((quant_fp8_kernel<SILU, TPR>), dim3(CEIL_DIV(T, 256 / TPR)), dim3(256), 0, st, \
+                       (const uint4*)x, (uint2*)q, (float*)scales, T, K / 8)
+    if (K <= 512 || (K < 2048 && T >= 4096)) QUANT(64);
+    else QUANT(256);
+#undef QUANT
 }
 
 extern "C" int oa_quant_fp8(void* stream, const void* x, void* q, void* scales,
                             int T, int K) {
     if (K % 8 != 0) return -100;
-    hipLaunchKernelGGL(quant_fp8_kernel<false>, dim3(T), dim3(256), 0, (hipStream_t)stream,
-                       (const uint4*)x, (uint2*)q, (float*)scales, K / 8);
+    quant_fp8<false>((hipStream_t)stream, x, q, scales, T, K);
     HIP_CHECK_LAUNCH();
     return 0;
 }
@@ -120,8 +137,7 @@ extern "C" int oa_silu_quant_fp8(void* stream, const void* gu, void* q, void* sc
                                  int T, int K) {
     if (K % 8 != 0) return -100;
     if ((uintptr_t)gu % 16 != 0) return -101;
-    hipLaunchKernelGGL(quant_fp8_kernel<true>, dim3(T), dim3(256), 0, (hipStream_t)stream,
-                       (const uint4*)gu, (uint2*)q, (float*)scales, K / 8);
+    quant_fp8<true>((hipStream_t)stream, gu, q, scales, T, K);
     HIP_CHECK_LAUNCH();
     return 0;
 }
@@ -1237,8 +1253,7 @@ extern "C" int oa_gemv_fp8_mfma(void* stream, const void* x, const void* w8,
                            (const uint32_t*)wn, g_gemv8_x8, g_gemv8_xsc, M, K,
                            eps);
     } else {
-        hipLaunchKernelGGL(quant_fp8_kernel<false>, dim3(M), dim3(256), 0, s,
-                           (const uint4*)x, (uint2*)g_gemv8_x8, g_gemv8_xsc, K / 8);
+        quant_fp8<false>(s, x, g_gemv8_x8, g_gemv8_xsc, M, K);
     }
     const size_t shmem =
         img > (size_t)(gateup ? 2 : 1) * 4 * 16 * 16 * 4 * 4

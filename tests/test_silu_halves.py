@@ -63,3 +63,26 @@ def test_mlp_fp8_is_its_parts():
     dq, ds = ops.quant_fp8(_rows(K, I, 8))
     parts = ops.linear_fp8(ops.gateup_silu_fp8(x, wq, ws, I), dq, ds)
     assert torch.equal(ops.mlp_fp8(x, wq, ws, I, dq, ds), parts)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,K", [(1, 8), (7, 128), (5, 512), (5, 520), (4095, 1024), (4097, 1024),
+                                 (4099, 2040), (4096, 2048), (2, 16392)])
+def test_quantization_by_waves_and_blocks(T, K):
+    """Short rows by a wave, long ones by a block: the same scales and bytes as in torch, and
+    of the activation as of its rounded result."""
+    gen = torch.Generator(device="cuda").manual_seed(T + K)
+    gu = torch.randn(T, 2 * K, generator=gen, device="cuda").bfloat16()
+    act = ops.silu_halves(gu, K)
+    q8 = torch.empty(T, K, dtype=torch.uint8, device="cuda")
+    s8 = torch.empty(T, dtype=torch.float32, device="cuda")
+    lib, hip = ops._lib()
+    hip.check(lib.oa_silu_quant_fp8(hip.current_stream_ptr(), gu.data_ptr(), q8.data_ptr(),
+                                    s8.data_ptr(), T, K), "oa_silu_quant_fp8")
+    q, s = ops.quant_fp8(act)
+    assert torch.equal(q, q8) and torch.equal(s, s8)
+    amax = act.float().abs().amax(-1).clamp_min(1e-8)
+    top = torch.full_like(amax, 448.0)               # a scalar would be multiplied by its inverse
+    assert torch.equal(s, amax / top)
+    want = (act.float() * (top / amax)[:, None]).clamp(-448, 448).to(torch.float8_e4m3fn)
+    assert torch.equal(q.view(torch.float8_e4m3fn).float(), want.float())
