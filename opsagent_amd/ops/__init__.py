@@ -903,15 +903,19 @@ def _prefill_splits(B: int, Hq: int, Hk: int, Sq: int, Skv: int) -> Tuple[int, b
 
     Few queries over many keys leave most CUs idle. Up to 128 queries: blocks of a
     head, from three tiles of 128 keys on (32 heads on 8, us before / split: 3 over
-    300 14.4 / 11.1, 16 over 2000 64 / 21, 77 over 1264 40.4 / 20.9). More: blocks
+    300 14.4 / 11.1, 16 over 2000 64 / 21, 77 over 1264 40.4 / 20.9), more tiles where
+    the rows that leave sums of their own, heads times queries, are many (64 x 77, 3 tiles
+    16.4 / 17.3, 4 20.0 / 19.6; 80 x 77, 4 20.3 / 21.0, 5 23.9 / 23.3; 128 x 128, 5 28.7 /
+    31.8, 6 33.1 / 32.0) or two splits share three (128 x 16 16.0 / 16.9). More: blocks
     of a key head, from twelve tiles on (300 over 4000 142 / 54, 1024 over 5000 171 /
     116; 1024 over 1024 would take 44 instead of 38.5)."""
     if Hk < 1 or Hq % Hk:
         return 1, False
     tiles = (Skv + 127) // 128
     if Sq <= 128:
-        splits = min(tiles, 256 // max(1, B * Hq)) if tiles >= 3 else 1
-        return max(1, splits), False
+        rows, splits = B * Hq * Sq, max(1, min(tiles, 256 // max(1, B * Hq)))
+        least = 6 if rows > 8192 else 5 if rows > 5200 else 4 if rows > 3200 or splits < 3 else 3
+        return (splits if tiles >= least else 1), False
     group = Hq // Hk
     if group not in (2, 4, 8) or tiles < 12:
         return 1, False

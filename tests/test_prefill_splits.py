@@ -71,3 +71,14 @@ def test_rule():
     assert split(1, 32, 8, 2048, 6144) == (1, True)
     assert split(1, 6, 2, 300, 4000) == (1, False)            # three heads a key head
     assert split(64, 32, 8, 77, 1264) == (1, False)
+
+
+def test_lines_by_rows():
+    """More key tiles where more rows leave sums: both sides of each line."""
+    split = ops._prefill_splits
+    for B, Hq, Sq, least in ((1, 16, 128, 3), (1, 32, 77, 3), (1, 32, 128, 4), (1, 64, 77, 4),
+                             (8, 16, 16, 4), (1, 80, 77, 5), (1, 64, 128, 5), (4, 32, 77, 6),
+                             (4, 32, 128, 6)):
+        assert split(B, Hq, Hq, Sq, 128 * least - 20)[0] > 1
+        assert split(B, Hq, Hq, Sq, 128 * (least - 1) - 20) == (1, False)
+    assert split(1, 8, 2, 0, 300)[0] >= 1 and split(2, 0, 1, 16, 900)[0] >= 1
