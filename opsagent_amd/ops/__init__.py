@@ -94,9 +94,9 @@ def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
     and row of x, blocks of one CU add up, and past 4.75 TB/s memory bounds all of them;
     measured over 64 weights this holds to a tenth. The library's best times over the same
     weights are 5 us + its bytes at 5.9 TB/s (gate-up with its activation 7.3 and 5.4), and
-    no less than `least`, which falls where its kernels split K. Strips take what
+    no less than `least` (another of its kernels takes over at 32 rows). Strips take what
     they finish sooner: 4096 x 4096, M = 16 10.6 against 15.5 and 32 15.2 against 13.3;
-    1024 x 4096, 32 14.4 / 11.8; 5120 x 13824, 3 39.1 / 28.4. Up to eight rows the staged
+    1024 x 2816, 28 10.3 / 10.9 and 32 10.9 / 9.3; 5120 x 13824, 3 39.1 / 28.4. Up to eight rows the staged
     GEMV is the other form where it runs, and strips are the faster one (12288 x 6144, 8
     35.0 / 41.2), except for rows too short to pipeline, four steps a wave, in more than
     one round (32000 x 1024, 8 19.9 / 16.0; the library 17.2). The persistent form is for
@@ -122,7 +122,7 @@ def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
     if gateup:
         library = max(17.6 if K >= 4096 and M <= 24 else 13.5, 7.3 + mb / 5.4)
     else:
-        least = 10.4 if M <= 16 else 8.4 if M > 24 else 12.6 if K >= 4096 else 11.5
+        least = 10.4 if M <= 16 else 8.4 if M == 32 else 12.6 if K >= 4096 else 10.2
         library = max(least, 5 + mb / 5.9)
     return int(strips < library)
 

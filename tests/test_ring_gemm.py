@@ -138,6 +138,7 @@ def test_lines_between_the_forms():
     # few strips or long ones: the library; short rows in many rounds: the staged GEMV
     assert forms(3, 5120, 13824) == (None, 0) and forms(2, 5120, 13824) == (None, 0)
     assert forms(32, 1024, 4096) == (None, 0) and forms(16, 2048, 5632) == (None, 0)
+    assert forms(28, 1024, 2816) == (None, 1) and forms(32, 1024, 2816) == (None, 0)
     assert forms(32, 1024, 4096, True) == (None, 0) and forms(4, 1024, 4096, True) == (None, 1)
     assert forms(8, 32000, 1024) == (None, 0) and ops._bf16_mfma_ok(8, 1024)
     assert forms(9, 16384, 1024) == (None, 0) and forms(9, 8192, 1024) == (None, 1)
