@@ -1,12 +1,10 @@
-// Paged decode attention for MI355X (gfx950) — SURVEY.md §2b "Decode (paged
-// KV) attention kernel".
+// Paged decode attention for MI355X (gfx950).
 //
 // Single new token per sequence attends to the whole paged KV cache. The op
-// is HBM-bound (reads n_tokens * 2 * Hk * D * 2 bytes); the design follows
-// the CDNA guide Appendix B "Attention decode": vectorized bf16 KV loads
-// (16 B/lane), shuffle-reduce dot products, online softmax in registers, and
-// sequence-split ("split-K over keys") so the grid covers the chip even at
-// batch 1 (B*Hk workgroups alone would leave 256 CUs mostly idle).
+// is HBM-bound (reads n_tokens * 2 * Hk * D * 2 bytes): 16-byte loads of cache
+// rows, scores on the matrix cores, online softmax in registers, and sequences
+// split over keys so that the grid covers the chip even at batch 1 (B*Hk
+// workgroups alone would leave 256 CUs mostly idle).
 //
 // Layouts:
 //   q        [B, Hq, 128] bf16
@@ -150,27 +148,15 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
         for (int i = 0; i < 4; ++i)
             vw[i] = *reinterpret_cast<const uint4*>(vc + ((size_t)vs[i] * Hk + h) * (DHEAD / 2) + dl * 4);
     };
-    int page = 0;
-    if (nt > 0) {
-        load_tile(0, page_of(0), kr_[0], vr_[0]);
-        page = page_of(1);
-    }
-
-    // queries: lane (column dl, channels s*32 + g16*8 .. + 7 of step s)
+    // Loads return in order: the queries and their angles are asked for first, so that they
+    // are rotated and split while the first keys, values and the new key are under way
     const int head = dl % GP, part = dl / GP;
     const bool have = head < G;
-    float qf[4][8];
+    uint4 qw[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        const uint4 w = *reinterpret_cast<const uint4*>(
+    for (int s = 0; s < 4; ++s)     // lane (column dl, channels s*32 + g16*8 .. + 7 of step s)
+        qw[s] = *reinterpret_cast<const uint4*>(
             q + (size_t)b * qs2 + ((size_t)(h * G + (have ? head : 0)) * DHEAD + s * 32 + g16 * 8) / 2);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            qf[s][j * 2] = have ? bf16_lo((&w.x)[j]) : 0.0f;
-            qf[s][j * 2 + 1] = have ? bf16_hi((&w.x)[j]) : 0.0f;
-        }
-    }
-    // ROPE: channel d pairs with d + 64, two steps on in the same lane
     float c8[2][8], s8[2][8];
     if (ROPE) {
         const int pos = max(n - 1, 0);
@@ -184,6 +170,34 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
                 s8[s][j] = srow[j];
             }
         }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    int page = 0;
+    if (nt > 0) {
+        load_tile(0, page_of(0), kr_[0], vr_[0]);
+        page = page_of(1);
+    }
+    const bool owner = ROPE && n - 1 >= kstart && n - 1 < kend && wid == 3;   // of the new key
+    uint4 nk[4], nv;
+    if (owner) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            nk[s] = *reinterpret_cast<const uint4*>(
+                kin + (size_t)b * ks2 + ((size_t)h * DHEAD + s * 32 + g16 * 8) / 2);
+        nv = *reinterpret_cast<const uint4*>(vin + (size_t)b * vs2 + ((size_t)h * DHEAD + dl * 8) / 2);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    float qf[4][8];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            qf[s][j * 2] = have ? bf16_lo((&qw[s].x)[j]) : 0.0f;
+            qf[s][j * 2 + 1] = have ? bf16_hi((&qw[s].x)[j]) : 0.0f;
+        }
+    // ROPE: channel d pairs with d + 64, two steps on in the same lane
+    if (ROPE) {
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -194,6 +208,25 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
             }
     }
 
+    // the lane's part of its query, and the third parts for a second product: the first
+    // bf16 of what the parts before leave
+    da_b8 qb[4], qb2[GP == 8 ? 4 : 1];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float x = qf[s][j], hi = (float)(__bf16)x;
+            if (GP == 8) {
+                const float r1 = x - hi, mid = (float)(__bf16)r1;
+                qb[s][j] = (__bf16)(part == 0 ? x : r1);
+                qb2[GP == 8 ? s : 0][j] = (__bf16)(part == 0 ? r1 - mid : 0.0f);
+            } else {
+                const float r1 = part > 0 ? x - hi : x;
+                const float r2 = part > 1 ? r1 - (float)(__bf16)r1 : r1;
+                qb[s][j] = (__bf16)(part < 3 ? r2 : 0.0f);
+            }
+        }
+
     // running maximum of the lane's head over its row's keys, the lane's share of
     // the sum of weights, value sums of all heads
     float m = -INFINITY, lsum = 0.0f, o[G][8];
@@ -202,20 +235,15 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
 #pragma unroll
         for (int j = 0; j < 8; ++j) o[gh][j] = 0.0f;
 
-    if (ROPE && n - 1 >= kstart && n - 1 < kend && wid == 3) {
-        uint4 vw = *reinterpret_cast<const uint4*>(
-            vin + (size_t)b * vs2 + ((size_t)h * DHEAD + dl * 8) / 2);
+    if (owner) {
         float kf[4][8];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const uint4 w = *reinterpret_cast<const uint4*>(
-                kin + (size_t)b * ks2 + ((size_t)h * DHEAD + s * 32 + g16 * 8) / 2);
+        for (int s = 0; s < 4; ++s)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                kf[s][j * 2] = bf16_lo((&w.x)[j]);
-                kf[s][j * 2 + 1] = bf16_hi((&w.x)[j]);
+                kf[s][j * 2] = bf16_lo((&nk[s].x)[j]);
+                kf[s][j * 2 + 1] = bf16_hi((&nk[s].x)[j]);
             }
-        }
         float dot = 0.0f;
 #pragma unroll
         for (int s = 0; s < 2; ++s)
@@ -238,36 +266,18 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
                                pack_bf16x2(kf[s][4], kf[s][5]), pack_bf16x2(kf[s][6], kf[s][7]));
         }
         if (g16 == 0) {
-            *reinterpret_cast<uint4*>(vcw + ((size_t)slot * Hk + h) * (DHEAD / 2) + dl * 4) = vw;
+            *reinterpret_cast<uint4*>(vcw + ((size_t)slot * Hk + h) * (DHEAD / 2) + dl * 4) = nv;
             m = dot * scale;
             lsum = part == 0 ? 1.0f : 0.0f;
 #pragma unroll
             for (int gh = 0; gh < G; ++gh)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    o[gh][j * 2] = bf16_lo((&vw.x)[j]);
-                    o[gh][j * 2 + 1] = bf16_hi((&vw.x)[j]);
+                    o[gh][j * 2] = bf16_lo((&nv.x)[j]);
+                    o[gh][j * 2 + 1] = bf16_hi((&nv.x)[j]);
                 }
         }
     }
-
-    // the lane's part of its query, and the third parts for a second product
-    da_b8 qb[4], qb2[GP == 8 ? 4 : 1];
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float hi = bf16_to_f32(f32_to_bf16(qf[s][j]));
-            const float r1 = qf[s][j] - hi;
-            const float mid = bf16_to_f32(f32_to_bf16(r1));
-            const float lo = r1 - mid;
-            if (GP == 8) {
-                qb[s][j] = (__bf16)(part == 0 ? hi : mid);
-                qb2[GP == 8 ? s : 0][j] = (__bf16)(part == 0 ? lo : 0.0f);
-            } else {
-                qb[s][j] = (__bf16)(part == 0 ? hi : part == 1 ? mid : part == 2 ? lo : 0.0f);
-            }
-        }
 
     auto process = [&](int t, const uint4 (&kw)[4], const uint4 (&vw)[4]) {
         da_f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -565,9 +575,7 @@ static int decode_chunk_base(int pairs) {
     return pairs <= 8 ? 64 : pairs <= 64 ? 128 : pairs <= 128 ? 256 : 512;
 }
 
-// fused: cnt_ws must be a zero-initialized... no — zeroed HERE each call via
-// hipMemsetAsync (graph-capturable memset node). fused=0 keeps the two-kernel
-// path (A/B reference and fallback).
+// fused: cnt_ws is zeroed here on each call (hipMemsetAsync). fused = 0: two kernels.
 extern "C" int oa_attention_decode(void* stream, const void* q, const void* kc,
                                    const void* vc, const void* block_table,
                                    const void* seq_lens, void* o_part,
