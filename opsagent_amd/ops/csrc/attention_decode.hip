@@ -297,6 +297,20 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
             if (GP == 4) x[i] += row_ror<4>(x[i]);
             x[i] += row_ror<8>(x[i]);
         }
+        // An infinite key times a part that is zero is NaN: such a key's score is that of the
+        // first parts alone, infinite or NaN as the whole query's is
+        const float xs = (x[0] + x[1]) + (x[2] + x[3]);
+        if (__any(xs != xs)) {
+            da_f4 first = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                first = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(da_b8, kw[s]), qb[s], first, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float y = __shfl(first[i], (lane & 48) | head, WAVE);
+                if (x[i] != x[i]) x[i] = y;
+            }
+        }
         // the lane's own keys of its row
         float sc[KL], p[KL];
         const int key = wstart + t * 16 + g16 * 4 + part * KL;

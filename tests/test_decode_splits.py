@@ -108,3 +108,25 @@ def test_decode_scores_in_32_bits():
     # scores are near 724, float32 keeps 6e-5 of them: weights to 1e-4, then one bf16
     # rounding
     assert ((got[0].double() - want).norm() / want.norm()) < 2.0 ** -8 + 2e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("G", [1, 2, 4, 8])
+def test_infinite_keys(G):
+    """A cached key with an infinite channel has weight zero for the heads whose score it
+    makes minus infinity, and leaves the other keys theirs."""
+    Hk, n, bs = 2, 300, 32
+    q, _, _, kc, vc, table, lens, _ = _case([n], Hk, G, bs, seed=G)
+    rows = lambda m: table[0, torch.arange(m, device="cuda") // bs].long() * bs + (  # noqa: E731
+        torch.arange(m, device="cuda") % bs)
+    q = q.clone()
+    q[..., 5] = -q[..., 5].abs() - 0.25
+    flat_k, flat_v = kc.view(-1, Hk, D), vc.view(-1, Hk, D)
+    at = rows(n)
+    flat_k[at[[7, 130, n - 1]], :, 5] = float("inf")
+    keep = torch.ones(n, dtype=torch.bool, device="cuda")
+    keep[[7, 130, n - 1]] = False
+    want = _attend(q[0].double(), flat_k[at[keep]].double(), flat_v[at[keep]].double(), G)
+    for nsplit in (1, 4):
+        got = ops.attention_decode_paged(q, kc, vc, table, lens, nsplit=nsplit)[0].double()
+        assert float((got - want).norm() / want.norm()) < 2.0 ** -8 + 1e-5
