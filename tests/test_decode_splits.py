@@ -65,12 +65,12 @@ def test_decode_attention(G, lens, bs, nsplit):
         ks, vs = torch.cat([ks[:-1], new_k[-1][None]]), torch.cat([vs[:-1], v[b].double()[None]])
         roped.append(_attend(_rotate(q[b].double(), n - 1, cos, sin), ks, vs, G))
 
-    # the result is one bf16 rounding (at most 2^-8 of a value, 0.0016 in the mean)
-    # of a float32 sum
+    # the result is one bf16 rounding of a float32 sum: 0.0016 in the mean over the 512
+    # values and more of each call (a second one would make it 0.0023)
     def check(got, want):
         want = torch.stack(want)
         err = (got.double() - want).norm() / want.norm()
-        assert err < 2.0 ** -8 + 1e-5, float(err)
+        assert err < 2e-3, float(err)
 
     check(ops.attention_decode_paged(q, kc, vc, table, lens_t, nsplit=nsplit), plain)
     check(ops.attention_decode_paged(q, kc, vc, table, lens_t, nsplit=nsplit, fused_combine=True),
@@ -129,4 +129,4 @@ def test_infinite_keys(G):
     want = _attend(q[0].double(), flat_k[at[keep]].double(), flat_v[at[keep]].double(), G)
     for nsplit in (1, 4):
         got = ops.attention_decode_paged(q, kc, vc, table, lens, nsplit=nsplit)[0].double()
-        assert float((got - want).norm() / want.norm()) < 2.0 ** -8 + 1e-5
+        assert float((got - want).norm() / want.norm()) < 2.1e-3     # 256 values and more

@@ -20,8 +20,10 @@ def test_one_row(N, K):
     normed = xd / torch.sqrt((xd * xd).mean() + 1e-5) * nw.double()
 
     def check(got, want):
-        # one bf16 rounding of a float32 sum: at most 2^-8 of a value
-        assert float((got.double() - want).norm() / want.norm()) < 2.0 ** -8 + 1e-5
+        # one bf16 rounding of a float32 sum: at most 2^-8 of a value, 0.0016 in the mean
+        # over many (a second one would make it 0.0023)
+        tol = 2e-3 if want.numel() >= 1024 else 2.0 ** -8 + 1e-5
+        assert float((got.double() - want).norm() / want.norm()) < tol
 
     check(ops.linear(x, w), xd @ wd.T)
     check(ops.linear_norm(x, nw, 1e-5, w), normed @ wd.T)
@@ -35,6 +37,19 @@ def test_one_row(N, K):
         check(ops.gateup_act(x, w, h, "silu"), g * torch.sigmoid(g) * u)
         check(ops.gateup_act(x, w, h, "gelu_tanh"),
               torch.nn.functional.gelu(g, approximate="tanh") * u)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K", [(8, 2048), (4097, 4096), (6144, 2048), (9001, 14336)])
+def test_one_row_whole_numbers(N, K):
+    """Whole numbers: every float32 sum is exact, the result its one rounding to bf16."""
+    gen = torch.Generator(device="cuda").manual_seed(N + K)
+    x = torch.randint(-8, 9, (1, K), generator=gen, device="cuda").bfloat16()
+    w = torch.randint(-8, 9, (N, K), generator=gen, device="cuda").bfloat16()
+    res = torch.randint(-99, 100, (1, N), generator=gen, device="cuda").bfloat16()
+    want = x.double() @ w.double().T
+    assert torch.equal(ops.linear(x, w), want.bfloat16())
+    assert torch.equal(ops.linear_addres(x, w, res), (want + res.double()).bfloat16())
 
 
 @pytest.mark.gpu

@@ -348,13 +348,30 @@ class TestMoeGrouped:
             spec = dataclasses.replace(spec, moe_dtype="fp8")
         gen = torch.Generator(device="cuda").manual_seed(4)
         moe = MoEMLP(spec, torch.bfloat16, gen).to("cuda")
-        # T=40, top_k=4 -> P=160 >= the default expert-major threshold (64)
+        # T=40, top_k=4 -> P=160 >= the default expert-major threshold (64); the layer
+        # itself sends so many pairs of so few experts to the sorted tiles
         x = (torch.randn(40, spec.hidden_size, device="cuda") * 0.3).to(torch.bfloat16)
+        idx, wts, tok = ops.moe_route(x, moe.router_w, moe.top_k)
+        w13, w2 = (moe.w13_q, moe.w2_q) if fp8 else (moe.w13, moe.w2)
+        s13, s2 = (moe.w13_s, moe.w2_s) if fp8 else (None, None)
+        from opsagent_amd.ops import hip_lib
+
+        lib, calls = hip_lib.get_lib(), []
         _os.environ["OPSAGENT_MOE_EMAJ_MIN_P"] = "64"
+        names = ("oa_moe_gateup_emaj_act", "oa_moe_down_emaj")
+        kept = [getattr(lib, n) for n in names]
         try:
-            out_emaj = moe(x)
+            for n, fn in zip(names, kept):
+                setattr(lib, n, lambda *a, n=n, fn=fn: calls.append(n) or fn(*a))
+            y = ops.moe_grouped_mlp(x, w13, s13, w2, s2, idx.view(-1), tok.view(-1), wts.view(-1),
+                                    moe.i_local, fp8, num_experts=moe.num_experts)
         finally:
+            for n, fn in zip(names, kept):
+                setattr(lib, n, fn)
             _os.environ.pop("OPSAGENT_MOE_EMAJ_MIN_P", None)
+        assert calls == list(names)
+        shared = moe.shared(x) if moe.shared is not None else None
+        out_emaj = ops.moe_combine(y, moe.top_k, shared)
         out_loop = moe.forward_loop(x)
         err = (out_emaj.float() - out_loop.float()).abs().max()
         scale = out_loop.float().abs().max().clamp_min(1e-3)
