@@ -128,11 +128,11 @@ def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
 
 
 def _skinny_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """16-byte loads of the rows of both operands, and no switch that asks for other
-    forms."""
+    """16-byte loads of the rows of both operands, on one device, and no switch that asks
+    for other forms."""
     return (
         x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-        and w.dim() == 2 and w.is_contiguous() and x.dim() >= 1 and x.shape[-1] == w.shape[1]
+        and w.device == x.device and w.dim() == 2 and w.is_contiguous() and x.dim() >= 1 and x.shape[-1] == w.shape[1]
         and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1
                                    and x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0))
         and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and not _gemv_switched()
@@ -844,7 +844,7 @@ def gateup_fused(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> bool
         x.is_cuda and x.dtype == torch.bfloat16 and K % 8 == 0 and x.is_contiguous()
         and gate_up_w.is_contiguous()
         and (_gemv_m_ok(M) or _bf16_mfma_ok(M, K, gateup=True)
-             or (_skinny_ok(x, gate_up_w)
+             or (_skinny_ok(x, gate_up_w) and gate_up_w.shape[0] == 2 * i_local
                  and (_ring_plan(M, i_local, K, gateup=True) is not None
                       or _skinny_form(M, i_local, K, gateup=True) > 0)))
     )
@@ -859,7 +859,7 @@ def gateup_act(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int,
     M = x.numel() // x.shape[-1]
     assert x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous()
     assert act in ("silu", "gelu_tanh")
-    if M > 1 and _skinny_ok(x, gate_up_w):
+    if M > 1 and _skinny_ok(x, gate_up_w) and gate_up_w.shape[0] == 2 * i_local:
         plan = _ring_plan(M, i_local, x.shape[-1], gateup=True)
         if plan:
             return _ring(x, gate_up_w, plan, act=1 + int(act == "gelu_tanh"))

@@ -118,3 +118,22 @@ def test_switches(monkeypatch):
     monkeypatch.delenv("OPSAGENT_BF16_GEMV_MFMA")
     monkeypatch.setenv("OPSAGENT_GEMV_MAX_M", "1")
     assert torch.equal(ops.linear(x[:2], w), torch.nn.functional.linear(x[:2], w))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [24, 64])
+def test_mismatches_are_refused(M):
+    """A weight on another device, of other columns or with other than 2 I rows is an error of
+    the general path, not an address that a kernel reads."""
+    x = torch.zeros(M, 4096, dtype=torch.bfloat16, device="cuda")
+    w = torch.zeros(8192, 4096, dtype=torch.bfloat16, device="cuda")
+    assert ops._skinny_form(M, 8192, 4096) or ops._ring_plan(M, 8192, 4096)
+    for other in (w.cpu(), w[:, :2048].contiguous()):
+        with pytest.raises(RuntimeError):
+            ops.linear(x, other)
+    for rows in (8064, 8192 + 128):
+        other = torch.zeros(rows, 4096, dtype=torch.bfloat16, device="cuda")
+        assert not ops.gateup_fused(x, other, 4096)
+        with pytest.raises(RuntimeError):
+            ops.gateup_silu(x, other, 4096)
+    assert ops.gateup_fused(x, w, 4096)
