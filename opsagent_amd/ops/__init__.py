@@ -485,6 +485,7 @@ def mlp_fp8(
     M, K = x.numel() // x.shape[-1], x.shape[-1]
     if not (
         _is_gpu(x) and M > 8 and K % 128 == 0 and i_local % 128 == 0
+        and gate_up_q.shape[0] == 2 * i_local
         and not _fp8_mfma_ok(M, K) and not _fp8_mfma_ok(M, i_local)
     ):
         return linear_fp8(gateup_silu_fp8(x, gate_up_q, gate_up_s, i_local), down_q, down_s)
@@ -591,6 +592,7 @@ def moe_route_ok(x: torch.Tensor, router_w: torch.Tensor, top: int) -> bool:
     return (
         x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
         and router_w.dtype == torch.float32 and router_w.is_contiguous()
+        and router_w.device == x.device and x.shape[1] == K
         and K % 8 == 0 and E <= 1024 and top <= min(E, 64)
         and x.data_ptr() % 16 == 0 and router_w.data_ptr() % 16 == 0
     )
@@ -647,6 +649,7 @@ def moe_sorted_ok(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, act=None
     128-column steps, a gate strip holds 64 rows."""
     return (
         x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
+        and w13.device == w2.device == x.device
         and w13.is_contiguous() and w2.is_contiguous() and w13.dtype == w2.dtype
         and w13.dtype in (torch.bfloat16, torch.uint8) and _moe_act(act) is not None
         and x.shape[1] % 128 == 0 and w2.shape[2] % 128 == 0 and w13.shape[0] <= 1024

@@ -178,3 +178,19 @@ def test_sorted_experts_refuse():
     w2 = torch.zeros(2, 128, 128, dtype=torch.bfloat16)
     assert not ops.moe_sorted_ok(x, w13, w2)
     assert ops._moe_act("gelu_tanh") is None and ops._moe_act(None) == (0, 0.0, 0.0)
+
+
+@pytest.mark.gpu
+def test_mismatches_are_refused():
+    """A router or experts on another device or of another width are errors of the general
+    path, not addresses that a kernel reads."""
+    x = torch.zeros(3, 256, dtype=torch.bfloat16, device="cuda")
+    router = torch.zeros(8, 256, device="cuda")
+    assert ops.moe_route_ok(x, router, 2)
+    for other in (router.cpu(), router[:, :128].contiguous(), torch.zeros(8, 264, device="cuda")):
+        with pytest.raises(RuntimeError):
+            ops.moe_route(x, other, 2)
+    w13 = torch.zeros(8, 256, 256, dtype=torch.bfloat16, device="cuda")
+    w2 = torch.zeros(8, 256, 128, dtype=torch.bfloat16, device="cuda")
+    assert ops.moe_sorted_ok(x, w13, w2)
+    assert not ops.moe_sorted_ok(x, w13.cpu(), w2) and not ops.moe_sorted_ok(x, w13, w2.cpu())

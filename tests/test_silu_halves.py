@@ -86,3 +86,14 @@ def test_quantization_by_waves_and_blocks(T, K):
     assert torch.equal(s, amax / top)
     want = (act.float() * (top / amax)[:, None]).clamp(-448, 448).to(torch.float8_e4m3fn)
     assert torch.equal(q.view(torch.float8_e4m3fn).float(), want.float())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [640, 896])
+def test_mlp_refuses_other_gate_rows(rows):
+    """gate-up weights of other than 2 I rows: an error, as of the split that was there."""
+    x = _rows(33, 256, 9)
+    wq, ws = ops.quant_fp8(_rows(rows, 256, 10))
+    dq, ds = ops.quant_fp8(_rows(256, 384, 11))
+    with pytest.raises(RuntimeError):
+        ops.mlp_fp8(x, wq, ws, 384, dq, ds)
