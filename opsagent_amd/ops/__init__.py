@@ -17,6 +17,7 @@ import os
 from typing import Optional, Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 from opsagent_amd.ops import torch_ref
 
@@ -127,11 +128,27 @@ def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
     return int(strips < library)
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+_traced = torch._C._get_tracing_state
+_transform = torch._C._functorch.maybe_current_level
+_modes = torch._C._len_torch_dispatch_stack
+
+
+def _plain_call(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Nobody asks for gradients or tangents, traces or transforms the call: a kernel sees
+    addresses alone, the library's product is an operation that all of these know."""
+    return not (
+        torch.compiler.is_compiling() or _traced() is not None or _transform() is not None
+        or _modes() or forward_ad._current_level >= 0
+        or ((x.requires_grad or w.requires_grad) and torch.is_grad_enabled())
+    ) and type(x) in _PLAIN and type(w) in _PLAIN
+
+
 def _skinny_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """16-byte loads of the rows of both operands, on one device, and no switch that asks
-    for other forms."""
+    """16-byte loads of the rows of both operands, on one device, a call that nothing
+    records, and no switch that asks for other forms."""
     return (
-        x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+        _plain_call(x, w) and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
         and w.device == x.device and w.dim() == 2 and w.is_contiguous() and x.dim() >= 1 and x.shape[-1] == w.shape[1]
         and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1
                                    and x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0))

@@ -137,3 +137,51 @@ def test_mismatches_are_refused(M):
         with pytest.raises(RuntimeError):
             ops.gateup_silu(x, other, 4096)
     assert ops.gateup_fused(x, w, 4096)
+
+
+def test_plain_calls():
+    x, w = torch.zeros(3, 8), torch.zeros(5, 8)
+    seen = []
+
+    def look(a, b=w):
+        seen.append(ops._plain_call(a, b))
+        return a @ b.T
+
+    look(x)
+    assert seen.pop()
+    torch.vmap(look)(x[None])
+    torch.func.jvp(look, (x,), (x,))
+    torch.jit.trace(look, (x, w), check_trace=False)
+    torch.fx.experimental.proxy_tensor.make_fx(look)(x, w)
+    look(x.clone().requires_grad_())
+    look(x, torch.nn.Parameter(w))
+    with torch.autograd.forward_ad.dual_level():
+        look(torch.autograd.forward_ad.make_dual(x, x))
+    assert len(seen) == 7 and not any(seen)
+    with torch.no_grad():
+        look(x, torch.nn.Parameter(w))
+    assert seen.pop()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [24, 64])
+def test_gradients_and_transforms(M):
+    """Rows that the library took before keep its gradients, transforms and traces."""
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, 4096, generator=gen, device="cuda").bfloat16()
+    w = (torch.randn(8192, 4096, generator=gen, device="cuda") * 2.0 ** -6).bfloat16()
+    plain = ops.linear(x, w)
+    assert ops._skinny_ok(x, w)
+    library = torch.nn.functional.linear(x, w)
+    assert _err(plain, library.double()) < 4e-3              # one rounding each
+    p, v = torch.nn.Parameter(w), x.clone().requires_grad_()
+    out = ops.linear(v, p)
+    assert torch.equal(out, library)
+    grad = torch.autograd.grad(out.float().sum(), [v, p])
+    want = [w.float().sum(0).expand(M, -1), x.float().sum(0).expand(8192, -1)]
+    for got, ref in zip(grad, want):
+        assert _err(got, ref.double()) < 4e-3
+    each = torch.vmap(lambda a: ops.linear(a, w))(torch.stack([x, x]))
+    assert _err(each[1], library.double()) < 4e-3
+    with torch.no_grad():
+        assert torch.equal(ops.linear(v, p), plain)
