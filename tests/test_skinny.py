@@ -152,7 +152,8 @@ def test_plain_calls():
     torch.vmap(look)(x[None])
     torch.func.jvp(look, (x,), (x,))
     torch.jit.trace(look, (x, w), check_trace=False)
-    torch.fx.experimental.proxy_tensor.make_fx(look)(x, w)
+    with torch._subclasses.FakeTensorMode(allow_non_fake_inputs=True):
+        look(torch.empty(3, 8))
     look(x.clone().requires_grad_())
     look(x, torch.nn.Parameter(w))
     with torch.autograd.forward_ad.dual_level():
