@@ -661,6 +661,24 @@ def moe_sorted_wins(pairs: int, experts: int, fp8: bool) -> bool:
     return pairs >= (max(24, experts // 2) if fp8 else max(32, experts))
 
 
+def _moe_tile_rows(pairs: int, experts: int, weights: int, fp8: bool) -> int:
+    """Rows of a tile of moe_sorted_mlp, by the rows that an expert has on average; weights
+    is the size of one expert matrix. The same bits with any of them.
+
+    Both products and the sort in graphs, us with 16 / 64 rows. fp8, 64 experts of 1408 x
+    2048: 1.5 rows 110 / 116, 4 rows 119 / 123, 6 rows 133 / 129; 128 of 768 x 2048: 1.5 rows
+    112 / 126, 4 rows 130 / 136. bf16: 206 / 198, 224 / 219, 244 / 229; 203 / 201, 243 / 235.
+    A tile slot that P pairs may need but mostly do not leaves a die short of work when there
+    are few experts: 16 bf16 experts of 1024 x 2048 48 pairs 68 / 54, 64 pairs 67 / 71; 8 of
+    14336 x 4096, 32 pairs 595 / 501; small matrices are launches either way, 16 of 512 x
+    1024, 48 pairs 25 / 26. 64 / 128 rows, 64 experts of 1408 x 2048, bf16: 48 rows 307 / 297,
+    96 rows 378 / 385, 192 rows 582 / 501."""
+    if pairs <= 4 * experts:
+        wide = not fp8 and experts * weights >= 2 ** 24 and (pairs < 64 or experts >= 64)
+        return 64 if wide else 16
+    return 64 if pairs < 128 * experts else 128
+
+
 def moe_sorted_ok(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, act=None) -> bool:
     """Whether moe_sorted_mlp takes these experts: both products run over
     128-column steps, a gate strip holds 64 rows."""
@@ -701,11 +719,7 @@ def moe_sorted_mlp(
     assert expert_ids.shape == pair_weights.shape == (T, top)
     assert (w13.dtype == torch.uint8) == (w13_scale is not None) == (w2_scale is not None)
     P = T * top
-    # rows of a tile, by the rows that an expert has on average (64 experts of
-    # 1408 x 2048, both products, bf16, us): 1.5 rows 193 with 16 to 182 with 64
-    # (fp8 99 to 112), 3.8 rows 206 to 203 (106 to 116), 6 rows 231 to 214; 48 rows
-    # 307 with 64 to 297 with 128, 96 rows 378 to 385, 192 rows 582 to 501
-    bm = 16 if P <= 4 * E else 64 if P < 128 * E else 128
+    bm = _moe_tile_rows(P, E, I * H, w13_scale is not None)
     max_tiles = P // bm + min(E, P)
     lib, hip = _lib()
     stream, dev = hip.current_stream_ptr(), x.device

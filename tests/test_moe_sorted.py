@@ -194,3 +194,14 @@ def test_mismatches_are_refused():
     w2 = torch.zeros(8, 256, 128, dtype=torch.bfloat16, device="cuda")
     assert ops.moe_sorted_ok(x, w13, w2)
     assert not ops.moe_sorted_ok(x, w13.cpu(), w2) and not ops.moe_sorted_ok(x, w13, w2.cpu())
+
+
+def test_tile_rows():
+    """bf16 experts take wide tiles from the start, but for small matrices and for few
+    experts whose pairs may fill one tile more; fp8 ones from five rows an expert."""
+    rows = ops._moe_tile_rows
+    big, small = 1408 * 2048, 512 * 1024
+    assert [rows(p, 64, big, False) for p in (48, 256, 257, 8191, 8192)] == [64, 64, 64, 64, 128]
+    assert [rows(p, 64, big, True) for p in (48, 256, 257, 8191, 8192)] == [16, 16, 64, 64, 128]
+    assert [rows(p, 16, big, False) for p in (63, 64, 65)] == [64, 16, 64]
+    assert [rows(p, 16, small, False) for p in (48, 64, 65)] == [16, 16, 64]
