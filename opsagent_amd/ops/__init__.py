@@ -47,9 +47,8 @@ _GEMV_MS = frozenset(range(1, 9))
 
 
 def _bf16_mfma_ok(M: int, K: int, gateup: bool = False) -> bool:
-    """Mirror of gemv.hip's gemv_bf16_use_mfma: the MFMA batched-decode
-    kernel (M 3..16) — concurrent decode's hipBLASLt fallback measured
-    ~2.5x off the stream roofline."""
+    """Mirror of gemv.hip's gemv_bf16_use_mfma: the staged MFMA kernel (M 3..8 unless
+    OPSAGENT_BF16_GEMV_MFMA asks for others)."""
     e = os.environ.get("OPSAGENT_BF16_GEMV_MFMA", "")
     if e == "0":
         return False
@@ -878,7 +877,7 @@ def gateup_fused(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> bool
         x.is_cuda and x.dtype == torch.bfloat16 and K % 8 == 0 and x.is_contiguous()
         and gate_up_w.is_contiguous()
         and (_gemv_m_ok(M) or _bf16_mfma_ok(M, K, gateup=True)
-             or (_skinny_ok(x, gate_up_w) and gate_up_w.shape[0] == 2 * i_local
+             or (M <= 128 and _skinny_ok(x, gate_up_w) and gate_up_w.shape[0] == 2 * i_local
                  and (_ring_plan(M, i_local, K, gateup=True) is not None
                       or _skinny_form(M, i_local, K, gateup=True) > 0)))
     )
@@ -1002,12 +1001,10 @@ def attention_prefill(
 
 
 def decode_nsplit(batch: int, n_kv_heads: int, max_len: int) -> int:
-    """Split the key range so the grid covers 256 CUs with a couple of
-    blocks each (≫256 workgroups rule). Minimum split granule is 64 keys
-    (16 per wave). Target 512 blocks, not more: each extra split adds a
-    partial the combine must re-read, and the 4-deep load pipeline wants
-    ≥8 key-quads per wave to hide HBM latency (A/B at B=1 len 8192:
-    nsplit 128 -> 64 cut the step's attention+combine time)."""
+    """The most splits of a sequence's keys: blocks for the 256 CUs, a couple each. Target
+    512, not more: every split leaves a partial result that the combine reads again.
+    The kernel gives a split at least 64 keys (16 per wave), more for larger launches
+    (decode_chunk in attention_decode.hip), so short sequences use fewer."""
     tgt_blocks = int(os.environ.get("OPSAGENT_DECODE_NSPLIT_TARGET", "512"))
     target = max(1, tgt_blocks // max(1, batch * n_kv_heads))
     return int(max(1, min(target, (max_len + 63) // 64)))
