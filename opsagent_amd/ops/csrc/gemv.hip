@@ -466,11 +466,6 @@ extern "C" int oa_gemv_gateup_ex(void* stream, const void* x, const void* w,
     return gemv_gateup_impl(stream, x, w, out, wn, M, I, K, eps, norm, 0);
 }
 
-extern "C" int oa_gemv_gateup(void* stream, const void* x, const void* w,
-                              void* out, int M, int I, int K) {
-    return gemv_gateup_impl(stream, x, w, out, nullptr, M, I, K, 0.0f, 0, 0);
-}
-
 // act: 0 silu, 1 gelu (tanh form)
 extern "C" int oa_gemv_gateup_act(void* stream, const void* x, const void* w,
                                   void* out, int M, int I, int K, int act) {
