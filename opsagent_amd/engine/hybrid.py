@@ -954,12 +954,11 @@ class GatedMLP(nn.Module):
         self.down_w = _param(_rand(gen, hidden, ff, std=1.0 / math.sqrt(ff), dtype=dtype))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        K = x.shape[1]
-        if (
-            K % 8 == 0 and self.ff % 8 == 0 and isinstance(self.act, str)
-            and ops.gateup_fused(x, self.gate_up_w, self.ff)
-        ):
-            act = ops.gateup_act(x, self.gate_up_w, self.ff, self.act)   # fused decode GEMV
+        form = None
+        if x.shape[1] % 8 == 0 and self.ff % 8 == 0 and isinstance(self.act, str):
+            form = ops._gateup_form(x, self.gate_up_w, self.ff)
+        if form:
+            act = ops.gateup_act(x, self.gate_up_w, self.ff, self.act, form)   # fused decode GEMV
         else:
             act = mx.act_mul_rows(ops.linear(x, self.gate_up_w), self.ff, self.act)
         return ops.linear(act, self.down_w)

@@ -46,18 +46,24 @@ _GEMV_MS = frozenset(range(1, 9))
 # take over. Default cap 2; OPSAGENT_GEMV_MAX_M overrides for experiments.
 
 
+# The mapping under os.environ, which changes with it: a lookup in it takes 0.05 us, one
+# through os.environ, where a variable is not set, 0.6 (it raises inside), and a product
+# of a short prompt makes several.
+_ENV = os.environ._data
+
+
 def _bf16_mfma_ok(M: int, K: int, gateup: bool = False) -> bool:
     """Mirror of gemv.hip's gemv_bf16_use_mfma: the staged MFMA kernel (M 3..8 unless
     OPSAGENT_BF16_GEMV_MFMA asks for others)."""
-    e = os.environ.get("OPSAGENT_BF16_GEMV_MFMA", "")
-    if e == "0":
+    e = _ENV.get(b"OPSAGENT_BF16_GEMV_MFMA", b"")
+    if e == b"0":
         return False
-    min_m = int(e[1:]) if e.startswith("m") else 3
+    min_m = int(e[1:]) if e.startswith(b"m") else 3
     if M < min_m or M > 16:
         return False
     if K % (512 if gateup else 1024) != 0:
         return False
-    if not e.startswith("m"):
+    if not e.startswith(b"m"):
         # measured win region only (see gemv.hip's gemv_bf16_use_mfma)
         if K > 6144 or M > 8:
             return False
@@ -65,16 +71,14 @@ def _bf16_mfma_ok(M: int, K: int, gateup: bool = False) -> bool:
 
 
 def _gemv_m_ok(M: int) -> bool:
-    import os
-
-    cap = int(os.environ.get("OPSAGENT_GEMV_MAX_M", "2"))
+    cap = int(_ENV.get(b"OPSAGENT_GEMV_MAX_M", 2))
     return M in _GEMV_MS and M <= cap
 
 
 def _gemv_switched() -> bool:
     """OPSAGENT_BF16_GEMV_MFMA or OPSAGENT_GEMV_MAX_M is set: the two choose between the
     staged GEMVs and the library, and the newer forms step aside for both."""
-    return "OPSAGENT_BF16_GEMV_MFMA" in os.environ or "OPSAGENT_GEMV_MAX_M" in os.environ
+    return b"OPSAGENT_BF16_GEMV_MFMA" in _ENV or b"OPSAGENT_GEMV_MAX_M" in _ENV
 
 
 def _two_rows_valu(M: int, K: int) -> bool:
@@ -130,6 +134,7 @@ def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+_compiling = torch.compiler.is_compiling
 _traced = torch._C._get_tracing_state
 _transform = torch._C._functorch.maybe_current_level
 _modes = torch._C._len_torch_dispatch_stack
@@ -139,7 +144,7 @@ def _plain_call(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Nobody asks for gradients or tangents, traces or transforms the call: a kernel sees
     addresses alone, the library's product is an operation that all of these know."""
     return not (
-        torch.compiler.is_compiling() or _traced() is not None or _transform() is not None
+        _compiling() or _traced() is not None or _transform() is not None
         or _modes() or forward_ad._current_level >= 0
         or ((x.requires_grad or w.requires_grad) and torch.is_grad_enabled())
     ) and type(x) in _PLAIN and type(w) in _PLAIN
@@ -865,42 +870,52 @@ def gateup_silu(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> torch
 
     GPU decode: one fused HIP kernel, no [*, 2I] intermediate, where gateup_fused
     says so. Otherwise: library GEMM + the silu_mul kernel."""
-    if gateup_fused(x, gate_up_w, i_local):
-        return gateup_act(x, gate_up_w, i_local)
+    form = _gateup_form(x, gate_up_w, i_local)
+    if form:
+        return gateup_act(x, gate_up_w, i_local, form=form)
     return silu_halves(linear(x, gate_up_w), i_local)
 
 
+def _gateup_form(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int):
+    """What takes this product in one launch, None if nothing does: ("ring", plan) and
+    ("skinny", form), the transfer ring and the skinny matrix-core product where they win;
+    ("staged", None), the VALU GEMV up to two rows and the staged matrix-core GEMV for what
+    3 to 8 rows are left."""
+    K = x.shape[-1]
+    M = x.numel() // K
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and K % 8 == 0 and x.is_contiguous()
+            and gate_up_w.is_contiguous()):
+        return None
+    if 1 < M <= 128 and _skinny_ok(x, gate_up_w) and gate_up_w.shape[0] == 2 * i_local:
+        plan = _ring_plan(M, i_local, K, gateup=True)
+        if plan:
+            return "ring", plan
+        form = _skinny_form(M, i_local, K, gateup=True)
+        if form:
+            return "skinny", form
+    return ("staged", None) if _gemv_m_ok(M) or _bf16_mfma_ok(M, K, gateup=True) else None
+
+
 def gateup_fused(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> bool:
-    """Whether gateup_act takes this product in one launch: the VALU GEMV up to
-    two rows, the transfer ring and the skinny matrix-core product where they win, the
-    staged matrix-core GEMV for what 3 to 8 rows are left."""
-    M, K = x.numel() // x.shape[-1], x.shape[-1]
-    return (
-        x.is_cuda and x.dtype == torch.bfloat16 and K % 8 == 0 and x.is_contiguous()
-        and gate_up_w.is_contiguous()
-        and (_gemv_m_ok(M) or _bf16_mfma_ok(M, K, gateup=True)
-             or (M <= 128 and _skinny_ok(x, gate_up_w) and gate_up_w.shape[0] == 2 * i_local
-                 and (_ring_plan(M, i_local, K, gateup=True) is not None
-                      or _skinny_form(M, i_local, K, gateup=True) > 0)))
-    )
+    """Whether gateup_act takes this product in one launch."""
+    return _gateup_form(x, gate_up_w, i_local) is not None
 
 
 def gateup_act(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int,
-               act: str = "silu") -> torch.Tensor:
+               act: str = "silu", form=None) -> torch.Tensor:
     """act(x @ gate^T) * (x @ up^T), act "silu" | "gelu_tanh", for decode-sized
-    bf16 batches that gateup_fused names: one launch."""
+    bf16 batches that gateup_fused names: one launch. form: _gateup_form's answer, where the
+    caller has asked it."""
     from opsagent_amd.ops import hip_lib
 
     M = x.numel() // x.shape[-1]
     assert x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous()
     assert act in ("silu", "gelu_tanh")
-    if M > 1 and _skinny_ok(x, gate_up_w) and gate_up_w.shape[0] == 2 * i_local:
-        plan = _ring_plan(M, i_local, x.shape[-1], gateup=True)
-        if plan:
-            return _ring(x, gate_up_w, plan, act=1 + int(act == "gelu_tanh"))
-        form = _skinny_form(M, i_local, x.shape[-1], gateup=True)
-        if form:
-            return _skinny(x, gate_up_w, form, gateup=True, act=int(act == "gelu_tanh"))
+    kind, plan = form or _gateup_form(x, gate_up_w, i_local) or ("staged", None)
+    if kind == "ring":
+        return _ring(x, gate_up_w, plan, act=1 + int(act == "gelu_tanh"))
+    if kind == "skinny":
+        return _skinny(x, gate_up_w, plan, gateup=True, act=int(act == "gelu_tanh"))
     lib = hip_lib.get_lib()
     out = torch.empty(*x.shape[:-1], i_local, dtype=x.dtype, device=x.device)
     rc = lib.oa_gemv_gateup_act(
