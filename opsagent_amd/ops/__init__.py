@@ -85,11 +85,12 @@ def _two_rows_valu(M: int, K: int) -> bool:
     """Two rows that the VALU GEMV takes better than the matrix-core forms (us, VALU /
     best of those, 2 GB of weights in turn: gate-up 2 x 14336 x 4096 41.1 / 45.3, 6144 x
     4096 10.7 / 12.7, 5120 x 5120 10.7 / 13.5, 32000 x 2048 25.1 / 26.0, 4096 x 4096 8.5 /
-    8.2), long rows (4096 x 14336 26.6 / 23.0) apart."""
-    return M == 2 and K <= 8192 and _gemv_m_ok(M)
+    8.2), long rows (4096 x 14336 26.6 / 23.0) and short ones (2048 x 128 2.7 / 2.1, 4096 x
+    256 3.0 / 2.7, 1024 x 512 2.6 / 2.6; gate-up 2 x 2048 x 128 3.1 / 2.4) apart."""
+    return M == 2 and 256 < K <= 8192 and _gemv_m_ok(M)
 
 
-def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
+def _skinny_form(M: int, N: int, K: int, gateup: bool = False, strided: bool = False) -> int:
     """Which form of the skinny product (skinny.hip; figures there) takes M rows
     of K columns against N (gate-up: 2N) weight rows: 0 none, 1 strips, 2
     persistent.
@@ -108,11 +109,15 @@ def _skinny_form(M: int, N: int, K: int, gateup: bool = False) -> int:
     2 x 3584 16.5 / 13.8) and N >= 6144 up to 16 rows, N >= 16384 up to 32. Under 2^18
     weights the library stays for its order of sums, not for its speed: a pair of equal
     choices in a small routed model falls the other way with strips, which take 2.5 us
-    against 4.3 (480 x 512, 3 rows; 512 x 512 2.5 / 4.3, 64 x 2048, 32 rows 7.1 / 7.9)."""
+    against 4.3 (480 x 512, 3 rows; 512 x 512 2.5 / 4.3, 64 x 2048, 32 rows 7.1 / 7.9).
+    strided: rows of x that lie apart, which the VALU GEMV does not take. Two of them go to
+    strips (us, strips / library: 2048 x 128 2.1 / 3.4, 2048 x 2048 4.8 / 10.9, 8192 x 4096
+    14.1 / 16.9; the persistent form 18.4, the ring 14.0)."""
     R = 2 if gateup else 1
-    if M < 1 or M > 32 or K % 32 != 0 or R * N * K < 2 ** 18 or _two_rows_valu(M, K):
+    two = M == 2 and strided
+    if M < 1 or M > 32 or K % 32 != 0 or R * N * K < 2 ** 18 or (not two and _two_rows_valu(M, K)):
         return 0
-    if K == 4096 and (M <= 16 and N >= 8192 if gateup else N >= (6144 if M <= 16 else 16384)):
+    if K == 4096 and not two and (M <= 16 and N >= 8192 if gateup else N >= (6144 if M <= 16 else 16384)):
         return 2
     blocks = -(-N // 16)
     if K < 2048 and not gateup and blocks > (256 if M <= 8 else 512):
@@ -266,7 +271,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         plan = _ring_plan(M, w.shape[0], w.shape[1])
         if plan:
             return _ring(x, w, plan)
-        form = _skinny_form(M, w.shape[0], w.shape[1])
+        form = _skinny_form(M, w.shape[0], w.shape[1], strided=not x.is_contiguous())
         if form:
             return _skinny(x, w, form)
     if (

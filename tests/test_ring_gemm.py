@@ -148,6 +148,12 @@ def test_lines_between_the_forms():
     assert forms(8, 18432, 7168, True) == (None, 0)
     for N, K, gateup in ((512, 1024, True), (18432, 5120, False), (256, 2048, False)):
         assert forms(2, N, K, gateup) == (None, 0)
+    # two rows of few columns, and two that lie apart
+    assert forms(2, 2048, 128) == forms(2, 2048, 256) == forms(2, 1024, 256, True) == (None, 1)
+    assert forms(2, 2048, 288) == (None, 0)
+    assert [ops._skinny_form(2, N, K, strided=True) for N, K in
+            ((2048, 128), (2048, 288), (4096, 4096), (8192, 4096), (512, 480))] == [1, 1, 1, 1, 0]
+    assert ops._skinny_form(8, 8192, 4096, strided=True) == 2
 
 
 @pytest.mark.gpu

@@ -186,3 +186,15 @@ def test_gradients_and_transforms(M):
     assert _err(each[1], library.double()) < 4e-3
     with torch.no_grad():
         assert torch.equal(ops.linear(v, p), plain)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K", [(2048, 128), (2040, 288), (4096, 4096), (1000, 8192)])
+def test_two_rows_that_lie_apart(N, K):
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(2, K + 64, generator=gen, device="cuda").bfloat16()[:, 32 : 32 + K]
+    w = (torch.randn(N, K, generator=gen, device="cuda") * K ** -0.5).bfloat16()
+    assert ops._skinny_form(2, N, K, strided=True) == 1
+    got = ops.linear(x, w)
+    assert torch.equal(got, ops._skinny(x, w, 1))
+    assert _err(got, x.double() @ w.double().T) < _tol(got)
