@@ -81,13 +81,16 @@ def _gemv_switched() -> bool:
     return b"OPSAGENT_BF16_GEMV_MFMA" in _ENV or b"OPSAGENT_GEMV_MAX_M" in _ENV
 
 
-def _two_rows_valu(M: int, K: int) -> bool:
+def _two_rows_valu(M: int, N: int, K: int, gateup: bool = False) -> bool:
     """Two rows that the VALU GEMV takes better than the matrix-core forms (us, VALU /
     best of those, 2 GB of weights in turn: gate-up 2 x 14336 x 4096 41.1 / 45.3, 6144 x
     4096 10.7 / 12.7, 5120 x 5120 10.7 / 13.5, 32000 x 2048 25.1 / 26.0, 4096 x 4096 8.5 /
-    8.2), long rows (4096 x 14336 26.6 / 23.0) and short ones (2048 x 128 2.7 / 2.1, 4096 x
-    256 3.0 / 2.7, 1024 x 512 2.6 / 2.6; gate-up 2 x 2048 x 128 3.1 / 2.4) apart."""
-    return M == 2 and 256 < K <= 8192 and _gemv_m_ok(M)
+    8.2, 14336 x 384 5.0 / 5.6), long rows (4096 x 14336 26.6 / 23.0), short ones (2048 x 128
+    2.7 / 2.1, 14336 x 256 4.6 / 4.5; gate-up 2 x 2048 x 128 3.1 / 2.4, 2 x 512 x 512 2.9 /
+    3.2) and few of them (1024 x 640 3.2 / 2.8, 1024 x 1024 3.2 / 3.8) apart."""
+    if M != 2 or K > 8192 or K <= 256 or (not gateup and K < 1024 and N * K <= 2 ** 20):
+        return False
+    return _gemv_m_ok(M)
 
 
 def _skinny_form(M: int, N: int, K: int, gateup: bool = False, strided: bool = False) -> int:
@@ -104,9 +107,13 @@ def _skinny_form(M: int, N: int, K: int, gateup: bool = False, strided: bool = F
     1024 x 2816, 28 10.3 / 10.9 and 32 10.9 / 9.3; 5120 x 13824, 3 39.1 / 28.4. Up to eight rows the staged
     GEMV is the other form where it runs, and strips are the faster one (12288 x 6144, 8
     35.0 / 41.2), except for rows too short to pipeline, four steps a wave, in more than
-    one round (32000 x 1024, 8 19.9 / 16.0; the library 17.2). The persistent form is for
-    blocks that go over several strips: gate-up from N = 8192 on (2 x 11008, 8 36.2 / 38.4;
-    2 x 3584 16.5 / 13.8) and N >= 6144 up to 16 rows, N >= 16384 up to 32. Under 2^18
+    one round (32000 x 1024, 8 19.9 / 16.0; the library 17.2). Against the library strips
+    of rows under 2048 columns pay in two rounds (8192 x 1408, 5 8.3 / 10.1), in more of
+    them with up to 512 columns (14336 x 128, 8 3.5 / 5.0, 31 4.3 / 4.4; 32000 x 512, 17
+    14.5 / 17.9; but 32000 x 64, 8 4.8 / 4.6, 65536 x 256, 8 14.1 / 10.4), and with up to 768
+    from 17 rows on (14336 x 768, 16 10.1 / 8.4, 24 11.9 / 17.4; 16384 x 768, 24 12.3 / 10.7).
+    The persistent form is for blocks that go over several strips: gate-up from N = 8192
+    on (2 x 11008, 8 36.2 / 38.4; 2 x 3584 16.5 / 13.8) and N >= 6144 up to 16 rows, N >= 16384 up to 32. Under 2^18
     weights the library stays for its order of sums, not for its speed: a pair of equal
     choices in a small routed model falls the other way with strips, which take 2.5 us
     against 4.3 (480 x 512, 3 rows; 512 x 512 2.5 / 4.3, 64 x 2048, 32 rows 7.1 / 7.9).
@@ -115,14 +122,23 @@ def _skinny_form(M: int, N: int, K: int, gateup: bool = False, strided: bool = F
     14.1 / 16.9; the persistent form 18.4, the ring 14.0)."""
     R = 2 if gateup else 1
     two = M == 2 and strided
-    if M < 1 or M > 32 or K % 32 != 0 or R * N * K < 2 ** 18 or (not two and _two_rows_valu(M, K)):
+    if M < 1 or M > 32 or K % 32 != 0 or R * N * K < 2 ** 18 or (
+            not two and _two_rows_valu(M, N, K, gateup)):
         return 0
     if K == 4096 and not two and (M <= 16 and N >= 8192 if gateup else N >= (6144 if M <= 16 else 16384)):
         return 2
     blocks = -(-N // 16)
-    if K < 2048 and not gateup and blocks > (256 if M <= 8 else 512):
-        return 0
-    if M > 2 and _bf16_mfma_ok(M, K, gateup):
+    staged = M > 2 and _bf16_mfma_ok(M, K, gateup)
+    if K < 2048 and not gateup and blocks > 256:
+        if K <= 512:
+            rounds = (4 if K < 256 else 8) if M < 32 else 3.5 if K <= 128 else 2
+        else:
+            rounds = 2 if M <= 16 or K > 768 else 3.5
+        if (staged and not strided) or blocks > 256 * rounds:
+            return 0
+        if K <= 512:
+            return 1
+    if staged:
         return 1
     if M <= 16:
         col = (2.5 + 0.06 * M) if gateup else (1.3 + 0.05 * M)
@@ -187,7 +203,8 @@ def _ring_plan(M: int, N: int, K: int, gateup: bool = False) -> Optional[Tuple[i
     The lines, measured at 2 to 128 rows over 64 weights, 2 GB of them in turn (us,
     other / ring): light weights end before the ring pays for its start (4096 x 4096,
     M = 8 9.1 / 10.8, 24 13.4 / 11.7; gate-up 2 x 2816 x 2048, 24 10.6 / 10.7, 47
-    15.4 / 12.8, 112 16.7 / 17.8), short rows at few rows too (2 x 8192 x 2048, 8 14.5 /
+    15.4 / 12.8, 112 16.7 / 17.8; but where two tiles of 64 rows fill the CUs 2 x 8192 x 640,
+    128 14.1 / 11.0, 2 x 4096 x 1408 18.9 / 16.5), short rows at few rows too (2 x 8192 x 2048, 8 14.5 /
     14.7; 2 x 8192 x 3072 23.0 / 20.3), long ones less (2048 x 8192, 8 12.6 / 11.3).
     Column splits fill the CUs; less than 0.8 of the last round filled loses (12288 x
     4096, 24 22.7 / 25.0), and at two or three rows so does adding up many splits (4096 x
@@ -207,18 +224,20 @@ def _ring_plan(M: int, N: int, K: int, gateup: bool = False) -> Optional[Tuple[i
     round (32000 x 1024, 112 24.2 / 25.4). Without splits tiles of 96 pay in one round or
     from rows of 4096 on (128256 x 2048, 96 130 / 132, 32000 x 2048 32.5 / 30.8, 128256 x
     4096 228 / 225), tiles of 128 not at all (2 x 14336 x 4096, 58.0 / 59.5)."""
-    if not 1 < M <= 128 or K % 64 or K < 256 or N % 8 or _two_rows_valu(M, K):
+    if not 1 < M <= 128 or K % 64 or K < 256 or N % 8 or _two_rows_valu(M, N, K, gateup):
         return None
     weights = (2 if gateup else 1) * N * K
     if M <= 16:
         ok = weights >= (2 ** 24 if K >= 8192 else 24e6 if K >= 4096 else 40e6 if K >= 3072 else 60e6)
     else:
-        ok = weights >= (10e6 if gateup and 32 < M <= 80 else 2 ** 24)
+        ok = weights >= (10e6 if gateup and M > 32 else 2 ** 24)
     if not ok:
         return None
     strips = -(-N // (64 if gateup else 128))
     one = 32 * -(-M // 32)
     two = M > 64 and weights < (2 ** 25 if M > 96 else 2 ** 24 + 1)
+    if gateup and M > 80 and weights < 2 ** 24:
+        one = 64
     for tile in (64, one) if two else (one,):
         tiles = strips * -(-M // tile)
         splits = max(1, min(256 // tiles, K // 256))

@@ -149,10 +149,20 @@ def test_lines_between_the_forms():
     for N, K, gateup in ((512, 1024, True), (18432, 5120, False), (256, 2048, False)):
         assert forms(2, N, K, gateup) == (None, 0)
     # two rows of few columns, and two that lie apart
-    assert forms(2, 2048, 128) == forms(2, 2048, 256) == forms(2, 1024, 256, True) == (None, 1)
-    assert forms(2, 2048, 288) == (None, 0)
+    assert forms(2, 2048, 128) == forms(2, 4112, 256) == forms(2, 1024, 256, True) == (None, 1)
+    assert forms(2, 2048, 512) == (None, 1) and forms(2, 2064, 512) == (None, 0)
+    assert forms(2, 512, 512, True) == forms(2, 1024, 1024) == (None, 0)
     assert [ops._skinny_form(2, N, K, strided=True) for N, K in
-            ((2048, 128), (2048, 288), (4096, 4096), (8192, 4096), (512, 480))] == [1, 1, 1, 1, 0]
+            ((2048, 128), (2064, 512), (4096, 4096), (8192, 4096), (512, 480))] == [1, 1, 1, 1, 0]
+    # strips of short rows in several rounds
+    assert forms(8, 14336, 128) == forms(31, 16384, 128) == forms(17, 32000, 512) == (None, 1)
+    assert forms(32, 16384, 128) == forms(8, 32000, 64) == forms(8, 65536, 256) == (None, 0)
+    assert forms(5, 8192, 1408) == forms(24, 14336, 768) == (None, 1)
+    assert forms(16, 14336, 768) == forms(24, 16384, 768) == forms(5, 8208, 1408) == (None, 0)
+    assert [ops._skinny_form(8, 8192, 1024, strided=far) for far in (False, True)] == [0, 1]
+    # two tiles of 64 rows on light gate-up weights
+    assert ops._ring_plan(128, 8192, 640, True) == (64, 1)
+    assert ops._ring_plan(128, 4096, 1408, True) == (64, 2)
     assert ops._skinny_form(8, 8192, 4096, strided=True) == 2
 
 

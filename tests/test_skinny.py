@@ -42,6 +42,19 @@ def test_skinny(M, N, K, form):
         assert ops._skinny_ok(x, w)
         got = ops._skinny(x, w, form)
         assert _err(got, x.double() @ w.double().T) < _tol(got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(2, 4104, 192), (8, 14344, 128), (31, 16384, 96), (17, 32000, 288),
+                                   (24, 14336, 768)])
+@pytest.mark.parametrize("far", [0, 64])
+def test_short_rows(M, N, K, far):
+    gen = torch.Generator(device="cuda").manual_seed(N + M)
+    x = torch.randn(M, K + far, generator=gen, device="cuda").bfloat16()[:, :K]
+    w = (torch.randn(N, K, generator=gen, device="cuda") * K ** -0.5).bfloat16()
+    got = ops.linear(x, w)
+    assert torch.equal(got, ops._skinny(x, w, 1))
+    assert _err(got, x.double() @ w.double().T) < _tol(got)
     assert not ops._skinny_ok(wide[:, 3 : 3 + K], w)          # rows start off 16 bytes
     if form == 2 and M > 16:
         return
@@ -189,12 +202,25 @@ def test_gradients_and_transforms(M):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("N,K", [(2048, 128), (2040, 288), (4096, 4096), (1000, 8192)])
+@pytest.mark.parametrize("N,K", [(2048, 128), (2040, 288), (4096, 4096), (1000, 4096)])
 def test_two_rows_that_lie_apart(N, K):
     gen = torch.Generator(device="cuda").manual_seed(N)
     x = torch.randn(2, K + 64, generator=gen, device="cuda").bfloat16()[:, 32 : 32 + K]
     w = (torch.randn(N, K, generator=gen, device="cuda") * K ** -0.5).bfloat16()
     assert ops._skinny_form(2, N, K, strided=True) == 1
+    got = ops.linear(x, w)
+    assert torch.equal(got, ops._skinny(x, w, 1))
+    assert _err(got, x.double() @ w.double().T) < _tol(got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(2, 4104, 192), (8, 14344, 128), (31, 16384, 96), (17, 32000, 288),
+                                   (24, 14336, 768)])
+@pytest.mark.parametrize("far", [0, 64])
+def test_short_rows(M, N, K, far):
+    gen = torch.Generator(device="cuda").manual_seed(N + M)
+    x = torch.randn(M, K + far, generator=gen, device="cuda").bfloat16()[:, :K]
+    w = (torch.randn(N, K, generator=gen, device="cuda") * K ** -0.5).bfloat16()
     got = ops.linear(x, w)
     assert torch.equal(got, ops._skinny(x, w, 1))
     assert _err(got, x.double() @ w.double().T) < _tol(got)
