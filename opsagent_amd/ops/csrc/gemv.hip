@@ -361,7 +361,12 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
     // Else: as many blocks of eight waves as stay resident (two per CU by registers, four
     // with short rows), fewer and fuller ones where that evens out the CUs by more than a
     // fifth.
-    const int wv = K == 4096 || (K == 2048 && (gateup ? N > 2048 && N <= 4096 : N > 4096)) ? 4 : 8;
+    // A norm makes the image of every block dearer: with one, gate-up of up to 8192 rows and
+    // few plain rows stay with eight waves (us, eight / four: 2 x 4096 x 4096 12.5 / 13.8, 2
+    // x 1408 x 4096 5.8 / 7.0, 2 x 9216 x 4096 27.4 / 26.2; 512 x 4096 4.2 / 4.5, 2048 x 4096
+    // 5.1 / 4.8).
+    const bool dear = (mode & 1) && (gateup ? N <= 8192 : N <= 1024);
+    const int wv = (K == 4096 && !dear) || (K == 2048 && (gateup ? N > 2048 && N <= 4096 : N > 4096)) ? 4 : 8;
     int per;
     if (wv == 4) {
         per = CEIL_DIV(N, 256 * 4 * 32);

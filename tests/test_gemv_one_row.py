@@ -96,3 +96,17 @@ def test_three_rows_a_wave():
     for got, ref in ((ops.linear_addres(x, w, res), want),
                      (ops.linear_addres_fp8(x, wq, ws, res), want8)):
         assert ((got.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4).all()
+
+
+@pytest.mark.gpu
+def test_blocks_of_four_and_eight_waves_agree():
+    """Both sides of the lines between them: the same sums in the same order."""
+    K, gen = 4096, torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(1, K, generator=gen, device="cuda").bfloat16()
+    nw = (1.0 + 0.1 * torch.randn(K, generator=gen, device="cuda")).bfloat16()
+    w = (torch.randn(16400, K, generator=gen, device="cuda") * K ** -0.5).bfloat16()
+    few = torch.cat([w[:8192], w[8200:16392]])
+    assert torch.equal(ops.gateup_silu_norm(x, nw, 1e-5, w, 8200)[:, :8192],
+                       ops.gateup_silu_norm(x, nw, 1e-5, few, 8192))
+    assert torch.equal(ops.linear_norm(x, nw, 1e-5, w[:1025])[:, :1024],
+                       ops.linear_norm(x, nw, 1e-5, w[:1024]))
