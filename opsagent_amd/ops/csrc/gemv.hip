@@ -370,7 +370,10 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
     int per;
     if (wv == 4) {
         per = CEIL_DIV(N, 256 * 4 * 32);
-        if (!gateup && per < 2) per = 2;
+        // one row a wave where two leave CUs uneven by a sixth (us, two / one: 5120 x 4096 9.8 /
+        // 9.5, 3072 x 4096 7.0 / 6.6, 512 x 4096 4.6 / 3.8)
+        const int one = CEIL_DIV(CEIL_DIV(N, 4), 256), two = 2 * CEIL_DIV(CEIL_DIV(N, 8), 256);
+        if (!gateup && per < 2 && two * 5 < one * 6) per = 2;
     } else {
         auto rounds = [&](int p) { return CEIL_DIV(CEIL_DIV(CEIL_DIV(N, p), 8), 256) * p; };
         per = CEIL_DIV(N, 2048 * (K == 2048 && !gateup ? 4 : 2));
