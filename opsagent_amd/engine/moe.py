@@ -107,7 +107,8 @@ class MoEMLP(nn.Module):
                 idx, wts, tok = ops.moe_route(x, self.router_w, self.top_k)
                 local = self.shared is not None and get_tp_size() == 1
                 shared = self.shared(x) if local else None
-                if tiles and not (few and not ops.moe_sorted_wins(P, self.num_experts, self.fp8)):
+                if tiles and not (few and not ops.moe_sorted_wins(P, self.num_experts, self.fp8,
+                                                                    self.i_local * H)):
                     out = ops.moe_sorted_mlp(x, w13, s13, w2, s2, idx, wts, more=shared)
                 else:
                     y = ops.moe_grouped_mlp(x, w13, s13, w2, s2, idx.view(-1), tok.view(-1),
@@ -273,7 +274,7 @@ class RoutedExperts(nn.Module):
                 and C % 16 == 0 and I % 16 == 0 and self.force_path is None):
             # the framework's grouped expert GEMV kernels (pair- or expert-major)
             if (ops.moe_sorted_ok(x, self.w13, self.w2, self.act)
-                    and ops.moe_sorted_wins(T * top, self.r.experts, False)):
+                    and ops.moe_sorted_wins(T * top, self.r.experts, False, I * C)):
                 return ops.moe_sorted_mlp(x, self.w13, None, self.w2, None, idx, wts, self.act)
             flat_t = torch.arange(T, device=x.device, dtype=torch.int32).repeat_interleave(top)
             y = ops.moe_grouped_mlp(x.contiguous(), self.w13, None, self.w2, None,

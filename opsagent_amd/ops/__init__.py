@@ -682,31 +682,51 @@ def moe_combine(y: torch.Tensor, top: int, more: Optional[torch.Tensor] = None) 
     return out
 
 
-def moe_sorted_wins(pairs: int, experts: int, fp8: bool) -> bool:
-    """Sorted tiles against a weight stream per pair, measured in graphs (both
-    products and the sort, us): 64 experts of 1408 x 2048, fp8: 24 pairs 47 to
-    49, 48 pairs 82 to 91, 78 pairs 102 to 144; bf16: 48 pairs 148 to 130, 78
-    pairs 181 to 204. 16 experts of 1024 x 2048, fp8: 16 pairs 34 to 25, 32
-    pairs 35 to 47; bf16: 32 pairs 62 to 65, 52 pairs 64 to 100."""
-    return pairs >= (max(24, experts // 2) if fp8 else max(32, experts))
+def moe_sorted_wins(pairs: int, experts: int, fp8: bool, weights: int = 0) -> bool:
+    """Sorted tiles against a weight stream per pair; weights is the size of one expert
+    matrix, 0 if unknown. Us in graphs, both products, the sort and the sum, pairs / sorted.
+    64 experts of 1408 x 2048, fp8: 6 pairs 22 / 28, 12 33 / 30, 24 53 / 44; bf16: 24 pairs
+    77 / 77, 36 107 / 96. 128 of 768 x 2048, fp8: 24 36 / 38, 32 44 / 39; bf16: 40 73 / 71, 48
+    87 / 84. 16 of 1024 x 2048, fp8: 12 24 / 25, 16 29 / 25; bf16: 12 34 / 37, 16 40 / 38. 8 of
+    14336 x 4096, fp8: 2 pairs 83 / 98, 4 148 / 123; bf16: 4 193 / 217, 6 322 / 255. Small
+    matrices are launches either way: 16 of 512 x 1024, fp8: 24 17 / 18, 32 20 / 18; bf16: 24
+    19 / 21, 32 22 / 21."""
+    heavy = 3 * weights * pairs >= 10 ** 8
+    if fp8:
+        return pairs >= max(32, experts // 4) or heavy and pairs >= max(4, experts // 6)
+    return pairs >= max(32, 3 * experts // 8) or heavy and pairs >= max(6, experts // 2)
 
 
 def _moe_tile_rows(pairs: int, experts: int, weights: int, fp8: bool) -> int:
-    """Rows of a tile of moe_sorted_mlp, by the rows that an expert has on average; weights
-    is the size of one expert matrix. The same bits with any of them.
-
-    Both products and the sort in graphs, us with 16 / 64 rows. fp8, 64 experts of 1408 x
-    2048: 1.5 rows 110 / 116, 4 rows 119 / 123, 6 rows 133 / 129; 128 of 768 x 2048: 1.5 rows
-    112 / 126, 4 rows 130 / 136. bf16: 206 / 198, 224 / 219, 244 / 229; 203 / 201, 243 / 235.
-    A tile slot that P pairs may need but mostly do not leaves a die short of work when there
-    are few experts: 16 bf16 experts of 1024 x 2048 48 pairs 68 / 54, 64 pairs 67 / 71; 8 of
-    14336 x 4096, 32 pairs 595 / 501; small matrices are launches either way, 16 of 512 x
-    1024, 48 pairs 25 / 26. 64 / 128 rows, 64 experts of 1408 x 2048, bf16: 48 rows 307 / 297,
-    96 rows 378 / 385, 192 rows 582 / 501."""
+    """Rows of an expert tile for operands that a block holds one step ahead, by the pairs:
+    16 or 64 up to four rows an expert, 64 below 128 rows, 128 from there on."""
     if pairs <= 4 * experts:
         wide = not fp8 and experts * weights >= 2 ** 24 and (pairs < 64 or experts >= 64)
         return 64 if wide else 16
     return 64 if pairs < 128 * experts else 128
+
+
+def _moe_ring_rows(pairs: int, experts: int, weights: int, fp8: bool) -> int:
+    """Rows of a tile of moe_sorted_mlp, by the rows that an expert has on average; weights
+    is the size of one expert matrix. The same bits with any of them.
+
+    A narrow tile costs a strip read again for every further tile of its expert, a wide one
+    LDS reads for rows that are not there. Both products in graphs, us with 16 / 32 / 64 rows.
+    fp8, 64 experts of 1408 x 2048: 2 rows 83 / 84 / 97, 8 90 / 92 / 100, 16 112 / 95 / 105, 24
+    134 / 102 / 107, 32 153 / 128 / 116; 8 of 14336 x 4096: 8 rows 216 / 219 / 295, 24 311 / 227 /
+    298, 32 391 / 326 / 304. bf16: 2 rows 160 / 158 / 167, 8 181 / 183 / 188, 16 207 / 187 / 191,
+    24 234 / 192 / 195, 32 270 / 218 / 202. Small matrices have too few strips to go round the
+    CUs, so that narrow tiles pay for longer: 16 fp8 experts of 512 x 1024, 16 rows 13.4 / 15.0 /
+    19.8, 32 15.7 / 15.5 / 20.6, 96 24.4 / 18.2 / 20.7, 192 39 / 30 / 25; bf16 96 rows 31 / 22 / 22.
+    64 / 128 rows, bf16 (fp8 has no room for a second block of 128): 64 experts of 1408 x 2048,
+    48 rows 213 / 239, 64 263 / 252, 192 429 / 404; 128 of 768 x 2048, 48 rows 242 / 255, 64 287 /
+    286; 16 of 512 x 1024, 192 rows 27 / 34."""
+    small = weights < 2 ** 20
+    if pairs <= (16 if small else 8) * experts:
+        return 16
+    if pairs <= (96 if small else 24) * experts:
+        return 32
+    return 64 if small or fp8 else _moe_tile_rows(2 * pairs, experts, weights, fp8)
 
 
 def moe_sorted_ok(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, act=None) -> bool:
@@ -749,7 +769,7 @@ def moe_sorted_mlp(
     assert expert_ids.shape == pair_weights.shape == (T, top)
     assert (w13.dtype == torch.uint8) == (w13_scale is not None) == (w2_scale is not None)
     P = T * top
-    bm = _moe_tile_rows(P, E, I * H, w13_scale is not None)
+    bm = _moe_ring_rows(P, E, I * H, w13_scale is not None)
     max_tiles = P // bm + min(E, P)
     lib, hip = _lib()
     stream, dev = hip.current_stream_ptr(), x.device

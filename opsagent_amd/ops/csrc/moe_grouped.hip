@@ -17,8 +17,6 @@
 // one order: the output does not depend on how pairs are placed in an expert.
 // Activations are bf16; weights bf16, or fp8 (e4m3, one float32 scale per row)
 // widened exactly to bf16 in registers. Sums are float32.
-#include <type_traits>
-
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) unsigned int mgu4;
@@ -238,135 +236,137 @@ __device__ __forceinline__ mgs8 mg_widen(uint32_t lo, uint32_t hi) {
     return r.v;
 }
 
-// A block of four waves takes BM sorted rows of one expert and 128 of its weight
-// rows (64 gate and the 64 up rows beside them). Weight rows go from memory
-// straight into the A fragments of v_mfma_f32_16x16x32_bf16, one 128-column step
-// ahead: 16 rows x 64 bytes per load reach 6.0 TB/s with plain loads (5.2 with
-// non-temporal ones, 6.4 for whole contiguous rows) and need no LDS. The
-// activation rows, which all four waves read, are staged in LDS in two buffers
-// with one barrier per step; 16-byte chunks are XORed with the row so that a
-// fragment read touches every bank once. Grid: work items in an order that puts
-// the row tiles of one expert and weight strip next to each other on ONE die
-// (block ids go round the eight dies), so the strip is read from memory once.
-template <int BM, bool FP8, int MODE>
-__global__ __launch_bounds__(256, BM > 64 ? 2 : 3) void moe_grouped_kernel(
+template <int V>
+__device__ __forceinline__ void mg_wait() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(V) : "memory");
+}
+
+// A block of four waves takes BM sorted rows of one expert and 128 of its weight rows (64
+// gate and the 64 up rows beside them); a wave all rows by 32 of the strip, weights as the
+// first operand of v_mfma_f32_16x16x32_bf16.
+//
+// What bounds it is the weight stream, up to some hundred rows an expert. Both operands come
+// by 16-byte transfers straight into a ring of STAGES steps in LDS (a step: 128 bytes of every
+// weight row and the same columns of the activation rows, whose addresses the lanes gather by
+// expert), STAGES - 1 under way, two blocks a CU so that one streams while the other starts or
+// ends. 16-byte chunk c of a 128-byte row r lies at c ^ (r >> 1 & 7), of a 256-byte one at c ^
+// (r & 15): the rows of a fragment read touch every bank once. Weights of an expert with one
+// row tile are read without being kept (nt), those of more tiles are met again in the die's L2.
+// Work items are in an order that puts the row tiles of one expert and strip next to each
+// other on ONE die (block ids go round the eight dies), and the dies share the items in use.
+//
+// Us over 2 GB of weights, up + down, with weight rows loaded one step ahead into registers
+// (before) / here: 64 experts of 1408 x 2048, top 6, fp8: 13 tokens 63 + 36 / 47 + 27, 64
+// tokens 78 + 47 / 57 + 32, 512 tokens 123 + 76 / 81 + 47; bf16: 8 tokens 92 + 56 / 65 + 32,
+// 64 tokens 142 + 76 / 118 + 58, 512 tokens 201 + 111 / 134 + 72, 2048 tokens 317 + 192 /
+// 233 + 158. The stream runs at 5.5 to 6.3 TB/s up to 6 rows an expert. One block a CU with
+// six steps is slower (54 + 28 for 13 fp8 tokens), three with two are as fast (51 + 24).
+template <int BM, int STAGES, bool FP8, int MODE>
+__global__ __launch_bounds__(256, 2) void moe_grouped_kernel(
     const uint16_t* __restrict__ x, const char* __restrict__ w, const float* __restrict__ wscale,
     const int* __restrict__ off, const int* __restrict__ pre, const int* __restrict__ tile_e,
     const int* __restrict__ perm, const float* __restrict__ pair_w, uint16_t* __restrict__ out,
     int E, int N, int K, int top, int strips, int act, float limit, float alpha) {
     constexpr int FM = BM / 16;                  // activation fragments
-    constexpr int XL = BM * 16 / 256;            // 16-byte chunks per thread and step
-    constexpr int WL = FP8 ? 2 : 4;              // weight loads per fragment and step
-    __shared__ __attribute__((aligned(16))) char xs[2][BM * 256];
-    __shared__ int rows_s[BM];
+    constexpr int XB = FP8 ? 256 : 128;          // bytes of an activation row in a step
+    constexpr int XT = BM * XB / 1024;           // transfers of them; of a wave:
+    constexpr int XPW = XT < 4 ? 1 : XT / 4;     // (two of 16 bf16 rows: waves repeat them)
+    constexpr int LPS = 4 + XPW, STEP = 128 * 128 + BM * XB;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
 
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int r = lane & 15, q = lane >> 4;
-    const int per = gridDim.x >> 3;              // work items per die
-    const int item = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    const int tiles = pre[E];
-    if (item >= tiles * strips) return;
+    const int items = pre[E] * strips, per = (items + 7) >> 3;
+    const int place = blockIdx.x >> 3, item = (blockIdx.x & 7) * per + place;
+    if (place >= per || item >= items) return;
     const int e = tile_e[item / strips];
     const int t0 = pre[e], mt = pre[e + 1] - t0;
     const int in = item - t0 * strips;
     const int strip = in / mt, mtile = in - strip * mt;
     const int s0 = off[e] + mtile * BM;
     const int m = min(BM, off[e + 1] - s0);
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t rb = FP8 ? (int64_t)K : 2 * (int64_t)K;    // bytes of a weight row
+    const int ns = (int)(rb / 128);
 
-    // source row of every activation row (rows past the end repeat the last one)
-    if (tid < BM) {
-        const int s = s0 + min(tid, m - 1);
-        rows_s[tid] = MODE == 0 ? s : perm[s] / top;
+    // this lane's row and chunk of every transfer; weight rows past N repeat the last one,
+    // rows past the end of the expert's too
+    const char* src[LPS];
+    uint32_t dst[LPS];
+    const char* we = w + (int64_t)e * (MODE == 1 ? 2 * N : N) * rb;
+    const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const int row = (wid * 4 + p) * 8 + (lane >> 3);
+        int64_t at;
+        if (MODE == 1) at = min(strip * 64 + (row >> 5) * 16 + (row & 15), N - 1) + (row & 16 ? N : 0);
+        else at = min(strip * 128 + row, N - 1);
+        src[p] = we + at * rb + ((lane & 7) ^ (row >> 1 & 7)) * 16;
+        dst[p] = base + (wid * 4 + p) * 1024;
     }
-    __syncthreads();
-    const uint16_t* xp[XL];
 #pragma unroll
-    for (int i = 0; i < XL; ++i) {
-        const int c = tid + i * 256;
-        xp[i] = x + (size_t)rows_s[c >> 4] * K + (c & 15) * 8;
+    for (int p = 0; p < XPW; ++p) {
+        const int tr = XT < 4 ? wid % XT : p * 4 + wid;
+        const int row = tr * (1024 / XB) + lane / (XB / 16);
+        const int chunk = FP8 ? (lane & 15) ^ (row & 15) : (lane & 7) ^ (row >> 1 & 7);
+        const int s = s0 + min(row, m - 1);
+        src[4 + p] = reinterpret_cast<const char*>(x) +
+                     (int64_t)(MODE == 0 ? s : perm[s] / top) * K * 2 + chunk * 16;
+        dst[4 + p] = base + 128 * 128 + tr * 1024;
     }
-    // weight rows of this wave: two fragments of 16
-    const size_t rb = FP8 ? (size_t)K : (size_t)K * 2;
-    const int n0 = MODE == 1 ? strip * 64 + wid * 16 : strip * 128 + wid * 32;
-    const char* we = w + (size_t)e * (MODE == 1 ? 2 * N : N) * rb;
-    const char* wp[2];
-    wp[0] = we + (size_t)min(n0 + r, N - 1) * rb + q * 16;
-    wp[1] = we + (size_t)(MODE == 1 ? N + min(n0 + r, N - 1) : min(n0 + 16 + r, N - 1)) * rb + q * 16;
-
-    mgf4 acc[2][FM];
+    auto stage = [&](int buf) {
 #pragma unroll
-    for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int j = 0; j < FM; ++j) acc[f][j] = mgf4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    mgu4 xr[XL], wb[2][2][WL];
-    const int ns = K / 128;
-#pragma unroll
-    for (int i = 0; i < XL; ++i) xr[i] = *reinterpret_cast<const mgu4*>(xp[i]);
-#pragma unroll
-    for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int j = 0; j < WL; ++j) wb[0][f][j] = *reinterpret_cast<const mgu4*>(wp[f] + j * 64);
-
-    // `more` is a compile-time constant: the loads of the next step are counted
-    // exactly, so a wait never drains them
-    auto step = [&](int s, mgu4 (&cur)[2][WL], mgu4 (&nxt)[2][WL], char* buf, auto more) {
-#pragma unroll
-        for (int i = 0; i < XL; ++i) {
-            const int c = tid + i * 256, row = c >> 4;
-            *reinterpret_cast<mgu4*>(buf + row * 256 + (((c & 15) ^ (row & 15)) << 4)) = xr[i];
-        }
-        __syncthreads();
-        if (decltype(more)::value) {
-#pragma unroll
-            for (int i = 0; i < XL; ++i)
-                xr[i] = *reinterpret_cast<const mgu4*>(xp[i] + (size_t)(s + 1) * 128);
-#pragma unroll
-            for (int f = 0; f < 2; ++f)
-#pragma unroll
-                for (int j = 0; j < WL; ++j)
-                    nxt[f][j] = *reinterpret_cast<const mgu4*>(wp[f] + (size_t)(s + 1) * (FP8 ? 128 : 256) + j * 64);
-            __builtin_amdgcn_sched_barrier(0);   // the loads are issued before the products
-        }
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            // fp8: one 16-byte load holds the lane's columns of two products
-            const int chunk = FP8 ? (ks >> 1) * 8 + q * 2 + (ks & 1) : ks * 4 + q;
-            mgs8 a[2];
-#pragma unroll
-            for (int f = 0; f < 2; ++f) {
-                if (FP8) {
-                    const mgu4 v = cur[f][ks >> 1];
-                    a[f] = (ks & 1) ? mg_widen(v[2], v[3]) : mg_widen(v[0], v[1]);
-                } else {
-                    a[f] = *reinterpret_cast<const mgs8*>(&cur[f][FP8 ? 0 : ks]);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < FM; ++j) {
-                const mgs8 b = *reinterpret_cast<const mgs8*>(buf + (j * 16 + r) * 256 + ((chunk ^ r) << 4));
-#pragma unroll
-                for (int f = 0; f < 2; ++f)
-                    acc[f][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(mgb8, a[f]), __builtin_bit_cast(mgb8, b), acc[f][j], 0, 0, 0);
-            }
+        for (int p = 0; p < LPS; ++p) {
+            if (p < 4 && mt == 1) lds_transfer16<true>(dst[p] + buf * STEP, src[p]);
+            else lds_transfer16(dst[p] + buf * STEP, src[p]);
+            src[p] += p < 4 ? 128 : XB;
         }
     };
-    const std::true_type yes;
-    const std::false_type no;
-    int s = 0;
-    for (; s + 2 < ns; s += 2) {
-        step(s, wb[0], wb[1], xs[0], yes);
-        step(s + 1, wb[1], wb[0], xs[1], yes);
-    }
-    if (s + 2 == ns) {
-        step(s, wb[0], wb[1], xs[0], yes);
-        step(s + 1, wb[1], wb[0], xs[1], no);
-    } else {
-        step(s, wb[0], wb[1], xs[0], no);
+
+    mgf4 acc[2][FM] = {};
+#pragma unroll
+    for (int t = 0; t < STAGES - 1; ++t)
+        if (t < ns) stage(t);
+    int buf = 0;
+    for (int t = 0; t < ns; ++t) {
+        const int behind = min(STAGES - 2, ns - 1 - t);      // younger steps under way
+        if (STAGES > 3 && behind >= 2) mg_wait<2 * LPS>();
+        else if (STAGES > 2 && behind >= 1) mg_wait<LPS>();
+        else mg_wait<0>();
+        if (t + STAGES - 1 < ns) stage(buf == 0 ? STAGES - 1 : buf - 1);
+        const char* bx = smem + buf * STEP + 128 * 128;
+        const char* bw = smem + buf * STEP + wid * 32 * 128;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int at = r * 128 + (((h * 4 + q) ^ (r >> 1)) << 4);
+            mgu4 v[2];
+#pragma unroll
+            for (int f = 0; f < 2; ++f) v[f] = *reinterpret_cast<const mgu4*>(bw + f * 16 * 128 + at);
+            // fp8: 16 bytes hold the lane's columns of two products
+#pragma unroll
+            for (int k = 0; k < (FP8 ? 2 : 1); ++k) {
+                mgs8 a[2];
+#pragma unroll
+                for (int f = 0; f < 2; ++f)
+                    a[f] = !FP8 ? __builtin_bit_cast(mgs8, v[f])
+                           : k  ? mg_widen(v[f][2], v[f][3])
+                                : mg_widen(v[f][0], v[f][1]);
+#pragma unroll
+                for (int j = 0; j < FM; ++j) {
+                    const mgs8 b = *reinterpret_cast<const mgs8*>(
+                        bx + (FP8 ? (j * 16 + r) * 256 + (((h * 8 + q * 2 + k) ^ r) << 4)
+                                  : j * 16 * 128 + at));
+#pragma unroll
+                    for (int f = 0; f < 2; ++f)
+                        acc[f][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            __builtin_bit_cast(mgb8, a[f]), __builtin_bit_cast(mgb8, b), acc[f][j], 0, 0, 0);
+                }
+            }
+        }
+        buf = buf + 1 == STAGES ? 0 : buf + 1;
     }
 
     // lane: sorted row r of a fragment, weight rows q * 4 .. + 3
+    const int n0 = MODE == 1 ? strip * 64 + wid * 16 : strip * 128 + wid * 32;
     float sc[2][4];
 #pragma unroll
     for (int f = 0; f < 2; ++f)
@@ -480,7 +480,7 @@ extern "C" int oa_moe_route(void* stream, const void* x, const void* rw, void* s
 
 extern "C" int oa_moe_sort(void* stream, const void* expert_ids, int P, int E, int bm, void* off,
                            void* pre, void* tile_e, void* perm) {
-    if (P < 1 || E < 1 || E > MG_MAX_E || (bm != 16 && bm != 64 && bm != 128)) return -100;
+    if (P < 1 || E < 1 || E > MG_MAX_E || (bm != 16 && bm != 32 && bm != 64 && bm != 128)) return -100;
     hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream,
                        (const int*)expert_ids, P, E, bm, (int*)off, (int*)pre, (int*)tile_e, (int*)perm);
     HIP_CHECK_LAUNCH();
@@ -501,29 +501,29 @@ extern "C" int oa_moe_grouped(void* stream, const void* x, const void* w, const 
     const int64_t items = (int64_t)strips * max_tiles;
     if (items > (1 << 28)) return -101;
     const dim3 grid((unsigned)(CEIL_DIV(items, 8) * 8)), block(256);
-#define MG(BMV, F, MO)                                                                              \
-    hipLaunchKernelGGL((moe_grouped_kernel<BMV, F, MO>), grid, block, 0, (hipStream_t)stream,      \
+#define MG(BMV, ST, F, MO)                                                                         \
+    hipLaunchKernelGGL((moe_grouped_kernel<BMV, ST, F, MO>), grid, block,                          \
+                       (ST) * (128 * 128 + (BMV) * ((F) ? 256 : 128)), (hipStream_t)stream,        \
                        (const uint16_t*)x, (const char*)w, (const float*)wscale, (const int*)off,  \
                        (const int*)pre, (const int*)tile_e, (const int*)perm, (const float*)pair_w, \
                        (uint16_t*)out, E, N, K, top, strips, act, limit, alpha)
-#define MGM(BMV, F)                    \
-    do {                               \
-        if (mode == 0) MG(BMV, F, 0);  \
-        else if (mode == 1) MG(BMV, F, 1); \
-        else MG(BMV, F, 2);            \
+#define MGM(BMV, ST, F)                    \
+    do {                                   \
+        if (mode == 0) MG(BMV, ST, F, 0);  \
+        else if (mode == 1) MG(BMV, ST, F, 1); \
+        else MG(BMV, ST, F, 2);            \
     } while (0)
-#define MGF(BMV)                   \
-    do {                           \
-        if (wscale) MGM(BMV, true); \
-        else MGM(BMV, false);      \
-    } while (0)
-    switch (bm) {
-        case 16: MGF(16); break;
-        case 64: MGF(64); break;
-        case 128: MGF(128); break;
+    // steps: as many as two blocks' rings leave room for
+    switch (bm + (wscale ? 1 : 0)) {
+        case 16: MGM(16, 4, false); break;
+        case 17: MGM(16, 4, true); break;
+        case 32: MGM(32, 4, false); break;
+        case 33: MGM(32, 3, true); break;
+        case 64: MGM(64, 3, false); break;
+        case 65: MGM(64, 2, true); break;
+        case 128: MGM(128, 2, false); break;
         default: return -102;
     }
-#undef MGF
 #undef MGM
 #undef MG
     HIP_CHECK_LAUNCH();

@@ -205,3 +205,46 @@ def test_tile_rows():
     assert [rows(p, 64, big, True) for p in (48, 256, 257, 8191, 8192)] == [16, 16, 64, 64, 128]
     assert [rows(p, 16, big, False) for p in (63, 64, 65)] == [64, 16, 64]
     assert [rows(p, 16, small, False) for p in (48, 64, 65)] == [16, 16, 64]
+
+
+def test_ring_rows():
+    """Tiles grow with the rows an expert has, later for small matrices; wide ones of 128
+    rows are for bf16 alone."""
+    rows = ops._moe_ring_rows
+    big, small = 1408 * 2048, 512 * 1024
+    assert [rows(p, 64, big, False) for p in (48, 512, 513, 1536, 1537, 4095, 4096)] == [
+        16, 16, 32, 32, 64, 64, 128]
+    assert [rows(p, 64, big, True) for p in (512, 513, 1536, 1537, 99999)] == [16, 32, 32, 64, 64]
+    assert [rows(p, 16, small, False) for p in (256, 257, 1536, 1537, 9999)] == [16, 32, 32, 64, 64]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8,tiles", [(False, (16, 32, 64, 128)), (True, (16, 32, 64))])
+@pytest.mark.parametrize("T,E,top,H,I", [
+    (5, 7, 2, 128, 128),          # fewer steps than the ring holds, experts without rows
+    (33, 9, 3, 256, 192 + 64),    # one row past a tile of 32
+    (131, 5, 2, 384, 128),        # odd steps; several tiles of most sizes an expert
+])
+def test_tiles_agree(monkeypatch, fp8, tiles, T, E, top, H, I):
+    """A pair's sums run over the columns in one order whatever the tile: the same bits."""
+    gen = torch.Generator(device="cuda").manual_seed(T + E)
+    rn = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    x = rn(T, H).bfloat16()
+    w13, w2 = (rn(E, 2 * I, H) * H ** -0.5).bfloat16(), (rn(E, H, I) * I ** -0.5).bfloat16()
+    s13 = s2 = None
+    d13, d2 = w13, w2
+    if fp8:
+        (w13, s13), (w2, s2) = ops.quant_fp8(w13), ops.quant_fp8(w2)
+        s13, s2 = s13.view(E, -1), s2.view(E, -1)
+        d13, d2 = torch_ref.dequant_fp8(w13, s13), torch_ref.dequant_fp8(w2, s2)
+    wts, idx = torch.softmax(rn(T, E), -1).topk(top, -1)
+    idx = idx.to(torch.int32)
+    outs = []
+    for rows in tiles:
+        monkeypatch.setattr(ops, "_moe_ring_rows", lambda *a, rows=rows: rows)
+        outs.append(ops.moe_sorted_mlp(x, w13, s13, w2, s2, idx, wts))
+    for o in outs[1:]:
+        assert torch.equal(o, outs[0])
+    want = _reference(x, d13, d2, idx, wts, None, None)
+    # the roundings of test_sorted_experts
+    assert float((outs[0].double() - want).norm() / want.norm()) < 4e-3
