@@ -16,6 +16,8 @@
 //
 // All sizes are run-time values; nothing assumes a multiple of 64.
 
+#include <type_traits>
+
 #include "mixer_util.h"
 
 // ---------------------------------------------------------------------------
@@ -1309,6 +1311,254 @@ __global__ __launch_bounds__(VEC ? 512 : 1024, VEC && RPL <= 8 && sizeof(TC) == 
     }
 }
 
+// ---------------------------------------------------------------------------
+// The gated delta rule over long portions, in two launches: what does not depend on
+// the state is prepared for all tokens at once, then the recurrence runs over the
+// prepared rows (the head norm follows as its own launch). Same lanes, state and
+// arithmetic as delta_fused_kernel, which stays for decode steps and the other sizes.
+//
+// What bounded that kernel on a prompt was the staging inside the chain (softplus,
+// exponential and unit vectors, once per block of a head's columns) and a read-out that
+// waited for the update: 1460 cycles a token. Here the chain of a token is one
+// decay, two dot products side by side and one update: with S' = decay * S,
+//   o = S^T q = S'^T q + u (k . q),   u = beta (v - S'^T k),
+// so the read-out needs only k . q, which is prepared.
+// One layer of 32 heads of 128 x 128, tokens 1024 + 333 + 77: 592 us before, 218 now
+// (prepare 32 at 2.2 TB/s written, recurrence 166 to 190, head norm 20); 410 cycles a token
+// of the longest portion, 52 vector instructions of 4 and the waits between them.
+//
+// kq [T + 16, G, 2, DP]: unit k, unit q times D^-1/2, rows past D zero; dec [T + 16, H, DP]
+// decay (HEAD: none); sc [T, H, 2]: beta, the decay of HEAD; dot [T, G]: k . q.
+template <int RPL, bool HEAD, typename TC>
+__global__ __launch_bounds__(256) void delta_prepare_kernel(
+    const TC* __restrict__ q, int64_t qs, const TC* __restrict__ k, int64_t ks,
+    const TC* __restrict__ bl, int64_t bs, const TC* __restrict__ a, int64_t as,
+    const TC* __restrict__ dt_bias, const TC* __restrict__ a_log, float* __restrict__ kq,
+    float* __restrict__ dec, float* __restrict__ sc, float* __restrict__ dot, int T, int H,
+    int G, int D) {
+    constexpr int DP = RPL * 16, KP = DP / 8;        // KP lanes of 8 elements a row
+    const int64_t i = (int64_t)blockIdx.x * (256 / KP) + threadIdx.x / KP;
+    if (i >= (int64_t)T * H) return;                 // whole groups of KP lanes
+    const int64_t t = i / H;
+    const int h = (int)(i % H), r0 = (threadIdx.x % KP) * 8;
+    const bool live = r0 < D;
+    const float A = expf(ldf(a_log, h));
+    float x[8] = {}, y[8] = {};
+    if (!HEAD) {
+        if (live) {
+            float z[8];
+            ld8(a, t * as + h * D + r0, z);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = expf(-A * softplusf_(z[e] + ldf(dt_bias, h * D + r0 + e)));
+        }
+        st8(dec, i * DP + r0, x);
+    }
+    if (r0 == 0) {
+        sc[i * 2] = sigmoidf_(ldf(bl, t * bs + h));
+        sc[i * 2 + 1] = HEAD ? expf(-A * softplusf_(ldf(a, t * as + h) + ldf(dt_bias, h))) : 0.0f;
+    }
+    if (h >= G) return;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = 0.0f;
+    if (live) {
+        ld8(k, t * ks + h * D + r0, x);
+        ld8(q, t * qs + h * D + r0, y);
+    }
+    float xx = 0.0f, yy = 0.0f, xy = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        xx += x[e] * x[e];
+        yy += y[e] * y[e];
+    }
+#pragma unroll
+    for (int off = KP / 2; off > 0; off >>= 1) {
+        xx += __shfl_xor(xx, off, WAVE);
+        yy += __shfl_xor(yy, off, WAVE);
+    }
+    const float rk = 1.0f / sqrtf(xx + 1e-6f), rq = 1.0f / sqrtf((float)D) / sqrtf(yy + 1e-6f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        x[e] *= rk;
+        y[e] *= rq;
+        xy += x[e] * y[e];
+    }
+#pragma unroll
+    for (int off = KP / 2; off > 0; off >>= 1) xy += __shfl_xor(xy, off, WAVE);
+    float* row = kq + (t * G + h) * 2 * DP;
+    st8(row, r0, x);
+    st8(row, DP + r0, y);
+    if (r0 == 0) dot[t * G + h] = xy;
+}
+
+// value of lane N of the own 16 lanes
+template <int N>
+__device__ __forceinline__ float row16_get(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + N, 0xf, 0xf, true));
+}
+
+template <int I, int N, typename F>
+__device__ __forceinline__ void for_each_token(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>());
+        for_each_token<I + 1, N>(f);
+    }
+}
+
+// Four waves of four columns each, P passes; a column's D rows over the 16 lanes of a DPP
+// row. Tokens come in chunks of 16: their k, q and decay rows by transfers into one of two
+// LDS buffers while the other chunk is worked on, their v, beta and k . q with lane = token.
+// Grid x: (column group, head) with the head fastest, so that the groups of a head,
+// which read the same rows, share a die's L2 where the heads are a multiple of eight.
+template <int RPL, int P, bool HEAD, typename TC>
+__global__ __launch_bounds__(256) void delta_scan_kernel(
+    const float* __restrict__ kq, const float* __restrict__ dec, const float* __restrict__ sc,
+    const float* __restrict__ dots, const TC* __restrict__ v, int64_t vs,
+    float* __restrict__ state, float* __restrict__ o_raw, const int* __restrict__ cu,
+    const int* __restrict__ past, const int* __restrict__ slots, int H, int G, int D, int Dv) {
+    constexpr int DP = RPL * 16, TCK = 16;
+    constexpr int KQ = TCK * 2 * DP * 4, BUF = KQ + (HEAD ? 0 : TCK * DP * 4);   // bytes
+    constexpr int NT = BUF / 4096, NK = KQ / 4096;   // transfers of a wave and chunk, of k and q
+    __shared__ __attribute__((aligned(16))) char lds[2 * BUF];
+    const int h = blockIdx.x % H, b = blockIdx.y;
+    const int lo = cu[b], n = cu[b + 1] - lo;
+    if (n <= 0) return;
+    const int lane = threadIdx.x & 63, rg = lane & 15, cs = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kvh = h / (H / G);
+    float* st = state + ((int64_t)slots[b] * H + h) * Dv * D;
+    const bool fresh = past[b] == 0;
+
+    // this lane's piece of every transfer: the k and q rows of a chunk first. Tokens past the
+    // portion's end are the next one's, or the 16 that the buffers have past the last: read,
+    // and not worked on
+    const char* src[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int u = (j * 4 + wave) * 64 + lane - (j < NK ? 0 : KQ / 16);
+        constexpr int KP = DP / 2, GP = DP / 4;      // 16-byte pieces of a token
+        src[j] = j < NK ? reinterpret_cast<const char*>(kq + ((int64_t)(lo + u / KP) * G + kvh) * 2 * DP) + u % KP * 16
+                        : reinterpret_cast<const char*>(dec + ((int64_t)(lo + u / GP) * H + h) * DP) + u % GP * 16;
+    }
+    const int64_t kstep = (int64_t)TCK * G * 2 * DP * 4, gstep = (int64_t)TCK * H * DP * 4;
+    const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            lds_transfer16(base + buf * BUF + (j * 4 + wave) * 1024, src[j]);
+            src[j] += j < NK ? kstep : gstep;
+        }
+    };
+
+    int col[P];
+    float S[P][RPL];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        col[p] = (blockIdx.x / H * 4 + wave) * (4 * P) + p * 4 + cs;
+#pragma unroll
+        for (int i4 = 0; i4 < RPL / 4; ++i4) {
+            const int r = 64 * i4 + 4 * rg;
+            float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (!fresh && col[p] < Dv && r < D)
+                x = *reinterpret_cast<const float4*>(st + (int64_t)col[p] * D + r);
+            S[p][4 * i4] = x.x; S[p][4 * i4 + 1] = x.y; S[p][4 * i4 + 2] = x.z; S[p][4 * i4 + 3] = x.w;
+        }
+    }
+    float vn[P], bn = 0.0f, gn = 0.0f, dn = 0.0f;    // of token c0 + rg
+    auto fetch = [&](int c0) {
+        const int64_t t = lo + min(c0 + rg, n - 1);
+#pragma unroll
+        for (int p = 0; p < P; ++p) vn[p] = ldf(v, t * vs + h * Dv + min(col[p], Dv - 1));
+        const float2 s2 = *reinterpret_cast<const float2*>(sc + (t * H + h) * 2);
+        bn = s2.x;
+        gn = s2.y;
+        dn = dots[t * G + kvh];
+    };
+    stage(0);
+    fetch(0);
+    int buf = 0;
+    for (int c0 = 0; c0 < n; c0 += TCK, buf ^= 1) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
+        float v1[P], o1[P];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            v1[p] = vn[p];
+            o1[p] = 0.0f;
+        }
+        const float b1 = bn, g1 = gn, d1 = dn;
+        if (c0 + TCK < n) {
+            stage(buf ^ 1);
+            fetch(c0 + TCK);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const int nc = min(TCK, n - c0);
+        const float* rows = reinterpret_cast<const float*>(lds + buf * BUF) + 4 * rg;
+        const float* grows = rows + TCK * 2 * DP;
+        // one token: its rows are in set TT & 1, the next token's are asked for first
+        float4 kr[2][RPL / 4], qr[2][RPL / 4], gr[2][RPL / 4];
+        auto read = [&](int tt, int set) {
+#pragma unroll
+            for (int i4 = 0; i4 < RPL / 4; ++i4) {
+                kr[set][i4] = *reinterpret_cast<const float4*>(rows + tt * 2 * DP + 64 * i4);
+                if (!HEAD) gr[set][i4] = *reinterpret_cast<const float4*>(grows + tt * DP + 64 * i4);
+                qr[set][i4] = *reinterpret_cast<const float4*>(rows + tt * 2 * DP + DP + 64 * i4);
+            }
+        };
+        auto token = [&](auto index) {
+            constexpr int TT = decltype(index)::value, A = TT & 1;
+            if (TT + 1 < TCK) read(TT + 1, A ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+            const float bt = row16_get<TT>(b1), kdq = row16_get<TT>(d1);
+            const float gh = HEAD ? row16_get<TT>(g1) : 0.0f;
+            float dk[P][2], dq[P][2];
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+#pragma unroll
+                for (int i = 0; i < RPL; ++i) {
+                    const float kv = (&kr[A][i / 4].x)[i % 4], qv = (&qr[A][i / 4].x)[i % 4];
+                    S[p][i] *= HEAD ? gh : (&gr[A][i / 4].x)[i % 4];
+                    dk[p][i & 1] = i < 2 ? S[p][i] * kv : fmaf(S[p][i], kv, dk[p][i & 1]);
+                    dq[p][i & 1] = i < 2 ? S[p][i] * qv : fmaf(S[p][i], qv, dq[p][i & 1]);
+                }
+            float u[P], o[P];
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                u[p] = bt * (row16_get<TT>(v1[p]) - row16_sum(dk[p][0] + dk[p][1]));
+                o[p] = fmaf(u[p], kdq, row16_sum(dq[p][0] + dq[p][1]));
+                o1[p] = rg == TT ? o[p] : o1[p];
+            }
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+#pragma unroll
+                for (int i = 0; i < RPL; ++i) S[p][i] = fmaf((&kr[A][i / 4].x)[i % 4], u[p], S[p][i]);
+        };
+        read(0, 0);
+        if (nc == TCK) {
+            for_each_token<0, TCK>(token);
+        } else {                                     // the last tokens of the portion
+            auto some = [&](auto index) {
+                if (decltype(index)::value < nc) token(index);
+            };
+            for_each_token<0, TCK>(some);
+        }
+        if (rg < nc) {
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+                if (col[p] < Dv) o_raw[((int64_t)(lo + c0 + rg) * H + h) * Dv + col[p]] = o1[p];
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        if (col[p] >= Dv) continue;
+#pragma unroll
+        for (int i4 = 0; i4 < RPL / 4; ++i4) {
+            const int r = 64 * i4 + 4 * rg;
+            if (r < D)
+                *reinterpret_cast<float4*>(st + (int64_t)col[p] * D + r) =
+                    make_float4(S[p][4 * i4], S[p][4 * i4 + 1], S[p][4 * i4 + 2], S[p][4 * i4 + 3]);
+        }
+    }
+}
+
 // per-head RMS norm of a float32 read-out, times w[Dv], times sigmoid|silu(gate):
 // one block per token, one wave per head (used when the delta rule's columns
 // were split over blocks)
@@ -1775,6 +2025,72 @@ extern "C" int oa_delta_rule_fused(void* stream, const void* q, int64_t qs, cons
         hipLaunchKernelGGL((gated_head_norm_kernel<bf16s>), dim3(T), dim3(256), 0, s, (const float*)o_raw,
                            (const bf16s*)norm_w, (const bf16s*)gate, gs, (bf16s*)out, H, Dv, eps, gate_silu, os);
     HIP_CHECK_LAUNCH();
+    return 0;
+}
+
+// The same over long portions (delta_prepare_kernel, delta_scan_kernel and the head norm):
+// D a multiple of 8 up to 128; q, k and a with one decay per channel are rows of whole
+// 16-byte pieces (32 in float32). prep: float32 workspace of (T + 16) * (2 * G * DP +
+// (head_decay ? 0 : H * DP)) + T * (G + 2 * H) values, DP = D rounded up to 64 or 128.
+// passes: 1 or 2 groups of four columns a wave.
+extern "C" int oa_delta_rule_long(void* stream, const void* q, int64_t qs, const void* k,
+                                  int64_t ks, const void* v, int64_t vs, const void* bl,
+                                  int64_t bs, const void* a, int64_t as, const void* dt_bias,
+                                  const void* a_log, const void* norm_w, const void* gate,
+                                  int64_t gs, void* state, void* out, void* o_raw, void* prep,
+                                  const void* cu, const void* past, const void* slots, int T,
+                                  int B, int H, int G, int D, int Dv, float eps, int dt,
+                                  int passes, int head_decay, int gate_silu, int64_t os) {
+    if (T <= 0 || B <= 0) return 0;
+    if (G < 1 || H % G != 0) return -100;
+    if (D < 8 || D > 128 || D % 8 != 0 || Dv < 1) return -105;
+    if (!o_raw || !prep || (uintptr_t)prep % 16 != 0 || (passes != 1 && passes != 2)) return -107;
+    if (os < (int64_t)H * Dv) return -108;
+    const int al = dt == 1 ? 32 : 16, DP = D <= 64 ? 64 : 128;
+    auto rows_ok = [&](const void* p, int64_t st) { return (uintptr_t)p % al == 0 && st % 8 == 0; };
+    if (!rows_ok(q, qs) || !rows_ok(k, ks) || (!head_decay && !rows_ok(a, as))) return -109;
+    hipStream_t s = (hipStream_t)stream;
+    float* kq = (float*)prep;
+    float* dec = kq + (int64_t)(T + 16) * 2 * G * DP;
+    float* sc = dec + (head_decay ? 0 : (int64_t)(T + 16) * H * DP);
+    float* dots = sc + (int64_t)T * H * 2;
+    const dim3 pgrid((unsigned)CEIL_DIV((int64_t)T * H * (DP / 8), 256)), blk(256);
+    const dim3 grid(H * CEIL_DIV(Dv, 16 * passes), B);
+#define DLONG(R, PP, HD, TC)                                                                       \
+    do {                                                                                           \
+        hipLaunchKernelGGL((delta_prepare_kernel<R, HD, TC>), pgrid, blk, 0, s, (const TC*)q, qs,   \
+                           (const TC*)k, ks, (const TC*)bl, bs, (const TC*)a, as,                   \
+                           (const TC*)dt_bias, (const TC*)a_log, kq, dec, sc, dots, T, H, G, D);    \
+        HIP_CHECK_LAUNCH();                                                                        \
+        hipLaunchKernelGGL((delta_scan_kernel<R, PP, HD, TC>), grid, blk, 0, s, kq, dec, sc, dots,  \
+                           (const TC*)v, vs, (float*)state, (float*)o_raw, (const int*)cu,          \
+                           (const int*)past, (const int*)slots, H, G, D, Dv);                       \
+        HIP_CHECK_LAUNCH();                                                                        \
+        hipLaunchKernelGGL((gated_head_norm_kernel<TC>), dim3(T), blk, 0, s, (const float*)o_raw,   \
+                           (const TC*)norm_w, (const TC*)gate, gs, (TC*)out, H, Dv, eps, gate_silu, \
+                           os);                                                                    \
+        HIP_CHECK_LAUNCH();                                                                        \
+    } while (0)
+#define DLONG_T(R, PP, HD)                   \
+    do {                                     \
+        if (dt == 1) DLONG(R, PP, HD, float); \
+        else DLONG(R, PP, HD, bf16s);        \
+    } while (0)
+#define DLONG_H(R, PP)                        \
+    do {                                      \
+        if (head_decay) DLONG_T(R, PP, true); \
+        else DLONG_T(R, PP, false);           \
+    } while (0)
+    if (DP == 64) {
+        if (passes == 1) DLONG_H(4, 1);
+        else DLONG_H(4, 2);
+    } else {
+        if (passes == 1) DLONG_H(8, 1);
+        else DLONG_H(8, 2);
+    }
+#undef DLONG_H
+#undef DLONG_T
+#undef DLONG
     return 0;
 }
 

@@ -171,6 +171,8 @@ def _declare_mixers(lib: ctypes.CDLL) -> None:
         "oa_moe_pairs_down": [p, p, p, p, p, p, i, i, i, i, i, i],
         "oa_delta_rule_fused": [p, p, i64, p, i64, p, i64, p, i64, p, i64, p, p, p, p, i64,
                                 p, p, p, p, p, p, i, i, i, i, i, i, f, i, i, i, i, i64],
+        "oa_delta_rule_long": [p, p, i64, p, i64, p, i64, p, i64, p, i64, p, p, p, p, i64,
+                               p, p, p, p, p, p, p, i, i, i, i, i, i, f, i, i, i, i, i64],
         "oa_softcap": [p, p, p, i64, f, i],
         "oa_silu_mul_rows": [p, p, p, i64, i, i],
         "oa_embed_rows": [p, p, p, p, i, i, i, f, p, p, p, p],

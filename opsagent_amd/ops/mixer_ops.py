@@ -603,6 +603,24 @@ def moe_pairs_mlp(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, idx: tor
     return out
 
 
+def _delta_long(sb: SeqBatch, D: int, rows) -> bool:
+    """Whether the delta rule prepares its rows in a launch of its own (delta_scan_kernel);
+    rows: the tensors it reads in whole 8-element pieces. Us of a layer in one launch / so,
+    32 heads of 128 x 128: one portion of 16 tokens 21 / 25, of 32 36 / 27, of 64 44 / 33, of
+    2000 896 / 374; four of 30 36 / 39, 16 of 32 77 / 75, 32 of 64 364 / 227."""
+    return sb.max_chunk >= 40 and D <= 128 and D % 8 == 0 and all(
+        _rows(t) % 8 == 0 and t.data_ptr() % (8 * t.element_size()) == 0 for t in rows)
+
+
+def _delta_passes(sb: SeqBatch, H: int, Dv: int) -> int:
+    """Column groups of a wave of delta_scan_kernel: one where a CU works on little beside the
+    longest portion, whose chain of tokens sets the time, two, which read the rows of a token
+    half as often, where the CUs are full. Us of a layer with 1 / 2, 32 heads of 128 x 128:
+    one portion of 2000 tokens 374 / 543, three of 700 275 / 329, four of 500 250 / 245, eight
+    of 1024 960 / 921."""
+    return 2 if sb.num_tokens * H * Dv >= 4 * 16 * 256 * sb.max_chunk else 1
+
+
 def channel_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                        b_logits: torch.Tensor, a: torch.Tensor, dt_bias: torch.Tensor,
                        a_log: torch.Tensor, norm_w: torch.Tensor, gate_logits: torch.Tensor,
@@ -634,8 +652,24 @@ def channel_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     assert head_decay or (a.shape[1] == H * D and dt_bias.numel() == H * D)
     assert state.dtype == torch.float32 and state.is_contiguous()
     assert state.shape[1:] == (H, Dv, D)
+    args = (hip.current_stream_ptr(), q.data_ptr(), _rows(q), k.data_ptr(), _rows(k),
+            v.data_ptr(), _rows(v), b_logits.data_ptr(), _rows(b_logits), a.data_ptr(), _rows(a),
+            dt_bias.data_ptr(), a_log.data_ptr(), norm_w.data_ptr(), gate_logits.data_ptr(),
+            _rows(gate_logits), state.data_ptr(), out.data_ptr())
+    sizes = (sb.cu_t.data_ptr(), sb.past_t.data_ptr(), sb.slots_t.data_ptr(), T, sb.num_seqs,
+             H, G, D, Dv, eps, _dt(q))
+    ends = int(head_decay), int(gate_act == "silu"), _rows(out)
+    DP = 64 if D <= 64 else 128
+    words = (T + 16) * (2 * G * DP + (0 if head_decay else H * DP)) + T * (G + 2 * H)
+    # the prepared rows (50 KB a token of 32 heads of 128) stay under 1 GB
+    if words <= 2 ** 28 and _delta_long(sb, D, (q, k) if head_decay else (q, k, a)):
+        o_raw = torch.empty(T, H * Dv, dtype=torch.float32, device=q.device)
+        prep = torch.empty(words, dtype=torch.float32, device=q.device)
+        hip.check(lib.oa_delta_rule_long(*args, o_raw.data_ptr(), prep.data_ptr(), *sizes,
+                                         _delta_passes(sb, H, Dv), *ends), "oa_delta_rule_long")
+        return out
     # one block per (sequence, head) runs the recurrence of ALL value columns
-    # on one CU; long portions of few sequences split the columns over blocks
+    # on one CU; long portions (of rows that _delta_long does not take) of few sequences split the columns over blocks
     # instead (the head norm then runs as its own launch on a float32 buffer)
     csplit, o_raw = _value_split(sb, H, D, Dv), None
     if D > 128 and Dv // csplit > 64:
@@ -647,14 +681,8 @@ def channel_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                 break
     if csplit > 1:
         o_raw = torch.empty(T, H * Dv, dtype=torch.float32, device=q.device)
-    rc = lib.oa_delta_rule_fused(
-        hip.current_stream_ptr(), q.data_ptr(), _rows(q), k.data_ptr(), _rows(k),
-        v.data_ptr(), _rows(v), b_logits.data_ptr(), _rows(b_logits), a.data_ptr(), _rows(a),
-        dt_bias.data_ptr(), a_log.data_ptr(), norm_w.data_ptr(), gate_logits.data_ptr(),
-        _rows(gate_logits), state.data_ptr(), out.data_ptr(),
-        o_raw.data_ptr() if o_raw is not None else None, sb.cu_t.data_ptr(),
-        sb.past_t.data_ptr(), sb.slots_t.data_ptr(), T, sb.num_seqs, H, G, D, Dv, eps, _dt(q),
-        csplit, int(head_decay), int(gate_act == "silu"), _rows(out))
+    rc = lib.oa_delta_rule_fused(*args, o_raw.data_ptr() if o_raw is not None else None, *sizes,
+                                 csplit, *ends)
     hip.check(rc, "oa_delta_rule_fused")
     return out
 
