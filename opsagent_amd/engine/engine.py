@@ -1234,15 +1234,15 @@ class LLMEngine:
         return logits[:B]
 
     # -- sampling --------------------------------------------------------
-    def _logprob_entry(self, row: torch.Tensor, tok: int, top_n: int) -> dict:
-        """Raw-model log-softmax of the sampled token (+ top alternatives)."""
-        lp = torch.log_softmax(row.float(), dim=-1)
-        entry = {"token_id": tok, "logprob": float(lp[tok])}
+    @staticmethod
+    def _logprob_entry(logprobs, i: int, tok: int, top_n: int) -> dict:
+        """Raw-model log-softmax of the sampled token of row i (+ top alternatives)."""
+        at, idx, val = logprobs
+        entry = {"token_id": tok, "logprob": float(at[i])}
         if top_n > 0:
-            vals, idx = torch.topk(lp, min(top_n, lp.shape[0]))
             entry["top"] = [
-                {"token_id": int(i), "logprob": float(v)}
-                for v, i in zip(vals.tolist(), idx.tolist())
+                {"token_id": t, "logprob": v}
+                for t, v in zip(idx[i, :top_n].tolist(), val[i, :top_n].tolist())
             ]
         return entry
 
@@ -1401,7 +1401,7 @@ class LLMEngine:
                 )
             elif lg.dtype != torch.bfloat16:
                 lg = lg.to(torch.bfloat16)
-            tokens = ops.greedy_sample_masked(lg, mask_t).cpu()
+            tokens = ops.greedy_sample_masked(lg, mask_t)
         else:
             mask_bool = None
             if mask_t is not None:
@@ -1415,7 +1415,13 @@ class LLMEngine:
             lf = logits.float()
             if needs:
                 lf = self._transform_logits(batch, lf.clone())
-            tokens = ops.greedy_sample_masked(lf, mask_bool).cpu()
+            tokens = ops.greedy_sample_masked(lf, mask_bool)
+        # all rows at once, and before the host waits for the tokens
+        logprobs = None
+        if any(r.params.logprobs for r in batch):
+            logprobs = ops.token_logprobs(
+                logits, tokens, max(r.params.top_logprobs for r in batch if r.params.logprobs))
+        tokens = tokens.cpu()
 
         for i, req in enumerate(batch):
             tok = int(tokens[i])
@@ -1432,9 +1438,7 @@ class LLMEngine:
                     req.seq.token_ids.append(tok)
                     if req.params.logprobs:
                         req.logprob_content.append(
-                            self._logprob_entry(
-                                logits[i], tok, req.params.top_logprobs
-                            )
+                            self._logprob_entry(logprobs, i, tok, req.params.top_logprobs)
                         )
                     req.finished = True
                     req.finish_reason = "grammar_complete"
@@ -1450,7 +1454,7 @@ class LLMEngine:
             self._tokens_done += 1
             if req.params.logprobs:
                 req.logprob_content.append(
-                    self._logprob_entry(logits[i], tok, req.params.top_logprobs)
+                    self._logprob_entry(logprobs, i, tok, req.params.top_logprobs)
                 )
             emitted = [tok]
             if self._match_stop(req, 1):

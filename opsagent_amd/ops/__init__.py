@@ -1326,3 +1326,29 @@ def greedy_sample_masked(
     )
     hip.check(rc, "oa_masked_argmax")
     return out
+
+
+def token_logprobs(logits: torch.Tensor, tokens: torch.Tensor, top: int):
+    """Log-softmax of logits [B, V] at tokens [B], and of the `top` most likely tokens of
+    each row: (logprobs [B], indices [B, top] int32, their logprobs [B, top]) on the host,
+    float32. Equal values go by index; NaN where a token is none (negative)."""
+    B, V = logits.shape
+    top = max(0, min(top, V))
+    if not (_is_gpu(logits) and logits.dtype in (torch.bfloat16, torch.float32)
+            and logits.stride(1) == 1 and 0 < B <= 65535 and top <= 32):
+        lp = torch.log_softmax(logits.float(), dim=-1)
+        t = tokens.long().to(lp.device)
+        at = torch.where((t >= 0) & (t < V), lp.gather(1, t.clamp(0, V - 1)[:, None])[:, 0], torch.nan)
+        val, idx = torch.topk(lp, top)
+        return at.cpu(), idx.to(torch.int32).cpu(), val.cpu()
+    lib, hip = _lib()
+    assert tokens.dtype == torch.int32 and tokens.is_contiguous() and tokens.shape == (B,)
+    ws = torch.empty(B * -(-V // 1024) * (top + 1), dtype=torch.int64, device=logits.device)
+    out = torch.empty(B, 1 + 2 * top, dtype=torch.int32, device=logits.device)
+    hip.check(lib.oa_token_logprobs(
+        hip.current_stream_ptr(), logits.data_ptr(), logits.stride(0), tokens.data_ptr(),
+        ws.data_ptr(), out.data_ptr(), B, V, top, int(logits.dtype == torch.float32)),
+        "oa_token_logprobs")
+    host = out.cpu()
+    values = host.view(torch.float32)
+    return values[:, 0], host[:, 1::2], values[:, 2::2]

@@ -1,0 +1,62 @@
+"""Log-probabilities of chosen and most likely tokens against a 64-bit log-softmax: rows that
+end anywhere in a wave's 1024, ties, rows with gaps between them, infinities and NaN."""
+
+import pytest
+import torch
+
+from opsagent_amd import ops
+
+DEVICES = ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)]
+
+
+def _check(logits, tokens, top, device):
+    V = logits.shape[1]
+    at, idx, val = ops.token_logprobs(logits.to(device), tokens.to(device), top)
+    lp = torch.log_softmax(logits.double(), -1)
+    top = min(top, V)
+    assert idx.shape == val.shape == (len(tokens), top)
+    # three roundings of values of this size, and the sum of V exponentials in 32 bits: by
+    # lanes and waves on the GPU, at worst one after the other on the CPU
+    bound = 2.0 ** -23 * (4 + float(logits.float().abs().max())) * 2
+    bound += V * 2.0 ** -24 * (device == "cpu")
+    assert torch.all((at.double() - lp.gather(1, tokens.long()[:, None])[:, 0]).abs() <= bound)
+    assert torch.all((val.double() - lp.topk(top).values).abs() <= bound)
+    got = logits.gather(1, idx.long()).float()
+    assert torch.equal(got, logits.float().topk(top).values)
+    if device == "cuda":                                     # equal values by index
+        order = torch.sort(logits.float(), descending=True, stable=True).indices[:, :top]
+        assert torch.equal(idx.long(), order)
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,V,top", [(1, 1, 5), (3, 7, 7), (2, 1023, 32), (2, 1024, 0), (3, 1025, 1),
+                                     (2, 4097, 20), (1, 128256, 5)])
+def test_rows(device, dtype, B, V, top):
+    g = torch.Generator().manual_seed(V + top)
+    wide = (4 * torch.randn(B, V + 3, generator=g)).to(dtype)
+    tokens = torch.randint(0, V, (B,), generator=g, dtype=torch.int32)
+    _check(wide[:, :V], tokens, top, device)                 # rows with gaps
+    _check(wide[:, :V].contiguous(), tokens, top, device)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_special_values(dtype):
+    V, inf, nan = 3000, float("inf"), float("nan")
+    g = torch.Generator().manual_seed(1)
+    rows = torch.randn(6, V, generator=g)
+    rows[1, 100:2900] = -inf                                 # parts without a finite logit
+    rows[2] = -inf
+    rows[3, 2000] = nan
+    rows[4, 2000] = inf
+    tokens = torch.tensor([-1, 50, 5, 7, 2000, V], dtype=torch.int32)
+    at, idx, val = ops.token_logprobs(rows.to(dtype).cuda(), tokens.cuda(), 4)
+    want = torch.log_softmax(rows.to(dtype).float(), -1)
+    assert torch.isnan(at[[0, 5]]).all()                     # no token, one past the row
+    assert torch.allclose(at[1], want[1, 50], atol=2e-6)
+    assert torch.allclose(val[[0, 1, 5]], want.topk(4).values[[0, 1, 5]], atol=2e-6)
+    assert torch.isnan(at[2:5]).all() and torch.isnan(val[2:5]).all()
+    assert torch.isnan(want[2:4]).all() and torch.isnan(want[4, 2000])
+    assert idx[3, 0] == 2000 and idx[4, 0] == 2000           # NaN, then infinity first
+    assert idx[2].tolist() == [0, 1, 2, 3]
