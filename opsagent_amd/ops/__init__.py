@@ -263,10 +263,70 @@ def _ring_plan(M: int, N: int, K: int, gateup: bool = False) -> Optional[Tuple[i
     return None
 
 
-def _ring(x: torch.Tensor, w: torch.Tensor, plan: Tuple[int, int], act: int = 0) -> torch.Tensor:
-    """x @ w^T, or act 1 (silu), 2 (tanh gelu) of the gate rows times the up rows."""
+def _ring_narrow(M: int, N: int, K: int, gateup: bool, wide) -> Optional[int]:
+    """Column splits of the ring product in strips of 64 weight rows, two blocks a CU
+    (ring_gemm.hip), None where strips of 128 (wide: their plan) or the other forms stay.
+
+    Measured over 40 weights at 3 to 64 rows, 1.5 GB of them in turn, us other / narrow. It
+    wants the CUs full: one round of half the blocks (12288 x 4096, M = 8 23.9 / 21.4 with
+    192), or rounds of 512 (gate-up 2 x 14336 x 4096, 8 45.0 / 40.3 with 448; 2 x 11008, 8 36.4
+    / 37.9 with 344). Weights under 10 MB end before it starts (2048 x 2048, 24 6.9 / 7.2), rows
+    under 2048 columns leave splits too short (4096 x 1408, 24 6.1 / 7.5), and wide weights of
+    many splits run as fast in one deep ring (8192 x 28672, 32 74.4 / 80.5; 10240 x 8192, 8 31.1
+    / 32.5). Gate-up pays twice for splits, and rows of 4 KiB start on the same channels (2 x
+    8192 x 2048, 24 15.3 / 15.7; 2 x 8192 x 3072 20.8 / 18.8); past 48 rows a strip of 128 reads
+    x half as often (2 x 14336 x 4096, 64 48.0 / 49.8; inside a model of 4096 x 14336 and 32000 x
+    4096 too both forms take the same). Up to 16 rows strips of skinny.hip are
+    the faster form for short rows (4096 x 4096, 8 9.1 / 9.8, 24 11.9 / 10.6; 32000 x 2048, 6
+    27.8 / 29.0) and the wide ring where it has splits of its own (16384 x 4096, 8 26.3 /
+    26.8)."""
+    if not 2 < M <= (64 if wide is None else 48) or K % 64 or N % 8:
+        return None
+    weights = (2 if gateup else 1) * N * K
+    strips = -(-N // (32 if gateup else 64))
+    splits = max(1, min(256 // strips, K // 256))
+    blocks = strips * splits
+    if blocks > 256:
+        full = 0.84 * 512 * -(-blocks // 512)
+    else:
+        full = (0.68 if splits == 1 or gateup else 0.85) * 256
+    if blocks < full or weights < 5e6 or K >= 8192 and N >= 8192:
+        return None
+    if gateup:
+        if splits == 1 and K >= 3072 and weights >= 45e6:
+            ok = M <= 48
+        elif M <= 16:
+            ok = wide is None and K >= 4096 and weights < 24e6
+        else:
+            ok = wide is None or weights < 24e6
+    elif splits == 1:
+        if M <= 16:
+            ok = wide is None and weights >= 45e6 and (K >= 3072 or M >= 8)
+        else:
+            ok = K >= 2048 and M <= 32 or K >= 4096 and strips <= 512 and blocks >= 0.9 * 256
+    elif M <= 16:
+        ok = K % (splits * 2048) != 0 and (K >= 5120 or K >= 3072 and weights >= 24e6)
+    else:
+        # a square weight that the library is best at (2560 x 2560, 40 9.4 / 9.5, 64 13.8 / 10.6)
+        ok = K >= 2048 and not (wide is None and K >= N and 32 < M <= 48)
+    return splits if ok else None
+
+
+def _ring_choice(M: int, N: int, K: int, gateup: bool = False):
+    """(rows of a tile, column splits, whether in strips of 64 weight rows) of the product on
+    the transfer ring, None where the other forms are faster."""
+    wide = _ring_plan(M, N, K, gateup)
+    splits = _ring_narrow(M, N, K, gateup, wide)
+    if splits:
+        return 32 * -(-M // 32), splits, True
+    return wide and (*wide, False)
+
+
+def _ring(x: torch.Tensor, w: torch.Tensor, plan: Tuple[int, ...], act: int = 0) -> torch.Tensor:
+    """x @ w^T, or act 1 (silu), 2 (tanh gelu) of the gate rows times the up rows. plan: (rows
+    of a tile, column splits), and whether in strips of 64 weight rows."""
     lib, hip = _lib()
-    K, (tile, splits) = x.shape[-1], plan
+    K, (tile, splits), narrow = x.shape[-1], plan[:2], len(plan) > 2 and plan[2]
     M, N = x.numel() // K, w.shape[0] // (2 if act else 1)
     out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
     # at most 256 tiles of 128 x 128 float32 (gate and up): 17 MB
@@ -275,7 +335,7 @@ def _ring(x: torch.Tensor, w: torch.Tensor, plan: Tuple[int, int], act: int = 0)
     hip.check(lib.oa_ring_gemm(hip.current_stream_ptr(), x.data_ptr(),
                                K if x.is_contiguous() else x.stride(0), w.data_ptr(),
                                out.data_ptr(), None if part is None else part.data_ptr(),
-                               M, N, K, tile, splits, act), "oa_ring_gemm")
+                               M, N, K, tile, int(narrow), splits, act), "oa_ring_gemm")
     return out
 
 
@@ -283,11 +343,11 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear with custom HIP paths for decode shapes: the VALU GEMV at M = 1
     (hipBLASLt's M=1 kernels run ~2.5x off the HBM roofline on gfx950), the transfer
     ring up to 128 rows and the skinny matrix-core products up to 32 where they win
-    (_ring_plan, _skinny_form), the VALU GEMV for what two rows are left and the
+    (_ring_choice, _skinny_form), the VALU GEMV for what two rows are left and the
     matrix-core GEMV for what 3 to 8 are; everything else goes to hipBLASLt."""
     M = x.numel() // x.shape[-1]
     if 1 < M <= 128 and _skinny_ok(x, w):
-        plan = _ring_plan(M, w.shape[0], w.shape[1])
+        plan = _ring_choice(M, w.shape[0], w.shape[1])
         if plan:
             return _ring(x, w, plan)
         form = _skinny_form(M, w.shape[0], w.shape[1], strided=not x.is_contiguous())
@@ -931,7 +991,7 @@ def _gateup_form(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int):
             and gate_up_w.is_contiguous()):
         return None
     if 1 < M <= 128 and _skinny_ok(x, gate_up_w) and gate_up_w.shape[0] == 2 * i_local:
-        plan = _ring_plan(M, i_local, K, gateup=True)
+        plan = _ring_choice(M, i_local, K, gateup=True)
         if plan:
             return "ring", plan
         form = _skinny_form(M, i_local, K, gateup=True)

@@ -1,8 +1,8 @@
 // Products of 2 to 128 rows with large weights: C[M, N] = x[M, K] W[N, K]^T in bf16, plain
 // or gate-up with its activation. What bounds them is the weight stream, so everything
 // serves to keep enough of it under way on every CU: both operands by direct transfers
-// into a deep ring in LDS (no registers held by loads in flight), one block per CU, columns
-// split where the strips alone would leave CUs idle, and weights read without being kept
+// into a deep ring in LDS (no registers held by loads in flight), one or two blocks per CU,
+// columns split where the strips alone would leave CUs idle, and weights read without being kept
 // (nt) where they pass once: 5.9 TB/s, plain transfers of the same pieces reach 5.3. Us in
 // graphs over 2 GB of weights, before (skinny.hip up to 32 rows, the library and the
 // activation kernel above) / here: gate-up 2 x 14336 x 4096, M = 32 56.5 / 47.6, 47 55.7 /
@@ -10,13 +10,22 @@
 // 75.4 / 33.5; 6144 x 4096, M = 8 17.4 / 13.2, 47 18.0 / 16.4, 77 22.7 / 18.0; 32000 x 4096,
 // M = 32 57.8 / 48.5, 77 56.3 / 53.7; 8192 x 28672, M = 8 89.3 / 75.4, 47 140 / 81.0, 77
 // 194 / 88.9. (The same over 0.5 GB reads up to a fifth better than inside a model.)
+//
+// Up to 64 rows a strip of 64 weight rows leaves LDS for two blocks a CU, whose rings keep
+// more under way than one deep ring and start and end at different times; one strip more
+// than fills the CUs no longer waits for a whole round either. Us, strips of 128 (or the
+// other forms where those were faster) / 64: gate-up 2 x 14336 x 4096, M = 8 45.0 / 40.3, 32
+// 45.4 / 42.7, 48 47.1 / 46.3; 32000 x 4096, M = 8 50.0 / 45.9, 24 51.1 / 44.7, 47 52.6 / 47.6;
+// 2048 x 8192, M = 8 11.1 / 10.2, 47 14.1 / 12.1; 4096 x 4096, M = 24 11.8 / 10.4, 47 13.5 /
+// 11.7; 3072 x 2048, M = 47 11.6 / 9.1. More rows are bound by what a CU reads of x, which
+// narrow strips double: 32000 x 4096, M = 80 55.2 / 55.4, gate-up 2 x 14336 x 4096, M = 64
+// 48.0 / 49.8, 80 49.3 / 54.1.
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) float rgf4;
 typedef __attribute__((ext_vector_type(8))) short rgs8;
 typedef __attribute__((ext_vector_type(8))) int rgi8;
 
-#define RG_N 128                        // weight rows of a strip
 #define RG_K 64                         // bf16 columns of a step: 128 bytes; fp8: 128
 
 template <int V>
@@ -32,12 +41,13 @@ __device__ __forceinline__ float rg_gate(float g, float u, int act) {
     return g / (1.0f + __expf(-g)) * u;
 }
 
-// A block of four waves takes BM rows, a strip of 128 weight rows (GU: 64 gate rows and
-// the 64 up rows beside them) and one of `splits` runs of 64-column steps; a wave takes
-// all rows by 32 of the strip on v_mfma_f32_16x16x32_bf16, weights as the first operand,
-// so that a lane ends with four neighbouring outputs of one row. Both operands come by
-// 16-byte global_load_lds into a ring of STAGES steps: STAGES - 1 under way while one
-// is in use, waits that leave the younger ones in flight (inline asm: hipcc's own waits
+// A block of four waves takes BM rows, a strip of RN = 128 or 64 weight rows (GU: half of
+// them gate rows, half the up rows beside them) and one of `splits` runs of 64-column steps;
+// a wave takes all rows by a quarter of the strip on v_mfma_f32_16x16x32_bf16, weights as
+// the first operand, so that a lane ends with four neighbouring outputs of one row (GU: with
+// gate and up of four outputs in its two fragments; in strips of 64 of two in its one, whose
+// rows go gate, gate, up, up). Both operands come by 16-byte global_load_lds into a ring of
+// STAGES steps: STAGES - 1 under way while one is in use, waits that leave the younger ones in flight (inline asm: hipcc's own waits
 // drain builtin transfers before the first LDS read), one barrier per step, which says
 // that the step has landed for every wave and that the one before is no longer read.
 // 16-byte chunk c of row r lies at c ^ (r >> 1 & 7): the 16 rows of a fragment read
@@ -49,13 +59,14 @@ __device__ __forceinline__ float rg_gate(float g, float u, int act) {
 // 37.5 / 31.1; 4096 x 14336, 9 66.3 / 14.9, 47 71.4 / 18.2, 128 78.9 / 26.5; 6144 x 4096, 47
 // 26.9 / 13.2; 4096 x 4096, 77 28.6 / 14.9; 8192 x 28672, 77 140 / 46.8; 2048 x 2816, 33 20.0
 // / 8.7.
-template <int BM, int STAGES, bool GU, bool NT, bool F8>
-__global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
+template <int BM, int RN, int STAGES, bool GU, bool NT, bool F8>
+__global__ __launch_bounds__(256, RN > 64 ? 1 : 2) void ring_gemm_kernel(
     const char* __restrict__ x, int64_t xs, const char* __restrict__ w,
     const float* __restrict__ xscale, const float* __restrict__ wscale,
     uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int K, int mtiles,
     int splits, int items, int act) {
-    constexpr int MT = BM / 16, LPS = 4 + BM / 32, STEP = (RG_N + BM) * 128;
+    constexpr int MT = BM / 16, NF = RN / 64, WPS = RN / 32;    // fragments, transfers of a wave
+    constexpr int LPS = WPS + BM / 32, STEP = (RN + BM) * 128;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int per = gridDim.x >> 3;
     const int item = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
@@ -74,26 +85,27 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
     uint32_t dst[LPS];
 #pragma unroll
     for (int p = 0; p < LPS; ++p) {
-        const bool isw = p < 4;
-        const int r = (isw ? wid * 4 + p : (p - 4) * 4 + wid) * 8 + lr;
+        const bool isw = p < WPS;
+        const int r = (isw ? wid * WPS + p : (p - WPS) * 4 + wid) * 8 + lr;
         const int chunk = (lane & 7) ^ (r >> 1 & 7);
         int64_t at;
         if (!isw) at = min(m0 + r, M - 1) * xs * (F8 ? 1 : 2);
-        else if (GU) at = (min(strip * 64 + (r >> 5) * 16 + (r & 15), N - 1) + (r & 16 ? N : 0)) * kb;
-        else at = min(strip * RG_N + r, N - 1) * kb;
+        else if (GU && NF == 2) at = (min(strip * 64 + (r >> 5) * 16 + (r & 15), N - 1) + (r & 16 ? N : 0)) * kb;
+        else if (GU) at = (min(strip * 32 + (r >> 2) * 2 + (r & 1), N - 1) + (r & 2 ? N : 0)) * kb;
+        else at = min(strip * RN + r, N - 1) * kb;
         src[p] = (isw ? w : x) + at + (int64_t)s0 * 128 + chunk * 16;
-        dst[p] = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + (isw ? 0 : RG_N * 128) +
+        dst[p] = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + (isw ? 0 : RN * 128) +
                                                 (r - lr) * 128);
     }
     auto stage = [&](int buf) {
 #pragma unroll
         for (int p = 0; p < LPS; ++p) {
-            if (NT && p < 4) lds_transfer16<true>(dst[p] + buf * STEP, src[p]);
+            if (NT && p < WPS) lds_transfer16<true>(dst[p] + buf * STEP, src[p]);
             else lds_transfer16(dst[p] + buf * STEP, src[p]);
             src[p] += 128;
         }
     };
-    rgf4 acc[2][MT] = {};
+    rgf4 acc[NF][MT] = {};
     const int n = s1 - s0;
 #pragma unroll
     for (int t = 0; t < STAGES - 1; ++t)
@@ -120,15 +132,15 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
                 f.h[1] = *reinterpret_cast<const uint4*>(rows + at2);
                 return f.v;
             };
-            rgi8 wf[2], xf[MT];
+            rgi8 wf[NF], xf[MT];
 #pragma unroll
-            for (int j = 0; j < 2; ++j) wf[j] = frag(b + (wid * 32 + j * 16) * 128);
+            for (int j = 0; j < NF; ++j) wf[j] = frag(b + (wid * NF + j) * 16 * 128);
 #pragma unroll
-            for (int m = 0; m < MT; ++m) xf[m] = frag(b + (RG_N + m * 16) * 128);
+            for (int m = 0; m < MT; ++m) xf[m] = frag(b + (RN + m * 16) * 128);
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+                for (int j = 0; j < NF; ++j)
                     acc[j][m] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
                         wf[j], xf[m], acc[j][m], 0, 0, 0, 0x7f, 0, 0x7f);
         } else {
@@ -136,17 +148,17 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
             for (int kk = 0; kk < 2; ++kk) {
                 const int r = lane & 15, c = kk * 4 + (lane >> 4);
                 const int at = r * 128 + ((c ^ (r >> 1)) << 4);         // rows step by 16: r >> 1 & 7 stays
-                rgs8 wf[2], xf[MT];
+                rgs8 wf[NF], xf[MT];
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    wf[j] = *reinterpret_cast<const rgs8*>(b + (wid * 32 + j * 16) * 128 + at);
-#pragma unroll
-                for (int m = 0; m < MT; ++m)
-                    xf[m] = *reinterpret_cast<const rgs8*>(b + (RG_N + m * 16) * 128 + at);
+                for (int j = 0; j < NF; ++j)
+                    wf[j] = *reinterpret_cast<const rgs8*>(b + (wid * NF + j) * 16 * 128 + at);
 #pragma unroll
                 for (int m = 0; m < MT; ++m)
+                    xf[m] = *reinterpret_cast<const rgs8*>(b + (RN + m * 16) * 128 + at);
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
+                for (int m = 0; m < MT; ++m)
+#pragma unroll
+                    for (int j = 0; j < NF; ++j)
                         acc[j][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[m], acc[j][m], 0, 0, 0);
             }
         }
@@ -158,24 +170,36 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
     for (int m = 0; m < MT; ++m) {
         const int row = m0 + m * 16 + (lane & 15);
         if (row >= M) continue;
-        if (GU) {
+        if (GU && NF == 1) {
+            const int col = strip * 32 + wid * 8 + q / 2;
+            if (col >= N) continue;
+            const rgf4 a = acc[0][m];
+            if (part) {
+                float* p = part + ((size_t)sp * M + row) * 2 * N + col;
+                *reinterpret_cast<float2*>(p) = make_float2(a[0], a[1]);
+                *reinterpret_cast<float2*>(p + N) = make_float2(a[2], a[3]);
+            } else {
+                *reinterpret_cast<uint32_t*>(out + (size_t)row * N + col) =
+                    pack_bf16x2(rg_gate(a[0], a[2], act), rg_gate(a[1], a[3], act));
+            }
+        } else if (GU) {
             const int col = strip * 64 + wid * 16 + q;
             if (col >= N) continue;
             if (part) {
                 float* p = part + ((size_t)sp * M + row) * 2 * N + col;
                 *reinterpret_cast<rgf4*>(p) = acc[0][m];
-                *reinterpret_cast<rgf4*>(p + N) = acc[1][m];
+                *reinterpret_cast<rgf4*>(p + N) = acc[NF - 1][m];
             } else {
                 float o[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) o[i] = rg_gate(acc[0][m][i], acc[1][m][i], act);
+                for (int i = 0; i < 4; ++i) o[i] = rg_gate(acc[0][m][i], acc[NF - 1][m][i], act);
                 *reinterpret_cast<uint2*>(out + (size_t)row * N + col) =
                     make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
             }
         } else {
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int col = strip * RG_N + wid * 32 + j * 16 + q;
+            for (int j = 0; j < NF; ++j) {
+                const int col = strip * RN + (wid * NF + j) * 16 + q;
                 if (col >= N) continue;
                 if (part) {
                     *reinterpret_cast<rgf4*>(part + ((size_t)sp * M + row) * N + col) = acc[j][m];
@@ -225,43 +249,48 @@ __global__ __launch_bounds__(256) void ring_sum_kernel(const float* __restrict__
 }
 
 // out [M, N] = x [M, K] w [N, K]^T, x rows xs elements apart. act 1 (silu), 2 (tanh gelu):
-// out = act(x w[:N]^T) * (x w[N:]^T), w [2 N, K]. bm: rows of a tile, 32, 64, 96 or 128.
+// out = act(x w[:N]^T) * (x w[N:]^T), w [2 N, K]. bm: rows of a tile, 32, 64, 96 or 128;
+// narrow: strips of 64 weight rows (bm 32 and 64).
 // scratch: splits * M * N floats (act: twice that), unused at splits 1.
 extern "C" int oa_ring_gemm(void* stream, const void* x, int64_t xs, const void* w, void* out,
-                            void* scratch, int M, int N, int K, int bm, int splits, int act) {
+                            void* scratch, int M, int N, int K, int bm, int narrow, int splits,
+                            int act) {
     if (M < 1 || M > 65535 || N < 4 || N % 4 != 0 || K < RG_K || K % RG_K != 0) return -100;
     if (splits < 1 || splits > K / RG_K || (splits > 1 && !scratch)) return -101;
     if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)scratch) % 16 != 0 || xs % 8 != 0)
         return -102;
-    if (act < 0 || act > 2 || (bm != 32 && bm != 64 && bm != 96 && bm != 128)) return -104;
+    if (act < 0 || act > 2 || (bm != 32 && bm != 64 && bm != 96 && bm != 128) || (narrow && bm > 64)) return -104;
     const bool gateup = act != 0;
     const int mtiles = CEIL_DIV(M, bm);
-    const int64_t items = (int64_t)(gateup ? CEIL_DIV(N, 64) : CEIL_DIV(N, RG_N)) * mtiles * splits;
+    const int64_t items = (int64_t)CEIL_DIV(N, (narrow ? 64 : 128) / (gateup ? 2 : 1)) * mtiles * splits;
     if (items > (1 << 28)) return -103;
     hipStream_t s = (hipStream_t)stream;
     const dim3 grid((unsigned)(CEIL_DIV(items, 8) * 8)), block(256);
     float* part = splits > 1 ? (float*)scratch : nullptr;
-#define RG(BMV, ST, G, NT)                                                                         \
-    hipLaunchKernelGGL((ring_gemm_kernel<BMV, ST, G, NT, false>), grid, block, (ST) * (RG_N + (BMV)) * 128, s, \
-                       (const char*)x, xs, (const char*)w, (const float*)nullptr,                  \
-                       (const float*)nullptr, (uint16_t*)out, part, M, N, K, mtiles, splits,       \
-                       (int)items, act)
-#define RGB(BMV, ST, NT)               \
-    do {                               \
-        if (gateup) RG(BMV, ST, true, NT); \
-        else RG(BMV, ST, false, NT);   \
+#define RG(BMV, RNV, ST, G, NT)                                                                    \
+    hipLaunchKernelGGL((ring_gemm_kernel<BMV, RNV, ST, G, NT, false>), grid, block,                 \
+                       (ST) * ((RNV) + (BMV)) * 128, s, (const char*)x, xs, (const char*)w,         \
+                       (const float*)nullptr, (const float*)nullptr, (uint16_t*)out, part, M, N, K, \
+                       mtiles, splits, (int)items, act)
+#define RGB(BMV, RNV, ST, NT)               \
+    do {                                    \
+        if (gateup) RG(BMV, RNV, ST, true, NT); \
+        else RG(BMV, RNV, ST, false, NT);   \
     } while (0)
     // read without being kept: weights no other row tile reads, unless there are many rows
     // and few weights (us kept / not, 6144 x 4096, M = 8 14.3 / 13.2, 77 18.2 / 20.2; 2 x 8192
     // x 2048, 47 18.5 / 16.4; 8192 x 28672, 77 98.9 / 88.6)
     const bool nt = mtiles == 1 && (bm == 32 || (int64_t)N * K * (gateup ? 2 : 1) >= 32000000);
-    if (bm == 32) RGB(32, 6, true);
-    else if (bm == 64 && nt) RGB(64, 5, true);
-    else if (bm == 64) RGB(64, 5, false);
-    else if (bm == 96 && nt) RGB(96, 5, true);
-    else if (bm == 96) RGB(96, 5, false);
-    else if (nt) RGB(128, 4, true);
-    else RGB(128, 4, false);
+    if (narrow && bm == 32) RGB(32, 64, 6, true);
+    else if (narrow && nt) RGB(64, 64, 4, true);
+    else if (narrow) RGB(64, 64, 4, false);
+    else if (bm == 32) RGB(32, 128, 6, true);
+    else if (bm == 64 && nt) RGB(64, 128, 5, true);
+    else if (bm == 64) RGB(64, 128, 5, false);
+    else if (bm == 96 && nt) RGB(96, 128, 5, true);
+    else if (bm == 96) RGB(96, 128, 5, false);
+    else if (nt) RGB(128, 128, 4, true);
+    else RGB(128, 128, 4, false);
 #undef RGB
 #undef RG
     if (splits > 1) {
@@ -289,14 +318,14 @@ extern "C" int oa_ring_gemm_fp8(void* stream, const void* x8, const void* xscale
     if (((uintptr_t)x8 | (uintptr_t)w8 | (uintptr_t)out | (uintptr_t)scratch) % 16 != 0) return -102;
     if ((bm != 32 && bm != 64 && bm != 96 && bm != 128) || (M > bm && bm != 128)) return -104;
     const int mtiles = CEIL_DIV(M, bm);
-    const int64_t items = (int64_t)CEIL_DIV(N, RG_N) * mtiles * splits;
+    const int64_t items = (int64_t)CEIL_DIV(N, 128) * mtiles * splits;
     if (items > (1 << 28)) return -103;
     hipStream_t s = (hipStream_t)stream;
     float* part = splits > 1 ? (float*)scratch : nullptr;
 #define RG8(BMV, ST, NT)                                                                           \
-    hipLaunchKernelGGL((ring_gemm_kernel<BMV, ST, false, NT, true>),                               \
+    hipLaunchKernelGGL((ring_gemm_kernel<BMV, 128, ST, false, NT, true>),                               \
                        dim3((unsigned)(CEIL_DIV(items, 8) * 8)), dim3(256),                        \
-                       (ST) * (RG_N + (BMV)) * 128, s, (const char*)x8, (int64_t)K, (const char*)w8, \
+                       (ST) * (128 + (BMV)) * 128, s, (const char*)x8, (int64_t)K, (const char*)w8, \
                        (const float*)xscale, (const float*)wscale, (uint16_t*)out, part, M, N, K,  \
                        mtiles, splits, (int)items, 0)
     if (bm == 32) RG8(32, 6, true);

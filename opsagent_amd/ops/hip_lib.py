@@ -55,7 +55,7 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_gemv_grouped.restype = i
     lib.oa_gemv_split.argtypes = [p, p, p, p, i, i, i, i]
     lib.oa_gemv_split.restype = i
-    lib.oa_ring_gemm.argtypes = [p, p, i64, p, p, p, i, i, i, i, i, i]
+    lib.oa_ring_gemm.argtypes = [p, p, i64, p, p, p, i, i, i, i, i, i, i]
     lib.oa_ring_gemm.restype = i
     lib.oa_ring_gemm_fp8.argtypes = [p, p, p, p, p, p, p, i, i, i, i, i]
     lib.oa_ring_gemm_fp8.restype = i

@@ -176,3 +176,48 @@ def test_lines_agree(M, N, K):
     want = x.double() @ w.double().T
     # one bf16 rounding of a float32 sum: 0.0016 in the mean
     assert float((ops.linear(x, w).double() - want).norm() / want.norm()) < 2e-3
+
+
+NARROW = [(3, 8, 64, 32, 1), (32, 200, 320, 32, 2), (33, 72, 448, 64, 3), (64, 264, 1024, 64, 1),
+          (17, 64, 4096, 32, 8), (48, 1000, 256, 64, 4)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,tile,splits", NARROW)
+def test_narrow_strips(M, N, K, tile, splits):
+    """Strips of 64 weight rows, two blocks a CU: fewer steps than the ring holds, runs that
+    differ by a step, strips and tiles part filled, rows of x that lie apart."""
+    torch.manual_seed(M + N + K)
+    wide, w = _whole(M, K + 8), _whole(N, K)
+    for x in (wide[:, :K].contiguous(), wide[:, :K]):
+        got = ops._ring(x, w, (tile, splits, True))
+        assert torch.equal(got, (x.double() @ w.double().T).to(torch.bfloat16))
+    x, w = _whole(M, K), _whole(2 * N, K, 2.0 ** -5)
+    g, u = (x.double() @ w.double().T).split(N, 1)
+    for act in (1, 2):
+        got = ops._ring(x, w, (tile, splits, True), act).double()
+        f = torch.nn.functional.silu(g) if act == 1 else torch.nn.functional.gelu(g, approximate="tanh")
+        # as in test_gateup
+        bound = 2.0 ** -8 * (f * u).abs() + 2.0 ** -20 * (1 + g.abs()) * (g * u).abs()
+        assert ((got - f * u).abs() <= bound).all()
+
+
+def test_narrow_plans():
+    choice = ops._ring_choice
+    assert choice(8, 14336, 4096, True) == (32, 1, True) and choice(48, 14336, 4096, True) == (64, 1, True)
+    assert choice(49, 14336, 4096, True) == (64, 1, False) and choice(2, 14336, 4096, True) is None
+    assert choice(8, 11008, 4096, True) is None                # 344 blocks: a round two thirds full
+    assert choice(24, 2048, 2048) is None                      # under 10 MB
+    assert choice(24, 4096, 4096) == (32, 4, True) and choice(8, 4096, 4096) is None
+    assert choice(48, 2048, 8192) == (64, 8, True) and choice(49, 2048, 8192)[2] is False
+    assert choice(64, 16384, 4096) == (64, 1, True)           # the library's otherwise
+    assert choice(32, 8192, 28672)[2] is False and choice(8, 16384, 4096)[2] is False
+    assert choice(8, 32000, 4096) == (32, 1, True) and choice(48, 32000, 4096) == (64, 1, True)
+    assert choice(24, 8192, 2048, True)[2] is False and choice(24, 8192, 3072, True) == (32, 1, True)
+    for gateup in (False, True):
+        for K in (64, 640, 1408, 2048, 4096, 14336):
+            for N in (8, 1024, 3072, 6144, 32000, 128256):
+                for M in range(1, 130):
+                    plan = choice(M, N, K, gateup)
+                    if plan and plan[2]:
+                        assert 2 < M <= plan[0] <= 64 and 1 <= plan[1] <= K // 64
