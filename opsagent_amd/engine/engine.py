@@ -642,7 +642,7 @@ class LLMEngine:
         Capacity for start+count tokens must already be ensured. Returns the
         model's hidden rows [sum(count), C] in work order and marks the
         tokens cached."""
-        from opsagent_amd.ops.mixer_ops import SeqBatch
+        from opsagent_amd.ops.mixer_ops import SeqBatch, to_device
 
         ids: List[int] = []
         chunks = []
@@ -661,7 +661,7 @@ class LLMEngine:
             sb = SeqBatch.build(chunks, self.block_size, self.device)
             fb = ForwardBatch(
                 kind="mixed",
-                input_ids=torch.tensor(ids, dtype=torch.int64).to(self.device),
+                input_ids=to_device(torch.tensor(ids, dtype=torch.int64), self.device),
                 positions=None,
                 slot_mapping=sb.slot_mapping,
                 seq_batch=sb,
@@ -682,35 +682,38 @@ class LLMEngine:
         bucket = self._bucket(B)
         ent = self._graphs.get(bucket)
         mb = self.max_blocks_per_seq
-        # flat int32 layout: cu | past | slots | seq_of | slot_map | block table
-        o1, o2, o3, o4, o5 = (bucket + 1, 2 * bucket + 1, 3 * bucket + 1,
-                              4 * bucket + 1, 5 * bucket + 1)
+        # flat int32 layout: token ids (int64) | cu | past | slots | seq_of | slot_map | block table
+        o0 = 2 * bucket
+        o1, o2, o3, o4, o5 = (o0 + bucket + 1, o0 + 2 * bucket + 1, o0 + 3 * bucket + 1,
+                              o0 + 4 * bucket + 1, o0 + 5 * bucket + 1)
         if ent is None:
-            dev = self.device
-            flat = torch.zeros(o5 + bucket * mb, dtype=torch.int32, device=dev)
+            flat = torch.zeros(o5 + bucket * mb, dtype=torch.int32, device=self.device)
             sb = SeqBatch(
                 cu=list(range(bucket + 1)), past=[0] * bucket, slots=[0] * bucket,
-                cu_t=flat[:o1], past_t=flat[o1:o2], slots_t=flat[o2:o3],
+                cu_t=flat[o0:o1], past_t=flat[o1:o2], slots_t=flat[o2:o3],
                 seq_of_t=flat[o3:o4], slot_mapping=flat[o4:o5],
                 block_table=flat[o5:].view(bucket, mb),
                 max_chunk=1, max_total=mb * self.block_size,
             )
             ent = {
                 "sb": sb, "flat": flat, "graph": None, "out": None,
-                "ids": torch.zeros(bucket, dtype=torch.int64, device=dev),
-                "h_flat": torch.zeros(o5 + bucket * mb, dtype=torch.int32, pin_memory=True),
-                "h_ids": torch.zeros(bucket, dtype=torch.int64, pin_memory=True),
+                "ids": flat[:o0].view(torch.int64),
             }
             self._graphs[bucket] = ent
         sb, ids_t = ent["sb"], ent["ids"]
-        # persistent pinned staging -> two copies per step. Padding rows hold
-        # zero tokens (cu stays flat), so no kernel touches any state for
-        # them. sb's HOST lists stay at the bucket's upper bound (one token
-        # per row): they only size launches; kernels read the device copies.
-        hf = ent["h_flat"].numpy()
+        # One copy per step, from a pinned buffer of its own that the allocator gives out
+        # again once the copy is done: the host does not wait for the step before. Padding
+        # rows hold zero tokens (cu stays flat), so no kernel touches any state for them.
+        # sb's HOST lists stay at the bucket's upper bound (one token per row): they only
+        # size launches; kernels read the device copies.
+        staged = torch.empty(o5 + bucket * mb, dtype=torch.int32, pin_memory=True)
+        hf = staged.numpy()
         bs = self.block_size
-        hf[:o1] = [min(i, B) for i in range(bucket + 1)]
-        hf[o1:o5] = 0
+        hi = hf[:o0].view("int64")
+        hi[:] = ids[0]
+        hi[:B] = ids
+        hf[o0:o1] = [min(i, B) for i in range(bucket + 1)]
+        hf[o1:] = 0
         hf[o1 : o1 + B] = [c[0] for c in chunks]
         hf[o2 : o2 + B] = [c[2] for c in chunks]
         hf[o3 : o3 + B] = range(B)
@@ -719,12 +722,7 @@ class LLMEngine:
         hf[o4 : o4 + B] = slot_map
         for b, c in enumerate(chunks):
             hf[o5 + b * mb : o5 + b * mb + len(c[3])] = c[3]
-        hi = ent["h_ids"].numpy()
-        hi[:] = ids[0]
-        hi[:B] = ids
-        # blocking copies: the staging buffers are rewritten next step
-        ent["flat"].copy_(ent["h_flat"])
-        ids_t.copy_(ent["h_ids"])
+        ent["flat"].copy_(staged, non_blocking=True)
         fb = ForwardBatch(kind="mixed", input_ids=ids_t, positions=None,
                           slot_mapping=sb.slot_mapping, seq_batch=sb)
         if ent["graph"] is None:
@@ -755,6 +753,8 @@ class LLMEngine:
         in the SAME forward — requests still reading their prompt (or owing
         fast-forwarded tokens) contribute a portion under a shared token
         budget, decoding requests one token each."""
+        from opsagent_amd.ops.mixer_ops import to_device
+
         t0 = time.perf_counter()
         work: List[Tuple[Request, int, int]] = []
         budget = self.max_prefill_chunk
@@ -787,9 +787,10 @@ class LLMEngine:
                 rows.append(off - 1)
                 batch.append(req)
         if batch:
-            idx = torch.tensor(rows, dtype=torch.int64).to(self.device)
-            logits = self.model.compute_logits(hidden.index_select(0, idx))
-            self._sample_and_append(batch, logits)
+            if rows != list(range(len(hidden))):
+                hidden = hidden.index_select(0, to_device(torch.tensor(rows, dtype=torch.int64),
+                                                          self.device))
+            self._sample_and_append(batch, self.model.compute_logits(hidden))
         self._reap()
         self.perf.record_metric("engine_mixed_step_ms", (time.perf_counter() - t0) * 1000.0)
         self.perf.record_metric("engine_mixed_step_tokens", float(off))

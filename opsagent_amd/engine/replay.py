@@ -21,6 +21,7 @@ import torch
 
 from opsagent_amd.engine.engine import LLMEngine, Request, SamplingParams
 from opsagent_amd.engine.kv_cache import SequenceState
+from opsagent_amd.ops.mixer_ops import to_device
 
 
 class TraceReplayer:
@@ -58,8 +59,10 @@ class TraceReplayer:
         if work:
             hidden = eng._forward_mixed(work)
             if rows:
-                idx = torch.tensor(rows, dtype=torch.int64).to(eng.device)
-                logits = eng.model.compute_logits(hidden.index_select(0, idx)).float()
+                if rows != list(range(len(hidden))):
+                    idx = to_device(torch.tensor(rows, dtype=torch.int64), eng.device)
+                    hidden = hidden.index_select(0, idx)
+                logits = eng.model.compute_logits(hidden).float()
         for rid in end:
             req = self.live.pop(rid, None)
             if req is not None:

@@ -16,9 +16,19 @@ import dataclasses
 import os
 from typing import List, Optional, Tuple
 
+import numpy as np
 import torch
 
 from opsagent_amd.ops import torch_ref
+
+
+def to_device(host: torch.Tensor, device) -> torch.Tensor:
+    """host on the device. A copy from ordinary memory waits for all work before it on the
+    stream; from pinned memory, which its allocator holds until the copy is done, it does not,
+    so that the host prepares a step while the GPU is at the one before."""
+    if torch.device(device).type != "cuda":
+        return host.to(device)
+    return host.pin_memory().to(device, non_blocking=True)
 
 
 @dataclasses.dataclass
@@ -51,23 +61,25 @@ class SeqBatch:
     def build(chunks: List[Tuple[int, int, int, List[int]]], block_size: int,
               device, max_blocks: Optional[int] = None) -> "SeqBatch":
         """chunks: per sequence (past_len, count, state_slot, block ids)."""
-        cu, past, slots, seq_of, slot_map, bt = [0], [], [], [], [], []
+        cu, past, slots = [0], [], []
         nb = max((len(c[3]) for c in chunks), default=1)
         max_blocks = max(max_blocks or 0, nb, 1)
-        for b, (p, n, slot, blocks) in enumerate(chunks):
+        for p, n, slot, _ in chunks:
             cu.append(cu[-1] + n)
             past.append(p)
             slots.append(slot if slot is not None else 0)
-            seq_of.extend([b] * n)
-            for pos in range(p, p + n):
-                slot_map.append(blocks[pos // block_size] * block_size + pos % block_size)
-            bt.extend(blocks)
-            bt.extend([0] * (max_blocks - len(blocks)))
-        # one host->device copy; the tensors are views of it
         B, T = len(chunks), cu[-1]
-        flat = torch.tensor(cu + past + slots + seq_of + slot_map + bt,
-                            dtype=torch.int32).to(device)
         o1, o2, o3, o4, o5 = B + 1, 2 * B + 1, 3 * B + 1, 3 * B + 1 + T, 3 * B + 1 + 2 * T
+        # one host->device copy; the tensors are views of it
+        host = np.zeros(o5 + B * max_blocks, dtype=np.int32)
+        host[:o1], host[o1:o2], host[o2:o3] = cu, past, slots
+        for b, (p, n, _, blocks) in enumerate(chunks):
+            row = host[o5 + b * max_blocks :][: len(blocks)]
+            row[:] = blocks
+            pos = np.arange(p, p + n)
+            host[o3 + cu[b] : o3 + cu[b + 1]] = b
+            host[o4 + cu[b] : o4 + cu[b + 1]] = row[pos // block_size] * block_size + pos % block_size
+        flat = to_device(torch.from_numpy(host), device)
         return SeqBatch(
             cu=cu, past=past, slots=slots, cu_t=flat[:o1], past_t=flat[o1:o2],
             slots_t=flat[o2:o3], seq_of_t=flat[o3:o4], slot_mapping=flat[o4:o5],

@@ -1,0 +1,58 @@
+"""Inputs of a flat step: their layout against plain loops, and steps that the host queues one
+after another without a wait for the GPU between them."""
+
+import pytest
+import torch
+
+import povazen_oracle as O
+from opsagent_amd.engine.replay import TraceReplayer
+from opsagent_amd.ops import mixer_ops as mx
+from test_povazen import build_engine, make_cfg, tokens_for
+
+
+@pytest.mark.parametrize("chunks", [
+    [(0, 5, 2, [7, 3]), (9, 1, 0, [4, 1, 9, 2]), (3, 0, None, [5]), (0, 11, 1, [8, 6, 0])],
+    [(0, 0, None, [])],
+    [],
+])
+@pytest.mark.parametrize("max_blocks", [None, 6])
+def test_layout(chunks, max_blocks):
+    sb = mx.SeqBatch.build(chunks, 4, "cpu", max_blocks)
+    width = max([max_blocks or 0, 1] + [len(c[3]) for c in chunks])
+    cu, seq, slot_map = [0], [], []
+    for b, (p, n, _, blocks) in enumerate(chunks):
+        cu.append(cu[-1] + n)
+        seq += [b] * n
+        slot_map += [blocks[i // 4] * 4 + i % 4 for i in range(p, p + n)]
+    assert sb.cu == cu and sb.cu_t.tolist() == cu
+    assert sb.past_t.tolist() == sb.past == [c[0] for c in chunks]
+    assert sb.slots_t.tolist() == sb.slots == [c[2] or 0 for c in chunks]
+    assert sb.seq_of_t.tolist() == seq and sb.slot_mapping.tolist() == slot_map
+    assert sb.block_table.tolist() == [c[3] + [0] * (width - len(c[3])) for c in chunks]
+    assert all(t.dtype == torch.int32 for t in (sb.cu_t, sb.slot_mapping, sb.block_table))
+    assert sb.max_chunk == max([c[1] for c in chunks], default=0)
+    assert sb.max_total == max([c[0] + c[1] for c in chunks], default=0)
+
+
+@pytest.mark.gpu
+def test_queued_steps():
+    """Forty decode steps of two traces, prompts among them: the same logits whether the host
+    waits after each step or never."""
+    cfg = make_cfg()
+    W = O.random_weights(cfg, 3)
+    a, b = tokens_for(cfg, 60, 1), tokens_for(cfg, 50, 2)
+
+    def run(wait):
+        rp = TraceReplayer(build_engine(cfg, W, "bf16"))
+        out = [rp.step([{"id": "a", "tokens": a[:20], "want": [19]}], [])]
+        out.append(rp.step([{"id": "a", "tokens": a[20:21], "want": [0]},
+                            {"id": "b", "tokens": b[:11], "want": [0, 10]}], []))
+        for t in range(39):
+            out.append(rp.step([{"id": "a", "tokens": [a[21 + t]], "want": [0]},
+                                {"id": "b", "tokens": [b[11 + t]], "want": [0]}],
+                               ["a", "b"] if t == 38 else []))
+            if wait:
+                torch.cuda.synchronize()
+        return torch.cat(out).cpu()
+
+    assert torch.equal(run(False), run(True))
