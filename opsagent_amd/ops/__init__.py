@@ -556,14 +556,29 @@ def _ring_plan_fp8(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
     return tile, 1 if splits == 2 and K < 4096 else splits
 
 
+def _ring_choice_fp8(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
+    """The ring's plan where it is faster than the tile product (fp8_moe.hip). Us, ring / tiles:
+    without splits its one block of four waves a CU falls behind with the rows (28672 x 4096,
+    M = 64 29.7 / 32.1, 96 32.9 / 32.0, 128 35.7 / 33.2; 16384 x 2048, 96 17.3 / 14.8; 4096 x 1024,
+    32 7.5 / 8.4, 48 8.7 / 8.4, 128 13.6 / 8.9); splits of short rows cost more than they fill
+    (3072 x 2048, 128 13.7 / 12.1, 200 14.9 / 12.1; 2048 x 2816, 128 13.8 / 14.5, 200 14.9 / 14.4;
+    4096 x 3072, 200 19.2 / 15.4), long rows do not (4096 x 14336, 512 48.7 / 67; 2048 x 8192, 512
+    23.2 / 37.3)."""
+    plan = _ring_plan_fp8(M, N, K)
+    if plan and (M > (32 if K < 2048 else 80) if plan[1] == 1
+                 else K < 4096 and M > 128 and M * N >= 390000):
+        return None
+    return plan
+
+
 def _gemm_fp8(a8: torch.Tensor, a_scale: torch.Tensor, w8: torch.Tensor,
               w_scale: torch.Tensor) -> torch.Tensor:
     """The product of fp8 rows a8 [M, K] (K % 128 == 0) and w8 [N, K] with their row
-    scales, bf16 [M, N]: on the transfer ring or in 128 x 128 tiles."""
+    scales, bf16 [M, N]: on the transfer ring or in tiles."""
     (M, K), N = a8.shape, w8.shape[0]
     lib, hip = _lib()
     out = torch.empty(M, N, dtype=torch.bfloat16, device=a8.device)
-    plan = _ring_plan_fp8(M, N, K)
+    plan = _ring_choice_fp8(M, N, K)
     if plan and w8.data_ptr() % 16 == 0 and a8.data_ptr() % 16 == 0:
         tile, splits = plan
         # at most 256 tiles of 128 x 128 float32: 17 MB

@@ -854,11 +854,12 @@ extern "C" int oa_gemv_gateup_fp8(void* stream, const void* x, const void* w8,
 // ---- fp8 MFMA tile GEMM (prefill path) -------------------------------------
 // C[M, N] = (A8[M, K] @ B8[N, K]^T) * a_scale[m] * b_scale[n], bf16 out.
 //
-// 128x128 tile, 4 waves (2x2 of 64x64), K-steps of 128 fp8 bytes, A and B staged by
-// 16-byte global_load_lds. XOR swizzle on the DMA source address (the LDS write is
-// lane-linear): byte ^= (row & 7) << 4 spreads the 16-lane fragment-read groups over
-// the banks at 16-byte granularity. Tail rows (M or N not a multiple of 128) clamp the
-// DMA source row and the epilogue masks the store.
+// A tile of BM x BN, sixteen waves (4 x 4), K-steps of 128 fp8 bytes, A and B staged by
+// 16-byte global_load_lds. 16-byte chunk c of row r lies at c ^ (r >> 1 & 7): LDS has 64
+// banks, and 16 rows of 128 bytes at one chunk touch each of them once (c ^ (r & 7) touches
+// half of them twice: 11 M conflict cycles of 22 M on 28672 x 4096, M = 700, none here). The
+// swizzle is on the source address, as the transfer writes lanes in order. Rows past M or N
+// repeat the last one and are not stored.
 //
 // The products are v_mfma_scale_f32_32x32x64_f8f6f4 with identity E8M0 scales (0x7f =
 // 2^0): the large-K scaled forms are the only fp8 MFMAs past the bf16 rate on gfx950;
@@ -868,153 +869,166 @@ extern "C" int oa_gemv_gateup_fp8(void* stream, const void* x, const void* w8,
 typedef __attribute__((ext_vector_type(8))) int i32x8_f8;   // 32 fp8 (MX operand)
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;  // 32x32 C/D
 
-#define GT 128    // tile M = N
 #define GK2 128   // K step in fp8 bytes
-#define GTILE_B (GT * GK2)  // 16 KiB per operand per buffer
 
-__device__ __forceinline__ uint32_t g8_swz(int row, int byte_in_row) {
-    return (uint32_t)(row * GK2 + (byte_in_row ^ ((row & 7) << 4)));
+template <int V>
+__device__ __forceinline__ void g8_wait() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(V) : "memory");
 }
 
-// A ring of STAGES K-steps: STAGES - 1 are under way while one is in use. A wait
-// leaves the younger steps' transfers in flight (vmcnt counts them in order: eight per
-// wave and step); the barrier after it says both that step t has landed for every wave
-// and that step t - 1 is no longer read, so its buffer can be filled. The transfers are
-// inline asm because hipcc's wait inserter drains builtin ones before the first LDS
-// read. Work items go to the dies in runs, with the row tiles of a column strip next to
-// each other: a strip is read into one die's L2 once.
+// A ring of ST K-steps: ST - 1 are under way while one is in use. A wait leaves the younger
+// steps' transfers in flight (vmcnt counts them in order); the barrier after it says both
+// that step t has landed for every wave and that step t - 1 is no longer read, so its
+// buffer can be filled. The transfers are inline asm because hipcc's wait inserter drains
+// builtin ones before the first LDS read. Work items go to the dies in runs, with the row
+// tiles of a column strip next to each other: a strip is read into one die's L2 once.
 //
-// What bounds it is what a CU draws from the L2, about 55 GB/s in every shape: two
-// blocks of two steps per CU reach 1.6 to 1.9 PFLOP/s, one block of four steps is the
-// faster form while there are no more blocks than CUs. Few tiles take the column-split
-// ring instead (ring_gemm.hip). us, the former kernel (two buffers, row tiles far apart;
-// register staging at K = 28672) / here: 28672 x 4096, M = 700 142 / 126, 2048 342 / 303;
-// 4096 x 14336, 700 127 / 75, 2048 145 / 132; 6144 x 4096, 700 44 / 35; 4096 x 4096, 700 39 /
-// 30; 8192 x 28672, 700 583 / 217, 2048 1201 / 502. Reading the next half-step's fragments under the
-// products made it slower (4096 x 14336, 700: 93).
-template <int STAGES>
-__global__ __launch_bounds__(256, 1) void gemm_fp8_ring_kernel(
-    const uint32_t* __restrict__ a8, const uint32_t* __restrict__ b8,
+// What bounds it is how well the waves of a CU cover each other's waits at the barrier and
+// for fragments: the matrix cores are busy for a third of the time, the LDS for a sixth, and
+// the L2 gives a CU 50 GB/s of the 150 it can. Hence sixteen waves, however small their part:
+// 4096 x 4096, M = 700 29.3 us with four waves, 23.5 with eight, 21.1 with sixteen; 4096 x
+// 14336 75 / 64 / 60; 28672 x 4096 in tiles of 128 x 256 114 with eight, 108 with sixteen.
+// Reading fragments ahead of the products, carrying them over the barrier and spreading the
+// transfers between the products were all slower. us, before (128 x 128, four waves) / 128 x
+// 128 in a ring of four / two blocks a CU in rings of two / 128 x 256 in three / 256 x 256 in
+// two: 28672 x 4096, M = 512 94 / 96 / 85 / 78 / 68, 700 128 / 130 / 119 / 108 / 119, 2048 306 /
+// 331 / 290 / 271 / 251; 4096 x 14336, 700 76 / 61 / 101 / 94 / 162, 2048 132 / 146 / 139 / 112 /
+// 173; 6144 x 4096, 700 34.5 / 40.5 / 30.1 / 31.8 / 49; 2048 x 8192, 700 45.9 / 33.7 / 43 / 49 /
+// 81; 16384 x 2048, 700 52.9 / 43.5 / 42.9 / 44.2 / 37.9.
+template <int BM, int BN, int ST, int BLOCKS>
+__global__ __launch_bounds__(1024, 4 * BLOCKS) void gemm_fp8_tile_kernel(
+    const char* __restrict__ a8, const char* __restrict__ b8,
     const float* __restrict__ ascale, const float* __restrict__ bscale,
     uint16_t* __restrict__ c, int M, int N, int K, int mtiles, int items) {
+    constexpr int FI = BM / 128, FJ = BN / 128;                        // fragments of a wave
+    constexpr int STEP = (BM + BN) * GK2, LPW = (BM + BN) / 128;       // transfers of a wave
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int per = gridDim.x >> 3;
     const int item = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (item >= items) return;
     const int nt = item / mtiles;
-    const int tm = (item - nt * mtiles) * GT, tn = nt * GT;
+    const int tm = (item - nt * mtiles) * BM, tn = nt * BN;
     const int lane = threadIdx.x & (WAVE - 1);
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const int wr = wid >> 1, wc = wid & 1;
+    const int wr = wid >> 2, wc = wid & 3;
 
-    f32x16_t accw[2][2] = {};
-    const int arow_l = lane >> 3;
-    const int abyte_l = ((lane & 7) * 16) ^ ((arow_l & 7) << 4);
-    const char* asrc[4];
-    const char* bsrc[4];
+    const char* src[LPW];
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        const int ch = wid * 4 + p;
-        asrc[p] = reinterpret_cast<const char*>(a8) + (size_t)min(tm + ch * 8 + arow_l, M - 1) * K + abyte_l;
-        bsrc[p] = reinterpret_cast<const char*>(b8) + (size_t)min(tn + ch * 8 + arow_l, N - 1) * K + abyte_l;
+    for (int p = 0; p < LPW; ++p) {
+        const int r = (p * 16 + wid) * 8 + (lane >> 3);      // row of A, then of B
+        const int64_t at = r < BM ? (int64_t)min(tm + r, M - 1) * K : (int64_t)min(tn + r - BM, N - 1) * K;
+        src[p] = (r < BM ? a8 : b8) + at + ((lane & 7) ^ (r >> 1 & 7)) * 16;
     }
-    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + wid * 4096);
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + wid * 1024);
     auto stage = [&](int buf) {
-        const uint32_t at = lds0 + buf * 2 * GTILE_B;
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            lds_transfer16(at + p * 1024, asrc[p]);
-            lds_transfer16(at + GTILE_B + p * 1024, bsrc[p]);
-        }
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            asrc[p] += GK2;
-            bsrc[p] += GK2;
+        for (int p = 0; p < LPW; ++p) {
+            lds_transfer16(lds0 + buf * STEP + p * 16 * 1024, src[p]);
+            src[p] += GK2;
         }
     };
-    auto compute = [&](const char* abuf, const char* bbuf) {
+    const int fr = lane & 31, kh = lane >> 5, sw = fr >> 1 & 7;
+    auto frag = [&](const char* rows, int kk) {
+        union {
+            uint4 h[2];
+            i32x8_f8 v;
+        } f;
+        f.h[0] = *reinterpret_cast<const uint4*>(rows + fr * GK2 + (((kk * 4 + kh * 2) ^ sw) << 4));
+        f.h[1] = *reinterpret_cast<const uint4*>(rows + fr * GK2 + (((kk * 4 + kh * 2 + 1) ^ sw) << 4));
+        return f.v;
+    };
+    f32x16_t acc[FI][FJ] = {};
+    const int ns = K / GK2;
+#pragma unroll
+    for (int t = 0; t < ST - 1; ++t)
+        if (t < ns) stage(t);
+    int buf = 0;
+    for (int t = 0; t < ns; ++t) {
+        const int behind = min(ST - 2, ns - 1 - t);          // younger steps under way
+        if (ST > 3 && behind >= 2) g8_wait<2 * LPW>();
+        else if (ST > 2 && behind >= 1) g8_wait<LPW>();
+        else g8_wait<0>();
+        const char* ab = smem + buf * STEP + wr * FI * 32 * GK2;
+        const char* bb = smem + buf * STEP + (BM + wc * FJ * 32) * GK2;
+        if (t + ST - 1 < ns) stage(buf == 0 ? ST - 1 : buf - 1);
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
-            const int kb = kk * 64 + (lane >> 5) * 32;
-            i32x8_f8 afrag[2], bfrag[2];
+            i32x8_f8 fa[FI], fb[FJ];
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int arow = wr * 64 + i * 32 + (lane & 31);
-                const int brow = wc * 64 + i * 32 + (lane & 31);
-                *reinterpret_cast<uint4*>(&afrag[i]) =
-                    *reinterpret_cast<const uint4*>(abuf + g8_swz(arow, kb));
-                *(reinterpret_cast<uint4*>(&afrag[i]) + 1) =
-                    *reinterpret_cast<const uint4*>(abuf + g8_swz(arow, kb + 16));
-                *reinterpret_cast<uint4*>(&bfrag[i]) =
-                    *reinterpret_cast<const uint4*>(bbuf + g8_swz(brow, kb));
-                *(reinterpret_cast<uint4*>(&bfrag[i]) + 1) =
-                    *reinterpret_cast<const uint4*>(bbuf + g8_swz(brow, kb + 16));
-            }
+            for (int i = 0; i < FI; ++i) fa[i] = frag(ab + i * 32 * GK2, kk);
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int j = 0; j < FJ; ++j) fb[j] = frag(bb + j * 32 * GK2, kk);
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    accw[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                        afrag[i], bfrag[j], accw[i][j], 0, 0, 0, 0x7f, 0, 0x7f);
+            for (int i = 0; i < FI; ++i)
+#pragma unroll
+                for (int j = 0; j < FJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                        fa[i], fb[j], acc[i][j], 0, 0, 0, 0x7f, 0, 0x7f);
         }
-    };
-    const int nsteps = K / GK2;
-#pragma unroll
-    for (int t = 0; t < STAGES - 1; ++t)
-        if (t < nsteps) stage(t);
-    int buf = 0;
-    for (int t = 0; t < nsteps; ++t) {
-        // steps behind t that are under way: up to STAGES - 2
-        const int behind = min(STAGES - 2, nsteps - 1 - t);
-        if (behind >= 2) asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)\n\ts_barrier" : : : "memory");
-        else if (behind == 1) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" : : : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
-        if (t + STAGES - 1 < nsteps) stage(buf == 0 ? STAGES - 1 : buf - 1);
-        compute(smem + buf * 2 * GTILE_B, smem + buf * 2 * GTILE_B + GTILE_B);
-        buf = buf + 1 == STAGES ? 0 : buf + 1;
+        buf = buf + 1 == ST ? 0 : buf + 1;
     }
 
     // 32x32 C/D map: col = lane & 31, row = (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5).
     // Row scales are read together (rows past the end repeat the last), not one by one
     // behind a branch each.
-    float as[2][16], bs[2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < FI; ++i) {
+        const int row0 = tm + (wr * FI + i) * 32 + 4 * kh;
+        float as[16];
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-            as[i][r] = ascale[min(tm + wr * 64 + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5), M - 1)];
+        for (int r = 0; r < 16; ++r) as[r] = ascale[min(row0 + (r & 3) + 8 * (r >> 2), M - 1)];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) bs[j] = bscale[min(tn + wc * 64 + j * 32 + (lane & 31), N - 1)];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int col = tn + wc * 64 + j * 32 + (lane & 31);
-        if (col >= N) continue;
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < FJ; ++j) {
+            const int col = tn + (wc * FJ + j) * 32 + fr;
+            if (col >= N) continue;
+            const float bs = bscale[col];
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int row = tm + wr * 64 + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
-                if (row < M) c[(size_t)row * N + col] = f32_to_bf16(accw[i][j][r] * as[i][r] * bs[j]);
+                const int row = row0 + (r & 3) + 8 * (r >> 2);
+                if (row < M) c[(size_t)row * N + col] = f32_to_bf16(acc[i][j][r] * as[r] * bs);
             }
+        }
     }
+}
+
+// Tile by the rounds that the tiles take over 256 CUs, in the time of a step in us (figures
+// above): one block of 128 x 128 a CU 0.62 (0.65 over several rounds, which start and end
+// bare), two of them 1.27 and less where the second ones are few, 128 x 256 1.12, 256 x 256
+// 1.9. It names the fastest for 39 of 40 sizes (12288 x 4096, M = 512: 42.1, 38.2).
+static int gemm_fp8_tile(int64_t M, int64_t N) {
+    const int64_t n1 = CEIL_DIV(M, 128) * CEIL_DIV(N, 128), rest = n1 % 512;
+    const int64_t n2 = CEIL_DIV(M, 128) * CEIL_DIV(N, 256), n3 = CEIL_DIV(M, 256) * CEIL_DIV(N, 256);
+    const double t[4] = {n1 <= 256 ? 0.62 : CEIL_DIV(n1, 256) * 0.65,
+                         n1 / 512 * 1.27 + (rest > 256 ? 0.86 + (rest - 256) * 0.0015 : rest > 0 ? 0.75 : 0.0),
+                         CEIL_DIV(n2, 256) * 1.12, CEIL_DIV(n3, 256) * 1.9};
+    int best = 0;
+    for (int i = 1; i < 4; ++i)
+        if (t[i] < t[best]) best = i;
+    return best;
 }
 
 extern "C" int oa_gemm_fp8(void* stream, const void* a8, const void* b8,
                            const void* ascale, const void* bscale, void* c,
                            int M, int N, int K) {
     if (K % GK2 != 0 || M < 1 || N < 1) return -100;
-    const int mt = CEIL_DIV(M, GT);
-    const int64_t items = (int64_t)CEIL_DIV(N, GT) * mt;
-    if (items > (1 << 28)) return -101;
-    const dim3 grid((unsigned)(CEIL_DIV(items, 8) * 8)), block(256);
-#define RING(STAGES)                                                                              \
-    hipLaunchKernelGGL((gemm_fp8_ring_kernel<STAGES>), grid, block, (STAGES) * 2 * GTILE_B,       \
-                       (hipStream_t)stream, (const uint32_t*)a8, (const uint32_t*)b8,             \
-                       (const float*)ascale, (const float*)bscale, (uint16_t*)c, M, N, K, mt,     \
-                       (int)items)
-    if (items <= 256) RING(4);
-    else RING(2);
-#undef RING
+#define G8(BM, BN, ST, BLOCKS)                                                                     \
+    do {                                                                                           \
+        const int mt = CEIL_DIV(M, BM);                                                            \
+        const int64_t items = (int64_t)CEIL_DIV(N, BN) * mt;                                       \
+        if (items > (1 << 28)) return -101;                                                        \
+        hipLaunchKernelGGL((gemm_fp8_tile_kernel<BM, BN, ST, BLOCKS>),                             \
+                           dim3((unsigned)(CEIL_DIV(items, 8) * 8)), dim3(1024),                   \
+                           (ST) * (BM + BN) * GK2, (hipStream_t)stream, (const char*)a8,           \
+                           (const char*)b8, (const float*)ascale, (const float*)bscale,            \
+                           (uint16_t*)c, M, N, K, mt, (int)items);                                 \
+    } while (0)
+    switch (gemm_fp8_tile(M, N)) {
+        case 0: G8(128, 128, 4, 1); break;
+        case 1: G8(128, 128, 2, 2); break;
+        case 2: G8(128, 256, 3, 1); break;
+        default: G8(256, 256, 2, 1);
+    }
+#undef G8
     HIP_CHECK_LAUNCH();
     return 0;
 }
