@@ -19,13 +19,19 @@
 // 2048 x 8192, M = 8 11.1 / 10.2, 47 14.1 / 12.1; 4096 x 4096, M = 24 11.8 / 10.4, 47 13.5 /
 // 11.7; 3072 x 2048, M = 47 11.6 / 9.1. More rows are bound by what a CU reads of x, which
 // narrow strips double: 32000 x 4096, M = 80 55.2 / 55.4, gate-up 2 x 14336 x 4096, M = 64
-// 48.0 / 49.8, 80 49.3 / 54.1.
+// 48.0 / 49.8, 80 49.3 / 54.1. There eight waves cover each other's waits better than four:
+// gate-up 2 x 14336 x 4096, M = 64 51.1 / 49.7, 77 54.2 / 51.5; 4096 x 14336, 77 30.4 / 29.5, 128
+// 34.1 / 32.4; fp8 28672 x 4096, 128 36.6 / 33.4. Sixteen are no faster, and tiles of 32 rows or
+// narrow strips lose with eight (4096 x 4096 fp8, 8 8.6 / 9.1).
+#include <type_traits>
+
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) float rgf4;
 typedef __attribute__((ext_vector_type(8))) short rgs8;
 typedef __attribute__((ext_vector_type(8))) int rgi8;
 
+#define RG_MG(BM, RN) ((RN) > 64 && (BM) > 32 ? 2 : 1)   // groups of four waves of a block
 #define RG_K 64                         // bf16 columns of a step: 128 bytes; fp8: 128
 
 template <int V>
@@ -41,9 +47,10 @@ __device__ __forceinline__ float rg_gate(float g, float u, int act) {
     return g / (1.0f + __expf(-g)) * u;
 }
 
-// A block of four waves takes BM rows, a strip of RN = 128 or 64 weight rows (GU: half of
-// them gate rows, half the up rows beside them) and one of `splits` runs of 64-column steps;
-// a wave takes all rows by a quarter of the strip on v_mfma_f32_16x16x32_bf16, weights as
+// A block of four waves, or of two such groups with half of the rows each, takes BM rows, a
+// strip of RN = 128 or 64 weight rows (GU: half of them gate rows, half the up rows beside
+// them) and one of `splits` runs of 64-column steps; a wave takes its rows by a quarter of the
+// strip on v_mfma_f32_16x16x32_bf16, weights as
 // the first operand, so that a lane ends with four neighbouring outputs of one row (GU: with
 // gate and up of four outputs in its two fragments; in strips of 64 of two in its one, whose
 // rows go gate, gate, up, up). Both operands come by 16-byte global_load_lds into a ring of
@@ -60,13 +67,14 @@ __device__ __forceinline__ float rg_gate(float g, float u, int act) {
 // 26.9 / 13.2; 4096 x 4096, 77 28.6 / 14.9; 8192 x 28672, 77 140 / 46.8; 2048 x 2816, 33 20.0
 // / 8.7.
 template <int BM, int RN, int STAGES, bool GU, bool NT, bool F8>
-__global__ __launch_bounds__(256, RN > 64 ? 1 : 2) void ring_gemm_kernel(
+__global__ __launch_bounds__(256 * RG_MG(BM, RN), RG_MG(BM, RN) == 2 || RN == 64 ? 2 : 1) void ring_gemm_kernel(
     const char* __restrict__ x, int64_t xs, const char* __restrict__ w,
     const float* __restrict__ xscale, const float* __restrict__ wscale,
     uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int K, int mtiles,
     int splits, int items, int act) {
-    constexpr int MT = BM / 16, NF = RN / 64, WPS = RN / 32;    // fragments, transfers of a wave
-    constexpr int LPS = WPS + BM / 32, STEP = (RN + BM) * 128;
+    constexpr int MG = RG_MG(BM, RN), MT = BM / 16 / MG, NF = RN / 64;   // fragments of a wave
+    constexpr int W = 4 * MG, TR = (RN + BM) / 8, LPS = (TR + W - 1) / W;    // transfers of a step, of a wave
+    constexpr int STEP = (RN + BM) * 128;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int per = gridDim.x >> 3;
     const int item = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
@@ -74,7 +82,9 @@ __global__ __launch_bounds__(256, RN > 64 ? 1 : 2) void ring_gemm_kernel(
     const int strip = item / (splits * mtiles), rest = item - strip * splits * mtiles;
     const int sp = rest / mtiles, m0 = (rest - sp * mtiles) * BM;
     const int lane = threadIdx.x & 63;
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wid = wave & 3, mg = wave >> 2;
+    const bool full = TR % W == 0 || wave < TR % W;  // the last waves have a transfer less
     const int64_t kb = F8 ? K : 2 * (int64_t)K;     // bytes of a weight row
     const int steps = (int)(kb / 128);
     const int s0 = (int)((int64_t)steps * sp / splits), s1 = (int)((int64_t)steps * (sp + 1) / splits);
@@ -85,8 +95,9 @@ __global__ __launch_bounds__(256, RN > 64 ? 1 : 2) void ring_gemm_kernel(
     uint32_t dst[LPS];
 #pragma unroll
     for (int p = 0; p < LPS; ++p) {
-        const bool isw = p < WPS;
-        const int r = (isw ? wid * WPS + p : (p - WPS) * 4 + wid) * 8 + lr;
+        const int tr = p * W + wave;
+        const bool isw = tr < RN / 8;
+        const int r = (isw ? tr : tr - RN / 8) * 8 + lr;
         const int chunk = (lane & 7) ^ (r >> 1 & 7);
         int64_t at;
         if (!isw) at = min(m0 + r, M - 1) * xs * (F8 ? 1 : 2);
@@ -94,16 +105,24 @@ __global__ __launch_bounds__(256, RN > 64 ? 1 : 2) void ring_gemm_kernel(
         else if (GU) at = (min(strip * 32 + (r >> 2) * 2 + (r & 1), N - 1) + (r & 2 ? N : 0)) * kb;
         else at = min(strip * RN + r, N - 1) * kb;
         src[p] = (isw ? w : x) + at + (int64_t)s0 * 128 + chunk * 16;
-        dst[p] = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + (isw ? 0 : RN * 128) +
-                                                (r - lr) * 128);
+        dst[p] = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + tr * 1024);
     }
     auto stage = [&](int buf) {
 #pragma unroll
         for (int p = 0; p < LPS; ++p) {
-            if (NT && p < WPS) lds_transfer16<true>(dst[p] + buf * STEP, src[p]);
+            if (p == LPS - 1 && !full) break;
+            if (NT && p * W + wave < RN / 8) lds_transfer16<true>(dst[p] + buf * STEP, src[p]);
             else lds_transfer16(dst[p] + buf * STEP, src[p]);
             src[p] += 128;
         }
+    };
+    auto wait = [&](auto count, int behind) {         // count: transfers of a step of this wave
+        constexpr int C = decltype(count)::value;
+        if (STAGES > 5 && behind >= 4) rg_wait<4 * C>();
+        else if (STAGES > 4 && behind >= 3) rg_wait<3 * C>();
+        else if (behind == 2) rg_wait<2 * C>();
+        else if (behind == 1) rg_wait<C>();
+        else rg_wait<0>();
     };
     rgf4 acc[NF][MT] = {};
     const int n = s1 - s0;
@@ -113,11 +132,8 @@ __global__ __launch_bounds__(256, RN > 64 ? 1 : 2) void ring_gemm_kernel(
     int buf = 0;
     for (int t = 0; t < n; ++t) {
         const int behind = min(STAGES - 2, n - 1 - t);    // younger steps under way
-        if (STAGES > 5 && behind >= 4) rg_wait<4 * LPS>();
-        else if (STAGES > 4 && behind >= 3) rg_wait<3 * LPS>();
-        else if (behind == 2) rg_wait<2 * LPS>();
-        else if (behind == 1) rg_wait<LPS>();
-        else rg_wait<0>();
+        if (full) wait(std::integral_constant<int, LPS>(), behind);
+        else wait(std::integral_constant<int, LPS - 1>(), behind);
         if (t + STAGES - 1 < n) stage(buf == 0 ? STAGES - 1 : buf - 1);
         const char* b = smem + buf * STEP;
         if constexpr (F8) {
@@ -136,7 +152,7 @@ __global__ __launch_bounds__(256, RN > 64 ? 1 : 2) void ring_gemm_kernel(
 #pragma unroll
             for (int j = 0; j < NF; ++j) wf[j] = frag(b + (wid * NF + j) * 16 * 128);
 #pragma unroll
-            for (int m = 0; m < MT; ++m) xf[m] = frag(b + (RN + m * 16) * 128);
+            for (int m = 0; m < MT; ++m) xf[m] = frag(b + (RN + (mg * MT + m) * 16) * 128);
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -154,7 +170,7 @@ __global__ __launch_bounds__(256, RN > 64 ? 1 : 2) void ring_gemm_kernel(
                     wf[j] = *reinterpret_cast<const rgs8*>(b + (wid * NF + j) * 16 * 128 + at);
 #pragma unroll
                 for (int m = 0; m < MT; ++m)
-                    xf[m] = *reinterpret_cast<const rgs8*>(b + (RN + m * 16) * 128 + at);
+                    xf[m] = *reinterpret_cast<const rgs8*>(b + (RN + (mg * MT + m) * 16) * 128 + at);
 #pragma unroll
                 for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -168,7 +184,7 @@ __global__ __launch_bounds__(256, RN > 64 ? 1 : 2) void ring_gemm_kernel(
     const int q = (lane >> 4) * 4;
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-        const int row = m0 + m * 16 + (lane & 15);
+        const int row = m0 + (mg * MT + m) * 16 + (lane & 15);
         if (row >= M) continue;
         if (GU && NF == 1) {
             const int col = strip * 32 + wid * 8 + q / 2;
@@ -265,10 +281,11 @@ extern "C" int oa_ring_gemm(void* stream, const void* x, int64_t xs, const void*
     const int64_t items = (int64_t)CEIL_DIV(N, (narrow ? 64 : 128) / (gateup ? 2 : 1)) * mtiles * splits;
     if (items > (1 << 28)) return -103;
     hipStream_t s = (hipStream_t)stream;
-    const dim3 grid((unsigned)(CEIL_DIV(items, 8) * 8)), block(256);
+    const dim3 grid((unsigned)(CEIL_DIV(items, 8) * 8));
     float* part = splits > 1 ? (float*)scratch : nullptr;
 #define RG(BMV, RNV, ST, G, NT)                                                                    \
-    hipLaunchKernelGGL((ring_gemm_kernel<BMV, RNV, ST, G, NT, false>), grid, block,                 \
+    hipLaunchKernelGGL((ring_gemm_kernel<BMV, RNV, ST, G, NT, false>), grid,                        \
+                       dim3(256 * RG_MG(BMV, RNV)),                                                 \
                        (ST) * ((RNV) + (BMV)) * 128, s, (const char*)x, xs, (const char*)w,         \
                        (const float*)nullptr, (const float*)nullptr, (uint16_t*)out, part, M, N, K, \
                        mtiles, splits, (int)items, act)
@@ -296,11 +313,11 @@ extern "C" int oa_ring_gemm(void* stream, const void* x, int64_t xs, const void*
     if (splits > 1) {
         const dim3 g(CEIL_DIV(N / 4, 256), M);
         if (gateup)
-            hipLaunchKernelGGL((ring_sum_kernel<true, false>), g, block, 0, s, part,
+            hipLaunchKernelGGL((ring_sum_kernel<true, false>), g, dim3(256), 0, s, part,
                                (const float*)nullptr, (const float*)nullptr, (uint16_t*)out, M, N,
                                splits, act);
         else
-            hipLaunchKernelGGL((ring_sum_kernel<false, false>), g, block, 0, s, part,
+            hipLaunchKernelGGL((ring_sum_kernel<false, false>), g, dim3(256), 0, s, part,
                                (const float*)nullptr, (const float*)nullptr, (uint16_t*)out, M, N,
                                splits, 0);
     }
@@ -324,7 +341,7 @@ extern "C" int oa_ring_gemm_fp8(void* stream, const void* x8, const void* xscale
     float* part = splits > 1 ? (float*)scratch : nullptr;
 #define RG8(BMV, ST, NT)                                                                           \
     hipLaunchKernelGGL((ring_gemm_kernel<BMV, 128, ST, false, NT, true>),                               \
-                       dim3((unsigned)(CEIL_DIV(items, 8) * 8)), dim3(256),                        \
+                       dim3((unsigned)(CEIL_DIV(items, 8) * 8)), dim3(256 * RG_MG(BMV, 128)),      \
                        (ST) * (128 + (BMV)) * 128, s, (const char*)x8, (int64_t)K, (const char*)w8, \
                        (const float*)xscale, (const float*)wscale, (uint16_t*)out, part, M, N, K,  \
                        mtiles, splits, (int)items, 0)
