@@ -124,10 +124,10 @@ class Attention(nn.Module):
             return ops.linear_fp8(x, self.qkv_q, self.qkv_s)
         return ops.linear(x, self.qkv_w)
 
-    def _o(self, x: torch.Tensor) -> torch.Tensor:
+    def _o(self, x: torch.Tensor, parts: bool = False) -> torch.Tensor:
         if self.fp8:
             return ops.linear_fp8(x, self.o_q, self.o_s)
-        return ops.linear(x, self.o_w)
+        return (ops.linear_parts if parts else ops.linear)(x, self.o_w)
 
     def forward(
         self,
@@ -137,6 +137,7 @@ class Attention(nn.Module):
         k_cache: torch.Tensor,
         v_cache: torch.Tensor,
         fb: ForwardBatch,
+        parts: bool = False,      # the output may be a product's parts (ops.linear_parts)
     ) -> torch.Tensor:
         T = x.shape[0]
         qkv = self._qkv(x)  # hipBLASLt / HIP gemv / fp8 at decode
@@ -157,7 +158,7 @@ class Attention(nn.Module):
                 cos, sin, fb.slot_mapping, scale=self.scale,
                 workspace=fb.decode_workspace, nsplit=fb.nsplit,
             ).view(T, self.hq * self.hd)
-            out = self._o(out)
+            out = self._o(out, parts)
             return tp_all_reduce(out)
         q, k, v = ops.rope_kv_fused(
             q, k, v, k_cache, v_cache, cos, sin, fb.positions, fb.slot_mapping
@@ -190,7 +191,7 @@ class Attention(nn.Module):
                 nsplit=fb.nsplit,
             )
             out = out.view(T, self.hq * self.hd)
-        out = self._o(out)
+        out = self._o(out, parts)
         return tp_all_reduce(out)
 
 
@@ -211,13 +212,13 @@ class DenseMLP(nn.Module):
         self.down_w = nn.Parameter(_shard(down, 1, rank, tp), requires_grad=False)
         self.fp8 = False  # set by LlamaForCausalLM.quantize_fp8_
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, parts: bool = False) -> torch.Tensor:
         if self.fp8:
             return tp_all_reduce(ops.mlp_fp8(
                 x, self.gate_up_q, self.gate_up_s, self.i_local, self.down_q, self.down_s
             ))
         act = ops.gateup_silu(x, self.gate_up_w, self.i_local)
-        return tp_all_reduce(ops.linear(act, self.down_w))
+        return tp_all_reduce((ops.linear_parts if parts else ops.linear)(act, self.down_w))
 
 
 class DecoderLayer(nn.Module):
@@ -245,12 +246,14 @@ class DecoderLayer(nn.Module):
             h = ops.rms_norm(x, self.input_norm_w, self.eps)
         else:
             h, residual = ops.fused_add_rms_norm(x, residual, self.input_norm_w, self.eps)
-        a = self.attn(h, cos, sin, k_cache, v_cache, fb)
+        # the norm after a sublayer adds up its last product's parts (not what ranks add up)
+        parts = get_tp_size() == 1
+        a = self.attn(h, cos, sin, k_cache, v_cache, fb, parts)
         h, residual = ops.fused_add_rms_norm(a, residual, self.post_norm_w, self.eps)
         if self.is_moe_layer:
             m = self.mlp(h, decode=fb.kind == "decode")
         else:
-            m = self.mlp(h)
+            m = self.mlp(h, parts)
         return m, residual
 
     def fused_decode(self, residual, cos, sin, k_cache, v_cache, fb):

@@ -322,21 +322,36 @@ def _ring_choice(M: int, N: int, K: int, gateup: bool = False):
     return wide and (*wide, False)
 
 
-def _ring(x: torch.Tensor, w: torch.Tensor, plan: Tuple[int, ...], act: int = 0) -> torch.Tensor:
+def _ring(x: torch.Tensor, w: torch.Tensor, plan: Tuple[int, ...], act: int = 0,
+          parts: bool = False) -> torch.Tensor:
     """x @ w^T, or act 1 (silu), 2 (tanh gelu) of the gate rows times the up rows. plan: (rows
-    of a tile, column splits), and whether in strips of 64 weight rows."""
+    of a tile, column splits), and whether in strips of 64 weight rows. parts: the float32
+    parts of a split product [splits, M, N], not added up."""
     lib, hip = _lib()
     K, (tile, splits), narrow = x.shape[-1], plan[:2], len(plan) > 2 and plan[2]
     M, N = x.numel() // K, w.shape[0] // (2 if act else 1)
-    out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
+    out = None if parts else torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
     # at most 256 tiles of 128 x 128 float32 (gate and up): 17 MB
-    part = None if splits == 1 else torch.empty(splits * M * w.shape[0], dtype=torch.float32,
+    part = None if splits == 1 else torch.empty(splits, M, w.shape[0], dtype=torch.float32,
                                                 device=x.device)
     hip.check(lib.oa_ring_gemm(hip.current_stream_ptr(), x.data_ptr(),
                                K if x.is_contiguous() else x.stride(0), w.data_ptr(),
-                               out.data_ptr(), None if part is None else part.data_ptr(),
+                               None if parts else out.data_ptr(),
+                               None if part is None else part.data_ptr(),
                                M, N, K, tile, int(narrow), splits, act), "oa_ring_gemm")
-    return out
+    return part if parts else out
+
+
+def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ w^T for rows x [T, K] that go through fused_add_rms_norm next: bf16 [T, N], or the
+    product's float32 column parts [parts, T, N], which the norm adds up, where the transfer
+    ring splits it."""
+    M = x.numel() // x.shape[-1]
+    if 1 < M <= 128 and x.dim() == 2 and w.shape[0] <= 8192 and _skinny_ok(x, w):
+        plan = _ring_choice(M, w.shape[0], w.shape[1])
+        if plan and plan[1] > 1:
+            return _ring(x, w, plan, parts=True)
+    return linear(x, w)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -408,9 +423,19 @@ def fused_add_rms_norm(
     x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     """Returns (rmsnorm(x+residual), x+residual). GPU path updates `residual`
-    in place as the new residual stream and returns it."""
+    in place as the new residual stream and returns it. x may be the parts of a
+    product (linear_parts)."""
     if not _is_gpu(x):
         return torch_ref.fused_add_rms_norm(x, residual, weight, eps)
+    if x.dim() == 3 and x.dtype == torch.float32:
+        parts, rows, dim = x.shape
+        assert x.is_contiguous() and residual.is_contiguous() and residual.shape == (rows, dim)
+        lib, hip = _lib()
+        out = torch.empty_like(residual)
+        hip.check(lib.oa_add_rmsnorm_parts(
+            hip.current_stream_ptr(), x.data_ptr(), parts, residual.data_ptr(),
+            weight.data_ptr(), out.data_ptr(), rows, dim, eps), "oa_add_rmsnorm_parts")
+        return out, residual
     assert x.dtype == torch.bfloat16 and x.is_contiguous() and residual.is_contiguous()
     lib, hip = _lib()
     rows = x.numel() // x.shape[-1]

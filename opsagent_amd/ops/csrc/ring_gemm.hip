@@ -267,12 +267,13 @@ __global__ __launch_bounds__(256) void ring_sum_kernel(const float* __restrict__
 // out [M, N] = x [M, K] w [N, K]^T, x rows xs elements apart. act 1 (silu), 2 (tanh gelu):
 // out = act(x w[:N]^T) * (x w[N:]^T), w [2 N, K]. bm: rows of a tile, 32, 64, 96 or 128;
 // narrow: strips of 64 weight rows (bm 32 and 64).
-// scratch: splits * M * N floats (act: twice that), unused at splits 1.
+// scratch: splits * M * N floats (act: twice that), unused at splits 1; out null: left
+// there, not added up.
 extern "C" int oa_ring_gemm(void* stream, const void* x, int64_t xs, const void* w, void* out,
                             void* scratch, int M, int N, int K, int bm, int narrow, int splits,
                             int act) {
     if (M < 1 || M > 65535 || N < 4 || N % 4 != 0 || K < RG_K || K % RG_K != 0) return -100;
-    if (splits < 1 || splits > K / RG_K || (splits > 1 && !scratch)) return -101;
+    if (splits < 1 || splits > K / RG_K || (splits > 1 ? !scratch : !out)) return -101;
     if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)scratch) % 16 != 0 || xs % 8 != 0)
         return -102;
     if (act < 0 || act > 2 || (bm != 32 && bm != 64 && bm != 96 && bm != 128) || (narrow && bm > 64)) return -104;
@@ -310,7 +311,7 @@ extern "C" int oa_ring_gemm(void* stream, const void* x, int64_t xs, const void*
     else RGB(128, 128, 4, false);
 #undef RGB
 #undef RG
-    if (splits > 1) {
+    if (splits > 1 && out) {
         const dim3 g(CEIL_DIV(N / 4, 256), M);
         if (gateup)
             hipLaunchKernelGGL((ring_sum_kernel<true, false>), g, dim3(256), 0, s, part,

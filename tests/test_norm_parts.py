@@ -1,0 +1,49 @@
+"""A norm that adds up the parts of the product before it, against the product by itself and
+the norm: one plane and many, widths of one wave to two rounds of a block."""
+
+import pytest
+import torch
+
+from opsagent_amd import ops
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("parts,T,D", [(1, 3, 64), (2, 1, 8), (3, 2, 1000), (8, 5, 4096), (16, 2, 4104),
+                                       (5, 3, 8192)])
+def test_planes(parts, T, D):
+    g = torch.Generator(device="cuda").manual_seed(D)
+    x = torch.randn(parts, T, D, generator=g, device="cuda")
+    residual = torch.randn(T, D, generator=g, device="cuda").bfloat16()
+    w = (1 + 0.1 * torch.randn(D, generator=g, device="cuda")).bfloat16()
+    total = x[0].clone()
+    for s in range(1, parts):
+        total += x[s]
+    want, want_r = ops.fused_add_rms_norm(total.bfloat16(), residual.clone(), w, 1e-5)
+    got, got_r = ops.fused_add_rms_norm(x, residual, w, 1e-5)
+    assert got_r.data_ptr() == residual.data_ptr() and torch.equal(got_r, want_r)
+    # the sum of squares in another order: a result may round to the neighbour
+    assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -7, atol=0)
+    assert (got != want).float().mean() < 0.01
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,N,K", [(8, 4096, 14336), (64, 4096, 4096), (77, 4096, 4096), (24, 2048, 8192),
+                                   (3, 2048, 2048), (200, 4096, 4096), (1, 4096, 4096)])
+def test_products(T, N, K):
+    g = torch.Generator(device="cuda").manual_seed(T + K)
+    x = torch.randn(T, K, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).bfloat16()
+    y = ops.linear_parts(x, w)
+    plan = 1 < T <= 128 and ops._ring_choice(T, N, K)
+    assert (y.dim() == 3) == bool(plan and plan[1] > 1)
+    if y.dim() == 3:
+        total = y[0].clone()
+        for s in range(1, y.shape[0]):
+            total += y[s]
+        y = total.bfloat16()
+    assert torch.equal(y, ops.linear(x, w))
+
+
+def test_cpu_is_linear():
+    x, w = torch.randn(8, 4096).bfloat16(), torch.randn(64, 4096).bfloat16()
+    assert torch.equal(ops.linear_parts(x, w), ops.linear(x, w))
