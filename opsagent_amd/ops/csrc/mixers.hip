@@ -928,6 +928,247 @@ __global__ __launch_bounds__(256) void attn_bias_mfma_kernel(
     }
 }
 
+// ---------------------------------------------------------------------------
+// Decode steps (one new token per sequence) of heads of D = Dv = 64, 128 or
+// 256 channels, bf16, fewer than 16 query heads per kv head. The tile kernel
+// above spends such a step on its tile: 16 token columns of which one is in
+// use, the values turned around through LDS, two barriers per 64 keys, and few
+// blocks to hide any of it. Here a wave works alone on pieces of TK keys
+// (up to 8 KB of K and of V) and takes both straight into registers: the next
+// piece's keys are asked for when the scores of this one are done, its values
+// when this one's are added up. The eight waves of a block meet once, at the
+// end.
+//   S^T = K Q^T on the matrix cores, as above, with the block's HB heads in
+//   the columns (the other columns repeat the last); the weights go through
+//   the wave's own LDS rows to the lanes that hold the values, D/8 lanes per
+//   key, and enter the sums as float32.
+// What bounds it: with few blocks the chain of loads (past, page, keys) and the
+// merge, beyond them the reads, at one block of eight waves a CU (220 registers
+// a lane at D = 128, HB = 4). us a call, tile kernel with its splits -> here:
+// one row, window 512, 4 kv heads of 4: 13.1 -> 8.4; contexts 1030, 340, 84,
+// 8 kv heads of 4: 17.3 -> 11.1; 64 rows of 500 to 3650: 305 -> 122 (4.5 TB/s);
+// one of 16000: 81 -> 25.5; four of 40: 8.7 -> 4.6. With the page looked up key
+// by key in each piece the last but one took 24.6 in the same splits, but the
+// 64 rows 143 and one block going through 16000 keys 214 instead of 174.
+constexpr int rows_piece(int D) { return D == 256 ? 16 : 32; }
+
+template <int D, int HB>
+__global__ __launch_bounds__(512) void attn_rows_kernel(
+    const bf16s* __restrict__ q, const bf16s* __restrict__ gate, int64_t gs,
+    const bf16s* __restrict__ k_cache, const bf16s* __restrict__ v_cache,
+    bf16s* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
+    const int* __restrict__ cu, const int* __restrict__ past,
+    const int* __restrict__ block_table, int max_blocks, int block_size,
+    const float* __restrict__ slopes, const float* __restrict__ sinks, int B, int H, int G,
+    float scale, int nsplit, int window, int64_t vrow, int Gv, float softcap, int64_t os,
+    float oscale, int keep, int gch) {
+    constexpr int NW = 8, KS = D / 32, TK = rows_piece(D), MT = TK / 16;
+    constexpr int VL = D / 8, KP = 64 / VL, NV = TK / KP;
+    __shared__ __align__(16) float ps[NW][TK * HB];
+    __shared__ __align__(16) float sums[NW][HB * D];
+    __shared__ float ml[NW][HB][2];
+    const int R = H / G, hgroups = R / HB;
+    const int g = blockIdx.y / hgroups, h0 = g * R + (blockIdx.y % hgroups) * HB;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lc = lane & 15, lg = lane >> 4;
+    const int split = blockIdx.z;
+    // the block's sequence: the blockIdx.x-th that brings a token
+    // (at most one each, so t tokens before sequence t make it that one)
+    int b = blockIdx.x, lo = cu[b], pos = past[b];
+    if (lo != b || cu[b + 1] == lo) {
+        b = 0;
+        for (int t = blockIdx.x; b < B; ++b) {
+            lo = cu[b];
+            const int n = cu[b + 1] - lo;
+            if (t < n) break;
+            t -= n;
+        }
+        if (b >= B) return;
+        pos = past[b];
+    }
+    const int* bt = block_table + (int64_t)b * max_blocks;
+    const float LOG2E = 1.4426950408889634f;
+    const int h = h0 + min(lc, HB - 1);
+    const float slope = slopes ? slopes[h] * LOG2E : 0.0f;
+    const float scale2 = scale * LOG2E;
+    const float cap_in = softcap > 0.0f ? 2.0f * scale * LOG2E / softcap : 0.0f;
+    const float cap_out = softcap * LOG2E;
+    const int wlim = window > 0 ? window : 0x7fffffff;
+    const int bsh = 31 - __clz(block_size), bmask = block_size - 1;
+
+    s8_t qf[KS], kf[MT][KS];
+    uint4 vf[NV];
+    const bf16s* qr = q + ((int64_t)lo * H + h) * D + 8 * lg;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const s8_t*>(qr + 32 * ks);
+    // A piece lies within one page if pages are no smaller: its page is then a
+    // value of the whole wave, and the wave looks 64 of its pieces up at once
+    const KeyTiles tiles = key_tiles(pos, pos / TK + 1, TK, window, keep);
+    const int step = nsplit * NW, first = split + nsplit * wave;
+    const bool whole = block_size >= TK;
+    int pages = 0;
+    auto look_up = [&](int it) {
+        const int mine = it + step * lane;
+        pages = mine < tiles.count ? bt[tiles.at(mine) * TK >> bsh] : 0;
+    };
+    // the piece's first slot (whole pages); keys past the last one repeat it and count for nothing
+    auto base = [&](int n, int k0) {
+        return ((int64_t)__builtin_amdgcn_readlane(pages, n & 63) << bsh) + (k0 & bmask);
+    };
+    auto slot = [&](int64_t base, int k0, int i) {
+        const int key = min(k0 + i, pos);
+        return whole ? base + (key - k0) : ((int64_t)bt[key >> bsh] << bsh) + (key & bmask);
+    };
+    auto fetch_k = [&](int64_t base, int k0) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const bf16s* kp = k_cache + (slot(base, k0, 16 * mt + lc) * G + g) * D + 8 * lg;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                kf[mt][ks] = *reinterpret_cast<const s8_t*>(kp + 32 * ks);
+        }
+    };
+    const bf16s* vbase = v_cache + (g % Gv) * D + 8 * (lane % VL);
+    auto fetch_v = [&](int64_t base, int k0) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+            vf[i] = *reinterpret_cast<const uint4*>(vbase + slot(base, k0, KP * i + lane / VL) * vrow);
+    };
+    float acc[HB][8], m = -INFINITY, l = 0.0f;
+#pragma unroll
+    for (int j = 0; j < HB; ++j)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) acc[j][c] = 0.0f;
+
+    int n = 0;                               // pieces done
+    int64_t at = 0;
+    if (first < tiles.count) {
+        if (whole) look_up(first);
+        const int k0 = tiles.at(first) * TK;
+        at = base(0, k0);
+        fetch_k(at, k0);
+        fetch_v(at, k0);
+    }
+    for (int it = first; it < tiles.count; it += step) {
+        const int k0 = tiles.at(it) * TK;
+        const bool more = it + step < tiles.count;
+        const int k1 = more ? tiles.at(it + step) * TK : 0;
+        if (more) {
+            if (whole && (++n & 63) == 0) look_up(it + step);
+            at = base(n, k1);
+        }
+        f4_t sc[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            sc[mt] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                sc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[mt][ks], qf[ks], sc[mt], 0, 0, 0);
+        }
+        if (more) fetch_k(at, k1);
+        float mloc = -INFINITY;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int key = k0 + 16 * mt + 4 * lg + r;
+                const float bias = slope * (float)(key - pos);
+                float v;
+                if (softcap > 0.0f) {
+                    const float e2 = __builtin_amdgcn_exp2f(sc[mt][r] * cap_in);
+                    v = cap_out - 2.0f * cap_out * __builtin_amdgcn_rcpf(e2 + 1.0f) + bias;
+                } else {
+                    v = fmaf(sc[mt][r], scale2, bias);
+                }
+                v = (key <= pos && (key > pos - wlim || key < keep)) ? v : -INFINITY;
+                sc[mt][r] = v;
+                mloc = fmaxf(mloc, v);
+            }
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 16, WAVE));
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 32, WAVE));
+        const float mnew = fmaxf(m, mloc);
+        const float msub = (mnew == -INFINITY) ? 0.0f : mnew;   // no key yet: keep off NaN
+        const float corr = __builtin_amdgcn_exp2f(m - msub);
+        m = mnew;
+        l *= corr;                                               // a lane's own keys; summed at the end
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float p = __builtin_amdgcn_exp2f(sc[mt][r] - msub);
+                l += p;
+                if (lc < HB) ps[wave][(16 * mt + 4 * lg + r) * HB + lc] = p;
+            }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < HB; ++j) {
+            const float cj = __shfl(corr, j, WAVE);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) acc[j][c] *= cj;
+        }
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            float p[HB];
+#pragma unroll
+            for (int j = 0; j < HB; ++j) p[j] = ps[wave][(KP * i + lane / VL) * HB + j];
+            const uint32_t w[4] = {vf[i].x, vf[i].y, vf[i].z, vf[i].w};
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const float v = __uint_as_float(c % 2 ? w[c / 2] & 0xffff0000u : w[c / 2] << 16);
+#pragma unroll
+                for (int j = 0; j < HB; ++j) acc[j][c] = fmaf(p[j], v, acc[j][c]);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (more) fetch_v(at, k1);
+    }
+    l += __shfl_xor(l, 16, WAVE);
+    l += __shfl_xor(l, 32, WAVE);
+    if (lane < HB) {
+        ml[wave][lane][0] = m;
+        ml[wave][lane][1] = l;
+    }
+#pragma unroll
+    for (int j = 0; j < HB; ++j) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int x = VL; x < 64; x <<= 1) acc[j][c] += __shfl_xor(acc[j][c], x, WAVE);
+        if (lane < VL) {
+            float* row = &sums[wave][j * D + 8 * lane];
+            *reinterpret_cast<f4_t*>(row) = f4_t{acc[j][0], acc[j][1], acc[j][2], acc[j][3]};
+            *reinterpret_cast<f4_t*>(row + 4) = f4_t{acc[j][4], acc[j][5], acc[j][6], acc[j][7]};
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < HB * D; i += 512) {
+        const int j = i / D, ch = i % D, hj = h0 + j;
+        float mx = -INFINITY, lt = 0.0f, v = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) mx = fmaxf(mx, ml[w][j][0]);
+        const float msub = (mx == -INFINITY) ? 0.0f : mx;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float wt = __builtin_amdgcn_exp2f(ml[w][j][0] - msub);
+            lt = fmaf(ml[w][j][1], wt, lt);
+            v = fmaf(sums[w][i], wt, v);
+        }
+        if (nsplit == 1) {
+            if (sinks) lt += __builtin_amdgcn_exp2f(sinks[hj] * LOG2E - mx);
+            v *= (gate && !gch ? sigmoidf_(ldf(gate, (int64_t)lo * gs + hj)) : 1.0f) * oscale / lt;
+            if (gate && gch) v *= sigmoidf_(ldf(gate, (int64_t)lo * gs + hj * D + ch));
+            stf(out, (int64_t)lo * os + hj * D + ch, v);
+        } else {
+            const int64_t pr = ((int64_t)lo * H + hj) * nsplit + split;
+            part_o[pr * D + ch] = v;
+            if (ch == 0) {
+                part_ml[pr * 2] = mx * 0.6931471805599453f;     // back to the natural-log domain
+                part_ml[pr * 2 + 1] = lt;
+            }
+        }
+    }
+}
+
 // merge key-split partials: one block per (token, head). Every wave first
 // takes the statistics of all splits, a lane each; then wave w adds up the
 // splits w, w + 4, ..., a lane per value channel, and the waves' sums meet in LDS
@@ -1856,6 +2097,40 @@ static void launch_attn_mfma(hipStream_t s, dim3 grid, int lds_bytes, const void
                        scale, nsplit, window, (int)vrow, hrows, Gv, softcap, os, oscale, keep, gch);
 }
 
+// Whether a decode step takes attn_rows_kernel.
+static bool attn_rows(int H, int G, int D, int Dv, int dt, int max_chunk) {
+    return attn_path(H, G, D, Dv, dt) && max_chunk == 1 && H / G < 16 && D == Dv &&
+           (D == 64 || D == 128 || D == 256);
+}
+
+// Key splits of a decode step whose longest context is `reach` keys, or 0 if
+// attn_rows_kernel does not take it. Eight waves go through up to 16 pieces
+// faster than a second launch could merge them. Beyond, splits fill the 256
+// CUs: with fewer heads a block where that leaves no wave more than one piece,
+// else with every head that shares the keys (one row of 16000 keys, 8 kv heads
+// of 4: 25.0 us in 32 splits of four heads, 29.8 in 16 of two, 49.5 in 8 of
+// one; 2000 keys, 4 kv heads: 12.1 in 16 of four, 9.3 in 16 of one).
+extern "C" int oa_attn_rows_splits(int H, int G, int D, int Dv, int dt, int max_chunk, int ntiles,
+                                   int reach) {
+    if (G < 1 || H % G != 0 || ntiles < 1 || !attn_rows(H, G, D, Dv, dt, max_chunk)) return 0;
+    const int pieces = CEIL_DIV(std::max(reach, 1), rows_piece(D));
+    if (pieces <= 16) return 1;
+    const int R = H / G, HB = attn_hb(R);
+    for (int hb = 1; hb <= HB; hb *= 2) {
+        const int n = std::min(std::min(256 / (ntiles * G * (R / hb)), 16), pieces / 2);
+        if (n >= 4 && n * 8 >= pieces) return n;
+    }
+    return std::max(1, std::min(256 / (ntiles * G * (R / HB)),
+                                std::max(16, std::min(pieces / 8, 64))));
+}
+
+template <int HB, typename... A>
+static void launch_attn_rows(int D, dim3 grid, hipStream_t s, A... a) {
+    if (D == 64) hipLaunchKernelGGL((attn_rows_kernel<64, HB>), grid, dim3(512), 0, s, a...);
+    else if (D == 128) hipLaunchKernelGGL((attn_rows_kernel<128, HB>), grid, dim3(512), 0, s, a...);
+    else hipLaunchKernelGGL((attn_rows_kernel<256, HB>), grid, dim3(512), 0, s, a...);
+}
+
 // ntiles = sum_b ceil(n_b / TQ) (host-computed). part_* may be null when nsplit == 1.
 extern "C" int oa_attn_bias_paged(void* stream, const void* q, const void* gate, int64_t gs,
                                   const void* k_cache, const void* v_cache, void* out,
@@ -1887,10 +2162,26 @@ extern "C" int oa_attn_bias_paged(void* stream, const void* q, const void* gate,
         if (os % 4 != 0 || (uintptr_t)out % 8 != 0) return -108;   // 8-byte output stores
         if (gate && gch && (gs % 4 != 0 || (uintptr_t)gate % 8 != 0)) return -110;   // and gate loads
         const int R = H / G, HB = attn_hb(R);
-        // decode steps of 16 or more query heads per kv head put the heads
-        // in the tile's columns
-        const int hrows = (max_chunk == 1 && R >= 16) ? 1 : 0;
-        dim3 grid(ntiles, hrows ? G * CEIL_DIV(R, 64) : G * (R / HB), nsplit);
+        if (attn_rows(H, G, D, Dv, dt, max_chunk)) {
+            // CUs left over: fewer heads a block, though keys are then read more than once
+            int hb = HB;
+            while (hb > 1 && ntiles * G * (R / hb) * nsplit * 2 <= 256) hb /= 2;
+            dim3 grid(ntiles, G * (R / hb), nsplit);
+#define ROW_ARGS                                                                                  \
+    D, grid, s, (const bf16s*)q, (const bf16s*)gate, gs, (const bf16s*)k_cache,                   \
+        (const bf16s*)v_cache, (bf16s*)out, (float*)part_o, (float*)part_ml, (const int*)cu,      \
+        (const int*)past, (const int*)block_table, max_blocks, block_size, (const float*)slopes,  \
+        (const float*)sinks, B, H, G, scale, nsplit, window, vrow, Gv, softcap, os, oscale, keep, gch
+            if (hb == 4) launch_attn_rows<4>(ROW_ARGS);
+            else if (hb == 2) launch_attn_rows<2>(ROW_ARGS);
+            else launch_attn_rows<1>(ROW_ARGS);
+#undef ROW_ARGS
+            HIP_CHECK_LAUNCH();
+        } else {
+            // decode steps of 16 or more query heads per kv head put the heads
+            // in the tile's columns
+            const int hrows = (max_chunk == 1 && R >= 16) ? 1 : 0;
+            dim3 grid(ntiles, hrows ? G * CEIL_DIV(R, 64) : G * (R / HB), nsplit);
 #define MF_ARGS                                                                                   \
     s, grid, lds_bytes, q, gate, gs, k_cache, v_cache, out, part_o, part_ml, cu, past, block_table, \
         max_blocks, block_size, slopes, sinks, B, H, G, D, Dv, HB, scale, nsplit, window, vrow, hrows, \
@@ -1900,19 +2191,20 @@ extern "C" int oa_attn_bias_paged(void* stream, const void* q, const void* gate,
         if (D % 32 == 0) launch_attn_mfma<A, Bv, true, 1>(MF_ARGS);             \
         else launch_attn_mfma<A, Bv, false, 1>(MF_ARGS);                        \
     } while (0)
-        const int a = D <= 64 ? 4 : (D <= 128 ? 8 : 16), bv = Dv <= 64 ? 4 : (Dv <= 128 ? 8 : 16);
-        if (a == 4 && bv == 4) MF(4, 4);
-        else if (a == 4 && bv == 8) MF(4, 8);
-        else if (a == 4) MF(4, 16);
-        else if (a == 8 && bv == 4) MF(8, 4);
-        else if (a == 8 && bv == 8) MF(8, 8);
-        else if (a == 8) MF(8, 16);
-        else if (bv == 4) launch_attn_mfma<16, 4, true, 1>(MF_ARGS);
-        else if (bv == 8) launch_attn_mfma<16, 8, true, 1>(MF_ARGS);
-        else launch_attn_mfma<16, 16, true, 1>(MF_ARGS);
+            const int a = D <= 64 ? 4 : (D <= 128 ? 8 : 16), bv = Dv <= 64 ? 4 : (Dv <= 128 ? 8 : 16);
+            if (a == 4 && bv == 4) MF(4, 4);
+            else if (a == 4 && bv == 8) MF(4, 8);
+            else if (a == 4) MF(4, 16);
+            else if (a == 8 && bv == 4) MF(8, 4);
+            else if (a == 8 && bv == 8) MF(8, 8);
+            else if (a == 8) MF(8, 16);
+            else if (bv == 4) launch_attn_mfma<16, 4, true, 1>(MF_ARGS);
+            else if (bv == 8) launch_attn_mfma<16, 8, true, 1>(MF_ARGS);
+            else launch_attn_mfma<16, 16, true, 1>(MF_ARGS);
 #undef MF
 #undef MF_ARGS
-        HIP_CHECK_LAUNCH();
+            HIP_CHECK_LAUNCH();
+        }
     } else {
         const int rb = std::min(H / G, 4 * ATT_MAXR);
         dim3 grid(ntiles, G * CEIL_DIV(H / G, rb), nsplit), blk(256);

@@ -319,6 +319,8 @@ def attention_paged(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             nsplit = int(min(nkt // 2, max(1, 256 // blocks), 16))
             if os.environ.get("OPSAGENT_ATTN_DECODE_SPLITS"):
                 nsplit = max(1, min(nkt, int(os.environ["OPSAGENT_ATTN_DECODE_SPLITS"])))
+    # decode steps of fewer heads have a kernel, and a rule, of their own
+    nsplit = lib.oa_attn_rows_splits(H, G, D, Dv, dt, sb.max_chunk, ntiles, reach) or nsplit
     if out is None:
         out = torch.empty(T, H * Dv, dtype=q.dtype, device=q.device)
     assert out.shape == (T, H * Dv) and out.dtype == q.dtype

@@ -1,0 +1,111 @@
+"""Decode attention with the keys and values in registers (attn_rows_kernel) against 64 bits:
+contexts around a piece, a page and a round of eight waves, pages smaller than a piece, every
+option of the call, split and whole. The rule of the splits is checked by itself."""
+
+import ctypes
+import os
+
+import pytest
+import torch
+
+from opsagent_amd.ops import mixer_ops as mx
+
+LIB = os.path.join(os.path.dirname(mx.__file__), "libopsagent_mixers.so")
+
+
+@pytest.mark.skipif(not os.path.exists(LIB), reason="mixers .so not built")
+def test_splits():
+    splits = ctypes.CDLL(LIB).oa_attn_rows_splits
+    assert splits(16, 1, 128, 128, 0, 1, 1, 4000) == 0      # 16 heads a kv head: columns of a tile
+    assert splits(8, 2, 128, 64, 0, 1, 1, 4000) == 0        # value heads of another size
+    assert splits(8, 2, 96, 96, 0, 1, 1, 4000) == 0
+    assert splits(8, 2, 128, 128, 1, 1, 1, 4000) == 0       # float32
+    assert splits(8, 2, 128, 128, 0, 2, 1, 4000) == 0       # not a decode step
+    for H, G in ((1, 1), (15, 1), (12, 2), (14, 2), (32, 8), (64, 64)):
+        hb = 4 if H // G % 4 == 0 else (2 if H // G % 2 == 0 else 1)
+        for D in (64, 128, 256):
+            for rows in (1, 3, 16, 300):
+                for reach in (1, 256, 512, 513, 2000, 100000):
+                    n = splits(H, G, D, D, 0, 1, rows, reach)
+                    assert 1 <= n <= 64
+                    assert n == 1 or rows * H // hb * n <= 256
+                    assert n == 1 or reach > 16 * (16 if D == 256 else 32)
+
+
+def _exact(q, k, v, table, past, page, scale, slopes, gate, window, sinks, softcap, keep, channels):
+    """(result, largest score magnitude) in 64 bits; k, v [pages, page, heads, D]"""
+    T, H, D = q.shape
+    G, Gv, out, big = k.shape[2], v.shape[2], [], 0.0
+    for t in range(T):
+        pos = torch.arange(past[t] + 1)
+        at = torch.tensor(table[t])[pos // page], pos % page
+        kt = k[at].double().repeat_interleave(H // G, 1)
+        vt = v[at].double()[:, torch.arange(G) % Gv].repeat_interleave(H // G, 1)
+        s = torch.einsum("hd,nhd->hn", q[t].double(), kt) * scale
+        big = max(big, float(torch.einsum("hd,nhd->hn", q[t].double().abs(), kt.abs()).max()) * scale)
+        if softcap:
+            s = softcap * torch.tanh(s / softcap)
+        if slopes is not None:
+            s = s - slopes.double()[:, None] * (past[t] - pos)
+        if window:
+            s[:, (past[t] - pos >= window) & (pos >= keep)] = -float("inf")
+        norm = torch.logsumexp(s, 1)
+        if sinks is not None:
+            norm = torch.logaddexp(norm, sinks.double())
+        o = torch.einsum("hn,nhd->hd", torch.exp(s - norm[:, None]), vt)
+        if gate is not None:
+            o = o * torch.sigmoid(gate[t].double().view(H, -1))
+        out.append(o.reshape(-1))
+    return torch.stack(out), big
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [None, 1, 3])
+@pytest.mark.parametrize("ctx,H,G,D,page,opts", [
+    ([1, 32, 33, 64, 513], 32, 8, 128, 32, dict(slopes=True, gate="heads")),
+    ([257, 16, 700], 6, 2, 128, 8, dict(sinks=True)),                     # pages below a piece
+    ([2005, 511], 16, 4, 128, 32, dict(window=512, sinks=True)),
+    ([31, 300, 1], 12, 2, 64, 16, dict(window=40, keep=5, gate="channels", softcap=20.0)),
+    ([129, 1030], 4, 4, 64, 64, dict(window=33, keep=70, value_heads=2)),
+    ([17, 128, 500], 15, 1, 256, 32, dict(slopes=True, wide_values=True)),
+    ([8300], 2, 2, 256, 16, dict()),                                      # above 64 pieces a wave
+    ([40, 95], 14, 2, 128, 32, dict(gate="heads", sinks=True, keep=64, window=1)),
+])
+def test_rows(monkeypatch, splits, ctx, H, G, D, page, opts):
+    g = torch.Generator().manual_seed(sum(ctx) + D)
+    rn = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    need = [(c + page - 1) // page for c in ctx]
+    perm = torch.randperm(sum(need), generator=g).tolist()
+    table = [perm[sum(need[:i]):sum(need[:i + 1])] for i in range(len(ctx))]
+    past = [c - 1 for c in ctx]
+    T, Gv = len(ctx), opts.get("value_heads", G)
+    q, k = rn(T, H, D).bfloat16(), rn(sum(need), page, G, D).bfloat16()
+    v = rn(sum(need), page, Gv, D * (2 if opts.get("wide_values") else 1)).bfloat16()
+    v = v[..., :D]                                   # the leading channels of wider rows
+    slopes = 0.1 * torch.rand(H, generator=g) if opts.get("slopes") else None
+    sinks = rn(H) if opts.get("sinks") else None
+    gate = opts.get("gate") and rn(T, H * (D if opts["gate"] == "channels" else 1)).bfloat16()
+    window, softcap, keep = (opts.get(n, 0) for n in ("window", "softcap", "keep"))
+    want, big = _exact(q, k, v, table, past, page, D ** -0.5, slopes, gate, window, sinks, softcap,
+                       keep, opts.get("gate") == "channels")
+
+    lib = mx._lib()[0]
+    assert lib.oa_attn_rows_splits(H, G, D, D, 0, 1, T, max(ctx)) > 0
+    if splits:
+        monkeypatch.setattr(lib, "oa_attn_rows_splits", lambda *args: splits)
+    sb = mx.SeqBatch.build([(p, 1, i, t) for i, (p, t) in enumerate(zip(past, table))], page, "cuda")
+    dev = lambda x: None if x is None else x.cuda()  # noqa: E731
+    vd = torch.empty(sum(need), page, Gv, 2 * D, dtype=torch.bfloat16, device="cuda")
+    vd = vd[..., :D] if opts.get("wide_values") else torch.empty(v.shape, dtype=v.dtype, device="cuda")
+    vd.copy_(v)
+    got = mx.attention_paged(dev(q), dev(k), vd, sb, D ** -0.5, dev(slopes), dev(gate), window or None,
+                             dev(sinks), softcap or None, keep_first=keep,
+                             gate_channels=opts.get("gate") == "channels").cpu().double()
+    # a float32 sum of n terms is off by about 4 sqrt(n) 2^-24 of their size: the scores (D terms),
+    # the cap (2 softcap log2(e) within 2^-21), the distance (exact to 2^-23), the weights and
+    # their sums (a term a key). A weight's relative error moves the result twice: in the sum
+    # over the values, at most their largest in size, and in the normaliser
+    rel = (4 * D ** 0.5 * 2.0 ** -24 * big + 3 * softcap * 2.0 ** -21 + 0.1 * max(ctx) * 2.0 ** -23
+           + 4 * max(ctx) ** 0.5 * 2.0 ** -24 + 2.0 ** -21)
+    bound = want.abs() * 2.0 ** -8 + 2 * rel * float(v.float().abs().max())
+    assert ((got - want).abs() <= bound).all(), ((got - want).abs() / bound).max()

@@ -56,7 +56,8 @@ MIXERS_LIB = LIB.replace("libopsagent_kernels", "libopsagent_mixers")
 def test_mixers_library_exports():
     lib = ctypes.CDLL(MIXERS_LIB)
     for s in ["oa_causal_conv_seq", "oa_group_rmsnorm", "oa_attn_prepare",
-              "oa_attn_bias_geometry", "oa_attn_bias_paged", "oa_delta_rule_fused",
+              "oa_attn_bias_geometry", "oa_attn_bias_paged", "oa_attn_rows_splits",
+              "oa_delta_rule_fused",
               "oa_softcap", "oa_silu_mul_rows", "oa_embed_rows", "oa_dyt_norm",
               "oa_attn_rope_prepare", "oa_act_mul_rows", "oa_route_topk",
               "oa_moe_pairs_gateup", "oa_moe_pairs_down", "oa_add_layer_norm",
