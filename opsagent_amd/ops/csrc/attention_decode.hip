@@ -43,6 +43,16 @@ __device__ __forceinline__ float row_ror(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, 0xf, 0xf, true));
 }
 
+// halves (DIST 32) or neighbouring rows of 16 lanes (16) of a and b added up: the lanes of
+// the first half (row) get a's sum, those of the second b's
+template <int DIST>
+__device__ __forceinline__ float swap_add(float a, float b) {
+    const auto r = DIST == 32
+        ? __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false)
+        : __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // Scores on the matrix cores, values on the vector units, all in 32 bits.
 //
 // 16 keys x 128 channels go from the cache straight into A fragments of
@@ -395,68 +405,64 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
     // sums and maxima of every head to all lanes of a row
     if (GP == 4) lsum += row_ror<4>(lsum);
     lsum += row_ror<8>(lsum);
-    float mh[8], lh[8];
-    mh[0] = row_bcast<0>(m); mh[1] = row_bcast<1>(m); mh[2] = row_bcast<2>(m); mh[3] = row_bcast<3>(m);
-    mh[4] = row_bcast<4>(m); mh[5] = row_bcast<5>(m); mh[6] = row_bcast<6>(m); mh[7] = row_bcast<7>(m);
-    lh[0] = row_bcast<0>(lsum); lh[1] = row_bcast<1>(lsum); lh[2] = row_bcast<2>(lsum); lh[3] = row_bcast<3>(lsum);
-    lh[4] = row_bcast<4>(lsum); lh[5] = row_bcast<5>(lsum); lh[6] = row_bcast<6>(lsum); lh[7] = row_bcast<7>(lsum);
+    // Merge the wave's 4 rows: to their common maximum, then lane by lane. Swapping halves
+    // (quarters) of two registers and adding them leaves each lane with half (a quarter) of
+    // the sums, so that 24 swaps and as many additions do for G = 4 what took 80 exchanges
+    // through the LDS
+    float mt4 = fmaxf(m, __shfl_xor(m, 16, WAVE));
+    mt4 = fmaxf(mt4, __shfl_xor(mt4, 32, WAVE));
+    const float a4 = __expf(m - (mt4 == -INFINITY ? 0.0f : mt4));
+    lsum *= a4;
+    lsum += __shfl_xor(lsum, 16, WAVE);
+    lsum += __shfl_xor(lsum, 32, WAVE);
+    float al4[8];
+    al4[0] = row_bcast<0>(a4); al4[1] = row_bcast<1>(a4);
+    al4[2] = row_bcast<2>(a4); al4[3] = row_bcast<3>(a4);
+    al4[4] = row_bcast<4>(a4); al4[5] = row_bcast<5>(a4);
+    al4[6] = row_bcast<6>(a4); al4[7] = row_bcast<7>(a4);
+    constexpr int NO = G * 8;
+    float os[NO];
+#pragma unroll
+    for (int i = 0; i < NO; ++i) os[i] = o[i / 8][i % 8] * al4[i / 8];
+#pragma unroll
+    for (int i = 0; i < NO / 2; ++i) os[i] = swap_add<32>(os[i], os[i + NO / 2]);
+#pragma unroll
+    for (int i = 0; i < NO / 4; ++i) os[i] = swap_add<16>(os[i], os[i + NO / 4]);
 
-    // merge the wave's 4 key-groups (lanes l, l^16, l^32 hold same dims)
-#pragma unroll
-    for (int off = 16; off <= 32; off <<= 1) {
-#pragma unroll
-        for (int gh = 0; gh < G; ++gh) {
-            const float m2 = __shfl_xor(mh[gh], off, WAVE);
-            const float l2 = __shfl_xor(lh[gh], off, WAVE);
-            float o2[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) o2[j] = __shfl_xor(o[gh][j], off, WAVE);
-            const float mn = fmaxf(mh[gh], m2);
-            // guard: empty partial (l == 0, m == -inf) must not produce NaN
-            const float a1 = (lh[gh] > 0.0f) ? __expf(mh[gh] - mn) : 0.0f;
-            const float a2 = (l2 > 0.0f) ? __expf(m2 - mn) : 0.0f;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) o[gh][j] = o[gh][j] * a1 + o2[j] * a2;
-            lh[gh] = lh[gh] * a1 + l2 * a2;
-            mh[gh] = (lh[gh] > 0.0f) ? mn : -INFINITY;
-        }
-    }
-
-    // cross-wave combine through LDS
-    __shared__ float lds_o[4][G][DHEAD];
+    // cross-wave combine through LDS: row g16 now holds sums g16 * NO / 4 ... of its channels
+    __shared__ __attribute__((aligned(16))) float lds_o[4][G][DHEAD];
     __shared__ float lds_ml[4][G][2];
-    if (lane < 16) {
 #pragma unroll
-        for (int gh = 0; gh < G; ++gh) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) lds_o[wid][gh][dl * 8 + j] = o[gh][j];
-            if (dl == 0) {
-                lds_ml[wid][gh][0] = mh[gh];
-                lds_ml[wid][gh][1] = lh[gh];
-            }
-        }
+    for (int i = 0; i < NO / 4; ++i) {
+        const int at = g16 * (NO / 4) + i;
+        lds_o[wid][at / 8][dl * 8 + at % 8] = os[i];
+    }
+    if (lane < G) {
+        lds_ml[wid][lane][0] = lsum > 0.0f ? mt4 : -INFINITY;
+        lds_ml[wid][lane][1] = lsum;
     }
     __syncthreads();
 
-    // 256 threads cover G*128 outputs
-    for (int idx = threadIdx.x; idx < G * DHEAD; idx += blockDim.x) {
+    // 256 threads cover G*128 outputs, two channels each
+    for (int idx = 2 * threadIdx.x; idx < G * DHEAD; idx += 2 * blockDim.x) {
         const int gh = idx / DHEAD;
         const int d = idx % DHEAD;
         float mt = -INFINITY;
 #pragma unroll
         for (int w = 0; w < 4; ++w)
             if (lds_ml[w][gh][1] > 0.0f) mt = fmaxf(mt, lds_ml[w][gh][0]);
-        float lt = 0.0f, ot = 0.0f;
+        float lt = 0.0f;
+        float2 ot = {0.0f, 0.0f};
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
             const float lw = lds_ml[w][gh][1];
-            if (lw > 0.0f) {
-                const float sc = __expf(lds_ml[w][gh][0] - mt);
-                lt += lw * sc;
-                ot += lds_o[w][gh][d] * sc;
-            }
+            const float sc = lw > 0.0f ? __expf(lds_ml[w][gh][0] - mt) : 0.0f;
+            const float2 ow = *reinterpret_cast<const float2*>(&lds_o[w][gh][d]);
+            lt += lw > 0.0f ? lw * sc : 0.0f;
+            ot.x += lw > 0.0f ? ow.x * sc : 0.0f;
+            ot.y += lw > 0.0f ? ow.y * sc : 0.0f;
         }
-        opart_row[gh * DHEAD + d] = ot;
+        *reinterpret_cast<float2*>(opart_row + gh * DHEAD + d) = ot;
         if (d == 0) {
             mlpart_row[gh * 2 + 0] = mt;
             mlpart_row[gh * 2 + 1] = lt;
@@ -512,81 +518,107 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
     }
 }
 
-// Combine split partials -> final output. Grid: B*Hq blocks, 512 threads:
-// thread (d = tid & 127, sh = tid >> 7) accumulates splits sh, sh+4, ... so
-// the split loop runs nsplit/4 iterations with 4-way ILP, then the 4 partial
-// (m, l, o_d) triples merge through LDS. The (m, l) table is staged into LDS
-// once by the first wave (the naive one-thread-one-d loop over 64 splits was
-// 32 us/launch — 3x the attention kernel itself).
-template <int G>
-__global__ __launch_bounds__(512) void decode_combine_kernel(
+// Combine split partials -> final output. Grid: B*Hq blocks of NG groups of 32 lanes; a
+// group takes the splits s, s + NG, ..., a lane four channels. A small launch like this is
+// its chain of loads, so a group's first two splits and all statistics are asked for
+// together, and where the chip has room to spare (EARLY) even before the length says
+// which of them exist: what a split past the end left is not looked at. Every wave works
+// the common maximum and sum out for itself.
+template <int G, bool EARLY>
+__global__ __launch_bounds__(EARLY ? 512 : 256) void decode_combine_kernel(
     const float* __restrict__ o_part, const float* __restrict__ ml_part,
     const int* __restrict__ seq_lens, uint32_t* __restrict__ out, int B, int Hk, int nsplit,
     int chunk_base) {
+    constexpr int NG = EARLY ? 16 : 8;
     const int bq = blockIdx.x;
     const int Hq = Hk * G;
     const int b = bq / Hq;
     const int qh = bq % Hq;
     const int h = qh / G;
     const int gh = qh % G;
-    const int d = threadIdx.x & (DHEAD - 1);
-    const int sh = threadIdx.x >> 7;  // 0..3
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int grp = threadIdx.x >> 5, ch = (threadIdx.x & 31) * 4;
+    const size_t first = (size_t)(b * Hk + h) * nsplit * G + gh;
+    const float2* ml = reinterpret_cast<const float2*>(ml_part) + first;
+    const float* op = o_part + first * DHEAD + ch;
 
-    extern __shared__ __attribute__((aligned(16))) float sml[];  // [nsplit][2]
-    const int base = (b * Hk + h) * nsplit;
     const int n = seq_lens[b];
     const int ns = CEIL_DIV(n, decode_chunk(n, nsplit, chunk_base));
-    for (int s = threadIdx.x; s < ns; s += blockDim.x) {
-        const float2 ml = *reinterpret_cast<const float2*>(
-            ml_part + ((size_t)(base + s) * G + gh) * 2);
-        sml[s * 2] = ml.x;
-        sml[s * 2 + 1] = ml.y;
-    }
-    __syncthreads();
-
-    float mt = -INFINITY;
-    for (int s = sh; s < ns; s += 4)
-        if (sml[s * 2 + 1] > 0.0f) mt = fmaxf(mt, sml[s * 2]);
-    float lt = 0.0f, ot = 0.0f;
-    for (int s = sh; s < ns; s += 4) {
-        const float lw = sml[s * 2 + 1];
-        if (lw > 0.0f) {
-            const float sc = __expf(sml[s * 2] - mt);
-            lt += lw * sc;
-            ot += o_part[((size_t)(base + s) * G + gh) * DHEAD + d] * sc;
-        }
-    }
-    // merge the 4 split-groups via LDS (per d): (m, l, o) online combine
-    __shared__ float red_m[4][DHEAD], red_l[4][DHEAD], red_o[4][DHEAD];
-    red_m[sh][d] = mt;
-    red_l[sh][d] = lt;
-    red_o[sh][d] = ot;
-    __syncthreads();
-    if (sh == 0) {
+    // EARLY repeats the last split instead of a branch for each load
+    const float2 none = {0.0f, 0.0f};
+    const float2 mine = EARLY || lane < ns ? ml[(EARLY ? min(lane, nsplit - 1) : lane) * G] : none;
+    float2 mo[2];
+    float4 ov[2];
 #pragma unroll
-        for (int g2 = 1; g2 < 4; ++g2) {
-            const float m2 = red_m[g2][d], l2 = red_l[g2][d], o2 = red_o[g2][d];
-            const float mn = fmaxf(mt, m2);
-            const float a1 = (lt > 0.0f) ? __expf(mt - mn) : 0.0f;
-            const float a2 = (l2 > 0.0f) ? __expf(m2 - mn) : 0.0f;
-            ot = ot * a1 + o2 * a2;
-            lt = lt * a1 + l2 * a2;
-            mt = (lt > 0.0f) ? mn : -INFINITY;
-        }
-        const float res = (lt > 0.0f) ? ot / lt : 0.0f;
-        reinterpret_cast<uint16_t*>(out)[(size_t)(b * Hq + qh) * DHEAD + d] =
-            f32_to_bf16(res);
+    for (int i = 0; i < 2; ++i) {
+        const int s = EARLY ? min(grp + NG * i, nsplit - 1) : grp + NG * i;
+        mo[i] = EARLY || s < ns ? ml[s * G] : none;
+        ov[i] = EARLY || s < ns ? *reinterpret_cast<const float4*>(op + (size_t)s * G * DHEAD)
+                                : float4{0.0f, 0.0f, 0.0f, 0.0f};
     }
+
+    float mt = lane < ns && mine.y > 0.0f ? mine.x : -INFINITY;
+    for (int s = lane + WAVE; s < ns; s += WAVE)
+        if (ml[s * G].y > 0.0f) mt = fmaxf(mt, ml[s * G].x);
+    mt = wave_reduce_max(mt);
+    float lt = lane < ns && mine.y > 0.0f ? mine.y * __expf(mine.x - mt) : 0.0f;
+    for (int s = lane + WAVE; s < ns; s += WAVE)
+        if (ml[s * G].y > 0.0f) lt += ml[s * G].y * __expf(ml[s * G].x - mt);
+    lt = wave_reduce_sum(lt);
+
+    float4 ot = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto add = [&](const float2& m2, const float4& o4) {
+        const float sc = __expf(m2.x - mt);
+        ot.x += o4.x * sc;
+        ot.y += o4.y * sc;
+        ot.z += o4.z * sc;
+        ot.w += o4.w * sc;
+    };
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        if (grp + NG * i < ns && mo[i].y > 0.0f) add(mo[i], ov[i]);
+    for (int s = grp + 2 * NG; s < ns; s += NG)
+        if (ml[s * G].y > 0.0f)
+            add(ml[s * G], *reinterpret_cast<const float4*>(op + (size_t)s * G * DHEAD));
+
+    __shared__ __attribute__((aligned(16))) float red[NG][DHEAD];
+    *reinterpret_cast<float4*>(&red[grp][ch]) = ot;
+    __syncthreads();
+    const int d = threadIdx.x;
+    if (d >= DHEAD) return;
+    float sum = 0.0f;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) sum += red[g][d];
+    const float res = (lt > 0.0f) ? sum / lt : 0.0f;
+    reinterpret_cast<uint16_t*>(out)[(size_t)(b * Hq + qh) * DHEAD + d] = f32_to_bf16(res);
 }
 
 // Keys of the smallest split, by the (sequence, key head) pairs of the launch. Both
-// launches, 8 key heads, us with 64 / 128 / 256 / 512 keys: one sequence of 1151
-// tokens 14.4 / 14.5 / 15.9 / 19.3 (16.8 before scores ran on the matrix cores),
-// 8 of up to 1500 29.3 / 20.6 / 20.6 / 21.2 (38.5), 16 43.3 / 32.0 / 27.8 / 30.4
-// (64.3), 32 of up to 3000 104 / 86 / 72 / 69 (146), 64 180 / 153 / 129 / 117 (266;
-// its cache rows alone take 89 at 5.5 TB/s), 64 of up to 300 39 / 31 / 27 / 26 (152).
+// launches, 8 key heads unless said, us with 64 / 128 / 256 / 512 keys: one sequence of
+// 1151 tokens 9.9 / 10.6 / 11.4 / 14.4, 4 of 700 11.9 / 10.8 / 12.1 / 14.5, 13 of up to 900
+// (4 key heads) 16.4 / 13.0 / 12.1 / 14.8, 8 of up to 1500 20.7 / 16.6 / 16.4 / 15.9, 16
+// 32.7 / 25.9 / 24.1 / 25.8, 32 of up to 3000 84 / 75 / 65 / 63, 64 147 / 133 / 117 / 109
+// (its cache rows alone take 82 at 6 TB/s), 64 of up to 300 30 / 26 / 23 / 22. Before rows
+// merged by swaps and the combine asked ahead, the sizes in use took 13.0, 12.6, 15.0,
+// 19.0, 26.3, 64.8, 112.8 and 24.0.
 static int decode_chunk_base(int pairs) {
-    return pairs <= 8 ? 64 : pairs <= 64 ? 128 : pairs <= 128 ? 256 : 512;
+    return pairs <= 8 ? 64 : pairs <= 32 ? 128 : pairs <= 128 ? 256 : 512;
+}
+
+// Early loads pay while the launch is a few blocks (both launches, us: one sequence of 1151
+// tokens 10.4 -> 9.9, 8 of up to 1500 16.9 -> 16.5) and cost where 2048 of them ask for
+// splits that do not exist (64 of up to 300: 24.1 -> 25.0).
+template <int G>
+static void launch_combine(hipStream_t s, const void* o_part, const void* ml_part,
+                           const void* seq_lens, void* out, int B, int Hk, int nsplit, int cb) {
+    if (B * Hk <= 64)
+        hipLaunchKernelGGL((decode_combine_kernel<G, true>), dim3(B * Hk * G), dim3(512), 0, s,
+                           (const float*)o_part, (const float*)ml_part, (const int*)seq_lens,
+                           (uint32_t*)out, B, Hk, nsplit, cb);
+    else
+        hipLaunchKernelGGL((decode_combine_kernel<G, false>), dim3(B * Hk * G), dim3(256), 0, s,
+                           (const float*)o_part, (const float*)ml_part, (const int*)seq_lens,
+                           (uint32_t*)out, B, Hk, nsplit, cb);
 }
 
 // fused: cnt_ws is zeroed here on each call (hipMemsetAsync). fused = 0: two kernels.
@@ -605,8 +637,6 @@ extern "C" int oa_attention_decode(void* stream, const void* q, const void* kc,
     int block_shift = 0;
     while ((1 << block_shift) < block_size) ++block_shift;
     dim3 grid(B * Hk, nsplit), block(256);
-    dim3 cgrid(B * Hq), cblock(512);
-    const int clds = nsplit * 2 * (int)sizeof(float);
 
     if (fused) {
         hipError_t e = hipMemsetAsync(cnt_ws, 0, B * Hk * 4, (hipStream_t)stream);
@@ -640,10 +670,8 @@ extern "C" int oa_attention_decode(void* stream, const void* q, const void* kc,
                                (const float*)nullptr, (const int*)nullptr,          \
                                (uint32_t*)nullptr, (uint32_t*)nullptr, 0, 0);       \
             HIP_CHECK_LAUNCH();                                                     \
-            hipLaunchKernelGGL((decode_combine_kernel<GV>), cgrid, cblock, clds,    \
-                               (hipStream_t)stream, (const float*)o_part,           \
-                               (const float*)ml_part, (const int*)seq_lens,         \
-                               (uint32_t*)out, B, Hk, nsplit, cb);                                             \
+            launch_combine<GV>((hipStream_t)stream, o_part, ml_part, seq_lens, out, B, Hk, \
+                               nsplit, cb);                                         \
             HIP_CHECK_LAUNCH();                                                     \
         }                                                                           \
     } while (0)
@@ -676,8 +704,6 @@ extern "C" int oa_attention_decode_rope(
     int block_shift = 0;
     while ((1 << block_shift) < block_size) ++block_shift;
     dim3 grid(B * Hk, nsplit), block(256);
-    dim3 cgrid(B * Hq), cblock(512);
-    const int clds = nsplit * 2 * (int)sizeof(float);
 
     const int cb = decode_chunk_base(B * Hk);
 #define LAUNCH_GR(GV)                                                              \
@@ -693,10 +719,8 @@ extern "C" int oa_attention_decode_rope(
                            (const float*)sin_t, (const int*)slots, (uint32_t*)kc,   \
                            (uint32_t*)vc, k_stride / 2, v_stride / 2);              \
         HIP_CHECK_LAUNCH();                                                         \
-        hipLaunchKernelGGL((decode_combine_kernel<GV>), cgrid, cblock, clds,        \
-                           (hipStream_t)stream, (const float*)o_part,               \
-                           (const float*)ml_part, (const int*)seq_lens,             \
-                           (uint32_t*)out, B, Hk, nsplit, cb);                      \
+        launch_combine<GV>((hipStream_t)stream, o_part, ml_part, seq_lens, out, B, Hk,     \
+                           nsplit, cb);                                             \
         HIP_CHECK_LAUNCH();                                                         \
     } while (0)
 

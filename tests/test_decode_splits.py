@@ -130,3 +130,24 @@ def test_infinite_keys(G):
     for nsplit in (1, 4):
         got = ops.attention_decode_paged(q, kc, vc, table, lens, nsplit=nsplit)[0].double()
         assert float((got - want).norm() / want.norm()) < 2.1e-3     # 256 values and more
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,nsplit,Hk", [
+    ([9000, 4600, 1, 64], 128, 4),                   # 71 splits: more than lanes, asked for ahead
+    ([10300, 257] + [5] * 18, 40, 4),                # 33 of 40 beside many short sequences
+    ([2000, 33], 32, 32),                            # 64 pairs, asked for ahead
+    ([2000, 33, 300], 32, 32),                       # 96 pairs, not
+])
+def test_combine_of_many_splits(lens, nsplit, Hk):
+    G, bs = 2, 32
+    q, _, _, kc, vc, table, lens_t, _ = _case(lens, Hk, G, bs, seed=sum(lens))
+    want = []
+    for b, n in enumerate(lens):
+        at = torch.arange(n, device="cuda")
+        r = table[b, at // bs].long() * bs + at % bs
+        want.append(_attend(q[b].double(), kc.view(-1, Hk, D)[r].double(),
+                            vc.view(-1, Hk, D)[r].double(), G))
+    got = ops.attention_decode_paged(q, kc, vc, table, lens_t, nsplit=nsplit).double()
+    want = torch.stack(want)
+    assert (got - want).norm() / want.norm() < 2e-3      # as above: one bf16 rounding
