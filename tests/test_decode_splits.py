@@ -151,3 +151,37 @@ def test_combine_of_many_splits(lens, nsplit, Hk):
     got = ops.attention_decode_paged(q, kc, vc, table, lens_t, nsplit=nsplit).double()
     want = torch.stack(want)
     assert (got - want).norm() / want.norm() < 2e-3      # as above: one bf16 rounding
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("G,Hk,lens", [(4, 8, [700, 65, 130]), (8, 4, [513, 64]), (1, 33, [1, 90])])
+def test_copies_of_the_first_row(G, Hk, lens):
+    """Rows that repeat the first are answered by its results; rows that write its slot but differ
+    in a query or an earlier page are answered by themselves."""
+    bs, B = 32, 24
+    cos, sin = (t.cuda() for t in ops.rope_cos_sin(1024, D))
+
+    def batch(rows):
+        q, k, v, kc, vc, table, n, slots = _case(lens, Hk, G, bs, seed=G)
+        at = torch.tensor(rows, device="cuda")
+        return [x[at].contiguous() for x in (q, k, v)] + [kc, vc, table[at], n[at], cos, sin, slots[at]]
+
+    plain = ops.attention_decode_rope(*batch(range(len(lens))), nsplit=4)
+    args = batch([*range(len(lens)), *[0] * (B - len(lens))])
+    got = ops.attention_decode_rope(*args, nsplit=4)
+    rel = (got[: len(lens)].float() - plain.float()).norm() / plain.float().norm()
+    assert rel < 2e-3                                 # splits of other sizes: one bf16 rounding apart
+    assert torch.equal(got[len(lens):], got[:1].expand_as(got[len(lens):]))
+
+    args = batch([*range(len(lens)), *[0] * (B - len(lens))])
+    args[0][B - 1, 0, 5] += 1.0                       # one query of one head
+    if lens[0] > bs:
+        args[5][B - 2, 0] = args[5][1, 0]             # another first page
+    other = ops.attention_decode_rope(*args, nsplit=4)
+    assert torch.equal(other[: B - 2], got[: B - 2])
+    alone = [x[-2:].contiguous() for x in (*args[:3], *args[5:7], args[9])]
+    want = ops.attention_decode_rope(*alone[:3], args[3], args[4], *alone[3:5], cos, sin, alone[5],
+                                     nsplit=4)
+    assert (other[-2:].float() - want.float()).norm() / want.float().norm() < 2e-3
+    assert lens[0] == 1 or not torch.equal(other[-1], got[0])
+    assert lens[0] <= bs or not torch.equal(other[-2], got[0])
