@@ -1416,13 +1416,11 @@ def greedy_sample_masked(
         hip.check(rc, "oa_masked_argmax_f32")
         return out
     assert logits.dtype == torch.bfloat16 and logits.is_contiguous()
-    ws = torch.empty(B, dtype=torch.int64, device=logits.device)
     mask_ptr = mask_bits.data_ptr() if mask_bits is not None else None
     if mask_bits is not None:
         assert mask_bits.dtype == torch.int32 and mask_bits.is_contiguous()
     rc = lib.oa_masked_argmax(
-        hip.current_stream_ptr(), logits.data_ptr(), mask_ptr, ws.data_ptr(),
-        out.data_ptr(), B, V,
+        hip.current_stream_ptr(), logits.data_ptr(), mask_ptr, out.data_ptr(), B, V,
     )
     hip.check(rc, "oa_masked_argmax")
     return out

@@ -65,7 +65,7 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_skinny.restype = i
     lib.oa_gemv_gateup_ex.argtypes = [p, p, p, p, p, i, i, i, f, i]
     lib.oa_gemv_gateup_ex.restype = i
-    lib.oa_masked_argmax.argtypes = [p, p, p, p, p, i, i]
+    lib.oa_masked_argmax.argtypes = [p, p, p, p, i, i]
     lib.oa_masked_argmax.restype = i
     lib.oa_masked_argmax_f32.argtypes = [p, p, p, p, p, i, i]
     lib.oa_masked_argmax_f32.restype = i
