@@ -251,7 +251,7 @@ class DecoderLayer(nn.Module):
         a = self.attn(h, cos, sin, k_cache, v_cache, fb, parts)
         h, residual = ops.fused_add_rms_norm(a, residual, self.post_norm_w, self.eps)
         if self.is_moe_layer:
-            m = self.mlp(h, decode=fb.kind == "decode")
+            m = self.mlp(h, decode=fb.kind == "decode", parts=parts)
         else:
             m = self.mlp(h, parts)
         return m, residual

@@ -88,7 +88,8 @@ class MoEMLP(nn.Module):
         else:
             self.shared = None
 
-    def forward(self, x: torch.Tensor, decode: bool = False) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, decode: bool = False, parts: bool = False):
+        """parts: the result may be an ops.PairSum, for the norm that follows (one rank)."""
         T, H = x.shape
         w13, w2 = (self.w13_q, self.w2_q) if self.fp8 else (self.w13, self.w2)
         s13, s2 = (self.w13_s, self.w2_s) if self.fp8 else (None, None)
@@ -109,12 +110,14 @@ class MoEMLP(nn.Module):
                 shared = self.shared(x) if local else None
                 if tiles and not (few and not ops.moe_sorted_wins(P, self.num_experts, self.fp8,
                                                                     self.i_local * H)):
-                    out = ops.moe_sorted_mlp(x, w13, s13, w2, s2, idx, wts, more=shared)
+                    out = ops.moe_sorted_mlp(x, w13, s13, w2, s2, idx, wts, more=shared, parts=parts)
                 else:
                     y = ops.moe_grouped_mlp(x, w13, s13, w2, s2, idx.view(-1), tok.view(-1),
                                             wts.view(-1), self.i_local, self.fp8,
                                             num_experts=self.num_experts)
-                    out = ops.moe_combine(y, self.top_k, shared)
+                    out = ops.moe_combine(y, self.top_k, shared, parts)
+                if parts:                                # one rank, the shared expert inside
+                    return out
                 if local or self.shared is None:
                     return tp_all_reduce(out)
                 return tp_all_reduce(out) + self.shared(x)

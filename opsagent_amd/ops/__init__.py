@@ -14,7 +14,7 @@ attention, activation, sampling) are the HIP kernels here.
 from __future__ import annotations
 
 import os
-from typing import Optional, Tuple
+from typing import NamedTuple, Optional, Tuple, Union
 
 import torch
 from torch.autograd import forward_ad
@@ -419,12 +419,31 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.
     return out
 
 
+class PairSum(NamedTuple):
+    """A sum that the norm behind it takes: for each token its `top` rows of y
+    [T * top, H], bf16, plus its row of `more`."""
+
+    y: torch.Tensor
+    top: int
+    more: Optional[torch.Tensor]
+
+
 def fused_add_rms_norm(
-    x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5
+    x: Union[torch.Tensor, PairSum], residual: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     """Returns (rmsnorm(x+residual), x+residual). GPU path updates `residual`
     in place as the new residual stream and returns it. x may be the parts of a
-    product (linear_parts)."""
+    product (linear_parts) or a sum over pairs (PairSum)."""
+    if isinstance(x, PairSum):
+        rows, dim = residual.shape
+        assert residual.is_contiguous() and x.y.shape == (rows * x.top, dim)
+        lib, hip = _lib()
+        out = torch.empty_like(residual)
+        hip.check(lib.oa_add_rmsnorm_pairs(
+            hip.current_stream_ptr(), x.y.data_ptr(), x.top,
+            x.more.data_ptr() if x.more is not None else None, residual.data_ptr(),
+            weight.data_ptr(), out.data_ptr(), rows, dim, eps), "oa_add_rmsnorm_pairs")
+        return out, residual
     if not _is_gpu(x):
         return torch_ref.fused_add_rms_norm(x, residual, weight, eps)
     if x.dim() == 3 and x.dtype == torch.float32:
@@ -767,13 +786,16 @@ def moe_route(x: torch.Tensor, router_w: torch.Tensor, top: int):
     return idx, wts, tok
 
 
-def moe_combine(y: torch.Tensor, top: int, more: Optional[torch.Tensor] = None) -> torch.Tensor:
+def moe_combine(y: torch.Tensor, top: int, more: Optional[torch.Tensor] = None,
+                parts: bool = False) -> Union[torch.Tensor, PairSum]:
     """out[t] = sum of rows t * top .. + top of y [T * top, H] (+ more[t]), bf16
-    with float32 sums in one order."""
+    with float32 sums in one order. With `parts` it may be left to the norm that follows."""
     T, H = y.shape[0] // top, y.shape[1]
     assert y.is_cuda and y.dtype == torch.bfloat16 and y.is_contiguous()
     assert more is None or (more.shape == (T, H) and more.dtype == y.dtype
                             and more.is_contiguous())
+    if parts and H % 8 == 0 and H <= 8192 and (more is None or more.data_ptr() % 16 == 0):
+        return PairSum(y, top, more)
     lib, hip = _lib()
     out = torch.empty(T, H, dtype=y.dtype, device=y.device)
     hip.check(lib.oa_moe_combine(hip.current_stream_ptr(), y.data_ptr(),
@@ -852,13 +874,14 @@ def moe_sorted_mlp(
     pair_weights: torch.Tensor,
     act=None,
     more: Optional[torch.Tensor] = None,
-) -> torch.Tensor:
+    parts: bool = False,
+) -> Union[torch.Tensor, PairSum]:
     """Routed experts of a prompt-sized batch (GPU): out[t] = sum over token t's
     choices j of weight_tj * W2[e_tj] act(W13[e_tj] x_t), plus more[t] if given.
     x [T, H] bf16; expert_ids int32 and pair_weights float32 [T, top]; experts as
     in moe_grouped_mlp, bf16 or fp8 with row scales. Pairs are sorted by expert
     on the GPU and every expert's rows run as matrix-core tiles: no host sync,
-    static shapes."""
+    static shapes. With `parts` the sum may be left to the norm that follows."""
     T, H = x.shape
     top = expert_ids.shape[1]
     E, I = w13.shape[0], w2.shape[2]
@@ -886,7 +909,7 @@ def moe_sorted_mlp(
     hip.check(lib.oa_moe_grouped(stream, mid.data_ptr(), w2.data_ptr(), ptr(w2_scale), *lists,
                                  pair_weights.data_ptr(), y.data_ptr(), E, H, I, top, bm, max_tiles,
                                  0, 0, 0.0, 0.0), "oa_moe_grouped(down)")
-    return moe_combine(y, top, more)
+    return moe_combine(y, top, more, parts)
 
 
 def moe_grouped_mlp(

@@ -105,8 +105,8 @@ extern "C" int oa_fused_add_rmsnorm(void* stream, const void* x, void* residual,
 // The same behind a product whose columns are split: x is the sum of `parts` float32 planes
 // [parts, rows, D], added in order and rounded to bf16 as the product by itself would be. One
 // launch less per product, us of the sum and the norm / of this, 64 rows of 4096 in 8
-// planes: 9.6 / 5.2. What bounds it is the
-// launch and one round of loads: a thread takes four columns of all planes.
+// planes: 9.6 / 5.2. What bounds it is the launch and one round of loads: a thread takes
+// four columns of all planes.
 __global__ __launch_bounds__(1024) void rmsnorm_parts_kernel(
     const float* __restrict__ x, int parts, int64_t plane, uint16_t* __restrict__ residual,
     const uint16_t* __restrict__ w, uint16_t* __restrict__ out, int D, float inv_d, float eps) {
@@ -159,6 +159,72 @@ extern "C" int oa_add_rmsnorm_parts(void* stream, const void* x, int parts, void
     hipLaunchKernelGGL(rmsnorm_parts_kernel, dim3(rows), dim3(threads), 0, (hipStream_t)stream,
                        (const float*)x, parts, (int64_t)rows * dim, (uint16_t*)residual,
                        (const uint16_t*)w, (uint16_t*)out, dim, 1.0f / dim, eps);
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
+// The same behind routed experts: x is the sum of a token's `top` rows of y [rows * top, D],
+// bf16, and its row of `more` if there is one, in that order in float32, rounded to bf16 as
+// the sum by itself would be. One launch and one pass less: a decode step of 13 tokens over 4
+// layers of 64 experts 599 -> 586 us, a prompt of 512 1427 -> 1418.
+__global__ __launch_bounds__(1024) void rmsnorm_pairs_kernel(
+    const uint4* __restrict__ y, int top, const uint4* __restrict__ more,
+    uint4* __restrict__ residual, const uint4* __restrict__ w, uint4* __restrict__ out, int D8,
+    float inv_d, float eps) {
+    __shared__ float red[16];
+    const int c = threadIdx.x;                       // eight columns
+    const int64_t at = (int64_t)blockIdx.x * D8 + c;
+    float v[8], sumsq = 0.0f;
+    uint4 g;
+    if (c < D8) {
+        const uint4 r = residual[at];
+        g = w[c];
+        const uint4 m = more ? more[at] : make_uint4(0, 0, 0, 0);
+        const uint4* row = y + (int64_t)blockIdx.x * top * D8 + c;
+        float a[8] = {};
+#pragma unroll 8
+        for (int k = 0; k < top; ++k) {
+            const uint4 u = row[(int64_t)k * D8];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                a[2 * j] += bf16_lo((&u.x)[j]);
+                a[2 * j + 1] += bf16_hi((&u.x)[j]);
+            }
+        }
+        uint4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (more) {
+                a[2 * j] += bf16_lo((&m.x)[j]);
+                a[2 * j + 1] += bf16_hi((&m.x)[j]);
+            }
+            const uint32_t x = pack_bf16x2(a[2 * j], a[2 * j + 1]);
+            v[2 * j] = bf16_lo(x) + bf16_lo((&r.x)[j]);
+            v[2 * j + 1] = bf16_hi(x) + bf16_hi((&r.x)[j]);
+            sumsq += v[2 * j] * v[2 * j] + v[2 * j + 1] * v[2 * j + 1];
+            (&o.x)[j] = pack_bf16x2(v[2 * j], v[2 * j + 1]);
+        }
+        residual[at] = o;
+    }
+    const float scale = rsqrtf(block_reduce_sum<16>(sumsq, red) * inv_d + eps);
+    if (c >= D8) return;
+    uint4 o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        (&o.x)[j] = pack_bf16x2(v[2 * j] * scale * bf16_lo((&g.x)[j]),
+                                v[2 * j + 1] * scale * bf16_hi((&g.x)[j]));
+    out[at] = o;
+}
+
+extern "C" int oa_add_rmsnorm_pairs(void* stream, const void* y, int top, const void* more,
+                                    void* residual, const void* w, void* out, int rows, int dim,
+                                    float eps) {
+    if (dim % 8 != 0 || dim > 8192 || top < 1 || rows < 1) return -100;
+    if (((uintptr_t)y | (uintptr_t)more | (uintptr_t)residual | (uintptr_t)w | (uintptr_t)out) % 16 != 0)
+        return -101;
+    hipLaunchKernelGGL(rmsnorm_pairs_kernel, dim3(rows), dim3(CEIL_DIV(dim / 8, WAVE) * WAVE), 0,
+                       (hipStream_t)stream, (const uint4*)y, top, (const uint4*)more,
+                       (uint4*)residual, (const uint4*)w, (uint4*)out, dim / 8, 1.0f / dim, eps);
     HIP_CHECK_LAUNCH();
     return 0;
 }

@@ -27,6 +27,28 @@ def test_planes(parts, T, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,top,D,shared", [(1, 1, 8, False), (3, 6, 2048, True), (16, 9, 520, False),
+                                            (70, 2, 8192, True)])
+def test_pairs(T, top, D, shared):
+    g = torch.Generator(device="cuda").manual_seed(D)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()  # noqa: E731
+    y, more, residual, w = rn(T * top, D), rn(T, D) if shared else None, rn(T, D), 1 + 0.1 * rn(D)
+    x = ops.moe_combine(y, top, more, parts=True)
+    assert isinstance(x, ops.PairSum)
+    want, want_r = ops.fused_add_rms_norm(ops.moe_combine(y, top, more), residual.clone(), w, 1e-5)
+    got, got_r = ops.fused_add_rms_norm(x, residual, w, 1e-5)
+    assert got_r.data_ptr() == residual.data_ptr() and torch.equal(got_r, want_r)
+    assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -7, atol=0)    # as above
+    assert (got != want).float().mean() < 0.01
+
+
+@pytest.mark.gpu
+def test_wide_pairs_are_summed():
+    assert ops.moe_combine(torch.zeros(4, 8200, dtype=torch.bfloat16, device="cuda"), 2,
+                           parts=True).shape == (2, 8200)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,N,K", [(8, 4096, 14336), (64, 4096, 4096), (77, 4096, 4096), (24, 2048, 8192),
                                    (3, 2048, 2048), (200, 4096, 4096), (1, 4096, 4096)])
 def test_products(T, N, K):
