@@ -608,18 +608,26 @@ __global__ __launch_bounds__(256) void attn_bias_paged_kernel(
 typedef short s4_t __attribute__((ext_vector_type(4)));
 typedef short s8_t __attribute__((ext_vector_type(8)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
+// What bounds it: instructions, 504 vector ones a wave and tile at 128 channels
+// beside 48 products, so the chip needs waves beside each other. FULL gives the
+// compiler the head size: tests around every fragment kept a read and its product
+// in one small block each. With that, three waves a SIMD (163 registers) and the
+// pages a tile ahead, us: prompts of 1024, 333 and 77, 32 heads of 128, 8 kv
+// heads 105.9 -> 58.2 (74.1 with FULL alone, 64.6 with three waves), one of 4096
+// 826 -> 463, 500 tokens behind 3000 254 -> 159, a window of 512 over 2000, 4 kv
+// heads 52.8 -> 39.5, heads of 256 154 -> 105, of 64 72 -> 59.
 #define MF_KT 64
 #define MF_KPAD 8
 
-template <int MAXD, int MAXDV, bool QK32, int NT>
-__global__ __launch_bounds__(256) void attn_bias_mfma_kernel(
+template <int MAXD, int MAXDV, bool QK32, int NT, bool FULL>
+__global__ __launch_bounds__(256, FULL && MAXD <= 8 ? 3 : 1) void attn_bias_mfma_kernel(
     const bf16s* __restrict__ q, const bf16s* __restrict__ gate, int64_t gs,
     const bf16s* __restrict__ k_cache, const bf16s* __restrict__ v_cache,
     bf16s* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
     const int* __restrict__ cu, const int* __restrict__ past,
     const int* __restrict__ block_table, int max_blocks, int block_size,
     const float* __restrict__ slopes, const float* __restrict__ sinks, int B, int H, int G,
-    int D, int Dv, int HB, float scale, int nsplit, int window, int vrow, int hrows, int Gv,
+    int D_, int Dv_, int HB, float scale, int nsplit, int window, int vrow, int hrows, int Gv,
     float softcap, int64_t os, float oscale, int keep, int gch) {
     // hrows (decode steps of many query heads per kv head): a step brings one
     // token per sequence, so the 16 columns of a wave's tile are 16 HEADS at
@@ -627,8 +635,10 @@ __global__ __launch_bounds__(256) void attn_bias_mfma_kernel(
     // 64 heads of one kv head and every staged key/value tile serves them
     // all. The head (and with it slope, sink, gate and output row) is then a
     // per-lane value.
+    // FULL: D = 16 MAXD and Dv = 16 MAXDV, known to the compiler.
     // NT: 16-token sub-tiles per wave. Every K and V fragment read from LDS
     // feeds NT MFMAs, and a staged tile serves NT times the query rows.
+    const int D = FULL ? 16 * MAXD : D_, Dv = FULL ? 16 * MAXDV : Dv_;
     extern __shared__ float lds[];
     bf16s* Ks = (bf16s*)lds;                        // [64][D+8]
     const int kst = D + MF_KPAD;
@@ -724,19 +734,24 @@ __global__ __launch_bounds__(256) void attn_bias_mfma_kernel(
     const int bsh = 31 - __clz(block_size), bmask = block_size - 1;
     // Staging map: a thread owns ONE key per tile for K (key tid/4, every 4th
     // 16-byte piece of its row) and one for V (key tid%64, every 4th piece),
-    // so a tile costs it two page lookups. The next tile's pieces are loaded
-    // into registers while the current tile is computed.
+    // so a tile costs it two page lookups, made a tile ahead. The next tile's
+    // pieces are loaded into registers while the current tile is computed.
     constexpr int KC = MAXD / 2, VC = MAXDV / 2;
     const int kj = threadIdx.x >> 2, kc0 = threadIdx.x & 3;
     const int vj = threadIdx.x & 63, vc0 = threadIdx.x >> 6;
     uint4 kreg[KC], vreg[VC];
+    int pagek = 0, pagev = 0;
+    auto look_up = [&](int kt) {
+        pagek = bt[min(kt * MF_KT + kj, block_last) >> bsh];
+        pagev = bt[min(kt * MF_KT + vj, block_last) >> bsh];
+    };
     auto fetch = [&](int kt) {
         const int k0 = kt * MF_KT;
         const int nk = min(MF_KT, block_last + 1 - k0);
         const int keyk = k0 + kj, keyv = k0 + vj;
         const bool okk = kj < nk, okv = vj < nk;
-        const int64_t sk_ = okk ? ((int64_t)bt[keyk >> bsh] << bsh) + (keyk & bmask) : 0;
-        const int64_t sv_ = okv ? ((int64_t)bt[keyv >> bsh] << bsh) + (keyv & bmask) : 0;
+        const int64_t sk_ = okk ? ((int64_t)pagek << bsh) + (keyk & bmask) : 0;
+        const int64_t sv_ = okv ? ((int64_t)pagev << bsh) + (keyv & bmask) : 0;
         const bf16s* kp = k_cache + (sk_ * G + g) * D;
         const bf16s* vp = v_cache + (sv_ * vrow + (g % Gv) * Dv);
 #pragma unroll
@@ -755,7 +770,12 @@ __global__ __launch_bounds__(256) void attn_bias_mfma_kernel(
     // key tiles before the window of the block's first query are skipped,
     // except those that hold kept first keys
     const KeyTiles tiles = key_tiles(pb + tile * TQ, nkt, MF_KT, window, keep);
+    auto look_ahead = [&](int it) {
+        if (it < tiles.count) look_up(tiles.at(it));
+    };
+    look_ahead(split);
     if (split < tiles.count) fetch(tiles.at(split));
+    look_ahead(split + nsplit);
     for (int it = split; it < tiles.count; it += nsplit) {
         const int k0 = tiles.at(it) * MF_KT;
         __syncthreads();
@@ -778,6 +798,7 @@ __global__ __launch_bounds__(256) void attn_bias_mfma_kernel(
         }
         __syncthreads();
         if (it + nsplit < tiles.count) fetch(tiles.at(it + nsplit));
+        look_ahead(it + 2 * nsplit);
         if (wave_ntok <= 0 || k0 > wave_last || (k0 + MF_KT - 1 <= pb + t0 - wlim && k0 >= keep))
             continue;
         // S^T tiles: keys k0 + 16*mt + 4*lg + r, token lc of sub-tile u
@@ -2077,7 +2098,7 @@ extern "C" int oa_attn_bias_geometry(int H, int G, int D, int Dv, int dt, int ma
     return -103;
 }
 
-template <int MAXD, int MAXDV, bool QK32, int NT>
+template <int MAXD, int MAXDV, bool QK32, int NT, bool FULL = false>
 static void launch_attn_mfma(hipStream_t s, dim3 grid, int lds_bytes, const void* q, const void* gate,
                              int64_t gs, const void* k_cache, const void* v_cache, void* out,
                              void* part_o, void* part_ml, const void* cu, const void* past,
@@ -2087,9 +2108,9 @@ static void launch_attn_mfma(hipStream_t s, dim3 grid, int lds_bytes, const void
                              int hrows, int Gv, float softcap, int64_t os, float oscale, int keep,
                              int gch) {
     if (lds_bytes > 48 * 1024)
-        (void)hipFuncSetAttribute((const void*)attn_bias_mfma_kernel<MAXD, MAXDV, QK32, NT>,
+        (void)hipFuncSetAttribute((const void*)attn_bias_mfma_kernel<MAXD, MAXDV, QK32, NT, FULL>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    hipLaunchKernelGGL((attn_bias_mfma_kernel<MAXD, MAXDV, QK32, NT>), grid, dim3(256), lds_bytes, s,
+    hipLaunchKernelGGL((attn_bias_mfma_kernel<MAXD, MAXDV, QK32, NT, FULL>), grid, dim3(256), lds_bytes, s,
                        (const bf16s*)q, (const bf16s*)gate, gs, (const bf16s*)k_cache,
                        (const bf16s*)v_cache, (bf16s*)out, (float*)part_o, (float*)part_ml,
                        (const int*)cu, (const int*)past, (const int*)block_table, max_blocks,
@@ -2192,7 +2213,10 @@ extern "C" int oa_attn_bias_paged(void* stream, const void* q, const void* gate,
         else launch_attn_mfma<A, Bv, false, 1>(MF_ARGS);                        \
     } while (0)
             const int a = D <= 64 ? 4 : (D <= 128 ? 8 : 16), bv = Dv <= 64 ? 4 : (Dv <= 128 ? 8 : 16);
-            if (a == 4 && bv == 4) MF(4, 4);
+            if (D == 64 && Dv == 64) launch_attn_mfma<4, 4, true, 1, true>(MF_ARGS);
+            else if (D == 128 && Dv == 128) launch_attn_mfma<8, 8, true, 1, true>(MF_ARGS);
+            else if (D == 256 && Dv == 256) launch_attn_mfma<16, 16, true, 1, true>(MF_ARGS);
+            else if (a == 4 && bv == 4) MF(4, 4);
             else if (a == 4 && bv == 8) MF(4, 8);
             else if (a == 4) MF(4, 16);
             else if (a == 8 && bv == 4) MF(8, 4);

@@ -109,3 +109,38 @@ def test_rows(monkeypatch, splits, ctx, H, G, D, page, opts):
            + 4 * max(ctx) ** 0.5 * 2.0 ** -24 + 2.0 ** -21)
     bound = want.abs() * 2.0 ** -8 + 2 * rel * float(v.float().abs().max())
     assert ((got - want).abs() <= bound).all(), ((got - want).abs() / bound).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("H,G,chunks,page,opts", [
+    (4, 1, [(0, 17), (63, 2), (100, 64)], 32, dict(slopes=True)),
+    (6, 3, [(0, 130), (5, 1)], 8, dict(window=33, keep=5, sinks=True)),   # pages below a tile's 64 keys
+    (3, 1, [(190, 3)], 64, dict(softcap=20.0, gate="heads")),
+])
+def test_prompts(D, H, G, chunks, page, opts):
+    """The tile kernel at the head sizes that it is built for, against 64 bits."""
+    g = torch.Generator().manual_seed(D + H)
+    rn = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    need = [(p + n + page - 1) // page for p, n in chunks]
+    perm = torch.randperm(sum(need), generator=g).tolist()
+    table = [perm[sum(need[:i]):sum(need[:i + 1])] for i in range(len(chunks))]
+    T = sum(n for _, n in chunks)
+    q, k, v = rn(T, H, D).bfloat16(), rn(sum(need), page, G, D).bfloat16(), rn(sum(need), page, G, D).bfloat16()
+    slopes = 0.1 * torch.rand(H, generator=g) if opts.get("slopes") else None
+    sinks = rn(H) if opts.get("sinks") else None
+    gate = rn(T, H).bfloat16() if opts.get("gate") else None
+    window, softcap, keep = (opts.get(n, 0) for n in ("window", "softcap", "keep"))
+    rows = [(t, p + i) for t, (p, n) in zip(table, chunks) for i in range(n)]
+    want, big = _exact(q, k, v, [t for t, _ in rows], [p for _, p in rows], page, D ** -0.5, slopes, gate,
+                       window, sinks, softcap, keep, False)
+    sb = mx.SeqBatch.build([(p, n, i, t) for i, ((p, n), t) in enumerate(zip(chunks, table))], page, "cuda")
+    dev = lambda x: None if x is None else x.cuda()  # noqa: E731
+    got = mx.attention_paged(q.cuda(), k.cuda(), v.cuda(), sb, D ** -0.5, dev(slopes), dev(gate), window or None,
+                             dev(sinks), softcap or None, keep_first=keep).cpu().double()
+    # as above; a weight enters its product as two bf16, within 2^-15 of itself
+    ctx = max(p + n for p, n in chunks)
+    rel = (4 * D ** 0.5 * 2.0 ** -24 * big + 3 * softcap * 2.0 ** -21 + 0.1 * ctx * 2.0 ** -23
+           + 4 * ctx ** 0.5 * 2.0 ** -24 + 2.0 ** -21 + 2.0 ** -15)
+    bound = want.abs() * 2.0 ** -8 + 2 * rel * float(v.float().abs().max())
+    assert ((got - want).abs() <= bound).all(), ((got - want).abs() / bound).max()
