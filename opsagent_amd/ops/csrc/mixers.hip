@@ -966,9 +966,9 @@ __global__ __launch_bounds__(256, FULL && MAXD <= 8 ? 3 : 1) void attn_bias_mfma
 // What bounds it: with few blocks the chain of loads (past, page, keys) and the
 // merge, beyond them the reads, at one block of eight waves a CU (220 registers
 // a lane at D = 128, HB = 4). us a call, tile kernel with its splits -> here:
-// one row, window 512, 4 kv heads of 4: 13.1 -> 8.4; contexts 1030, 340, 84,
-// 8 kv heads of 4: 17.3 -> 11.1; 64 rows of 500 to 3650: 305 -> 122 (4.5 TB/s);
-// one of 16000: 81 -> 25.5; four of 40: 8.7 -> 4.6. With the page looked up key
+// one row, window 512, 4 kv heads of 4: 13.1 -> 7.8; contexts 1030, 340, 84,
+// 8 kv heads of 4: 17.3 -> 10.1; 64 rows of 500 to 3650: 305 -> 122 (4.5 TB/s);
+// one of 16000: 81 -> 23.8; four of 40: 8.7 -> 4.6. With the page looked up key
 // by key in each piece the last but one took 24.6 in the same splits, but the
 // 64 rows 143 and one block going through 16000 keys 214 instead of 174.
 constexpr int rows_piece(int D) { return D == 256 ? 16 : 32; }
@@ -1192,7 +1192,10 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
 
 // merge key-split partials: one block per (token, head). Every wave first
 // takes the statistics of all splits, a lane each; then wave w adds up the
-// splits w, w + 4, ..., a lane per value channel, and the waves' sums meet in LDS
+// splits w, w + 4, ..., a lane per value channel, and the waves' sums meet in LDS.
+// A launch like this is its chain of loads: a wave's first four splits are asked
+// for with the statistics (attention and this, one row, window 512: 8.4 -> 7.8 us;
+// 4 rows of 900, heads of 256, 13.0 -> 10.7; one of 16000, 32 splits, 25.3 -> 23.8).
 template <typename TC>
 __global__ __launch_bounds__(256) void attn_combine_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml,
@@ -1202,6 +1205,16 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(
     const int64_t row = blockIdx.x;  // tok * H + h
     const int tok = (int)(row / H), h = (int)(row % H);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int AHEAD = 4;
+    float pm[AHEAD], po_[AHEAD][ATT_MAXV];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+        const int64_t at = row * nsplit + min(wave + 4 * i, nsplit - 1);
+        pm[i] = part_ml[at * 2];
+#pragma unroll
+        for (int c = 0; c < ATT_MAXV; ++c)
+            po_[i][c] = 64 * c < Dv ? part_o[at * Dv + min(lane + 64 * c, Dv - 1)] : 0.0f;
+    }
     float mx = -INFINITY, lsum = 0.0f;
     for (int s0 = 0; s0 < nsplit; s0 += 64) {          // running merge over groups of 64 splits
         const int s = s0 + lane;
@@ -1216,8 +1229,15 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(
     float acc[ATT_MAXV];
 #pragma unroll
     for (int c = 0; c < ATT_MAXV; ++c) acc[c] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+        if (wave + 4 * i >= nsplit) break;
+        const float wj = (pm[i] == -INFINITY) ? 0.0f : expf(pm[i] - mx);
+#pragma unroll
+        for (int c = 0; c < ATT_MAXV; ++c) acc[c] += po_[i][c] * wj;
+    }
 #pragma unroll 4
-    for (int s = wave; s < nsplit; s += 4) {
+    for (int s = wave + 4 * AHEAD; s < nsplit; s += 4) {
         const float ms = part_ml[(row * nsplit + s) * 2];
         const float wj = (ms == -INFINITY) ? 0.0f : expf(ms - mx);
         const float* po = part_o + (row * nsplit + s) * Dv;
@@ -2130,7 +2150,8 @@ static bool attn_rows(int H, int G, int D, int Dv, int dt, int max_chunk) {
 // CUs: with fewer heads a block where that leaves no wave more than one piece,
 // else with every head that shares the keys (one row of 16000 keys, 8 kv heads
 // of 4: 25.0 us in 32 splits of four heads, 29.8 in 16 of two, 49.5 in 8 of
-// one; 2000 keys, 4 kv heads: 12.1 in 16 of four, 9.3 in 16 of one).
+// one; 2000 keys, 4 kv heads: 12.1 in 16 of four, 9.3 in 16 of one; all before the
+// merge asked ahead, which takes a microsecond off each).
 extern "C" int oa_attn_rows_splits(int H, int G, int D, int Dv, int dt, int max_chunk, int ntiles,
                                    int reach) {
     if (G < 1 || H % G != 0 || ntiles < 1 || !attn_rows(H, G, D, Dv, dt, max_chunk)) return 0;
