@@ -240,10 +240,11 @@ class DecoderLayer(nn.Module):
         else:
             self.mlp = DenseMLP(spec, dtype, gen)
 
-    def forward(self, x, residual, cos, sin, k_cache, v_cache, fb):
+    def forward(self, x, residual, cos, sin, k_cache, v_cache, fb, normed=None):
+        """normed: the input norm of x, where the first layer's caller has it."""
         if residual is None:
             residual = x
-            h = ops.rms_norm(x, self.input_norm_w, self.eps)
+            h = ops.rms_norm(x, self.input_norm_w, self.eps) if normed is None else normed
         else:
             h, residual = ops.fused_add_rms_norm(x, residual, self.input_norm_w, self.eps)
         # the norm after a sublayer adds up its last product's parts (not what ranks add up)
@@ -412,20 +413,21 @@ class LlamaForCausalLM(nn.Module):
             torch.cuda.empty_cache()
 
     def forward(self, fb: ForwardBatch, kv_caches: List[Tuple[torch.Tensor, torch.Tensor]]):
-        x = F.embedding(fb.input_ids, self.embed)
-        if self._use_fused_decode(fb, x):
-            residual = x.contiguous()
+        if self._use_fused_decode(fb, fb.input_ids):
+            residual = F.embedding(fb.input_ids, self.embed).contiguous()
             for i, layer in enumerate(self.layers):
                 residual = layer.fused_decode(
                     residual, self.rope_cos, self.rope_sin,
                     kv_caches[i][0], kv_caches[i][1], fb,
                 )
             return ops.rms_norm(residual, self.final_norm_w, self.spec.rms_eps)
+        x, normed = ops.embed_rms_norm(fb.input_ids, self.embed, self.layers[0].input_norm_w,
+                                       self.spec.rms_eps)
         residual = None
         for i, layer in enumerate(self.layers):
             x, residual = layer(
                 x, residual, self.rope_cos, self.rope_sin,
-                kv_caches[i][0], kv_caches[i][1], fb,
+                kv_caches[i][0], kv_caches[i][1], fb, normed if i == 0 else None,
             )
         x, _ = ops.fused_add_rms_norm(x, residual, self.final_norm_w, self.spec.rms_eps)
         return x  # [T, hidden]

@@ -419,6 +419,26 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.
     return out
 
 
+def embed_rms_norm(ids: torch.Tensor, table: torch.Tensor, weight: torch.Tensor,
+                   eps: float = 1e-5) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(table[ids], its rms_norm) for token ids [T]."""
+    D = table.shape[1]
+    if not (table.is_cuda and table.dtype == torch.bfloat16 and weight.dtype == table.dtype
+            and table.is_contiguous() and weight.is_contiguous()
+            and ids.dim() == 1 and ids.is_contiguous()
+            and ids.dtype in (torch.int64, torch.int32) and ids.device == table.device
+            and D % 8 == 0 and D <= 8192 and (table.data_ptr() | weight.data_ptr()) % 16 == 0):
+        x = torch.nn.functional.embedding(ids, table)
+        return x, rms_norm(x, weight, eps)
+    lib, hip = _lib()
+    x, out = torch.empty(2, ids.numel(), D, dtype=table.dtype, device=table.device)
+    hip.check(lib.oa_embed_rmsnorm(
+        hip.current_stream_ptr(), table.data_ptr(), ids.data_ptr(), int(ids.dtype == torch.int64),
+        table.shape[0], weight.data_ptr(), x.data_ptr(), out.data_ptr(), ids.numel(), D, eps),
+        "oa_embed_rmsnorm")
+    return x, out
+
+
 class PairSum(NamedTuple):
     """A sum that the norm behind it takes: for each token its `top` rows of y
     [T * top, H], bf16, plus its row of `more`."""

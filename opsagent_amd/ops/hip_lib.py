@@ -33,6 +33,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     f = ctypes.c_float
     lib.oa_rmsnorm.argtypes = [p, p, p, p, i, i, f]
     lib.oa_rmsnorm.restype = i
+    lib.oa_embed_rmsnorm.argtypes = [p, p, p, i, ctypes.c_int64, p, p, p, i, i, f]
+    lib.oa_embed_rmsnorm.restype = i
     lib.oa_add_rmsnorm_pairs.argtypes = [p, p, i, p, p, p, p, i, i, f]
     lib.oa_add_rmsnorm_pairs.restype = i
     lib.oa_add_rmsnorm_parts.argtypes = [p, p, i, p, p, p, i, i, f]

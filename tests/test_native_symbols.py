@@ -23,7 +23,7 @@ ENTRY_POINTS = [
     "oa_gemv_gateup_ex", "oa_gemv_grouped", "oa_gemv_split", "oa_gemv_gateup_fp8", "oa_gemv_rw4", "oa_kv_write",
     "oa_masked_argmax", "oa_masked_argmax_f32", "oa_moe_down", "oa_moe_down_emaj", "oa_moe_gateup",
     "oa_moe_gateup_emaj", "oa_moe_gateup_act", "oa_moe_gateup_emaj_act", "oa_quant_fp8", "oa_rmsnorm", "oa_rope",
-    "oa_rope_kv", "oa_silu_mul", "oa_token_logprobs", "oa_add_rmsnorm_parts", "oa_add_rmsnorm_pairs",
+    "oa_rope_kv", "oa_silu_mul", "oa_token_logprobs", "oa_add_rmsnorm_parts", "oa_add_rmsnorm_pairs", "oa_embed_rmsnorm",
 ]
 
 

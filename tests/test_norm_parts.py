@@ -27,6 +27,25 @@ def test_planes(parts, T, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,D", [(1, 8), (3, 2048), (17, 2056), (70, 8192)])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_embedding_and_norm(T, D, dtype):
+    g = torch.Generator(device="cuda").manual_seed(D + T)
+    table = torch.randn(300, D, generator=g, device="cuda").bfloat16()
+    w = (1 + 0.1 * torch.randn(D, generator=g, device="cuda")).bfloat16()
+    ids = torch.randint(0, 300, (T,), generator=g, device="cuda", dtype=dtype)
+    ids[0], ids[-1] = 299, 0
+    x, h = ops.embed_rms_norm(ids, table, w, 1e-5)
+    assert torch.equal(x, table[ids.long()]) and torch.equal(h, ops.rms_norm(x, w, 1e-5))
+
+
+def test_embedding_and_norm_on_the_cpu():
+    table, w, ids = torch.randn(9, 16), torch.rand(16), torch.tensor([3, 8, 0])
+    x, h = ops.embed_rms_norm(ids, table, w, 1e-5)
+    assert torch.equal(x, table[ids]) and torch.equal(h, ops.rms_norm(x, w, 1e-5))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,top,D,shared", [(1, 1, 8, False), (3, 6, 2048, True), (16, 9, 520, False),
                                             (70, 2, 8192, True)])
 def test_pairs(T, top, D, shared):
