@@ -781,28 +781,48 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
 // Splits added up: one wave per (query, head) row, two channels per lane. rows = B * Sq
 // * Hq; scale2 turns a difference of maxima into a power of two. A split without a visible
 // key has weight sum 0; one with a NaN or an infinite score has a NaN sum, and counts.
+// The launch is its chain of loads: the first eight splits are asked for together, weights
+// or not (77 queries of 32 heads behind 1187 keys, 8 splits: 7.4 us -> 3.9).
 __global__ __launch_bounds__(256) void prefill_combine_kernel(const float* __restrict__ po,
                                                               const float* __restrict__ pml,
                                                               uint32_t* __restrict__ out, int rows,
                                                               int nsplit, float scale2) {
     const int row = blockIdx.x * 4 + threadIdx.x / WAVE, lane = threadIdx.x & (WAVE - 1);
     if (row >= rows) return;
+    constexpr int AHEAD = 8;
+    auto stats = [&](int s) {
+        return *reinterpret_cast<const float2*>(pml + ((size_t)s * rows + row) * 2);
+    };
+    auto part = [&](int s) {
+        return *reinterpret_cast<const float2*>(po + ((size_t)s * rows + row) * DHEAD + lane * 2);
+    };
+    float2 ml[AHEAD], o[AHEAD];
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) {
+        ml[s] = stats(min(s, nsplit - 1));
+        o[s] = part(min(s, nsplit - 1));
+    }
     float mx = -INFINITY;
-    for (int s = 0; s < nsplit; ++s) {
-        const float2 ml = *reinterpret_cast<const float2*>(pml + ((size_t)s * rows + row) * 2);
-        if (ml.y != 0.0f) mx = fmaxf(mx, ml.x);
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s)
+        if (s < nsplit && ml[s].y != 0.0f) mx = fmaxf(mx, ml[s].x);
+    for (int s = AHEAD; s < nsplit; ++s) {
+        const float2 m = stats(s);
+        if (m.y != 0.0f) mx = fmaxf(mx, m.x);
     }
     float l = 0.0f, a = 0.0f, b = 0.0f;
-    for (int s = 0; s < nsplit; ++s) {
-        const size_t r = (size_t)s * rows + row;
-        const float2 ml = *reinterpret_cast<const float2*>(pml + r * 2);
-        if (ml.y != 0.0f) {
-            const float w = __builtin_amdgcn_exp2f((ml.x - mx) * scale2);
-            const float2 o = *reinterpret_cast<const float2*>(po + r * DHEAD + lane * 2);
-            l = fmaf(ml.y, w, l);
-            a = fmaf(o.x, w, a);
-            b = fmaf(o.y, w, b);
-        }
+    auto add = [&](const float2& m, const float2& v) {
+        const float w = __builtin_amdgcn_exp2f((m.x - mx) * scale2);
+        l = fmaf(m.y, w, l);
+        a = fmaf(v.x, w, a);
+        b = fmaf(v.y, w, b);
+    };
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s)
+        if (s < nsplit && ml[s].y != 0.0f) add(ml[s], o[s]);
+    for (int s = AHEAD; s < nsplit; ++s) {
+        const float2 m = stats(s);
+        if (m.y != 0.0f) add(m, part(s));
     }
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
     out[(size_t)row * (DHEAD / 2) + lane] = pack_bf16x2(a * inv, b * inv);
