@@ -279,7 +279,9 @@ def _ring_narrow(M: int, N: int, K: int, gateup: bool, wide) -> Optional[int]:
     4096 too both forms take the same). Up to 16 rows strips of skinny.hip are
     the faster form for short rows (4096 x 4096, 8 9.1 / 9.8, 24 11.9 / 10.6; 32000 x 2048, 6
     27.8 / 29.0) and the wide ring where it has splits of its own (16384 x 4096, 8 26.3 /
-    26.8)."""
+    26.8). Splits of a multiple of 2048 columns start on the same channels, which the wide ring
+    mends by more of them (8192 x 4096, 24 15.1 / 17.2, 48 16.1 / 18.6; 4096 x 8192, 24 16.9 /
+    18.0; 4096 x 24576 37 / 44; but 4096 x 16384 30.7 / 28.9)."""
     if not 2 < M <= (64 if wide is None else 48) or K % 64 or N % 8:
         return None
     weights = (2 if gateup else 1) * N * K
@@ -308,7 +310,8 @@ def _ring_narrow(M: int, N: int, K: int, gateup: bool, wide) -> Optional[int]:
         ok = K % (splits * 2048) != 0 and (K >= 5120 or K >= 3072 and weights >= 24e6)
     else:
         # a square weight that the library is best at (2560 x 2560, 40 9.4 / 9.5, 64 13.8 / 10.6)
-        ok = K >= 2048 and not (wide is None and K >= N and 32 < M <= 48)
+        ok = K >= 2048 and not (wide is None and K >= N and 32 < M <= 48) and not (
+            wide and K % (splits * 2048) == 0)
     return splits if ok else None
 
 

@@ -208,6 +208,7 @@ def test_narrow_plans():
     assert choice(49, 14336, 4096, True) == (64, 1, False) and choice(2, 14336, 4096, True) is None
     assert choice(8, 11008, 4096, True) is None                # 344 blocks: a round two thirds full
     assert choice(24, 2048, 2048) is None                      # under 10 MB
+    assert choice(24, 8192, 4096) == (32, 4, False)            # two splits of 2048 columns each
     assert choice(24, 4096, 4096) == (32, 4, True) and choice(8, 4096, 4096) is None
     assert choice(48, 2048, 8192) == (64, 8, True) and choice(49, 2048, 8192)[2] is False
     assert choice(64, 16384, 4096) == (64, 1, True)           # the library's otherwise
