@@ -202,14 +202,16 @@ extern "C" int oa_masked_argmax_f32(void* stream, const void* logits, const void
 // the lookups took 150 and the host waited for each of them.
 //
 // An entry is value << 32 | ~index in an order that floats keep as integers: equal values
-// go by index, NaN is the largest.
+// go by index, NaN is the largest. Every entry lies above 0 and below LP_START, also a NaN's
+// at index 0: a merge that takes the largest below the last one finds all that are there.
 typedef unsigned long long lp_u64;
+#define LP_START (~(lp_u64)0)
 
 __device__ __forceinline__ float lp_load(const float* p) { return *p; }
 __device__ __forceinline__ float lp_load(const uint16_t* p) { return bf16_to_f32(*p); }
 
 __device__ __forceinline__ lp_u64 lp_entry(float v, int i) {
-    const uint32_t key = v != v ? 0xffffffffu : ordered_f32(v);
+    const uint32_t key = v != v ? 0xfffffffeu : ordered_f32(v);
     return (lp_u64)key << 32 | (uint32_t)~i;
 }
 __device__ __forceinline__ lp_u64 wave_max_u64(lp_u64 v) {
@@ -300,7 +302,7 @@ __global__ __launch_bounds__(256) void logprob_finish_kernel(
         const int t = tokens[b];
         out[0] = __float_as_int(t >= 0 && t < V ? (lp_load(row + t) - m) - ls : NAN);
     }
-    lp_u64 prev = ~(lp_u64)0;
+    lp_u64 prev = LP_START;
     for (int r = 0; r < top; ++r) {
         lp_u64 x = 0;
         for (int i = tid; i < waves * top; i += 256) {
@@ -313,7 +315,7 @@ __global__ __launch_bounds__(256) void logprob_finish_kernel(
         x = max(max(win[0], win[1]), max(win[2], win[3]));
         prev = x;
         if (tid == 0) {
-            const int t = (int)~(uint32_t)x;
+            const int t = (int)~(uint32_t)x;         // found: top <= V, and no wave has less to give
             out[1 + 2 * r] = t;
             out[2 + 2 * r] = __float_as_int((lp_load(row + t) - m) - ls);
         }

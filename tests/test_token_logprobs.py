@@ -60,3 +60,20 @@ def test_special_values(dtype):
     assert torch.isnan(want[2:4]).all() and torch.isnan(want[4, 2000])
     assert idx[3, 0] == 2000 and idx[4, 0] == 2000           # NaN, then infinity first
     assert idx[2].tolist() == [0, 1, 2, 3]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V", [7, 1000, 1024, 3000])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_nan_at_any_token(V, dtype):
+    """NaN counts as the largest wherever it stands, the first token and all of them included."""
+    nan = float("nan")
+    rows = torch.randn(4, V, generator=torch.Generator().manual_seed(V)).to(dtype)
+    rows[0, 0] = nan
+    rows[1] = nan
+    rows[2, [0, V - 1]] = nan
+    for top in (1, 7):
+        _, idx, val = ops.token_logprobs(rows.cuda(), torch.zeros(4, dtype=torch.int32, device="cuda"), top)
+        order = torch.sort(rows.float(), descending=True, stable=True).indices[:, :top]
+        assert torch.equal(idx.long(), order)
+        assert torch.isnan(val[:3]).all() and not torch.isnan(val[3]).any()
