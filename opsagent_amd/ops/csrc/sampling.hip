@@ -201,9 +201,10 @@ extern "C" int oa_masked_argmax_f32(void* stream, const void* logits, const void
 // of 128256 bf16 takes 12.5 us with its 5 best (5.6 with none, 46 with 20), where a float32 copy, log-softmax, a sort of the row and
 // the lookups took 150 and the host waited for each of them.
 //
-// An entry is value << 32 | ~index in an order that floats keep as integers: equal values
-// go by index, NaN is the largest. Every entry lies above 0 and below LP_START, also a NaN's
-// at index 0: a merge that takes the largest below the last one finds all that are there.
+// An entry is value << 32 | ~index in an order that floats keep as integers: equal values go
+// by index (-0 and +0 are one), NaN is the largest. Every entry lies above 0 and below
+// LP_START, also a NaN's at index 0: a merge that takes the largest below the last one finds
+// all that are there.
 typedef unsigned long long lp_u64;
 #define LP_START (~(lp_u64)0)
 
@@ -211,7 +212,7 @@ __device__ __forceinline__ float lp_load(const float* p) { return *p; }
 __device__ __forceinline__ float lp_load(const uint16_t* p) { return bf16_to_f32(*p); }
 
 __device__ __forceinline__ lp_u64 lp_entry(float v, int i) {
-    const uint32_t key = v != v ? 0xfffffffeu : ordered_f32(v);
+    const uint32_t key = v != v ? 0xfffffffeu : ordered_f32(v + 0.0f);    // -0 + 0 is +0
     return (lp_u64)key << 32 | (uint32_t)~i;
 }
 __device__ __forceinline__ lp_u64 wave_max_u64(lp_u64 v) {

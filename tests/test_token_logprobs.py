@@ -77,3 +77,16 @@ def test_nan_at_any_token(V, dtype):
         order = torch.sort(rows.float(), descending=True, stable=True).indices[:, :top]
         assert torch.equal(idx.long(), order)
         assert torch.isnan(val[:3]).all() and not torch.isnan(val[3]).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_signed_zeros(dtype):
+    """-0 and +0 are one value, which goes by index within a wave and between waves."""
+    rows = torch.full((3, 3000), -1.0, dtype=dtype)
+    rows[0, [5, 6]] = torch.tensor([-0.0, 0.0], dtype=dtype)
+    rows[1, [5, 2500]] = torch.tensor([-0.0, 0.0], dtype=dtype)
+    rows[2, [5, 2500]] = torch.tensor([0.0, -0.0], dtype=dtype)
+    _, idx, val = ops.token_logprobs(rows.cuda(), torch.zeros(3, dtype=torch.int32, device="cuda"), 3)
+    assert idx.tolist() == [[5, 6, 0], [5, 2500, 0], [5, 2500, 0]]
+    assert torch.equal(val[:, 0], val[:, 1]) and (val[:, 1] > val[:, 2]).all()
