@@ -394,10 +394,7 @@ class LLMEngine:
 
     # -- request API ----------------------------------------------------
     def add_request(self, prompt_ids: List[int], params: SamplingParams) -> int:
-        if self.request_bcast and self.tp_rank == 0:
-            # record the PRE-normalization arguments; followers re-run this
-            # exact function, so clamping/truncation replays identically
-            self._bcast_pending.append((list(prompt_ids), _params_to_wire(params)))
+        given = prompt_ids, params
         if params.max_new_tokens >= self.max_seq_len:
             # a budget >= the context window would otherwise invert the
             # truncation slice below and empty the prompt
@@ -420,6 +417,14 @@ class LLMEngine:
             )
             self.perf.record_metric("engine_prompt_truncated_tokens", float(truncated))
             prompt_ids = prompt_ids[-keep:]
+        if len(prompt_ids) and not 0 <= min(prompt_ids) <= max(prompt_ids) < self.spec.vocab_size:
+            # on the host: the device reads the embedding row of whatever id it is given
+            raise ValueError(f"prompt token ids lie outside the model's vocabulary of "
+                             f"{self.spec.vocab_size}")
+        if self.request_bcast and self.tp_rank == 0:
+            # record the PRE-normalization arguments; followers re-run this
+            # exact function, so clamping/truncation replays identically
+            self._bcast_pending.append((list(given[0]), _params_to_wire(given[1])))
         rid = self._next_id
         self._next_id += 1
         req = Request(rid, list(prompt_ids), params)

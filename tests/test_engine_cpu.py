@@ -633,3 +633,14 @@ def test_grammar_check_tokens_and_masks_along():
     assert gs.forced_peek(16).startswith(b'{"question"')
     masks = gs.masks_along(list(b'{"q'))
     assert masks.shape[0] == 4
+
+
+@pytest.mark.parametrize("bad", [-1, 512, 2 ** 40])
+def test_ids_outside_the_vocabulary_are_refused(engine, bad):
+    """A prompt with such an id is no request; dropped by the truncation it does no harm."""
+    with pytest.raises(ValueError, match="vocabulary"):
+        engine.add_request([1, bad, 2], SamplingParams(max_new_tokens=4))
+    assert not engine.requests and not engine.waiting
+    out, _ = engine.generate([bad] + [7] * 300, SamplingParams(max_new_tokens=4))
+    assert len(out) > 0
+    assert engine.generate([0, 511], SamplingParams(max_new_tokens=2))[0]
