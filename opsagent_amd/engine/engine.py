@@ -1432,6 +1432,14 @@ class LLMEngine:
         for i, req in enumerate(batch):
             tok = int(tokens[i])
             gs = req.grammar_state
+            if gs is None and tok < 0:
+                # no logit of the row can be chosen (all NaN or -inf): there is no token to
+                # append, and none whose embedding the next step could read
+                log.warning("request %d: no token can be sampled from its logits", req.req_id)
+                req.finished = True
+                req.finish_reason = "no_token"
+                req._emit([])
+                continue
             if gs is not None:
                 if tok < 0 or not gs.accept(tok):
                     # mask guaranteed validity; a -1 means no token was allowed

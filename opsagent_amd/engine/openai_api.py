@@ -42,6 +42,7 @@ _FINISH_MAP = {
     "length": "length",
     "max_seq_len": "length",
     "grammar_dead_end": "stop",
+    "no_token": "stop",
 }
 
 

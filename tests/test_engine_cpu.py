@@ -644,3 +644,30 @@ def test_ids_outside_the_vocabulary_are_refused(engine, bad):
     out, _ = engine.generate([bad] + [7] * 300, SamplingParams(max_new_tokens=4))
     assert len(out) > 0
     assert engine.generate([0, 511], SamplingParams(max_new_tokens=2))[0]
+
+
+def test_row_without_a_token_ends_its_request(engine, monkeypatch):
+    """-1 (no logit can be chosen) is no token: it is not appended, and the others go on."""
+    from opsagent_amd import ops
+
+    params = SamplingParams(max_new_tokens=8, stop_on_eos=False, logprobs=True, top_logprobs=2)
+    want, _ = engine.generate([5, 6, 7], params)
+    real = ops.greedy_sample_masked
+
+    def sample(logits, mask):
+        tokens = real(logits, mask)
+        if len(tokens) == 2:
+            tokens[0] = -1
+        return tokens
+
+    monkeypatch.setattr(ops, "greedy_sample_masked", sample)
+    bad, good = (engine.add_request(p, params) for p in ([9, 8], [5, 6, 7]))
+    reqs = [engine.requests[r] for r in (bad, good)]
+    while not all(r.finished for r in reqs):
+        engine.step()
+    assert reqs[0].finish_reason == "no_token" and reqs[1].finish_reason == "length"
+    assert len(reqs[0].output_ids) == 1 and min(reqs[0].output_ids) >= 0
+    assert len(reqs[0].logprob_content) == 1
+    assert reqs[1].output_ids == want
+    for r in (bad, good):
+        engine.requests.pop(r)
