@@ -424,7 +424,8 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.
 
 def embed_rms_norm(ids: torch.Tensor, table: torch.Tensor, weight: torch.Tensor,
                    eps: float = 1e-5) -> Tuple[torch.Tensor, torch.Tensor]:
-    """(table[ids], its rms_norm) for token ids [T]."""
+    """(table[ids], its rms_norm) for token ids [T]; rows of NaN for ids outside the table
+    (the GPU path, which cannot raise)."""
     D = table.shape[1]
     if not (table.is_cuda and table.dtype == torch.bfloat16 and weight.dtype == table.dtype
             and table.is_contiguous() and weight.is_contiguous()

@@ -11,7 +11,8 @@
 // token, and becomes the residual: one launch for the gather and the norm of a step's
 // first layer, which the library walks token by token up to 16 of them (us, gather and
 // norm in a step of 8 rows of 4096: 7.7 + 4.4, of 16 of 2048 10.8 + 4.8; a step of 13
-// tokens through experts 590 -> 580, of 8 sequences 505 -> 502, of 47 885 -> 866).
+// tokens through experts 590 -> 580, of 8 sequences 505 -> 502, of 47 885 -> 866). An id
+// outside the table, which the engine refuses before, reads nothing: its row is NaN.
 enum { RN_PLAIN, RN_ADD, RN_EMBED };
 template <int MODE, typename ID>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(
@@ -22,9 +23,10 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
     __shared__ float red[16];
     const int64_t row = blockIdx.x;
     int64_t from = row;
+    bool known = true;                               // the same for the block
     if (MODE == RN_EMBED) {
         from = ids[row];
-        if (from < 0 || from >= vocab) __builtin_trap();    // no such token
+        known = from >= 0 && from < vocab;
     }
     const uint4* xrow = x + from * D8;
     float v[4][8], sumsq = 0.0f;
@@ -32,7 +34,8 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
     for (int k = 0; k < 4; ++k) {
         const int c = k * 256 + threadIdx.x;
         if (c >= D8) break;
-        const uint4 xv = xrow[c];
+        const uint32_t nan = 0x7fc07fc0u;
+        const uint4 xv = MODE != RN_EMBED || known ? xrow[c] : make_uint4(nan, nan, nan, nan);
         uint4 r;
         if (MODE == RN_ADD) r = residual[row * D8 + c];
 #pragma unroll

@@ -39,6 +39,21 @@ def test_embedding_and_norm(T, D, dtype):
     assert torch.equal(x, table[ids.long()]) and torch.equal(h, ops.rms_norm(x, w, 1e-5))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_ids_outside_the_table(dtype):
+    """Nothing is read for them: rows of NaN, the others as they are."""
+    table = torch.randn(300, 2056, device="cuda").bfloat16()
+    w = torch.ones(2056, device="cuda").bfloat16()
+    far = 2 ** 40 if dtype == torch.int64 else 2 ** 31 - 1
+    ids = torch.tensor([299, -1, 0, 300, far, -far, 7], dtype=dtype, device="cuda")
+    x, h = ops.embed_rms_norm(ids, table, w, 1e-5)
+    good = [0, 2, 6]
+    assert torch.equal(x[good], table[ids[good].long()])
+    assert torch.equal(h[good], ops.rms_norm(x, w, 1e-5)[good])
+    assert x[[1, 3, 4, 5]].isnan().all() and h[[1, 3, 4, 5]].isnan().all()
+
+
 def test_embedding_and_norm_on_the_cpu():
     table, w, ids = torch.randn(9, 16), torch.rand(16), torch.tensor([3, 8, 0])
     x, h = ops.embed_rms_norm(ids, table, w, 1e-5)
