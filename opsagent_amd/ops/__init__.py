@@ -345,15 +345,14 @@ def _ring(x: torch.Tensor, w: torch.Tensor, plan: Tuple[int, ...], act: int = 0,
     return part if parts else out
 
 
-def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+def linear_parts(x: torch.Tensor, w: torch.Tensor) -> Union[torch.Tensor, PlaneSum]:
     """x @ w^T for rows x [T, K] that go through fused_add_rms_norm next: bf16 [T, N], or the
-    product's float32 column parts [parts, T, N], which the norm adds up, where the transfer
-    ring splits it."""
+    product's float32 column parts, which the norm adds up, where the transfer ring splits it."""
     M = x.numel() // x.shape[-1]
     if 1 < M <= 128 and x.dim() == 2 and w.shape[0] <= 8192 and _skinny_ok(x, w):
         plan = _ring_choice(M, w.shape[0], w.shape[1])
         if plan and plan[1] > 1:
-            return _ring(x, w, plan, parts=True)
+            return PlaneSum(_ring(x, w, plan, parts=True))
     return linear(x, w)
 
 
@@ -443,6 +442,12 @@ def embed_rms_norm(ids: torch.Tensor, table: torch.Tensor, weight: torch.Tensor,
     return x, out
 
 
+class PlaneSum(NamedTuple):
+    """A product whose float32 column parts [parts, T, N] the norm behind it adds up."""
+
+    planes: torch.Tensor
+
+
 class PairSum(NamedTuple):
     """A sum that the norm behind it takes: for each token its `top` rows of y
     [T * top, H], bf16, plus its row of `more`."""
@@ -452,33 +457,56 @@ class PairSum(NamedTuple):
     more: Optional[torch.Tensor]
 
 
-def fused_add_rms_norm(
-    x: Union[torch.Tensor, PairSum], residual: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5
-) -> Tuple[torch.Tensor, torch.Tensor]:
-    """Returns (rmsnorm(x+residual), x+residual). GPU path updates `residual`
-    in place as the new residual stream and returns it. x may be the parts of a
-    product (linear_parts) or a sum over pairs (PairSum)."""
+def _added_up(x: Union[PlaneSum, PairSum]) -> torch.Tensor:
+    """The hidden rows that x stands for, bf16, in the order of the norms' kernels."""
     if isinstance(x, PairSum):
-        rows, dim = residual.shape
-        assert residual.is_contiguous() and x.y.shape == (rows * x.top, dim)
-        lib, hip = _lib()
-        out = torch.empty_like(residual)
+        return moe_combine(x.y, x.top, x.more)
+    total = x.planes[0].clone()
+    for plane in x.planes[1:]:
+        total += plane
+    return total.to(torch.bfloat16)
+
+
+def _add_norm_parts(x: Union[PlaneSum, PairSum], residual: torch.Tensor, weight: torch.Tensor,
+                    eps: float) -> torch.Tensor:
+    """fused_add_rms_norm's first result from what is not added up yet."""
+    rows, dim = residual.shape
+    assert residual.dtype == weight.dtype == torch.bfloat16 and weight.numel() == dim
+    assert residual.is_contiguous() and weight.is_contiguous()
+    if isinstance(x, PlaneSum):
+        assert x.planes.dtype == torch.float32 and x.planes.is_contiguous()
+        assert x.planes.shape[1:] == residual.shape and residual.device == x.planes.device
+    else:
+        assert x.y.dtype == torch.bfloat16 and x.y.is_contiguous()
+        assert x.y.shape == (rows * x.top, dim) and residual.device == x.y.device
+    assert weight.device == residual.device
+    lib, hip = _lib()
+    out = torch.empty_like(residual)
+    if isinstance(x, PlaneSum):
+        hip.check(lib.oa_add_rmsnorm_parts(
+            hip.current_stream_ptr(), x.planes.data_ptr(), x.planes.shape[0], residual.data_ptr(),
+            weight.data_ptr(), out.data_ptr(), rows, dim, eps), "oa_add_rmsnorm_parts")
+    else:
         hip.check(lib.oa_add_rmsnorm_pairs(
             hip.current_stream_ptr(), x.y.data_ptr(), x.top,
             x.more.data_ptr() if x.more is not None else None, residual.data_ptr(),
             weight.data_ptr(), out.data_ptr(), rows, dim, eps), "oa_add_rmsnorm_pairs")
-        return out, residual
+    return out
+
+
+def fused_add_rms_norm(
+    x: Union[torch.Tensor, PlaneSum, PairSum], residual: torch.Tensor, weight: torch.Tensor,
+    eps: float = 1e-5
+) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Returns (rmsnorm(x+residual), x+residual). GPU path updates `residual`
+    in place as the new residual stream and returns it. x may be a product's parts
+    (linear_parts) or a sum over pairs (moe_combine) that is not added up yet."""
+    if not isinstance(x, torch.Tensor):
+        if _is_gpu(residual):
+            return _add_norm_parts(x, residual, weight, eps), residual
+        x = _added_up(x)
     if not _is_gpu(x):
         return torch_ref.fused_add_rms_norm(x, residual, weight, eps)
-    if x.dim() == 3 and x.dtype == torch.float32:
-        parts, rows, dim = x.shape
-        assert x.is_contiguous() and residual.is_contiguous() and residual.shape == (rows, dim)
-        lib, hip = _lib()
-        out = torch.empty_like(residual)
-        hip.check(lib.oa_add_rmsnorm_parts(
-            hip.current_stream_ptr(), x.data_ptr(), parts, residual.data_ptr(),
-            weight.data_ptr(), out.data_ptr(), rows, dim, eps), "oa_add_rmsnorm_parts")
-        return out, residual
     assert x.dtype == torch.bfloat16 and x.is_contiguous() and residual.is_contiguous()
     lib, hip = _lib()
     rows = x.numel() // x.shape[-1]

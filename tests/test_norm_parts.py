@@ -19,7 +19,7 @@ def test_planes(parts, T, D):
     for s in range(1, parts):
         total += x[s]
     want, want_r = ops.fused_add_rms_norm(total.bfloat16(), residual.clone(), w, 1e-5)
-    got, got_r = ops.fused_add_rms_norm(x, residual, w, 1e-5)
+    got, got_r = ops.fused_add_rms_norm(ops.PlaneSum(x), residual, w, 1e-5)
     assert got_r.data_ptr() == residual.data_ptr() and torch.equal(got_r, want_r)
     # the sum of squares in another order: a result may round to the neighbour
     assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -7, atol=0)
@@ -91,11 +91,11 @@ def test_products(T, N, K):
     w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).bfloat16()
     y = ops.linear_parts(x, w)
     plan = 1 < T <= 128 and ops._ring_choice(T, N, K)
-    assert (y.dim() == 3) == bool(plan and plan[1] > 1)
-    if y.dim() == 3:
-        total = y[0].clone()
-        for s in range(1, y.shape[0]):
-            total += y[s]
+    assert isinstance(y, ops.PlaneSum) == bool(plan and plan[1] > 1)
+    if isinstance(y, ops.PlaneSum):
+        total = y.planes[0].clone()
+        for plane in y.planes[1:]:
+            total += plane
         y = total.bfloat16()
     assert torch.equal(y, ops.linear(x, w))
 
@@ -103,3 +103,30 @@ def test_products(T, N, K):
 def test_cpu_is_linear():
     x, w = torch.randn(8, 4096).bfloat16(), torch.randn(64, 4096).bfloat16()
     assert torch.equal(ops.linear_parts(x, w), ops.linear(x, w))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["planes", "pairs"])
+def test_what_the_norm_refuses(kind):
+    """Other types are refused as the plain norm refuses them, float32 planes that are not said to
+    be parts among them."""
+    T, D = 5, 2048
+    rn = lambda *s: torch.randn(*s, device="cuda")  # noqa: E731
+    if kind == "planes":
+        x, wrong = ops.PlaneSum(rn(3, T, D)), ops.PlaneSum(rn(3, T, D).bfloat16())
+    else:
+        x, wrong = ops.PairSum(rn(T * 2, D).bfloat16(), 2, None), ops.PairSum(rn(T * 2, D), 2, None)
+    residual, w = rn(T, D).bfloat16(), 1 + 0.1 * rn(D).bfloat16()
+    for args in [(x, residual.float(), w), (x, residual, w.float()), (wrong, residual, w),
+                 (x, residual[:4], w), (x, residual, w[:1024]), (x, residual.half(), w),
+                 (rn(3, T, D), residual, w), (rn(1, T, D), residual, w)]:
+        with pytest.raises(AssertionError):
+            ops.fused_add_rms_norm(*args)
+
+
+def test_planes_on_the_cpu():
+    x, residual, w = torch.randn(3, 4, 16), torch.randn(4, 16).bfloat16(), torch.rand(16).bfloat16()
+    total = ((x[0] + x[1]) + x[2]).bfloat16()
+    for got, want in zip(ops.fused_add_rms_norm(ops.PlaneSum(x), residual, w),
+                         ops.fused_add_rms_norm(total, residual, w)):
+        assert torch.equal(got, want)
