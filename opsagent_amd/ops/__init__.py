@@ -468,8 +468,9 @@ def _added_up(x: Union[PlaneSum, PairSum]) -> torch.Tensor:
 
 
 def _add_norm_parts(x: Union[PlaneSum, PairSum], residual: torch.Tensor, weight: torch.Tensor,
-                    eps: float) -> torch.Tensor:
-    """fused_add_rms_norm's first result from what is not added up yet."""
+                    eps: float) -> Optional[torch.Tensor]:
+    """fused_add_rms_norm's first result from what is not added up yet, None where the
+    kernels do not take the residual or the weight."""
     rows, dim = residual.shape
     assert residual.dtype == weight.dtype == torch.bfloat16 and weight.numel() == dim
     assert residual.is_contiguous() and weight.is_contiguous()
@@ -480,6 +481,8 @@ def _add_norm_parts(x: Union[PlaneSum, PairSum], residual: torch.Tensor, weight:
         assert x.y.dtype == torch.bfloat16 and x.y.is_contiguous()
         assert x.y.shape == (rows * x.top, dim) and residual.device == x.y.device
     assert weight.device == residual.device
+    if dim % 8 or dim > 8192 or (residual.data_ptr() | weight.data_ptr()) % 16:
+        return None
     lib, hip = _lib()
     out = torch.empty_like(residual)
     if isinstance(x, PlaneSum):
@@ -502,8 +505,9 @@ def fused_add_rms_norm(
     in place as the new residual stream and returns it. x may be a product's parts
     (linear_parts) or a sum over pairs (moe_combine) that is not added up yet."""
     if not isinstance(x, torch.Tensor):
-        if _is_gpu(residual):
-            return _add_norm_parts(x, residual, weight, eps), residual
+        out = _add_norm_parts(x, residual, weight, eps) if _is_gpu(residual) else None
+        if out is not None:
+            return out, residual
         x = _added_up(x)
     if not _is_gpu(x):
         return torch_ref.fused_add_rms_norm(x, residual, weight, eps)

@@ -124,6 +124,25 @@ def test_what_the_norm_refuses(kind):
             ops.fused_add_rms_norm(*args)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["planes", "pairs"])
+def test_operands_off_the_grid(kind):
+    """Residual and weight that do not start at a multiple of 16 bytes are taken, as the plain norm
+    takes them."""
+    T, D = 5, 2048
+    rn = lambda *s: torch.randn(*s, device="cuda")  # noqa: E731
+    x = (ops.PlaneSum(rn(3, T, D)) if kind == "planes"
+         else ops.PairSum(rn(T * 2, D).bfloat16(), 2, rn(T, D).bfloat16()))
+    residual, w = rn(T, D).bfloat16(), 1 + 0.1 * rn(D).bfloat16()
+    want, want_r = ops.fused_add_rms_norm(x, residual.clone(), w)
+    for at, aw in [(1, 0), (0, 1), (4, 4)]:
+        r = torch.empty(T * D + at, dtype=torch.bfloat16, device="cuda")[at:].view(T, D).copy_(residual)
+        v = torch.empty(D + aw, dtype=torch.bfloat16, device="cuda")[aw:].copy_(w)
+        got, got_r = ops.fused_add_rms_norm(x, r, v)
+        assert got_r.data_ptr() == r.data_ptr() and torch.equal(got_r, want_r)
+        assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -7, atol=0)    # as above
+
+
 def test_planes_on_the_cpu():
     x, residual, w = torch.randn(3, 4, 16), torch.randn(4, 16).bfloat16(), torch.rand(16).bfloat16()
     total = ((x[0] + x[1]) + x[2]).bfloat16()
