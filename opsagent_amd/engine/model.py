@@ -89,6 +89,8 @@ def _init_linear(gen: torch.Generator, out_f: int, in_f: int, dtype) -> torch.Te
 
 
 class Attention(nn.Module):
+    sums_parts = True           # see _sums_parts
+
     def __init__(self, spec: ModelSpec, dtype: torch.dtype, gen: torch.Generator):
         super().__init__()
         tp, rank = get_tp_size(), get_tp_rank()
@@ -196,6 +198,8 @@ class Attention(nn.Module):
 
 
 class DenseMLP(nn.Module):
+    sums_parts = True           # see _sums_parts
+
     def __init__(self, spec: ModelSpec, dtype: torch.dtype, gen: torch.Generator):
         super().__init__()
         tp, rank = get_tp_size(), get_tp_rank()
@@ -221,7 +225,18 @@ class DenseMLP(nn.Module):
         return tp_all_reduce((ops.linear_parts if parts else ops.linear)(act, self.down_w))
 
 
+def _sums_parts(module: nn.Module) -> bool:
+    """Whether a caller here may ask `module` for parts in place of hidden rows: it is one of the
+    classes that have them, as it is, and no forward hook sees what goes in or comes out."""
+    every = torch.nn.modules.module
+    return "sums_parts" in type(module).__dict__ and "forward" not in module.__dict__ and not (
+        module._forward_hooks or module._forward_pre_hooks
+        or every._global_forward_hooks or every._global_forward_pre_hooks)
+
+
 class DecoderLayer(nn.Module):
+    sums_parts = True           # see _sums_parts
+
     def __init__(self, spec: ModelSpec, dtype: torch.dtype, gen: torch.Generator):
         super().__init__()
         self.input_norm_w = nn.Parameter(
@@ -240,21 +255,25 @@ class DecoderLayer(nn.Module):
         else:
             self.mlp = DenseMLP(spec, dtype, gen)
 
-    def forward(self, x, residual, cos, sin, k_cache, v_cache, fb, normed=None):
-        """normed: the input norm of x, where the first layer's caller has it."""
+    def forward(self, x, residual, cos, sin, k_cache, v_cache, fb, normed=None, parts=False):
+        """normed: the input norm of x, where the first layer's caller has it. parts: the first
+        result may be left for the norm that follows to add up (ops.PlaneSum, ops.PairSum)."""
         if residual is None:
             residual = x
             h = ops.rms_norm(x, self.input_norm_w, self.eps) if normed is None else normed
         else:
             h, residual = ops.fused_add_rms_norm(x, residual, self.input_norm_w, self.eps)
         # the norm after a sublayer adds up its last product's parts (not what ranks add up)
-        parts = get_tp_size() == 1
-        a = self.attn(h, cos, sin, k_cache, v_cache, fb, parts)
-        h, residual = ops.fused_add_rms_norm(a, residual, self.post_norm_w, self.eps)
-        if self.is_moe_layer:
-            m = self.mlp(h, decode=fb.kind == "decode", parts=parts)
+        one = get_tp_size() == 1
+        if one and _sums_parts(self.attn):
+            a = self.attn(h, cos, sin, k_cache, v_cache, fb, True)
         else:
-            m = self.mlp(h, parts)
+            a = self.attn(h, cos, sin, k_cache, v_cache, fb)
+        h, residual = ops.fused_add_rms_norm(a, residual, self.post_norm_w, self.eps)
+        kw = {"decode": fb.kind == "decode"} if self.is_moe_layer else {}
+        if parts and one and _sums_parts(self.mlp):
+            kw["parts"] = True
+        m = self.mlp(h, **kw)
         return m, residual
 
     def fused_decode(self, residual, cos, sin, k_cache, v_cache, fb):
@@ -423,11 +442,12 @@ class LlamaForCausalLM(nn.Module):
             return ops.rms_norm(residual, self.final_norm_w, self.spec.rms_eps)
         x, normed = ops.embed_rms_norm(fb.input_ids, self.embed, self.layers[0].input_norm_w,
                                        self.spec.rms_eps)
-        residual = None
+        residual, parts = None, all(map(_sums_parts, self.layers))
         for i, layer in enumerate(self.layers):
+            more = (normed if i == 0 else None, True) if parts else ()
             x, residual = layer(
                 x, residual, self.rope_cos, self.rope_sin,
-                kv_caches[i][0], kv_caches[i][1], fb, normed if i == 0 else None,
+                kv_caches[i][0], kv_caches[i][1], fb, *more,
             )
         x, _ = ops.fused_add_rms_norm(x, residual, self.final_norm_w, self.spec.rms_eps)
         return x  # [T, hidden]

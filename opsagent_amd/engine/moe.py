@@ -25,6 +25,8 @@ from opsagent_amd.parallel import get_tp_rank, get_tp_size, tp_all_reduce
 
 
 class MoEMLP(nn.Module):
+    sums_parts = True           # see model._sums_parts
+
     def __init__(self, spec: ModelSpec, dtype: torch.dtype, gen: torch.Generator):
         super().__init__()
         tp, rank = get_tp_size(), get_tp_rank()

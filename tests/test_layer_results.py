@@ -1,0 +1,129 @@
+"""What the decoder's layers and their sublayers give and are given, where a caller or a hook looks
+at it: hidden rows, as if no norm added up the parts of the product before it."""
+
+import dataclasses
+
+import pytest
+import torch
+
+from opsagent_amd import ops
+from opsagent_amd.engine.config import get_model_spec
+from opsagent_amd.engine.model import DenseMLP, ForwardBatch, LlamaForCausalLM
+
+T, BLOCK = 6, 16
+
+
+def _model(moe=False):
+    spec = get_model_spec("llama3-tiny")
+    if moe:
+        spec = dataclasses.replace(spec, moe_num_experts=4, moe_top_k=2, moe_shared_experts=1,
+                                   moe_intermediate_size=64)
+    return LlamaForCausalLM(spec, torch.bfloat16, "cpu", 3)
+
+
+def _batch(model):
+    s = model.spec
+    pos = torch.arange(T, dtype=torch.int32)
+    fb = ForwardBatch(kind="prefill", input_ids=torch.arange(3, 3 + T), positions=pos, slot_mapping=pos,
+                      prefill_past_len=0, prefill_slot_gather=None)
+    cache = [tuple(torch.zeros(1, BLOCK, s.num_kv_heads, s.head_dim, dtype=torch.bfloat16) for _ in range(2))
+             for _ in range(s.num_layers)]
+    return fb, cache
+
+
+@pytest.fixture
+def parts(monkeypatch):
+    """Products in two planes where the caller takes them so; counts them."""
+    taken = []
+
+    def linear_parts(x, w):
+        taken.append(w)
+        k = x.shape[1] // 2
+        x, w = x.float(), w.float()
+        return ops.PlaneSum(torch.stack([x[:, :k] @ w[:, :k].T, x[:, k:] @ w[:, k:].T]))
+
+    monkeypatch.setattr(ops, "linear_parts", linear_parts)
+    return taken
+
+
+@pytest.mark.parametrize("where", ["attn", "mlp", "layer"])
+def test_hooks_see_hidden_rows(parts, where):
+    model = _model()
+    fb, cache = _batch(model)
+    want = model(fb, cache)
+    assert len(parts) == 2 * len(model.layers)
+    seen = []
+    for layer in model.layers:
+        at = layer if where == "layer" else getattr(layer, where)
+        at.register_forward_pre_hook(lambda m, args: seen.append(args[0]))
+        at.register_forward_hook(lambda m, args, out: seen.append(out[0] if where == "layer" else out))
+    before = len(parts)
+    got = model(fb, _batch(model)[1])
+    assert len(seen) == 2 * len(model.layers)
+    assert all(isinstance(x, torch.Tensor) and x.shape == (T, model.spec.hidden_size) for x in seen)
+    assert len(parts) - before == len(model.layers)            # the other sublayer's, as before
+    assert (got - want).norm() / want.norm() < 2e-2            # bf16, rounded at other places
+
+
+def test_a_hook_on_every_module(parts):
+    seen = []
+    model = _model()
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, a, out: seen.append(out))
+    try:
+        model(*_batch(model))
+    finally:
+        handle.remove()
+    assert not parts and len(seen) == 1 + 3 * len(model.layers)
+    assert not any(isinstance(x, (ops.PlaneSum, ops.PairSum)) for x in seen)
+
+
+def test_a_layer_by_itself(parts):
+    model = _model()
+    fb, cache = _batch(model)
+    x = model.embed[fb.input_ids]
+    for layer, (k, v) in zip(model.layers, cache):
+        m, residual = layer(x, None, model.rope_cos, model.rope_sin, k, v, fb)
+        assert isinstance(m, torch.Tensor) and m.shape == residual.shape == x.shape
+
+
+@pytest.mark.parametrize("how", ["module", "forward"])
+def test_sublayers_of_another_kind(parts, how):
+    """One that takes hidden rows alone stands in for a layer's MLP."""
+    class Double(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, x):
+            return 2 * self.inner(x)
+
+    model, ref = _model(), _model()
+    want = ref(*_batch(ref))
+    for layer in model.layers:
+        if how == "module":
+            layer.mlp = Double(layer.mlp)
+        else:
+            layer.mlp.forward = lambda x, mlp=layer.mlp: 2 * DenseMLP.forward(mlp, x)
+    got = model(*_batch(model))
+    for layer in ref.layers:
+        layer.mlp.down_w.mul_(2)
+    want = ref(*_batch(ref))
+    assert (got - want).norm() / want.norm() < 2e-2
+
+
+@pytest.mark.parametrize("hooked", [False, True])
+def test_experts_are_asked_for_parts(monkeypatch, hooked):
+    from opsagent_amd.engine.moe import MoEMLP
+
+    asked, real = [], MoEMLP.forward
+
+    def forward(self, x, decode=False, parts=False):
+        asked.append(parts)
+        return real(self, x, decode)
+
+    monkeypatch.setattr(MoEMLP, "forward", forward)
+    model = _model(moe=True)
+    if hooked:
+        model.layers[0].mlp.register_forward_hook(lambda m, args, out: None)
+    model(*_batch(model))
+    assert asked == [not hooked] + [True] * (len(model.layers) - 1)
