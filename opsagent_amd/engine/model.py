@@ -440,9 +440,13 @@ class LlamaForCausalLM(nn.Module):
                     kv_caches[i][0], kv_caches[i][1], fb,
                 )
             return ops.rms_norm(residual, self.final_norm_w, self.spec.rms_eps)
-        x, normed = ops.embed_rms_norm(fb.input_ids, self.embed, self.layers[0].input_norm_w,
-                                       self.spec.rms_eps)
+        # what goes into a layer that is looked at may change on the way: its norm is its own then
         residual, parts = None, all(map(_sums_parts, self.layers))
+        if parts:
+            x, normed = ops.embed_rms_norm(fb.input_ids, self.embed, self.layers[0].input_norm_w,
+                                           self.spec.rms_eps)
+        else:
+            x = F.embedding(fb.input_ids, self.embed)
         for i, layer in enumerate(self.layers):
             more = (normed if i == 0 else None, True) if parts else ()
             x, residual = layer(

@@ -127,3 +127,24 @@ def test_experts_are_asked_for_parts(monkeypatch, hooked):
         model.layers[0].mlp.register_forward_hook(lambda m, args, out: None)
     model(*_batch(model))
     assert asked == [not hooked] + [True] * (len(model.layers) - 1)
+
+
+@pytest.mark.parametrize("how", ["hook", "module"])
+def test_a_hook_before_the_first_layer(how):
+    """What it makes of the embeddings is what the layer normalizes and adds to."""
+    class Shifted(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, x, *args):
+            return self.inner(x + shift, *args)
+
+    model, ref = _model(), _model()
+    shift = torch.linspace(-1, 1, model.spec.hidden_size).bfloat16()
+    if how == "hook":
+        model.layers[0].register_forward_pre_hook(lambda m, args: (args[0] + shift, *args[1:]))
+    else:
+        model.layers[0] = Shifted(model.layers[0])
+    ref.embed.add_(shift)
+    assert torch.equal(model(*_batch(model)), ref(*_batch(ref)))
