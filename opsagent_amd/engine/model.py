@@ -225,13 +225,16 @@ class DenseMLP(nn.Module):
         return tp_all_reduce((ops.linear_parts if parts else ops.linear)(act, self.down_w))
 
 
+_every_module = torch.nn.modules.module        # holds the hooks that are common to all
+
+
 def _sums_parts(module: nn.Module) -> bool:
     """Whether a caller here may ask `module` for parts in place of hidden rows: it is one of the
     classes that have them, as it is, and no forward hook sees what goes in or comes out."""
-    every = torch.nn.modules.module
-    return "sums_parts" in type(module).__dict__ and "forward" not in module.__dict__ and not (
-        module._forward_hooks or module._forward_pre_hooks
-        or every._global_forward_hooks or every._global_forward_pre_hooks)
+    own = module.__dict__
+    return "sums_parts" in type(module).__dict__ and "forward" not in own and not (
+        own["_forward_hooks"] or own["_forward_pre_hooks"]
+        or _every_module._global_forward_hooks or _every_module._global_forward_pre_hooks)
 
 
 class DecoderLayer(nn.Module):
@@ -264,16 +267,16 @@ class DecoderLayer(nn.Module):
         else:
             h, residual = ops.fused_add_rms_norm(x, residual, self.input_norm_w, self.eps)
         # the norm after a sublayer adds up its last product's parts (not what ranks add up)
-        one = get_tp_size() == 1
-        if one and _sums_parts(self.attn):
-            a = self.attn(h, cos, sin, k_cache, v_cache, fb, True)
+        one, attn, mlp = get_tp_size() == 1, self.attn, self.mlp
+        if one and _sums_parts(attn):
+            a = attn(h, cos, sin, k_cache, v_cache, fb, True)
         else:
-            a = self.attn(h, cos, sin, k_cache, v_cache, fb)
+            a = attn(h, cos, sin, k_cache, v_cache, fb)
         h, residual = ops.fused_add_rms_norm(a, residual, self.post_norm_w, self.eps)
         kw = {"decode": fb.kind == "decode"} if self.is_moe_layer else {}
-        if parts and one and _sums_parts(self.mlp):
+        if parts and one and _sums_parts(mlp):
             kw["parts"] = True
-        m = self.mlp(h, **kw)
+        m = mlp(h, **kw)
         return m, residual
 
     def fused_decode(self, residual, cos, sin, k_cache, v_cache, fb):

@@ -430,7 +430,8 @@ def embed_rms_norm(ids: torch.Tensor, table: torch.Tensor, weight: torch.Tensor,
             and table.is_contiguous() and weight.is_contiguous()
             and ids.dim() == 1 and ids.is_contiguous()
             and ids.dtype in (torch.int64, torch.int32) and ids.device == table.device
-            and D % 8 == 0 and D <= 8192 and (table.data_ptr() | weight.data_ptr()) % 16 == 0):
+            and D % 8 == 0 and D <= 8192 and (table.data_ptr() | weight.data_ptr()) % 16 == 0
+            and table.shape[0] > 0):
         x = torch.nn.functional.embedding(ids, table)
         return x, rms_norm(x, weight, eps)
     lib, hip = _lib()
@@ -472,28 +473,27 @@ def _add_norm_parts(x: Union[PlaneSum, PairSum], residual: torch.Tensor, weight:
     """fused_add_rms_norm's first result from what is not added up yet, None where the
     kernels do not take the residual or the weight."""
     rows, dim = residual.shape
-    assert residual.dtype == weight.dtype == torch.bfloat16 and weight.numel() == dim
-    assert residual.is_contiguous() and weight.is_contiguous()
-    if isinstance(x, PlaneSum):
-        assert x.planes.dtype == torch.float32 and x.planes.is_contiguous()
-        assert x.planes.shape[1:] == residual.shape and residual.device == x.planes.device
-    else:
-        assert x.y.dtype == torch.bfloat16 and x.y.is_contiguous()
-        assert x.y.shape == (rows * x.top, dim) and residual.device == x.y.device
-    assert weight.device == residual.device
-    if dim % 8 or dim > 8192 or (residual.data_ptr() | weight.data_ptr()) % 16:
+    planes = isinstance(x, PlaneSum)
+    data, n = (x.planes, x.planes.shape[0]) if planes else (x.y, x.top)
+    assert data.shape == ((n, rows, dim) if planes else (rows * n, dim)) and weight.numel() == dim
+    assert residual.dtype == weight.dtype == torch.bfloat16 and data.dtype == (
+        torch.float32 if planes else torch.bfloat16)
+    assert data.get_device() == residual.get_device() == weight.get_device()
+    assert data.is_contiguous() and residual.is_contiguous() and weight.is_contiguous()
+    at, w = residual.data_ptr(), weight.data_ptr()
+    if dim % 8 or dim > 8192 or (at | w) % 16:
         return None
     lib, hip = _lib()
     out = torch.empty_like(residual)
-    if isinstance(x, PlaneSum):
+    if planes:
         hip.check(lib.oa_add_rmsnorm_parts(
-            hip.current_stream_ptr(), x.planes.data_ptr(), x.planes.shape[0], residual.data_ptr(),
-            weight.data_ptr(), out.data_ptr(), rows, dim, eps), "oa_add_rmsnorm_parts")
+            hip.current_stream_ptr(), data.data_ptr(), n, at, w, out.data_ptr(), rows, dim, eps),
+            "oa_add_rmsnorm_parts")
     else:
         hip.check(lib.oa_add_rmsnorm_pairs(
-            hip.current_stream_ptr(), x.y.data_ptr(), x.top,
-            x.more.data_ptr() if x.more is not None else None, residual.data_ptr(),
-            weight.data_ptr(), out.data_ptr(), rows, dim, eps), "oa_add_rmsnorm_pairs")
+            hip.current_stream_ptr(), data.data_ptr(), n,
+            x.more.data_ptr() if x.more is not None else None, at, w, out.data_ptr(), rows, dim, eps),
+            "oa_add_rmsnorm_pairs")
     return out
 
 

@@ -12,7 +12,7 @@
 // first layer, which the library walks token by token up to 16 of them (us, gather and
 // norm in a step of 8 rows of 4096: 7.7 + 4.4, of 16 of 2048 10.8 + 4.8; a step of 13
 // tokens through experts 590 -> 580, of 8 sequences 505 -> 502, of 47 885 -> 866). An id
-// outside the table, which the engine refuses before, reads nothing: its row is NaN.
+// outside the table, which the engine refuses before, gets a row of NaN.
 enum { RN_PLAIN, RN_ADD, RN_EMBED };
 template <int MODE, typename ID>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(
@@ -27,6 +27,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
     if (MODE == RN_EMBED) {
         from = ids[row];
         known = from >= 0 && from < vocab;
+        if (!known) from = 0;                        // loads behind a branch wait one by one
     }
     const uint4* xrow = x + from * D8;
     float v[4][8], sumsq = 0.0f;
@@ -35,7 +36,8 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
         const int c = k * 256 + threadIdx.x;
         if (c >= D8) break;
         const uint32_t nan = 0x7fc07fc0u;
-        const uint4 xv = MODE != RN_EMBED || known ? xrow[c] : make_uint4(nan, nan, nan, nan);
+        uint4 xv = xrow[c];
+        if (MODE == RN_EMBED && !known) xv = make_uint4(nan, nan, nan, nan);
         uint4 r;
         if (MODE == RN_ADD) r = residual[row * D8 + c];
 #pragma unroll
@@ -94,6 +96,7 @@ extern "C" int oa_embed_rmsnorm(void* stream, const void* table, const void* ids
                                 int64_t vocab, const void* w, void* residual, void* out, int rows,
                                 int dim, float eps) {
     if (rows < 1) return 0;
+    if (vocab < 1) return -102;
     if (((uintptr_t)table | (uintptr_t)residual | (uintptr_t)w | (uintptr_t)out) % 16 != 0) return -101;
     if (wide) return launch_rmsnorm<RN_EMBED, int64_t>(stream, table, residual, w, out, ids, vocab, rows, dim, eps);
     return launch_rmsnorm<RN_EMBED, int>(stream, table, residual, w, out, ids, vocab, rows, dim, eps);

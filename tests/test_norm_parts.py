@@ -42,7 +42,7 @@ def test_embedding_and_norm(T, D, dtype):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
 def test_ids_outside_the_table(dtype):
-    """Nothing is read for them: rows of NaN, the others as they are."""
+    """They get rows of NaN, the others are as they are."""
     table = torch.randn(300, 2056, device="cuda").bfloat16()
     w = torch.ones(2056, device="cuda").bfloat16()
     far = 2 ** 40 if dtype == torch.int64 else 2 ** 31 - 1
