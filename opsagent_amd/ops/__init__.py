@@ -875,15 +875,6 @@ def moe_sorted_wins(pairs: int, experts: int, fp8: bool, weights: int = 0) -> bo
     return pairs >= max(32, 3 * experts // 8) or heavy and pairs >= max(6, experts // 2)
 
 
-def _moe_tile_rows(pairs: int, experts: int, weights: int, fp8: bool) -> int:
-    """Rows of an expert tile for operands that a block holds one step ahead, by the pairs:
-    16 or 64 up to four rows an expert, 64 below 128 rows, 128 from there on."""
-    if pairs <= 4 * experts:
-        wide = not fp8 and experts * weights >= 2 ** 24 and (pairs < 64 or experts >= 64)
-        return 64 if wide else 16
-    return 64 if pairs < 128 * experts else 128
-
-
 def _moe_ring_rows(pairs: int, experts: int, weights: int, fp8: bool) -> int:
     """Rows of a tile of moe_sorted_mlp, by the rows that an expert has on average; weights
     is the size of one expert matrix. The same bits with any of them.
@@ -904,7 +895,7 @@ def _moe_ring_rows(pairs: int, experts: int, weights: int, fp8: bool) -> int:
         return 16
     if pairs <= (96 if small else 24) * experts:
         return 32
-    return 64 if small or fp8 else _moe_tile_rows(2 * pairs, experts, weights, fp8)
+    return 64 if small or fp8 or pairs < 64 * experts else 128
 
 
 def moe_sorted_ok(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, act=None) -> bool:

@@ -196,17 +196,6 @@ def test_mismatches_are_refused():
     assert not ops.moe_sorted_ok(x, w13.cpu(), w2) and not ops.moe_sorted_ok(x, w13, w2.cpu())
 
 
-def test_tile_rows():
-    """bf16 experts take wide tiles from the start, but for small matrices and for few
-    experts whose pairs may fill one tile more; fp8 ones from five rows an expert."""
-    rows = ops._moe_tile_rows
-    big, small = 1408 * 2048, 512 * 1024
-    assert [rows(p, 64, big, False) for p in (48, 256, 257, 8191, 8192)] == [64, 64, 64, 64, 128]
-    assert [rows(p, 64, big, True) for p in (48, 256, 257, 8191, 8192)] == [16, 16, 64, 64, 128]
-    assert [rows(p, 16, big, False) for p in (63, 64, 65)] == [64, 16, 64]
-    assert [rows(p, 16, small, False) for p in (48, 64, 65)] == [16, 16, 64]
-
-
 def test_ring_rows():
     """Tiles grow with the rows an expert has, later for small matrices; wide ones of 128
     rows are for bf16 alone."""
