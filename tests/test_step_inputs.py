@@ -37,10 +37,12 @@ def test_layout(chunks, max_blocks):
 @pytest.mark.gpu
 def test_queued_steps():
     """Forty decode steps of two traces, prompts among them: the same logits whether the host
-    waits after each step or never."""
+    waits after each step or never. In the run without waits the last steps are queued behind work
+    that keeps the GPU busy until the host has prepared all of them."""
     cfg = make_cfg()
     W = O.random_weights(cfg, 3)
     a, b = tokens_for(cfg, 60, 1), tokens_for(cfg, 50, 2)
+    work = torch.full((8192, 8192), 2.0 ** -13, dtype=torch.bfloat16, device="cuda")
 
     def run(wait):
         rp = TraceReplayer(build_engine(cfg, W, "bf16"))
@@ -48,11 +50,17 @@ def test_queued_steps():
         out.append(rp.step([{"id": "a", "tokens": a[20:21], "want": [0]},
                             {"id": "b", "tokens": b[:11], "want": [0, 10]}], []))
         for t in range(39):
+            if t == 9 and not wait:                  # captured by now, which waits by itself
+                for _ in range(200):                 # about 0.8 ms each
+                    torch.mm(work, work)
+                busy = torch.cuda.Event()
+                busy.record()
             out.append(rp.step([{"id": "a", "tokens": [a[21 + t]], "want": [0]},
                                 {"id": "b", "tokens": [b[11 + t]], "want": [0]}],
                                ["a", "b"] if t == 38 else []))
             if wait:
                 torch.cuda.synchronize()
+        assert wait or not busy.query()              # all thirty were queued
         return torch.cat(out).cpu()
 
     assert torch.equal(run(False), run(True))
