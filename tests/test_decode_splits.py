@@ -185,3 +185,45 @@ def test_copies_of_the_first_row(G, Hk, lens):
     assert (other[-2:].float() - want.float()).norm() / want.float().norm() < 2e-3
     assert lens[0] == 1 or not torch.equal(other[-1], got[0])
     assert lens[0] <= bs or not torch.equal(other[-2], got[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("G,Hk", [(4, 8), (8, 4), (1, 33)])
+def test_rows_that_are_nearly_copies(G, Hk):
+    """Rows with the first row's slot that differ from it in one thing alone (a query, the new key
+    or value of one key head, the length, the last page) are answered by themselves. The marks in
+    the workspace say which (row, key head) was taken for a copy; a copy's partial results stay as
+    they were before the launch."""
+    bs, B, n, nsplit = 32, 24, 700, 4
+    cos, sin = (t.cuda() for t in ops.rope_cos_sin(1024, D))
+    q, k, v, kc, vc, table, lens, slots = _case([n, 65], Hk, G, bs, seed=Hk)
+    at = torch.tensor([0, 1] + [0] * (B - 2), device="cuda")
+    q, k, v, table, lens, slots = (x[at].contiguous() for x in (q, k, v, table, lens, slots))
+    copied = torch.ones(B, Hk, dtype=torch.bool, device="cuda")
+    copied[:2] = False
+    q[3, Hk * G - 1, D - 1] += 1.0                    # last channel of the last head
+    copied[3, Hk - 1] = False
+    k[4, 1, 0] += 1.0
+    copied[4, 1] = False
+    v[5, 0, D - 1] += 1.0
+    copied[5, 0] = False
+    lens[6] -= 1                                      # its cached keys end before the shared slot
+    table[7, (n - 1) // bs] = table[1, 0]
+    copied[6:8] = False
+    ws = (torch.full((B * Hk * nsplit, G, D), 7.0, device="cuda"),
+          torch.full((B * Hk * nsplit, G, 2), 7.0, device="cuda"))
+    got = ops.attention_decode_rope(q, k, v, kc.clone(), vc.clone(), table, lens, cos, sin, slots,
+                                    workspace=ws, nsplit=nsplit)
+    marks = ws[1].view(B, Hk, nsplit, G, 2)[:, :, 0, :, 1]
+    assert torch.equal(marks == -1.0, copied[..., None].expand(B, Hk, G))
+    assert (ws[0].view(B, Hk, -1)[copied] == 7.0).all()
+
+    by_head = got.view(B, Hk, -1)
+    assert torch.equal(by_head[copied], by_head[0].expand(B, -1, -1)[copied])
+    for b in range(3, 8):
+        alone = [x[b : b + 1] for x in (q, k, v, table, lens, slots)]
+        want = ops.attention_decode_rope(*alone[:3], kc.clone(), vc.clone(), *alone[3:5], cos, sin,
+                                         alone[5], nsplit=nsplit).view(Hk, -1)
+        own = ~copied[b]                              # splits of other sizes: one bf16 rounding apart
+        diff = (by_head[b] - want)[own].float().norm() / want[own].float().norm()
+        assert diff < 2e-3 and not torch.equal(by_head[b][own], by_head[0][own])
