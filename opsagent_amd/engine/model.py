@@ -273,10 +273,12 @@ class DecoderLayer(nn.Module):
         else:
             a = attn(h, cos, sin, k_cache, v_cache, fb)
         h, residual = ops.fused_add_rms_norm(a, residual, self.post_norm_w, self.eps)
-        kw = {"decode": fb.kind == "decode"} if self.is_moe_layer else {}
-        if parts and one and _sums_parts(mlp):
-            kw["parts"] = True
-        m = mlp(h, **kw)
+        parts = parts and one and _sums_parts(mlp)
+        if self.is_moe_layer:
+            decode = fb.kind == "decode"
+            m = mlp(h, decode, True) if parts else mlp(h, decode=decode)
+        else:
+            m = mlp(h, True) if parts else mlp(h)
         return m, residual
 
     def fused_decode(self, residual, cos, sin, k_cache, v_cache, fb):
@@ -444,18 +446,17 @@ class LlamaForCausalLM(nn.Module):
                 )
             return ops.rms_norm(residual, self.final_norm_w, self.spec.rms_eps)
         # what goes into a layer that is looked at may change on the way: its norm is its own then
-        residual, parts = None, all(map(_sums_parts, self.layers))
-        if parts:
-            x, normed = ops.embed_rms_norm(fb.input_ids, self.embed, self.layers[0].input_norm_w,
+        layers, cos, sin = list(self.layers), self.rope_cos, self.rope_sin
+        residual, more, rest = None, (), ()
+        if all(map(_sums_parts, layers)):
+            x, normed = ops.embed_rms_norm(fb.input_ids, self.embed, layers[0].input_norm_w,
                                            self.spec.rms_eps)
+            more, rest = (normed, True), (None, True)
         else:
             x = F.embedding(fb.input_ids, self.embed)
-        for i, layer in enumerate(self.layers):
-            more = (normed if i == 0 else None, True) if parts else ()
-            x, residual = layer(
-                x, residual, self.rope_cos, self.rope_sin,
-                kv_caches[i][0], kv_caches[i][1], fb, *more,
-            )
+        for i, layer in enumerate(layers):
+            x, residual = layer(x, residual, cos, sin, kv_caches[i][0], kv_caches[i][1], fb, *more)
+            more = rest
         x, _ = ops.fused_add_rms_norm(x, residual, self.final_norm_w, self.spec.rms_eps)
         return x  # [T, hidden]
 
