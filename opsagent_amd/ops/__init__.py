@@ -267,51 +267,63 @@ def _ring_narrow(M: int, N: int, K: int, gateup: bool, wide) -> Optional[int]:
     """Column splits of the ring product in strips of 64 weight rows, two blocks a CU
     (ring_gemm.hip), None where strips of 128 (wide: their plan) or the other forms stay.
 
-    Measured over 40 weights at 3 to 64 rows, 1.5 GB of them in turn, us other / narrow. It
-    wants the CUs full: one round of half the blocks (12288 x 4096, M = 8 23.9 / 21.4 with
-    192), or rounds of 512 (gate-up 2 x 14336 x 4096, 8 45.0 / 40.3 with 448; 2 x 11008, 8 36.4
-    / 37.9 with 344). Weights under 10 MB end before it starts (2048 x 2048, 24 6.9 / 7.2), rows
-    under 2048 columns leave splits too short (4096 x 1408, 24 6.1 / 7.5), and wide weights of
-    many splits run as fast in one deep ring (8192 x 28672, 32 74.4 / 80.5; 10240 x 8192, 8 31.1
-    / 32.5). Gate-up pays twice for splits, and rows of 4 KiB start on the same channels (2 x
-    8192 x 2048, 24 15.3 / 15.7; 2 x 8192 x 3072 20.8 / 18.8); past 48 rows a strip of 128 reads
-    x half as often (2 x 14336 x 4096, 64 48.0 / 49.8; inside a model of 4096 x 14336 and 32000 x
-    4096 too both forms take the same). Up to 16 rows strips of skinny.hip are
-    the faster form for short rows (4096 x 4096, 8 9.1 / 9.8, 24 11.9 / 10.6; 32000 x 2048, 6
-    27.8 / 29.0) and the wide ring where it has splits of its own (16384 x 4096, 8 26.3 /
-    26.8). Splits of a multiple of 2048 columns start on the same channels, which the wide ring
-    mends by more of them (8192 x 4096, 24 15.1 / 17.2, 48 16.1 / 18.6; 4096 x 8192, 24 16.9 /
-    18.0; 4096 x 24576 37 / 44; but 4096 x 16384 30.7 / 28.9)."""
+    What decides is, in this order, how full the CUs are, how many columns a split has, and what
+    the other form is. Measured over 190 weights, 150 of them drawn, at 3 to 64 rows, 0.7 GB of
+    them in turn, us other / narrow:
+
+    One round of half the blocks (12288 x 4096, M = 8 24.6 / 20.7 with 192), or rounds of 512
+    (gate-up 2 x 14336 x 4096, 8 46.1 / 39.4 with 448; 2 x 11008, 8 37.8 / 39.4 with 344), and
+    against strips of 128 that fill them better no fewer (2 x 2816 x 3520, 24 15.4 / 15.8 with
+    176). Weights under 10 MB end before it starts (2048 x 2048, 24 6.9 / 7.2); wide weights of
+    many splits run as fast in one deep ring (8192 x 28672, 32 74.4 / 80.5).
+
+    Against strips of 128 in as many rounds it halves the splits or has none to add up: short
+    ones gain most (4096 x 4096, 24 12.0 / 10.4; 2 x 7704 x 1216, 24 .76 of the time). Above 32
+    rows eight waves a block carry those strips, and only splits of up to 1700 columns are better
+    here (4096 x 4096, 48 13.4 / 11.7; 4096 x 14336, 33 1.06 of the time; 7768 x 6208 1.13). Where
+    neither form splits it has nothing to save (28160 x 5632, 24 1.08, 48 1.16), but rows of 4 KiB
+    start on the same channels, which strips of half the height spread, wherever the weights lie
+    (32000 x 4096, 24 50.4 / 45.6, 48 49.5 / 46.7; 2 x 14336 x 4096, 32 on one card 40.3 / 41.2,
+    on another 48.4 / 42.8, inside a model 6 us more without). Splits of such a size start
+    together too, which more of them mend (8192 x 4096, 24 15.1 / 17.2; 4096 x 8192 16.9 / 18.0).
+
+    Strips of skinny.hip are the faster form of short rows: up to 16 rows (4096 x 4096, 8 9.1 /
+    9.8; 32000 x 2048, 6 27.8 / 29.0), up to 32 where columns of gate-up would be split (2 x 2560
+    x 1024, 24 1.35 of the time; 2 x 3072 x 1536 1.04) or rows of 4 KiB are cut to a few hundred
+    columns (3072 x 2048, 17 1.11, 24 1.01, 32 .93)."""
     if not 2 < M <= (64 if wide is None else 48) or K % 64 or N % 8:
         return None
     weights = (2 if gateup else 1) * N * K
     strips = -(-N // (32 if gateup else 64))
     splits = max(1, min(256 // strips, K // 256))
-    blocks = strips * splits
+    blocks, many = strips * splits, M > 32
     if blocks > 256:
         full = 0.84 * 512 * -(-blocks // 512)
     else:
-        full = (0.68 if splits == 1 or gateup else 0.85) * 256
+        full = 256 * (0.85 if splits > 1 and not gateup else 0.8 if wide and not many else 0.68)
     if blocks < full or weights < 5e6 or K >= 8192 and N >= 8192:
+        return None
+    if wide and (K % 2048 if wide[1] == 1 else many and K // splits > 1700):
         return None
     if gateup:
         if splits == 1 and K >= 3072 and weights >= 45e6:
-            ok = M <= 48
+            ok = M <= (48 if K < 8192 else 32)       # 2 x 6144 x 12288, 40 1.03 of the time
         elif M <= 16:
             ok = wide is None and K >= 4096 and weights < 24e6
         else:
-            ok = wide is None or weights < 24e6
+            ok = (wide is None or weights < 24e6) and (many or splits == 1 or K >= 2048)
     elif splits == 1:
         if M <= 16:
             ok = wide is None and weights >= 45e6 and (K >= 3072 or M >= 8)
         else:
-            ok = K >= 2048 and M <= 32 or K >= 4096 and strips <= 512 and blocks >= 0.9 * 256
+            ok = K >= 2048 and not many or K >= 4096 and strips <= 512 and blocks >= 0.9 * 256
     elif M <= 16:
         ok = K % (splits * 2048) != 0 and (K >= 5120 or K >= 3072 and weights >= 24e6)
     else:
-        # a square weight that the library is best at (2560 x 2560, 40 9.4 / 9.5, 64 13.8 / 10.6)
-        ok = K >= 2048 and not (wide is None and K >= N and 32 < M <= 48) and not (
-            wide and K % (splits * 2048) == 0)
+        # the library is the best form of a square weight in one of its rounds (2560 x 2560, 48
+        # 1.07 of the time)
+        ok = K >= (2048 if M > 24 or weights >= 1e7 else 2049) and not (
+            wide and K % (splits * 2048) == 0) and not (wide is None and K == N and 32 < M <= 48)
     return splits if ok else None
 
 

@@ -215,6 +215,12 @@ def test_narrow_plans():
     assert choice(32, 8192, 28672)[2] is False and choice(8, 16384, 4096)[2] is False
     assert choice(8, 32000, 4096) == (32, 1, True) and choice(48, 32000, 4096) == (64, 1, True)
     assert choice(24, 8192, 2048, True)[2] is False and choice(24, 8192, 3072, True) == (32, 1, True)
+    assert choice(24, 2560, 1024, True) is None and choice(40, 2560, 1024, True) == (64, 3, True)
+    assert choice(24, 2816, 3520, True)[2] is False            # 176 blocks beside 220
+    # as many rounds and nothing to add up; eight waves a block beside four
+    assert choice(24, 28160, 5632)[2] is choice(48, 31056, 4224)[2] is choice(33, 7768, 6208)[2] is False
+    assert choice(17, 3072, 2048) is None and choice(40, 3072, 2048) == (64, 5, True)
+    assert choice(40, 2560, 2560) is None and choice(40, 2048, 3584) == (64, 8, True)
     for gateup in (False, True):
         for K in (64, 640, 1408, 2048, 4096, 14336):
             for N in (8, 1024, 3072, 6144, 32000, 128256):
