@@ -676,12 +676,13 @@ def _ring_plan_fp8(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
 
 def _ring_choice_fp8(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
     """The ring's plan where it is faster than the tile product (fp8_moe.hip). Us, ring / tiles:
-    without splits its one block of four waves a CU falls behind with the rows (28672 x 4096,
-    M = 64 29.7 / 32.1, 96 32.9 / 32.0, 128 35.7 / 33.2; 16384 x 2048, 96 17.3 / 14.8; 4096 x 1024,
-    32 7.5 / 8.4, 48 8.7 / 8.4, 128 13.6 / 8.9); splits of short rows cost more than they fill
-    (3072 x 2048, 128 13.7 / 12.1, 200 14.9 / 12.1; 2048 x 2816, 128 13.8 / 14.5, 200 14.9 / 14.4;
-    4096 x 3072, 200 19.2 / 15.4), long rows do not (4096 x 14336, 512 48.7 / 67; 2048 x 8192, 512
-    23.2 / 37.3)."""
+    without splits its one block a CU, of eight waves above 32 rows, falls behind with the rows,
+    sooner with short ones (4096 x 1024, 32 7.8 / 8.0, 48 8.4 / 8.2, 128 11.6 / 8.7; 16384 x 2048,
+    64 13.0 / 13.5, 80 15.2 / 14.0, 128 17.7 / 15.5; 28672 x 4096, 64 29.1 / 31.7, 80 30.9 / 31.8,
+    96 31.2 / 31.8, 128 33.0 / 33.0): 80 rows lie between. Splits of short rows cost more than they
+    fill (3072 x 2048, 80 11.0 / 11.5, 128 13.1 / 11.9, 200 14.5 / 11.8; 2048 x 2816, 128 13.2 /
+    14.3, 200 14.4 / 14.3; 4096 x 3072, 200 18.7 / 17.9), long rows do not (4096 x 14336, 512 47.8
+    / 67; 2048 x 8192, 512 22.7 / 38.5)."""
     plan = _ring_plan_fp8(M, N, K)
     if plan and (M > (32 if K < 2048 else 80) if plan[1] == 1
                  else K < 4096 and M > 128 and M * N >= 390000):
