@@ -663,10 +663,10 @@ class LLMEngine:
         ):
             hidden = self._mixed_decode_graphed(ids, chunks)
         else:
-            sb = SeqBatch.build(chunks, self.block_size, self.device)
+            sb = SeqBatch.build(chunks, self.block_size, self.device, wait=False)
             fb = ForwardBatch(
                 kind="mixed",
-                input_ids=to_device(torch.tensor(ids, dtype=torch.int64), self.device),
+                input_ids=to_device(torch.tensor(ids, dtype=torch.int64), self.device, wait=False),
                 positions=None,
                 slot_mapping=sb.slot_mapping,
                 seq_batch=sb,
@@ -794,7 +794,7 @@ class LLMEngine:
         if batch:
             if rows != list(range(len(hidden))):
                 hidden = hidden.index_select(0, to_device(torch.tensor(rows, dtype=torch.int64),
-                                                          self.device))
+                                                          self.device, wait=False))
             self._sample_and_append(batch, self.model.compute_logits(hidden))
         self._reap()
         self.perf.record_metric("engine_mixed_step_ms", (time.perf_counter() - t0) * 1000.0)

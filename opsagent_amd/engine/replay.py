@@ -60,7 +60,7 @@ class TraceReplayer:
             hidden = eng._forward_mixed(work)
             if rows:
                 if rows != list(range(len(hidden))):
-                    idx = to_device(torch.tensor(rows, dtype=torch.int64), eng.device)
+                    idx = to_device(torch.tensor(rows, dtype=torch.int64), eng.device, wait=False)
                     hidden = hidden.index_select(0, idx)
                 logits = eng.model.compute_logits(hidden).float()
         for rid in end:

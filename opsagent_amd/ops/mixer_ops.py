@@ -22,11 +22,12 @@ import torch
 from opsagent_amd.ops import torch_ref
 
 
-def to_device(host: torch.Tensor, device) -> torch.Tensor:
+def to_device(host: torch.Tensor, device, wait: bool = True) -> torch.Tensor:
     """host on the device. A copy from ordinary memory waits for all work before it on the
-    stream; from pinned memory, which its allocator holds until the copy is done, it does not,
-    so that the host prepares a step while the GPU is at the one before."""
-    if torch.device(device).type != "cuda":
+    stream, after which any stream may read it. Without `wait` it comes from pinned memory, which
+    its allocator holds until the copy is done: the host prepares a step while the GPU is at the
+    one before, and the tensor is for the current stream alone."""
+    if wait or torch.device(device).type != "cuda":
         return host.to(device)
     return host.pin_memory().to(device, non_blocking=True)
 
@@ -59,8 +60,8 @@ class SeqBatch:
 
     @staticmethod
     def build(chunks: List[Tuple[int, int, int, List[int]]], block_size: int,
-              device, max_blocks: Optional[int] = None) -> "SeqBatch":
-        """chunks: per sequence (past_len, count, state_slot, block ids)."""
+              device, max_blocks: Optional[int] = None, wait: bool = True) -> "SeqBatch":
+        """chunks: per sequence (past_len, count, state_slot, block ids). wait: see to_device."""
         cu, past, slots = [0], [], []
         nb = max((len(c[3]) for c in chunks), default=1)
         max_blocks = max(max_blocks or 0, nb, 1)
@@ -79,7 +80,7 @@ class SeqBatch:
             pos = np.arange(p, p + n)
             host[o3 + cu[b] : o3 + cu[b + 1]] = b
             host[o4 + cu[b] : o4 + cu[b + 1]] = row[pos // block_size] * block_size + pos % block_size
-        flat = to_device(torch.from_numpy(host), device)
+        flat = to_device(torch.from_numpy(host), device, wait)
         return SeqBatch(
             cu=cu, past=past, slots=slots, cu_t=flat[:o1], past_t=flat[o1:o2],
             slots_t=flat[o2:o3], seq_of_t=flat[o3:o4], slot_mapping=flat[o4:o5],

@@ -64,3 +64,33 @@ def test_queued_steps():
         return torch.cat(out).cpu()
 
     assert torch.equal(run(False), run(True))
+
+
+@pytest.mark.gpu
+def test_inputs_for_any_stream():
+    """What a caller builds is on the device when it has it: another stream reads it at once, though
+    the current one is busy. Without the wait the host is back before the copy."""
+    work = torch.full((8192, 8192), 2.0 ** -13, dtype=torch.bfloat16, device="cuda")
+    side = torch.cuda.Stream()
+    blocks = list(range(1, 9))
+
+    def build(**kw):
+        for _ in range(40):                          # about 0.8 ms each
+            torch.mm(work, work)
+        busy = torch.cuda.Event()
+        busy.record()
+        return mx.SeqBatch.build([(5, 200, 3, blocks)], 32, "cuda", **kw), busy
+
+    for kw in (dict(wait=False), {}):                # the first round loads and allocates
+        sb, busy = build(**kw)
+        torch.cuda.synchronize()
+    sb, busy = build(wait=False)
+    assert not busy.query()
+    torch.cuda.synchronize()
+    sb, _ = build()
+    with torch.cuda.stream(side):
+        got = [t.cpu() for t in (sb.cu_t, sb.past_t, sb.slots_t, sb.block_table, sb.slot_mapping)]
+    want = mx.SeqBatch.build([(5, 200, 3, blocks)], 32, "cpu")
+    for g, w in zip(got, (want.cu_t, want.past_t, want.slots_t, want.block_table, want.slot_mapping)):
+        assert torch.equal(g, w)
+    torch.cuda.synchronize()
