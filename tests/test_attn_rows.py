@@ -117,6 +117,7 @@ def test_rows(monkeypatch, splits, ctx, H, G, D, page, opts):
     (4, 1, [(0, 17), (63, 2), (100, 64)], 32, dict(slopes=True)),
     (6, 3, [(0, 130), (5, 1)], 8, dict(window=33, keep=5, sinks=True)),   # pages below a tile's 64 keys
     (3, 1, [(190, 3)], 64, dict(softcap=20.0, gate="heads")),
+    (40, 2, [(300, 1), (16, 1), (0, 1)], 32, dict(slopes=True, sinks=True)),   # heads in the columns
 ])
 def test_prompts(D, H, G, chunks, page, opts):
     """The tile kernel at the head sizes that it is built for, against 64 bits."""
