@@ -38,3 +38,21 @@ def test_masked_argmax(V, masked):
         ok = allow[b] & ~x[b].isnan() & (x[b] != -float("inf"))
         v = torch.where(ok, x[b].float(), torch.tensor(-float("inf")))
         assert got[b] == (int((v == v.max()).nonzero()[0]) if ok.any() else -1), b
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("V", [8, 8200])
+def test_signaling_nan(V, masked):
+    """It is never chosen and hides no other token, whatever its place in a group of 8."""
+    x = torch.full((4, V), -1.0, dtype=torch.bfloat16)
+    bits = x.view(torch.int16)
+    bits[0] = 0x7f81
+    x[0, 5] = -3.0
+    bits[1, 0], bits[1, 6] = 0x7f81, 0x7fa0
+    x[1, 7] = 2.0
+    bits[2, 3], bits[2, 7] = -0x7f, 0x7fbf            # 0xff81: the sign set
+    x[2, 4] = 5.0
+    bits[3] = 0x7f81
+    words = torch.full((4, (V + 31) // 32), -1, dtype=torch.int32, device="cuda") if masked else None
+    assert ops.greedy_sample_masked(x.cuda(), words).tolist() == [5, 7, 4, -1]
