@@ -13,6 +13,7 @@ attention, activation, sampling) are the HIP kernels here.
 
 from __future__ import annotations
 
+import functools
 import os
 from typing import NamedTuple, Optional, Tuple, Union
 
@@ -327,14 +328,24 @@ def _ring_narrow(M: int, N: int, K: int, gateup: bool, wide) -> Optional[int]:
     return splits if ok else None
 
 
-def _ring_choice(M: int, N: int, K: int, gateup: bool = False):
-    """(rows of a tile, column splits, whether in strips of 64 weight rows) of the product on
-    the transfer ring, None where the other forms are faster."""
+@functools.lru_cache(maxsize=4096)
+def _ring_sizes(M: int, N: int, K: int, gateup: bool):
     wide = _ring_plan(M, N, K, gateup)
     splits = _ring_narrow(M, N, K, gateup, wide)
     if splits:
         return 32 * -(-M // 32), splits, True
     return wide and (*wide, False)
+
+
+def _ring_choice(M: int, N: int, K: int, gateup: bool = False):
+    """(rows of a tile, column splits, whether in strips of 64 weight rows) of the product on
+    the transfer ring, None where the other forms are faster. The sizes alone decide, so that
+    the rules are gone through once for each (2 to 3 us, 17 times in a prompt of four layers,
+    which up to some tens of rows takes as long as its host), but for two rows, where a switch
+    has a say."""
+    if M == 2:
+        return _ring_sizes.__wrapped__(M, N, K, gateup)
+    return _ring_sizes(M, N, K, gateup)
 
 
 def _ring(x: torch.Tensor, w: torch.Tensor, plan: Tuple[int, ...], act: int = 0,

@@ -228,3 +228,15 @@ def test_narrow_plans():
                     plan = choice(M, N, K, gateup)
                     if plan and plan[2]:
                         assert 2 < M <= plan[0] <= 64 and 1 <= plan[1] <= K // 64
+
+
+def test_choices_are_those_of_the_rules(monkeypatch):
+    """Asked again, a size is answered as the rules answer it; two rows follow the GEMV switch."""
+    for gateup in (False, True):
+        for N, K in ((3072, 2048), (4096, 14336), (14336, 4096), (1408, 2048), (7, 64)):
+            for M in (1, 2, 3, 16, 47, 64, 65, 128, 129):
+                fresh = ops._ring_sizes.__wrapped__(M, N, K, gateup)
+                assert ops._ring_choice(M, N, K, gateup) == ops._ring_choice(M, N, K, gateup) == fresh
+    before = ops._ring_choice(2, 6144, 4096)
+    monkeypatch.setenv("OPSAGENT_GEMV_MAX_M", "1")
+    assert before is None and ops._ring_choice(2, 6144, 4096)[:2] == ops._ring_plan(2, 6144, 4096)
