@@ -38,8 +38,12 @@ class TraceReplayer:
         `want` order, or None if nothing is wanted."""
         eng = self.engine
         work, rows, off = [], [], 0
-        for e in entries:
-            toks = [int(t) for t in e["tokens"]]
+        given = [[int(t) for t in e["tokens"]] for e in entries]
+        for e, toks in zip(entries, given):
+            if toks and not 0 <= min(toks) <= max(toks) < eng.spec.vocab_size:
+                raise ValueError(f"{e['id']}: token ids lie outside the model's vocabulary of "
+                                 f"{eng.spec.vocab_size}")
+        for e, toks in zip(entries, given):
             if not toks:
                 continue
             req = self.live.get(e["id"])

@@ -34,6 +34,21 @@ def test_layout(chunks, max_blocks):
     assert sb.max_total == max([c[0] + c[1] for c in chunks], default=0)
 
 
+@pytest.mark.parametrize("bad", [-1, 10 ** 6])
+def test_traces_stay_in_the_vocabulary(bad):
+    """A token outside the table is refused before any sequence of the step has its tokens; the
+    trace goes on without."""
+    cfg = make_cfg()
+    rp = TraceReplayer(build_engine(cfg, O.random_weights(cfg, 3), "fp32"))
+    toks = tokens_for(cfg, 12, 1)
+    rp.step([{"id": "a", "tokens": toks[:5]}], [])
+    with pytest.raises(ValueError, match="vocabulary"):
+        rp.step([{"id": "a", "tokens": [toks[5]]}, {"id": "c", "tokens": [toks[0], bad]}], [])
+    got = rp.step([{"id": "a", "tokens": toks[5:], "want": [0]}], ["a"])
+    want = TraceReplayer(rp.engine).step([{"id": "b", "tokens": toks, "want": [5]}], ["b"])
+    assert torch.allclose(got, want, rtol=1e-4, atol=1e-4)
+
+
 @pytest.mark.gpu
 def test_queued_steps():
     """Forty decode steps of two traces, prompts among them: the same logits whether the host
