@@ -368,11 +368,56 @@ def _ring(x: torch.Tensor, w: torch.Tensor, plan: Tuple[int, ...], act: int = 0,
     return part if parts else out
 
 
+@functools.lru_cache(maxsize=4096)
+def _tile_sizes(M: int, N: int, K: int, gateup: bool, summed: bool) -> Optional[int]:
+    weights = N * K * (2 if gateup else 1)
+    if summed and K < 2 * N:             # deep products split, others hardly
+        return None
+    if weights < (2 ** 22 if gateup or summed or M >= 500 else 9e6) or (
+            M >= 3500 and not gateup):
+        return None
+    plan = _lib()[0].oa_tile_gemm_plan(M, N, K, int(gateup), int(summed))
+    return plan if plan >= 0 else None
+
+
+def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = False) -> Optional[int]:
+    """Form and column splits of the tile product (tile_gemm.hip; figures and the rule by sizes
+    there) of more than 128 rows, None where the library is faster: light weights at few rows (us,
+    library / tiles: 2048 x 2048, 256 rows 10.1 / 13.0, 800 15.3 / 14.5; deep ones with a norm behind
+    them split, 1024 x 4096, 338 16.9 / 15.0), and from some thousand rows on, where power bounds
+    both (4096 x 4096, 4067 92 / 103, 2900 79 / 78), but for gate-up, whose activation rides along.
+    Over 3200 products of the models' weights and of 512 to 16000 x 512 to 14336, 129 to 6000 rows,
+    those taken are 1.17 times as fast as the library on average (gate-up 1.2), one in twenty up to
+    1.1 times slower. summed: for linear_parts, where a norm adds up the splits."""
+    return _tile_sizes(M, N, K, gateup, summed) if M > 128 else None
+
+
+def _tile(x: torch.Tensor, w: torch.Tensor, plan: int, act: int = 0,
+          parts: bool = False) -> torch.Tensor:
+    """x @ w^T, or act 1 (silu), 2 (tanh gelu) of the gate rows times the up rows, in the form
+    and splits of plan. parts: the float32 parts of a split product, as of _ring."""
+    lib, hip = _lib()
+    K, splits = x.shape[-1], plan & 255
+    M, N = x.numel() // K, w.shape[0] // (2 if act else 1)
+    out = None if parts else torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
+    # at most 256 tiles of 256 x 256 float32: 67 MB
+    part = None if splits == 1 else torch.empty(splits, M, N, dtype=torch.float32, device=x.device)
+    hip.check(lib.oa_tile_gemm(hip.current_stream_ptr(), x.data_ptr(),
+                               K if x.is_contiguous() else x.stride(0), w.data_ptr(),
+                               None if parts else out.data_ptr(),
+                               None if part is None else part.data_ptr(), M, N, K, plan, act),
+              "oa_tile_gemm")
+    return part if parts else out
+
+
 def linear_parts(x: torch.Tensor, w: torch.Tensor) -> Union[torch.Tensor, PlaneSum]:
     """x @ w^T for rows x [T, K] that go through fused_add_rms_norm next: bf16 [T, N], or the
     product's float32 column parts, which the norm adds up, where the transfer ring splits it."""
     M = x.numel() // x.shape[-1]
-    if 1 < M <= 128 and x.dim() == 2 and w.shape[0] <= 8192 and _skinny_ok(x, w):
+    if M > 1 and x.dim() == 2 and w.shape[0] <= 8192 and _skinny_ok(x, w):
+        if M > 128:
+            tile = _tile_choice(M, w.shape[0], w.shape[1], summed=True)
+            return PlaneSum(_tile(x, w, tile, parts=True)) if tile and tile & 255 > 1 else linear(x, w)
         plan = _ring_choice(M, w.shape[0], w.shape[1])
         if plan and plan[1] > 1:
             return PlaneSum(_ring(x, w, plan, parts=True))
@@ -384,7 +429,8 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     (hipBLASLt's M=1 kernels run ~2.5x off the HBM roofline on gfx950), the transfer
     ring up to 128 rows and the skinny matrix-core products up to 32 where they win
     (_ring_choice, _skinny_form), the VALU GEMV for what two rows are left and the
-    matrix-core GEMV for what 3 to 8 are; everything else goes to hipBLASLt."""
+    matrix-core GEMV for what 3 to 8 are, the tile product for more than 128 (_tile_choice);
+    everything else goes to hipBLASLt."""
     M = x.numel() // x.shape[-1]
     if 1 < M <= 128 and _skinny_ok(x, w):
         plan = _ring_choice(M, w.shape[0], w.shape[1])
@@ -393,6 +439,10 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         form = _skinny_form(M, w.shape[0], w.shape[1], strided=not x.is_contiguous())
         if form:
             return _skinny(x, w, form)
+    if M > 128 and _skinny_ok(x, w):
+        plan = _tile_choice(M, w.shape[0], w.shape[1])
+        if plan is not None:
+            return _tile(x, w, plan)
     if (
         x.is_cuda
         and x.dtype == torch.bfloat16
@@ -1122,7 +1172,8 @@ def gateup_silu(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> torch
 
 def _gateup_form(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int):
     """What takes this product in one launch, None if nothing does: ("ring", plan) and
-    ("skinny", form), the transfer ring and the skinny matrix-core product where they win;
+    ("skinny", form), the transfer ring and the skinny matrix-core product where they win,
+    ("tile", plan), the tile product of more than 128 rows;
     ("staged", None), the VALU GEMV up to two rows and the staged matrix-core GEMV for what
     3 to 8 rows are left."""
     K = x.shape[-1]
@@ -1130,6 +1181,9 @@ def _gateup_form(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int):
     if not (x.is_cuda and x.dtype == torch.bfloat16 and K % 8 == 0 and x.is_contiguous()
             and gate_up_w.is_contiguous()):
         return None
+    if M > 128 and _skinny_ok(x, gate_up_w) and gate_up_w.shape[0] == 2 * i_local:
+        plan = _tile_choice(M, i_local, K, gateup=True)
+        return None if plan is None else ("tile", plan)
     if 1 < M <= 128 and _skinny_ok(x, gate_up_w) and gate_up_w.shape[0] == 2 * i_local:
         plan = _ring_choice(M, i_local, K, gateup=True)
         if plan:
@@ -1160,6 +1214,8 @@ def gateup_act(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int,
         return _ring(x, gate_up_w, plan, act=1 + int(act == "gelu_tanh"))
     if kind == "skinny":
         return _skinny(x, gate_up_w, plan, gateup=True, act=int(act == "gelu_tanh"))
+    if kind == "tile":
+        return _tile(x, gate_up_w, plan, act=1 + int(act == "gelu_tanh"))
     lib = hip_lib.get_lib()
     out = torch.empty(*x.shape[:-1], i_local, dtype=x.dtype, device=x.device)
     rc = lib.oa_gemv_gateup_act(

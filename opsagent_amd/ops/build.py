@@ -28,6 +28,7 @@ SOURCES = [
     "moe_grouped.hip",
     "skinny.hip",
     "ring_gemm.hip",
+    "tile_gemm.hip",
 ]
 
 # the sequence-mixer kernels of hybrid decoders live in a library of their

@@ -75,6 +75,12 @@ __device__ __forceinline__ void lds_transfer16(uint32_t lds, const char* src) {
                      : : "s"(lds), "v"(src) : "memory");
 }
 
+// the same from a uniform base and a lane's offset
+__device__ __forceinline__ void lds_transfer16(uint32_t lds, uint32_t off, const char* base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 : : "s"(lds), "v"(off), "s"(base) : "memory");
+}
+
 // ---- wave reductions --------------------------------------------------------
 __device__ __forceinline__ float wave_reduce_sum(float v) {
 #pragma unroll

@@ -264,6 +264,17 @@ __global__ __launch_bounds__(256) void ring_sum_kernel(const float* __restrict__
         make_uint2(pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]));
 }
 
+// out [M, N] = the sum of parts [splits, M, N], in order
+extern "C" int oa_ring_sum(void* stream, const void* part, void* out, int M, int N, int splits) {
+    if (M < 1 || M > 65535 || N < 4 || N % 4 != 0 || splits < 1 || !part || !out) return -100;
+    if (((uintptr_t)part | (uintptr_t)out) % 16 != 0) return -102;
+    hipLaunchKernelGGL((ring_sum_kernel<false, false>), dim3(CEIL_DIV(N / 4, 256), M), dim3(256), 0,
+                       (hipStream_t)stream, (const float*)part, (const float*)nullptr,
+                       (const float*)nullptr, (uint16_t*)out, M, N, splits, 0);
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
 // out [M, N] = x [M, K] w [N, K]^T, x rows xs elements apart. act 1 (silu), 2 (tanh gelu):
 // out = act(x w[:N]^T) * (x w[N:]^T), w [2 N, K]. bm: rows of a tile, 32, 64, 96 or 128;
 // narrow: strips of 64 weight rows (bm 32 and 64).

@@ -1,0 +1,472 @@
+// Products of more than 128 rows: C[M, N] = x[M, K] W[N, K]^T in bf16, plain, gate-up with its
+// activation, or as float32 column parts.
+//
+// Three things bound them, measured apart on 2048 x 8192 x 4096 in tiles of 256 x 256. The matrix
+// cores take 1.05 us a step of 64 columns on random operands that LDS feeds (1.75 PFLOP/s; 2.4 on
+// zeros: power, not issue). The LDS reads of a step take 0.64 us. And the transfers into LDS stop at
+// 64 KB under way a CU, whatever the depth of the ring: 150 GB/s a CU from the L2, 110 where x and
+// W lie in the cache before memory, 65 where W comes from memory, which is 1 us a step. So small
+// tiles are bound by transfers (128 x 128 runs at 1.3 PFLOP/s without them, at 0.9 with) and large
+// ones by power, and what is won lies in tiles that fill the CUs. Two groups of four waves, a wave of
+// each on every SIMD, therefore take turns: while one reads its fragments from LDS and sends for a
+// later step, the other multiplies; a barrier ends each phase. Us, the library (gate-up: and the
+// activation kernel) / here (splits: and the sum): 4096 x 14336, M = 130 55 / 36, 512 91 / 67, 800
+// 124 / 94, 2048 206 / 183; 4096 x 4096, 800 39 / 34, 2048 59 / 56; 6144 x 4096, 130 40 / 24, 700 49 /
+// 41, 2048 82 / 84; 2048 x 8192, 256 28 / 24, 1024 50 / 48, 2048 72 / 68; gate-up 2 x 14336 x 4096, 130
+// 63 / 58, 800 189 / 167, 2048 391 / 366; 2 x 2816 x 2048, 512 29 / 22, 1434 52 / 35.
+// Slower: transfers in turn with the LDS reads or between the products; four waves of 128 x 128 (the
+// compiler copies sums between register files); v_mfma_f32_32x32x16_bf16 (1.6 PFLOP/s from LDS);
+// touching the lines of later steps (results come in order: it waits behind them).
+#include <algorithm>
+
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(4))) float tgf4;
+typedef __attribute__((ext_vector_type(8))) short tgs8;
+
+template <int V>
+__device__ __forceinline__ void tg_wait() {
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(V) : "memory");
+}
+
+__device__ __forceinline__ void tg_read_done() {
+    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+}
+
+__device__ __forceinline__ void tg_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_barrier" : : : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+__device__ __forceinline__ float tg_gate(float g, float u, int act) {
+    if (act == 2) {
+        const float t = 0.7978845608028654f * fmaf(0.044715f * g * g, g, g);
+        return 0.5f * g * (1.0f + tanhf(t)) * u;
+    }
+    return g / (1.0f + __expf(-g)) * u;
+}
+
+// the weight row (from the strip's first on) that LDS row b of the strip holds: a wave's fragments in
+// pairs whose lanes hold eight neighbouring outputs together, gate rows beside their up rows
+template <int FJ, bool GU>
+__device__ __forceinline__ int tg_wrow(int b) {
+    static_assert(FJ % 2 == 0, "pairs");
+    const int wv = b / (16 * FJ), j = b / 16 % FJ, r = b & 15;
+    if (GU) {
+        if (FJ % 4 == 0) return wv * FJ * 8 + (j >> 2) * 32 + (r >> 2) * 8 + (j & 1) * 4 + (r & 3);
+        return wv * FJ * 8 + (j >> 1) * 16 + r;
+    }
+    return wv * FJ * 16 + (j >> 1) * 32 + (r >> 2) * 8 + (j & 1) * 4 + (r & 3);
+}
+template <int FJ, bool GU>
+__device__ __forceinline__ bool tg_isup(int b) {
+    const int j = b / 16 % FJ;
+    return GU && (FJ % 4 == 0 ? (j >> 1 & 1) : (j & 1));
+}
+
+// fragments I0 .. I1 of a wave whose first row is row0
+template <int FI, int FJ, bool GU, int I0, int I1>
+__device__ __forceinline__ void tg_store(const tgf4 (&acc)[FI][FJ], uint16_t* out, float* part, int row0,
+                                         int n0, int wc, int M, int N, int sp, int act) {
+    const int fr = threadIdx.x & 15, fc = threadIdx.x >> 4 & 3;
+    // D: column (row of x) lane & 15, rows (weight rows) (lane >> 4) * 4 and up
+#pragma unroll
+    for (int i = I0; i < I1; ++i) {
+        const int row = row0 + i * 16 + fr;
+        if (row >= M) continue;
+        if (GU) {
+#pragma unroll
+            for (int j = 0; j < FJ; j += (FJ % 4 == 0 ? 4 : 2)) {
+                constexpr int V = FJ % 4 == 0 ? 2 : 1;
+                const int col = n0 + wc * FJ * 8 + (V == 2 ? (j >> 2) * 32 + fc * 8 : (j >> 1) * 16 + fc * 4);
+                if (col >= N) continue;
+                uint32_t o[2 * V];
+#pragma unroll
+                for (int v = 0; v < V; ++v)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        o[v * 2 + e] = pack_bf16x2(tg_gate(acc[i][j + v][2 * e], acc[i][j + V + v][2 * e], act),
+                                                   tg_gate(acc[i][j + v][2 * e + 1], acc[i][j + V + v][2 * e + 1], act));
+                if constexpr (V == 2)
+                    *reinterpret_cast<uint4*>(out + (size_t)row * N + col) = make_uint4(o[0], o[1], o[2], o[3]);
+                else
+                    *reinterpret_cast<uint2*>(out + (size_t)row * N + col) = make_uint2(o[0], o[1]);
+            }
+            continue;
+        }
+#pragma unroll
+        for (int j = 0; j < FJ; ++j) {
+            const int col = n0 + tg_wrow<FJ, false>((wc * FJ + j) * 16 + fc * 4);
+            if (col >= N) continue;
+            if (part)
+                *reinterpret_cast<tgf4*>(part + ((int64_t)sp * M + row) * N + col) = acc[i][j];
+            else if (j % 2 == 0)
+                *reinterpret_cast<uint4*>(out + (size_t)row * N + col) =
+                    make_uint4(pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3]),
+                               pack_bf16x2(acc[i][j + 1][0], acc[i][j + 1][1]),
+                               pack_bf16x2(acc[i][j + 1][2], acc[i][j + 1][3]));
+        }
+    }
+}
+
+// Tiles of 32 FI x 64 FJ: group 0 takes the upper half of the rows, group 1 the lower, a wave a quarter of
+// the columns. Phase 2 t: group 0 reads step t and group 1 multiplies step t - 1; phase 2 t + 1: group
+// 1 reads step t. Group 0 sends for x, XS steps deep, group 1 for W, WS deep: W comes from further away.
+// What phase 2 t sends for takes the place of step t - 1, which both have read. A wave waits for its own
+// transfers before the barrier that lets step t + 1 be read.
+//
+// Both operands come by 16-byte global_load_lds, inline asm: hipcc's own waits drain builtin transfers
+// before the first LDS read. 16-byte chunk c of row r lies at c ^ (r >> 1 & 7): the 16 rows of a fragment
+// read touch every bank once. Rows past M and weight rows past N repeat the last one. Work items go to the
+// dies in runs, the row tiles of a strip of weight rows next to each other.
+template <int FI, int FJ, int XS, int WS, bool GU>
+__global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
+    const char* __restrict__ x, int64_t xs, const char* __restrict__ w,
+    uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int K, int mtiles,
+    int splits, int items, int act) {
+    constexpr int BM = 32 * FI, BN = 64 * FJ;
+    constexpr int XB = BM * 128, WB = BN * 128;      // bytes of a step
+    constexpr int LP = FI > 2 * FJ ? FI : 2 * FJ;    // transfers of a wave and step, at most
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int per = gridDim.x >> 3;
+    const int item = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (item >= items) return;
+    const int strip = item / (splits * mtiles), rest = item - strip * splits * mtiles;
+    const int sp = rest / mtiles, m0 = (rest - sp * mtiles) * BM;
+    const int n0 = strip * (GU ? BN / 2 : BN);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int grp = wave >> 2, wc = wave & 3;
+    const int steps = K / 64;
+    const int s0 = (int)((int64_t)steps * sp / splits), s1 = (int)((int64_t)steps * (sp + 1) / splits);
+    const int n = s1 - s0;
+
+    // transfers of eight rows: group 0 those of x, group 1 those of w
+    const char* base = grp ? w + (int64_t)n0 * K * 2 + (int64_t)s0 * 128
+                           : x + (int64_t)m0 * xs * 2 + (int64_t)s0 * 128;
+    uint32_t off[LP];
+#pragma unroll
+    for (int p = 0; p < LP; ++p) {
+        const int r = (p * 4 + wc) * 8 + (lane >> 3);
+        const int chunk = ((lane & 7) ^ (r >> 1 & 7)) * 16;
+        if (!grp) off[p] = (uint32_t)min(r, M - 1 - m0) * (uint32_t)(xs * 2) + chunk;
+        else off[p] = (uint32_t)(min(tg_wrow<FJ, GU>(r), N - 1 - n0) + (tg_isup<FJ, GU>(r) ? N : 0)) * (uint32_t)(K * 2) + chunk;
+    }
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + (grp ? XS * XB : 0) + wc * 1024);
+    auto stage_x = [&](int buf) {
+#pragma unroll
+        for (int p = 0; p < FI; ++p) lds_transfer16(lds0 + buf * XB + p * 4096, off[p], base);
+        base += 128;
+    };
+    auto stage_w = [&](int buf) {
+#pragma unroll
+        for (int p = 0; p < 2 * FJ; ++p) lds_transfer16(lds0 + buf * WB + p * 4096, off[p], base);
+        base += 128;
+    };
+    // this wave's transfers of the step that `behind` younger ones follow
+    auto landed_x = [&](int behind) {
+        if (XS > 3 && behind >= 2) tg_wait<2 * FI>();
+        else if (XS > 2 && behind >= 1) tg_wait<FI>();
+        else tg_wait<0>();
+    };
+    auto landed_w = [&](int behind) {
+        if (WS > 3 && behind >= 2) tg_wait<4 * FJ>();
+        else if (WS > 2 && behind >= 1) tg_wait<2 * FJ>();
+        else tg_wait<0>();
+    };
+
+    tgf4 acc[FI][FJ] = {};
+    if (!grp) {
+#pragma unroll
+        for (int t = 0; t < XS - 1; ++t)
+            if (t < n) stage_x(t);
+        landed_x(min(XS - 2, n - 1));
+        tg_barrier();
+    } else {
+#pragma unroll
+        for (int t = 0; t < WS - 1; ++t)
+            if (t < n) stage_w(t);
+        landed_w(min(WS - 2, n - 1));
+        tg_barrier();
+        tg_barrier();
+    }
+    const int fr = lane & 15, fc = lane >> 4;
+    const int at0 = fr * 128 + ((fc ^ (fr >> 1)) << 4), at1 = fr * 128 + (((fc + 4) ^ (fr >> 1)) << 4);
+    int xbuf = 0, wbuf = 0;
+    for (int t = 0; t < n; ++t) {
+        const char* xr = smem + xbuf * XB + grp * FI * 16 * 128;
+        const char* wr = smem + XS * XB + wbuf * WB + wc * FJ * 16 * 128;
+        tgs8 xf[2][FI], wf[2][FJ];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+#pragma unroll
+            for (int j = 0; j < FJ; ++j) wf[k][j] = *reinterpret_cast<const tgs8*>(wr + j * 2048 + (k ? at1 : at0));
+#pragma unroll
+            for (int i = 0; i < FI; ++i) xf[k][i] = *reinterpret_cast<const tgs8*>(xr + i * 2048 + (k ? at1 : at0));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (!grp) {
+            if (t + XS - 1 < n) stage_x(xbuf == 0 ? XS - 1 : xbuf - 1);
+        } else {
+            if (t + WS - 1 < n) stage_w(wbuf == 0 ? WS - 1 : wbuf - 1);
+            landed_w(min(WS - 2, n - 2 - t));
+        }
+        tg_read_done();
+        tg_barrier();
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int i = 0; i < FI; ++i)
+#pragma unroll
+                for (int j = 0; j < FJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[k][j], xf[k][i], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!grp) landed_x(min(XS - 2, n - 2 - t));
+        tg_barrier();
+        xbuf = xbuf + 1 == XS ? 0 : xbuf + 1;
+        wbuf = wbuf + 1 == WS ? 0 : wbuf + 1;
+    }
+    if (!grp) tg_barrier();
+
+    tg_store<FI, FJ, GU, 0, FI>(acc, out, part, m0 + grp * FI * 16, n0, wc, M, N, sp, act);
+}
+
+// Tiles of 32 FI x 32 FJ: a wave of 2 x 2 takes a quarter of the tile and the groups take the steps in
+// turn, each into sums of its own, which are added up at the end. A quarter a wave reads less LDS than
+// an eighth (128 x 128: 64 KB a step and not 98), and a phase is a whole step for both (800 x 4096 x 4096
+// 40 us with eighths, 34 here; 800 x 4096 x 14336 126, 103).
+template <int FI, int FJ, int ST, bool GU>
+__global__ __launch_bounds__(512, 2) void tile_gemm_turns_kernel(
+    const char* __restrict__ x, int64_t xs, const char* __restrict__ w,
+    uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int K, int mtiles,
+    int splits, int items, int act) {
+    constexpr int BM = 32 * FI, BN = 32 * FJ;
+    constexpr int STEP = (BM + BN) * 128, LP = FI + FJ;      // transfers of a wave: FI of x, FJ of w
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int per = gridDim.x >> 3;
+    const int item = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (item >= items) return;
+    const int strip = item / (splits * mtiles), rest = item - strip * splits * mtiles;
+    const int sp = rest / mtiles, m0 = (rest - sp * mtiles) * BM;
+    const int n0 = strip * (GU ? BN / 2 : BN);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int grp = wave >> 2, wid = wave & 3, wm = wid >> 1, wc = wid & 1;
+    const int steps = K / 64;
+    const int s0 = (int)((int64_t)steps * sp / splits), s1 = (int)((int64_t)steps * (sp + 1) / splits);
+    const int n = s1 - s0;
+
+    const char* xb = x + (int64_t)m0 * xs * 2 + (int64_t)s0 * 128;
+    const char* wb = w + (int64_t)n0 * K * 2 + (int64_t)s0 * 128;
+    uint32_t off[LP];
+#pragma unroll
+    for (int p = 0; p < LP; ++p) {
+        const int r = ((p < FI ? p : p - FI) * 4 + wid) * 8 + (lane >> 3);
+        const int chunk = ((lane & 7) ^ (r >> 1 & 7)) * 16;
+        if (p < FI) off[p] = (uint32_t)min(r, M - 1 - m0) * (uint32_t)(xs * 2) + chunk;
+        else off[p] = (uint32_t)(min(tg_wrow<FJ, GU>(r), N - 1 - n0) + (tg_isup<FJ, GU>(r) ? N : 0)) * (uint32_t)(K * 2) + chunk;
+    }
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + wid * 1024);
+    auto stage = [&](int step, int buf) {
+        const char* xt = xb + (int64_t)step * 128;
+        const char* wt = wb + (int64_t)step * 128;
+#pragma unroll
+        for (int p = 0; p < LP; ++p) lds_transfer16(lds0 + buf * STEP + p * 4096, off[p], p < FI ? xt : wt);
+    };
+    // Phase p: group p & 1 reads step p and sends for step p + ST - 1, into the place of step p - 1,
+    // while the other multiplies step p - 1. Step s is sent for by group (s + ST - 1) & 1, which
+    // waits for it at the end of phase s - 1: after reading (ST even) or after multiplying.
+    constexpr int OWN = (ST - 1) & 1;
+    auto landed = [&](int s) {
+        const int young = (min(s + ST - 2, n - 1) - s) / 2;     // younger steps of this group under way
+        if (ST > 5 && young >= 2) tg_wait<2 * LP>();
+        else if (ST > 3 && young >= 1) tg_wait<LP>();
+        else tg_wait<0>();
+    };
+#pragma unroll
+    for (int t = 0; t < ST - 1; ++t)
+        if (((t + OWN) & 1) == grp && t < n) stage(t, t);
+    if (grp == OWN) landed(0);
+    tg_barrier();
+    if (grp) {
+        if (ST % 2 && n > 1) landed(1);
+        tg_barrier();
+    }
+    tgf4 acc[FI][FJ] = {};
+    const int fr = lane & 15, fc = lane >> 4;
+    const int at0 = fr * 128 + ((fc ^ (fr >> 1)) << 4), at1 = fr * 128 + (((fc + 4) ^ (fr >> 1)) << 4);
+    int buf = grp;
+    for (int s = grp; s < n; s += 2) {
+        const char* xr = smem + buf * STEP + wm * FI * 2048;
+        const char* wr = smem + buf * STEP + BM * 128 + wc * FJ * 2048;
+        tgs8 xf[2][FI], wf[2][FJ];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+#pragma unroll
+            for (int j = 0; j < FJ; ++j) wf[k][j] = *reinterpret_cast<const tgs8*>(wr + j * 2048 + (k ? at1 : at0));
+#pragma unroll
+            for (int i = 0; i < FI; ++i) xf[k][i] = *reinterpret_cast<const tgs8*>(xr + i * 2048 + (k ? at1 : at0));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (s + ST - 1 < n) stage(s + ST - 1, buf == 0 ? ST - 1 : buf - 1);
+        if (ST % 2 == 0 && s + 1 < n) landed(s + 1);
+        tg_read_done();
+        tg_barrier();                                        // the end of phase s
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int i = 0; i < FI; ++i)
+#pragma unroll
+                for (int j = 0; j < FJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[k][j], xf[k][i], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (s + 1 < n) {
+            if (ST % 2 && s + 2 < n) landed(s + 2);
+            tg_barrier();                                    // the end of phase s + 1
+        }
+        buf = buf + 2 >= ST ? buf + 2 - ST : buf + 2;
+    }
+    // each group takes the other's sums of half of its fragments
+    constexpr int FH = (FI + 1) / 2;
+    tgf4* ex = reinterpret_cast<tgf4*>(smem);
+    if (grp) {
+#pragma unroll
+        for (int i = 0; i < FH; ++i)
+#pragma unroll
+            for (int j = 0; j < FJ; ++j) ex[((i * FJ + j) * 4 + wid) * 64 + lane] = acc[i][j];
+    } else {
+#pragma unroll
+        for (int i = FH; i < FI; ++i)
+#pragma unroll
+            for (int j = 0; j < FJ; ++j) ex[((i * FJ + j) * 4 + wid) * 64 + lane] = acc[i][j];
+    }
+    __syncthreads();
+    if (grp) {
+#pragma unroll
+        for (int i = FH; i < FI; ++i)
+#pragma unroll
+            for (int j = 0; j < FJ; ++j) acc[i][j] += ex[((i * FJ + j) * 4 + wid) * 64 + lane];
+        tg_store<FI, FJ, GU, FH, FI>(acc, out, part, m0 + wm * FI * 16, n0, wc, M, N, sp, act);
+    } else {
+#pragma unroll
+        for (int i = 0; i < FH; ++i)
+#pragma unroll
+            for (int j = 0; j < FJ; ++j) acc[i][j] += ex[((i * FJ + j) * 4 + wid) * 64 + lane];
+        tg_store<FI, FJ, GU, 0, FH>(acc, out, part, m0 + wm * FI * 16, n0, wc, M, N, sp, act);
+    }
+}
+
+// Forms, and what they take: `step` us a step of 64 columns and `more` of it when all CUs work (power,
+// and x from beside the chip), `tile` us to start and end a tile; least squares over 2700 times of 110
+// products, to 6 to 11%. The choice by them takes 1.01 of the time of the best form (1.13 at most).
+struct TgForm {
+    int bm, bn;
+    float step, more, tile;
+};
+static const TgForm tg_forms[] = {
+    {256, 256, 0.872f, 0.498f, 9.2f}, {224, 256, 0.796f, 0.425f, 8.3f}, {192, 256, 0.734f, 0.381f, 7.6f},
+    {160, 256, 0.673f, 0.295f, 7.2f}, {256, 128, 0.531f, 0.295f, 6.7f}, {224, 128, 0.471f, 0.264f, 6.1f},
+    {160, 128, 0.393f, 0.201f, 5.3f}, {128, 128, 0.352f, 0.195f, 4.1f}, {96, 128, 0.292f, 0.170f, 2.8f},
+    {128, 64, 0.259f, 0.116f, 2.5f},
+};
+
+// The fastest form and column splits as form * 256 + splits, and its time in *us.
+static int tg_choose(int M, int rows, int K, bool split, bool summed, float* us_best) {
+    const int steps = K / 64;
+    const float mn = (float)M * rows;
+    float best = 1e30f;
+    int plan = -1;
+    for (int f = 0; f < (int)(sizeof(tg_forms) / sizeof(tg_forms[0])); ++f) {
+        const TgForm& t = tg_forms[f];
+        const int64_t tiles = (int64_t)CEIL_DIV(M, t.bm) * CEIL_DIV(rows, t.bn);
+        const int most = split && tiles < 256 ? (int)std::min<int64_t>(8, 256 / tiles) : 1;
+        for (int sp = 1; sp <= most && (sp == 1 || steps / sp >= 8); ++sp) {
+            const int64_t blocks = tiles * sp, full = blocks / 256, rest = blocks % 256;
+            const float n = (float)steps / sp;
+            float us = full * (n * (t.step + t.more) + 0.6f * t.tile) + 0.4f * t.tile + 2;
+            if (rest) us += n * (t.step + t.more * rest / 256) + 0.6f * t.tile;
+            if (sp > 1) us += sp * mn * 0.36e-6f + (summed ? (sp * 4 - 2) * mn / 4.5e6f : 2.5f + sp * mn * 4 / 4.5e6f);
+            if (us < best) best = us, plan = f * 256 + sp;
+        }
+    }
+    *us_best = best;
+    return plan;
+}
+
+// The plan of M rows, N (gate-up: 2 N) weight rows and K columns; -1 for sizes that the product does not
+// take, and for gate-up products that other forms take sooner. Splits fill the CUs where the tiles leave
+// some idle, at most one block a CU; their parts are written, and read again by a kernel of their own (4.5
+// TB/s, 2.5 us) or, summed, by a norm that would have read the product. Gate-up does not split: where
+// splits and an activation kernel would be the faster way (2 x 2048 x 8192, M = 246 50.9 us in one, 38.4
+// the library and the kernel) it is left to them.
+extern "C" int oa_tile_gemm_plan(int M, int N, int K, int gateup, int summed) {
+    if (M < 1 || N < 8 || N % 8 != 0 || N > (1 << 29) || K < 512 || K % 64 != 0) return -1;
+    float one, two;
+    if (!gateup) return tg_choose(M, N, K, true, summed, &one);
+    const int plan = tg_choose(M, 2 * N, K, false, false, &one);
+    tg_choose(M, 2 * N, K, true, false, &two);
+    return one > two + 3 + (float)M * N * 6 / 4.5e6f ? -1 : plan;
+}
+
+extern "C" int oa_ring_sum(void* stream, const void* part, void* out, int M, int N, int splits);
+
+// out [M, N] = x [M, K] w [N, K]^T, x rows xs elements apart. act 1 (silu), 2 (tanh gelu): out =
+// act(x w[:N]^T) * (x w[N:]^T), w [2 N, K]. plan: oa_tile_gemm_plan's. scratch: splits * M * N floats,
+// unused at one split; out null: left there, not added up.
+extern "C" int oa_tile_gemm(void* stream, const void* x, int64_t xs, const void* w, void* out,
+                            void* scratch, int M, int N, int K, int plan, int act) {
+    const int form = plan >> 8, splits = plan & 255;
+    if (M < 1 || N < 8 || N % 8 != 0 || K < 64 || K % 64 != 0) return -100;
+    if (splits < 1 || splits > K / 64 || (splits > 1 ? !scratch || act : !out)) return -101;
+    if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)scratch) % 16 != 0 || xs % 8 != 0)
+        return -102;
+    if (act < 0 || act > 2 || plan < 0) return -104;
+    // a lane's place in a tile is 32 bits wide
+    if (xs < K || xs >= (1 << 22) || ((int64_t)(act ? N : 0) + 256) * K * 2 >= ((int64_t)1 << 32)) return -103;
+    hipStream_t s = (hipStream_t)stream;
+    float* part = splits > 1 ? (float*)scratch : nullptr;
+#define TG_LAUNCH(kernel, BM, BN, lds)                                                             \
+    do {                                                                                           \
+        const int mt = CEIL_DIV(M, BM);                                                            \
+        const int64_t items = (int64_t)CEIL_DIV(N, (BN) / (act ? 2 : 1)) * mt * splits;            \
+        if (items > (1 << 28)) return -103;                                                        \
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(CEIL_DIV(items, 8) * 8)), dim3(512), lds, s,    \
+                           (const char*)x, xs, (const char*)w, (uint16_t*)out, part, M, N, K, mt,  \
+                           splits, (int)items, act);                                               \
+    } while (0)
+#define TG_HALVES(FI, FJ, XS, WS)                                                                       \
+    do {                                                                                                \
+        constexpr int lds = ((XS) * 32 * (FI) + (WS) * 64 * (FJ)) * 128;                                \
+        if (act) TG_LAUNCH((tile_gemm_kernel<FI, FJ, XS, WS, true>), 32 * (FI), 64 * (FJ), lds);        \
+        else TG_LAUNCH((tile_gemm_kernel<FI, FJ, XS, WS, false>), 32 * (FI), 64 * (FJ), lds);           \
+    } while (0)
+#define TG_TURNS(FI, FJ, ST)                                                                            \
+    do {                                                                                                \
+        constexpr int lds = (ST) * 32 * ((FI) + (FJ)) * 128;                                            \
+        if (act) TG_LAUNCH((tile_gemm_turns_kernel<FI, FJ, ST, true>), 32 * (FI), 32 * (FJ), lds);      \
+        else TG_LAUNCH((tile_gemm_turns_kernel<FI, FJ, ST, false>), 32 * (FI), 32 * (FJ), lds);         \
+    } while (0)
+    switch (form) {
+        case 0: TG_HALVES(8, 4, 2, 3); break;
+        case 1: TG_HALVES(7, 4, 2, 3); break;
+        case 2: TG_HALVES(6, 4, 2, 3); break;
+        case 3: TG_HALVES(5, 4, 3, 3); break;
+        case 4: TG_TURNS(8, 4, 3); break;
+        case 5: TG_TURNS(7, 4, 3); break;
+        case 6: TG_TURNS(5, 4, 4); break;
+        case 7: TG_TURNS(4, 4, 4); break;
+        case 8: TG_TURNS(3, 4, 5); break;
+        case 9: TG_TURNS(4, 2, 6); break;
+        default: return -105;
+    }
+#undef TG_TURNS
+#undef TG_HALVES
+#undef TG_LAUNCH
+    HIP_CHECK_LAUNCH();
+    return splits > 1 && out ? oa_ring_sum(stream, scratch, out, M, N, splits) : 0;
+}

@@ -16,7 +16,7 @@ CSRC = os.path.join(
 
 FILES = ["gemv.hip", "attention_prefill.hip", "attention_decode.hip", "fp8_moe.hip",
          "mixers.hip", "blocks.hip", "prenorm.hip", "recurrent.hip", "hyper.hip", "moe_gemv.hip",
-         "moe_grouped.hip", "skinny.hip", "ring_gemm.hip", "rmsnorm.hip", "sampling.hip"]
+         "moe_grouped.hip", "skinny.hip", "ring_gemm.hip", "tile_gemm.hip", "rmsnorm.hip", "sampling.hip"]
 
 # Known, measured-benign exceptions: kernel name fragment -> max scratch bytes/lane.
 # delta_fused_kernel<16, 2|4>: key sizes above 128 with more than 64 value

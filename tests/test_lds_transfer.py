@@ -16,7 +16,7 @@ WITH_TRANSFERS = [s for s in build.SOURCES + build.MIXER_SOURCES
 
 
 def test_files():
-    assert {"attention_prefill.hip", "fp8_moe.hip", "ring_gemm.hip"} <= set(WITH_TRANSFERS)
+    assert {"attention_prefill.hip", "fp8_moe.hip", "ring_gemm.hip", "tile_gemm.hip"} <= set(WITH_TRANSFERS)
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="hipcc not on PATH")

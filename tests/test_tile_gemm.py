@@ -1,0 +1,90 @@
+"""Tile products of more than 128 rows against float64: every form, row and strip remainders, fewer
+steps than a ring holds, odd and even numbers of them, column splits, both activations, rows
+apart; and which products take them."""
+
+import pytest
+import torch
+
+from opsagent_amd import ops
+
+FORMS = range(10)
+# M, N, K, splits
+SIZES = [(129, 8, 64, 1), (256, 520, 128, 1), (300, 136, 192, 1), (161, 264, 448, 3),
+         (513, 392, 512, 2), (700, 1000, 1088, 1)]
+
+
+def _whole(rows, cols, scale=1.0):
+    """Whole numbers up to 2 times a power of two: every product and sum is exact."""
+    return (torch.randint(-2, 3, (rows, cols), device="cuda") * scale).to(torch.bfloat16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,splits", SIZES)
+@pytest.mark.parametrize("form", FORMS)
+def test_plain(form, M, N, K, splits):
+    torch.manual_seed(M + N + K)
+    wide, w = _whole(M, K + 8), _whole(N, K)
+    for x in (wide[:, :K].contiguous(), wide[:, :K]):      # rows apart as well
+        want = x.double() @ w.double().T
+        assert torch.equal(ops._tile(x, w, form * 256 + splits), want.to(torch.bfloat16))
+        if splits > 1:
+            parts = ops._tile(x, w, form * 256 + splits, parts=True)
+            assert parts.shape == (splits, M, N) and torch.equal(parts.double().sum(0), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,splits", SIZES)
+@pytest.mark.parametrize("form", FORMS)
+def test_gateup(form, M, N, K, splits):
+    torch.manual_seed(M + N + K)
+    x, w = _whole(M, K), _whole(2 * N, K, 2.0 ** -5)
+    g, u = (x.double() @ w.double().T).split(N, 1)
+    for act in (1, 2):
+        got = ops._tile(x, w, form * 256 + 1, act).double()
+        f = torch.nn.functional.silu(g) if act == 1 else torch.nn.functional.gelu(g, approximate="tanh")
+        # one rounding to bf16, and some float32 roundings (exp of up to |g| / ln 2 scaled
+        # bits, 1 + tanh near -1) of the exact halves
+        bound = 2.0 ** -8 * (f * u).abs() + 2.0 ** -20 * (1 + g.abs()) * (g * u).abs()
+        assert ((got - f * u).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+def test_dispatch():
+    """The public products take the tiles, parts reach the norm behind them, and the results are
+    those of the library's product to the rounding of bf16."""
+    torch.manual_seed(0)
+    x = torch.randn(333, 8192, device="cuda").bfloat16()
+    w = (torch.randn(2048, 8192, device="cuda") / 90).bfloat16()
+    want = x.double() @ w.double().T
+    assert ops._tile_choice(333, 2048, 8192) & 255 > 1
+    parts = ops.linear_parts(x, w)
+    assert isinstance(parts, ops.PlaneSum)
+    for got in (ops.linear(x, w), ops._added_up(parts)):
+        assert (got.double() - want).norm() <= 2.0 ** -8 * want.norm()
+    grad = w.clone().requires_grad_()
+    ops.linear(x, grad).sum().backward()                 # gradients go through the library
+    assert grad.grad is not None
+
+
+def test_plan():
+    """Sizes that no form takes, and what the rule answers for those it takes: a form of the table,
+    splits that leave every block eight steps and no more blocks than CUs."""
+    plan = ops._lib()[0].oa_tile_gemm_plan
+    for args in ((0, 64, 512), (200, 12, 512), (200, 64, 448), (200, 64, 520)):
+        assert plan(*args, 0, 0) == -1
+    tiles = [(256, 256), (224, 256), (192, 256), (160, 256), (256, 128), (224, 128), (160, 128),
+             (128, 128), (96, 128), (128, 64)]
+    for M in (129, 200, 333, 800, 2048, 8192):
+        for N, K in ((2048, 2048), (4096, 14336), (12288, 4096), (128256, 4096), (264, 576)):
+            for gateup in (0, 1):
+                for summed in (0, 1):
+                    answer = plan(M, N, K, gateup, summed)
+                    if answer < 0:
+                        assert gateup                    # left to splits and the activation kernel
+                        continue
+                    form, splits = divmod(answer, 256)
+                    bm, bn = tiles[form]
+                    blocks = -(-M // bm) * -(-N * (1 + gateup) // bn) * splits
+                    assert splits == 1 or (not gateup and blocks <= 256 and K // 64 // splits >= 8)
+    assert ops._tile_choice(128, 4096, 14336) is None    # the ring's
+    assert ops._tile_choice(200, 2048, 2048) is None     # light weights, few rows: the library
