@@ -1,5 +1,5 @@
 // Products of more than 128 rows: C[M, N] = x[M, K] W[N, K]^T in bf16, plain, gate-up with its
-// activation, or as float32 column parts.
+// activation, or as float32 column parts, and in e4m3 with a scale a row of both.
 //
 // Three things bound them, measured apart on 2048 x 8192 x 4096 in tiles of 256 x 256. The matrix
 // cores take 1.05 us a step of 64 columns on random operands that LDS feeds (1.75 PFLOP/s; 2.4 on
@@ -23,6 +23,54 @@
 
 typedef __attribute__((ext_vector_type(4))) float tgf4;
 typedef __attribute__((ext_vector_type(8))) short tgs8;
+typedef __attribute__((ext_vector_type(8))) int tgi8;
+
+// A fragment's 16 rows of a step: 128 bytes of each, 32 a lane. Lane group c has chunks c and c + 4, in
+// bf16 the columns of the two products that they stand for; in e4m3 the order of a product's columns is
+// free as long as both operands share it, and chunks 2 c and 2 c + 1 collide in the LDS banks (256 x 256
+// 1.66 us a step, 1.37 so).
+union TgFrag {
+    tgs8 b[2];
+    tgi8 f8;
+};
+struct TgAt {
+    int a, b;
+    __device__ __forceinline__ TgAt(int lane) {
+        const int r = lane & 15, c = lane >> 4;
+        a = r * 128 + ((c ^ (r >> 1)) << 4);
+        b = r * 128 + (((c + 4) ^ (r >> 1)) << 4);
+    }
+};
+
+// the fragments of FI x FJ over a step: the products of bf16, or of e4m3 with unit block scales (the only
+// fp8 products past the bf16 rate)
+template <bool F8, int FI, int FJ>
+__device__ __forceinline__ void tg_multiply(tgf4 (&acc)[FI][FJ], const TgFrag (&wf)[FJ], const TgFrag (&xf)[FI]) {
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int k = 0; k < (F8 ? 1 : 2); ++k)
+#pragma unroll
+        for (int i = 0; i < FI; ++i)
+#pragma unroll
+            for (int j = 0; j < FJ; ++j)
+                if constexpr (F8)
+                    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[j].f8, xf[i].f8, acc[i][j], 0, 0, 0, 0x7f, 0, 0x7f);
+                else
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j].b[k], xf[i].b[k], acc[i][j], 0, 0, 0);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+}
+template <int FI, int FJ>
+__device__ __forceinline__ void tg_read(TgFrag (&wf)[FJ], TgFrag (&xf)[FI], const char* wr, const char* xr, const TgAt& at) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+        for (int j = 0; j < FJ; ++j) wf[j].b[k] = *reinterpret_cast<const tgs8*>(wr + j * 2048 + (k ? at.b : at.a));
+#pragma unroll
+        for (int i = 0; i < FI; ++i) xf[i].b[k] = *reinterpret_cast<const tgs8*>(xr + i * 2048 + (k ? at.b : at.a));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
 
 template <int V>
 __device__ __forceinline__ void tg_wait() {
@@ -66,9 +114,9 @@ __device__ __forceinline__ bool tg_isup(int b) {
 }
 
 // fragments I0 .. I1 of a wave whose first row is row0
-template <int FI, int FJ, bool GU, int I0, int I1>
-__device__ __forceinline__ void tg_store(const tgf4 (&acc)[FI][FJ], uint16_t* out, float* part, int row0,
-                                         int n0, int wc, int M, int N, int sp, int act) {
+template <int FI, int FJ, bool GU, bool F8, int I0, int I1>
+__device__ __forceinline__ void tg_store(tgf4 (&acc)[FI][FJ], const float* xscale, const float* wscale,
+                                         uint16_t* out, float* part, int row0, int n0, int wc, int M, int N, int sp, int act) {
     const int fr = threadIdx.x & 15, fc = threadIdx.x >> 4 & 3;
     // D: column (row of x) lane & 15, rows (weight rows) (lane >> 4) * 4 and up
 #pragma unroll
@@ -99,13 +147,23 @@ __device__ __forceinline__ void tg_store(const tgf4 (&acc)[FI][FJ], uint16_t* ou
         for (int j = 0; j < FJ; ++j) {
             const int col = n0 + tg_wrow<FJ, false>((wc * FJ + j) * 16 + fc * 4);
             if (col >= N) continue;
-            if (part)
+            if (part) {
                 *reinterpret_cast<tgf4*>(part + ((int64_t)sp * M + row) * N + col) = acc[i][j];
-            else if (j % 2 == 0)
-                *reinterpret_cast<uint4*>(out + (size_t)row * N + col) =
-                    make_uint4(pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3]),
-                               pack_bf16x2(acc[i][j + 1][0], acc[i][j + 1][1]),
-                               pack_bf16x2(acc[i][j + 1][2], acc[i][j + 1][3]));
+                continue;
+            }
+            if (j % 2) continue;
+            if constexpr (F8) {
+                const float sx = xscale[row];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    acc[i][j][e] = acc[i][j][e] * sx * wscale[col + e];
+                    acc[i][j + 1][e] = acc[i][j + 1][e] * sx * wscale[col + 4 + e];
+                }
+            }
+            *reinterpret_cast<uint4*>(out + (size_t)row * N + col) =
+                make_uint4(pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3]),
+                           pack_bf16x2(acc[i][j + 1][0], acc[i][j + 1][1]),
+                           pack_bf16x2(acc[i][j + 1][2], acc[i][j + 1][3]));
         }
     }
 }
@@ -120,10 +178,10 @@ __device__ __forceinline__ void tg_store(const tgf4 (&acc)[FI][FJ], uint16_t* ou
 // before the first LDS read. 16-byte chunk c of row r lies at c ^ (r >> 1 & 7): the 16 rows of a fragment
 // read touch every bank once. Rows past M and weight rows past N repeat the last one. Work items go to the
 // dies in runs, the row tiles of a strip of weight rows next to each other.
-template <int FI, int FJ, int XS, int WS, bool GU>
+template <int FI, int FJ, int XS, int WS, bool GU, bool F8>
 __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
     const char* __restrict__ x, int64_t xs, const char* __restrict__ w,
-    uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int K, int mtiles,
+    const float* __restrict__ xscale, const float* __restrict__ wscale, uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int64_t kb, int mtiles,
     int splits, int items, int act) {
     constexpr int BM = 32 * FI, BN = 64 * FJ;
     constexpr int XB = BM * 128, WB = BN * 128;      // bytes of a step
@@ -138,20 +196,20 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int grp = wave >> 2, wc = wave & 3;
-    const int steps = K / 64;
+    const int steps = (int)(kb / 128);                // kb: bytes of a weight row, xs: of a row of x
     const int s0 = (int)((int64_t)steps * sp / splits), s1 = (int)((int64_t)steps * (sp + 1) / splits);
     const int n = s1 - s0;
 
     // transfers of eight rows: group 0 those of x, group 1 those of w
-    const char* base = grp ? w + (int64_t)n0 * K * 2 + (int64_t)s0 * 128
-                           : x + (int64_t)m0 * xs * 2 + (int64_t)s0 * 128;
+    const char* base = grp ? w + (int64_t)n0 * kb + (int64_t)s0 * 128
+                           : x + (int64_t)m0 * xs + (int64_t)s0 * 128;
     uint32_t off[LP];
 #pragma unroll
     for (int p = 0; p < LP; ++p) {
         const int r = (p * 4 + wc) * 8 + (lane >> 3);
         const int chunk = ((lane & 7) ^ (r >> 1 & 7)) * 16;
-        if (!grp) off[p] = (uint32_t)min(r, M - 1 - m0) * (uint32_t)(xs * 2) + chunk;
-        else off[p] = (uint32_t)(min(tg_wrow<FJ, GU>(r), N - 1 - n0) + (tg_isup<FJ, GU>(r) ? N : 0)) * (uint32_t)(K * 2) + chunk;
+        if (!grp) off[p] = (uint32_t)min(r, M - 1 - m0) * (uint32_t)xs + chunk;
+        else off[p] = (uint32_t)(min(tg_wrow<FJ, GU>(r), N - 1 - n0) + (tg_isup<FJ, GU>(r) ? N : 0)) * (uint32_t)kb + chunk;
     }
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + (grp ? XS * XB : 0) + wc * 1024);
     auto stage_x = [&](int buf) {
@@ -191,21 +249,13 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
         tg_barrier();
         tg_barrier();
     }
-    const int fr = lane & 15, fc = lane >> 4;
-    const int at0 = fr * 128 + ((fc ^ (fr >> 1)) << 4), at1 = fr * 128 + (((fc + 4) ^ (fr >> 1)) << 4);
+    const TgAt at(lane);
     int xbuf = 0, wbuf = 0;
     for (int t = 0; t < n; ++t) {
         const char* xr = smem + xbuf * XB + grp * FI * 16 * 128;
         const char* wr = smem + XS * XB + wbuf * WB + wc * FJ * 16 * 128;
-        tgs8 xf[2][FI], wf[2][FJ];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-#pragma unroll
-            for (int j = 0; j < FJ; ++j) wf[k][j] = *reinterpret_cast<const tgs8*>(wr + j * 2048 + (k ? at1 : at0));
-#pragma unroll
-            for (int i = 0; i < FI; ++i) xf[k][i] = *reinterpret_cast<const tgs8*>(xr + i * 2048 + (k ? at1 : at0));
-        }
-        __builtin_amdgcn_sched_barrier(0);
+        TgFrag xf[FI], wf[FJ];
+        tg_read<FI, FJ>(wf, xf, wr, xr, at);
         if (!grp) {
             if (t + XS - 1 < n) stage_x(xbuf == 0 ? XS - 1 : xbuf - 1);
         } else {
@@ -214,16 +264,7 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
         }
         tg_read_done();
         tg_barrier();
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-#pragma unroll
-            for (int i = 0; i < FI; ++i)
-#pragma unroll
-                for (int j = 0; j < FJ; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[k][j], xf[k][i], acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_s_setprio(0);
-        __builtin_amdgcn_sched_barrier(0);
+        tg_multiply<F8, FI, FJ>(acc, wf, xf);
         if (!grp) landed_x(min(XS - 2, n - 2 - t));
         tg_barrier();
         xbuf = xbuf + 1 == XS ? 0 : xbuf + 1;
@@ -231,17 +272,17 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
     }
     if (!grp) tg_barrier();
 
-    tg_store<FI, FJ, GU, 0, FI>(acc, out, part, m0 + grp * FI * 16, n0, wc, M, N, sp, act);
+    tg_store<FI, FJ, GU, F8, 0, FI>(acc, xscale, wscale, out, part, m0 + grp * FI * 16, n0, wc, M, N, sp, act);
 }
 
 // Tiles of 32 FI x 32 FJ: a wave of 2 x 2 takes a quarter of the tile and the groups take the steps in
 // turn, each into sums of its own, which are added up at the end. A quarter a wave reads less LDS than
 // an eighth (128 x 128: 64 KB a step and not 98), and a phase is a whole step for both (800 x 4096 x 4096
 // 40 us with eighths, 34 here; 800 x 4096 x 14336 126, 103).
-template <int FI, int FJ, int ST, bool GU>
+template <int FI, int FJ, int ST, bool GU, bool F8>
 __global__ __launch_bounds__(512, 2) void tile_gemm_turns_kernel(
     const char* __restrict__ x, int64_t xs, const char* __restrict__ w,
-    uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int K, int mtiles,
+    const float* __restrict__ xscale, const float* __restrict__ wscale, uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int64_t kb, int mtiles,
     int splits, int items, int act) {
     constexpr int BM = 32 * FI, BN = 32 * FJ;
     constexpr int STEP = (BM + BN) * 128, LP = FI + FJ;      // transfers of a wave: FI of x, FJ of w
@@ -255,19 +296,19 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_turns_kernel(
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int grp = wave >> 2, wid = wave & 3, wm = wid >> 1, wc = wid & 1;
-    const int steps = K / 64;
+    const int steps = (int)(kb / 128);                // kb: bytes of a weight row, xs: of a row of x
     const int s0 = (int)((int64_t)steps * sp / splits), s1 = (int)((int64_t)steps * (sp + 1) / splits);
     const int n = s1 - s0;
 
-    const char* xb = x + (int64_t)m0 * xs * 2 + (int64_t)s0 * 128;
-    const char* wb = w + (int64_t)n0 * K * 2 + (int64_t)s0 * 128;
+    const char* xb = x + (int64_t)m0 * xs + (int64_t)s0 * 128;
+    const char* wb = w + (int64_t)n0 * kb + (int64_t)s0 * 128;
     uint32_t off[LP];
 #pragma unroll
     for (int p = 0; p < LP; ++p) {
         const int r = ((p < FI ? p : p - FI) * 4 + wid) * 8 + (lane >> 3);
         const int chunk = ((lane & 7) ^ (r >> 1 & 7)) * 16;
-        if (p < FI) off[p] = (uint32_t)min(r, M - 1 - m0) * (uint32_t)(xs * 2) + chunk;
-        else off[p] = (uint32_t)(min(tg_wrow<FJ, GU>(r), N - 1 - n0) + (tg_isup<FJ, GU>(r) ? N : 0)) * (uint32_t)(K * 2) + chunk;
+        if (p < FI) off[p] = (uint32_t)min(r, M - 1 - m0) * (uint32_t)xs + chunk;
+        else off[p] = (uint32_t)(min(tg_wrow<FJ, GU>(r), N - 1 - n0) + (tg_isup<FJ, GU>(r) ? N : 0)) * (uint32_t)kb + chunk;
     }
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + wid * 1024);
     auto stage = [&](int step, int buf) {
@@ -296,35 +337,18 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_turns_kernel(
         tg_barrier();
     }
     tgf4 acc[FI][FJ] = {};
-    const int fr = lane & 15, fc = lane >> 4;
-    const int at0 = fr * 128 + ((fc ^ (fr >> 1)) << 4), at1 = fr * 128 + (((fc + 4) ^ (fr >> 1)) << 4);
+    const TgAt at(lane);
     int buf = grp;
     for (int s = grp; s < n; s += 2) {
         const char* xr = smem + buf * STEP + wm * FI * 2048;
         const char* wr = smem + buf * STEP + BM * 128 + wc * FJ * 2048;
-        tgs8 xf[2][FI], wf[2][FJ];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-#pragma unroll
-            for (int j = 0; j < FJ; ++j) wf[k][j] = *reinterpret_cast<const tgs8*>(wr + j * 2048 + (k ? at1 : at0));
-#pragma unroll
-            for (int i = 0; i < FI; ++i) xf[k][i] = *reinterpret_cast<const tgs8*>(xr + i * 2048 + (k ? at1 : at0));
-        }
-        __builtin_amdgcn_sched_barrier(0);
+        TgFrag xf[FI], wf[FJ];
+        tg_read<FI, FJ>(wf, xf, wr, xr, at);
         if (s + ST - 1 < n) stage(s + ST - 1, buf == 0 ? ST - 1 : buf - 1);
         if (ST % 2 == 0 && s + 1 < n) landed(s + 1);
         tg_read_done();
         tg_barrier();                                        // the end of phase s
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-#pragma unroll
-            for (int i = 0; i < FI; ++i)
-#pragma unroll
-                for (int j = 0; j < FJ; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[k][j], xf[k][i], acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_s_setprio(0);
-        __builtin_amdgcn_sched_barrier(0);
+        tg_multiply<F8, FI, FJ>(acc, wf, xf);
         if (s + 1 < n) {
             if (ST % 2 && s + 2 < n) landed(s + 2);
             tg_barrier();                                    // the end of phase s + 1
@@ -351,45 +375,47 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_turns_kernel(
         for (int i = FH; i < FI; ++i)
 #pragma unroll
             for (int j = 0; j < FJ; ++j) acc[i][j] += ex[((i * FJ + j) * 4 + wid) * 64 + lane];
-        tg_store<FI, FJ, GU, FH, FI>(acc, out, part, m0 + wm * FI * 16, n0, wc, M, N, sp, act);
+        tg_store<FI, FJ, GU, F8, FH, FI>(acc, xscale, wscale, out, part, m0 + wm * FI * 16, n0, wc, M, N, sp, act);
     } else {
 #pragma unroll
         for (int i = 0; i < FH; ++i)
 #pragma unroll
             for (int j = 0; j < FJ; ++j) acc[i][j] += ex[((i * FJ + j) * 4 + wid) * 64 + lane];
-        tg_store<FI, FJ, GU, 0, FH>(acc, out, part, m0 + wm * FI * 16, n0, wc, M, N, sp, act);
+        tg_store<FI, FJ, GU, F8, 0, FH>(acc, xscale, wscale, out, part, m0 + wm * FI * 16, n0, wc, M, N, sp, act);
     }
 }
 
-// Forms, and what they take: `step` us a step of 64 columns and `more` of it when all CUs work (power,
-// and x from beside the chip), `tile` us to start and end a tile; least squares over 2700 times of 110
-// products, to 6 to 11%. The choice by them takes 1.01 of the time of the best form (1.13 at most).
+// Forms, and what they take in us: a step (64 columns, e4m3 128), more of it when all CUs work (power, and
+// x from beside the chip), starting and ending a tile; least squares over 2700 times of 110 products
+// (e4m3: 1900 of 90), to 6 to 11%. The choice by them takes 1.01 of the time of the best form (1.13 at
+// most).
 struct TgForm {
     int bm, bn;
-    float step, more, tile;
+    float step, more, tile, step8, more8, tile8;
 };
 static const TgForm tg_forms[] = {
-    {256, 256, 0.872f, 0.498f, 9.2f}, {224, 256, 0.796f, 0.425f, 8.3f}, {192, 256, 0.734f, 0.381f, 7.6f},
-    {160, 256, 0.673f, 0.295f, 7.2f}, {256, 128, 0.531f, 0.295f, 6.7f}, {224, 128, 0.471f, 0.264f, 6.1f},
-    {160, 128, 0.393f, 0.201f, 5.3f}, {128, 128, 0.352f, 0.195f, 4.1f}, {96, 128, 0.292f, 0.170f, 2.8f},
-    {128, 64, 0.259f, 0.116f, 2.5f},
+    {256, 256, 0.872f, 0.498f, 9.2f, 1.192f, 0.343f, 6.8f}, {224, 256, 0.796f, 0.425f, 8.3f, 1.100f, 0.275f, 6.6f},
+    {192, 256, 0.734f, 0.381f, 7.6f, 0.944f, 0.310f, 6.0f}, {160, 256, 0.673f, 0.295f, 7.2f, 0.741f, 0.195f, 6.6f},
+    {256, 128, 0.531f, 0.295f, 6.7f, 0.849f, 0.122f, 6.8f}, {224, 128, 0.471f, 0.264f, 6.1f, 0.730f, 0.125f, 6.9f},
+    {160, 128, 0.393f, 0.201f, 5.3f, 0.558f, 0.126f, 6.3f}, {128, 128, 0.352f, 0.195f, 4.1f, 0.453f, 0.120f, 5.5f},
+    {96, 128, 0.292f, 0.170f, 2.8f, 0.350f, 0.115f, 4.4f},  {128, 64, 0.259f, 0.116f, 2.5f, 0.276f, 0.108f, 3.8f},
 };
 
-// The fastest form and column splits as form * 256 + splits, and its time in *us.
-static int tg_choose(int M, int rows, int K, bool split, bool summed, float* us_best) {
-    const int steps = K / 64;
+// The fastest form and column splits as form * 256 + splits, and its time in *us. A split has `least` steps.
+static int tg_choose(int M, int rows, int steps, bool split, int least, bool summed, bool f8, float* us_best) {
     const float mn = (float)M * rows;
     float best = 1e30f;
     int plan = -1;
     for (int f = 0; f < (int)(sizeof(tg_forms) / sizeof(tg_forms[0])); ++f) {
         const TgForm& t = tg_forms[f];
+        const float step = f8 ? t.step8 : t.step, more = f8 ? t.more8 : t.more, tile = f8 ? t.tile8 : t.tile;
         const int64_t tiles = (int64_t)CEIL_DIV(M, t.bm) * CEIL_DIV(rows, t.bn);
         const int most = split && tiles < 256 ? (int)std::min<int64_t>(8, 256 / tiles) : 1;
-        for (int sp = 1; sp <= most && (sp == 1 || steps / sp >= 8); ++sp) {
+        for (int sp = 1; sp <= most && (sp == 1 || steps / sp >= least); ++sp) {
             const int64_t blocks = tiles * sp, full = blocks / 256, rest = blocks % 256;
             const float n = (float)steps / sp;
-            float us = full * (n * (t.step + t.more) + 0.6f * t.tile) + 0.4f * t.tile + 2;
-            if (rest) us += n * (t.step + t.more * rest / 256) + 0.6f * t.tile;
+            float us = full * (n * (step + more) + 0.6f * tile) + 0.4f * tile + 2;
+            if (rest) us += n * (step + more * rest / 256) + 0.6f * tile;
             if (sp > 1) us += sp * mn * 0.36e-6f + (summed ? (sp * 4 - 2) * mn / 4.5e6f : 2.5f + sp * mn * 4 / 4.5e6f);
             if (us < best) best = us, plan = f * 256 + sp;
         }
@@ -407,49 +433,55 @@ static int tg_choose(int M, int rows, int K, bool split, bool summed, float* us_
 extern "C" int oa_tile_gemm_plan(int M, int N, int K, int gateup, int summed) {
     if (M < 1 || N < 8 || N % 8 != 0 || N > (1 << 29) || K < 512 || K % 64 != 0) return -1;
     float one, two;
-    if (!gateup) return tg_choose(M, N, K, true, summed, &one);
-    const int plan = tg_choose(M, 2 * N, K, false, false, &one);
-    tg_choose(M, 2 * N, K, true, false, &two);
+    if (!gateup) return tg_choose(M, N, K / 64, true, 8, summed, false, &one);
+    const int plan = tg_choose(M, 2 * N, K / 64, false, 8, false, false, &one);
+    tg_choose(M, 2 * N, K / 64, true, 8, false, false, &two);
     return one > two + 3 + (float)M * N * 6 / 4.5e6f ? -1 : plan;
 }
 
-extern "C" int oa_ring_sum(void* stream, const void* part, void* out, int M, int N, int splits);
+extern "C" double oa_gemm_fp8_us(int M, int N, int K);
 
-// out [M, N] = x [M, K] w [N, K]^T, x rows xs elements apart. act 1 (silu), 2 (tanh gelu): out =
-// act(x w[:N]^T) * (x w[N:]^T), w [2 N, K]. plan: oa_tile_gemm_plan's. scratch: splits * M * N floats,
-// unused at one split; out null: left there, not added up.
-extern "C" int oa_tile_gemm(void* stream, const void* x, int64_t xs, const void* w, void* out,
-                            void* scratch, int M, int N, int K, int plan, int act) {
-    const int form = plan >> 8, splits = plan & 255;
-    if (M < 1 || N < 8 || N % 8 != 0 || K < 64 || K % 64 != 0) return -100;
-    if (splits < 1 || splits > K / 64 || (splits > 1 ? !scratch || act : !out)) return -101;
-    if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)scratch) % 16 != 0 || xs % 8 != 0)
-        return -102;
-    if (act < 0 || act > 2 || plan < 0) return -104;
-    // a lane's place in a tile is 32 bits wide
-    if (xs < K || xs >= (1 << 22) || ((int64_t)(act ? N : 0) + 256) * K * 2 >= ((int64_t)1 << 32)) return -103;
-    hipStream_t s = (hipStream_t)stream;
-    float* part = splits > 1 ? (float*)scratch : nullptr;
+// The plan of an e4m3 product, -1 for sizes that it does not take and where the one-barrier tiles
+// (fp8_moe.hip) are the faster ones by both models: at 90 sizes of 130 to 2048 rows this takes 0.90 of the
+// time of those and the ring, 0.89 would be the best. Us, those / here: 28672 x 4096, M = 256 45.8 / 41.7,
+// 700 104 / 91, 2048 249 / 218; 4096 x 14336, 333 45.4 / 37.3, 700 58.7 / 52.8; 6144 x 4096, 700 34.4 /
+// 29.5, 1434 56.2 / 37.3; 2048 x 2048, 512 12.6 / 10.7; but 3072 x 2048, 1024 13.6 / 15.5.
+extern "C" int oa_tile_gemm_fp8_plan(int M, int N, int K) {
+    if (M < 1 || N < 8 || N % 8 != 0 || N > (1 << 29) || K < 512 || K % 128 != 0 || K >= (1 << 23)) return -1;
+    float us;
+    const int plan = tg_choose(M, N, K / 128, true, 4, false, true, &us);
+    return us < oa_gemm_fp8_us(M, N, K) ? plan : -1;
+}
+
+extern "C" int oa_ring_sum(void* stream, const void* part, const void* xscale, const void* wscale, void* out,
+                           int M, int N, int splits);
+
+// xs, kb: bytes of a row of x and of a weight row
+static int tg_run(hipStream_t s, const void* x, int64_t xs, const void* w, const void* xscale, const void* wscale,
+                  void* out, void* part, int M, int N, int64_t kb, int form, int splits, int act, bool f8) {
 #define TG_LAUNCH(kernel, BM, BN, lds)                                                             \
     do {                                                                                           \
         const int mt = CEIL_DIV(M, BM);                                                            \
         const int64_t items = (int64_t)CEIL_DIV(N, (BN) / (act ? 2 : 1)) * mt * splits;            \
         if (items > (1 << 28)) return -103;                                                        \
         hipLaunchKernelGGL(kernel, dim3((unsigned)(CEIL_DIV(items, 8) * 8)), dim3(512), lds, s,    \
-                           (const char*)x, xs, (const char*)w, (uint16_t*)out, part, M, N, K, mt,  \
+                           (const char*)x, xs, (const char*)w, (const float*)xscale,               \
+                           (const float*)wscale, (uint16_t*)out, (float*)part, M, N, kb, mt,       \
                            splits, (int)items, act);                                               \
     } while (0)
-#define TG_HALVES(FI, FJ, XS, WS)                                                                       \
-    do {                                                                                                \
-        constexpr int lds = ((XS) * 32 * (FI) + (WS) * 64 * (FJ)) * 128;                                \
-        if (act) TG_LAUNCH((tile_gemm_kernel<FI, FJ, XS, WS, true>), 32 * (FI), 64 * (FJ), lds);        \
-        else TG_LAUNCH((tile_gemm_kernel<FI, FJ, XS, WS, false>), 32 * (FI), 64 * (FJ), lds);           \
+#define TG_HALVES(FI, FJ, XS, WS)                                                                            \
+    do {                                                                                                     \
+        constexpr int lds = ((XS) * 32 * (FI) + (WS) * 64 * (FJ)) * 128;                                     \
+        if (f8) TG_LAUNCH((tile_gemm_kernel<FI, FJ, XS, WS, false, true>), 32 * (FI), 64 * (FJ), lds);       \
+        else if (act) TG_LAUNCH((tile_gemm_kernel<FI, FJ, XS, WS, true, false>), 32 * (FI), 64 * (FJ), lds); \
+        else TG_LAUNCH((tile_gemm_kernel<FI, FJ, XS, WS, false, false>), 32 * (FI), 64 * (FJ), lds);         \
     } while (0)
-#define TG_TURNS(FI, FJ, ST)                                                                            \
-    do {                                                                                                \
-        constexpr int lds = (ST) * 32 * ((FI) + (FJ)) * 128;                                            \
-        if (act) TG_LAUNCH((tile_gemm_turns_kernel<FI, FJ, ST, true>), 32 * (FI), 32 * (FJ), lds);      \
-        else TG_LAUNCH((tile_gemm_turns_kernel<FI, FJ, ST, false>), 32 * (FI), 32 * (FJ), lds);         \
+#define TG_TURNS(FI, FJ, ST)                                                                                  \
+    do {                                                                                                      \
+        constexpr int lds = (ST) * 32 * ((FI) + (FJ)) * 128;                                                  \
+        if (f8) TG_LAUNCH((tile_gemm_turns_kernel<FI, FJ, ST, false, true>), 32 * (FI), 32 * (FJ), lds);      \
+        else if (act) TG_LAUNCH((tile_gemm_turns_kernel<FI, FJ, ST, true, false>), 32 * (FI), 32 * (FJ), lds); \
+        else TG_LAUNCH((tile_gemm_turns_kernel<FI, FJ, ST, false, false>), 32 * (FI), 32 * (FJ), lds);        \
     } while (0)
     switch (form) {
         case 0: TG_HALVES(8, 4, 2, 3); break;
@@ -468,5 +500,36 @@ extern "C" int oa_tile_gemm(void* stream, const void* x, int64_t xs, const void*
 #undef TG_HALVES
 #undef TG_LAUNCH
     HIP_CHECK_LAUNCH();
-    return splits > 1 && out ? oa_ring_sum(stream, scratch, out, M, N, splits) : 0;
+    return 0;
+}
+
+// out [M, N] = x [M, K] w [N, K]^T, x rows xs elements apart. act 1 (silu), 2 (tanh gelu): out =
+// act(x w[:N]^T) * (x w[N:]^T), w [2 N, K]. plan: oa_tile_gemm_plan's. scratch: splits * M * N floats,
+// unused at one split; out null: left there, not added up.
+extern "C" int oa_tile_gemm(void* stream, const void* x, int64_t xs, const void* w, void* out,
+                            void* scratch, int M, int N, int K, int plan, int act) {
+    const int form = plan >> 8, splits = plan & 255;
+    if (M < 1 || N < 8 || N % 8 != 0 || K < 64 || K % 64 != 0) return -100;
+    if (splits < 1 || splits > K / 64 || (splits > 1 ? !scratch || act : !out)) return -101;
+    if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)scratch) % 16 != 0 || xs % 8 != 0)
+        return -102;
+    if (act < 0 || act > 2 || plan < 0) return -104;
+    // a lane's place in a tile is 32 bits wide
+    if (xs < K || xs >= (1 << 22) || ((int64_t)(act ? N : 0) + 256) * K * 2 >= ((int64_t)1 << 32)) return -103;
+    const int rc = tg_run((hipStream_t)stream, x, xs * 2, w, nullptr, nullptr, out, splits > 1 ? scratch : nullptr,
+                          M, N, (int64_t)K * 2, form, splits, act, false);
+    return rc || splits == 1 || !out ? rc : oa_ring_sum(stream, scratch, nullptr, nullptr, out, M, N, splits);
+}
+
+// out [M, N] = (x8 [M, K] w8 [N, K]^T) * xscale[m] * wscale[n], e4m3 rows; plan: oa_tile_gemm_fp8_plan's
+extern "C" int oa_tile_gemm_fp8(void* stream, const void* x8, const void* xscale, const void* w8,
+                                const void* wscale, void* out, void* scratch, int M, int N, int K, int plan) {
+    const int form = plan >> 8, splits = plan & 255;
+    if (M < 1 || N < 8 || N % 8 != 0 || K < 128 || K % 128 != 0 || K >= (1 << 23)) return -100;
+    if (splits < 1 || splits > K / 128 || (splits > 1 && !scratch)) return -101;
+    if (((uintptr_t)x8 | (uintptr_t)w8 | (uintptr_t)out | (uintptr_t)scratch) % 16 != 0) return -102;
+    if (plan < 0) return -104;
+    const int rc = tg_run((hipStream_t)stream, x8, K, w8, xscale, wscale, out, splits > 1 ? scratch : nullptr, M,
+                          N, K, form, splits, 0, true);
+    return rc || splits == 1 ? rc : oa_ring_sum(stream, scratch, xscale, wscale, out, M, N, splits);
 }
