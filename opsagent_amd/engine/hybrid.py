@@ -75,7 +75,7 @@ from torch import nn
 
 from opsagent_amd import ops
 from opsagent_amd.engine.config import HybridLayerSpec, HybridSpec, MixerSpec
-from opsagent_amd.engine.model import ForwardBatch
+from opsagent_amd.engine.model import ForwardBatch, _sums_parts
 from opsagent_amd.ops import mixer_ops as mx
 from opsagent_amd.parallel import get_tp_size
 
@@ -173,6 +173,8 @@ class RotaryWindowAttentionMixer(nn.Module):
 
     Fused projection rows: q | k | v."""
 
+    sums_parts = True           # see _sums_parts: `context`, and the output product for the caller
+
     def __init__(self, hidden: int, m: MixerSpec, eps: float, dtype, gen):
         super().__init__()
         self.H, self.G, self.D, self.Dv = m.heads, m.kv_heads, m.dim, m.vdim
@@ -198,14 +200,17 @@ class RotaryWindowAttentionMixer(nn.Module):
         return {}
 
     def forward(self, h, sb: mx.SeqBatch, kv, state) -> torch.Tensor:
+        return ops.linear(self.context(h, sb, kv), self.o_w)
+
+    def context(self, h, sb: mx.SeqBatch, kv) -> torch.Tensor:
+        """What the output product reads."""
         k_cache, v_cache = kv
         proj = ops.linear(h, self.proj_w)                     # [T, q|k|v]
         q = mx.attn_rope_prepare(proj, self.q_norm_w, self.k_norm_w, self.inv_freq,
                                  self.H, self.G, self.D, self.Dv, self.eps,
                                  k_cache, v_cache, sb)
-        ctx = mx.attention_paged(q, k_cache, v_cache, sb, self.scale,
-                                 window=self.window, sinks=self.sinks)
-        return ops.linear(ctx, self.o_w)
+        return mx.attention_paged(q, k_cache, v_cache, sb, self.scale,
+                                  window=self.window, sinks=self.sinks)
 
     def load(self, get, put, p: str) -> None:
         put(self.proj_w, [get(p + "q"), get(p + "k"), get(p + "v")])
@@ -946,6 +951,8 @@ class GatedMLP(nn.Module):
     """down(act(gate x) * (up x)); gate|up fused; act "silu" | "gelu_tanh" |
     ("clamp_swish", limit, alpha)."""
 
+    sums_parts = True           # see _sums_parts: `inner`, and the down product for the caller
+
     def __init__(self, hidden: int, ff: int, dtype, gen, act: str = "silu"):
         super().__init__()
         self.ff = ff
@@ -954,14 +961,16 @@ class GatedMLP(nn.Module):
         self.down_w = _param(_rand(gen, hidden, ff, std=1.0 / math.sqrt(ff), dtype=dtype))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        return ops.linear(self.inner(x), self.down_w)
+
+    def inner(self, x: torch.Tensor) -> torch.Tensor:
+        """What the down product reads."""
         form = None
         if x.shape[1] % 8 == 0 and self.ff % 8 == 0 and isinstance(self.act, str):
             form = ops._gateup_form(x, self.gate_up_w, self.ff)
         if form:
-            act = ops.gateup_act(x, self.gate_up_w, self.ff, self.act, form)   # fused decode GEMV
-        else:
-            act = mx.act_mul_rows(ops.linear(x, self.gate_up_w), self.ff, self.act)
-        return ops.linear(act, self.down_w)
+            return ops.gateup_act(x, self.gate_up_w, self.ff, self.act, form)   # one launch
+        return mx.act_mul_rows(ops.linear(x, self.gate_up_w), self.ff, self.act)
 
     def load(self, get, put, p: str) -> None:
         put(self.gate_up_w, [get(p + "gate"), get(p + "up")])
@@ -1072,10 +1081,18 @@ class SandwichLayer(nn.Module):
         """x: float32 residual [T, C] (updated in place); h = pre1(x).
         next_norm: the following layer's first norm (None after the last
         layer). Returns (x, next layer's h or None)."""
-        y = self.mixer(h, sb, kv, state)
+        post, nxt = self.post1.params(), self.pre2.params() if self.mlp is not None else next_norm
+        # one row: the add and the norm ride along with the sublayer's last product
+        if x.shape[0] == 1 and _sums_parts(self.mixer):
+            h2 = mx.linear_dyt_norm(self.mixer.context(h, sb, kv), self.mixer.o_w, x, nxt,
+                                    self.dtype, post)
+        else:
+            h2 = mx.dyt_norm(x, nxt, self.dtype, y=self.mixer(h, sb, kv, state), post=post)
         if self.mlp is None:
-            return x, mx.dyt_norm(x, next_norm, self.dtype, y=y, post=self.post1.params())
-        h2 = mx.dyt_norm(x, self.pre2.params(), self.dtype, y=y, post=self.post1.params())
+            return x, h2
+        if x.shape[0] == 1 and _sums_parts(self.mlp):
+            return x, mx.linear_dyt_norm(self.mlp.inner(h2), self.mlp.down_w, x, next_norm,
+                                         self.dtype, self.post2.params())
         m = self.mlp(h2, decode=sb.max_chunk == 1) if self.routed else self.mlp(h2)
         return x, mx.dyt_norm(x, next_norm, self.dtype, y=m, post=self.post2.params())
 

@@ -14,9 +14,7 @@
 // Requires K % 512 == 0 (64 lanes x 8 bf16); callers fall back to hipBLASLt
 // otherwise (and for M > 8, where the MFMA path wins).
 
-#include "common.h"
-#include <algorithm>
-#include <cstdlib>
+#include "mixer_util.h"
 
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 
@@ -205,14 +203,24 @@ __global__ __launch_bounds__(256) void gemv_gateup_kernel(
 // 8.1 / 7.3, 128256 x 2048 85.3 / 81.2, 2048 x 8192 11.7 / 8.3, 16384 x 2048 gate-up 13.4 /
 // 12.7, 2048 x 2048 4.4 / 4.0 (contiguous reads alone run at 6.4 to 6.9 TB/s); asking for
 // the activations before the weights takes another half a microsecond each.
-template <bool NORM, bool ADDRES, int RT, int GR, int XV, int WV>
+//
+// EPI 1 adds a residual row. EPI 2 is followed by what dyt_norm (blocks.hip) would do with the bf16
+// product y in a launch of its own, 3.2 us for 2048 columns in a chain of launches: r += dyt(y; post),
+// out = dyt(r; next) where there is a next norm. A wave's lane i keeps the sum of its row i until all
+// are done and then treats that row, for which it asked at the start.
+struct DytEpilogue {
+    const float *pw, *pb, *pa, *nw, *nb, *na;
+    float* residual;
+};
+
+template <bool NORM, int EPI, int RT, int GR, int XV, int WV>
 __global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restrict__ x,
                                                     const uint32_t* __restrict__ w,
                                                     uint16_t* __restrict__ out,
                                                     const uint32_t* __restrict__ wn,
                                                     const uint16_t* __restrict__ res, int N, int K,
                                                     int waves, int full, int extra, float eps,
-                                                    int act) {
+                                                    int act, DytEpilogue dy) {
     extern __shared__ __attribute__((aligned(16))) float xl[];   // [2][K / 2]
     __shared__ float part[8];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -247,7 +255,13 @@ __global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restri
         xv[j] = reinterpret_cast<const uint4*>(x)[i];
         if (NORM) nv[j] = reinterpret_cast<const uint4*>(wn)[i];
     }
-    const float rs = ADDRES ? bf16_to_f32(res[min(wave + lane * (int64_t)waves, N - (int64_t)1)]) : 0.0f;
+    const int own = (int)min(wave + lane * (int64_t)waves, N - (int64_t)1);
+    const float rs = EPI == 1 ? bf16_to_f32(res[own]) : EPI == 2 ? dy.residual[own] : 0.0f;
+    float pw = 0, pb = 0, pa = 0, nw = 0, nb = 0, na = 0, mine = 0;
+    if constexpr (EPI == 2) {
+        pw = dy.pw[own], pb = dy.pb[own], pa = dy.pa[0];
+        if (out) nw = dy.nw[own], nb = dy.nb[own], na = dy.na[0];
+    }
     __builtin_amdgcn_sched_barrier(0);
     load(a);
     __builtin_amdgcn_sched_barrier(0);
@@ -322,9 +336,10 @@ __global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restri
         if (++ug == groups) {
             float v0 = wave_reduce_sum(acc[0]);
             if (RT == 2) v0 = gate_act(v0, act) * wave_reduce_sum(acc[RT - 1]);
-            if (ADDRES)
+            if (EPI == 1)
                 v0 += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rs), un));
-            if (lane == 0) out[ur] = f32_to_bf16(v0);
+            if (EPI == 2) mine = lane == un ? v0 : mine;
+            else if (lane == 0) out[ur] = f32_to_bf16(v0);
 #pragma unroll
             for (int t = 0; t < RT; ++t) acc[t] = 0.0f;
             ug = 0;
@@ -347,11 +362,19 @@ __global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restri
     } else if (n < total) {
         use(a);
     }
+    if constexpr (EPI == 2) {
+        if (lane < full + (wave < extra)) {
+            const float y = bf16_to_f32(f32_to_bf16(mine)), r = rs + (tanh_f32(pa * y) * pw + pb);
+            dy.residual[own] = r;
+            if (out) out[own] = f32_to_bf16(tanh_f32(na * r) * nw + nb);
+        }
+    }
 }
 
-// mode as in oa_gemv_ex; gateup > 0: N gate and N up rows, activation gateup - 1
+// mode as in oa_gemv_ex, 4: dy; gateup > 0: N gate and N up rows, activation gateup - 1
 static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const void* wn,
-                 const void* res, int N, int K, float eps, int mode, int gateup) {
+                 const void* res, int N, int K, float eps, int mode, int gateup,
+                 const DytEpilogue& dy = {}) {
     // Rows of 4096, and many of 2048: blocks of four waves, of two rows a wave (gate-up one
     // pair), so that CUs even out; the image of a block is quickly made. No more than 32
     // blocks per CU. Us, blocks of eight waves and up to 64 rows a wave / this: 6144 x 4096
@@ -387,7 +410,7 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
 #define G1X(NV, RV, RT, GR, XV, WV)                                                                   \
     hipLaunchKernelGGL((gemv1_kernel<NV, RV, RT, GR, XV, WV>), dim3(blocks), dim3(WV * 64), lds, st,  \
                        (const uint32_t*)x, (const uint32_t*)w, (uint16_t*)out, (const uint32_t*)wn,   \
-                       (const uint16_t*)res, N, K, waves, N / waves, N % waves, eps, gateup - 1)
+                       (const uint16_t*)res, N, K, waves, N / waves, N % waves, eps, gateup - 1, dy)
 #define G1(NV, RV, RT, GR)                   \
     do {                                     \
         if (wv == 4) G1X(NV, RV, RT, GR, 2, 4);         \
@@ -395,21 +418,23 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
         else G1X(NV, RV, RT, GR, 4, 8);                 \
     } while (0)
     if (gateup) {
-        if (mode & 1) G1(true, false, 2, 4);
-        else G1(false, false, 2, 4);
+        if (mode & 1) G1(true, 0, 2, 4);
+        else G1(false, 0, 2, 4);
     } else if (K % 4096 == 0) {
         switch (mode) {
-            case 0: G1(false, false, 1, 8); break;
-            case 1: G1(true, false, 1, 8); break;
-            case 2: G1(false, true, 1, 8); break;
-            default: G1(true, true, 1, 8); break;
+            case 0: G1(false, 0, 1, 8); break;
+            case 1: G1(true, 0, 1, 8); break;
+            case 2: G1(false, 1, 1, 8); break;
+            case 3: G1(true, 1, 1, 8); break;
+            default: G1(false, 2, 1, 8); break;
         }
     } else {
         switch (mode) {
-            case 0: G1(false, false, 1, 4); break;
-            case 1: G1(true, false, 1, 4); break;
-            case 2: G1(false, true, 1, 4); break;
-            default: G1(true, true, 1, 4); break;
+            case 0: G1(false, 0, 1, 4); break;
+            case 1: G1(true, 0, 1, 4); break;
+            case 2: G1(false, 1, 1, 4); break;
+            case 3: G1(true, 1, 1, 4); break;
+            default: G1(false, 2, 1, 4); break;
         }
     }
 #undef G1
@@ -419,6 +444,19 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
 }
 // the float32 image of the activations fits the LDS of two blocks per CU
 static bool gemv1_ok(int M, int K) { return M == 1 && K % 2048 == 0 && K <= 16384; }
+
+// residual += dyt(x W^T; pw, pb, pa), out = dyt(residual; nw, nb, na) unless null: one row x [K],
+// residual [N] and the norms float32 (pa, na: one number each); nothing where gemv1 does not take it
+extern "C" int oa_gemv_dyt(void* stream, const void* x, const void* w, void* residual, const void* pw,
+                           const void* pb, const void* pa, const void* nw, const void* nb, const void* na,
+                           void* out, int N, int K) {
+    if (N < 1 || !gemv1_ok(1, K) || N > 256 * 64 * 8) return -100;
+    if (!x || !w || !residual || !pw || !pb || !pa || (out && (!nw || !nb || !na))) return -101;
+    if (((uintptr_t)x | (uintptr_t)w) % 16 != 0) return -102;
+    const DytEpilogue dy = {(const float*)pw, (const float*)pb, (const float*)pa, (const float*)nw,
+                            (const float*)nb, (const float*)na, (float*)residual};
+    return gemv1((hipStream_t)stream, x, w, out, nullptr, nullptr, N, K, 0.0f, 4, 0, dy);
+}
 
 static bool gemv_bf16_use_mfma(int M, int K, int gateup);
 extern "C" int oa_gemv_bf16_mfma(void* stream, const void* x, const void* w,

@@ -417,6 +417,36 @@ def dyt_norm(residual: torch.Tensor, nxt: Optional[Tuple[torch.Tensor, ...]], ou
     return out
 
 
+def linear_dyt_norm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
+                    nxt: Optional[Tuple[torch.Tensor, ...]], out_dtype,
+                    post: Tuple[torch.Tensor, ...]) -> Optional[torch.Tensor]:
+    """dyt_norm with y = x @ w^T: for one row of bf16 in one launch, the epilogue of the one-row
+    product (gemv.hip), where that takes the row."""
+    from opsagent_amd import ops
+
+    K = x.shape[-1]
+    if not (x.is_cuda and x.shape[0] == 1 and x.dtype == w.dtype == out_dtype == torch.bfloat16
+            and x.dim() == w.dim() == 2 and w.shape[1] == K and residual.shape == (1, w.shape[0])
+            and K % 2048 == 0 and K <= 16384 and w.shape[0] <= 131072 and ops._gemv_m_ok(1)
+            and x.is_contiguous() and w.is_contiguous() and ops._plain_call(x, w)
+            and residual.dtype == torch.float32 and residual.is_contiguous()
+            and x.device == w.device == residual.device
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0):
+        return dyt_norm(residual, nxt, out_dtype, y=ops.linear(x, w), post=post)
+    N = w.shape[0]
+    for t in post + (nxt or ()):
+        assert t.dtype == torch.float32 and t.is_contiguous() and t.numel() in (1, N)
+    lib, hip = _lib()
+    out = torch.empty(1, N, dtype=out_dtype, device=x.device) if nxt is not None else None
+    kernels = hip.get_lib()
+    hip.check(kernels.oa_gemv_dyt(
+        hip.current_stream_ptr(), x.data_ptr(), w.data_ptr(), residual.data_ptr(),
+        *(t.data_ptr() for t in post),
+        *((t.data_ptr() for t in nxt) if nxt is not None else (None, None, None)),
+        out.data_ptr() if out is not None else None, N, K), "oa_gemv_dyt")
+    return out
+
+
 def rotary_inv_freq(dims: int, base: float, scaling: Optional[dict] = None) -> torch.Tensor:
     """float32 [dims/2] rotation frequencies base^(-2i/dims). `scaling`
     {factor, low, high, original} slows long waves: a wavelength below
