@@ -206,11 +206,9 @@ class RotaryWindowAttentionMixer(nn.Module):
         """What the output product reads."""
         k_cache, v_cache = kv
         proj = ops.linear(h, self.proj_w)                     # [T, q|k|v]
-        q = mx.attn_rope_prepare(proj, self.q_norm_w, self.k_norm_w, self.inv_freq,
-                                 self.H, self.G, self.D, self.Dv, self.eps,
-                                 k_cache, v_cache, sb)
-        return mx.attention_paged(q, k_cache, v_cache, sb, self.scale,
-                                  window=self.window, sinks=self.sinks)
+        return mx.attn_rope_rows(proj, self.q_norm_w, self.k_norm_w, self.inv_freq,
+                                 self.H, self.G, self.D, self.Dv, self.eps, k_cache, v_cache, sb,
+                                 self.scale, window=self.window, sinks=self.sinks)
 
     def load(self, get, put, p: str) -> None:
         put(self.proj_w, [get(p + "q"), get(p + "k"), get(p + "v")])

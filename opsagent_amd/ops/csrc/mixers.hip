@@ -971,9 +971,24 @@ __global__ __launch_bounds__(256, FULL && MAXD <= 8 ? 3 : 1) void attn_bias_mfma
 // one of 16000: 81 -> 23.8; four of 40: 8.7 -> 4.6. With the page looked up key
 // by key in each piece the last but one took 24.6 in the same splits, but the
 // 64 rows 143 and one block going through 16000 keys 214 instead of 174.
+//
+// ROPE: q is the projection itself, rows of q | k | v: what attn_rope_prepare (blocks.hip; norm and
+// rotation of the heads, the new key and value to their slot) does in a launch of 4 us before this one,
+// every block does for its own heads while its first keys are on their way, each sum of squares
+// over four lanes. The slot of the new key is written by one block of its kv head and read by none: its key
+// and value go from registers into the pieces that hold it. Keys past it count for nothing and repeat it.
+struct RowsRope {
+    const float *qw, *kw, *inv_freq;
+    const int* slots;
+    bf16s *k_cache, *v_cache;
+    int64_t qs;
+    int nfreq;
+    float eps;
+};
+
 constexpr int rows_piece(int D) { return D == 256 ? 16 : 32; }
 
-template <int D, int HB>
+template <int D, int HB, bool ROPE = false>
 __global__ __launch_bounds__(512) void attn_rows_kernel(
     const bf16s* __restrict__ q, const bf16s* __restrict__ gate, int64_t gs,
     const bf16s* __restrict__ k_cache, const bf16s* __restrict__ v_cache,
@@ -982,7 +997,7 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
     const int* __restrict__ block_table, int max_blocks, int block_size,
     const float* __restrict__ slopes, const float* __restrict__ sinks, int B, int H, int G,
     float scale, int nsplit, int window, int64_t vrow, int Gv, float softcap, int64_t os,
-    float oscale, int keep, int gch) {
+    float oscale, int keep, int gch, RowsRope rp) {
     constexpr int NW = 8, KS = D / 32, TK = rows_piece(D), MT = TK / 16;
     constexpr int VL = D / 8, KP = 64 / VL, NV = TK / KP;
     __shared__ __align__(16) float ps[NW][TK * HB];
@@ -1017,11 +1032,64 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
     const int wlim = window > 0 ? window : 0x7fffffff;
     const int bsh = 31 - __clz(block_size), bmask = block_size - 1;
 
-    s8_t qf[KS], kf[MT][KS];
-    uint4 vf[NV];
-    const bf16s* qr = q + ((int64_t)lo * H + h) * D + 8 * lg;
+    s8_t qf[KS], kf[MT][KS], nk[ROPE ? KS : 1];
+    uint4 vf[NV], nv = {};
+    const bf16s* qr = ROPE ? q + lo * rp.qs + h * D + 8 * lg : q + ((int64_t)lo * H + h) * D + 8 * lg;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const s8_t*>(qr + 32 * ks);
+    for (int ks = 0; ks < KS; ++ks) {
+        qf[ks] = *reinterpret_cast<const s8_t*>(qr + 32 * ks);
+        if constexpr (ROPE) nk[ks] = *reinterpret_cast<const s8_t*>(q + lo * rp.qs + (H + g) * D + 8 * lg + 32 * ks);
+    }
+    if constexpr (ROPE) {
+        nv = *reinterpret_cast<const uint4*>(q + lo * rp.qs + (H + G + g % Gv) * D + 8 * (lane % VL));
+        __shared__ float turn[2][D / 2];
+        if (threadIdx.x < D / 2) {
+            float s_ = 0.0f, c_ = 1.0f;
+            if ((int)threadIdx.x < rp.nfreq) sincosf((float)pos * rp.inv_freq[threadIdx.x], &s_, &c_);
+            turn[0][threadIdx.x] = c_;
+            turn[1][threadIdx.x] = s_;
+        }
+        __syncthreads();
+        // this lane's channels of a head, 32 ks + 8 lg and up: normed, rotated, as bf16 again
+        auto prepare = [&](s8_t (&f)[KS], const float* w) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float v = bf16_to_f32((uint16_t)f[ks][e]);
+                    ss = fmaf(v, v, ss);
+                }
+            ss += __shfl_xor(ss, 16, WAVE);
+            ss += __shfl_xor(ss, 32, WAVE);
+            const float rn = 1.0f / sqrtf(ss / (float)D + rp.eps);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const int ch = 32 * ks + 8 * lg;
+                float wv[8];
+                ld8(w, ch, wv);
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) {
+                    const float a = bf16_to_f32((uint16_t)f[ks][e]) * rn * wv[e];
+                    const float c = bf16_to_f32((uint16_t)f[ks][e + 1]) * rn * wv[e + 1];
+                    const float cc = turn[0][(ch + e) >> 1], sv = turn[1][(ch + e) >> 1];
+                    f[ks][e] = (short)f32_to_bf16(a * cc - c * sv);
+                    f[ks][e + 1] = (short)f32_to_bf16(c * cc + a * sv);
+                }
+            }
+        };
+        prepare(qf, rp.qw);
+        prepare(nk, rp.kw);
+        if (split == 0 && wave == 0 && blockIdx.y % hgroups == 0) {
+            const int64_t slot = rp.slots[lo];
+            if (lc == 0)
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+                    *reinterpret_cast<s8_t*>(rp.k_cache + (slot * G + g) * D + 8 * lg + 32 * ks) = nk[ks];
+            if (g < Gv && lane < VL)
+                *reinterpret_cast<uint4*>(rp.v_cache + slot * vrow + g * D + 8 * lane) = nv;
+        }
+    }
     // A piece lies within one page if pages are no smaller: its page is then a
     // value of the whole wave, and the wave looks 64 of its pieces up at once
     const KeyTiles tiles = key_tiles(pos, pos / TK + 1, TK, window, keep);
@@ -1047,6 +1115,10 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks)
                 kf[mt][ks] = *reinterpret_cast<const s8_t*>(kp + 32 * ks);
+            if constexpr (ROPE)
+                if (k0 + TK > pos && k0 + 16 * mt + lc >= pos)
+#pragma unroll
+                    for (int ks = 0; ks < KS; ++ks) kf[mt][ks] = nk[ks];
         }
     };
     const bf16s* vbase = v_cache + (g % Gv) * D + 8 * (lane % VL);
@@ -1054,6 +1126,11 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
 #pragma unroll
         for (int i = 0; i < NV; ++i)
             vf[i] = *reinterpret_cast<const uint4*>(vbase + slot(base, k0, KP * i + lane / VL) * vrow);
+        if constexpr (ROPE)
+            if (k0 + TK > pos)
+#pragma unroll
+                for (int i = 0; i < NV; ++i)
+                    if (k0 + KP * i + lane / VL >= pos) vf[i] = nv;
     };
     float acc[HB][8], m = -INFINITY, l = 0.0f;
 #pragma unroll
@@ -2166,11 +2243,60 @@ extern "C" int oa_attn_rows_splits(int H, int G, int D, int Dv, int dt, int max_
                                 std::max(16, std::min(pieces / 8, 64))));
 }
 
-template <int HB, typename... A>
+template <int HB, bool ROPE, typename... A>
 static void launch_attn_rows(int D, dim3 grid, hipStream_t s, A... a) {
-    if (D == 64) hipLaunchKernelGGL((attn_rows_kernel<64, HB>), grid, dim3(512), 0, s, a...);
-    else if (D == 128) hipLaunchKernelGGL((attn_rows_kernel<128, HB>), grid, dim3(512), 0, s, a...);
-    else hipLaunchKernelGGL((attn_rows_kernel<256, HB>), grid, dim3(512), 0, s, a...);
+    if (D == 64) hipLaunchKernelGGL((attn_rows_kernel<64, HB, ROPE>), grid, dim3(512), 0, s, a...);
+    else if (D == 128) hipLaunchKernelGGL((attn_rows_kernel<128, HB, ROPE>), grid, dim3(512), 0, s, a...);
+    else if constexpr (!ROPE) hipLaunchKernelGGL((attn_rows_kernel<256, HB>), grid, dim3(512), 0, s, a...);
+}
+
+// heads of a block: fewer than share the keys where CUs are left over, though keys are then read
+// more than once
+static int rows_hb(int R, int pairs, int nsplit) {
+    int hb = attn_hb(R);
+    while (hb > 1 && pairs * (R / hb) * nsplit * 2 <= 256) hb /= 2;
+    return hb;
+}
+
+// Decode steps straight from the projection rows q | k | v [T, >= (H + G + Gv) * D]: attn_rope_prepare and
+// attn_bias_paged in one launch (two with splits). One new token a sequence, heads that attn_rows_kernel
+// takes (of 64 or 128: at 256 the new key's registers spill), weighted head norms, values of the keys'
+// size in a cache of their own (rows of Gv * D).
+extern "C" int oa_attn_rows_rope(void* stream, const void* qkv, int64_t qs, const void* qw, const void* kw,
+                                 const void* inv_freq, int nfreq, float eps, const void* slot_mapping,
+                                 void* k_cache, void* v_cache, void* out, void* part_o, void* part_ml,
+                                 const void* cu, const void* past, const void* block_table, int max_blocks,
+                                 int block_size, const void* sinks, int T, int B, int ntiles, int H, int G,
+                                 int Gv, int D, float scale, int nsplit, int window, int64_t os) {
+    if (T <= 0 || ntiles <= 0) return 0;
+    if (G < 1 || H % G != 0 || Gv < 1 || G % Gv != 0 || D > 128 || !attn_rows(H, G, D, D, 0, 1)) return -100;
+    if (nfreq < 0 || 2 * nfreq > D || !qw || !kw || (nfreq && !inv_freq) || !slot_mapping) return -101;
+    if (qs % 8 != 0 || qs < (int64_t)(H + G + Gv) * D || window < 0 || os < (int64_t)H * D) return -105;
+    if (((uintptr_t)qkv | (uintptr_t)qw | (uintptr_t)kw | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 != 0)
+        return -102;
+    if (nsplit < 1 || (nsplit > 1 && (!part_o || !part_ml))) return -104;
+    hipStream_t s = (hipStream_t)stream;
+    const int R = H / G, hb = rows_hb(R, ntiles * G, nsplit);
+    const dim3 grid(ntiles, G * (R / hb), nsplit);
+    const RowsRope rp = {(const float*)qw, (const float*)kw, (const float*)inv_freq, (const int*)slot_mapping,
+                         (bf16s*)k_cache, (bf16s*)v_cache, qs, nfreq, eps};
+#define ROPE_ARGS                                                                                     \
+    D, grid, s, (const bf16s*)qkv, (const bf16s*)nullptr, (int64_t)0, (const bf16s*)k_cache,          \
+        (const bf16s*)v_cache, (bf16s*)out, (float*)part_o, (float*)part_ml, (const int*)cu,          \
+        (const int*)past, (const int*)block_table, max_blocks, block_size, (const float*)nullptr,     \
+        (const float*)sinks, B, H, G, scale, nsplit, window, (int64_t)Gv * D, Gv, 0.0f, os, 1.0f, 0, 0, rp
+    if (hb == 4) launch_attn_rows<4, true>(ROPE_ARGS);
+    else if (hb == 2) launch_attn_rows<2, true>(ROPE_ARGS);
+    else launch_attn_rows<1, true>(ROPE_ARGS);
+#undef ROPE_ARGS
+    HIP_CHECK_LAUNCH();
+    if (nsplit > 1) {
+        hipLaunchKernelGGL((attn_combine_kernel<bf16s>), dim3((unsigned)((int64_t)T * H)), dim3(256), 0, s,
+                           (const float*)part_o, (const float*)part_ml, (const bf16s*)nullptr, (int64_t)0,
+                           (const float*)sinks, (bf16s*)out, H, D, nsplit, os, 1.0f, 0);
+        HIP_CHECK_LAUNCH();
+    }
+    return 0;
 }
 
 // ntiles = sum_b ceil(n_b / TQ) (host-computed). part_* may be null when nsplit == 1.
@@ -2205,18 +2331,16 @@ extern "C" int oa_attn_bias_paged(void* stream, const void* q, const void* gate,
         if (gate && gch && (gs % 4 != 0 || (uintptr_t)gate % 8 != 0)) return -110;   // and gate loads
         const int R = H / G, HB = attn_hb(R);
         if (attn_rows(H, G, D, Dv, dt, max_chunk)) {
-            // CUs left over: fewer heads a block, though keys are then read more than once
-            int hb = HB;
-            while (hb > 1 && ntiles * G * (R / hb) * nsplit * 2 <= 256) hb /= 2;
+            const int hb = rows_hb(R, ntiles * G, nsplit);
             dim3 grid(ntiles, G * (R / hb), nsplit);
 #define ROW_ARGS                                                                                  \
     D, grid, s, (const bf16s*)q, (const bf16s*)gate, gs, (const bf16s*)k_cache,                   \
         (const bf16s*)v_cache, (bf16s*)out, (float*)part_o, (float*)part_ml, (const int*)cu,      \
         (const int*)past, (const int*)block_table, max_blocks, block_size, (const float*)slopes,  \
-        (const float*)sinks, B, H, G, scale, nsplit, window, vrow, Gv, softcap, os, oscale, keep, gch
-            if (hb == 4) launch_attn_rows<4>(ROW_ARGS);
-            else if (hb == 2) launch_attn_rows<2>(ROW_ARGS);
-            else launch_attn_rows<1>(ROW_ARGS);
+        (const float*)sinks, B, H, G, scale, nsplit, window, vrow, Gv, softcap, os, oscale, keep, gch, RowsRope{}
+            if (hb == 4) launch_attn_rows<4, false>(ROW_ARGS);
+            else if (hb == 2) launch_attn_rows<2, false>(ROW_ARGS);
+            else launch_attn_rows<1, false>(ROW_ARGS);
 #undef ROW_ARGS
             HIP_CHECK_LAUNCH();
         } else {

@@ -171,6 +171,8 @@ def _declare_mixers(lib: ctypes.CDLL) -> None:
         "oa_attn_prepare": [p, p, i64, p, p, p, p, p, p, p, p, i, i, i, i, i, i, f, i],
         "oa_attn_bias_geometry": [i, i, i, i, i, i, ip, ip, ip, ip],
         "oa_attn_rows_splits": [i, i, i, i, i, i, i, i],
+        "oa_attn_rows_rope": [p, p, i64, p, p, p, i, f, p, p, p, p, p, p, p, p, p, i, i, p,
+                              i, i, i, i, i, i, i, f, i, i, i64],
         "oa_attn_bias_paged": [p, p, p, i64, p, p, p, p, p, p, p, p, i, i, p, p,
                                i, i, i, i, i, i, i, f, i, i, i, i, i64, i, f, i64, f, i, i],
         "oa_dyt_norm": [p, p, i64, i, i64, i, p, p, p, p, p, p, p, p, p, p, i, i, i, p, p, p, p, p, p, i, i],

@@ -557,6 +557,54 @@ def attn_rope_prepare(qkv: torch.Tensor, q_norm_w: Optional[torch.Tensor],
     return q
 
 
+def attn_rope_rows(qkv: torch.Tensor, q_norm_w: torch.Tensor, k_norm_w: torch.Tensor,
+                   inv_freq: torch.Tensor, H: int, G: int, D: int, Dv: int, eps: float,
+                   k_cache: torch.Tensor, v_cache: torch.Tensor, sb: SeqBatch, scale: float,
+                   window: Optional[int] = None,
+                   sinks: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """attn_rope_prepare and attention_paged of its queries, [T, H*Dv]; decode steps in one launch
+    (two with key splits) where the kernel for them takes the heads (mixers.hip)."""
+    splits = 0
+    # (the attributes first: most calls that are no such step end there)
+    if (sb.max_chunk == 1 and qkv.is_cuda and qkv.dtype == torch.bfloat16 and D == Dv <= 128
+            and k_cache.dtype == v_cache.dtype == qkv.dtype and H % G == 0
+            and k_cache.shape[2:] == v_cache.shape[2:] == (G, D)
+            and k_cache.is_contiguous() and v_cache.is_contiguous()
+            and qkv.stride(1) == 1 and qkv.stride(0) % 8 == 0
+            and (qkv.data_ptr() | q_norm_w.data_ptr() | k_norm_w.data_ptr()) % 16 == 0
+            and all(t.dtype == torch.float32 and t.is_contiguous()
+                    for t in (q_norm_w, k_norm_w, inv_freq))
+            and q_norm_w.numel() == k_norm_w.numel() == D and 2 * inv_freq.numel() <= D):
+        lib, hip = _lib()
+        tokens = sb.cu[sb.num_seqs] - sb.cu[0]         # one block row each
+        KT = attn_geometry(H, G, D, Dv, 0, 1)[1]
+        reach = min(sb.max_total, window + 1 + KT) if window else sb.max_total
+        splits = lib.oa_attn_rows_splits(H, G, D, Dv, 0, 1, tokens, reach) if tokens > 0 else 0
+    if not splits:
+        q = attn_rope_prepare(qkv, q_norm_w, k_norm_w, inv_freq, H, G, D, Dv, eps, k_cache,
+                              v_cache, sb)
+        return attention_paged(q, k_cache, v_cache, sb, scale, window=window, sinks=sinks)
+    assert sinks is None or (sinks.dtype == torch.float32 and sinks.numel() == H
+                             and sinks.is_contiguous())
+    T = qkv.shape[0]
+    out = torch.empty(T, H * D, dtype=qkv.dtype, device=qkv.device)
+    part_o = part_ml = None
+    if splits > 1:
+        part_o = torch.empty(T * H * splits, D, dtype=torch.float32, device=qkv.device)
+        part_ml = torch.empty(T * H * splits, 2, dtype=torch.float32, device=qkv.device)
+    hip.check(lib.oa_attn_rows_rope(
+        hip.current_stream_ptr(), qkv.data_ptr(), qkv.stride(0), q_norm_w.data_ptr(),
+        k_norm_w.data_ptr(), inv_freq.data_ptr(), inv_freq.numel(), eps,
+        sb.slot_mapping.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
+        part_o.data_ptr() if part_o is not None else None,
+        part_ml.data_ptr() if part_ml is not None else None,
+        sb.cu_t.data_ptr(), sb.past_t.data_ptr(), sb.block_table.data_ptr(),
+        sb.block_table.shape[1], k_cache.shape[1],
+        sinks.data_ptr() if sinks is not None else None, T, sb.num_seqs, tokens, H, G, G, D,
+        float(scale), splits, int(window) if window else 0, H * D), "oa_attn_rows_rope")
+    return out
+
+
 ACTS = {"silu": 0, "gelu_tanh": 1, "clamp_swish": 2, "relu2": 3}
 
 

@@ -145,3 +145,47 @@ def test_prompts(D, H, G, chunks, page, opts):
            + 4 * ctx ** 0.5 * 2.0 ** -24 + 2.0 ** -21 + 2.0 ** -15)
     bound = want.abs() * 2.0 ** -8 + 2 * rel * float(v.float().abs().max())
     assert ((got - want).abs() <= bound).all(), ((got - want).abs() / bound).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [None, 1, 3])
+@pytest.mark.parametrize("ctx,H,G,D,page,window,nfreq,sinks", [
+    ([1, 32, 33, 64, 513], 32, 8, 128, 32, None, 64, False),
+    ([257, 16, 700, 1], 6, 2, 128, 8, 40, 20, True),             # pages below a piece
+    ([2005, 511], 16, 4, 128, 32, 512, 64, True),
+    ([31, 300, 1], 12, 2, 64, 16, 1, 32, False),
+    ([129, 1030], 4, 4, 64, 64, 33, 0, True),
+])
+def test_from_the_projection(monkeypatch, splits, ctx, H, G, D, page, window, nfreq, sinks):
+    """Head norms, rotation and cache writes inside the launch: the rows that are written, and the
+    result, against the two launches; every other row of the cache stays, and what lies in the new
+    token's slots before does not matter."""
+    g = torch.Generator(device="cuda").manual_seed(sum(ctx) + D)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    need = [(c + page - 1) // page for c in ctx]
+    perm = torch.randperm(sum(need), generator=torch.Generator().manual_seed(1)).tolist()
+    table = [perm[sum(need[:i]):sum(need[:i + 1])] for i in range(len(ctx))]
+    past, T = [c - 1 for c in ctx], len(ctx)
+    qkv = rn(T, (H + 2 * G) * D + 8).bfloat16()[:, :(H + 2 * G) * D]        # rows apart
+    qw, kw = 1 + 0.1 * rn(D), 1 + 0.1 * rn(D)
+    freq = mx.rotary_inv_freq(2 * nfreq, 10000.0).cuda() if nfreq else torch.empty(0, device="cuda")
+    k, v = rn(sum(need), page, G, D).bfloat16(), rn(sum(need), page, G, D).bfloat16()
+    sk = rn(H) if sinks else None
+    sb = mx.SeqBatch.build([(p, 1, i, t) for i, (p, t) in enumerate(zip(past, table))], page, "cuda")
+    lib = mx._lib()[0]
+    if splits:
+        monkeypatch.setattr(lib, "oa_attn_rows_splits", lambda *args: splits)
+    k1, v1, k2, v2 = k.clone(), v.clone(), k.clone(), v.clone()
+    q = mx.attn_rope_prepare(qkv, qw, kw, freq, H, G, D, D, 1e-6, k1, v1, sb)
+    want = mx.attention_paged(q, k1, v1, sb, D ** -0.5, window=window, sinks=sk)
+    slots = sb.slot_mapping.long()
+    k2.view(-1, G, D)[slots] = float("nan")
+    v2.view(-1, G, D)[slots] = float("nan")
+    got = mx.attn_rope_rows(qkv, qw, kw, freq, H, G, D, D, 1e-6, k2, v2, sb, D ** -0.5,
+                            window=window, sinks=sk)
+    # the sums of squares in another order: a few queries and keys round to the other neighbour
+    assert torch.equal(v2, v1)
+    assert torch.allclose(k2.float(), k1.float(), rtol=2.0 ** -7, atol=0)
+    assert (k2 != k1).float().mean() < 0.01
+    assert (got.float() - want.float()).norm() <= 2.0 ** -8 * want.float().norm()
+    assert (got.float() - want.float()).abs().max() <= 2.0 ** -6 * v.float().abs().max()
