@@ -120,6 +120,7 @@ class Attention(nn.Module):
         )
         self.o_w = nn.Parameter(_shard(o_w, 1, rank, tp), requires_grad=False)
         self.fp8 = False  # set by LlamaForCausalLM.quantize_fp8_
+        self.fp8_experts = spec.moe_dtype == "fp8"
 
     def _qkv(self, x: torch.Tensor) -> torch.Tensor:
         if self.fp8:
@@ -178,7 +179,8 @@ class Attention(nn.Module):
                 k_full = k.unsqueeze(0)
                 v_full = v.unsqueeze(0)
             out = ops.attention_prefill(
-                q.unsqueeze(0), k_full, v_full, scale=self.scale
+                q.unsqueeze(0), k_full, v_full, scale=self.scale,
+                steady=self.fp8 or self.fp8_experts,
             )
             out = out.view(T, self.hq * self.hd)
         else:

@@ -1290,15 +1290,49 @@ def _prefill_splits(B: int, Hq: int, Hk: int, Sq: int, Skv: int) -> Tuple[int, b
     return max(1, min(tiles, 256 // max(1, blocks))), True
 
 
+def _prefill_plan(
+    B: int, Hq: int, Hk: int, Sq: int, Skv: int, steady: bool = False
+) -> Tuple[int, int]:
+    """(key splits, form) of prefill attention: form 0 in key groups, 1 merged, 2 steady.
+
+    What :func:`_prefill_splits` splits, the steady form as it says; the others where that is
+    faster than key groups within a block, which halve and quarter a chain of tiles without
+    sums in memory. Up to 128 queries by the estimates below, us: over 260 sizes (4 to 128
+    heads, 2 to 128 queries, 3 to 24 tiles) 0.2 per cent from the better of the two on average
+    and 12 at the most (4 heads, 128 queries, 3 tiles, not split / split: 11.8 / 13.2; both
+    sides: 80 heads, 128 queries, 6 tiles 18.2 / 25.8, 4 heads, 16 queries, 11 tiles 22.3 /
+    12.2). More queries: where few splits fill the chip, from as
+    many tiles as make up for the sums that they leave (16, 20 or 26, 34 and 70 tiles, not split
+    / in two, 32 heads on 8 of 700 to 1000 queries: 45 / 67, 55 / 74, 88 / 102, 183 / 175; in
+    three, 520 queries, 12 and 20 tiles: 36 / 42, 54 / 52; in four, 400 queries, 16 and 26
+    tiles: 35 / 40, 51 / 49, and 1000 queries of 16 heads, 26 and 34: 51 / 56, 64 / 65; in
+    six, 300 queries, 12 and 20 tiles: 26 / 30, 39 / 37)."""
+    splits, merged = _prefill_splits(B, Hq, Hk, Sq, Skv)
+    if steady or splits == 1:
+        return splits, 1 if merged else 2 * steady
+    tiles = (Skv + 127) // 128
+    if merged:
+        least = (0, 0, 64, 20, 28, 18, 16)
+        worth = splits >= len(least) or tiles >= least[splits]
+    else:
+        sums = B * Hq * Sq * splits * 520e-6          # MB
+        chain = (2.0 if Sq <= 64 else 2.6) * -(-tiles // splits)
+        worth = chain + 6.0 + 0.6 * sums < 1.85 * tiles + 4.0
+    return (splits if worth else 1), int(merged)
+
+
 def attention_prefill(
     q: torch.Tensor,
     k: torch.Tensor,
     v: torch.Tensor,
     scale: Optional[float] = None,
     causal: bool = True,
+    steady: bool = False,
 ) -> torch.Tensor:
     """q [B, Sq, Hq, D]; k, v [B, Skv, Hk, D] (token-major layouts; the CPU
-    reference uses [B, H, S, D], so the dispatch transposes for it)."""
+    reference uses [B, H, S, D], so the dispatch transposes for it). ``steady``: a row's keys
+    added up in the one order that callers with 8-bit activations are held to: any other
+    rounding of a weight moves some of those to the next 8-bit value."""
     if not _is_gpu(q):
         out = torch_ref.attention_prefill(
             q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), scale, causal
@@ -1314,21 +1348,22 @@ def attention_prefill(
     scale = scale if scale is not None else D ** -0.5
     lib, hip = _lib()
     out = torch.empty(B, Sq, Hq, D, dtype=q.dtype, device=q.device)
-    splits, merged = _prefill_splits(B, Hq, Hk, Sq, Skv)
+    steady = steady or scale <= 0.0        # the other forms take their maxima before the scale
+    splits, form = _prefill_plan(B, Hq, Hk, Sq, Skv, steady)
     if splits > 1 and D == 128 and "OPSAGENT_PREFILL_VARIANT" not in os.environ:
         part = torch.empty(splits, B, Sq, Hq, D + 2, dtype=torch.float32, device=q.device)
         sums = splits * B * Sq * Hq * D * 4
         rc = lib.oa_attention_prefill_split(
             hip.current_stream_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
             out.data_ptr(), part.data_ptr(), part.data_ptr() + sums, B, Hq, Hk, Sq, Skv, D,
-            scale, q.stride(1), k.stride(1), v.stride(1), splits, int(merged),
+            scale, q.stride(1), k.stride(1), v.stride(1), splits, form,
         )
         hip.check(rc, "oa_attention_prefill_split")
         return out
     rc = lib.oa_attention_prefill(
         hip.current_stream_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
         out.data_ptr(), B, Hq, Hk, Sq, Skv, D, scale,
-        q.stride(1), k.stride(1), v.stride(1),
+        q.stride(1), k.stride(1), v.stride(1), int(steady),
     )
     hip.check(rc, "oa_attention_prefill")
     return out

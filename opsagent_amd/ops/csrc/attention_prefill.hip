@@ -1,32 +1,42 @@
-// Flash-style causal prefill attention for MI355X (gfx950) — SURVEY.md §2b
-// "Prefill attention kernel (HIP, bf16 MFMA, LDS-staged KV tiles, gfx950
-// tiling)".
+// Flash-style causal prefill attention for MI355X (gfx950): bf16 matrix instructions, K and V
+// staged through LDS, softmax in registers.
 //
-// v2 structure:
-//   * workgroup = 512 threads = 8 waves; wave owns RB x 16 q-rows
-//     (RB=2 -> 256-row q-tile; RB=1 -> 128-row tile used when the grid
-//     would underfill the 256 CUs at small Sq)
-//   * K AND V staged by global_load_lds (16-B pieces, 4 glds per wave per
-//     64-key tile) into a 2-deep LDS ring: tile t+1's DMA is in flight
-//     under tile t's compute; __syncthreads() doubles as the vmcnt(0)
-//     drain (hipcc emits it while a glds is outstanding), which is the
-//     guide's verified 2-buffer glds pattern (+40% class vs serial)
+//   * K AND V staged by transfers into LDS (16-B pieces) in a 2-deep ring: tile t+1's
+//     transfers are in flight under tile t's compute
 //   * K image: 256-B key rows, XOR swizzle byte^=(key&15)<<4 applied on
-//     the glds SOURCE address (guide rule 21: the LDS write is
+//     the transfer's SOURCE address (the LDS write is
 //     lane-linear, so the swizzle moves to the per-lane global address)
-//     and on the ds_read_b128 B-fragment reads
-//   * V image: [2 key-half][8 d-block] subtiles of [32 key][16 d] bf16
+//     and on the ds_read_b128 A-fragment reads
+//   * V image: [KB/32 key blocks][8 d-block] subtiles of [32 key][16 d] bf16
 //     with key bits permuted (img_row = (k&3) + ((k>>3)<<2) + ((k&4)<<2))
-//     so each ds_read_b64_tr_b16 serves the P·V B-fragment conflict-free:
-//     the hardware transpose read replaces v1's 8 scalar ds_write_b16
-//     per staged piece (the transpose moves from the write side to a
-//     2-cycle read) — guide T10
-//   * online softmax per q-row in registers; 16-lane __shfl_xor reductions
-//   * P round-trips through a per-wave LDS tile (swizzled) to re-shape
-//     C-fragment -> next A-fragment (v3 below REPLACES this with the
-//     swapped-QK^T 32x32 in-register form; v2 stays for small grids)
+//     so each ds_read_b64_tr_b16 serves the P·V fragment conflict-free
+//   * a wave owns 32 q-rows; lane's l&31 IS its q-row, so softmax stats are
+//     per-lane scalars and each row reduction is ONE exchange with lane^32
+//   * S^T = mfma(A=K, B=Q): C[row=key][col=q-row] puts half of a tile's scores of a
+//     lane's row (partner lane l^32 holds the other half) in 32x32 accumulators,
+//     masked and softmaxed in registers
+//   * P -> P·V operand WITHOUT an LDS round-trip: score quads packed to
+//     bf16 pairs, one half exchanged with the partner lane, and
+//     O^T = mfma(A=V^T, B=P^T) keeps the lane<->q-row mapping (alpha rescale
+//     stays a per-lane scalar multiply)
+//   * per-tile wave-uniform branches skip masking on fully-unmasked tiles
+//     and skip compute entirely on tiles past the wave's causal diagonal
 //
-// Out-of-range keys are CLAMPED to Skv-1 on the glds source and their
+// What bounds it: with two waves a SIMD the matrix instructions (4096 cycles for 256 rows x
+// 128 keys, 1.7 us) and about as many cycles of vector instructions hardly overlap, and a
+// tile takes 4.2 us. So the time of a launch is the longest chain of tiles on one CU, and
+// the split of the work is about chains:
+//   * Key groups (KG): 8 waves as one group of 256 rows, two of 128 or four of 64, each group
+//     on its own tiles of the keys, summed up in LDS at the end. 128 keys take 4.2, 2.6 and
+//     2.0 us: the chip's rate falls, but so do a short prompt's chains, with the same blocks.
+//   * Longest chains first (causal prompts have blocks of one to many tiles): late blocks fill
+//     up the CUs that are done, and the heads of a key head are a multiple of 8 blocks apart
+//     (8 key heads), that is on one XCD, whose L2 then holds their keys.
+// us, 32 heads on 8, before both / now: 800 queries of 1024 keys 41.7 / 27.2, 700 of 700
+// 27.4 / 19.2, 1434 of 1434 53 / 34.4, 2048 of 2048 74 / 53.6, 4096 of 4096 250 / 153, 2048 of
+// 6144 201 / 199; 16 on 4, 512 of 512 19.1 / 13.2; split, 77 of 1187 26 / 17.
+//
+// Out-of-range keys are CLAMPED to Skv-1 on the transfer source and their
 // scores masked to -inf (P=0 nullifies the garbage V contribution), so
 // partial tail tiles need no separate path.
 //
@@ -38,15 +48,12 @@
 #include "common.h"
 
 #define DHEAD 128
-#define KVBLK 64
 #define NWAVE 8
 
 typedef __attribute__((ext_vector_type(8))) short bf16x8_t;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4v;
-
-#define K_BYTES (KVBLK * DHEAD * 2)   // 16 KiB per buffer
-#define V_BYTES (KVBLK * DHEAD * 2)   // 16 KiB per buffer
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
 __device__ __forceinline__ uint32_t k_swz_read(int key, int byte_in_row) {
     return (uint32_t)(key * (DHEAD * 2) + (byte_in_row ^ ((key & 15) << 4)));
@@ -58,432 +65,51 @@ __device__ __forceinline__ int v_img_row_inv(int r) {
     return (r & 3) + (((r >> 4) & 1) << 2) + (((r >> 2) & 3) << 3);
 }
 
-// VRM: stage V ROW-MAJOR (like K — 4 contiguous 256-B rows per DMA chunk,
-// ~8 cachelines per glds) instead of the [32 key][16 d] subtile image whose
-// gather touches 32 rows x 32 B per chunk (25% line utilization — measured
-// DMA-bound at ~11 GB/s/CU). The tr16 reads then address (row, d-quad)
-// pieces of the row-major image directly; the same (key&15)<<4 XOR that
-// decollides the K reads spreads the tr read's bank pattern.
-// SPLIT: blockIdx.z takes a run of the q-tile's key tiles and leaves its unnormalised
-// float32 sums with their maximum (scaled scores) and weight sum for
-// prefill_combine_kernel: few queries over many keys fill the chip this way.
-template <int RB, bool PIPE, bool VRM = false, int KB = KVBLK, bool SPLIT = false>
-__global__ __launch_bounds__(512, 1) void attn_prefill_v2(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
-    const uint16_t* __restrict__ v, uint16_t* __restrict__ out, int B, int Hq,
-    int Hk, int Sq, int Skv, float scale, int qs, int ks, int vs,
-    float* __restrict__ po, float* __restrict__ pml) {
-    constexpr int QROWS = 16 * RB;
-    constexpr int QTILE = QROWS * NWAVE;
-    constexpr int P_BYTES = QROWS * KB * 2;
-    constexpr int KBYTES = KB * DHEAD * 2;   // one K (or V) ring buffer
-    constexpr int PIECES = KB / 32;          // 1-KiB DMA chunks per wave
-    constexpr int NKB = KB / 16;             // 16-key QK column blocks
-    constexpr int NKB2 = KB / 32;            // 32-key PV k-blocks
-    __shared__ __attribute__((aligned(16))) char smem[4 * KBYTES +
-                                                      NWAVE * P_BYTES];
-    const uint32_t voff = 2 * KBYTES;        // V buffers after the K ring
-    const uint32_t poff = voff + 2 * KBYTES;
-
-    const int qtile = blockIdx.x;
-    const int bh = blockIdx.y;
-    const int b = bh / Hq;
-    const int h = bh % Hq;
-    const int hk = h / (Hq / Hk);
-    const int offset = Skv - Sq;  // causal diagonal offset
-
-    const int tid = threadIdx.x;
-    const int lane = tid & (WAVE - 1);
-    const int wid = tid / WAVE;
-    const int fr = lane & 15;  // fragment row/col index (0..15)
-    const int fs = lane >> 4;  // k-slice 0..3
-
-    // ---- Q fragments: aq[rb][dblk] = Q[qrow = rb*16 + fr][d = dblk*32 + fs*8]
-    const int qrow0 = qtile * QTILE + wid * QROWS;
-    uint4 aq[RB][4];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-        const int row = qrow0 + rb * 16 + fr;
-        if (row < Sq) {
-            const uint16_t* qp = q + (size_t)(b * Sq + row) * qs + (size_t)h * DHEAD;
-#pragma unroll
-            for (int dblk = 0; dblk < 4; ++dblk)
-                aq[rb][dblk] = *reinterpret_cast<const uint4*>(qp + dblk * 32 + fs * 8);
-        } else {
-#pragma unroll
-            for (int dblk = 0; dblk < 4; ++dblk) aq[rb][dblk] = make_uint4(0, 0, 0, 0);
-        }
-    }
-
-    float m[RB][4], lsum[RB][4];
-    f32x4_t o_acc[RB][8];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            m[rb][r] = -INFINITY;
-            lsum[rb][r] = 0.0f;
-        }
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int nb = 0; nb < 8; ++nb) o_acc[rb][nb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-
-    const int kv_needed = min(Skv, offset + qtile * QTILE + QTILE);
-    const int all_tiles = CEIL_DIV(max(kv_needed, 0), KB);
-    const int run = SPLIT ? CEIL_DIV(all_tiles, (int)gridDim.z) : all_tiles;
-    const int tile0 = SPLIT ? (int)blockIdx.z * run : 0;
-    const int ntiles = SPLIT ? min(all_tiles, tile0 + run) : all_tiles;
-
-    const char* kbase = reinterpret_cast<const char*>(k) +
-                        ((size_t)b * Skv * ks + (size_t)hk * DHEAD) * 2;
-    const char* vbase = reinterpret_cast<const char*>(v) +
-                        ((size_t)b * Skv * vs + (size_t)hk * DHEAD) * 2;
-
-    const int skv_clamp = Skv - 1;
-
-    // Each wave issues 2 K-glds + 2 V-glds per tile (chunk c = wid*2 + p):
-    //   K chunk covers keys c*4 + (lane>>4), XOR-swizzled source address
-    //   V chunk is subtile c: lane -> image row lane>>1 (permuted keys)
-    //
-    // The DMA is issued by INLINE ASM, not the builtin: hipcc's machine-
-    // level wait inserter cannot disambiguate a runtime LDS-DMA destination
-    // from the compute phase's ds_reads and drains the ring with a vmcnt(0)
-    // before the first ds_read of every tile — which serializes the whole
-    // pipeline (measured in the .s for both builtin forms). Untracked asm
-    // glds leave wait placement to us: one explicit vmcnt(0) right before
-    // each tile barrier, so tile t+1's DMA streams under tile t's MFMAs.
-    // (Untracked VMEM only ever makes the compiler's own counted waits
-    // MORE conservative — vmcnt retires in issue order — never unsafe.)
-    //
-    // EVERY asm operand is a LOOP-PERSISTENT value updated only at the loop
-    // top: the wait inserter marks asm operands as pending defs, so if a
-    // compute-phase instruction reuses one of those registers it inserts a
-    // drain mid-compute (measured: vmcnt(3..0) before the first MFMAs when
-    // the address temps died into ds_read destinations). Persistent
-    // operands pin the registers for the whole loop; the only inserted
-    // waits land right after our own vmcnt(0), where they are free.
-
-    // per-piece invariants
-    int k_byte[PIECES], v_byte[PIECES], kkey0[PIECES], vkey0[PIECES];
-#pragma unroll
-    for (int p = 0; p < PIECES; ++p) {
-        const int c = wid * PIECES + p;
-        const int kkey = c * 4 + (lane >> 4);
-        kkey0[p] = kkey;
-        k_byte[p] = ((lane & 15) * 16) ^ ((kkey & 15) << 4);
-        if (VRM) {
-            vkey0[p] = kkey;
-            v_byte[p] = k_byte[p];
-        } else {
-            const int kb2 = c >> 3, nb = c & 7;
-            vkey0[p] = kb2 * 32 + v_img_row_inv(lane >> 1);
-            v_byte[p] = (nb * 16 + (lane & 1) * 8) * 2;
-        }
-    }
-    // LDS destinations (uniform per wave): [buf][piece] for K and V
-    uint32_t m0k[2][PIECES], m0v[2][PIECES];
-#pragma unroll
-    for (int buf = 0; buf < 2; ++buf)
-#pragma unroll
-        for (int p = 0; p < PIECES; ++p) {
-            const int c = wid * PIECES + p;
-            m0k[buf][p] = __builtin_amdgcn_readfirstlane(
-                (uint32_t)(uintptr_t)smem + buf * KBYTES + c * 1024);
-            m0v[buf][p] = __builtin_amdgcn_readfirstlane(
-                (uint32_t)(uintptr_t)smem + voff + buf * KBYTES + c * 1024);
-        }
-    // persistent asm operands: current tile's source addresses + LDS bases
-    const char* ksrc[PIECES];
-    const char* vsrc[PIECES];
-    uint32_t m0k_cur[PIECES], m0v_cur[PIECES];
-    auto set_tile = [&](int t, int buf) {
-        const int kv0 = t * KB;
-#pragma unroll
-        for (int p = 0; p < PIECES; ++p) {
-            ksrc[p] = kbase + (size_t)min(kv0 + kkey0[p], skv_clamp) * ks * 2 +
-                      k_byte[p];
-            vsrc[p] = vbase + (size_t)min(kv0 + vkey0[p], skv_clamp) * vs * 2 +
-                      v_byte[p];
-            m0k_cur[p] = m0k[buf][p];
-            m0v_cur[p] = m0v[buf][p];
-        }
-    };
-    auto stage = [&]() {
-#pragma unroll
-        for (int p = 0; p < PIECES; ++p) {
-            lds_transfer16(m0k_cur[p], ksrc[p]);
-            lds_transfer16(m0v_cur[p], vsrc[p]);
-        }
-    };
-
-    auto compute = [&](int t, const char* kbuf, const char* vbuf) {
-        const int kv0 = t * KB;
-
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-            // ---- QK^T ----------------------------------------------------
-            f32x4_t s[NKB];
-#pragma unroll
-            for (int kb = 0; kb < NKB; ++kb) {
-                f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int dblk = 0; dblk < 4; ++dblk) {
-                    uint4 bk = *reinterpret_cast<const uint4*>(
-                        kbuf + k_swz_read(kb * 16 + fr, (dblk * 32 + fs * 8) * 2));
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        *reinterpret_cast<bf16x8_t*>(&aq[rb][dblk]),
-                        *reinterpret_cast<bf16x8_t*>(&bk), acc, 0, 0, 0);
-                }
-                s[kb] = acc;
-            }
-
-            // ---- mask + online softmax -----------------------------------
-            const int qpos = offset + qrow0 + rb * 16 + fs * 4;  // + reg
-            float rowmax[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) rowmax[r] = -INFINITY;
-#pragma unroll
-            for (int kb = 0; kb < NKB; ++kb) {
-                const int kg = kv0 + kb * 16 + fr;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float sv = s[kb][r] * scale;
-                    if (kg > qpos + r || kg >= Skv) sv = -INFINITY;
-                    s[kb][r] = sv;
-                    rowmax[r] = fmaxf(rowmax[r], sv);
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) rowmax[r] = group16_reduce_max(rowmax[r]);
-
-            float alpha[4], psum[4], mref[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float mn = fmaxf(m[rb][r], rowmax[r]);
-                // a split may show a row none of its keys
-                mref[r] = SPLIT && mn == -INFINITY ? 0.0f : mn;
-                alpha[r] = __expf(m[rb][r] - mref[r]);
-                m[rb][r] = mn;
-                psum[r] = 0.0f;
-            }
-            // fully-masked padding rows produce NaN locally, never stored.
-
-#pragma unroll
-            for (int kb = 0; kb < NKB; ++kb) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float p = __expf(s[kb][r] - mref[r]);
-                    s[kb][r] = p;
-                    psum[r] += p;
-                    *reinterpret_cast<uint16_t*>(
-                        smem + poff + wid * P_BYTES +
-                        (rb * 16 + fs * 4 + r) * (KB * 2) +
-                        (((kb * 16 + fr) * 2) ^ (((rb * 16 + fs * 4 + r) & 7) << 4))) =
-                        f32_to_bf16(p);
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                psum[r] = group16_reduce_sum(psum[r]);
-                lsum[rb][r] = lsum[rb][r] * alpha[r] + psum[r];
-            }
-#pragma unroll
-            for (int nb = 0; nb < 8; ++nb)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) o_acc[rb][nb][r] *= alpha[r];
-
-            // ---- P·V (V via hardware transpose reads) --------------------
-            uint4 ap[NKB2];
-#pragma unroll
-            for (int kb2 = 0; kb2 < NKB2; ++kb2) {
-                const int prow = rb * 16 + fr;
-                ap[kb2] = *reinterpret_cast<const uint4*>(
-                    smem + poff + wid * P_BYTES + prow * (KB * 2) +
-                    (((kb2 * 32 + fs * 8) * 2) ^ ((prow & 7) << 4)));
-            }
-            // VRM per-lane supplier addressing: lane i (in its 16-lane
-            // group) supplies piece (row i>>2, d-quad i&3) of the [4 key]
-            // x[16 d] block; the hardware transpose hands lane i column i.
-            const int vq8 = (fr & 3) * 8;
-            const int vrow0 = fs * 8 + (fr >> 2);       // read0 key-in-32
-            const int vrow1 = vrow0 + 4;                // read1
-#pragma unroll
-            for (int nb = 0; nb < 8; ++nb) {
-#pragma unroll
-                for (int kb2 = 0; kb2 < NKB2; ++kb2) {
-                    bf16x4v r0, r1;
-                    if (VRM) {
-                        const char* vb2 = vbuf + kb2 * 8192;
-                        const int t0 = ((nb * 32) | vq8) ^ ((vrow0 & 15) << 4);
-                        const int t1 = ((nb * 32) | vq8) ^ ((vrow1 & 15) << 4);
-                        r0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-                            (__attribute__((address_space(3))) bf16x4v*)(
-                                vb2 + vrow0 * 256 + t0));
-                        r1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-                            (__attribute__((address_space(3))) bf16x4v*)(
-                                vb2 + vrow1 * 256 + t1));
-                    } else {
-                        const char* sub = vbuf + (kb2 * 8 + nb) * 1024;
-                        r0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-                            (__attribute__((address_space(3))) bf16x4v*)(sub + lane * 8));
-                        r1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-                            (__attribute__((address_space(3))) bf16x4v*)(sub + 512 + lane * 8));
-                    }
-                    union {
-                        struct { bf16x4v lo, hi; } p;
-                        bf16x8_t v8;
-                    } bv;
-                    bv.p.lo = r0;
-                    bv.p.hi = r1;
-                    o_acc[rb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        *reinterpret_cast<bf16x8_t*>(&ap[kb2]), bv.v8,
-                        o_acc[rb][nb], 0, 0, 0);
-                }
-            }
-        }
-    };
-
-    // 2-deep ring, hand-unrolled so every buffer index is a literal: tile
-    // t+1's glds stream under tile t's MFMAs; __syncthreads() both drains
-    // this wave's own glds (hipcc emits the vmcnt(0) there) and fences the
-    // buffer swap across waves.
-    // Drain + keep the staging addresses LIVE across compute: without the
-    // dummy operands the address registers die at the glds asm, the
-    // allocator reuses them for ds_read destinations, and the wait inserter
-    // (which models asm operands as pending) re-serializes the pipeline
-    // with vmcnt(3..0) in front of the first MFMAs (measured).
-    auto drain = [&]() {
-        if constexpr (PIECES == 2) {
-            asm volatile("s_waitcnt vmcnt(0)"
-                         :
-                         : "v"(ksrc[0]), "v"(ksrc[1]), "v"(vsrc[0]),
-                           "v"(vsrc[1]), "s"(m0k_cur[0]), "s"(m0k_cur[1]),
-                           "s"(m0v_cur[0]), "s"(m0v_cur[1])
-                         : "memory");
-        } else {
-            static_assert(PIECES == 4, "drain operand list covers 2/4 pieces");
-            asm volatile("s_waitcnt vmcnt(0)"
-                         :
-                         : "v"(ksrc[0]), "v"(ksrc[1]), "v"(ksrc[2]),
-                           "v"(ksrc[3]), "v"(vsrc[0]), "v"(vsrc[1]),
-                           "v"(vsrc[2]), "v"(vsrc[3]), "s"(m0k_cur[0]),
-                           "s"(m0k_cur[1]), "s"(m0k_cur[2]), "s"(m0k_cur[3]),
-                           "s"(m0v_cur[0]), "s"(m0v_cur[1]), "s"(m0v_cur[2]),
-                           "s"(m0v_cur[3])
-                         : "memory");
-        }
-    };
-    if (ntiles > tile0) {
-        set_tile(tile0, 0);
-        stage();
-    }
-    // static priority for the second-dispatched half (guide T5 static
-    // form): the younger 4 waves lose VALU arbitration on every segment;
-    // one setprio before the loop removes their start-of-segment penalty.
-    // The readfirstlane guard keeps the condition provably wave-uniform
-    // (a divergent guard lowers to exec-masking, which s_setprio ignores).
-    if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256)
-        __builtin_amdgcn_s_setprio(1);
-    drain();
-    __syncthreads();
-    for (int t = tile0; t < ntiles; ++t) {
-        const int cur = (t - tile0) & 1;
-        if (t + 1 < ntiles) set_tile(t + 1, cur ^ 1);
-        if (PIPE && t + 1 < ntiles) stage();
-        compute(t, smem + cur * KBYTES, smem + voff + cur * KBYTES);
-        if (!PIPE && t + 1 < ntiles) stage();  // A/B reference: issue late
-        drain();          // tile t+1's DMA landed
-        __syncthreads();  // all waves' reads of buf[cur] complete
-    }
-
-    // ---- epilogue: out[row][d] = o / l ------------------------------------
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = qrow0 + rb * 16 + fs * 4 + r;
-            if (row >= Sq) continue;
-            if (SPLIT) {
-                const size_t at = ((size_t)blockIdx.z * B * Sq + (size_t)b * Sq + row) * Hq + h;
-#pragma unroll
-                for (int nb = 0; nb < 8; ++nb) po[at * DHEAD + nb * 16 + fr] = o_acc[rb][nb][r];
-                if (fr == 0) *reinterpret_cast<float2*>(pml + at * 2) = make_float2(m[rb][r], lsum[rb][r]);
-                continue;
-            }
-            const float inv_l = (lsum[rb][r] > 0.0f) ? 1.0f / lsum[rb][r] : 0.0f;
-            uint16_t* op = out + ((size_t)(b * Sq + row) * Hq + h) * DHEAD;
-#pragma unroll
-            for (int nb = 0; nb < 8; ++nb)
-                op[nb * 16 + fr] = f32_to_bf16(o_acc[rb][nb][r] * inv_l);
-        }
-}
-
-// ---------------------------------------------------------------------------
-// v3: swapped-QK^T structure on 32x32x16 MFMAs with IN-REGISTER P (guide T12)
-//
-//   * wave owns 32 q-rows; lane's l&31 IS its q-row, so softmax stats are
-//     per-lane scalars and each row reduction is ONE __shfl_xor(.,32)
-//     (v2: 4-step group16 reductions per row-quad)
-//   * S^T = mfma(A=K, B=Q): C[row=key][col=q-row] puts all 64 of a lane's
-//     key-scores (of its row; partner lane l^32 holds the other 64) in the
-//     four 32x32 accumulators — masked/softmaxed in registers
-//   * P -> PV A-operand WITHOUT the LDS round-trip: pack score quads to
-//     bf16 pairs, exchange the partner half with __shfl_xor(.,32), and feed
-//     the assembled 8-key fragments straight into mfma(A=V^T, B=P^T) so
-//     O[row=dim][col=q-row] keeps the lane<->q-row mapping (alpha rescale
-//     stays a per-lane scalar multiply)
-//   * K/V LDS images, glds staging ring, drain discipline: identical to v2
-//     (KB=128); the per-wave P tile is GONE (128 KiB LDS total)
-//   * per-tile wave-uniform branches skip masking on fully-unmasked tiles
-//     and skip compute entirely on tiles past the wave's causal diagonal
-// ---------------------------------------------------------------------------
-typedef __attribute__((ext_vector_type(16))) float f32x16_t;
-
 // Partner-half (lane ^ 32) value on the VALU: v_permlane32_swap with equal
 // inputs yields r[0] = [lo|lo], r[1] = [hi|hi], so the partner's value is
 // r[1] for the low half and r[0] for the high half. The two-asm-operand
 // form is NOT equivalent (measured on-box: the upper half saw its own
 // value) — the builtin models both register updates correctly.
-__device__ __forceinline__ uint32_t xor32_u32(uint32_t v, int lh) {
-    auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    return lh ? r[0] : r[1];
-}
 __device__ __forceinline__ float xor32_f32(float v, int lh) {
-    return __uint_as_float(xor32_u32(__float_as_uint(v), lh));
+    auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(lh ? r[0] : r[1]);
 }
 
-// GQ > 1 (v4): the workgroup carries GQ q-heads that SHARE one KV head
-// (requires Hq/Hk == GQ) — waves split into GQ groups of NWAVE/GQ, each
-// group owning QTILE/GQ q-rows of its head. Every staged K/V tile feeds
-// all GQ heads, cutting the kernel's total KV DMA by GQ: the v3 PMC put
-// the residual WAIT at the staged-KV demand of the co-resident
-// workgroups (~9.6 TB/s against L2+HBM), which this divides by 4.
+// GQ > 1: the workgroup carries GQ q-heads that SHARE one KV head
+// (requires Hq/Hk == GQ): waves split into GQ sets, each owning QTILE/GQ q-rows of its head,
+// and every staged K/V tile feeds all of them (2 to 4 per cent over a block per head).
 // SPLIT: blockIdx.z takes a run of the q-tile's key tiles and leaves its unnormalised
 // float32 sums with their maximum (raw scores) and weight sum for
 // prefill_combine_kernel: few queries over many keys fill the chip this way.
-template <int KB = 128, int GQ = 1, bool SPLIT = false>
-__global__ __launch_bounds__(512, 1) void attn_prefill_v3(
+template <int KG, int GQ, bool SPLIT>
+__global__ __launch_bounds__(512, 1) void attn_prefill_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, uint16_t* __restrict__ out, int B, int Hq,
     int Hk, int Sq, int Skv, float scale, int qs, int ks, int vs,
     float* __restrict__ po, float* __restrict__ pml) {
+    constexpr int KB = 128 / KG;             // keys of a group's tile: 128 of LDS' 160 KiB
     constexpr int QROWS = 32;                // per wave
-    constexpr int QTILE = QROWS * NWAVE;     // 256 across the WG
+    constexpr int NG = NWAVE / KG;           // waves of a key group
+    constexpr int QTILE = QROWS * NG;        // 256 / KG across the WG
     constexpr int QTILE_H = QTILE / GQ;      // rows per head per WG
-    constexpr int KBYTES = KB * DHEAD * 2;
-    constexpr int PIECES = KB / 32;          // 1-KiB DMA chunks per wave
+    constexpr int KBYTES = KB * DHEAD * 2;   // one K (or V) ring buffer
+    constexpr int PIECES = KB / (4 * NG);    // 1-KiB DMA chunks per wave
     constexpr int NKB32 = KB / 32;           // 32-key score blocks
-    __shared__ __attribute__((aligned(16))) char smem[4 * KBYTES];
-    const uint32_t voff = 2 * KBYTES;
+    __shared__ __attribute__((aligned(16))) char lds[4 * KBYTES * KG];
+    const uint32_t voff = 2 * KBYTES;        // V buffers after the K ring
 
-    const int qtile = blockIdx.x;
-    const int bh = blockIdx.y;               // spans B * (Hq/GQ)
+    // longest chains first; the heads of a key head B * Hk blocks apart
+    const int groups = Hq / Hk / GQ, pairs = B * Hk, nbh = pairs * groups;
+    const int turn = blockIdx.x / nbh, place = blockIdx.x % nbh;
+    const int qtile = CEIL_DIV(Sq, QTILE_H) - 1 - turn;
+    const int bh = place % pairs * groups + place / pairs;   // spans B * (Hq/GQ)
     const int tid = threadIdx.x;
     const int lane = tid & (WAVE - 1);
-    const int wid = tid / WAVE;
+    const int gid = KG > 1 ? __builtin_amdgcn_readfirstlane(tid / (WAVE * NG)) : 0;
+    const int wid = tid / WAVE - gid * NG;   // within the key group
+    char* const smem = lds + gid * 4 * KBYTES;
     const int b = bh / (Hq / GQ);
-    const int h = (bh % (Hq / GQ)) * GQ + wid / (NWAVE / GQ);
+    const int h = (bh % (Hq / GQ)) * GQ + wid / (NG / GQ);
     const int hk = h / (Hq / Hk);
     const int offset = Skv - Sq;
 
@@ -491,7 +117,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
     const int lh = lane >> 5;   // fragment k-half (and score key-quad offset)
 
     // ---- Q: B-fragment per d-step s: bq[s] = Q[row l31][d = s*16 + lh*8 ..+7]
-    const int qrow0 = qtile * QTILE_H + (wid % (NWAVE / GQ)) * QROWS;
+    const int qrow0 = qtile * QTILE_H + (wid % (NG / GQ)) * QROWS;
     const int qrow = qrow0 + l31;
     uint4 bq[8];
     if (qrow < Sq) {
@@ -521,10 +147,22 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
                         ((size_t)b * Skv * vs + (size_t)hk * DHEAD) * 2;
     const int skv_clamp = Skv - 1;
 
-    // glds staging: identical images and discipline to v2 (see the comment
-    // blocks above attn_prefill_v2) — K row-major XOR-swizzled, V subtile
-    // image for the tr16 B-fragments, inline-asm DMA with loop-persistent
-    // operands and an explicit vmcnt(0) drain.
+    // The transfers are issued by INLINE ASM, not the builtin: hipcc's machine-
+    // level wait inserter cannot disambiguate a runtime LDS destination
+    // from the compute phase's ds_reads and drains the ring with a vmcnt(0)
+    // before the first ds_read of every tile, which serializes the whole
+    // pipeline (measured in the assembly for both builtin forms). Untracked asm
+    // transfers leave wait placement to us: one explicit vmcnt(0) right before
+    // each tile barrier, so tile t+1's transfers stream under tile t's MFMAs.
+    // (Untracked VMEM only ever makes the compiler's own counted waits
+    // MORE conservative, as vmcnt retires in issue order, never unsafe.)
+    //
+    // EVERY asm operand is a LOOP-PERSISTENT value updated only at the loop
+    // top: the wait inserter marks asm operands as pending defs, so if a
+    // compute-phase instruction reuses one of those registers it inserts a
+    // drain mid-compute. Persistent
+    // operands pin the registers for the whole loop; the only inserted
+    // waits land right after our own vmcnt(0), where they are free.
     int k_byte[PIECES], v_byte[PIECES], kkey0[PIECES], vkey0[PIECES];
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
@@ -570,7 +208,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
         }
     };
     auto drain = [&]() {
-        static_assert(PIECES == 4, "drain operand list covers KB=128");
+        static_assert(PIECES == 4, "drain operand list");
         asm volatile("s_waitcnt vmcnt(0)"
                      :
                      : "v"(ksrc[0]), "v"(ksrc[1]), "v"(ksrc[2]), "v"(ksrc[3]),
@@ -589,10 +227,9 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
                        bool need_mask) {
         const int kv0 = t * KB;
 
-        // ---- S^T = K·Q^T: four 32x32 blocks of 32 keys ---------------------
+        // ---- S^T = K·Q^T: 32x32 blocks of 32 keys ---------------------
         f32x16_t sa[NKB32];
-#pragma unroll
-        for (int kb = 0; kb < NKB32; ++kb) sa[kb] = (f32x16_t)(0.0f);
+        const f32x16_t zero = (f32x16_t)(0.0f);
 #pragma unroll
         for (int s = 0; s < 8; ++s)
 #pragma unroll
@@ -601,7 +238,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
                     kbuf + k_swz_read(kb * 32 + l31, s * 32 + lh * 16));
                 sa[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                     *reinterpret_cast<bf16x8_t*>(&ak),
-                    *reinterpret_cast<bf16x8_t*>(&bq[s]), sa[kb], 0, 0, 0);
+                    *reinterpret_cast<bf16x8_t*>(&bq[s]), s ? sa[kb] : zero, 0, 0, 0);
             }
 
         // ---- mask + online softmax (per-lane row, RAW-score domain) --------
@@ -637,7 +274,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
         const float mn = fmaxf(m_old, rowmax);
         m = mn;
         // a split may show a row none of its keys
-        const float mnb = SPLIT && mn == -INFINITY ? 0.0f : mn * scale2;
+        const float mnb = (SPLIT || KG > 1) && mn == -INFINITY ? 0.0f : mn * scale2;
         float psum = 0.0f;
 
         // ---- exp + pack to bf16 quads: pk[kb][g] = keys kb*32+g*8+4*lh+{0..3}
@@ -665,7 +302,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
         // the first few tiles most tiles leave every row max unchanged and
         // the 64 accumulator multiplies + lsum scale are skipped outright
         if (__any(rowmax > m_old)) {
-            const float alpha = SPLIT && mn == -INFINITY
+            const float alpha = (SPLIT || KG > 1) && mn == -INFINITY
                                     ? 1.0f : __builtin_amdgcn_exp2f((m_old - mn) * scale2);
             lsum *= alpha;
 #pragma unroll
@@ -676,26 +313,22 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
         lsum += psum;
 
         // ---- P·V: O^T[dim][q-row] via mfma(A=V^T, B=P^T) -------------------
-        // k-step ks2 covers keys ks2*16 + lh*8 + {0..7}: own quad = pk[kb][e*2
-        // + lh], partner quad arrives by shfl_xor(32) of pk[kb][e*2 + (lh^1)]
-        // (each lane sends what its partner needs and receives what it needs).
+        // k-step ks2 covers keys ks2*16 + lh*8 + {0..7}: the lower half's lanes have their own
+        // quad e2 and the partner's, the upper half's the partner's quad e2 + 1 and their own,
+        // which is what one swap of the quads' halves leaves in its two registers.
 #pragma unroll
         for (int ks2 = 0; ks2 < KB / 16; ++ks2) {
             const int kb = ks2 >> 1, e2 = (ks2 & 1) * 2;
-            const uint32_t own0 = lh ? pk[kb][e2 + 1][0] : pk[kb][e2][0];
-            const uint32_t own1 = lh ? pk[kb][e2 + 1][1] : pk[kb][e2][1];
-            const uint32_t snd0 = lh ? pk[kb][e2][0] : pk[kb][e2 + 1][0];
-            const uint32_t snd1 = lh ? pk[kb][e2][1] : pk[kb][e2 + 1][1];
-            const uint32_t rcv0 = xor32_u32(snd0, lh);
-            const uint32_t rcv1 = xor32_u32(snd1, lh);
+            const auto w0 = __builtin_amdgcn_permlane32_swap(pk[kb][e2][0], pk[kb][e2 + 1][0], false, false);
+            const auto w1 = __builtin_amdgcn_permlane32_swap(pk[kb][e2][1], pk[kb][e2 + 1][1], false, false);
             union {
                 uint32_t u[4];
                 bf16x8_t v8;
             } pf;
-            pf.u[0] = lh ? rcv0 : own0;
-            pf.u[1] = lh ? rcv1 : own1;
-            pf.u[2] = lh ? own0 : rcv0;
-            pf.u[3] = lh ? own1 : rcv1;
+            pf.u[0] = w0[0];
+            pf.u[1] = w1[0];
+            pf.u[2] = w0[1];
+            pf.u[3] = w1[1];
 
             // V^T A-fragment: subtile tr16 reads — group-uniform 128-B runs
             // (fs_eff = (ks2&1)*2 + lh selects the key octet, col = l31&15)
@@ -722,20 +355,25 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
         }
     };
 
-    if (ntiles > tile0) {
-        set_tile(tile0, 0);
+    const int first = tile0 + gid;
+    if (first < ntiles) {
+        set_tile(first, 0);
         stage();
     }
+    // static priority for the second half of the waves: the younger 4 lose VALU
+    // arbitration on every segment otherwise. The readfirstlane keeps the condition
+    // provably wave-uniform (exec-masking is ignored by s_setprio).
     if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256)
         __builtin_amdgcn_s_setprio(1);
     drain();
     __syncthreads();
-    for (int t = tile0; t < ntiles; ++t) {
-        const int cur = (t - tile0) & 1;
+    // every group takes as many steps as the first, which may have one tile more
+    int cur = 0;
+    for (int t = first; t - gid < ntiles; t += KG, cur ^= 1) {
         const int kv0 = t * KB;
-        if (t + 1 < ntiles) set_tile(t + 1, cur ^ 1);
-        if (t + 1 < ntiles) stage();
-        if (kv0 < wave_kv_last) {  // wave-uniform: skip past-diagonal tiles
+        if (t + KG < ntiles) set_tile(t + KG, cur ^ 1);
+        if (t + KG < ntiles) stage();
+        if (t < ntiles && kv0 < wave_kv_last) {  // wave-uniform: skip past-diagonal tiles
             // fully-unmasked tile: every key <= every lane's diagonal
             const bool need_mask =
                 !(kv0 + KB <= offset + qrow0 + 1 && kv0 + KB <= Skv);
@@ -746,16 +384,69 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
         __syncthreads();
     }
 
+    // ---- key groups added up: each keeps 128 / KG channels and takes the other groups' sums
+    // of them, behind the loop's last barrier. A wave's area is [64][lane]: its sums by
+    // channel, and where its own would be its maximum and weight sum
+    constexpr int NDB = 4 / KG;
+    if constexpr (KG > 1) {
+        float* const area = reinterpret_cast<float*>(lds) + wid * WAVE * 64 + lane;
+        float* const mine = area + gid * NG * WAVE * 64;
+        mine[gid * NDB * 16 * WAVE] = m;
+        mine[(gid * NDB * 16 + 1) * WAVE] = lsum;
+#pragma unroll
+        for (int db = 0; db < 4; ++db) {
+            if (db / NDB == gid) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) oa[db % NDB][i] = oa[db][i];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) mine[(db * 16 + i) * WAVE] = oa[db][i];
+            }
+        }
+        __syncthreads();
+        const float scale2 = scale * 1.4426950408889634f;
+        float mo[KG - 1], lo[KG - 1], both = m;
+#pragma unroll
+        for (int o = 0; o < KG - 1; ++o) {
+            const int g = o + (o >= gid);
+            mo[o] = area[(g * NG * 64 + g * NDB * 16) * WAVE];
+            lo[o] = area[(g * NG * 64 + g * NDB * 16 + 1) * WAVE];
+            both = fmaxf(both, mo[o]);
+        }
+        // a split that shows a row no key leaves zeros; elsewhere the softmax of nothing is NaN
+        const bool none = both == -INFINITY && (SPLIT || ntiles <= tile0);
+        const float a = none ? 1.0f : __builtin_amdgcn_exp2f((m - both) * scale2);
+        m = both;
+        lsum *= a;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) oa[db][i] *= a;
+#pragma unroll
+        for (int o = 0; o < KG - 1; ++o) {
+            const int g = o + (o >= gid);
+            const float c = none ? 1.0f : __builtin_amdgcn_exp2f((mo[o] - both) * scale2);
+            lsum += lo[o] * c;
+#pragma unroll
+            for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    oa[db][i] = __builtin_fmaf(
+                        area[(g * NG * 64 + (gid * NDB + db) * 16 + i) * WAVE], c, oa[db][i]);
+        }
+    }
+    const int dim0 = KG > 1 ? gid * 32 * NDB : 0;  // of the channels left in oa[0 .. NDB)
+
     if (SPLIT) {
         if (qrow < Sq) {
             const size_t row = ((size_t)blockIdx.z * B * Sq + (size_t)b * Sq + qrow) * Hq + h;
 #pragma unroll
-            for (int db = 0; db < 4; ++db)
+            for (int db = 0; db < NDB; ++db)
 #pragma unroll
                 for (int g = 0; g < 4; ++g)
-                    *reinterpret_cast<float4*>(po + row * DHEAD + db * 32 + g * 8 + 4 * lh) =
+                    *reinterpret_cast<float4*>(po + row * DHEAD + dim0 + db * 32 + g * 8 + 4 * lh) =
                         make_float4(oa[db][g * 4], oa[db][g * 4 + 1], oa[db][g * 4 + 2], oa[db][g * 4 + 3]);
-            if (lh == 0) *reinterpret_cast<float2*>(pml + row * 2) = make_float2(m, lsum);
+            if (lh == 0 && gid == 0) *reinterpret_cast<float2*>(pml + row * 2) = make_float2(m, lsum);
         }
         return;
     }
@@ -764,10 +455,10 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
         const float inv_l = (lsum > 0.0f) ? 1.0f / lsum : 0.0f;
         uint16_t* op = out + ((size_t)(b * Sq + qrow) * Hq + h) * DHEAD;
 #pragma unroll
-        for (int db = 0; db < 4; ++db)
+        for (int db = 0; db < NDB; ++db)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const int d0 = db * 32 + g * 8 + 4 * lh;
+                const int d0 = dim0 + db * 32 + g * 8 + 4 * lh;
                 uint2 pkd;
                 pkd.x = (uint32_t)f32_to_bf16(oa[db][g * 4 + 0] * inv_l) |
                         ((uint32_t)f32_to_bf16(oa[db][g * 4 + 1] * inv_l) << 16);
@@ -778,8 +469,296 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v3(
     }
 }
 
+// The sums of a row in one order of the keys, 128 queries of a head a block: for callers that
+// quantise what follows. There another rounding of a weight moves activations to the
+// next 8-bit value, and two forms that are each 0.036 from 64 bits end 0.037 apart; so 8-bit
+// models keep the form and the splits that they had, whatever is the fastest. Waves of
+// 16 rows on 16x16x32 products; P goes through LDS to become an operand. A tile takes 5 us,
+// its LDS reads (512 KB for 128 rows) the most of it.
+template <bool SPLIT>
+__global__ __launch_bounds__(512, 1) void attn_prefill_steady_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+    const uint16_t* __restrict__ v, uint16_t* __restrict__ out, int B, int Hq,
+    int Hk, int Sq, int Skv, float scale, int qs, int ks, int vs,
+    float* __restrict__ po, float* __restrict__ pml) {
+    constexpr int KB = 128, QROWS = 16;
+    constexpr int QTILE = QROWS * NWAVE;
+    constexpr int P_BYTES = QROWS * KB * 2;
+    constexpr int KBYTES = KB * DHEAD * 2;   // one K (or V) ring buffer
+    constexpr int PIECES = KB / 32;          // 1-KiB DMA chunks per wave
+    constexpr int NKB = KB / 16;             // 16-key QK column blocks
+    constexpr int NKB2 = KB / 32;            // 32-key PV k-blocks
+    __shared__ __attribute__((aligned(16))) char smem[4 * KBYTES +
+                                                      NWAVE * P_BYTES];
+    const uint32_t voff = 2 * KBYTES;        // V buffers after the K ring
+    const uint32_t poff = voff + 2 * KBYTES;
+
+    const int groups = Hq / Hk, pairs = B * Hk, nbh = pairs * groups;
+    const int turn = blockIdx.x / nbh, place = blockIdx.x % nbh;
+    const int qtile = CEIL_DIV(Sq, QTILE) - 1 - turn;        // as in attn_prefill_kernel
+    const int bh = place % pairs * groups + place / pairs;
+    const int b = bh / Hq;
+    const int h = bh % Hq;
+    const int hk = h / (Hq / Hk);
+    const int offset = Skv - Sq;  // causal diagonal offset
+
+    const int tid = threadIdx.x;
+    const int lane = tid & (WAVE - 1);
+    const int wid = tid / WAVE;
+    const int fr = lane & 15;  // fragment row/col index (0..15)
+    const int fs = lane >> 4;  // k-slice 0..3
+
+    // ---- Q fragments: aq[dblk] = Q[qrow0 + fr][d = dblk*32 + fs*8]
+    const int qrow0 = qtile * QTILE + wid * QROWS;
+    uint4 aq[4];
+    if (qrow0 + fr < Sq) {
+        const uint16_t* qp = q + (size_t)(b * Sq + qrow0 + fr) * qs + (size_t)h * DHEAD;
+#pragma unroll
+        for (int dblk = 0; dblk < 4; ++dblk)
+            aq[dblk] = *reinterpret_cast<const uint4*>(qp + dblk * 32 + fs * 8);
+    } else {
+#pragma unroll
+        for (int dblk = 0; dblk < 4; ++dblk) aq[dblk] = make_uint4(0, 0, 0, 0);
+    }
+
+    float m[4], lsum[4];
+    f32x4_t o_acc[8];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        m[r] = -INFINITY;
+        lsum[r] = 0.0f;
+    }
+#pragma unroll
+    for (int nb = 0; nb < 8; ++nb) o_acc[nb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+
+    const int kv_needed = min(Skv, offset + qtile * QTILE + QTILE);
+    const int all_tiles = CEIL_DIV(max(kv_needed, 0), KB);
+    const int run = SPLIT ? CEIL_DIV(all_tiles, (int)gridDim.z) : all_tiles;
+    const int tile0 = SPLIT ? (int)blockIdx.z * run : 0;
+    const int ntiles = SPLIT ? min(all_tiles, tile0 + run) : all_tiles;
+
+    const char* kbase = reinterpret_cast<const char*>(k) +
+                        ((size_t)b * Skv * ks + (size_t)hk * DHEAD) * 2;
+    const char* vbase = reinterpret_cast<const char*>(v) +
+                        ((size_t)b * Skv * vs + (size_t)hk * DHEAD) * 2;
+
+    const int skv_clamp = Skv - 1;
+
+    // transfers as in attn_prefill_kernel
+    // per-piece invariants
+    int k_byte[PIECES], v_byte[PIECES], kkey0[PIECES], vkey0[PIECES];
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+        const int c = wid * PIECES + p;
+        const int kkey = c * 4 + (lane >> 4);
+        kkey0[p] = kkey;
+        k_byte[p] = ((lane & 15) * 16) ^ ((kkey & 15) << 4);
+        const int kb2 = c >> 3, nb = c & 7;
+        vkey0[p] = kb2 * 32 + v_img_row_inv(lane >> 1);
+        v_byte[p] = (nb * 16 + (lane & 1) * 8) * 2;
+    }
+    // LDS destinations (uniform per wave): [buf][piece] for K and V
+    uint32_t m0k[2][PIECES], m0v[2][PIECES];
+#pragma unroll
+    for (int buf = 0; buf < 2; ++buf)
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {
+            const int c = wid * PIECES + p;
+            m0k[buf][p] = __builtin_amdgcn_readfirstlane(
+                (uint32_t)(uintptr_t)smem + buf * KBYTES + c * 1024);
+            m0v[buf][p] = __builtin_amdgcn_readfirstlane(
+                (uint32_t)(uintptr_t)smem + voff + buf * KBYTES + c * 1024);
+        }
+    // persistent asm operands: current tile's source addresses + LDS bases
+    const char* ksrc[PIECES];
+    const char* vsrc[PIECES];
+    uint32_t m0k_cur[PIECES], m0v_cur[PIECES];
+    auto set_tile = [&](int t, int buf) {
+        const int kv0 = t * KB;
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {
+            ksrc[p] = kbase + (size_t)min(kv0 + kkey0[p], skv_clamp) * ks * 2 +
+                      k_byte[p];
+            vsrc[p] = vbase + (size_t)min(kv0 + vkey0[p], skv_clamp) * vs * 2 +
+                      v_byte[p];
+            m0k_cur[p] = m0k[buf][p];
+            m0v_cur[p] = m0v[buf][p];
+        }
+    };
+    auto stage = [&]() {
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {
+            lds_transfer16(m0k_cur[p], ksrc[p]);
+            lds_transfer16(m0v_cur[p], vsrc[p]);
+        }
+    };
+
+    auto compute = [&](int t, const char* kbuf, const char* vbuf) {
+        const int kv0 = t * KB;
+        const bool need_mask = !(kv0 + KB <= offset + qrow0 + 1 && kv0 + KB <= Skv);
+
+        // ---- QK^T ----------------------------------------------------
+        f32x4_t s[NKB];
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb) {
+            f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int dblk = 0; dblk < 4; ++dblk) {
+                uint4 bk = *reinterpret_cast<const uint4*>(
+                    kbuf + k_swz_read(kb * 16 + fr, (dblk * 32 + fs * 8) * 2));
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    *reinterpret_cast<bf16x8_t*>(&aq[dblk]),
+                    *reinterpret_cast<bf16x8_t*>(&bk), acc, 0, 0, 0);
+            }
+            s[kb] = acc;
+        }
+
+        // ---- mask + online softmax -----------------------------------
+        const int qpos = offset + qrow0 + fs * 4;  // + reg
+        float rowmax[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) rowmax[r] = -INFINITY;
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[kb][r] *= scale;
+        }
+        if (need_mask) {  // wave-uniform
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb) {
+                const int kg = kv0 + kb * 16 + fr;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (kg > qpos + r || kg >= Skv) s[kb][r] = -INFINITY;
+            }
+        }
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) rowmax[r] = fmaxf(rowmax[r], s[kb][r]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) rowmax[r] = group16_reduce_max(rowmax[r]);
+
+        float alpha[4], psum[4], mref[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float mn = fmaxf(m[r], rowmax[r]);
+            // a split may show a row none of its keys
+            mref[r] = SPLIT && mn == -INFINITY ? 0.0f : mn;
+            alpha[r] = __expf(m[r] - mref[r]);
+            m[r] = mn;
+            psum[r] = 0.0f;
+        }
+        // fully-masked padding rows produce NaN locally, never stored.
+
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float p = __expf(s[kb][r] - mref[r]);
+                s[kb][r] = p;
+                psum[r] += p;
+                *reinterpret_cast<uint16_t*>(
+                    smem + poff + wid * P_BYTES +
+                    (fs * 4 + r) * (KB * 2) +
+                    (((kb * 16 + fr) * 2) ^ (((fs * 4 + r) & 7) << 4))) =
+                    f32_to_bf16(p);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            psum[r] = group16_reduce_sum(psum[r]);
+            lsum[r] = lsum[r] * alpha[r] + psum[r];
+        }
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o_acc[nb][r] *= alpha[r];
+
+        // ---- P·V (V via hardware transpose reads) --------------------
+        uint4 ap[NKB2];
+#pragma unroll
+        for (int kb2 = 0; kb2 < NKB2; ++kb2) {
+            const int prow = fr;
+            ap[kb2] = *reinterpret_cast<const uint4*>(
+                smem + poff + wid * P_BYTES + prow * (KB * 2) +
+                (((kb2 * 32 + fs * 8) * 2) ^ ((prow & 7) << 4)));
+        }
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb) {
+#pragma unroll
+            for (int kb2 = 0; kb2 < NKB2; ++kb2) {
+                bf16x4v r0, r1;
+                const char* sub = vbuf + (kb2 * 8 + nb) * 1024;
+                r0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+                    (__attribute__((address_space(3))) bf16x4v*)(sub + lane * 8));
+                r1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+                    (__attribute__((address_space(3))) bf16x4v*)(sub + 512 + lane * 8));
+                union {
+                    struct { bf16x4v lo, hi; } p;
+                    bf16x8_t v8;
+                } bv;
+                bv.p.lo = r0;
+                bv.p.hi = r1;
+                o_acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    *reinterpret_cast<bf16x8_t*>(&ap[kb2]), bv.v8,
+                    o_acc[nb], 0, 0, 0);
+            }
+        }
+    };
+
+    auto drain = [&]() {
+        static_assert(PIECES == 4, "drain operand list");
+        asm volatile("s_waitcnt vmcnt(0)"
+                     :
+                     : "v"(ksrc[0]), "v"(ksrc[1]), "v"(ksrc[2]), "v"(ksrc[3]),
+                       "v"(vsrc[0]), "v"(vsrc[1]), "v"(vsrc[2]), "v"(vsrc[3]),
+                       "s"(m0k_cur[0]), "s"(m0k_cur[1]), "s"(m0k_cur[2]),
+                       "s"(m0k_cur[3]), "s"(m0v_cur[0]), "s"(m0v_cur[1]),
+                       "s"(m0v_cur[2]), "s"(m0v_cur[3])
+                     : "memory");
+    };
+    if (ntiles > tile0) {
+        set_tile(tile0, 0);
+        stage();
+    }
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256)
+        __builtin_amdgcn_s_setprio(1);
+    drain();
+    __syncthreads();
+    for (int t = tile0; t < ntiles; ++t) {
+        const int cur = (t - tile0) & 1;
+        if (t + 1 < ntiles) set_tile(t + 1, cur ^ 1);
+        if (t + 1 < ntiles) stage();
+        compute(t, smem + cur * KBYTES, smem + voff + cur * KBYTES);
+        drain();          // tile t+1 has landed
+        __syncthreads();  // all waves' reads of buf[cur] complete
+    }
+
+    // ---- epilogue: out[row][d] = o / l ------------------------------------
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int row = qrow0 + fs * 4 + r;
+        if (row >= Sq) continue;
+        if (SPLIT) {
+            const size_t at = ((size_t)blockIdx.z * B * Sq + (size_t)b * Sq + row) * Hq + h;
+#pragma unroll
+            for (int nb = 0; nb < 8; ++nb) po[at * DHEAD + nb * 16 + fr] = o_acc[nb][r];
+            if (fr == 0) *reinterpret_cast<float2*>(pml + at * 2) = make_float2(m[r], lsum[r]);
+            continue;
+        }
+        const float inv_l = (lsum[r] > 0.0f) ? 1.0f / lsum[r] : 0.0f;
+        uint16_t* op = out + ((size_t)(b * Sq + row) * Hq + h) * DHEAD;
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb)
+            op[nb * 16 + fr] = f32_to_bf16(o_acc[nb][r] * inv_l);
+    }
+}
+
 // Splits added up: one wave per (query, head) row, two channels per lane. rows = B * Sq
-// * Hq; scale2 turns a difference of maxima into a power of two. A split without a visible
+// * Hq; scale2 turns a difference of maxima (of unscaled scores but in the steady form) into a
+// power of two. A split without a visible
 // key has weight sum 0; one with a NaN or an infinite score has a NaN sum, and counts.
 // The launch is its chain of loads: the first eight splits are asked for together, weights
 // or not (77 queries of 32 heads behind 1187 keys, 8 splits: 7.4 us -> 3.9).
@@ -828,9 +807,17 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const float* __res
     out[(size_t)row * (DHEAD / 2) + lane] = pack_bf16x2(a * inv, b * inv);
 }
 
-// Key-split forms: merged = 0, a block per head and 128 queries (variant 7); 1, a block
-// per key head and 256 / (Hq / Hk) queries (variant 9; Hq / Hk of 2, 4 or 8).
+// Key-split forms: merged = 0, a block per head and 128 queries (64 up to 64 queries); 1, a
+// block per key head and 256 / (Hq / Hk) queries (Hq / Hk of 2, 4 or 8); 2, the steady form.
 // po [nsplit, B, Sq, Hq, 128] and pml [nsplit, B, Sq, Hq, 2]: float32 scratch.
+#define LAUNCH_PREFILL(KG, GQ, SPLIT, NSPLIT)                                                      \
+    LAUNCH_BLOCKS((attn_prefill_kernel<KG, GQ, SPLIT>), 256 / (KG) / (GQ), B * (Hq / (GQ)), NSPLIT)
+#define LAUNCH_BLOCKS(KERN, ROWS, HEADS, NSPLIT)                                                   \
+    hipLaunchKernelGGL((KERN), dim3(CEIL_DIV(Sq, ROWS) * (HEADS), 1, NSPLIT),                      \
+                       dim3(512), 0, (hipStream_t)stream, (const uint16_t*)q, (const uint16_t*)k,  \
+                       (const uint16_t*)v, (uint16_t*)out, B, Hq, Hk, Sq, Skv, scale, q_stride,    \
+                       k_stride, v_stride, (float*)po, (float*)pml)
+
 extern "C" int oa_attention_prefill_split(
     void* stream, const void* q, const void* k, const void* v, void* out, void* po, void* pml,
     int B, int Hq, int Hk, int Sq, int Skv, int D, float scale, int q_stride, int k_stride,
@@ -841,27 +828,21 @@ extern "C" int oa_attention_prefill_split(
     if (nsplit < 1 || nsplit > 65535 || (int64_t)B * Sq * Hq > (1 << 30)) return -105;
     const int gq = Hq / Hk, rows = B * Sq * Hq;
     if (rows < 1) return 0;
-#define LAUNCH_SPLIT(KERN, QT, Y)                                                                  \
-    hipLaunchKernelGGL((KERN), dim3(CEIL_DIV(Sq, QT), Y, nsplit), dim3(512), 0,                    \
-                       (hipStream_t)stream, (const uint16_t*)q, (const uint16_t*)k,                \
-                       (const uint16_t*)v, (uint16_t*)out, B, Hq, Hk, Sq, Skv, scale, q_stride,    \
-                       k_stride, v_stride, (float*)po, (float*)pml)
-    // the maxima of the merged form are unscaled scores
-    float scale2 = 1.4426950408889634f;
-    if (!merged) {
-        LAUNCH_SPLIT((attn_prefill_v2<1, true, false, 128, true>), 128, B * Hq);
-    } else {
-        scale2 *= scale;
-        if (gq == 2) LAUNCH_SPLIT((attn_prefill_v3<128, 2, true>), 128, B * Hk);
-        else if (gq == 4) LAUNCH_SPLIT((attn_prefill_v3<128, 4, true>), 64, B * Hk);
-        else if (gq == 8) LAUNCH_SPLIT((attn_prefill_v3<128, 8, true>), 32, B * Hk);
-        else return -104;
+    if (merged == 2) {
+        LAUNCH_BLOCKS(attn_prefill_steady_kernel<true>, 128, B * Hq, nsplit);
     }
-#undef LAUNCH_SPLIT
+    else if (!merged) {
+        if (Sq <= 64) LAUNCH_PREFILL(4, 1, true, nsplit);
+        else LAUNCH_PREFILL(2, 1, true, nsplit);
+    }
+    else if (gq == 2) LAUNCH_PREFILL(1, 2, true, nsplit);
+    else if (gq == 4) LAUNCH_PREFILL(1, 4, true, nsplit);
+    else if (gq == 8) LAUNCH_PREFILL(1, 8, true, nsplit);
+    else return -104;
     HIP_CHECK_LAUNCH();
     hipLaunchKernelGGL(prefill_combine_kernel, dim3(CEIL_DIV(rows, 4)), dim3(256), 0,
                        (hipStream_t)stream, (const float*)po, (const float*)pml, (uint32_t*)out, rows,
-                       nsplit, scale2);
+                       nsplit, merged == 2 ? 1.4426950408889634f : scale * 1.4426950408889634f);
     HIP_CHECK_LAUNCH();
     return 0;
 }
@@ -873,88 +854,70 @@ extern "C" int oa_attention_prefill_variant(
     if (D != DHEAD) return -100;
     if (Hq % Hk != 0) return -101;
     if ((q_stride | k_stride | v_stride) % 8 != 0) return -102;
-    dim3 block(512);
-    const dim3 grid1(CEIL_DIV(Sq, 128), B * Hq);
-    const dim3 grid2(CEIL_DIV(Sq, 256), B * Hq);
-#define LAUNCH(KERN, GRID)                                                      \
-    hipLaunchKernelGGL(KERN, GRID, block, 0, (hipStream_t)stream,               \
-                       (const uint16_t*)q, (const uint16_t*)k,                  \
-                       (const uint16_t*)v, (uint16_t*)out, B, Hq, Hk, Sq, Skv,  \
-                       scale, q_stride, k_stride, v_stride, (float*)nullptr,    \
-                       (float*)nullptr)
-#define LAUNCH3(GQV, GRID)                                                      \
-    hipLaunchKernelGGL((attn_prefill_v3<128, GQV, false>), GRID, block, 0,      \
-                       (hipStream_t)stream, (const uint16_t*)q,                 \
-                       (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)out,  \
-                       B, Hq, Hk, Sq, Skv, scale, q_stride, k_stride, v_stride, \
-                       (float*)nullptr, (float*)nullptr)
-    // RB=2 (256-row q-tile) instantiations were REMOVED: every form spilled
-    // 25-43 VGPRs past the 256 cap and lost all A/Bs to the RB1 kernels.
-    (void)grid2;
+    float* const po = nullptr;
+    float* const pml = nullptr;
     switch (variant) {
-        case 1:  // RB1 pipelined, 64-key tiles
-            LAUNCH((attn_prefill_v2<1, true>), grid1);
+        case 1: case 3: case 5: case 7:  // the steady form, 128 rows
+            LAUNCH_BLOCKS(attn_prefill_steady_kernel<false>, 128, B * Hq, 1);
             break;
-        case 3:  // RB1 late-issue (A/B reference: DMA after compute)
-            LAUNCH((attn_prefill_v2<1, false>), grid1);
+        case 10:  // two key groups, 128 rows
+            LAUNCH_PREFILL(2, 1, false, 1);
             break;
-        case 5:  // RB1 pipelined, row-major V (coalesced V DMA — measured
-                 // 15% SLOWER than the subtile image; kept for A/B)
-            LAUNCH((attn_prefill_v2<1, true, true>), grid1);
+        case 11:  // four key groups, 64 rows
+            LAUNCH_PREFILL(4, 1, false, 1);
             break;
-        case 7:  // RB1 pipelined, 128-key tiles (160 KiB LDS: half the
-                 // barriers per key, double the MFMAs per phase)
-            LAUNCH((attn_prefill_v2<1, true, false, 128>), grid1);
+        case 8:  // 256 rows of one head
+            LAUNCH_PREFILL(1, 1, false, 1);
             break;
-        case 8:  // v3: swapped-QK^T 32x32 MFMAs, in-register P (256-row tile)
-            LAUNCH3(1, dim3(CEIL_DIV(Sq, 256), B * Hq));
-            break;
-        case 9:  // v4: GQA-merged v3 — GQ q-heads share each staged KV tile
+        case 9:  // 256 rows: the q-heads of a KV head share each staged KV tile
             if (Hq == 2 * Hk)
-                LAUNCH3(2, dim3(CEIL_DIV(Sq, 128), B * (Hq / 2)));
+                LAUNCH_PREFILL(1, 2, false, 1);
             else if (Hq == 4 * Hk)
-                LAUNCH3(4, dim3(CEIL_DIV(Sq, 64), B * (Hq / 4)));
+                LAUNCH_PREFILL(1, 4, false, 1);
             else if (Hq == 8 * Hk)
-                LAUNCH3(8, dim3(CEIL_DIV(Sq, 32), B * (Hq / 8)));
+                LAUNCH_PREFILL(1, 8, false, 1);
             else
                 return -104;
             break;
         default:
             return -103;
     }
-#undef LAUNCH
-#undef LAUNCH3
     HIP_CHECK_LAUNCH();
     return 0;
+}
+
+// Time of KG key groups without key splits in us, over 256 CUs: a chain of 128-key tiles is the
+// longest block's, or, where there are more blocks than CUs, the chip's share of all tiles
+// and half a block for the uneven end. Over 170 sizes (1 to 64 heads, 16 to 4096 queries,
+// up to 9000 keys) the form it names took 0.1 per cent more than the best of the three,
+// 19 at the most (64 blocks of 282 queries: 16.4 for 13.8).
+static float prefill_us(int kg, int B, int Hq, int Sq, int Skv) {
+    const float tile = kg == 1 ? 4.2f : kg == 2 ? 2.6f : 2.0f;
+    const int qt = 256 / kg, nq = CEIL_DIV(Sq, qt);
+    const float last = CEIL_DIV(Skv, 128), blocks = (float)nq * B * Hq;
+    const float first = nq > 1 ? fminf(CEIL_DIV(Skv - Sq + qt, 128), last) : last;
+    const float mean = (first + last) / 2;
+    return tile * (blocks <= 256 ? last : fmaxf(last, mean * (blocks / 256 + 0.5f)));
 }
 
 extern "C" int oa_attention_prefill(void* stream, const void* q, const void* k,
                                     const void* v, void* out, int B, int Hq,
                                     int Hk, int Sq, int Skv, int D, float scale,
-                                    int q_stride, int k_stride, int v_stride) {
-    // OPSAGENT_PREFILL_VARIANT=1..4 forces a variant (read per call so one
+                                    int q_stride, int k_stride, int v_stride, int steady) {
+    // OPSAGENT_PREFILL_VARIANT forces a variant (read per call so one
     // process can A/B all variants).
     const char* e = getenv("OPSAGENT_PREFILL_VARIANT");
     int variant = e ? atoi(e) : 0;
-    // A/B-measured on MI355X (profiles/README.md): the GQA-merged form
-    // (v4) shares each staged KV tile across the q-heads of one KV head
-    // and wins whenever it applies (S8192 721 vs 556 vs 350 TF; S2048 439;
-    // B16/S1024 426): the v3 PMC put the residual WAIT at staged-KV DMA
-    // pressure, which merging divides by GQ. v3 covers non-4/8 GQA
-    // ratios; while its blocks fit one round the 128-row v2 keeps more CUs busy.
-    if (variant <= 0) {
-        const int gq = (Hk > 0 && Hq % Hk == 0) ? Hq / Hk : 1;
-        const int64_t grid256 = (int64_t)CEIL_DIV(Sq, 256) * B * Hq;
-        // a second round of 128-row blocks costs more than the merged form's idle
-        // CUs (32 heads on 8: 1500 tokens 85 us in 384 blocks, 58 merged in 192;
-        // 1024 tokens 38.5 in 256 blocks, 42.6 merged in 128)
-        const int64_t grid128 = (int64_t)CEIL_DIV(Sq, 128) * B * Hq;
-        if ((gq == 2 || gq == 4 || gq == 8) && grid128 > 256)
-            variant = 9;
-        else if (grid256 >= 256)
-            variant = 8;
-        else
-            variant = 7;
+    const int gq = (Hk > 0 && Hq % Hk == 0) ? Hq / Hk : 1;
+    const bool shared = gq == 2 || gq == 4 || gq == 8;
+    if (variant <= 0 && steady) {
+        const int64_t heads = (int64_t)B * Hq;
+        variant = shared && CEIL_DIV(Sq, 128) * heads > 256 ? 9
+                  : CEIL_DIV(Sq, 256) * heads >= 256 ? 8 : 7;
+    } else if (variant <= 0) {
+        const float one = prefill_us(1, B, Hq, Sq, Skv), two = prefill_us(2, B, Hq, Sq, Skv),
+                    four = prefill_us(4, B, Hq, Sq, Skv);
+        variant = four <= two && four <= one ? 11 : two <= one ? 10 : shared ? 9 : 8;
     }
     return oa_attention_prefill_variant(stream, q, k, v, out, B, Hq, Hk, Sq,
                                         Skv, D, scale, q_stride, k_stride,

@@ -1,5 +1,5 @@
 """Prefill-attention variant bench: correctness vs torch fp32 + TF/s per
-variant (OPSAGENT_PREFILL_VARIANT 1..4) at agent-relevant shapes.
+variant (OPSAGENT_PREFILL_VARIANT 7 to 11) at agent-relevant shapes.
 
 Run under gpurun; summary goes to stdout (commit to profiles/README.md).
 """
@@ -51,7 +51,7 @@ def timeit(fn, iters, warmup=5):
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--iters", type=int, default=20)
-    ap.add_argument("--variants", default="1,2,3,4")
+    ap.add_argument("--variants", default="7,8,9,10,11")
     ap.add_argument("--shapes", default="", help="comma list of shape indices")
     args = ap.parse_args()
     assert torch.cuda.is_available()

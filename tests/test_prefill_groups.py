@@ -1,0 +1,94 @@
+"""Prefill attention in one, two and four key groups a block, at the edges of query tiles, key
+tiles and groups, against float64: groups that see no key of a row, groups without a tile."""
+
+import pytest
+import torch
+
+from opsagent_amd import ops
+
+D = 128
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("variant", [7, 8, 10, 11, 0])   # steady, 1, 2, 4 groups, by the rule
+@pytest.mark.parametrize("B,Hq,Hk,Sq,Skv", [
+    (1, 4, 4, 1, 1),              # one key: three of four groups have no tile
+    (1, 4, 2, 33, 33),            # a second wave of one row, groups behind the diagonal
+    (2, 6, 2, 65, 97),            # three heads a key head, a tile of one key more
+    (1, 3, 1, 129, 191),
+    (1, 16, 2, 64, 64),
+    (3, 8, 8, 257, 257),          # a query tile of one row in every form
+    (1, 8, 1, 127, 300),
+    (1, 32, 8, 700, 740),         # more blocks than CUs
+])
+def test_forms(monkeypatch, variant, B, Hq, Hk, Sq, Skv):
+    if variant:
+        monkeypatch.setenv("OPSAGENT_PREFILL_VARIANT", str(variant))
+    gen = torch.Generator(device="cuda").manual_seed(Sq + Skv)
+    q = torch.randn(B, Sq, Hq + 1, D, generator=gen, device="cuda").bfloat16()[:, :, :Hq]
+    kv = torch.randn(B, Skv, 2 * Hk, D, generator=gen, device="cuda").bfloat16()
+    k, v = kv[:, :, :Hk], kv[:, :, Hk:]
+    check(ops.attention_prefill(q, k, v), q, k, v)
+
+
+def check(got, q, k, v):
+    (B, Sq, Hq, _), (Skv, Hk) = q.shape, k.shape[1:3]
+    i = torch.arange(Skv - Sq, Skv, device="cuda")[:, None]
+    hidden = torch.arange(Skv, device="cuda")[None] > i
+    for b in range(B):
+        for h in range(Hq):
+            g = h // (Hq // Hk)
+            s = (q[b, :, h].double() @ k[b, :, g].double().T * D ** -0.5).masked_fill(hidden, -1e30)
+            want = torch.softmax(s, -1) @ v[b, :, g].double()
+            # weights enter the value product in bf16 (2^-8 at most, 0.0016 in the
+            # mean, over many keys of either sign) and the result is rounded once
+            err = (got[b, :, h].double() - want).norm() / want.norm()
+            assert err < 6e-3, (b, h, float(err))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hk,Sq,Skv", [(8, 2, 40, 700), (8, 2, 128, 383), (8, 2, 300, 1600),
+                                          (32, 8, 130, 200), (32, 8, 1100, 1100)])
+def test_steady(Hq, Hk, Sq, Skv):
+    """What 8-bit models call: split and not, 128 rows and 256."""
+    gen = torch.Generator(device="cuda").manual_seed(Sq)
+    q, k, v = (torch.randn(1, n, h, D, generator=gen, device="cuda").bfloat16()
+               for n, h in ((Sq, Hq), (Skv, Hk), (Skv, Hk)))
+    check(ops.attention_prefill(q, k, v, steady=True), q, k, v)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("variant", [10, 11])
+def test_scores_that_do_not_compare(monkeypatch, variant):
+    """A row with a NaN or a positive infinite score is NaN in whichever group the score lies,
+    and so is the softmax of no key; other rows of its block are not."""
+    monkeypatch.setenv("OPSAGENT_PREFILL_VARIANT", str(variant))
+    gen = torch.Generator(device="cuda").manual_seed(variant)
+    Sq, Skv = 60, 340
+    q, k, v = (torch.randn(1, n, 2, D, generator=gen, device="cuda").bfloat16()
+               for n in (Sq, Skv, Skv))
+    q[0, 3, 1, 5] = float("nan")
+    k[0, 70, 0, 7] = float("inf")
+    v[0, 100, 1, 9] = float("nan")
+    bad = torch.zeros(1, Sq, 2, D, dtype=torch.bool, device="cuda")
+    bad[0, 3, 1] = True
+    bad[0, :, 0] |= (q[0, :, 0, 7] > 0)[:, None]
+    bad[0, :, 1, 9] = True
+    assert torch.equal(torch.isnan(ops.attention_prefill(q, k, v)), bad)
+    # ten rows in front of the first key
+    got = ops.attention_prefill(q[:, :, :1], k[:, :50, 1:], v[:, :50, :1])
+    assert torch.isnan(got[0, :10]).all() and torch.isfinite(got[0, 10:]).all()
+
+
+def test_few_splits():
+    """Splits only where they beat key groups: more tiles where few splits fill the chip or
+    where many rows leave sums; the steady form by its own rule."""
+    plan = ops._prefill_plan
+    for Hq, Sq, n, least in ((32, 1000, 2, 64), (32, 520, 3, 20), (32, 400, 4, 28),
+                             (16, 700, 5, 18), (32, 300, 6, 16)):
+        assert plan(1, Hq, Hq // 4, Sq, 128 * least) == (n, 1)
+        assert plan(1, Hq, Hq // 4, Sq, 128 * (least - 1)) == (1, 1)
+        assert plan(1, Hq, Hq // 4, Sq, 128 * (least - 1), True) == (n, 1)
+    assert plan(1, 32, 8, 77, 1264) == (8, 0) and plan(1, 32, 8, 77, 1264, True) == (8, 2)
+    assert plan(1, 80, 20, 128, 768) == (1, 0) and plan(1, 80, 20, 128, 768, True) == (3, 2)
+    assert plan(1, 80, 20, 40, 2048) == (3, 0) and plan(1, 6, 2, 300, 4000) == (1, 0)
