@@ -752,29 +752,19 @@ def _ring_choice_fp8(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
 
 
 @functools.lru_cache(maxsize=4096)
-def _tile_plan_fp8(M: int, N: int, K: int) -> int:
-    return _lib()[0].oa_tile_gemm_fp8_plan(M, N, K)
+def _tile_form_fp8(M: int, N: int, K: int) -> int:
+    return _lib()[0].oa_tile_gemm_fp8_form(M, N, K)
 
 
 def _gemm_fp8(a8: torch.Tensor, a_scale: torch.Tensor, w8: torch.Tensor,
               w_scale: torch.Tensor) -> torch.Tensor:
     """The product of fp8 rows a8 [M, K] (K % 128 == 0) and w8 [N, K] with their row
-    scales, bf16 [M, N]: on the transfer ring up to 128 rows, above in tiles of one kind or the
-    other (tile_gemm.hip; the rule there)."""
+    scales, bf16 [M, N]: on the transfer ring where its column splits fill the chip, above 128
+    rows in tiles of one kind or the other (tile_gemm.hip; the rule there), bit for bit the
+    same."""
     (M, K), N = a8.shape, w8.shape[0]
     lib, hip = _lib()
     out = torch.empty(M, N, dtype=torch.bfloat16, device=a8.device)
-    tile = _tile_plan_fp8(M, N, K) if M > 128 else -1
-    if tile >= 0 and w8.data_ptr() % 16 == 0 and a8.data_ptr() % 16 == 0:
-        splits = tile & 255
-        # at most 256 tiles of 256 x 256 float32: 67 MB
-        part = None if splits == 1 else torch.empty(splits * M * N, dtype=torch.float32,
-                                                    device=a8.device)
-        hip.check(lib.oa_tile_gemm_fp8(
-            hip.current_stream_ptr(), a8.data_ptr(), a_scale.data_ptr(), w8.data_ptr(),
-            w_scale.data_ptr(), out.data_ptr(), None if part is None else part.data_ptr(),
-            M, N, K, tile), "oa_tile_gemm_fp8")
-        return out
     plan = _ring_choice_fp8(M, N, K)
     if plan and w8.data_ptr() % 16 == 0 and a8.data_ptr() % 16 == 0:
         tile, splits = plan
@@ -785,6 +775,12 @@ def _gemm_fp8(a8: torch.Tensor, a_scale: torch.Tensor, w8: torch.Tensor,
             hip.current_stream_ptr(), a8.data_ptr(), a_scale.data_ptr(), w8.data_ptr(),
             w_scale.data_ptr(), out.data_ptr(), None if part is None else part.data_ptr(),
             M, N, K, tile, splits), "oa_ring_gemm_fp8")
+        return out
+    form = _tile_form_fp8(M, N, K) if M > 128 else -1
+    if form >= 0 and w8.data_ptr() % 16 == 0 and a8.data_ptr() % 16 == 0:
+        hip.check(lib.oa_tile_gemm_fp8(
+            hip.current_stream_ptr(), a8.data_ptr(), a_scale.data_ptr(), w8.data_ptr(),
+            w_scale.data_ptr(), out.data_ptr(), M, N, K, form), "oa_tile_gemm_fp8")
         return out
     rc = lib.oa_gemm_fp8(
         hip.current_stream_ptr(), a8.data_ptr(), w8.data_ptr(),
@@ -1290,6 +1286,7 @@ def _prefill_splits(B: int, Hq: int, Hk: int, Sq: int, Skv: int) -> Tuple[int, b
     return max(1, min(tiles, 256 // max(1, blocks))), True
 
 
+@functools.lru_cache(maxsize=4096)
 def _prefill_plan(
     B: int, Hq: int, Hk: int, Sq: int, Skv: int, steady: bool = False
 ) -> Tuple[int, int]:

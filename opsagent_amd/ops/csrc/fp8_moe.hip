@@ -995,7 +995,7 @@ __global__ __launch_bounds__(1024, 4 * BLOCKS) void gemm_fp8_tile_kernel(
 // above): one block of 128 x 128 a CU 0.62 (0.65 over several rounds, which start and end
 // bare), two of them 1.27 and less where the second ones are few, 128 x 256 1.12, 256 x 256
 // 1.9. It names the fastest for 39 of 40 sizes (12288 x 4096, M = 512: 42.1, 38.2).
-static int gemm_fp8_tile(int64_t M, int64_t N, double* us = nullptr) {
+static int gemm_fp8_tile(int64_t M, int64_t N, double* us = nullptr, int64_t* rounds = nullptr) {
     const int64_t n1 = CEIL_DIV(M, 128) * CEIL_DIV(N, 128), rest = n1 % 512;
     const int64_t n2 = CEIL_DIV(M, 128) * CEIL_DIV(N, 256), n3 = CEIL_DIV(M, 256) * CEIL_DIV(N, 256);
     const double t[4] = {n1 <= 256 ? 0.62 : CEIL_DIV(n1, 256) * 0.65,
@@ -1005,14 +1005,16 @@ static int gemm_fp8_tile(int64_t M, int64_t N, double* us = nullptr) {
     for (int i = 1; i < 4; ++i)
         if (t[i] < t[best]) best = i;
     if (us) *us = t[best];
+    if (rounds) *rounds = best == 1 ? CEIL_DIV(n1, 512) : CEIL_DIV(best == 0 ? n1 : best == 2 ? n2 : n3, 256);
     return best;
 }
 
-// its time, us: of the steps, to start and to end (13% rms over 90 sizes)
+// its time, us: of the steps, and to start and to end each round (11% rms over 50 sizes)
 extern "C" double oa_gemm_fp8_us(int M, int N, int K) {
     double us;
-    gemm_fp8_tile(M, N, &us);
-    return us * (K / GK2) + 3.4;
+    int64_t rounds;
+    gemm_fp8_tile(M, N, &us, &rounds);
+    return 0.93 * us * (K / GK2) + 4.9 * rounds + 0.3;
 }
 
 extern "C" int oa_gemm_fp8(void* stream, const void* a8, const void* b8,

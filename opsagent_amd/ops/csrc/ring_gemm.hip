@@ -264,19 +264,13 @@ __global__ __launch_bounds__(256) void ring_sum_kernel(const float* __restrict__
         make_uint2(pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]));
 }
 
-// out [M, N] = the sum of parts [splits, M, N], in order, times xscale[m] * wscale[n] where given
-extern "C" int oa_ring_sum(void* stream, const void* part, const void* xscale, const void* wscale, void* out,
-                           int M, int N, int splits) {
+// out [M, N] = the sum of parts [splits, M, N], in order
+extern "C" int oa_ring_sum(void* stream, const void* part, void* out, int M, int N, int splits) {
     if (M < 1 || M > 65535 || N < 4 || N % 4 != 0 || splits < 1 || !part || !out) return -100;
     if (((uintptr_t)part | (uintptr_t)out) % 16 != 0) return -102;
     const dim3 grid(CEIL_DIV(N / 4, 256), M);
-#define RGS(F8V)                                                                                         \
-    hipLaunchKernelGGL((ring_sum_kernel<false, F8V>), grid, dim3(256), 0, (hipStream_t)stream,           \
-                       (const float*)part, (const float*)xscale, (const float*)wscale, (uint16_t*)out, M, \
-                       N, splits, 0)
-    if (xscale) RGS(true);
-    else RGS(false);
-#undef RGS
+    hipLaunchKernelGGL((ring_sum_kernel<false, false>), grid, dim3(256), 0, (hipStream_t)stream, (const float*)part,
+                       (const float*)nullptr, (const float*)nullptr, (uint16_t*)out, M, N, splits, 0);
     HIP_CHECK_LAUNCH();
     return 0;
 }

@@ -18,20 +18,19 @@
 // compiler copies sums between register files); v_mfma_f32_32x32x16_bf16 (1.6 PFLOP/s from LDS);
 // touching the lines of later steps (results come in order: it waits behind them).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) float tgf4;
 typedef __attribute__((ext_vector_type(8))) short tgs8;
 typedef __attribute__((ext_vector_type(8))) int tgi8;
+typedef __attribute__((ext_vector_type(16))) float tgf16;
 
-// A fragment's 16 rows of a step: 128 bytes of each, 32 a lane. Lane group c has chunks c and c + 4, in
-// bf16 the columns of the two products that they stand for; in e4m3 the order of a product's columns is
-// free as long as both operands share it, and chunks 2 c and 2 c + 1 collide in the LDS banks (256 x 256
-// 1.66 us a step, 1.37 so).
-union TgFrag {
+// A fragment's 16 rows of a step: 128 bytes of each, 32 a lane. Lane group c has chunks c and c + 4, the
+// columns of the two products that they stand for.
+struct TgFrag {
     tgs8 b[2];
-    tgi8 f8;
 };
 struct TgAt {
     int a, b;
@@ -42,21 +41,17 @@ struct TgAt {
     }
 };
 
-// the fragments of FI x FJ over a step: the products of bf16, or of e4m3 with unit block scales (the only
-// fp8 products past the bf16 rate)
-template <bool F8, int FI, int FJ>
+// the fragments of FI x FJ over a step
+template <int FI, int FJ>
 __device__ __forceinline__ void tg_multiply(tgf4 (&acc)[FI][FJ], const TgFrag (&wf)[FJ], const TgFrag (&xf)[FI]) {
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int k = 0; k < (F8 ? 1 : 2); ++k)
+    for (int k = 0; k < 2; ++k)
 #pragma unroll
         for (int i = 0; i < FI; ++i)
 #pragma unroll
             for (int j = 0; j < FJ; ++j)
-                if constexpr (F8)
-                    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[j].f8, xf[i].f8, acc[i][j], 0, 0, 0, 0x7f, 0, 0x7f);
-                else
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j].b[k], xf[i].b[k], acc[i][j], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j].b[k], xf[i].b[k], acc[i][j], 0, 0, 0);
     __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
 }
@@ -69,6 +64,58 @@ __device__ __forceinline__ void tg_read(TgFrag (&wf)[FJ], TgFrag (&xf)[FI], cons
 #pragma unroll
         for (int i = 0; i < FI; ++i) xf[i].b[k] = *reinterpret_cast<const tgs8*>(xr + i * 2048 + (k ? at.b : at.a));
     }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// e4m3: fragments of 32 rows, two products of 64 columns a step with unit block scales (the only fp8
+// products past the bf16 rate). Lane half h has bytes 64 k + 32 h and up of its row: products, order
+// and rounding of the one-barrier tiles (fp8_moe.hip), since an 8-bit model turns another order of the
+// sums into 0.01 to 0.03 of its activations. v_mfma_scale_f32_16x16x128 gains 2% more (28672 x 4096,
+// M = 700 93.4 us, here 94).
+struct TgFrag8 {
+    tgi8 k[2];
+};
+struct TgAt8 {
+    int at[2][2];
+    __device__ __forceinline__ TgAt8(int lane) {
+        const int r = lane & 31, h = lane >> 5;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) at[k][c] = r * 128 + (((k * 4 + h * 2 + c) ^ (r >> 1 & 7)) << 4);
+    }
+};
+template <int FI, int FJ>
+__device__ __forceinline__ void tg_read(TgFrag8 (&wf)[FJ], TgFrag8 (&xf)[FI], const char* wr, const char* xr, const TgAt8& at) {
+    auto one = [&](const char* rows, int k) {
+        union {
+            uint4 c[2];
+            tgi8 v;
+        } f;
+        f.c[0] = *reinterpret_cast<const uint4*>(rows + at.at[k][0]);
+        f.c[1] = *reinterpret_cast<const uint4*>(rows + at.at[k][1]);
+        return f.v;
+    };
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+        for (int j = 0; j < FJ; ++j) wf[j].k[k] = one(wr + j * 4096, k);
+#pragma unroll
+        for (int i = 0; i < FI; ++i) xf[i].k[k] = one(xr + i * 4096, k);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+template <int FI, int FJ>
+__device__ __forceinline__ void tg_multiply(tgf16 (&acc)[FI][FJ], const TgFrag8 (&wf)[FJ], const TgFrag8 (&xf)[FI]) {
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int i = 0; i < FI; ++i)
+#pragma unroll
+            for (int j = 0; j < FJ; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wf[j].k[k], xf[i].k[k], acc[i][j], 0, 0, 0, 0x7f, 0, 0x7f);
+    __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
 }
 
@@ -97,9 +144,10 @@ __device__ __forceinline__ float tg_gate(float g, float u, int act) {
 
 // the weight row (from the strip's first on) that LDS row b of the strip holds: a wave's fragments in
 // pairs whose lanes hold eight neighbouring outputs together, gate rows beside their up rows
-template <int FJ, bool GU>
+template <int FJ, bool GU, bool F8 = false>
 __device__ __forceinline__ int tg_wrow(int b) {
     static_assert(FJ % 2 == 0, "pairs");
+    if (F8) return (b & ~15) + (b >> 2 & 1) * 8 + (b >> 3 & 1) * 4 + (b & 3);    // a lane's eights together
     const int wv = b / (16 * FJ), j = b / 16 % FJ, r = b & 15;
     if (GU) {
         if (FJ % 4 == 0) return wv * FJ * 8 + (j >> 2) * 32 + (r >> 2) * 8 + (j & 1) * 4 + (r & 3);
@@ -114,9 +162,8 @@ __device__ __forceinline__ bool tg_isup(int b) {
 }
 
 // fragments I0 .. I1 of a wave whose first row is row0
-template <int FI, int FJ, bool GU, bool F8, int I0, int I1>
-__device__ __forceinline__ void tg_store(tgf4 (&acc)[FI][FJ], const float* xscale, const float* wscale,
-                                         uint16_t* out, float* part, int row0, int n0, int wc, int M, int N, int sp, int act) {
+template <int FI, int FJ, bool GU, int I0, int I1>
+__device__ __forceinline__ void tg_store(tgf4 (&acc)[FI][FJ], uint16_t* out, float* part, int row0, int n0, int wc, int M, int N, int sp, int act) {
     const int fr = threadIdx.x & 15, fc = threadIdx.x >> 4 & 3;
     // D: column (row of x) lane & 15, rows (weight rows) (lane >> 4) * 4 and up
 #pragma unroll
@@ -152,19 +199,38 @@ __device__ __forceinline__ void tg_store(tgf4 (&acc)[FI][FJ], const float* xscal
                 continue;
             }
             if (j % 2) continue;
-            if constexpr (F8) {
-                const float sx = xscale[row];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    acc[i][j][e] = acc[i][j][e] * sx * wscale[col + e];
-                    acc[i][j + 1][e] = acc[i][j + 1][e] * sx * wscale[col + 4 + e];
-                }
-            }
             *reinterpret_cast<uint4*>(out + (size_t)row * N + col) =
                 make_uint4(pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3]),
                            pack_bf16x2(acc[i][j + 1][0], acc[i][j + 1][1]),
                            pack_bf16x2(acc[i][j + 1][2], acc[i][j + 1][3]));
         }
+    }
+}
+
+// 32 x 32 fragments: column (row of x) lane & 31, a lane half twice eight weight rows beside the other's
+template <int FI, int FJ>
+__device__ __forceinline__ void tg_store8(const tgf16 (&acc)[FI][FJ], const float* xscale, const float* wscale,
+                                          uint16_t* out, int row0, int n0, int wc, int M, int N) {
+    const int fr = threadIdx.x & 31, half = threadIdx.x >> 5 & 1;
+#pragma unroll
+    for (int i = 0; i < FI; ++i) {
+        const int row = row0 + i * 32 + fr;
+        if (row >= M) continue;
+        const float sx = xscale[row];
+#pragma unroll
+        for (int j = 0; j < FJ; ++j)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int col = n0 + (wc * FJ + j) * 32 + c * 16 + half * 8;
+                if (col >= N) continue;                       // N % 8 == 0
+                uint32_t o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int k = c * 8 + 2 * e;
+                    o[e] = pack_bf16x2(acc[i][j][k] * sx * wscale[col + 2 * e], acc[i][j][k + 1] * sx * wscale[col + 2 * e + 1]);
+                }
+                *reinterpret_cast<uint4*>(out + (size_t)row * N + col) = make_uint4(o[0], o[1], o[2], o[3]);
+            }
     }
 }
 
@@ -209,7 +275,7 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
         const int r = (p * 4 + wc) * 8 + (lane >> 3);
         const int chunk = ((lane & 7) ^ (r >> 1 & 7)) * 16;
         if (!grp) off[p] = (uint32_t)min(r, M - 1 - m0) * (uint32_t)xs + chunk;
-        else off[p] = (uint32_t)(min(tg_wrow<FJ, GU>(r), N - 1 - n0) + (tg_isup<FJ, GU>(r) ? N : 0)) * (uint32_t)kb + chunk;
+        else off[p] = (uint32_t)(min(tg_wrow<FJ, GU, F8>(r), N - 1 - n0) + (tg_isup<FJ, GU>(r) ? N : 0)) * (uint32_t)kb + chunk;
     }
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + (grp ? XS * XB : 0) + wc * 1024);
     auto stage_x = [&](int buf) {
@@ -234,7 +300,9 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
         else tg_wait<0>();
     };
 
-    tgf4 acc[FI][FJ] = {};
+    constexpr int AI = F8 ? FI / 2 : FI, AJ = F8 ? FJ / 2 : FJ;
+    static_assert(!F8 || (FI % 2 == 0 && !GU), "fragments of 32 rows");
+    std::conditional_t<F8, tgf16, tgf4> acc[AI][AJ] = {};
     if (!grp) {
 #pragma unroll
         for (int t = 0; t < XS - 1; ++t)
@@ -249,13 +317,13 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
         tg_barrier();
         tg_barrier();
     }
-    const TgAt at(lane);
+    const std::conditional_t<F8, TgAt8, TgAt> at(lane);
     int xbuf = 0, wbuf = 0;
     for (int t = 0; t < n; ++t) {
         const char* xr = smem + xbuf * XB + grp * FI * 16 * 128;
         const char* wr = smem + XS * XB + wbuf * WB + wc * FJ * 16 * 128;
-        TgFrag xf[FI], wf[FJ];
-        tg_read<FI, FJ>(wf, xf, wr, xr, at);
+        std::conditional_t<F8, TgFrag8, TgFrag> xf[AI], wf[AJ];
+        tg_read<AI, AJ>(wf, xf, wr, xr, at);
         if (!grp) {
             if (t + XS - 1 < n) stage_x(xbuf == 0 ? XS - 1 : xbuf - 1);
         } else {
@@ -264,7 +332,7 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
         }
         tg_read_done();
         tg_barrier();
-        tg_multiply<F8, FI, FJ>(acc, wf, xf);
+        tg_multiply<AI, AJ>(acc, wf, xf);
         if (!grp) landed_x(min(XS - 2, n - 2 - t));
         tg_barrier();
         xbuf = xbuf + 1 == XS ? 0 : xbuf + 1;
@@ -272,14 +340,16 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
     }
     if (!grp) tg_barrier();
 
-    tg_store<FI, FJ, GU, F8, 0, FI>(acc, xscale, wscale, out, part, m0 + grp * FI * 16, n0, wc, M, N, sp, act);
+    const int row0 = m0 + grp * FI * 16;
+    if constexpr (F8) tg_store8<AI, AJ>(acc, xscale, wscale, out, row0, n0, wc, M, N);
+    else tg_store<FI, FJ, GU, 0, FI>(acc, out, part, row0, n0, wc, M, N, sp, act);
 }
 
 // Tiles of 32 FI x 32 FJ: a wave of 2 x 2 takes a quarter of the tile and the groups take the steps in
 // turn, each into sums of its own, which are added up at the end. A quarter a wave reads less LDS than
 // an eighth (128 x 128: 64 KB a step and not 98), and a phase is a whole step for both (800 x 4096 x 4096
 // 40 us with eighths, 34 here; 800 x 4096 x 14336 126, 103).
-template <int FI, int FJ, int ST, bool GU, bool F8>
+template <int FI, int FJ, int ST, bool GU>
 __global__ __launch_bounds__(512, 2) void tile_gemm_turns_kernel(
     const char* __restrict__ x, int64_t xs, const char* __restrict__ w,
     const float* __restrict__ xscale, const float* __restrict__ wscale, uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int64_t kb, int mtiles,
@@ -348,7 +418,7 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_turns_kernel(
         if (ST % 2 == 0 && s + 1 < n) landed(s + 1);
         tg_read_done();
         tg_barrier();                                        // the end of phase s
-        tg_multiply<F8, FI, FJ>(acc, wf, xf);
+        tg_multiply<FI, FJ>(acc, wf, xf);
         if (s + 1 < n) {
             if (ST % 2 && s + 2 < n) landed(s + 2);
             tg_barrier();                                    // the end of phase s + 1
@@ -375,49 +445,52 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_turns_kernel(
         for (int i = FH; i < FI; ++i)
 #pragma unroll
             for (int j = 0; j < FJ; ++j) acc[i][j] += ex[((i * FJ + j) * 4 + wid) * 64 + lane];
-        tg_store<FI, FJ, GU, F8, FH, FI>(acc, xscale, wscale, out, part, m0 + wm * FI * 16, n0, wc, M, N, sp, act);
+        tg_store<FI, FJ, GU, FH, FI>(acc, out, part, m0 + wm * FI * 16, n0, wc, M, N, sp, act);
     } else {
 #pragma unroll
         for (int i = 0; i < FH; ++i)
 #pragma unroll
             for (int j = 0; j < FJ; ++j) acc[i][j] += ex[((i * FJ + j) * 4 + wid) * 64 + lane];
-        tg_store<FI, FJ, GU, F8, 0, FH>(acc, xscale, wscale, out, part, m0 + wm * FI * 16, n0, wc, M, N, sp, act);
+        tg_store<FI, FJ, GU, 0, FH>(acc, out, part, m0 + wm * FI * 16, n0, wc, M, N, sp, act);
     }
 }
 
 // Forms, and what they take in us: a step (64 columns, e4m3 128), more of it when all CUs work (power, and
 // x from beside the chip), starting and ending a tile; least squares over 2700 times of 110 products
-// (e4m3: 1900 of 90), to 6 to 11%. The choice by them takes 1.01 of the time of the best form (1.13 at
-// most).
+// (e4m3: 460 of 104), to 6 to 11% (6%). The choice by them takes 1.01 of the time of the best form (1.13 at
+// most). e4m3 has forms of the first kernel only: the turns of the second and column splits add up in
+// another order, and an 8-bit model turns that into 0.01 to 0.03 of its activations.
 struct TgForm {
-    int bm, bn;
-    float step, more, tile, step8, more8, tile8;
+    int id, bm, bn;
+    float step, more, tile;
 };
 static const TgForm tg_forms[] = {
-    {256, 256, 0.872f, 0.498f, 9.2f, 1.192f, 0.343f, 6.8f}, {224, 256, 0.796f, 0.425f, 8.3f, 1.100f, 0.275f, 6.6f},
-    {192, 256, 0.734f, 0.381f, 7.6f, 0.944f, 0.310f, 6.0f}, {160, 256, 0.673f, 0.295f, 7.2f, 0.741f, 0.195f, 6.6f},
-    {256, 128, 0.531f, 0.295f, 6.7f, 0.849f, 0.122f, 6.8f}, {224, 128, 0.471f, 0.264f, 6.1f, 0.730f, 0.125f, 6.9f},
-    {160, 128, 0.393f, 0.201f, 5.3f, 0.558f, 0.126f, 6.3f}, {128, 128, 0.352f, 0.195f, 4.1f, 0.453f, 0.120f, 5.5f},
-    {96, 128, 0.292f, 0.170f, 2.8f, 0.350f, 0.115f, 4.4f},  {128, 64, 0.259f, 0.116f, 2.5f, 0.276f, 0.108f, 3.8f},
+    {0, 256, 256, 0.872f, 0.498f, 9.2f}, {1, 224, 256, 0.796f, 0.425f, 8.3f}, {2, 192, 256, 0.734f, 0.381f, 7.6f},
+    {3, 160, 256, 0.673f, 0.295f, 7.2f}, {4, 256, 128, 0.531f, 0.295f, 6.7f}, {5, 224, 128, 0.471f, 0.264f, 6.1f},
+    {6, 160, 128, 0.393f, 0.201f, 5.3f}, {7, 128, 128, 0.352f, 0.195f, 4.1f}, {8, 96, 128, 0.292f, 0.170f, 2.8f},
+    {9, 128, 64, 0.259f, 0.116f, 2.5f},
+};
+static const TgForm tg_forms8[] = {
+    {0, 256, 256, 1.063f, 0.734f, 6.6f}, {1, 192, 256, 0.887f, 0.539f, 5.3f}, {2, 128, 256, 0.583f, 0.349f, 5.6f},
+    {3, 192, 128, 0.525f, 0.227f, 5.3f}, {4, 64, 128, 0.396f, 0.066f, 3.5f},
 };
 
-// The fastest form and column splits as form * 256 + splits, and its time in *us. A split has `least` steps.
-static int tg_choose(int M, int rows, int steps, bool split, int least, bool summed, bool f8, float* us_best) {
+// The fastest of the forms and column splits as form * 256 + splits, and its time in *us. A split has eight steps.
+template <int FORMS>
+static int tg_choose(const TgForm (&forms)[FORMS], int M, int rows, int steps, bool split, bool summed, float* us_best) {
     const float mn = (float)M * rows;
     float best = 1e30f;
     int plan = -1;
-    for (int f = 0; f < (int)(sizeof(tg_forms) / sizeof(tg_forms[0])); ++f) {
-        const TgForm& t = tg_forms[f];
-        const float step = f8 ? t.step8 : t.step, more = f8 ? t.more8 : t.more, tile = f8 ? t.tile8 : t.tile;
+    for (const TgForm& t : forms) {
         const int64_t tiles = (int64_t)CEIL_DIV(M, t.bm) * CEIL_DIV(rows, t.bn);
         const int most = split && tiles < 256 ? (int)std::min<int64_t>(8, 256 / tiles) : 1;
-        for (int sp = 1; sp <= most && (sp == 1 || steps / sp >= least); ++sp) {
+        for (int sp = 1; sp <= most && (sp == 1 || steps / sp >= 8); ++sp) {
             const int64_t blocks = tiles * sp, full = blocks / 256, rest = blocks % 256;
             const float n = (float)steps / sp;
-            float us = full * (n * (step + more) + 0.6f * tile) + 0.4f * tile + 2;
-            if (rest) us += n * (step + more * rest / 256) + 0.6f * tile;
+            float us = full * (n * (t.step + t.more) + 0.6f * t.tile) + 0.4f * t.tile + 2;
+            if (rest) us += n * (t.step + t.more * rest / 256) + 0.6f * t.tile;
             if (sp > 1) us += sp * mn * 0.36e-6f + (summed ? (sp * 4 - 2) * mn / 4.5e6f : 2.5f + sp * mn * 4 / 4.5e6f);
-            if (us < best) best = us, plan = f * 256 + sp;
+            if (us < best) best = us, plan = t.id * 256 + sp;
         }
     }
     *us_best = best;
@@ -433,28 +506,28 @@ static int tg_choose(int M, int rows, int steps, bool split, int least, bool sum
 extern "C" int oa_tile_gemm_plan(int M, int N, int K, int gateup, int summed) {
     if (M < 1 || N < 8 || N % 8 != 0 || N > (1 << 29) || K < 512 || K % 64 != 0) return -1;
     float one, two;
-    if (!gateup) return tg_choose(M, N, K / 64, true, 8, summed, false, &one);
-    const int plan = tg_choose(M, 2 * N, K / 64, false, 8, false, false, &one);
-    tg_choose(M, 2 * N, K / 64, true, 8, false, false, &two);
+    if (!gateup) return tg_choose(tg_forms, M, N, K / 64, true, summed, &one);
+    const int plan = tg_choose(tg_forms, M, 2 * N, K / 64, false, false, &one);
+    tg_choose(tg_forms, M, 2 * N, K / 64, true, false, &two);
     return one > two + 3 + (float)M * N * 6 / 4.5e6f ? -1 : plan;
 }
 
 extern "C" double oa_gemm_fp8_us(int M, int N, int K);
 
-// The plan of an e4m3 product, -1 for sizes that it does not take and where the one-barrier tiles
-// (fp8_moe.hip) are the faster ones by both models: at 90 sizes of 130 to 2048 rows this takes 0.90 of the
-// time of those and the ring, 0.89 would be the best. Us, those / here: 28672 x 4096, M = 256 45.8 / 41.7,
-// 700 104 / 91, 2048 249 / 218; 4096 x 14336, 333 45.4 / 37.3, 700 58.7 / 52.8; 6144 x 4096, 700 34.4 /
-// 29.5, 1434 56.2 / 37.3; 2048 x 2048, 512 12.6 / 10.7; but 3072 x 2048, 1024 13.6 / 15.5.
-extern "C" int oa_tile_gemm_fp8_plan(int M, int N, int K) {
+// The form of an e4m3 product, -1 for sizes that it does not take and where the one-barrier tiles
+// (fp8_moe.hip), which answer the same bit for bit, are the faster ones by both models (they are late by 6%
+// here): at 84 sizes of 130 to 2048 rows this takes 0.929 of the time of those, 0.926 would be the best. Us,
+// those / here: 28672 x 4096, M = 130 41.6 / 36.6, 700 109.6 / 94.7, 1700 228 / 193, 2048 259 / 236; 6144 x
+// 4096, 700 33.6 / 28.2, 1400 56.3 / 44.4; 4096 x 14336, 1400 110 / 88; 2048 x 2048, 450 13.2 / 12.1; 16384
+// x 2048, 450 25.7 / 23.4; but 6144 x 4096, 450 21.5 / 26.9 and 2048 x 8192, 1400 34.8 / 45.6.
+extern "C" int oa_tile_gemm_fp8_form(int M, int N, int K) {
     if (M < 1 || N < 8 || N % 8 != 0 || N > (1 << 29) || K < 512 || K % 128 != 0 || K >= (1 << 23)) return -1;
     float us;
-    const int plan = tg_choose(M, N, K / 128, true, 4, false, true, &us);
-    return us < oa_gemm_fp8_us(M, N, K) ? plan : -1;
+    const int plan = tg_choose(tg_forms8, M, N, K / 128, false, false, &us);
+    return us < 1.06 * oa_gemm_fp8_us(M, N, K) ? plan >> 8 : -1;
 }
 
-extern "C" int oa_ring_sum(void* stream, const void* part, const void* xscale, const void* wscale, void* out,
-                           int M, int N, int splits);
+extern "C" int oa_ring_sum(void* stream, const void* part, void* out, int M, int N, int splits);
 
 // xs, kb: bytes of a row of x and of a weight row
 static int tg_run(hipStream_t s, const void* x, int64_t xs, const void* w, const void* xscale, const void* wscale,
@@ -469,25 +542,36 @@ static int tg_run(hipStream_t s, const void* x, int64_t xs, const void* w, const
                            (const float*)wscale, (uint16_t*)out, (float*)part, M, N, kb, mt,       \
                            splits, (int)items, act);                                               \
     } while (0)
-#define TG_HALVES(FI, FJ, XS, WS)                                                                            \
-    do {                                                                                                     \
-        constexpr int lds = ((XS) * 32 * (FI) + (WS) * 64 * (FJ)) * 128;                                     \
-        if (f8) TG_LAUNCH((tile_gemm_kernel<FI, FJ, XS, WS, false, true>), 32 * (FI), 64 * (FJ), lds);       \
-        else if (act) TG_LAUNCH((tile_gemm_kernel<FI, FJ, XS, WS, true, false>), 32 * (FI), 64 * (FJ), lds); \
-        else TG_LAUNCH((tile_gemm_kernel<FI, FJ, XS, WS, false, false>), 32 * (FI), 64 * (FJ), lds);         \
+#define TG_HALVES(FI, FJ, XS, WS, GU, F8)                                                        \
+    TG_LAUNCH((tile_gemm_kernel<FI, FJ, XS, WS, GU, F8>), 32 * (FI), 64 * (FJ), ((XS) * 32 * (FI) + (WS) * 64 * (FJ)) * 128)
+#define TG_WIDE(FI, XS)                                  \
+    do {                                                 \
+        if (act) TG_HALVES(FI, 4, XS, 3, true, false);   \
+        else TG_HALVES(FI, 4, XS, 3, false, false);      \
     } while (0)
-#define TG_TURNS(FI, FJ, ST)                                                                                  \
-    do {                                                                                                      \
-        constexpr int lds = (ST) * 32 * ((FI) + (FJ)) * 128;                                                  \
-        if (f8) TG_LAUNCH((tile_gemm_turns_kernel<FI, FJ, ST, false, true>), 32 * (FI), 32 * (FJ), lds);      \
-        else if (act) TG_LAUNCH((tile_gemm_turns_kernel<FI, FJ, ST, true, false>), 32 * (FI), 32 * (FJ), lds); \
-        else TG_LAUNCH((tile_gemm_turns_kernel<FI, FJ, ST, false, false>), 32 * (FI), 32 * (FJ), lds);        \
+#define TG_TURNS(FI, FJ, ST)                                                                             \
+    do {                                                                                                 \
+        constexpr int lds = (ST) * 32 * ((FI) + (FJ)) * 128;                                             \
+        if (act) TG_LAUNCH((tile_gemm_turns_kernel<FI, FJ, ST, true>), 32 * (FI), 32 * (FJ), lds);       \
+        else TG_LAUNCH((tile_gemm_turns_kernel<FI, FJ, ST, false>), 32 * (FI), 32 * (FJ), lds);          \
     } while (0)
+    if (f8) {
+        switch (form) {
+            case 0: TG_HALVES(8, 4, 2, 3, false, true); break;
+            case 1: TG_HALVES(6, 4, 2, 3, false, true); break;
+            case 2: TG_HALVES(4, 4, 3, 3, false, true); break;
+            case 3: TG_HALVES(6, 2, 3, 4, false, true); break;
+            case 4: TG_HALVES(2, 2, 4, 4, false, true); break;
+            default: return -105;
+        }
+        HIP_CHECK_LAUNCH();
+        return 0;
+    }
     switch (form) {
-        case 0: TG_HALVES(8, 4, 2, 3); break;
-        case 1: TG_HALVES(7, 4, 2, 3); break;
-        case 2: TG_HALVES(6, 4, 2, 3); break;
-        case 3: TG_HALVES(5, 4, 3, 3); break;
+        case 0: TG_WIDE(8, 2); break;
+        case 1: TG_WIDE(7, 2); break;
+        case 2: TG_WIDE(6, 2); break;
+        case 3: TG_WIDE(5, 3); break;
         case 4: TG_TURNS(8, 4, 3); break;
         case 5: TG_TURNS(7, 4, 3); break;
         case 6: TG_TURNS(5, 4, 4); break;
@@ -497,6 +581,7 @@ static int tg_run(hipStream_t s, const void* x, int64_t xs, const void* w, const
         default: return -105;
     }
 #undef TG_TURNS
+#undef TG_WIDE
 #undef TG_HALVES
 #undef TG_LAUNCH
     HIP_CHECK_LAUNCH();
@@ -518,18 +603,13 @@ extern "C" int oa_tile_gemm(void* stream, const void* x, int64_t xs, const void*
     if (xs < K || xs >= (1 << 22) || ((int64_t)(act ? N : 0) + 256) * K * 2 >= ((int64_t)1 << 32)) return -103;
     const int rc = tg_run((hipStream_t)stream, x, xs * 2, w, nullptr, nullptr, out, splits > 1 ? scratch : nullptr,
                           M, N, (int64_t)K * 2, form, splits, act, false);
-    return rc || splits == 1 || !out ? rc : oa_ring_sum(stream, scratch, nullptr, nullptr, out, M, N, splits);
+    return rc || splits == 1 || !out ? rc : oa_ring_sum(stream, scratch, out, M, N, splits);
 }
 
-// out [M, N] = (x8 [M, K] w8 [N, K]^T) * xscale[m] * wscale[n], e4m3 rows; plan: oa_tile_gemm_fp8_plan's
+// out [M, N] = (x8 [M, K] w8 [N, K]^T) * xscale[m] * wscale[n], e4m3 rows; form: oa_tile_gemm_fp8_form's
 extern "C" int oa_tile_gemm_fp8(void* stream, const void* x8, const void* xscale, const void* w8,
-                                const void* wscale, void* out, void* scratch, int M, int N, int K, int plan) {
-    const int form = plan >> 8, splits = plan & 255;
+                                const void* wscale, void* out, int M, int N, int K, int form) {
     if (M < 1 || N < 8 || N % 8 != 0 || K < 128 || K % 128 != 0 || K >= (1 << 23)) return -100;
-    if (splits < 1 || splits > K / 128 || (splits > 1 && !scratch)) return -101;
-    if (((uintptr_t)x8 | (uintptr_t)w8 | (uintptr_t)out | (uintptr_t)scratch) % 16 != 0) return -102;
-    if (plan < 0) return -104;
-    const int rc = tg_run((hipStream_t)stream, x8, K, w8, xscale, wscale, out, splits > 1 ? scratch : nullptr, M,
-                          N, K, form, splits, 0, true);
-    return rc || splits == 1 ? rc : oa_ring_sum(stream, scratch, xscale, wscale, out, M, N, splits);
+    if (((uintptr_t)x8 | (uintptr_t)w8 | (uintptr_t)out) % 16 != 0) return -102;
+    return tg_run((hipStream_t)stream, x8, K, w8, xscale, wscale, out, nullptr, M, N, K, form, 1, 0, true);
 }
