@@ -168,19 +168,14 @@ class Attention(nn.Module):
         )
 
         if fb.kind == "prefill":
-            skv = fb.prefill_past_len + T
-            nb, bs, hk, hd = k_cache.shape
-            if fb.prefill_past_len > 0:
-                flat_k = k_cache.view(nb * bs, hk, hd)
-                flat_v = v_cache.view(nb * bs, hk, hd)
-                k_full = flat_k[fb.prefill_slot_gather].view(1, skv, hk, hd)
-                v_full = flat_v[fb.prefill_slot_gather].view(1, skv, hk, hd)
-            else:
-                k_full = k.unsqueeze(0)
-                v_full = v.unsqueeze(0)
+            # behind a past the keys come from the cache, this prompt's among them
+            past = fb.prefill_past_len > 0
             out = ops.attention_prefill(
-                q.unsqueeze(0), k_full, v_full, scale=self.scale,
-                steady=self.fp8 or self.fp8_experts,
+                q.unsqueeze(0),
+                k_cache.flatten(0, 1) if past else k.unsqueeze(0),
+                v_cache.flatten(0, 1) if past else v.unsqueeze(0),
+                scale=self.scale, steady=self.fp8 or self.fp8_experts,
+                slots=fb.prefill_slot_gather if past else None,
             )
             out = out.view(T, self.hq * self.hd)
         else:

@@ -43,7 +43,8 @@
 // Layouts: q [B, Sq, Hq, 128], k/v [B, Skv, Hk, 128] with per-token strides
 // (they may be head-slices of one fused qkv buffer), out [B, Sq, Hq, 128]
 // contiguous; causal offset = Skv - Sq (query i attends keys [0..Skv-Sq+i])
-// so multi-turn chunked prefill reuses the same kernel.
+// so multi-turn chunked prefill reuses the same kernel. With `slots` (int64 [Skv], one
+// sequence) key i is row slots[i] of k and v, the cache's rows as they lie.
 
 #include "common.h"
 
@@ -81,12 +82,12 @@ __device__ __forceinline__ float xor32_f32(float v, int lh) {
 // SPLIT: blockIdx.z takes a run of the q-tile's key tiles and leaves its unnormalised
 // float32 sums with their maximum (raw scores) and weight sum for
 // prefill_combine_kernel: few queries over many keys fill the chip this way.
-template <int KG, int GQ, bool SPLIT>
+template <int KG, int GQ, bool SPLIT, bool PAGED>
 __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, uint16_t* __restrict__ out, int B, int Hq,
     int Hk, int Sq, int Skv, float scale, int qs, int ks, int vs,
-    float* __restrict__ po, float* __restrict__ pml) {
+    float* __restrict__ po, float* __restrict__ pml, const int64_t* __restrict__ slots) {
     constexpr int KB = 128 / KG;             // keys of a group's tile: 128 of LDS' 160 KiB
     constexpr int QROWS = 32;                // per wave
     constexpr int NG = NWAVE / KG;           // waves of a key group
@@ -163,7 +164,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(
     // drain mid-compute. Persistent
     // operands pin the registers for the whole loop; the only inserted
     // waits land right after our own vmcnt(0), where they are free.
-    int k_byte[PIECES], v_byte[PIECES], kkey0[PIECES], vkey0[PIECES];
+    // a wave's pieces of V are channels of the same keys
+    int k_byte[PIECES], v_byte[PIECES], kkey0[PIECES], vkey0 = 0;
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
         const int c = wid * PIECES + p;
@@ -171,7 +173,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(
         kkey0[p] = kkey;
         k_byte[p] = ((lane & 15) * 16) ^ ((kkey & 15) << 4);
         const int kb2 = c >> 3, nb = c & 7;
-        vkey0[p] = kb2 * 32 + v_img_row_inv(lane >> 1);
+        vkey0 = kb2 * 32 + v_img_row_inv(lane >> 1);
         v_byte[p] = (nb * 16 + (lane & 1) * 8) * 2;
     }
     uint32_t m0k[2][PIECES], m0v[2][PIECES];
@@ -188,14 +190,24 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(
     const char* ksrc[PIECES];
     const char* vsrc[PIECES];
     uint32_t m0k_cur[PIECES], m0v_cur[PIECES];
-    auto set_tile = [&](int t, int buf) {
+    // PAGED: the rows of a tile are looked up a tile ahead of its transfers, straight-line and
+    // as loaded, so that the only wait for them is the drain
+    int krow[PIECES], vrow = 0;
+    auto find_rows = [&](int t) {
         const int kv0 = t * KB;
+        auto row = [&](int key) {
+            const int at = min(kv0 + key, skv_clamp);
+            return PAGED ? reinterpret_cast<const int*>(slots)[2 * at] : at;
+        };
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) krow[p] = row(kkey0[p]);
+        vrow = row(vkey0);
+    };
+    auto set_tile = [&](int buf) {
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
-            ksrc[p] = kbase + (size_t)min(kv0 + kkey0[p], skv_clamp) * ks * 2 +
-                      k_byte[p];
-            vsrc[p] = vbase + (size_t)min(kv0 + vkey0[p], skv_clamp) * vs * 2 +
-                      v_byte[p];
+            ksrc[p] = kbase + (size_t)krow[p] * ks * 2 + k_byte[p];
+            vsrc[p] = vbase + (size_t)vrow * vs * 2 + v_byte[p];
             m0k_cur[p] = m0k[buf][p];
             m0v_cur[p] = m0v[buf][p];
         }
@@ -357,8 +369,10 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(
 
     const int first = tile0 + gid;
     if (first < ntiles) {
-        set_tile(first, 0);
+        find_rows(first);
+        set_tile(0);
         stage();
+        if (PAGED) find_rows(first + KG);
     }
     // static priority for the second half of the waves: the younger 4 lose VALU
     // arbitration on every segment otherwise. The readfirstlane keeps the condition
@@ -371,8 +385,12 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(
     int cur = 0;
     for (int t = first; t - gid < ntiles; t += KG, cur ^= 1) {
         const int kv0 = t * KB;
-        if (t + KG < ntiles) set_tile(t + KG, cur ^ 1);
-        if (t + KG < ntiles) stage();
+        if (t + KG < ntiles) {
+            if (!PAGED) find_rows(t + KG);
+            set_tile(cur ^ 1);
+            stage();
+            if (PAGED) find_rows(t + 2 * KG);
+        }
         if (t < ntiles && kv0 < wave_kv_last) {  // wave-uniform: skip past-diagonal tiles
             // fully-unmasked tile: every key <= every lane's diagonal
             const bool need_mask =
@@ -475,12 +493,12 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(
 // models keep the form and the splits that they had, whatever is the fastest. Waves of
 // 16 rows on 16x16x32 products; P goes through LDS to become an operand. A tile takes 5 us,
 // its LDS reads (512 KB for 128 rows) the most of it.
-template <bool SPLIT>
+template <bool SPLIT, bool PAGED>
 __global__ __launch_bounds__(512, 1) void attn_prefill_steady_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, uint16_t* __restrict__ out, int B, int Hq,
     int Hk, int Sq, int Skv, float scale, int qs, int ks, int vs,
-    float* __restrict__ po, float* __restrict__ pml) {
+    float* __restrict__ po, float* __restrict__ pml, const int64_t* __restrict__ slots) {
     constexpr int KB = 128, QROWS = 16;
     constexpr int QTILE = QROWS * NWAVE;
     constexpr int P_BYTES = QROWS * KB * 2;
@@ -546,7 +564,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_steady_kernel(
 
     // transfers as in attn_prefill_kernel
     // per-piece invariants
-    int k_byte[PIECES], v_byte[PIECES], kkey0[PIECES], vkey0[PIECES];
+    // a wave's pieces of V are channels of the same keys
+    int k_byte[PIECES], v_byte[PIECES], kkey0[PIECES], vkey0 = 0;
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
         const int c = wid * PIECES + p;
@@ -554,7 +573,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_steady_kernel(
         kkey0[p] = kkey;
         k_byte[p] = ((lane & 15) * 16) ^ ((kkey & 15) << 4);
         const int kb2 = c >> 3, nb = c & 7;
-        vkey0[p] = kb2 * 32 + v_img_row_inv(lane >> 1);
+        vkey0 = kb2 * 32 + v_img_row_inv(lane >> 1);
         v_byte[p] = (nb * 16 + (lane & 1) * 8) * 2;
     }
     // LDS destinations (uniform per wave): [buf][piece] for K and V
@@ -573,14 +592,24 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_steady_kernel(
     const char* ksrc[PIECES];
     const char* vsrc[PIECES];
     uint32_t m0k_cur[PIECES], m0v_cur[PIECES];
-    auto set_tile = [&](int t, int buf) {
+    // PAGED: the rows of a tile are looked up a tile ahead of its transfers, straight-line and
+    // as loaded, so that the only wait for them is the drain
+    int krow[PIECES], vrow = 0;
+    auto find_rows = [&](int t) {
         const int kv0 = t * KB;
+        auto row = [&](int key) {
+            const int at = min(kv0 + key, skv_clamp);
+            return PAGED ? reinterpret_cast<const int*>(slots)[2 * at] : at;
+        };
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) krow[p] = row(kkey0[p]);
+        vrow = row(vkey0);
+    };
+    auto set_tile = [&](int buf) {
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
-            ksrc[p] = kbase + (size_t)min(kv0 + kkey0[p], skv_clamp) * ks * 2 +
-                      k_byte[p];
-            vsrc[p] = vbase + (size_t)min(kv0 + vkey0[p], skv_clamp) * vs * 2 +
-                      v_byte[p];
+            ksrc[p] = kbase + (size_t)krow[p] * ks * 2 + k_byte[p];
+            vsrc[p] = vbase + (size_t)vrow * vs * 2 + v_byte[p];
             m0k_cur[p] = m0k[buf][p];
             m0v_cur[p] = m0v[buf][p];
         }
@@ -720,8 +749,10 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_steady_kernel(
                      : "memory");
     };
     if (ntiles > tile0) {
-        set_tile(tile0, 0);
+        find_rows(tile0);
+        set_tile(0);
         stage();
+        if (PAGED) find_rows(tile0 + 1);
     }
     if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256)
         __builtin_amdgcn_s_setprio(1);
@@ -729,8 +760,12 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_steady_kernel(
     __syncthreads();
     for (int t = tile0; t < ntiles; ++t) {
         const int cur = (t - tile0) & 1;
-        if (t + 1 < ntiles) set_tile(t + 1, cur ^ 1);
-        if (t + 1 < ntiles) stage();
+        if (t + 1 < ntiles) {
+            if (!PAGED) find_rows(t + 1);
+            set_tile(cur ^ 1);
+            stage();
+            if (PAGED) find_rows(t + 2);
+        }
         compute(t, smem + cur * KBYTES, smem + voff + cur * KBYTES);
         drain();          // tile t+1 has landed
         __syncthreads();  // all waves' reads of buf[cur] complete
@@ -811,25 +846,34 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const float* __res
 // block per key head and 256 / (Hq / Hk) queries (Hq / Hk of 2, 4 or 8); 2, the steady form.
 // po [nsplit, B, Sq, Hq, 128] and pml [nsplit, B, Sq, Hq, 2]: float32 scratch.
 #define LAUNCH_PREFILL(KG, GQ, SPLIT, NSPLIT)                                                      \
-    LAUNCH_BLOCKS((attn_prefill_kernel<KG, GQ, SPLIT>), 256 / (KG) / (GQ), B * (Hq / (GQ)), NSPLIT)
+    do {                                                                                           \
+        if (slots) LAUNCH_BLOCKS((attn_prefill_kernel<KG, GQ, SPLIT, true>), 256 / (KG) / (GQ), B * (Hq / (GQ)), NSPLIT); \
+        else LAUNCH_BLOCKS((attn_prefill_kernel<KG, GQ, SPLIT, false>), 256 / (KG) / (GQ), B * (Hq / (GQ)), NSPLIT); \
+    } while (0)
+#define LAUNCH_STEADY(SPLIT, NSPLIT)                                                               \
+    do {                                                                                           \
+        if (slots) LAUNCH_BLOCKS((attn_prefill_steady_kernel<SPLIT, true>), 128, B * Hq, NSPLIT);  \
+        else LAUNCH_BLOCKS((attn_prefill_steady_kernel<SPLIT, false>), 128, B * Hq, NSPLIT);       \
+    } while (0)
 #define LAUNCH_BLOCKS(KERN, ROWS, HEADS, NSPLIT)                                                   \
-    hipLaunchKernelGGL((KERN), dim3(CEIL_DIV(Sq, ROWS) * (HEADS), 1, NSPLIT),                      \
+    hipLaunchKernelGGL(KERN, dim3(CEIL_DIV(Sq, ROWS) * (HEADS), 1, NSPLIT),                        \
                        dim3(512), 0, (hipStream_t)stream, (const uint16_t*)q, (const uint16_t*)k,  \
                        (const uint16_t*)v, (uint16_t*)out, B, Hq, Hk, Sq, Skv, scale, q_stride,    \
-                       k_stride, v_stride, (float*)po, (float*)pml)
+                       k_stride, v_stride, (float*)po, (float*)pml, (const int64_t*)slots)
 
 extern "C" int oa_attention_prefill_split(
     void* stream, const void* q, const void* k, const void* v, void* out, void* po, void* pml,
     int B, int Hq, int Hk, int Sq, int Skv, int D, float scale, int q_stride, int k_stride,
-    int v_stride, int nsplit, int merged) {
+    int v_stride, int nsplit, int merged, const void* slots) {
     if (D != DHEAD) return -100;
     if (Hk < 1 || Hq % Hk != 0) return -101;
     if ((q_stride | k_stride | v_stride) % 8 != 0) return -102;
+    if (slots && B != 1) return -106;
     if (nsplit < 1 || nsplit > 65535 || (int64_t)B * Sq * Hq > (1 << 30)) return -105;
     const int gq = Hq / Hk, rows = B * Sq * Hq;
     if (rows < 1) return 0;
     if (merged == 2) {
-        LAUNCH_BLOCKS(attn_prefill_steady_kernel<true>, 128, B * Hq, nsplit);
+        LAUNCH_STEADY(true, nsplit);
     }
     else if (!merged) {
         if (Sq <= 64) LAUNCH_PREFILL(4, 1, true, nsplit);
@@ -850,15 +894,16 @@ extern "C" int oa_attention_prefill_split(
 extern "C" int oa_attention_prefill_variant(
     void* stream, const void* q, const void* k, const void* v, void* out,
     int B, int Hq, int Hk, int Sq, int Skv, int D, float scale,
-    int q_stride, int k_stride, int v_stride, int variant) {
+    int q_stride, int k_stride, int v_stride, int variant, const void* slots) {
     if (D != DHEAD) return -100;
     if (Hq % Hk != 0) return -101;
     if ((q_stride | k_stride | v_stride) % 8 != 0) return -102;
+    if (slots && B != 1) return -106;
     float* const po = nullptr;
     float* const pml = nullptr;
     switch (variant) {
         case 1: case 3: case 5: case 7:  // the steady form, 128 rows
-            LAUNCH_BLOCKS(attn_prefill_steady_kernel<false>, 128, B * Hq, 1);
+            LAUNCH_STEADY(false, 1);
             break;
         case 10:  // two key groups, 128 rows
             LAUNCH_PREFILL(2, 1, false, 1);
@@ -903,7 +948,8 @@ static float prefill_us(int kg, int B, int Hq, int Sq, int Skv) {
 extern "C" int oa_attention_prefill(void* stream, const void* q, const void* k,
                                     const void* v, void* out, int B, int Hq,
                                     int Hk, int Sq, int Skv, int D, float scale,
-                                    int q_stride, int k_stride, int v_stride, int steady) {
+                                    int q_stride, int k_stride, int v_stride, int steady,
+                                    const void* slots) {
     // OPSAGENT_PREFILL_VARIANT forces a variant (read per call so one
     // process can A/B all variants).
     const char* e = getenv("OPSAGENT_PREFILL_VARIANT");
@@ -921,5 +967,5 @@ extern "C" int oa_attention_prefill(void* stream, const void* q, const void* k,
     }
     return oa_attention_prefill_variant(stream, q, k, v, out, B, Hq, Hk, Sq,
                                         Skv, D, scale, q_stride, k_stride,
-                                        v_stride, variant);
+                                        v_stride, variant, slots);
 }

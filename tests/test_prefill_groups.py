@@ -58,6 +58,34 @@ def test_steady(Hq, Hk, Sq, Skv):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("variant", [7, 8, 9, 10, 11, 0])
+@pytest.mark.parametrize("steady", [False, True])
+@pytest.mark.parametrize("Hq,Hk,Sq,Skv", [(8, 2, 1, 1), (8, 4, 33, 129), (16, 2, 200, 257),
+                                          (8, 2, 70, 900), (8, 2, 300, 1700)])
+def test_cache_rows(monkeypatch, variant, steady, Hq, Hk, Sq, Skv):
+    """Keys and values read from the cache's rows, split and not: bit for bit the results of
+    gathered ones."""
+    if variant:
+        monkeypatch.setenv("OPSAGENT_PREFILL_VARIANT", str(variant))
+    gen = torch.Generator(device="cuda").manual_seed(Sq + Skv)
+    q, k, v = (torch.randn(n, h, D, generator=gen, device="cuda").bfloat16()
+               for n, h in ((Sq, Hq), (Skv + 40, Hk), (Skv + 40, Hk)))
+    slots = torch.randperm(Skv + 40, generator=gen, device="cuda")[:Skv].contiguous()
+    want = ops.attention_prefill(q[None], k[slots][None], v[slots][None], steady=steady)
+    assert torch.equal(ops.attention_prefill(q[None], k, v, steady=steady, slots=slots), want)
+    apart = torch.stack([slots, slots], 1)[:, 0]         # rows that are not side by side
+    assert torch.equal(ops.attention_prefill(q[None], k, v, steady=steady, slots=apart), want)
+
+
+def test_cache_rows_on_the_host():
+    gen = torch.Generator().manual_seed(0)
+    q, k, v = (torch.randn(n, 2, 16, generator=gen) for n in (5, 20, 20))
+    slots = torch.randperm(20, generator=gen)[:9]
+    assert torch.equal(ops.attention_prefill(q[None], k, v, slots=slots),
+                       ops.attention_prefill(q[None], k[slots][None], v[slots][None]))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("variant", [10, 11])
 def test_scores_that_do_not_compare(monkeypatch, variant):
     """A row with a NaN or a positive infinite score is NaN in whichever group the score lies,
