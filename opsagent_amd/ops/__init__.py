@@ -348,6 +348,71 @@ def _ring_choice(M: int, N: int, K: int, gateup: bool = False):
     return _ring_sizes(M, N, K, gateup)
 
 
+# us of a step of 64 columns where a block is alone on its CU's part of the chip, of starting and
+# ending a round, and the share of the first that is left where few blocks run; by rows of a
+# tile and whether strips are of 64 weight rows
+_RING_STEPS = {(32, False): (0.443, 1.5, 0.85), (32, True): (0.306, 1.3, 0.69),
+               (64, False): (0.472, 1.9, 0.86), (64, True): (0.527, 2.5, 0.20),
+               (96, False): (0.688, 2.0, 0.72), (128, False): (0.754, 1.5, 0.77)}
+
+
+def _ring_us(M: int, N: int, K: int, gateup: bool, tile: int, splits: int, narrow: bool) -> float:
+    """The ring product's time by rounds of its blocks: a step takes what a CU needs for it or
+    what memory needs for all of them (6.46 TB/s; where some CUs have two blocks and others one,
+    partly for two each), splits 2.3 us and their sums on top. Least squares over 7600 times of
+    130 weights at 3 to 128 rows, 6% rms."""
+    step, ends, few = _RING_STEPS[tile, narrow]
+    slots, rows, mtiles = 512 if narrow else 256, N * (1 + gateup), -(-M // tile)
+    height = 64 if narrow else 128
+    rounds, rest = divmod(-(-rows // height) * mtiles * splits, slots)
+    steps, us = K / 64 / splits, 2.0
+    for blocks, times in ((slots, rounds), (rest, int(rest > 0))):
+        busy = blocks / slots if not narrow else 1.0 if blocks > 256 else 0.5
+        full = blocks + 0.3 * (512 - blocks) if narrow and blocks > 256 else blocks
+        read = height * 128 / mtiles * full / 6.46e6
+        us += times * (steps * max(step * (few + (1 - few) * busy), read) + ends)
+    if splits == 1:
+        return us * 1.08 if tile == 64 and narrow else us
+    return us + 2.3 + splits * M * rows * 1.7e-6
+
+
+@functools.lru_cache(maxsize=4096)
+def _ring_fastest(M: int, N: int, K: int, gateup: bool):
+    if K % 64 or K < 256 or N % 8:
+        return None
+    forms = []
+    for tile, narrow in {(32 * -(-M // 32), False), (64, False), (32 * -(-M // 32), True)}:
+        if tile > 32 * -(-M // 32) or narrow and tile > 64:
+            continue
+        tiles = -(-N // ((64 if gateup else 128) // (1 + narrow))) * -(-M // tile)
+        for splits in {1, 256 // tiles, 256 // tiles * 2, 512 // tiles if narrow else 1}:
+            if 1 <= splits <= min(16, K // 256) and (splits == 1 or tiles * splits <= 520):
+                forms.append((_ring_us(M, N, K, gateup, tile, splits, narrow), tile, splits, narrow))
+    us, *form = min(forms)
+    plan = _ring_choice(M, N, K, gateup)
+    if plan:
+        return tuple(form) if us < 0.97 * _ring_us(M, N, K, gateup, *plan) else plan
+    stream = N * (1 + gateup) * K * 2 / 6.2e6 + 3.0
+    near = 1.3 if M > 32 and not form[2] else 1.2
+    return tuple(form) if K >= (1536 if M <= 16 else 1024) and us < near * stream else None
+
+
+def _ring_form(M: int, N: int, K: int, gateup: bool = False):
+    """The ring's form that the products take, laid out as _ring_choice's answer.
+
+    Those lines were drawn where all blocks read the same columns at a time; since strips start at
+    steps of their own (ring_gemm.hip) the wide forms run up to a quarter faster, and an
+    estimate finds the form: over 130 weights at 3 to 128 rows, 105 of them drawn, 0.957 of the
+    time of _ring_choice's, 1.035 of the best form's, 1.11 of _ring_choice's at the most. Its form
+    is taken where it is 3 per cent ahead of that one's by the same estimate, and where that is
+    none, if it comes within 1.2 (above 32 rows, where those are slower, 1.3) of reading the
+    weights at 6.2 TB/s; skinny.hip is the better one for up to 16 short rows (2 x 25088 x 1024, 3
+    19.8 / 22.5). us, _ring_choice's form or the others / here: gate-up 2 x 14336 x 4096, M = 47 44.2
+    / 38.1, 128 58.3 / 48.2; 32000 x 4096, 47 48.5 / 41.5, 112 76.6 / 51.8; 20288 x 1664, 16 41.5 /
+    15.2; 12584 x 3520, 40 32.7 / 21.6; but 2 x 5632 x 2048, 48 14.2 / 15.7."""
+    return _ring_choice(M, N, K, gateup) if M == 2 else _ring_fastest(M, N, K, gateup)
+
+
 def _ring(x: torch.Tensor, w: torch.Tensor, plan: Tuple[int, ...], act: int = 0,
           parts: bool = False) -> torch.Tensor:
     """x @ w^T, or act 1 (silu), 2 (tanh gelu) of the gate rows times the up rows. plan: (rows
@@ -418,7 +483,7 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor) -> Union[torch.Tensor, PlaneS
         if M > 128:
             tile = _tile_choice(M, w.shape[0], w.shape[1], summed=True)
             return PlaneSum(_tile(x, w, tile, parts=True)) if tile and tile & 255 > 1 else linear(x, w)
-        plan = _ring_choice(M, w.shape[0], w.shape[1])
+        plan = _ring_form(M, w.shape[0], w.shape[1])
         if plan and plan[1] > 1:
             return PlaneSum(_ring(x, w, plan, parts=True))
     return linear(x, w)
@@ -428,12 +493,12 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear with custom HIP paths for decode shapes: the VALU GEMV at M = 1
     (hipBLASLt's M=1 kernels run ~2.5x off the HBM roofline on gfx950), the transfer
     ring up to 128 rows and the skinny matrix-core products up to 32 where they win
-    (_ring_choice, _skinny_form), the VALU GEMV for what two rows are left and the
+    (_ring_form, _skinny_form), the VALU GEMV for what two rows are left and the
     matrix-core GEMV for what 3 to 8 are, the tile product for more than 128 (_tile_choice);
     everything else goes to hipBLASLt."""
     M = x.numel() // x.shape[-1]
     if 1 < M <= 128 and _skinny_ok(x, w):
-        plan = _ring_choice(M, w.shape[0], w.shape[1])
+        plan = _ring_form(M, w.shape[0], w.shape[1])
         if plan:
             return _ring(x, w, plan)
         form = _skinny_form(M, w.shape[0], w.shape[1], strided=not x.is_contiguous())
@@ -1198,7 +1263,7 @@ def _gateup_form(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int):
         plan = _tile_choice(M, i_local, K, gateup=True)
         return None if plan is None else ("tile", plan)
     if 1 < M <= 128 and _skinny_ok(x, gate_up_w) and gate_up_w.shape[0] == 2 * i_local:
-        plan = _ring_choice(M, i_local, K, gateup=True)
+        plan = _ring_form(M, i_local, K, gateup=True)
         if plan:
             return "ring", plan
         form = _skinny_form(M, i_local, K, gateup=True)

@@ -11,6 +11,14 @@
 // M = 32 57.8 / 48.5, 77 56.3 / 53.7; 8192 x 28672, M = 8 89.3 / 75.4, 47 140 / 81.0, 77
 // 194 / 88.9. (The same over 0.5 GB reads up to a fifth better than inside a model.)
 //
+// Rows lie a few KiB apart, so blocks at the same columns read the same few memory channels, and
+// all blocks start together. In bf16 each eight strips therefore start two steps further into
+// their columns and go round. Us, together / apart: gate-up 2 x 14336 x 4096 in strips of 128, M =
+// 8 46.6 / 36.6, 47 47.3 / 37.6 (6.2 TB/s), 77 49.9 / 41.6, 128 52.7 / 48.2; 32000 x 4096, 47 55.5 /
+// 41.5, 77 57.4 / 43.8; in strips of 64, which had spread the starts some, M = 8 40.3 / 37.7 and 44.2
+// / 40.8; 4096 x 14336 in seven splits, 47 32.0 / 30.4; 2 x 8192 x 2048, 8 15.3 / 13.3. Other steps
+// between them were as good but one a strip (47.3); sixteen neighbours together too.
+//
 // Up to 64 rows a strip of 64 weight rows leaves LDS for two blocks a CU, whose rings keep
 // more under way than one deep ring and start and end at different times; one strip more
 // than fills the CUs no longer waits for a whole round either. Us, strips of 128 (or the
@@ -89,6 +97,13 @@ __global__ __launch_bounds__(256 * RG_MG(BM, RN), RG_MG(BM, RN) == 2 || RN == 64
     const int steps = (int)(kb / 128);
     const int s0 = (int)((int64_t)steps * sp / splits), s1 = (int)((int64_t)steps * (sp + 1) / splits);
 
+    const int n = s1 - s0;
+    // Strips start at steps of their own: rows lie some KiB apart, and blocks that all read the
+    // same columns read the same few memory channels. Eight neighbours share a start. fp8 keeps
+    // the order of its sums.
+    const int turned = F8 ? 0 : (strip >> 3) * 2 % n;
+    int ahead = n - turned;                          // steps to the last column
+
     // a transfer takes eight rows; this lane's row of it and its chunk
     const int lr = lane >> 3;
     const char* src[LPS];
@@ -104,7 +119,7 @@ __global__ __launch_bounds__(256 * RG_MG(BM, RN), RG_MG(BM, RN) == 2 || RN == 64
         else if (GU && NF == 2) at = (min(strip * 64 + (r >> 5) * 16 + (r & 15), N - 1) + (r & 16 ? N : 0)) * kb;
         else if (GU) at = (min(strip * 32 + (r >> 2) * 2 + (r & 1), N - 1) + (r & 2 ? N : 0)) * kb;
         else at = min(strip * RN + r, N - 1) * kb;
-        src[p] = (isw ? w : x) + at + (int64_t)s0 * 128 + chunk * 16;
+        src[p] = (isw ? w : x) + at + (int64_t)(s0 + turned) * 128 + chunk * 16;
         dst[p] = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + tr * 1024);
     }
     auto stage = [&](int buf) {
@@ -114,6 +129,10 @@ __global__ __launch_bounds__(256 * RG_MG(BM, RN), RG_MG(BM, RN) == 2 || RN == 64
             if (NT && p * W + wave < RN / 8) lds_transfer16<true>(dst[p] + buf * STEP, src[p]);
             else lds_transfer16(dst[p] + buf * STEP, src[p]);
             src[p] += 128;
+        }
+        if (!F8 && --ahead == 0) {
+#pragma unroll
+            for (int p = 0; p < LPS; ++p) src[p] -= (int64_t)n * 128;
         }
     };
     auto wait = [&](auto count, int behind) {         // count: transfers of a step of this wave
@@ -125,7 +144,6 @@ __global__ __launch_bounds__(256 * RG_MG(BM, RN), RG_MG(BM, RN) == 2 || RN == 64
         else rg_wait<0>();
     };
     rgf4 acc[NF][MT] = {};
-    const int n = s1 - s0;
 #pragma unroll
     for (int t = 0; t < STAGES - 1; ++t)
         if (t < n) stage(t);
