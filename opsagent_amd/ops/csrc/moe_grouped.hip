@@ -261,6 +261,9 @@ __device__ __forceinline__ void mg_wait() {
 // 64 tokens 142 + 76 / 118 + 58, 512 tokens 201 + 111 / 134 + 72, 2048 tokens 317 + 192 /
 // 233 + 158. The stream runs at 5.5 to 6.3 TB/s up to 6 rows an expert. One block a CU with
 // six steps is slower (54 + 28 for 13 fp8 tokens), three with two are as fast (51 + 24).
+// Strips that start apart, us, together / apart: 64 experts of 1408 x 2048, bf16: 13 tokens 94 +
+// 45 / 91 + 45, 512 tokens 135 + 75 / 130 + 74, fp8 1500 tokens 193 + 106 / 167 + 104; 8 experts of
+// 14336 x 4096, top 2, bf16: 13 tokens 292 + 164 / 276 + 139, 512 tokens 586 + 328 / 541 + 319.
 template <int BM, int STAGES, bool FP8, int MODE>
 __global__ __launch_bounds__(256, 2) void moe_grouped_kernel(
     const uint16_t* __restrict__ x, const char* __restrict__ w, const float* __restrict__ wscale,
@@ -288,6 +291,13 @@ __global__ __launch_bounds__(256, 2) void moe_grouped_kernel(
     const int64_t rb = FP8 ? (int64_t)K : 2 * (int64_t)K;    // bytes of a weight row
     const int ns = (int)(rb / 128);
 
+    // Strips start at steps of their own, the row tiles of one together: rows a few KiB apart
+    // lie on the same memory channels, and blocks that read the same columns share those. Narrow
+    // fp8 tiles lose more by it (64 x 1408 x 2048, 13 tokens 47.5 us, 48.2) than they win.
+    constexpr bool TURN = !FP8 || BM >= 64;
+    const int turned = TURN ? (e * strips + strip) * 3 % ns : 0;
+    int ahead = ns - turned;                         // steps to the last column
+
     // this lane's row and chunk of every transfer; weight rows past N repeat the last one,
     // rows past the end of the expert's too
     const char* src[LPS];
@@ -300,7 +310,7 @@ __global__ __launch_bounds__(256, 2) void moe_grouped_kernel(
         int64_t at;
         if (MODE == 1) at = min(strip * 64 + (row >> 5) * 16 + (row & 15), N - 1) + (row & 16 ? N : 0);
         else at = min(strip * 128 + row, N - 1);
-        src[p] = we + at * rb + ((lane & 7) ^ (row >> 1 & 7)) * 16;
+        src[p] = we + at * rb + turned * 128 + ((lane & 7) ^ (row >> 1 & 7)) * 16;
         dst[p] = base + (wid * 4 + p) * 1024;
     }
 #pragma unroll
@@ -310,7 +320,7 @@ __global__ __launch_bounds__(256, 2) void moe_grouped_kernel(
         const int chunk = FP8 ? (lane & 15) ^ (row & 15) : (lane & 7) ^ (row >> 1 & 7);
         const int s = s0 + min(row, m - 1);
         src[4 + p] = reinterpret_cast<const char*>(x) +
-                     (int64_t)(MODE == 0 ? s : perm[s] / top) * K * 2 + chunk * 16;
+                     (int64_t)(MODE == 0 ? s : perm[s] / top) * K * 2 + turned * XB + chunk * 16;
         dst[4 + p] = base + 128 * 128 + tr * 1024;
     }
     auto stage = [&](int buf) {
@@ -319,6 +329,10 @@ __global__ __launch_bounds__(256, 2) void moe_grouped_kernel(
             if (p < 4 && mt == 1) lds_transfer16<true>(dst[p] + buf * STEP, src[p]);
             else lds_transfer16(dst[p] + buf * STEP, src[p]);
             src[p] += p < 4 ? 128 : XB;
+        }
+        if (TURN && --ahead == 0) {
+#pragma unroll
+            for (int p = 0; p < LPS; ++p) src[p] -= ns * (p < 4 ? 128 : XB);
         }
     };
 
