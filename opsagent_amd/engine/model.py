@@ -120,7 +120,6 @@ class Attention(nn.Module):
         )
         self.o_w = nn.Parameter(_shard(o_w, 1, rank, tp), requires_grad=False)
         self.fp8 = False  # set by LlamaForCausalLM.quantize_fp8_
-        self.fp8_experts = spec.moe_dtype == "fp8"
 
     def _qkv(self, x: torch.Tensor) -> torch.Tensor:
         if self.fp8:
@@ -174,7 +173,7 @@ class Attention(nn.Module):
                 q.unsqueeze(0),
                 k_cache.flatten(0, 1) if past else k.unsqueeze(0),
                 v_cache.flatten(0, 1) if past else v.unsqueeze(0),
-                scale=self.scale, steady=self.fp8 or self.fp8_experts,
+                scale=self.scale, steady=self.fp8,
                 slots=fb.prefill_slot_gather if past else None,
             )
             out = out.view(T, self.hq * self.hd)

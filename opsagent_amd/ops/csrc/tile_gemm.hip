@@ -119,6 +119,15 @@ __device__ __forceinline__ void tg_multiply(tgf16 (&acc)[FI][FJ], const TgFrag8 
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// The step of its columns that a strip of weight rows starts at, to go round them: rows a few KiB apart
+// lie on the same memory channels, and blocks that read the same columns share those. Few rows of x
+// wait for it, us together / apart: gate-up 2 x 14336 x 4096, M = 130 61 / 57, 200 69 / 65, 333 81 / 78;
+// 32000 x 4096, 130 63 / 52, 200 68 / 61; 4096 x 4096, 130 19.8 / 17.2. More tiles of rows are bound by other
+// things, and what they share of x is read again by strips apart (2048 x 8192, 2000 69 / 74).
+__device__ __forceinline__ int tg_turned(int strip, int steps, int mtiles) {
+    return mtiles > 2 ? 0 : (strip >> 1) * 3 % steps;
+}
+
 template <int V>
 __device__ __forceinline__ void tg_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(V) : "memory");
@@ -266,9 +275,11 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
     const int s0 = (int)((int64_t)steps * sp / splits), s1 = (int)((int64_t)steps * (sp + 1) / splits);
     const int n = s1 - s0;
 
+    const int turned = F8 ? 0 : tg_turned(strip, n, mtiles);
+    int ahead = n - turned;                          // steps to the last column
     // transfers of eight rows: group 0 those of x, group 1 those of w
-    const char* base = grp ? w + (int64_t)n0 * kb + (int64_t)s0 * 128
-                           : x + (int64_t)m0 * xs + (int64_t)s0 * 128;
+    const char* base = grp ? w + (int64_t)n0 * kb + (int64_t)(s0 + turned) * 128
+                           : x + (int64_t)m0 * xs + (int64_t)(s0 + turned) * 128;
     uint32_t off[LP];
 #pragma unroll
     for (int p = 0; p < LP; ++p) {
@@ -282,11 +293,13 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_kernel(
 #pragma unroll
         for (int p = 0; p < FI; ++p) lds_transfer16(lds0 + buf * XB + p * 4096, off[p], base);
         base += 128;
+        if (!F8 && --ahead == 0) base -= (int64_t)n * 128;
     };
     auto stage_w = [&](int buf) {
 #pragma unroll
         for (int p = 0; p < 2 * FJ; ++p) lds_transfer16(lds0 + buf * WB + p * 4096, off[p], base);
         base += 128;
+        if (!F8 && --ahead == 0) base -= (int64_t)n * 128;
     };
     // this wave's transfers of the step that `behind` younger ones follow
     auto landed_x = [&](int behind) {
@@ -381,9 +394,11 @@ __global__ __launch_bounds__(512, 2) void tile_gemm_turns_kernel(
         else off[p] = (uint32_t)(min(tg_wrow<FJ, GU>(r), N - 1 - n0) + (tg_isup<FJ, GU>(r) ? N : 0)) * (uint32_t)kb + chunk;
     }
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + wid * 1024);
+    const int turned = tg_turned(strip, n, mtiles);
     auto stage = [&](int step, int buf) {
-        const char* xt = xb + (int64_t)step * 128;
-        const char* wt = wb + (int64_t)step * 128;
+        const int at = step + turned < n ? step + turned : step + turned - n;
+        const char* xt = xb + (int64_t)at * 128;
+        const char* wt = wb + (int64_t)at * 128;
 #pragma unroll
         for (int p = 0; p < LP; ++p) lds_transfer16(lds0 + buf * STEP + p * 4096, off[p], p < FI ? xt : wt);
     };
