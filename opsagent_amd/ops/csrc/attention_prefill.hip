@@ -76,6 +76,24 @@ __device__ __forceinline__ float xor32_f32(float v, int lh) {
     return __uint_as_float(lh ? r[0] : r[1]);
 }
 
+// PAGED: the blocks of a key head, which share an XCD's L2, ask for up to four lines a lane of
+// all its keys and values while the first tile is under way: cache rows come from memory, and a
+// step of 1 to 2 us is less than its latency. `me` of `sharers` blocks; the caller waits. Four
+// layers of a model, us, gathered / from the cache / so: 1500 tokens behind 3000, 16 heads on
+// 4, 1222 / 1300 / 1242, 600 behind 1800, 32 on 8, 1430 / 1458 / 1426.
+constexpr int TOUCHES = 4;
+__device__ __forceinline__ void touch_rows(uint32_t (&t)[TOUCHES], const char* kbase, const char* vbase,
+                                           const int64_t* slots, int64_t kstep, int64_t vstep,
+                                           int key0, int key1, int me, int sharers) {
+#pragma unroll
+    for (int i = 0; i < TOUCHES; ++i) {
+        const int line = min((i * sharers + me) * 512 + (int)threadIdx.x, 4 * (key1 - key0) - 1);
+        const int row = reinterpret_cast<const int*>(slots)[2 * (key0 + (line >> 2))];
+        const char* at = line & 2 ? vbase + row * vstep : kbase + row * kstep;
+        t[i] = *reinterpret_cast<const uint32_t*>(at + (line & 1) * 128);
+    }
+}
+
 // GQ > 1: the workgroup carries GQ q-heads that SHARE one KV head
 // (requires Hq/Hk == GQ): waves split into GQ sets, each owning QTILE/GQ q-rows of its head,
 // and every staged K/V tile feeds all of them (2 to 4 per cent over a block per head).
@@ -374,12 +392,20 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(
         stage();
         if (PAGED) find_rows(first + KG);
     }
+    const bool far = PAGED && ntiles - tile0 > 3 * KG;
+    uint32_t touched[TOUCHES];
+    if (far) {
+        const int part = SPLIT ? CEIL_DIV(Skv, (int)gridDim.z) : Skv, key0 = SPLIT ? (int)blockIdx.z * part : 0;
+        touch_rows(touched, kbase, vbase, slots, (int64_t)ks * 2, (int64_t)vs * 2, min(key0, Skv - 1),
+                   min(key0 + part, Skv), turn * groups + place / pairs, CEIL_DIV(Sq, QTILE_H) * groups);
+    }
     // static priority for the second half of the waves: the younger 4 lose VALU
     // arbitration on every segment otherwise. The readfirstlane keeps the condition
     // provably wave-uniform (exec-masking is ignored by s_setprio).
     if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256)
         __builtin_amdgcn_s_setprio(1);
     drain();
+    if (far) asm volatile("" : : "v"(touched[0]), "v"(touched[1]), "v"(touched[2]), "v"(touched[3]));
     __syncthreads();
     // every group takes as many steps as the first, which may have one tile more
     int cur = 0;
@@ -754,9 +780,17 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_steady_kernel(
         stage();
         if (PAGED) find_rows(tile0 + 1);
     }
+    const bool far = PAGED && ntiles - tile0 > 3;
+    uint32_t touched[TOUCHES];
+    if (far) {
+        const int part = SPLIT ? CEIL_DIV(Skv, (int)gridDim.z) : Skv, key0 = SPLIT ? (int)blockIdx.z * part : 0;
+        touch_rows(touched, kbase, vbase, slots, (int64_t)ks * 2, (int64_t)vs * 2, min(key0, Skv - 1),
+                   min(key0 + part, Skv), turn * groups + place / pairs, CEIL_DIV(Sq, QTILE) * groups);
+    }
     if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256)
         __builtin_amdgcn_s_setprio(1);
     drain();
+    if (far) asm volatile("" : : "v"(touched[0]), "v"(touched[1]), "v"(touched[2]), "v"(touched[3]));
     __syncthreads();
     for (int t = tile0; t < ntiles; ++t) {
         const int cur = (t - tile0) & 1;
