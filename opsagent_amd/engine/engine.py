@@ -327,17 +327,15 @@ class LLMEngine:
         pin = self.device == "cuda"
         # persistent PINNED host staging (fresh pageable tensors per decode
         # step cost ~0.1-0.2 ms/step of host time at B=1)
-        self._h_in = torch.empty(self.max_batch, dtype=torch.int64, pin_memory=pin)
-        self._h_pos = torch.empty(self.max_batch, dtype=torch.int32, pin_memory=pin)
-        self._h_slots = torch.empty(self.max_batch, dtype=torch.int32, pin_memory=pin)
-        self._h_lens = torch.empty(self.max_batch, dtype=torch.int32, pin_memory=pin)
-        self._dec_input = torch.zeros(self.max_batch, dtype=torch.int64, device=dev)
-        self._dec_pos = torch.zeros(self.max_batch, dtype=torch.int32, device=dev)
-        self._dec_slots = torch.zeros(self.max_batch, dtype=torch.int32, device=dev)
-        self._dec_block_table = torch.zeros(
-            self.max_batch, self.max_blocks_per_seq, dtype=torch.int32, device=dev
-        )
-        self._dec_seq_lens = torch.zeros(self.max_batch, dtype=torch.int32, device=dev)
+        # All inputs of a decode step lie in one buffer here and on the device: ids, positions,
+        # slots and lengths of max_batch rows, then the block table, so that the rows in use
+        # are its start and go over in one copy
+        words = self.max_batch * (5 + self.max_blocks_per_seq)
+        self._h_step = torch.zeros(words, dtype=torch.int32, pin_memory=pin)
+        self._d_step = torch.zeros(words, dtype=torch.int32, device=dev)
+        self._h_rows = self._step_rows(self._h_step)
+        (self._dec_input, self._dec_pos, self._dec_slots, self._dec_seq_lens,
+         self._dec_block_table) = self._step_rows(self._d_step)
         hq_local = self.spec.num_heads // self.tp
         G = hq_local // hk_local if hk_local else 1
         # split count is frozen into the captured graph: size it for typical
@@ -359,6 +357,12 @@ class LLMEngine:
             self._dec_ws = None
 
     # ------------------------------------------------------------------
+    def _step_rows(self, buf: torch.Tensor) -> Tuple[torch.Tensor, ...]:
+        """Ids, positions, slots, lengths and block table of a decode step's buffer."""
+        n = self.max_batch
+        return (buf[: 2 * n].view(torch.int64), buf[2 * n : 3 * n], buf[3 * n : 4 * n],
+                buf[4 * n : 5 * n], buf[5 * n :].view(n, self.max_blocks_per_seq))
+
     def _pick_num_blocks(self, cfg: dict) -> int:
         if cfg.get("kv_num_blocks"):
             return int(cfg["kv_num_blocks"])
@@ -1134,28 +1138,26 @@ class LLMEngine:
             self._reap()
             return
         B = len(batch)
-        # fill static buffers (pinned persistent staging)
-        in_cpu = self._h_in[:B]
-        pos_cpu = self._h_pos[:B]
-        slot_cpu = self._h_slots[:B]
-        len_cpu = self._h_lens[:B]
-        bt_cpu = torch.zeros(B, self.max_blocks_per_seq, dtype=torch.int32)
+        # fill static buffers (pinned persistent staging), as arrays: an element of a tensor
+        # costs a microsecond
+        rows = tuple(t[:B] for t in self._h_rows)
+        ids, positions, slots, lens, table = (t.numpy() for t in rows)
+        table[:] = 0
         for i, req in enumerate(batch):
             seq = req.seq
             pos = len(seq.token_ids) - 1           # position of the new token
-            in_cpu[i] = seq.token_ids[-1]
-            pos_cpu[i] = pos
-            slot_cpu[i] = seq.blocks[pos // self.kv.block_size] * self.kv.block_size + (
+            ids[i] = seq.token_ids[-1]
+            positions[i] = pos
+            slots[i] = seq.blocks[pos // self.kv.block_size] * self.kv.block_size + (
                 pos % self.kv.block_size
             )
-            len_cpu[i] = pos + 1
-            nb = len(seq.blocks)
-            bt_cpu[i, :nb] = torch.tensor(seq.blocks, dtype=torch.int32)
+            lens[i] = pos + 1
+            table[i, : len(seq.blocks)] = seq.blocks
 
         if self.device == "cuda" and self.use_hipgraph:
-            logits = self._decode_graphed(B, in_cpu, pos_cpu, slot_cpu, len_cpu, bt_cpu)
+            logits = self._decode_graphed(B, *rows)
         else:
-            logits = self._decode_eager(B, in_cpu, pos_cpu, slot_cpu, len_cpu, bt_cpu)
+            logits = self._decode_eager(B, *rows)
 
         # this step wrote KV for each sequence's current last token
         for req in batch:
@@ -1172,20 +1174,16 @@ class LLMEngine:
         return min(b, self.max_batch)
 
     def _fill_static(self, B: int, in_cpu, pos_cpu, slot_cpu, len_cpu, bt_cpu, pad_to: int):
-        self._dec_input[:B].copy_(in_cpu, non_blocking=True)
-        self._dec_pos[:B].copy_(pos_cpu, non_blocking=True)
-        self._dec_slots[:B].copy_(slot_cpu, non_blocking=True)
-        self._dec_seq_lens[:B].copy_(len_cpu, non_blocking=True)
-        self._dec_block_table[:B].copy_(bt_cpu, non_blocking=True)
-        if pad_to > B:
+        for staged, row in zip(self._h_rows, (in_cpu, pos_cpu, slot_cpu, len_cpu, bt_cpu)):
+            if row.data_ptr() != staged.data_ptr():
+                staged[:B].copy_(row)
             # pad with copies of row 0 (harmless writes to row 0's slot are
             # NOT acceptable — instead repeat row 0 but redirect its slot to a
             # scratch: reuse row 0's own slot is idempotent (same k/v written)
-            self._dec_input[B:pad_to] = self._dec_input[0].clone()
-            self._dec_pos[B:pad_to] = self._dec_pos[0].clone()
-            self._dec_slots[B:pad_to] = self._dec_slots[0].clone()
-            self._dec_seq_lens[B:pad_to] = self._dec_seq_lens[0].clone()
-            self._dec_block_table[B:pad_to] = self._dec_block_table[0].clone()
+            if pad_to > B:
+                staged[B:pad_to] = staged[0]
+        used = self.max_batch * 5 + pad_to * self.max_blocks_per_seq
+        self._d_step[:used].copy_(self._h_step[:used], non_blocking=True)
 
     def _make_decode_fb(self, B: int) -> ForwardBatch:
         return ForwardBatch(
