@@ -5,9 +5,9 @@ GPU (ROCm) path → hand-written HIP/CDNA4 kernels from the in-tree library
 box, per the build contract). CPU path → opsagent_amd.ops.torch_ref (also the
 numerics oracle for the GPU parity tests).
 
-GEMM-shaped work that is a plain library GEMM (QKV/O/MLP projections,
-lm_head) goes through torch.nn.functional.linear → hipBLASLt/rocBLAS, which
-is the sanctioned path for non-fused GEMMs; the fused hot ops (norms, RoPE,
+GEMM-shaped work (QKV/O/MLP projections, lm_head) takes the kernels of its number of rows
+(linear, gateup_silu); what they do not take, and every call under gradients, goes through
+torch.nn.functional.linear → hipBLASLt/rocBLAS. The fused hot ops (norms, RoPE,
 attention, activation, sampling) are the HIP kernels here.
 """
 
