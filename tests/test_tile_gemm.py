@@ -11,7 +11,7 @@ FORMS = range(10)
 FORMS8 = range(5)
 # M, N, K, splits
 SIZES = [(129, 8, 64, 1), (256, 520, 128, 1), (300, 136, 192, 1), (161, 264, 448, 3),
-         (513, 392, 512, 2), (700, 1000, 1088, 1)]
+         (513, 392, 512, 2), (700, 1000, 1088, 1), (200, 1104, 1984, 1)]
 
 
 def _whole(rows, cols, scale=1.0):
