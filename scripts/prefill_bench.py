@@ -1,7 +1,7 @@
 """Prefill-attention variant bench: correctness vs torch fp32 + TF/s per
 variant (OPSAGENT_PREFILL_VARIANT 7 to 11) at agent-relevant shapes.
 
-Run under gpurun; summary goes to stdout (commit to profiles/README.md).
+The summary goes to stdout.
 """
 
 from __future__ import annotations
