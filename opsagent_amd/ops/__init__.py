@@ -441,6 +441,10 @@ def _tile_sizes(M: int, N: int, K: int, gateup: bool, summed: bool) -> Optional[
     if weights < (2 ** 22 if gateup or summed or M >= 500 else 9e6) or (
             M >= 3500 and not gateup):
         return None
+    if gateup and M > 4000 and M * weights >= 7.2e11:
+        tiles = -(-M // 256) * -(-2 * N // 256)
+        if K >= 8192 or K >= 4096 and -tiles % 256 < tiles // 100:
+            return None
     plan = _lib()[0].oa_tile_gemm_plan(M, N, K, int(gateup), int(summed))
     return plan if plan >= 0 else None
 
@@ -451,6 +455,11 @@ def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = Fa
     library / tiles: 2048 x 2048, 256 rows 10.1 / 13.0, 800 15.3 / 14.5; deep ones with a norm behind
     them split, 1024 x 4096, 338 16.9 / 15.0), and from some thousand rows on, where power bounds
     both (4096 x 4096, 4067 92 / 103, 2900 79 / 78), but for gate-up, whose activation rides along.
+    Of that the largest of more than 4000 rows go there where columns are many (library and
+    activation / tiles: 8000 rows of 4096 x 14336 1261 / 1346, 8192 of 7168 x 8192 1312 / 1387, 16000 of
+    28672 x 8192 10379 / 11276; smaller ones not, 5500 of 4096 x 14336 1029 / 931) or where the
+    library's tiles of 256 x 256 fill their rounds (14336 x 4096, 8192 rows 1423 / 1451, inside a
+    model 8000 1491 / 1545; 7500 1393 / 1338, 9200 1638 / 1596).
     Over 3200 products of the models' weights and of 512 to 16000 x 512 to 14336, 129 to 6000 rows,
     those taken are 1.17 times as fast as the library on average (gate-up 1.2), one in twenty up to
     1.1 times slower. summed: for linear_parts, where a norm adds up the splits."""

@@ -120,3 +120,7 @@ def test_plan():
         assert ops._tile_form_fp8(*args) == -1
     assert ops._tile_choice(128, 4096, 14336) is None    # the ring's
     assert ops._tile_choice(200, 2048, 2048) is None     # light weights, few rows: the library
+    for args, taken in (((8192, 14336, 4096), False), ((7500, 14336, 4096), True),
+                        ((9200, 14336, 4096), True), ((4000, 14336, 4096), True), ((8192, 2816, 2048), True),
+                        ((8192, 4096, 14336), False), ((5500, 4096, 14336), True), ((8000, 3584, 8192), True)):
+        assert (ops._tile_choice(*args, gateup=True) is not None) == taken
