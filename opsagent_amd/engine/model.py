@@ -167,14 +167,19 @@ class Attention(nn.Module):
         )
 
         if fb.kind == "prefill":
-            # behind a past the keys come from the cache, this prompt's among them
-            past = fb.prefill_past_len > 0
+            slots = None
+            if fb.prefill_past_len > 0:
+                # behind a past the keys come from the cache, this prompt's among them
+                skv, slots = fb.prefill_past_len + T, fb.prefill_slot_gather
+                nb, bs, hk, hd = k_cache.shape
+                k, v = k_cache.view(nb * bs, hk, hd), v_cache.view(nb * bs, hk, hd)
+                if slots is None or slots.shape != (skv,) or slots.dtype != torch.int64:
+                    # any other index that names as many rows; one that does not is refused here
+                    k, v, slots = k[slots].view(1, skv, hk, hd), v[slots].view(1, skv, hk, hd), None
+            else:
+                k, v = k.unsqueeze(0), v.unsqueeze(0)
             out = ops.attention_prefill(
-                q.unsqueeze(0),
-                k_cache.flatten(0, 1) if past else k.unsqueeze(0),
-                v_cache.flatten(0, 1) if past else v.unsqueeze(0),
-                scale=self.scale, steady=self.fp8,
-                slots=fb.prefill_slot_gather if past else None,
+                q.unsqueeze(0), k, v, scale=self.scale, steady=self.fp8, slots=slots,
             )
             out = out.view(T, self.hq * self.hd)
         else:

@@ -1392,6 +1392,18 @@ def _prefill_plan(
     return (splits if worth else 1), int(merged)
 
 
+def _rows_in_place(k: torch.Tensor, v: torch.Tensor, slots: torch.Tensor, D: int) -> bool:
+    """Whether the prefill kernel may read rows ``slots`` of k and v [rows, Hk, D] where they lie: a
+    list of int64 beside them, heads side by side, rows from 16 bytes to 16 bytes. Everything else
+    that an index of a tensor may be is gathered."""
+    steps = k.stride()
+    return (len(steps) == 3 and steps[1:] == (D, 1) and 0 < steps[0] < 2 ** 31 and steps[0] % 8 == 0
+            and v.stride() == steps and v.shape == k.shape and 0 < k.shape[0] < 2 ** 31
+            and (k.data_ptr() | v.data_ptr()) % 16 == 0
+            and slots.dtype == torch.int64 and slots.dim() == 1 and slots.is_contiguous()
+            and slots.get_device() == k.get_device() == v.get_device())
+
+
 def attention_prefill(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -1404,11 +1416,12 @@ def attention_prefill(
     """q [B, Sq, Hq, D]; k, v [B, Skv, Hk, D] (token-major layouts; the CPU
     reference uses [B, H, S, D], so the dispatch transposes for it). ``steady``: a row's keys
     added up in the one order that callers with 8-bit activations are held to: any other
-    rounding of a weight moves some of those to the next 8-bit value. ``slots``: int64 [Skv],
-    key i of the one sequence is row slots[i] of the caches k, v [rows, Hk, D]; the kernel
-    reads them where they lie (us, two gathers and attention / here, 32 heads on 8: 77 queries
-    of 1264 keys 20.6 / 15.3, 800 of 1056 33.9 / 29.1, 2048 of 6144 215 / 204)."""
-    if slots is not None and not (_is_gpu(q) and slots.dtype == torch.int64 and slots.is_contiguous()):
+    rounding of a weight moves some of those to the next 8-bit value. ``slots``: [Skv],
+    key i of the one sequence is row slots[i] of the caches k, v [rows, Hk, D], counted from the
+    end below 0; the kernel reads them where they lie (us, two gathers and attention / here, 32 heads
+    on 8: 77 queries of 1264 keys 20.6 / 15.3, 800 of 1056 33.9 / 29.1, 2048 of 6144 215 / 204),
+    and takes the last row for a slot outside the caches (by its low 32 bits), which a gather faults on."""
+    if slots is not None and not (_is_gpu(q) and _rows_in_place(k, v, slots, q.shape[-1])):
         k, v, slots = k[slots], v[slots], None
         k, v = k.unsqueeze(0), v.unsqueeze(0)
     if not _is_gpu(q):
@@ -1420,16 +1433,17 @@ def attention_prefill(
     assert q.dtype == torch.bfloat16
     B, Sq, Hq, D = q.shape
     if slots is not None:
-        assert B == 1 and k.dim() == v.dim() == 3 and slots.dim() == 1
-        k, v = k.unsqueeze(0), v.unsqueeze(0)
-    Skv, Hk = k.shape[1] if slots is None else slots.shape[0], k.shape[2]
-    for t, name in ((q, "q"), (k, "k"), (v, "v")):
+        assert B == 1
+        Skv, Hk, at, rows = slots.shape[0], k.shape[1], slots.data_ptr(), k.shape[0]
+    else:
+        Skv, Hk, at, rows = k.shape[1], k.shape[2], None, 0
+    k_step, v_step = k.stride(-3), v.stride(-3)
+    for t, name in ((q, "q"), (k, "k"), (v, "v")) if slots is None else ((q, "q"),):
         assert t.stride(3) == 1 and t.stride(2) == D, f"{name} heads must be inner-contiguous"
         assert t.shape[0] == 1 or t.stride(0) == t.shape[1] * t.stride(1), f"{name} batch stride"
     scale = scale if scale is not None else D ** -0.5
     lib, hip = _lib()
     out = torch.empty(B, Sq, Hq, D, dtype=q.dtype, device=q.device)
-    at = None if slots is None else slots.data_ptr()
     steady = steady or scale <= 0.0        # the other forms take their maxima before the scale
     splits, form = _prefill_plan(B, Hq, Hk, Sq, Skv, steady)
     if splits > 1 and D == 128 and "OPSAGENT_PREFILL_VARIANT" not in os.environ:
@@ -1438,14 +1452,14 @@ def attention_prefill(
         rc = lib.oa_attention_prefill_split(
             hip.current_stream_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
             out.data_ptr(), part.data_ptr(), part.data_ptr() + sums, B, Hq, Hk, Sq, Skv, D,
-            scale, q.stride(1), k.stride(1), v.stride(1), splits, form, at,
+            scale, q.stride(1), k_step, v_step, splits, form, at, rows,
         )
         hip.check(rc, "oa_attention_prefill_split")
         return out
     rc = lib.oa_attention_prefill(
         hip.current_stream_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
         out.data_ptr(), B, Hq, Hk, Sq, Skv, D, scale,
-        q.stride(1), k.stride(1), v.stride(1), int(steady), at,
+        q.stride(1), k_step, v_step, int(steady), at, rows,
     )
     hip.check(rc, "oa_attention_prefill")
     return out

@@ -85,9 +85,9 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_masked_argmax_f32.restype = i
     lib.oa_token_logprobs.argtypes = [p, p, ctypes.c_int64, p, p, p, i, i, i, i]
     lib.oa_token_logprobs.restype = i
-    lib.oa_attention_prefill.argtypes = [p, p, p, p, p, i, i, i, i, i, i, f, i, i, i, i, p]
+    lib.oa_attention_prefill.argtypes = [p, p, p, p, p, i, i, i, i, i, i, f, i, i, i, i, p, i]
     lib.oa_attention_prefill.restype = i
-    lib.oa_attention_prefill_split.argtypes = [p] * 7 + [i] * 6 + [f, i, i, i, i, i, p]
+    lib.oa_attention_prefill_split.argtypes = [p] * 7 + [i] * 6 + [f, i, i, i, i, i, p, i]
     lib.oa_attention_prefill_split.restype = i
     lib.oa_attention_decode.argtypes = [p, p, p, p, p, p, p, p, p, p, i, i, i, i, i, i, i, f, i, i]
     lib.oa_attention_decode.restype = i

@@ -86,6 +86,86 @@ def test_cache_rows_on_the_host():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["host", "int32", "below 0", "wider rows", "off the grid", "mask"])
+def test_any_index_of_rows(kind):
+    """Every index that a gather takes: on the host, of 32 bits, from the end; caches that the kernel
+    cannot read in place."""
+    gen = torch.Generator(device="cuda").manual_seed(len(kind))
+    Hq, Hk, Sq, Skv, rows = 8, 2, 70, 410, 450
+    q = torch.randn(1, Sq, Hq, D, generator=gen, device="cuda").bfloat16()
+    k, v = (torch.randn(rows, Hk, D + 8, generator=gen, device="cuda").bfloat16() for _ in range(2))
+    if kind == "wider rows":
+        k, v = k[:, :, :D], v[:, :, :D]
+    elif kind == "off the grid":
+        k, v = (t.flatten()[1:1 + rows * Hk * D].view(rows, Hk, D) for t in (k, v))
+    else:
+        k, v = k[:, :, :D].contiguous(), v[:, :, :D].contiguous()
+    slots = torch.randperm(rows, generator=gen, device="cuda")[:Skv].contiguous()
+    if kind == "host":
+        slots = slots.cpu()
+    elif kind == "int32":
+        slots = slots.int()
+    elif kind == "below 0":
+        slots[::3] -= rows
+    elif kind == "mask":
+        slots = torch.zeros(rows, dtype=torch.bool, device="cuda").index_fill(0, slots, True)
+    want = ops.attention_prefill(q, k[slots].view(1, Skv, Hk, D), v[slots].view(1, Skv, Hk, D))
+    assert torch.equal(ops.attention_prefill(q, k, v, slots=slots), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("steady", [False, True])
+def test_rows_outside(steady):
+    """A slot outside the caches reads their last row, on either side; of more bits the low 32 count."""
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    Sq, Skv, rows = 40, 700, 750
+    q, k, v = (torch.randn(n, 2, D, generator=gen, device="cuda").bfloat16() for n in (Sq, rows, rows))
+    slots = torch.randperm(rows, generator=gen, device="cuda")[:Skv].contiguous()
+    far = slots.clone()
+    for i, at in ((5, rows), (133, 2 ** 31 - 1), (300, -rows - 1), (450, -2 ** 31), (699, 2 ** 40 + rows)):
+        slots[i], far[i] = rows - 1, at
+    want = ops.attention_prefill(q[None], k[slots][None], v[slots][None], steady=steady)
+    assert torch.equal(ops.attention_prefill(q[None], k, v, steady=steady, slots=far), want)
+
+
+def _attend(device, dtype, gather, past=24, T=9, block=8, heads=2):
+    """One attention sublayer over T rows behind a past, its caches' rows named by gather(list)."""
+    from opsagent_amd.engine import model as m
+    from opsagent_amd.engine.config import get_model_spec
+
+    spec = get_model_spec("llama3-tiny") if dtype == torch.float32 else get_model_spec("llama3-micro")
+    gen = torch.Generator().manual_seed(1)
+    layer = m.Attention(spec, dtype, gen).to(device)
+    hd, rows = spec.head_dim, 6 * block
+    caches = [torch.randn(6, block, spec.num_kv_heads, hd, generator=gen).to(dtype).to(device) for _ in "kv"]
+    cos, sin = (torch.randn(past + T, hd // 2, generator=gen).to(device) for _ in "cs")
+    slots = torch.randperm(rows, generator=gen)[:past + T]
+    x = torch.randn(T, spec.hidden_size, generator=gen).to(dtype).to(device)
+    fb = m.ForwardBatch(kind="prefill", input_ids=torch.zeros(T, dtype=torch.int64, device=device),
+                        positions=torch.arange(past, past + T, dtype=torch.int32, device=device),
+                        slot_mapping=slots[past:].int().to(device), prefill_past_len=past,
+                        prefill_slot_gather=gather(slots.to(device), rows))
+    with torch.no_grad():
+        return layer(x, cos, sin, *caches, fb)
+
+
+GATHERS = {"host": lambda s, n: s.cpu(), "int32": lambda s, n: s.int(), "table": lambda s, n: s.view(3, -1),
+           "below 0": lambda s, n: s - n}
+
+
+@pytest.mark.parametrize("device,dtype", [("cpu", torch.float32), pytest.param(
+    "cuda", torch.bfloat16, marks=pytest.mark.gpu)])
+def test_rows_of_a_past(device, dtype):
+    """What a sublayer's caller may hand in as the rows of a past, and lengths that are refused."""
+    want = _attend(device, dtype, lambda s, n: s)
+    for name, gather in GATHERS.items():
+        assert torch.equal(_attend(device, dtype, gather), want), name
+    for wrong in (lambda s, n: s[:-1], lambda s, n: torch.cat([s, s[:1]]), lambda s, n: s[:0], lambda s, n: None):
+        with pytest.raises(RuntimeError):
+            _attend(device, dtype, wrong)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("variant", [10, 11])
 def test_scores_that_do_not_compare(monkeypatch, variant):
     """A row with a NaN or a positive infinite score is NaN in whichever group the score lies,
