@@ -466,6 +466,12 @@ def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = Fa
     return _tile_sizes(M, N, K, gateup, summed) if M > 128 else None
 
 
+def _near_rows(x: torch.Tensor) -> bool:
+    """Rows of x that the tile product's 32-bit places span (tile_gemm.hip): less than 8 MB apart.
+    Others, one token of each of many long sequences, go to the library."""
+    return x.is_contiguous() or x.stride(0) < 2 ** 22
+
+
 def _tile(x: torch.Tensor, w: torch.Tensor, plan: int, act: int = 0,
           parts: bool = False) -> torch.Tensor:
     """x @ w^T, or act 1 (silu), 2 (tanh gelu) of the gate rows times the up rows, in the form
@@ -490,7 +496,7 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor) -> Union[torch.Tensor, PlaneS
     M = x.numel() // x.shape[-1]
     if M > 1 and x.dim() == 2 and w.shape[0] <= 8192 and _skinny_ok(x, w):
         if M > 128:
-            tile = _tile_choice(M, w.shape[0], w.shape[1], summed=True)
+            tile = _tile_choice(M, w.shape[0], w.shape[1], summed=True) if _near_rows(x) else None
             return PlaneSum(_tile(x, w, tile, parts=True)) if tile and tile & 255 > 1 else linear(x, w)
         plan = _ring_form(M, w.shape[0], w.shape[1])
         if plan and plan[1] > 1:
@@ -513,7 +519,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         form = _skinny_form(M, w.shape[0], w.shape[1], strided=not x.is_contiguous())
         if form:
             return _skinny(x, w, form)
-    if M > 128 and _skinny_ok(x, w):
+    if M > 128 and _skinny_ok(x, w) and _near_rows(x):
         plan = _tile_choice(M, w.shape[0], w.shape[1])
         if plan is not None:
             return _tile(x, w, plan)

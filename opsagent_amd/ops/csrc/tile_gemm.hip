@@ -512,6 +512,12 @@ static int tg_choose(const TgForm (&forms)[FORMS], int M, int rows, int steps, b
     return plan;
 }
 
+// A lane's place in a tile is 32 bits wide: rows of x less than 8 MB apart, and the weight rows of a strip
+// (gate-up: and their up rows, N further on) within 4 GB
+static bool tg_within(int64_t xs, int64_t N, int64_t K, bool gateup) {
+    return xs < (1 << 22) && ((gateup ? N : 0) + 256) * K * 2 < ((int64_t)1 << 32);
+}
+
 // The plan of M rows, N (gate-up: 2 N) weight rows and K columns; -1 for sizes that the product does not
 // take, and for gate-up products that other forms take sooner. Splits fill the CUs where the tiles leave
 // some idle, at most one block a CU; their parts are written, and read again by a kernel of their own (4.5
@@ -520,6 +526,7 @@ static int tg_choose(const TgForm (&forms)[FORMS], int M, int rows, int steps, b
 // the library and the kernel) it is left to them.
 extern "C" int oa_tile_gemm_plan(int M, int N, int K, int gateup, int summed) {
     if (M < 1 || N < 8 || N % 8 != 0 || N > (1 << 29) || K < 512 || K % 64 != 0) return -1;
+    if (!tg_within(K, N, K, gateup)) return -1;
     float one, two;
     if (!gateup) return tg_choose(tg_forms, M, N, K / 64, true, summed, &one);
     const int plan = tg_choose(tg_forms, M, 2 * N, K / 64, false, false, &one);
@@ -614,8 +621,7 @@ extern "C" int oa_tile_gemm(void* stream, const void* x, int64_t xs, const void*
     if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)scratch) % 16 != 0 || xs % 8 != 0)
         return -102;
     if (act < 0 || act > 2 || plan < 0) return -104;
-    // a lane's place in a tile is 32 bits wide
-    if (xs < K || xs >= (1 << 22) || ((int64_t)(act ? N : 0) + 256) * K * 2 >= ((int64_t)1 << 32)) return -103;
+    if (xs < K || !tg_within(xs, N, K, act != 0)) return -103;
     const int rc = tg_run((hipStream_t)stream, x, xs * 2, w, nullptr, nullptr, out, splits > 1 ? scratch : nullptr,
                           M, N, (int64_t)K * 2, form, splits, act, false);
     return rc || splits == 1 || !out ? rc : oa_ring_sum(stream, scratch, out, M, N, splits);

@@ -94,6 +94,37 @@ def test_dispatch():
     assert grad.grad is not None
 
 
+@pytest.mark.gpu
+def test_rows_far_apart():
+    """One token of each of many long sequences, 8 MB apart and a step less."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    w = (torch.randn(4096, 4096, generator=g, device="cuda") / 64).bfloat16()
+    rows = torch.randn(160, 4096, generator=g, device="cuda").bfloat16()
+    want = rows.double() @ w.double().T
+    for step in (2 ** 22 - 8, 2 ** 22, 2 ** 22 + 8):
+        x = torch.empty(160 * step, dtype=torch.bfloat16, device="cuda").view(160, step)[:, :4096]
+        x.copy_(rows)
+        parts = ops.linear_parts(x, w)
+        for got in (ops.linear(x, w), ops._added_up(parts) if isinstance(parts, ops.PlaneSum) else parts):
+            assert (got.double() - want).norm() <= 2.0 ** -8 * want.norm()     # one rounding
+
+
+def test_plan_within_reach():
+    """A plan is a product that the launch takes: what its 32-bit places do not span has none."""
+    plan = ops._lib()[0].oa_tile_gemm_plan
+    for M in (129, 4000):
+        for N, K in ((2 ** 21, 1024), (2 ** 21 - 256, 1024), (2 ** 21 - 264, 1024), (2 ** 18, 8192),
+                     (512, 2 ** 22), (512, 2 ** 22 - 64), (8, 2 ** 23), (2 ** 20, 2048)):
+            for gateup in (0, 1):
+                within = K < 2 ** 22 and (gateup * N + 256) * K * 2 < 2 ** 32
+                assert within or plan(M, N, K, gateup, 0) == -1, (M, N, K, gateup)
+                assert not within or gateup or plan(M, N, K, 0, 0) >= 0
+    assert ops._tile_choice(1000, 2 ** 21, 1024, gateup=True) is None
+    for step in (64, 2 ** 22 - 8, 2 ** 22):
+        x = torch.empty_strided((200, 64), (step, 1), dtype=torch.bfloat16, device="meta")
+        assert ops._near_rows(x) == (step < 2 ** 22)
+
+
 def test_plan():
     """Sizes that no form takes, and what the rule answers for those it takes: a form of the table,
     splits that leave every block eight steps and no more blocks than CUs."""
