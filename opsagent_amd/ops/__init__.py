@@ -1368,9 +1368,10 @@ def _prefill_splits(B: int, Hq: int, Hk: int, Sq: int, Skv: int) -> Tuple[int, b
 
 @functools.lru_cache(maxsize=4096)
 def _prefill_plan(
-    B: int, Hq: int, Hk: int, Sq: int, Skv: int, steady: bool = False
+    B: int, Hq: int, Hk: int, Sq: int, Skv: int, steady: bool = False, scaled: bool = False
 ) -> Tuple[int, int]:
-    """(key splits, form) of prefill attention: form 0 in key groups, 1 merged, 2 steady.
+    """(key splits, form) of prefill attention: form 0 in key groups, 1 merged, 2 steady, which alone
+    takes the maxima of scaled scores (scaled).
 
     What :func:`_prefill_splits` splits, the steady form as it says; the others where that is
     faster than key groups within a block, which halve and quarter a chain of tiles without
@@ -1385,6 +1386,8 @@ def _prefill_plan(
     tiles: 35 / 40, 51 / 49, and 1000 queries of 16 heads, 26 and 34: 51 / 56, 64 / 65; in
     six, 300 queries, 12 and 20 tiles: 26 / 30, 39 / 37)."""
     splits, merged = _prefill_splits(B, Hq, Hk, Sq, Skv)
+    if scaled:
+        return splits, 2
     if steady or splits == 1:
         return splits, 1 if merged else 2 * steady
     tiles = (Skv + 127) // 128
@@ -1450,8 +1453,8 @@ def attention_prefill(
     scale = scale if scale is not None else D ** -0.5
     lib, hip = _lib()
     out = torch.empty(B, Sq, Hq, D, dtype=q.dtype, device=q.device)
-    steady = steady or scale <= 0.0        # the other forms take their maxima before the scale
-    splits, form = _prefill_plan(B, Hq, Hk, Sq, Skv, steady)
+    # where a larger score is no larger weight, maxima before the scale would not bound the weights
+    splits, form = _prefill_plan(B, Hq, Hk, Sq, Skv, steady, not scale > 0.0)
     if splits > 1 and D == 128 and "OPSAGENT_PREFILL_VARIANT" not in os.environ:
         part = torch.empty(splits, B, Sq, Hq, D + 2, dtype=torch.float32, device=q.device)
         sums = splits * B * Sq * Hq * D * 4

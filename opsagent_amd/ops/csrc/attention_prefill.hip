@@ -528,7 +528,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_kernel(
 // next 8-bit value, and two forms that are each 0.036 from 64 bits end 0.037 apart; so 8-bit
 // models keep the form and the splits that they had, whatever is the fastest. Waves of
 // 16 rows on 16x16x32 products; P goes through LDS to become an operand. A tile takes 5 us,
-// its LDS reads (512 KB for 128 rows) the most of it.
+// its LDS reads (512 KB for 128 rows) the most of it. It alone takes its maxima of scaled scores, which
+// scales of 0 and below need.
 template <bool SPLIT, bool PAGED>
 __global__ __launch_bounds__(512, 1) void attn_prefill_steady_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
@@ -1002,7 +1003,9 @@ extern "C" int oa_attention_prefill(void* stream, const void* q, const void* k,
     int variant = e ? atoi(e) : 0;
     const int gq = (Hk > 0 && Hq % Hk == 0) ? Hq / Hk : 1;
     const bool shared = gq == 2 || gq == 4 || gq == 8;
-    if (variant <= 0 && steady) {
+    if (variant <= 0 && !(scale > 0.0f)) {
+        variant = 7;     // the maximum of scores that are scaled; the others scale maxima
+    } else if (variant <= 0 && steady) {
         const int64_t heads = (int64_t)B * Hq;
         variant = shared && CEIL_DIV(Sq, 128) * heads > 256 ? 9
                   : CEIL_DIV(Sq, 256) * heads >= 256 ? 8 : 7;

@@ -166,6 +166,31 @@ def test_rows_of_a_past(device, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("steady", [False, True])
+@pytest.mark.parametrize("scale", [-1.0, -0.0, 0.0])
+@pytest.mark.parametrize("Hq,Hk,Sq,Skv", [(8, 2, 40, 900), (32, 8, 300, 4000), (32, 8, 1100, 1100),
+                                          (48, 16, 1500, 1500), (4, 4, 65, 65)])
+def test_scales_that_turn_scores(Hq, Hk, Sq, Skv, scale, steady):
+    """Negative and zero scales, where the largest score has not the largest weight: split over many
+    and few queries, blocks of a key head, of 256 rows and of fewer."""
+    gen = torch.Generator(device="cuda").manual_seed(Sq)
+    q, k, v = (torch.randn(1, n, h, D, generator=gen, device="cuda").bfloat16()
+               for n, h in ((Sq, Hq), (Skv, Hk), (Skv, Hk)))
+    got = ops.attention_prefill(q, k, v, scale=scale, steady=steady)
+    check(got, q.double() * (scale * D ** 0.5), k, v)
+    slots = torch.randperm(Skv, generator=gen, device="cuda")
+    back = torch.argsort(slots)                          # row slots[i] is key i
+    assert torch.equal(ops.attention_prefill(q, k[0][back], v[0][back], scale=scale, steady=steady,
+                                             slots=slots), got)
+
+
+def test_scales_have_one_form():
+    for Hq, Hk, Sq, Skv in ((32, 8, 300, 4000), (32, 8, 40, 900), (32, 8, 2048, 2048), (4, 4, 5, 5)):
+        assert ops._prefill_plan(1, Hq, Hk, Sq, Skv, scaled=True)[1] == 2
+        assert ops._prefill_plan(1, Hq, Hk, Sq, Skv, True, True)[1] == 2
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("variant", [10, 11])
 def test_scores_that_do_not_compare(monkeypatch, variant):
     """A row with a NaN or a positive infinite score is NaN in whichever group the score lies,
