@@ -434,8 +434,9 @@ def linear_dyt_norm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
             and (x.data_ptr() | w.data_ptr()) % 16 == 0):
         return dyt_norm(residual, nxt, out_dtype, y=ops.linear(x, w), post=post)
     N = w.shape[0]
-    for t in post + (nxt or ()):
-        assert t.dtype == torch.float32 and t.is_contiguous() and t.numel() in (1, N)
+    for norm in (post,) if nxt is None else (post, nxt):
+        for t, n in zip(norm, (N, N, 1)):
+            assert t.dtype == torch.float32 and t.is_contiguous() and t.numel() == n
     lib, hip = _lib()
     out = torch.empty(1, N, dtype=out_dtype, device=x.device) if nxt is not None else None
     kernels = hip.get_lib()

@@ -37,6 +37,20 @@ def test_against_two_launches(N, K, last):
 
 
 @pytest.mark.gpu
+def test_norms_of_another_width():
+    """A weight or bias of one number, or a slope of many, is refused and not read past its end."""
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x, w = (torch.randn(n, 2048, generator=g, device="cuda").bfloat16() for n in (1, 64))
+    r, good = torch.zeros(1, 64, device="cuda"), _norm(g, 64)
+    for i in range(3):
+        bad = tuple(t.new_ones(1 if n < 2 else 64) if n == i else t for n, t in enumerate(good))
+        for post, nxt in ((bad, good), (good, bad), (bad, None)):
+            with pytest.raises(AssertionError):
+                mx.linear_dyt_norm(x, w, r, nxt, torch.bfloat16, post)
+    assert not r.any()
+
+
+@pytest.mark.gpu
 def test_others_go_the_old_way():
     """Two rows, short rows, float32 and operands off the 16-byte grid."""
     g = torch.Generator(device="cuda").manual_seed(0)
