@@ -147,6 +147,15 @@ def test_prompts(D, H, G, chunks, page, opts):
     assert ((got - want).abs() <= bound).all(), ((got - want).abs() / bound).max()
 
 
+def _counted(monkeypatch, lib):
+    """The launches of a decode step's preparation and attention, as they are made."""
+    calls = []
+    for name in ("oa_attn_rows_rope", "oa_attn_rope_prepare", "oa_attn_bias_paged"):
+        inner = getattr(lib, name)
+        monkeypatch.setattr(lib, name, lambda *a, name=name, inner=inner: calls.append(name) or inner(*a))
+    return calls
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("splits", [None, 1, 3])
 @pytest.mark.parametrize("ctx,H,G,D,page,window,nfreq,sinks", [
@@ -181,11 +190,40 @@ def test_from_the_projection(monkeypatch, splits, ctx, H, G, D, page, window, nf
     slots = sb.slot_mapping.long()
     k2.view(-1, G, D)[slots] = float("nan")
     v2.view(-1, G, D)[slots] = float("nan")
+    calls = _counted(monkeypatch, lib)
     got = mx.attn_rope_rows(qkv, qw, kw, freq, H, G, D, D, 1e-6, k2, v2, sb, D ** -0.5,
                             window=window, sinks=sk)
+    assert calls == ["oa_attn_rows_rope"]
     # the sums of squares in another order: a few queries and keys round to the other neighbour
     assert torch.equal(v2, v1)
     assert torch.allclose(k2.float(), k1.float(), rtol=2.0 ** -7, atol=0)
     assert (k2 != k1).float().mean() < 0.01
     assert (got.float() - want.float()).norm() <= 2.0 ** -8 * want.float().norm()
     assert (got.float() - want.float()).abs().max() <= 2.0 ** -6 * v.float().abs().max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("other", ["float32", "prompt", "256", "value heads", "16 heads", "rows off the grid",
+                                   "weights off the grid"])
+def test_others_take_two_launches(monkeypatch, other):
+    """What the fused launch does not take is prepared and attended as before, bit for bit."""
+    g = torch.Generator(device="cuda").manual_seed(2)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    dtype = torch.float32 if other == "float32" else torch.bfloat16
+    H, G, D, page, past, new = 8, 2, 128, 16, 37, 2 if other == "prompt" else 1
+    D, Dv = {"256": (256, 256), "value heads": (128, 64)}.get(other, (D, D))
+    H = 32 if other == "16 heads" else H
+    n = (H + G) * D + G * Dv
+    qkv = rn(new, n + 7).to(dtype)[:, :n] if other == "rows off the grid" else rn(new, n).to(dtype)
+    off = int(other == "weights off the grid")
+    qw, kw = ((1 + 0.1 * rn(D + off))[off:] for _ in "qk")
+    freq = mx.rotary_inv_freq(D, 10000.0).cuda()
+    sb = mx.SeqBatch.build([(past, new, 0, [2, 0, 1])], page, "cuda")
+    k, v = rn(3, page, G, D).to(dtype), rn(3, page, G, Dv).to(dtype)
+    k1, v1, k2, v2 = k.clone(), v.clone(), k.clone(), v.clone()
+    q = mx.attn_rope_prepare(qkv, qw, kw, freq, H, G, D, Dv, 1e-6, k1, v1, sb)
+    want = mx.attention_paged(q, k1, v1, sb, D ** -0.5, window=20)
+    calls = _counted(monkeypatch, mx._lib()[0])
+    got = mx.attn_rope_rows(qkv, qw, kw, freq, H, G, D, Dv, 1e-6, k2, v2, sb, D ** -0.5, window=20)
+    assert calls == ["oa_attn_rope_prepare", "oa_attn_bias_paged"]
+    assert torch.equal(got, want) and torch.equal(k1, k2) and torch.equal(v1, v2)

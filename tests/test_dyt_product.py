@@ -14,11 +14,19 @@ def _norm(g, n):
     return 1 + 0.1 * r(n), 0.1 * r(n), 0.5 + 0.1 * r(1)
 
 
+def _counted(monkeypatch):
+    """The fused launches, as they are made."""
+    calls, lib = [], ops._lib()[0]
+    inner = lib.oa_gemv_dyt
+    monkeypatch.setattr(lib, "oa_gemv_dyt", lambda *a: calls.append(a) or inner(*a))
+    return calls
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("last", [False, True])
 @pytest.mark.parametrize("N,K", [(2048, 2048), (2048, 8192), (4096, 14336), (1, 2048), (37, 4096),
                                  (5001, 6144), (20000, 2048), (33000, 4096), (7, 16384)])
-def test_against_two_launches(N, K, last):
+def test_against_two_launches(monkeypatch, N, K, last):
     g = torch.Generator(device="cuda").manual_seed(N + K)
     x = torch.randn(1, K, generator=g, device="cuda").bfloat16()
     w = (torch.randn(N, K, generator=g, device="cuda") * 2 * K ** -0.5).bfloat16()
@@ -26,7 +34,9 @@ def test_against_two_launches(N, K, last):
     post, nxt = _norm(g, N), None if last else _norm(g, N)
     want_r, got_r = r.clone(), r.clone()
     want = mx.dyt_norm(want_r, nxt, torch.bfloat16, y=ops.linear(x, w), post=post)
+    calls = _counted(monkeypatch)
     got = mx.linear_dyt_norm(x, w, got_r, nxt, torch.bfloat16, post)
+    assert len(calls) == 1
     # the same operations in float32: a contraction apart, 4 roundings of numbers up to 4
     assert (got_r - want_r).abs().max() <= 4 * 4 * 2.0 ** -24
     if last:
@@ -51,10 +61,10 @@ def test_norms_of_another_width():
 
 
 @pytest.mark.gpu
-def test_others_go_the_old_way():
+def test_others_go_the_old_way(monkeypatch):
     """Two rows, short rows, float32 and operands off the 16-byte grid."""
     g = torch.Generator(device="cuda").manual_seed(0)
-    N = 64
+    N, calls = 64, _counted(monkeypatch)
     for T, K, dtype, off in ((2, 2048, torch.bfloat16, 0), (1, 1024, torch.bfloat16, 0),
                              (1, 2048, torch.float32, 0), (1, 2048, torch.bfloat16, 1)):
         x = torch.randn(T * K + off, generator=g, device="cuda").to(dtype)[off:].view(T, K)
@@ -65,6 +75,7 @@ def test_others_go_the_old_way():
         want = mx.dyt_norm(want_r, nxt, dtype, y=ops.linear(x, w), post=post)
         got = mx.linear_dyt_norm(x, w, got_r, nxt, dtype, post)
         assert torch.equal(got, want) and torch.equal(got_r, want_r)
+    assert not calls
 
 
 def test_cpu():
