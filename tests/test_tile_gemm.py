@@ -94,6 +94,16 @@ def test_dispatch():
     assert grad.grad is not None
 
 
+def test_rounds_of_the_library():
+    """Large gate-up products: the library's where its tiles of 256 x 256 fill every round."""
+    for M, N, K, blocks, taken in ((8192, 14336, 4096, 14 * 256, False), (8193, 14336, 4096, 3696, True),
+                                   (7937, 14336, 4096, 14 * 256, False), (10319, 14336, 4096, 18 * 256 - 16, True),
+                                   (12288, 14336, 4096, 21 * 256, False), (13195, 13824, 5120, 22 * 256 - 16, True),
+                                   (14976, 13824, 5120, 25 * 256 - 28, True)):
+        assert -(-M // 256) * (2 * N // 256) == blocks
+        assert (ops._tile_choice(M, N, K, gateup=True) is not None) == taken
+
+
 @pytest.mark.gpu
 def test_rows_far_apart():
     """One token of each of many long sequences, 8 MB apart and a step less."""
