@@ -446,7 +446,9 @@ def _tile_sizes(M: int, N: int, K: int, gateup: bool, summed: bool) -> Optional[
         if K >= 8192 or K >= 4096 and tiles % 256 == 0:
             return None
     plan = _lib()[0].oa_tile_gemm_plan(M, N, K, int(gateup), int(summed))
-    return plan if plan >= 0 else None
+    if plan < 0 or plan == 1 and K >= 2048 and not gateup:       # tiles of 256 x 256, unsplit
+        return None
+    return plan
 
 
 def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = False) -> Optional[int]:
@@ -455,15 +457,19 @@ def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = Fa
     library / tiles: 2048 x 2048, 256 rows 10.1 / 13.0, 800 15.3 / 14.5; deep ones with a norm behind
     them split, 1024 x 4096, 338 16.9 / 15.0), and from some thousand rows on, where power bounds
     both (4096 x 4096, 4067 92 / 103, 2900 79 / 78), but for gate-up, whose activation rides along.
-    Of that the largest of more than 4000 rows go there where columns are many (library and
+    So do products that would run in whole tiles of 256 x 256, the library's own form and faster
+    there (8192 x 4096, 2048 rows 93 / 101; 16384 x 2048, 922 53 / 53, 1966 99 / 105, 2987 156 / 170; 14336 x
+    4096, 1024 89 / 94, 2092 180 / 194; 10240 x 8192, 3072 337 / 358), but for short rows, where it is
+    not (10296 x 640, 1430 35 / 23).
+    Of gate-up the largest of more than 4000 rows go there where columns are many (library and
     activation / tiles: 8000 rows of 4096 x 14336 1281 / 1371, 8192 of 7168 x 8192 1315 / 1385, 16000 of
     28672 x 8192 10213 / 10959, 9395 of 16848 x 13952 6023 / 6735; smaller ones not, 5500 of 4096 x 14336
     1049 / 964) or where its tiles, 256 x 256 by its kernel's name, which splits those left over by
-    columns, leave none over (14336 x 4096, 8000 rows 1403 / 1449, 8192 1412 / 1459, 12288 2084 / 2114; 7500 1404 / 1377, 8193
-    1576 / 1507, 9200 1601 / 1601, 10319, 16 of 4608 short, 1935 / 1796; 13195 of 13824 x 5120, 16 of 5632 short,
-    3038 / 2680). Over 113 products of 3000 to 16384 rows, 52 of them drawn, the choice is 0.5 per cent
-    from the better of the two on average; many columns in part of a round lose up to 6 (5084 rows of
-    8424 x 9984, 1346 / 1266).
+    columns, leave none over (14336 x 4096, 8000 rows 1403 / 1449, 8192 1412 / 1459, 12288 2084 / 2114;
+    7500 1404 / 1377, 8193 1576 / 1507, 9200 1601 / 1601, 10319, 16 tiles of 4608 short, 1935 / 1796;
+    13195 of 13824 x 5120, 16 of 5632 short, 3038 / 2680). Over 113 products of 3000 to 16384 rows, 52 of
+    them drawn, the choice is 0.5 per cent from the better of the two on average; many columns in
+    part of a round lose up to 6 (5084 rows of 8424 x 9984, 1346 / 1266).
     Over 3200 products of the models' weights and of 512 to 16000 x 512 to 14336, 129 to 6000 rows,
     those taken are 1.17 times as fast as the library on average (gate-up 1.2), one in twenty up to
     1.1 times slower. summed: for linear_parts, where a norm adds up the splits."""

@@ -94,6 +94,16 @@ def test_dispatch():
     assert grad.grad is not None
 
 
+def test_whole_tiles_of_the_library():
+    """Plain products in unsplit tiles of 256 x 256 are the library's, but for short rows."""
+    plan = ops._lib()[0].oa_tile_gemm_plan
+    for M, N, K, taken in ((2048, 8192, 4096, False), (1966, 16384, 2048, False), (1024, 14336, 4096, False),
+                           (1430, 10296, 640, True)):
+        assert plan(M, N, K, 0, 0) == 1 and (ops._tile_choice(M, N, K) is not None) == taken
+    assert plan(2048, 4096, 14336, 0, 0) == 2 == ops._tile_choice(2048, 4096, 14336)      # split in two
+    assert plan(3900, 8192, 2048, 1, 0) == 1 == ops._tile_choice(3900, 8192, 2048, gateup=True)
+
+
 def test_rounds_of_the_library():
     """Large gate-up products: the library's where its tiles of 256 x 256 fill every round."""
     for M, N, K, blocks, taken in ((8192, 14336, 4096, 14 * 256, False), (8193, 14336, 4096, 3696, True),
