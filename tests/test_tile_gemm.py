@@ -104,6 +104,14 @@ def test_whole_tiles_of_the_library():
     assert plan(3900, 8192, 2048, 1, 0) == 1 == ops._tile_choice(3900, 8192, 2048, gateup=True)
 
 
+def test_light_weights():
+    for N, K in ((2048, 2048), (2560, 2560), (3072, 2048), (2048, 2816)):
+        assert ops._tile_choice(512, N, K) is None and ops._tile_choice(599, N, K) is None
+        assert ops._tile_choice(640, N, K) is not None
+    assert ops._tile_choice(512, 2816, 2048, gateup=True) is not None
+    assert ops._tile_choice(512, 2048, 8192) is not None
+
+
 def test_rounds_of_the_library():
     """Large gate-up products: the library's where its tiles of 256 x 256 fill every round."""
     for M, N, K, blocks, taken in ((8192, 14336, 4096, 14 * 256, False), (8193, 14336, 4096, 3696, True),
