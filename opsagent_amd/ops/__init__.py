@@ -198,33 +198,32 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, form: int, gateup: bool = False,
 
 def _ring_plan(M: int, N: int, K: int, gateup: bool = False) -> Optional[Tuple[int, int]]:
     """(rows of a tile, column splits) of the product on the transfer ring
-    (ring_gemm.hip; figures there) of M rows of K columns against N (gate-up: 2N)
-    weight rows, None where the other forms are faster.
+    (ring_gemm.hip; figures there) in strips of 128 weight rows, of M rows of K columns against
+    N (gate-up: 2N) weight rows, None where these lines leave it to the other forms.
 
-    The lines, measured at 2 to 128 rows over 64 weights, 2 GB of them in turn (us,
-    other / ring): light weights end before the ring pays for its start (4096 x 4096,
-    M = 8 9.1 / 10.8, 24 13.4 / 11.7; gate-up 2 x 2816 x 2048, 24 10.6 / 10.7, 47
-    15.4 / 12.8, 112 16.7 / 17.8; but where two tiles of 64 rows fill the CUs 2 x 8192 x 640,
-    128 14.1 / 11.0, 2 x 4096 x 1408 18.9 / 16.5), short rows at few rows too (2 x 8192 x 2048, 8 14.5 /
-    14.7; 2 x 8192 x 3072 23.0 / 20.3), long ones less (2048 x 8192, 8 12.6 / 11.3).
-    Column splits fill the CUs; less than 0.8 of the last round filled loses (12288 x
-    4096, 24 22.7 / 25.0), and at two or three rows so does adding up many splits (4096 x
-    14336, 2 21.8 / 23.0). Runs of a multiple of 2048 columns, 4 KiB, keep all blocks on
-    the same channels: twice as many splits mend it up to 32 rows (16384 x 4096, M = 8, the
-    library 31.5, two splits 32.9, four 26.4; 8192 x 8192 29.3, 31.5, 25.8); above and for
-    gate-up the library is faster on weights of no fewer rows than columns (2 x 4096 x
-    8192, 8 31.6 / 33.0, four or eight splits; 8192 x 8192, 64 32.8 / 35.2; but 128 48.2 /
-    41.2, 4096 x 16384, 64 41.7 / 38.1). It also is for many rows on short wide weights
-    that need splits (8192 x 2048, 48 14.0 / 14.2; 8192 x 3072, 48 18.8 / 17.1, 80 19.7 /
-    20.9).
-    Up to 16 rows of 4096 the persistent skinny form is the better one where no
-    split is needed (2 x 14336, 8 45.2 / 45.4), under eight shorter rows the strips
-    (32000 x 2048, 4 26.6 / 29.4). Two tiles of 64 rows beat a tile of 128 under 64 MB of
-    weights and one of 96 under 32 MB (2048 x 8192, 80 16.7 / 15.9, 128 20.7 / 16.1; 2 x
-    3584 x 4096, 80 21.0 in one, 23.0 in two), as long as both read a strip in the same
-    round (32000 x 1024, 112 24.2 / 25.4). Without splits tiles of 96 pay in one round or
-    from rows of 4096 on (128256 x 2048, 96 130 / 132, 32000 x 2048 32.5 / 30.8, 128256 x
-    4096 228 / 225), tiles of 128 not at all (2 x 14336 x 4096, 58.0 / 59.5)."""
+    The lines were drawn at 2 to 128 rows over 64 weights, 2 GB of them in turn, when all strips
+    started together; _ring_form looks past them where strips apart are faster by its estimate.
+    What they go by, with today's us, best other form / this one: light weights end before the ring
+    pays for its start (4096 x 4096, M = 8 9.2 / 11.0, 24 13.3 / 12.1; gate-up 2 x 2816 x 2048, 24
+    10.7 / 11.3, 47 15.5 / 13.7, 112 17.0 / 16.2; but where two tiles of 64 rows fill the CUs 2 x
+    8192 x 640, 128 14.7 / 10.0, 2 x 4096 x 1408 19.1 / 14.0), short rows at few rows too (2 x
+    8192 x 2048, 8 15.4 / 15.9; 2 x 8192 x 3072 24.3 / 21.3), long ones less (2048 x 8192, 8 12.9 /
+    11.9). Column splits fill the CUs; unsplit, a round filled to less than 0.8 loses (12288 x 4096,
+    24 23.4 / 29.4, in two 21.9), and at two or three rows adding up many splits does (4096 x
+    14336, 2 23.2 / 23.8). Runs of a multiple of 2048 columns, 4 KiB, kept all blocks on the same
+    channels: twice as many splits mended it up to 32 rows, and above and for gate-up the library
+    was faster on weights of no fewer rows than columns. Apart that matters less (16384 x 4096, M = 8
+    30.3 / 26.9 in two splits, 28.2 in four; 8192 x 8192 30.7 / 30.2 in four, 27.3 in eight, 64 32.9 /
+    31.5, 128 48.3 / 37.2; 2 x 4096 x 8192, 8 30.0 / 29.2; 4096 x 16384, 64 42.2 / 35.0), and so do many
+    rows on short wide weights that need splits (8192 x 2048, 48 14.9 / 13.5; 8192 x 3072, 48 18.3 /
+    16.1, 80 19.3 / 18.6).
+    Up to 16 rows of 4096 the persistent skinny form was the better one where no split is needed
+    (2 x 14336, 8 47.5 / 39.9 now), under eight shorter rows the strips (32000 x 2048, 4 27.2 / 23.6
+    now). Two tiles of 64 rows beat a tile of 128 under 64 MB of weights and one of 96 under 32 MB
+    (us, one / two: 2048 x 8192, 80 16.9 / 16.5, 128 19.2 / 16.7; 2 x 3584 x 4096, 80 21.9 / 22.7), as
+    long as both read a strip in the same round (32000 x 1024, 112 18.1 / 24.5). Without splits
+    tiles of 96 pay in one round or from rows of 4096 on (128256 x 2048, 96 129 / 128, 32000 x 2048
+    35.0 / 27.9, 128256 x 4096 233 / 224); tiles of 128 did not (2 x 14336 x 4096, 62.7 / 53.6 now)."""
     if not 1 < M <= 128 or K % 64 or K < 256 or N % 8 or _two_rows_valu(M, N, K, gateup):
         return None
     weights = (2 if gateup else 1) * N * K
@@ -269,29 +268,29 @@ def _ring_narrow(M: int, N: int, K: int, gateup: bool, wide) -> Optional[int]:
     (ring_gemm.hip), None where strips of 128 (wide: their plan) or the other forms stay.
 
     What decides is, in this order, how full the CUs are, how many columns a split has, and what
-    the other form is. Measured over 190 weights, 150 of them drawn, at 3 to 64 rows, 0.7 GB of
-    them in turn, us other / narrow:
+    the other form is. Drawn from 190 weights, 150 of them random, at 3 to 64 rows, 0.7 GB of them in
+    turn, when all strips started together; today's us, other / narrow:
 
-    One round of half the blocks (12288 x 4096, M = 8 24.6 / 20.7 with 192), or rounds of 512
-    (gate-up 2 x 14336 x 4096, 8 46.1 / 39.4 with 448; 2 x 11008, 8 37.8 / 39.4 with 344), and
-    against strips of 128 that fill them better no fewer (2 x 2816 x 3520, 24 15.4 / 15.8 with
-    176). Weights under 10 MB end before it starts (2048 x 2048, 24 6.9 / 7.2); wide weights of
-    many splits run as fast in one deep ring (8192 x 28672, 32 74.4 / 80.5).
+    One round of half the blocks (12288 x 4096, M = 8 22.1 / 21.5 with 192), or rounds of 512
+    (gate-up 2 x 14336 x 4096, 8 39.9 / 40.7 with 448; 2 x 11008, 8 32.4 / 38.3 with 344), and
+    against strips of 128 that fill them better no fewer (2 x 2816 x 3520, 24 13.6 / 13.6 with
+    176). Weights under 10 MB end before it starts (2048 x 2048, 24 7.5 / 7.3); wide weights of
+    many splits run as fast in one deep ring (8192 x 28672, 32 79.4 / 78.6).
 
     Against strips of 128 in as many rounds it halves the splits or has none to add up: short
-    ones gain most (4096 x 4096, 24 12.0 / 10.4; 2 x 7704 x 1216, 24 .76 of the time). Above 32
+    ones gain most (4096 x 4096, 24 12.1 / 10.6; 2 x 7704 x 1216, 24 .73 of the time). Above 32
     rows eight waves a block carry those strips, and only splits of up to 1700 columns are better
-    here (4096 x 4096, 48 13.4 / 11.7; 4096 x 14336, 33 1.06 of the time; 7768 x 6208 1.13). Where
-    neither form splits it has nothing to save (28160 x 5632, 24 1.08, 48 1.16), but rows of 4 KiB
-    start on the same channels, which strips of half the height spread, wherever the weights lie
-    (32000 x 4096, 24 50.4 / 45.6, 48 49.5 / 46.7; 2 x 14336 x 4096, 32 on one card 40.3 / 41.2,
-    on another 48.4 / 42.8, inside a model 6 us more without). Splits of such a size start
-    together too, which more of them mend (8192 x 4096, 24 15.1 / 17.2; 4096 x 8192 16.9 / 18.0).
+    here (4096 x 4096, 48 13.8 / 12.3; 4096 x 14336, 33 1.04 of the time; 7768 x 6208 1.08). Where
+    neither form splits it has nothing to save (28160 x 5632, 24 1.11, 48 1.17); strips of 128 that
+    started together on rows of 4 KiB were the slower ones, which _ring_form knows they are no
+    longer (32000 x 4096, 24 41.7 / 41.8, 48 41.8 / 45.3; 2 x 14336 x 4096, 32 38.3 / 40.2). Splits of
+    such a size started together too (8192 x 4096, 24 15.4 / 14.3 in two, 15.0 in four; 4096 x 8192
+    17.3 / 16.8).
 
-    Strips of skinny.hip are the faster form of short rows: up to 16 rows (4096 x 4096, 8 9.1 /
-    9.8; 32000 x 2048, 6 27.8 / 29.0), up to 32 where columns of gate-up would be split (2 x 2560
-    x 1024, 24 1.35 of the time; 2 x 3072 x 1536 1.04) or rows of 4 KiB are cut to a few hundred
-    columns (3072 x 2048, 17 1.11, 24 1.01, 32 .93)."""
+    Strips of skinny.hip are the faster form of short rows: up to 16 rows (4096 x 4096, 8 9.2 /
+    10.1; but 32000 x 2048, 6 27.0 / 22.7 now), up to 32 where columns of gate-up would be split (2 x
+    2560 x 1024, 24 1.14 of the time; 2 x 3072 x 1536 1.01) or rows of 4 KiB are cut to a few hundred
+    columns (3072 x 2048, 17 1.10, 24 1.06, 32 .93)."""
     if not 2 < M <= (64 if wide is None else 48) or K % 64 or N % 8:
         return None
     weights = (2 if gateup else 1) * N * K
@@ -308,7 +307,7 @@ def _ring_narrow(M: int, N: int, K: int, gateup: bool, wide) -> Optional[int]:
         return None
     if gateup:
         if splits == 1 and K >= 3072 and weights >= 45e6:
-            ok = M <= (48 if K < 8192 else 32)       # 2 x 6144 x 12288, 40 1.03 of the time
+            ok = M <= (48 if K < 8192 else 32)       # 2 x 6144 x 12288, 40 1.16 of the time
         elif M <= 16:
             ok = wide is None and K >= 4096 and weights < 24e6
         else:
@@ -322,7 +321,7 @@ def _ring_narrow(M: int, N: int, K: int, gateup: bool, wide) -> Optional[int]:
         ok = K % (splits * 2048) != 0 and (K >= 5120 or K >= 3072 and weights >= 24e6)
     else:
         # the library is the best form of a square weight in one of its rounds (2560 x 2560, 48
-        # 1.07 of the time)
+        # 1.08 of the time)
         ok = K >= (2048 if M > 24 or weights >= 1e7 else 2049) and not (
             wide and K % (splits * 2048) == 0) and not (wide is None and K == N and 32 < M <= 48)
     return splits if ok else None
@@ -471,9 +470,10 @@ def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = Fa
     13195 of 13824 x 5120, 16 of 5632 short, 3038 / 2680). Over 113 products of 3000 to 16384 rows, 52 of
     them drawn, the choice is 0.5 per cent from the better of the two on average; many columns in
     part of a round lose up to 6 (5084 rows of 8424 x 9984, 1346 / 1266).
-    Over 3200 products of the models' weights and of 512 to 16000 x 512 to 14336, 129 to 6000 rows,
-    those taken are 1.17 times as fast as the library on average (gate-up 1.2), one in twenty up to
-    1.1 times slower. summed: for linear_parts, where a norm adds up the splits."""
+    570 plain products at 129 to 3500 rows, the models' weights and 210 drawn ones: 443 are taken,
+    1.12 times as fast as the library on average, 23 of them 3 per cent and more slower, two more than
+    10 (6144 x 4096, 286 rows 29.5 / 34.8); gate-up 1.2 times, none slower. summed: for linear_parts,
+    where a norm adds up the splits."""
     return _tile_sizes(M, N, K, gateup, summed) if M > 128 else None
 
 
@@ -1390,12 +1390,14 @@ def _prefill_plan(
     heads, 2 to 128 queries, 3 to 24 tiles) 0.2 per cent from the better of the two on average
     and 12 at the most (4 heads, 128 queries, 3 tiles, not split / split: 11.8 / 13.2; both
     sides: 80 heads, 128 queries, 6 tiles 18.2 / 25.8, 4 heads, 16 queries, 11 tiles 22.3 /
-    12.2). More queries: where few splits fill the chip, from as
-    many tiles as make up for the sums that they leave (16, 20 or 26, 34 and 70 tiles, not split
-    / in two, 32 heads on 8 of 700 to 1000 queries: 45 / 67, 55 / 74, 88 / 102, 183 / 175; in
-    three, 520 queries, 12 and 20 tiles: 36 / 42, 54 / 52; in four, 400 queries, 16 and 26
-    tiles: 35 / 40, 51 / 49, and 1000 queries of 16 heads, 26 and 34: 51 / 56, 64 / 65; in
-    six, 300 queries, 12 and 20 tiles: 26 / 30, 39 / 37)."""
+    12.2). More queries: where few splits fill the chip, from as many tiles as make up for the
+    sums that they leave, lines drawn with keys that the caches hold. Not split / split, and with
+    0.3 GB of keys in turn, 32 heads on 8 or 16 on 4: in two, 1000 queries of 32 heads and 50 and 64
+    tiles 134 / 139, 177 / 168 (163 / 147, 207 / 180); in three, 520 of 32, 16 and 20 tiles 43 / 45, 52 / 49
+    (47 / 46, 57 / 49); in four, 400 of 32, 24 and 28 46 / 45, 51 / 50 (57 / 47, 65 / 51), 1000 of 16, 28
+    and 34 52 / 54, 62 / 61 (65 / 53, 78 / 60); in five, 700 of 16, 16, 18 and 20 32 / 37, 35 / 38, 38 / 37
+    (41 / 38, 44 / 38, 48 / 38); in six, 300 of 32, 12, 16 and 20 26 / 29, 32 / 33, 38 / 37 (31 / 29, 40 / 33,
+    50 / 39). Keys from memory would draw them up to ten tiles, 15 per cent of a launch, lower."""
     splits, merged = _prefill_splits(B, Hq, Hk, Sq, Skv)
     if scaled:
         return splits, 2
@@ -1439,8 +1441,10 @@ def attention_prefill(
     rounding of a weight moves some of those to the next 8-bit value. ``slots``: [Skv],
     key i of the one sequence is row slots[i] of the caches k, v [rows, Hk, D], counted from the
     end below 0; the kernel reads them where they lie (us, two gathers and attention / here, 32 heads
-    on 8: 77 queries of 1264 keys 20.6 / 15.3, 800 of 1056 33.9 / 29.1, 2048 of 6144 215 / 204),
-    and takes the last row for a slot outside the caches (by its low 32 bits), which a gather faults on."""
+    on 8: 77 queries of 1264 keys 20.6 / 15.3, 800 of 1056 33.9 / 29.1, 2048 of 6144 215 / 204; whole
+    prompts of 5 to 2048 tokens behind 100 to 6000 0.90 to 1.0 of the time with gathers, but 16 heads on
+    4 and 1500 tokens or more behind 1800 1.007, 1500 behind 6000 1.02), and takes the last
+    row for a slot outside the caches (by its low 32 bits), where a gather has no answer."""
     if slots is not None and not (_is_gpu(q) and _rows_in_place(k, v, slots, q.shape[-1])):
         k, v, slots = k[slots], v[slots], None
         k, v = k.unsqueeze(0), v.unsqueeze(0)

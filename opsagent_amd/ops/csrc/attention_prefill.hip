@@ -87,8 +87,9 @@ __device__ __forceinline__ int cache_row(int slot, int rows) {
 // PAGED: the blocks of a key head, which share an XCD's L2, ask for up to four lines a lane of
 // all its keys and values while the first tile is under way: cache rows come from memory, and a
 // step of 1 to 2 us is less than its latency. `me` of `sharers` blocks; the caller waits. Four
-// layers of a model, us, gathered / from the cache / so: 1500 tokens behind 3000, 16 heads on
-// 4, 1222 / 1300 / 1242, 600 behind 1800, 32 on 8, 1430 / 1458 / 1426.
+// layers of a model, us, gathered / from the cache / so: 600 behind 1800, 32 heads on 8, 1430 / 1458 /
+// 1426; 1500 tokens behind 3000, 16 on 4, 1222 / 1300 / 1242, of the few that stay behind a gather (1500
+// behind 6000 1530 / - / 1562).
 constexpr int TOUCHES = 4;
 __device__ __forceinline__ void touch_rows(uint32_t (&t)[TOUCHES], const char* kbase, const char* vbase,
                                            const int64_t* slots, int rows, int64_t kstep, int64_t vstep,

@@ -90,7 +90,7 @@ def test_products(T, N, K):
     x = torch.randn(T, K, generator=g, device="cuda").bfloat16()
     w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).bfloat16()
     y = ops.linear_parts(x, w)
-    plan = 1 < T <= 128 and ops._ring_choice(T, N, K)
+    plan = 1 < T <= 128 and ops._ring_form(T, N, K)
     assert isinstance(y, ops.PlaneSum) == bool(plan and plan[1] > 1)
     if isinstance(y, ops.PlaneSum):
         total = y.planes[0].clone()
