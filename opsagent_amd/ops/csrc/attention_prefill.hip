@@ -950,7 +950,7 @@ extern "C" int oa_attention_prefill_variant(
     float* const po = nullptr;
     float* const pml = nullptr;
     switch (variant) {
-        case 1: case 3: case 5: case 7:  // the steady form, 128 rows
+        case 7:  // the steady form, 128 rows
             LAUNCH_STEADY(false, 1);
             break;
         case 10:  // two key groups, 128 rows
@@ -998,8 +998,8 @@ extern "C" int oa_attention_prefill(void* stream, const void* q, const void* k,
                                     int Hk, int Sq, int Skv, int D, float scale,
                                     int q_stride, int k_stride, int v_stride, int steady,
                                     const void* slots, int cache_rows) {
-    // OPSAGENT_PREFILL_VARIANT forces a variant (read per call so one
-    // process can A/B all variants).
+    // OPSAGENT_PREFILL_VARIANT (7 to 11, 9 where heads are shared) forces a variant
+    // (read per call so one process can A/B all variants).
     const char* e = getenv("OPSAGENT_PREFILL_VARIANT");
     int variant = e ? atoi(e) : 0;
     const int gq = (Hk > 0 && Hq % Hk == 0) ? Hq / Hk : 1;
