@@ -564,7 +564,9 @@ def attn_rope_rows(qkv: torch.Tensor, q_norm_w: torch.Tensor, k_norm_w: torch.Te
                    window: Optional[int] = None,
                    sinks: Optional[torch.Tensor] = None) -> torch.Tensor:
     """attn_rope_prepare and attention_paged of its queries, [T, H*Dv]; decode steps in one launch
-    (two with key splits) where the kernel for them takes the heads (mixers.hip)."""
+    (two with key splits) where the kernel for them takes the heads (mixers.hip). There a row's new
+    key is its own alone: no sequence of a step reads a slot that another one writes in it (pages are
+    shared when they are full)."""
     splits = 0
     # (the attributes first: most calls that are no such step end there)
     if (sb.max_chunk == 1 and qkv.is_cuda and qkv.dtype == torch.bfloat16 and D == Dv <= 128
