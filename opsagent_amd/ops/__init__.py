@@ -437,7 +437,7 @@ def _tile_sizes(M: int, N: int, K: int, gateup: bool, summed: bool) -> Optional[
     weights = N * K * (2 if gateup else 1)
     if summed and K < 2 * N:             # deep products split, others hardly
         return None
-    if weights < (2 ** 22 if gateup or summed or M >= 600 else 9e6) or (
+    if weights < (2 ** 22 if gateup or summed or M > 512 else 9e6) or (
             M >= 3500 and not gateup):
         return None
     if gateup and M > 4000 and M * weights >= 7.2e11:
@@ -453,8 +453,9 @@ def _tile_sizes(M: int, N: int, K: int, gateup: bool, summed: bool) -> Optional[
 def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = False) -> Optional[int]:
     """Form and column splits of the tile product (tile_gemm.hip; figures and the rule by sizes
     there) of more than 128 rows, None where the library is faster: light weights at few rows (us,
-    library / tiles: 2048 x 2048, 256 rows 10.1 / 13.0, 512 11.1 / 13.6, 800 15.3 / 14.5; 2560 x 2560,
-    542 15.6 / 17.0, 640 18.0 / 17.2; 3072 x 2048, 512 13.7 / 14.3, 638 17.1 / 16.3; deep ones with a norm behind
+    library / tiles: 2048 x 2048, 256 rows 10.1 / 13.0, 512 11.4 / 13.9, 599 13.6 / 14.0, 800 15.3 / 14.5;
+    2816 x 1664, 512 12.8 / 13.2, 550, where the library needs a tile of rows more, 16.7 / 12.8; 3072 x
+    2048, 512 15.3 / 16.2, 550 16.7 / 15.1; 2560 x 2560, 512 18.6 / 21.1, 599 20.8 / 19.9; deep ones with a norm behind
     them split, 1024 x 4096, 338 16.9 / 15.0), and from some thousand rows on, where power bounds
     both (4096 x 4096, 4067 92 / 103, 2900 79 / 78), but for gate-up, whose activation rides along.
     So do products that would run in whole tiles of 256 x 256, the library's own form and faster

@@ -106,8 +106,7 @@ def test_whole_tiles_of_the_library():
 
 def test_light_weights():
     for N, K in ((2048, 2048), (2560, 2560), (3072, 2048), (2048, 2816)):
-        assert ops._tile_choice(512, N, K) is None and ops._tile_choice(599, N, K) is None
-        assert ops._tile_choice(640, N, K) is not None
+        assert ops._tile_choice(512, N, K) is None and ops._tile_choice(513, N, K) is not None
     assert ops._tile_choice(512, 2816, 2048, gateup=True) is not None
     assert ops._tile_choice(512, 2048, 8192) is not None
 
