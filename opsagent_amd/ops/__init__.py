@@ -390,7 +390,8 @@ def _ring_fastest(M: int, N: int, K: int, gateup: bool):
     us, *form = min(forms)
     plan = _ring_choice(M, N, K, gateup)
     if plan:
-        return tuple(form) if us < 0.97 * _ring_us(M, N, K, gateup, *plan) else plan
+        full = gateup and plan[0] == 128 and form == [64, 1, False] and N > 64 * 112
+        return tuple(form) if us < (0.9 if full else 0.97) * _ring_us(M, N, K, gateup, *plan) else plan
     stream = N * (1 + gateup) * K * 2 / 6.2e6 + 3.0
     near = 1.3 if M > 32 and not form[2] else 1.2
     return tuple(form) if K >= (1536 if M <= 16 else 1024) and us < near * stream else None
@@ -408,7 +409,13 @@ def _ring_form(M: int, N: int, K: int, gateup: bool = False):
     weights at 6.2 TB/s; skinny.hip is the better one for up to 16 short rows (2 x 25088 x 1024, 3
     19.8 / 22.5). us, _ring_choice's form or the others / here: gate-up 2 x 14336 x 4096, M = 47 44.2
     / 38.1, 128 58.3 / 48.2; 32000 x 4096, 47 48.5 / 41.5, 112 76.6 / 51.8; 20288 x 1664, 16 41.5 /
-    15.2; 12584 x 3520, 40 32.7 / 21.6; but 2 x 5632 x 2048, 48 14.2 / 15.7."""
+    15.2; 12584 x 3520, 40 32.7 / 21.6; but 2 x 5632 x 2048, 48 14.2 / 15.7.
+
+    Two tiles of 64 gate-up rows on more than 224 of the CUs take up to 15 per cent longer than it
+    says; against splits of 128-row tiles, as full, they have to be 10 per cent ahead (us, splits
+    / two tiles: 2 x 7552 x 3648, M = 103 34.4 / 37.7, 2 x 8128 x 4160, 128 39.3 / 44.7, 2 x 8192 x
+    4032, 112 37.0 / 41.7; on fewer CUs 2 x 6720 x 3264, 128 35.2 / 32.7, 2 x 7040 x 3264 35.7 /
+    33.3; far ahead 2 x 8192 x 2048, 128 23.0 / 20.9)."""
     return _ring_choice(M, N, K, gateup) if M == 2 else _ring_fastest(M, N, K, gateup)
 
 

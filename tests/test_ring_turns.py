@@ -52,3 +52,12 @@ def test_forms():
                     if plan:
                         assert plan[0] in (32, 64, 96, 128) and 1 <= plan[1] <= K // 64
                         assert not plan[2] or plan[0] <= 64
+
+
+def test_full_rounds():
+    """Gate-up in two tiles of 64 rows that fill the CUs: only where the estimate is far ahead of the
+    splits of 128-row tiles, which answer sooner than it knows."""
+    for M, N, K in ((103, 7552, 3648), (128, 8128, 4160), (112, 8192, 4032)):
+        assert ops._ring_form(M, N, K, True) == ops._ring_choice(M, N, K, True) == (128, 2, False)
+    for M, N, K in ((128, 6720, 3264), (128, 7040, 3264), (128, 8192, 2048)):
+        assert ops._ring_form(M, N, K, True) == (64, 1, False)
