@@ -454,6 +454,9 @@ def _tile_sizes(M: int, N: int, K: int, gateup: bool, summed: bool) -> Optional[
     plan = _lib()[0].oa_tile_gemm_plan(M, N, K, int(gateup), int(summed))
     if plan < 0 or plan == 1 and K >= 2048 and not gateup:       # tiles of 256 x 256, unsplit
         return None
+    tile = {3 * 256 + 1: (160, 256), 4 * 256 + 1: (256, 128)}.get(plan)          # unsplit
+    if tile and 2048 <= K <= 8192 and not gateup and -(-M // tile[0]) * -(-N // tile[1]) <= 192:
+        return None                      # a quarter of the CUs and more idle
     return plan
 
 
@@ -468,7 +471,12 @@ def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = Fa
     So do products that would run in whole tiles of 256 x 256, the library's own form and faster
     there (8192 x 4096, 2048 rows 93 / 101; 16384 x 2048, 922 53 / 53, 1966 99 / 105, 2987 156 / 170; 14336 x
     4096, 1024 89 / 94, 2092 180 / 194; 10240 x 8192, 3072 337 / 358), but for short rows, where it is
-    not (10296 x 640, 1430 35 / 23).
+    not (10296 x 640, 1430 35 / 23). And tiles of 160 x 256 and 256 x 128 that leave a quarter of the
+    CUs idle: of 340 such products of 2048 to 8192 columns, on two cards, three in four were 3 per cent
+    and more slower, 1.05 times on average, and one in 25 faster (12288 x 4096, 514 61 / 68, 640 63 /
+    70, 486 57 / 58; 11072 x 5760, 517 87 / 92; 16640 x 3648, 315 61 / 66). With 193 tiles and more
+    they are ahead again, by 5 per cent, and on rows of 12000 columns the library is up to 1.5 times
+    slower (17856 x 12736, 279 293 / 191).
     Of gate-up the largest of more than 4000 rows go there where columns are many (library and
     activation / tiles: 8000 rows of 4096 x 14336 1281 / 1371, 8192 of 7168 x 8192 1315 / 1385, 16000 of
     28672 x 8192 10213 / 10959, 9395 of 16848 x 13952 6023 / 6735; smaller ones not, 5500 of 4096 x 14336

@@ -111,6 +111,20 @@ def test_light_weights():
     assert ops._tile_choice(512, 2048, 8192) is not None
 
 
+def test_idle_units():
+    """Plain products in 192 unsplit tiles and fewer of 160 x 256 or 256 x 128 are the library's, but
+    for rows out of 2048 to 8192 columns."""
+    plan = ops._lib()[0].oa_tile_gemm_plan
+    for M, N, K, form, tiles, taken in ((640, 12288, 4096, 3, 192, False), (514, 12288, 4096, 3, 192, False),
+                                        (486, 12288, 4096, 4, 192, False), (517, 11072, 5760, 3, 176, False),
+                                        (640, 13056, 4096, 3, 204, True), (514, 12288, 1984, 3, 192, True),
+                                        (279, 17856, 12736, 3, 140, True)):
+        rows, cols = ((160, 256), (256, 128))[form - 3]
+        assert plan(M, N, K, 0, 0) == form * 256 + 1 and -(-M // rows) * -(-N // cols) == tiles
+        assert (ops._tile_choice(M, N, K) is not None) == taken
+    assert ops._tile_choice(514, 6144, 4096, gateup=True) is not None
+
+
 def test_rounds_of_the_library():
     """Large gate-up products: the library's where its tiles of 256 x 256 fill every round."""
     for M, N, K, blocks, taken in ((8192, 14336, 4096, 14 * 256, False), (8193, 14336, 4096, 3696, True),
