@@ -439,6 +439,12 @@ def _ring(x: torch.Tensor, w: torch.Tensor, plan: Tuple[int, ...], act: int = 0,
     return part if parts else out
 
 
+# unsplit plans that leave CUs idle, to the library's gain: rows and weight rows of a tile, up to how
+# many tiles, and whether only above 256 rows of whole steps of 128 columns, the library's
+_TILES_IDLE = {3 * 256 + 1: (160, 256, 192, False), 4 * 256 + 1: (256, 128, 192, False),
+               8 * 256 + 1: (96, 128, 153, True), 9 * 256 + 1: (128, 64, 192, True)}
+
+
 @functools.lru_cache(maxsize=4096)
 def _tile_sizes(M: int, N: int, K: int, gateup: bool, summed: bool) -> Optional[int]:
     weights = N * K * (2 if gateup else 1)
@@ -454,9 +460,10 @@ def _tile_sizes(M: int, N: int, K: int, gateup: bool, summed: bool) -> Optional[
     plan = _lib()[0].oa_tile_gemm_plan(M, N, K, int(gateup), int(summed))
     if plan < 0 or plan == 1 and K >= 2048 and not gateup:       # tiles of 256 x 256, unsplit
         return None
-    tile = {3 * 256 + 1: (160, 256), 4 * 256 + 1: (256, 128)}.get(plan)          # unsplit
-    if tile and 2048 <= K <= 8192 and not gateup and -(-M // tile[0]) * -(-N // tile[1]) <= 192:
-        return None                      # a quarter of the CUs and more idle
+    rows, cols, most, even = _TILES_IDLE.get(plan, (0, 0, 0, False))
+    if most and 2048 <= K <= 8192 and not gateup and -(-M // rows) * -(-N // cols) <= most and not (
+            even and (K % 128 or M <= 256)):
+        return None
     return plan
 
 
@@ -476,7 +483,12 @@ def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = Fa
     and more slower, 1.05 times on average, and one in 25 faster (12288 x 4096, 514 61 / 68, 640 63 /
     70, 486 57 / 58; 11072 x 5760, 517 87 / 92; 16640 x 3648, 315 61 / 66). With 193 tiles and more
     they are ahead again, by 5 per cent, and on rows of 12000 columns the library is up to 1.5 times
-    slower (17856 x 12736, 279 293 / 191).
+    slower (17856 x 12736, 279 293 / 191). Above 256 rows tiles of 128 x 64 with as many idle and of 96 x
+    128 with two in five go there too, where rows are whole steps of 128 columns (6144 x 4096, 262
+    30.1 / 33.9, 283 30.4 / 35.2; 2048 x 2816, 514 17.1 / 18.5, 661 17.3 / 19.0; 2048 x 2048, 521 13.4 /
+    14.6, 752 14.1 / 15.0; of 330 on two cards three in four 3 per cent and more slower, 1.06 times on
+    average, one in 25 faster): half a step over costs the library a quarter (6144 x
+    3136, 268 31.4 / 27.9).
     Of gate-up the largest of more than 4000 rows go there where columns are many (library and
     activation / tiles: 8000 rows of 4096 x 14336 1281 / 1371, 8192 of 7168 x 8192 1315 / 1385, 16000 of
     28672 x 8192 10213 / 10959, 9395 of 16848 x 13952 6023 / 6735; smaller ones not, 5500 of 4096 x 14336
@@ -486,10 +498,11 @@ def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = Fa
     13195 of 13824 x 5120, 16 of 5632 short, 3038 / 2680). Over 113 products of 3000 to 16384 rows, 52 of
     them drawn, the choice is 0.5 per cent from the better of the two on average; many columns in
     part of a round lose up to 6 (5084 rows of 8424 x 9984, 1346 / 1266).
-    570 plain products at 129 to 3500 rows, the models' weights and 210 drawn ones: 443 are taken,
-    1.12 times as fast as the library on average, 23 of them 3 per cent and more slower, two more than
-    10 (6144 x 4096, 286 rows 29.5 / 34.8); gate-up 1.2 times, none slower. summed: for linear_parts,
-    where a norm adds up the splits."""
+    Of 33110 plain products at 129 to 3500 rows, 3000 weights but 19 of them drawn, 22300 are taken, 1.2
+    times as fast as the library on average (1.16 on whole steps of 128 columns), 4 in 100 of them 3 per
+    cent and more slower, 6 in 1000 more than 10 (16704 x 5120, 283 rows 81 / 98: three row tiles of
+    96 in a round and a half); gate-up 1.2 times, hardly one slower. summed: for linear_parts, where a
+    norm adds up the splits."""
     return _tile_sizes(M, N, K, gateup, summed) if M > 128 else None
 
 

@@ -105,21 +105,27 @@ def test_whole_tiles_of_the_library():
 
 
 def test_light_weights():
-    for N, K in ((2048, 2048), (2560, 2560), (3072, 2048), (2048, 2816)):
+    for N, K in ((2560, 2560), (3072, 2048)):
         assert ops._tile_choice(512, N, K) is None and ops._tile_choice(513, N, K) is not None
+    for N, K in ((2048, 2048), (2048, 2816)):          # 192 tiles up to 768 rows (test_idle_units)
+        assert ops._tile_choice(768, N, K) is None and ops._tile_choice(769, N, K) is not None
     assert ops._tile_choice(512, 2816, 2048, gateup=True) is not None
     assert ops._tile_choice(512, 2048, 8192) is not None
 
 
 def test_idle_units():
-    """Plain products in 192 unsplit tiles and fewer of 160 x 256 or 256 x 128 are the library's, but
-    for rows out of 2048 to 8192 columns."""
+    """Plain products in 192 unsplit tiles and fewer of 160 x 256, 256 x 128 or, with whole steps of the
+    library's above 256 rows, 128 x 64 (153 and fewer of 96 x 128) are the library's, but for rows
+    out of 2048 to 8192 columns."""
     plan = ops._lib()[0].oa_tile_gemm_plan
     for M, N, K, form, tiles, taken in ((640, 12288, 4096, 3, 192, False), (514, 12288, 4096, 3, 192, False),
                                         (486, 12288, 4096, 4, 192, False), (517, 11072, 5760, 3, 176, False),
                                         (640, 13056, 4096, 3, 204, True), (514, 12288, 1984, 3, 192, True),
-                                        (279, 17856, 12736, 3, 140, True)):
-        rows, cols = ((160, 256), (256, 128))[form - 3]
+                                        (279, 17856, 12736, 3, 140, True), (283, 6144, 4096, 8, 144, False),
+                                        (268, 6144, 3136, 8, 144, True), (283, 6656, 4096, 8, 156, True),
+                                        (700, 2048, 2816, 9, 192, False), (700, 2048, 2752, 9, 192, True),
+                                        (250, 6144, 4096, 9, 192, True), (800, 2048, 2816, 9, 224, True)):
+        rows, cols = {3: (160, 256), 4: (256, 128), 8: (96, 128), 9: (128, 64)}[form]
         assert plan(M, N, K, 0, 0) == form * 256 + 1 and -(-M // rows) * -(-N // cols) == tiles
         assert (ops._tile_choice(M, N, K) is not None) == taken
     assert ops._tile_choice(514, 6144, 4096, gateup=True) is not None
