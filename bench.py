@@ -1,20 +1,20 @@
-"""Flagship serving benchmark — BASELINE.json metric: agent-turn latency +
+"""Flagship serving benchmark — agent-turn latency and
 tool-call JSON validity %, synthetic k8s-state prompts, random-init weights.
 
-Modes (BASELINE configs):
-  turn        (default, config #2/#4): one "step" = one agent turn — prefill a
+Modes:
+  turn        (default) one "step" = one agent turn — prefill a
               synthetic analyze-pod prompt (shared ~250-token system prefix +
               fresh per-turn observation body) + decode a grammar-constrained
               ToolPrompt JSON reply.
-  multiturn   (config #3): one conversation; each step appends a synthetic
+  multiturn   one conversation; each step appends a synthetic
               tool observation and decodes the next ToolPrompt — the paged-KV
               prefix cache makes each iteration prefill only the new suffix.
-  concurrent  (config #5): C concurrent sessions submit turns to the engine
+  concurrent  C concurrent sessions submit turns to the engine
               loop (continuous batching, one hipGraph replay per token for
               the whole batch); value is still per-turn p50 latency and
               throughput is reported in config.
 
-Contract (driver): `python bench.py --gpus N --steps K --warmup W`; for N>1
+Contract: `python bench.py --gpus N --steps K --warmup W`; for N>1
 launched under torch.distributed.run with one rank per GPU (TP=N over RCCL).
 W untimed warmup steps, then EXACTLY K timed steps bracketed by barrier +
 torch.cuda.synchronize on both sides; MAX over ranks; rank 0 prints ONE JSON

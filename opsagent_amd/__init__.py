@@ -12,7 +12,7 @@ OpenAI-compatible endpoint) as an MI355X-first framework:
     tensor parallelism over RCCL/xGMI — replacing the reference's network
     boundary at `pkg/llms/openai.go:69`.
 
-Layer map (mirrors SURVEY.md §1):
+Layer map:
   cli.py / server/     — front ends              (ref: cmd/, pkg/api, pkg/handlers)
   agent/               — ReAct core + workflows  (ref: pkg/assistants, pkg/workflows)
   llm/                 — OpenAI-compatible client (ref: pkg/llms)

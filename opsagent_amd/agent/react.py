@@ -1,6 +1,6 @@
 """ReAct agent core.
 
-Capability parity with /root/reference/pkg/assistants/simple.go:287-616:
+Capability parity with pkg/assistants/simple.go:287-616:
 
   * `assistant(...)` sends the conversation, parses the reply into a
     ToolPrompt (question/thought/action/observation/final_answer), and
@@ -19,7 +19,7 @@ Capability parity with /root/reference/pkg/assistants/simple.go:287-616:
 MI355X note: when the client is the LocalEngineClient, each `chat` call hits
 the in-process engine, which caches the KV prefix of the growing conversation
 across iterations (prefix reuse), so ReAct iterations pay only for the new
-tokens — the agent-turn-latency lever named in SURVEY.md §2b.
+tokens — what agent-turn latency depends on most.
 """
 
 from __future__ import annotations

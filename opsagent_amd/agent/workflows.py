@@ -2,10 +2,10 @@
 
 The reference delegates analyze/audit/generate/format to the external
 swarm-go library (OpenAI-native function-calling agents,
-/root/reference/pkg/workflows/*.go via SimpleFlow.Run). Here the same flows
+pkg/workflows/*.go via SimpleFlow.Run). Here the same flows
 run on a native function-calling loop against any LLMClient — including the
 in-process MI355X engine, whose grammar-constrained sampler emits tool_calls
-in the same OpenAI wire format (SURVEY.md §2b "hard part (e)").
+in the same OpenAI wire format.
 
 Flows (ref files):
   analysis_flow   — pkg/workflows/analyze.go:47  (kubectl tool, MaxTurns 30)
@@ -13,7 +13,7 @@ Flows (ref files):
   generator_flow  — pkg/workflows/generate.go:56 (no tools)
   assistant_flow  — pkg/workflows/assistant.go:69 (formatting; the reference
                     buggily reuses the analysis prompt there — we use a real
-                    formatting prompt, per SURVEY.md "known inconsistencies")
+                    formatting prompt)
 """
 
 from __future__ import annotations

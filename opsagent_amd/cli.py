@@ -1,11 +1,10 @@
 """CLI front-end.
 
-Capability parity with /root/reference/cmd/kube-copilot/: subcommands
+Capability parity with cmd/kube-copilot/: subcommands
 execute, analyze, audit, diagnose, generate, serve(r), version, with the
 persistent flags --model --max-tokens --count-tokens --verbose
 --max-iterations (ref main.go:28-32). Unlike the reference snapshot — which
-registers only `server` on the root command (main.go:34, a known bug per
-SURVEY.md §1) — every subcommand here is wired.
+registers only `server` on the root command (main.go:34) — every subcommand here is wired.
 
 Entry point: `python -m opsagent_amd.cli <command>` or the `opsagent` script.
 """

@@ -1,10 +1,10 @@
 """Configuration system.
 
-Keeps the reference's `config.yaml` layout (ref /root/reference/configs/
+Keeps the reference's `config.yaml` layout (ref configs/
 config.yaml:1-20 and pkg/utils/config.go:10-53: jwt.key/expire, server.port/
 host, log.level/format/output, perf.enabled/reset_interval) and adds the
 `engine:` section for the in-process MI355X inference engine (model, dtype,
-tensor-parallel degree, KV budget, grammar mode) per SURVEY.md §5.
+tensor-parallel degree, KV budget, grammar mode).
 
 Search order mirrors the reference: ./configs/config.yaml then ./config.yaml,
 then coded defaults. Env overrides: OPSAGENT_<SECTION>_<KEY>.

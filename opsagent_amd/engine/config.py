@@ -1,7 +1,7 @@
 """Model architecture registry.
 
-Llama-3 family dims (8B / 70B per BASELINE.json configs #2-#4), a tiny config
-for CPU tests, and DeepSeek-V3-style MoE configs (BASELINE config #5). Random
+Llama-3 family dims (8B / 70B), a tiny config
+for CPU tests, and DeepSeek-V3-style MoE configs. Random
 initialization is the benchmark mode (no network for checkpoints); safetensors
 loading is supported for real weights.
 """
@@ -41,7 +41,7 @@ class ModelSpec:
 
 
 MODEL_REGISTRY = {
-    # Llama-3 8B (BASELINE configs #2/#3)
+    # Llama-3 8B
     "llama3-8b": ModelSpec(
         name="llama3-8b",
         hidden_size=4096,
@@ -50,7 +50,7 @@ MODEL_REGISTRY = {
         num_heads=32,
         num_kv_heads=8,
     ),
-    # Llama-3 70B (BASELINE config #4, TP=8)
+    # Llama-3 70B (TP=8)
     "llama3-70b": ModelSpec(
         name="llama3-70b",
         hidden_size=8192,
@@ -141,7 +141,7 @@ MODEL_REGISTRY = {
         moe_shared_experts=1,
     ),
     # DeepSeek-V3-style MoE, scaled down to fit one MI355X comfortably
-    # (BASELINE config #5: fp8 experts on CDNA4 MFMA)
+    # (fp8 experts on CDNA4 MFMA)
     "deepseek-moe-small": ModelSpec(
         name="deepseek-moe-small",
         vocab_size=128256,

@@ -2,7 +2,7 @@
 reuse, hipGraph-captured decode, grammar-constrained sampling.
 
 This is the in-process replacement for the reference's remote LLM boundary
-(/root/reference/pkg/llms/openai.go:69 — an HTTPS call per ReAct iteration).
+(pkg/llms/openai.go:69 — an HTTPS call per ReAct iteration).
 Architecture:
 
   * one process per GPU; TP over RCCL/xGMI (parallel/state.py). Rank 0 drives
@@ -12,7 +12,7 @@ Architecture:
   * step() = (at most one) chunked prefill OR one batched decode step over
     all running sequences. Decode steps replay a hipGraph captured per batch
     bucket (1,2,4,...,max_batch) — launch-bound decode loops become one
-    graph replay (SURVEY.md §2b).
+    graph replay.
   * sampling: grammar FSM (C++) emits an allowed-token bitmask per sequence;
     the fused HIP kernel masks+argmaxes the logits on-GPU. Temperature
     sampling adds host-side Gumbel noise before the same kernel.

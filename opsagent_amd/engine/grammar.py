@@ -4,7 +4,7 @@ Per-sequence constrained-decoding state: each decode step `fill_mask` writes
 the allowed-token bitmask (pinned int32 tensor), which is uploaded to the GPU
 and fused into the sampling kernel (ops.greedy_sample_masked). Invalid JSON
 becomes unrepresentable — replacing the reference's post-hoc JSON repair
-(/root/reference/pkg/utils/json.go:16-190).
+(pkg/utils/json.go:16-190).
 """
 
 from __future__ import annotations

@@ -1,8 +1,8 @@
 """Paged KV cache manager with block-level prefix caching.
 
-SURVEY.md §2b: "hipGraph-captured decode step, re-used across multi-turn
-ReAct iterations — the loop at simple.go:394-615 re-sends full history each
-turn; persistent KV across tool-call turns = the agent-turn-latency lever."
+The hipGraph-captured decode step is re-used across multi-turn ReAct iterations:
+the loop at simple.go:394-615 re-sends full history each turn, and agent-turn
+latency depends on KV that persists across tool-call turns.
 
 Mechanism: the cache is a pool of fixed-size token blocks
 ([num_blocks, block_size, Hk_local, D] bf16 per layer, sized against the

@@ -1,6 +1,6 @@
 """Weight checkpoint load/save (safetensors).
 
-The benchmark mode is random-init (no network for checkpoints — BASELINE),
+The benchmark mode is random-init (no network for checkpoints),
 but the engine supports real weights: a canonical full-weight safetensors
 layout (written by `save_weights` at TP=1) and HuggingFace Llama naming
 ("model.layers.N.self_attn.q_proj.weight", ...). Loading is TP-aware: every

@@ -1,13 +1,12 @@
 """Llama-3-family model with tensor parallelism, built on the ops dispatch
 layer (HIP kernels on GPU, torch_ref on CPU).
 
-Replaces the reference's remote model layer (SURVEY.md §2b). Weight layout is
+Replaces the reference's remote model layer. Weight layout is
 fused and token-major throughout — activations are [T, hidden]; attention
 tensors [T, H, D] (no [B, H, S, D] transposes; the HIP kernels take the
 token-major layout directly).
 
-TP sharding (SURVEY.md §2b "TP sharding (row/col-parallel linear,
-head-parallel attention)"): QKV and gate/up are column-parallel, o and down
+TP sharding (row/col-parallel linear, head-parallel attention): QKV and gate/up are column-parallel, o and down
 are row-parallel with one RCCL all-reduce each per layer; heads are divided
 across ranks (Hq % tp == 0 and Hk % tp == 0). Random init draws the FULL
 weight with a fixed seed on every rank and slices the local shard, so TP=k is

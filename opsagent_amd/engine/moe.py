@@ -1,4 +1,4 @@
-"""DeepSeek-V3-style Mixture-of-Experts MLP (BASELINE config #5).
+"""DeepSeek-V3-style Mixture-of-Experts MLP.
 
 Routing: softmax top-k over a router linear, normalized weights, plus
 `moe_shared_experts` always-on shared experts (DeepSeek style). Experts are

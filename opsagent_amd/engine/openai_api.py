@@ -1,7 +1,7 @@
 """OpenAI chat-completions + function-calling API over the local engine.
 
 The wire format matches what the reference's Go client and swarm-style flows
-expect (SURVEY.md hard part (e)): request {model, messages, max_tokens,
+expect: request {model, messages, max_tokens,
 tools?, temperature?, response_format?} → response {choices: [{message:
 {role, content, tool_calls?}, finish_reason}], usage}.
 

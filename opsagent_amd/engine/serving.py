@@ -1,7 +1,7 @@
 """Background engine loop for concurrent serving (continuous batching).
 
-The reference handles HTTP concurrency in gin only (SURVEY.md §2b
-"Continuous batching / concurrent request scheduler" is vacant). Here a
+The reference handles HTTP concurrency in gin only, with no
+continuous batching or request scheduler. Here a
 single loop thread owns the LLMEngine (which is not thread-safe); callers
 submit prompts from any thread and get a Future. Requests that arrive while
 a batch is decoding join the running batch at the next engine step — one
@@ -22,8 +22,8 @@ log = get_logger("serving")
 
 
 class EngineLoop:
-    """Owns the engine thread; also the engine watchdog (SURVEY.md §5
-    "failure detection ... engine watchdog for hung kernels/collectives"):
+    """Owns the engine thread; also the engine watchdog, for hung kernels
+    and collectives:
     a monitor thread flags the loop unhealthy when one engine step exceeds
     `watchdog_s` (a hung kernel or collective blocks the step forever —
     /api/health then reports engine: "unhealthy" so orchestration can

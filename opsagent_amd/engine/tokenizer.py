@@ -32,8 +32,7 @@ class ByteTokenizer:
     """ids 0..255 = bytes; 256.. = special tokens.
 
     `template` selects the chat rendering: "llama3" (header-id turns) or
-    "deepseek" (User:/Assistant: turns with <|end_of_text|> separators) —
-    SURVEY.md §2b "Tokenizer + chat templating: Llama-3 / DeepSeek templates".
+    "deepseek" (User:/Assistant: turns with <|end_of_text|> separators).
     """
 
     byte_level_ids = True  # ids 0..255 ARE output bytes (fast paths rely on it)

@@ -1,6 +1,6 @@
 """Kubernetes helpers.
 
-Capability parity with /root/reference/pkg/kubernetes/ (GetKubeConfig
+Capability parity with pkg/kubernetes/ (GetKubeConfig
 apply.go:24, GetYaml get.go:30, ApplyYaml apply.go:38). The reference uses
 client-go; here we use the kubectl binary (already a hard dependency of the
 kubectl tool), honoring in-cluster service accounts and ~/.kube/config the

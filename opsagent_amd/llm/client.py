@@ -1,7 +1,7 @@
 """LLM client layer — the boundary the MI355X engine replaces.
 
 The reference's model layer is an HTTPS call to a remote OpenAI-compatible
-endpoint with retry/backoff (/root/reference/pkg/llms/openai.go:29-104). Here
+endpoint with retry/backoff (pkg/llms/openai.go:29-104). Here
 the same `chat()` interface has three implementations:
 
   * LocalEngineClient — the in-process MI355X inference engine
@@ -11,8 +11,7 @@ the same `chat()` interface has three implementations:
   * RemoteOpenAIClient — parity with the reference: POST /chat/completions
     with 5 retries, 1 s base exponential backoff on 429/5xx, fail-fast on 401
     (ref openai.go:58-101), Azure detection by "azure" in base_url.
-  * ScriptedLLM — deterministic canned replies for hermetic agent tests
-    (BASELINE config #1: stub echo-LLM).
+  * ScriptedLLM — deterministic canned replies for hermetic agent tests.
 
 All return an OpenAI-shaped assistant message dict:
   {"role": "assistant", "content": str|None, "tool_calls": [...]|None}

@@ -1,6 +1,6 @@
 """Token budgeting utilities.
 
-Capability parity with /root/reference/pkg/llms/tokens.go:26-144:
+Capability parity with pkg/llms/tokens.go:26-144:
 per-model context-length table, token counting with per-message overhead,
 `constrict_messages` (drop oldest non-system messages until the budget fits),
 and `constrict_prompt` (drop the first third of lines until under the limit).

@@ -1,5 +1,5 @@
 """Build the HIP kernel library for gfx950 (MI355X) — in-tree, so the .so
-travels with the repo snapshot to GPU boxes.
+travels with the tree to machines with a GPU.
 
 Usage: python -m opsagent_amd.ops.build [--check]
 Called by __graft_entry__.build().

@@ -1,5 +1,5 @@
-// FP8 (OCP e4m3) expert-GEMM path for MoE on MI355X — SURVEY.md §2b "GEMM
-// path: ... custom fp8 MFMA for MoE experts".
+// FP8 (OCP e4m3) expert-GEMM path for MoE on MI355X: fp8 matrix instructions
+// of its own for the experts.
 //
 // gfx950 fp8 is OCP e4m3fn (NOT MI300X fnuz — CDNA guide §4). Weights are
 // quantized per output row (scale = absmax/448); activations per token.

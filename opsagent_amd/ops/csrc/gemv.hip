@@ -606,7 +606,7 @@ extern "C" int oa_gemv(void* stream, const void* x, const void* w, void* out,
     return oa_gemv_ex(stream, x, w, out, nullptr, nullptr, M, N, K, 0.0f, 0);
 }
 
-// RW=4 probe variant (within-probe A/B only — guide rule 24)
+// RW=4 probe variant (within-probe A/B only)
 extern "C" int oa_gemv_rw4(void* stream, const void* x, const void* w, void* out,
                            int M, int N, int K) {
     if (K % 8 != 0) return -100;

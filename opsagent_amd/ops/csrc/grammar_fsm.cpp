@@ -1,6 +1,6 @@
 // Byte-level JSON grammar FSM for constrained decoding (CPU, C++).
 //
-// the reference repairs invalid LLM JSON after the fact
+// The reference repairs invalid LLM JSON after the fact
 // (pkg/utils/json.go:16-190 CleanJSON/ExtractField); this FSM makes invalid
 // JSON impossible instead: each decode step it computes an allowed-token
 // bitmask over the vocabulary which the GPU sampling kernel

@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256) void moe_emaj_kernel(
         for (int g0 = 0; g0 < cnt; g0 += EMAJ_GROUP) {
             const int m = min(EMAJ_GROUP, cnt - g0);
             // all register arrays are indexed by the UNROLLED c only (a
-            // runtime index would demote them to scratch — guide rule 20)
+            // runtime index would demote them to scratch)
             float accg[EMAJ_GROUP], accu[EMAJ_GROUP];
             const uint32_t* xbase[EMAJ_GROUP];
 #pragma unroll

@@ -5,8 +5,6 @@
 // are precomputed on the HOST ([max_seq, D/2] f32) — on-device sinf/cosf
 // turns a memory-bound op VALU-bound (guide: 16% of HBM BW). Loads are
 // vectorized (4 bf16 = 8 B per half, plus 16 B of f32 table per lane).
-//
-// Replaces SURVEY.md §2b "RoPE kernel".
 
 #include "common.h"
 

@@ -5,7 +5,7 @@ per the MI355X-first design). Launch functions take raw device pointers plus
 the current torch HIP stream, so they compose with torch allocations and
 hipGraph capture (torch.cuda.graphs).
 
-Policy (per driver contract): on a GPU box the HIP library is REQUIRED — ops
+Policy: on a GPU machine the HIP library is REQUIRED — ops
 fail loudly if it is missing rather than silently falling back to eager
 PyTorch. CPU runs use opsagent_amd.ops.torch_ref.
 """

@@ -1,10 +1,10 @@
 """Pure-PyTorch reference implementations of the engine's hot ops.
 
 These are the numerics oracle for the HIP/CDNA4 kernels (tests compare the
-HIP kernel against these in fp32 — SURVEY.md §4 test strategy (c)) and the
+HIP kernel against these in fp32) and the
 CPU execution path. They are intentionally simple and readable; the GPU path
 never runs these (opsagent_amd.ops dispatch raises if the HIP extension is
-missing on a GPU box).
+missing on a machine with a GPU).
 """
 
 from __future__ import annotations

@@ -6,7 +6,7 @@ decode's small hidden-size messages (8-16 KB at batch 1) it is pure latency:
 2*(n-1) dependent hops. The one-shot form — every rank broadcasts its shard
 to all peers simultaneously over its 7 links, then reduces locally — costs
 one hop of latency and n-1 link-parallel transfers, the right trade below
-~256 KB (SURVEY.md §5 design note).
+~256 KB.
 
 `latency_all_reduce` implements the one-shot form portably on
 torch.distributed (all_gather into a preallocated buffer + local sum —

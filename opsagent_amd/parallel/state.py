@@ -1,7 +1,7 @@
 """Distributed/tensor-parallel process state — RCCL over xGMI.
 
 One process per GPU (torch.distributed backend "nccl" IS RCCL on ROCm); the
-whole single-node job is one TP group. Design notes: xGMI is
+whole single-node job is one TP group. xGMI is
 point-to-point (7 links x ~153 GB/s per MI355X), so decode's small per-layer
 all-reduces care about latency, not ring bandwidth — they stay inside the
 hipGraph-captured decode step (RCCL collectives are capturable), and prefill's
@@ -36,7 +36,7 @@ def init_distributed(backend: Optional[str] = None) -> None:
             backend = "nccl" if torch.cuda.is_available() else "gloo"
         if backend == "nccl":
             # modulo lets a world-N job run on fewer GPUs (e.g. tp=2 RCCL
-            # validation on a 1-GPU box: both ranks share device 0)
+            # validation on one GPU: both ranks share device 0)
             torch.cuda.set_device(
                 int(os.environ.get("LOCAL_RANK", "0")) %
                 max(torch.cuda.device_count(), 1))

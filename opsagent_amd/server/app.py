@@ -1,7 +1,6 @@
 """HTTP API server.
 
-Route parity with /root/reference/pkg/api/router.go:18-110 plus the fixes
-named in SURVEY.md "known inconsistencies":
+Route parity with pkg/api/router.go:18-110 plus fixes:
 
   POST /login                       (ref router.go:82, handlers/auth.go:25)
   GET  /api/version                 (ref router.go:88)
@@ -169,14 +168,14 @@ def create_app(cfg: Optional[Config] = None) -> FastAPI:
 
     @app.get("/api/health")
     def health():
-        # real health endpoint (the reference's probes point at a 404 — SURVEY.md)
+        # real health endpoint (the reference's probes point at a 404)
         engine_status = "not_loaded"
         try:
             from opsagent_amd.engine.openai_api import ChatCompletionAPI
 
             api = ChatCompletionAPI.instance()
             if api is not None:
-                # watchdog verdict (failure detection)
+                # watchdog verdict
                 engine_status = "ready" if api.loop.healthy else "unhealthy"
         except Exception:  # noqa: BLE001
             engine_status = "error"

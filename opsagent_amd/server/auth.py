@@ -1,6 +1,6 @@
 """HS256 JWT auth — dependency-free implementation.
 
-Capability parity with /root/reference/pkg/handlers/auth.go:25-73 (login with
+Capability parity with pkg/handlers/auth.go:25-73 (login with
 HS256, 24 h expiry) and pkg/middleware/jwt.go:18-64 (Bearer parse+validate).
 Credentials default to the reference's admin/novastar (server.go:28-32) but
 are configurable via config `jwt.*` / env.

@@ -1,6 +1,6 @@
 """Tool plugin registry.
 
-Capability parity with /root/reference/pkg/tools/tool.go:17-38: a tool is a
+Capability parity with pkg/tools/tool.go:17-38: a tool is a
 callable `str -> str` (raising ToolError on failure), registered by name in
 TOOLS. Default registry matches the reference's CopilotTools map
 (tool.go:20-26): search, python, trivy, kubectl, jq.

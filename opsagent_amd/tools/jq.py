@@ -1,4 +1,4 @@
-"""jq tool (ref /root/reference/pkg/tools/jq.go:25-143).
+"""jq tool (ref pkg/tools/jq.go:25-143).
 
 Input convention matches the reference: "<JSON> | <jq-expression>" split on
 the first pipe that is outside the JSON (we split on the last top-level '|').

@@ -1,4 +1,4 @@
-"""JSONPath-style extraction helper (ref /root/reference/pkg/tools/jsonpath.go:10-60).
+"""JSONPath-style extraction helper (ref pkg/tools/jsonpath.go:10-60).
 
 The reference ships an unexported helper that pulls namespace/name/images out
 of a Kubernetes List JSON; here it is a usable utility with a tiny

@@ -1,6 +1,6 @@
 """kubectl tool.
 
-Capability parity with /root/reference/pkg/tools/kubectl.go:21-194:
+Capability parity with pkg/tools/kubectl.go:21-194:
 runs through `bash -c` so pipes work, auto-prefixes "kubectl " when missing,
 classifies common failure modes (not found / forbidden / cluster unreachable),
 records a per-verb perf metric, and filters metrics-server noise and

@@ -1,4 +1,4 @@
-"""Python REPL tool (ref /root/reference/pkg/tools/python.go:25-77).
+"""Python REPL tool (ref pkg/tools/python.go:25-77).
 
 The reference shells into a hardcoded venv (`~/k8s/python-cli/k8s-env`) built
 in its Dockerfile; we run the current interpreter with `python3 -c` (the

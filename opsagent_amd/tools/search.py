@@ -1,4 +1,4 @@
-"""Google Custom Search tool (ref /root/reference/pkg/tools/googlesearch.go:28-44).
+"""Google Custom Search tool (ref pkg/tools/googlesearch.go:28-44).
 
 Uses GOOGLE_API_KEY / GOOGLE_CSE_ID env vars; plain HTTPS via httpx. Raises a
 clear ToolError when credentials or network are unavailable (offline clusters).

@@ -1,4 +1,4 @@
-"""Trivy image-scan tool (ref /root/reference/pkg/tools/trivy.go:23-53)."""
+"""Trivy image-scan tool (ref pkg/tools/trivy.go:23-53)."""
 
 from __future__ import annotations
 

@@ -1,6 +1,6 @@
 """JSON repair utilities for LLM output.
 
-Capability parity with /root/reference/pkg/utils/json.go:16-190 (CleanJSON /
+Capability parity with pkg/utils/json.go:16-190 (CleanJSON /
 ParseJSON / ExtractField): extract the outermost JSON object from surrounding
 prose or code fences, escape raw newlines inside strings, drop trailing
 commas, and fall back to regex field extraction.

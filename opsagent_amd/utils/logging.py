@@ -1,6 +1,6 @@
 """Logging bootstrap.
 
-Capability parity with /root/reference/pkg/utils/logger.go:31-234: configurable
+Capability parity with pkg/utils/logger.go:31-234: configurable
 level/format/output from config, dual sink (JSON file + colored console),
 daily file naming (`opsagent-YYYYMMDD.log`) with size-based rotation, and a
 date-rollover check on access. Uses stdlib logging + RotatingFileHandler.

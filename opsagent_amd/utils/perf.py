@@ -1,7 +1,7 @@
 """Performance statistics engine.
 
 Capability parity with the reference's PerfStats singleton
-(/root/reference/pkg/utils/perf.go:13-335): named start/stop timers, direct
+(pkg/utils/perf.go:13-335): named start/stop timers, direct
 metric recording, min/max/avg/p50/p95/p99 aggregation, a table printer, a
 `trace` decorator/context-manager (ref `TraceFunc`, perf.go:288), and
 `get_stats`/`reset` for the HTTP API (ref perf.go:296-335).

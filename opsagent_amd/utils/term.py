@@ -1,4 +1,4 @@
-"""Terminal markdown rendering (ref /root/reference/pkg/utils/term.go:11-30)."""
+"""Terminal markdown rendering (ref pkg/utils/term.go:11-30)."""
 
 from __future__ import annotations
 

@@ -1,4 +1,4 @@
-"""Extract YAML manifests from LLM output (ref /root/reference/pkg/utils/yaml.go:22-36)."""
+"""Extract YAML manifests from LLM output (ref pkg/utils/yaml.go:22-36)."""
 
 from __future__ import annotations
 

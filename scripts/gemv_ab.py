@@ -1,4 +1,4 @@
-"""Within-probe interleaved A/B of gemv variants (guide rule 24): RW=2 vs
+"""Within-probe interleaved A/B of gemv variants: RW=2 vs
 RW=4 per wave, on REAL-SIZE weights that do NOT fit L3 (many distinct W
 tensors cycled so every pass streams from HBM like a decode step does)."""
 

@@ -2,7 +2,7 @@
 at the 70B/8B decode shapes. Correctness vs a double-quantized torch ref
 (fp8 W AND fp8 x — the MFMA path's numerics), plus streamed TB/s.
 
-Run under gpurun; commit the summary to profiles/README.md.
+Run on an MI355X; summaries lie in profiles/README.md.
 """
 
 from __future__ import annotations

@@ -1,7 +1,6 @@
 """Per-kernel microbenchmarks on MI355X — prints a table of achieved
 bandwidth/TFLOPs vs the chip ceilings (HBM ~6.3 TB/s achievable, bf16 MFMA
-~2.5 PF dense). Run via gpurun; results land in gpurun_out/ and the summary
-is committed under profiles/.
+~2.5 PF dense). Run on an MI355X; summaries lie under profiles/.
 
 Usage: python scripts/kernel_bench.py [--iters 50]
 """

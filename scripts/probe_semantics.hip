@@ -1,7 +1,7 @@
 // One-off semantics probe for gfx950 idioms used by attn_prefill_v3:
 //   * v_permlane32_swap_b32 half-exchange direction
 //   * v_cvt_pk_bf16_f32 operand->lo/hi order
-// Build + run on a GPU box:
+// Build + run on an MI355X:
 //   hipcc --offload-arch=gfx950 -O2 scripts/probe_semantics.hip -o /tmp/sem && /tmp/sem
 #include <hip/hip_runtime.h>
 #include <cstdio>

@@ -1,6 +1,5 @@
 #!/bin/bash
-# AddressSanitizer run of the C++ grammar FSM (SURVEY §5 "race detection /
-# sanitizers"): builds an ASAN-instrumented libopsagent_grammar.so and runs
+# AddressSanitizer run of the C++ grammar FSM: builds an ASAN-instrumented libopsagent_grammar.so and runs
 # the full grammar + BPE test files against it. The FSM is the host-side
 # component with the most raw pointer math (token byte tables, mask buffers,
 # simulated-state walks); the HIP kernels are covered by the race-repeat

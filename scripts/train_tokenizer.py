@@ -1,7 +1,7 @@
 """Train the repo's offline byte-level BPE tokenizer (assets/tokenizer-32k.json).
 
 There is no network access for real Llama-3 tokenizer assets, so the
-benchmark's "real tokenizer"  is a byte-level BPE trained
+benchmark's "real tokenizer" is a byte-level BPE trained
 here on a synthetic corpus shaped like the workload: kubectl output, k8s
 events/manifests, ToolPrompt JSON documents, and English ops prose. The
 tokenizer.json is Llama-3-compatible in structure (HF `tokenizers` format,
