@@ -439,10 +439,11 @@ def _ring(x: torch.Tensor, w: torch.Tensor, plan: Tuple[int, ...], act: int = 0,
     return part if parts else out
 
 
-# unsplit plans that leave CUs idle, to the library's gain: rows and weight rows of a tile, up to how
-# many tiles, and whether only above 256 rows of whole steps of 128 columns, the library's
-_TILES_IDLE = {3 * 256 + 1: (160, 256, 192, False), 4 * 256 + 1: (256, 128, 192, False),
-               8 * 256 + 1: (96, 128, 153, True), 9 * 256 + 1: (128, 64, 192, True)}
+# unsplit forms that leave CUs idle, to the library's gain, by (form, gateup): rows and weight rows of
+# a tile, up to how many tiles, from how many columns on
+_TILES_IDLE = {(3, False): (160, 256, 192, 2048), (4, False): (256, 128, 192, 2048),
+               (8, False): (96, 128, 153, 2048), (9, False): (128, 64, 192, 2048),
+               (8, True): (96, 128, 160, 4224), (9, True): (128, 64, 88, 2048)}
 
 
 @functools.lru_cache(maxsize=4096)
@@ -460,10 +461,12 @@ def _tile_sizes(M: int, N: int, K: int, gateup: bool, summed: bool) -> Optional[
     plan = _lib()[0].oa_tile_gemm_plan(M, N, K, int(gateup), int(summed))
     if plan < 0 or plan == 1 and K >= 2048 and not gateup:       # tiles of 256 x 256, unsplit
         return None
-    rows, cols, most, even = _TILES_IDLE.get(plan, (0, 0, 0, False))
-    if most and 2048 <= K <= 8192 and not gateup and -(-M // rows) * -(-N // cols) <= most and not (
-            even and (K % 128 or M <= 256)):
-        return None
+    form, splits = plan >> 8, plan & 255
+    rows, cols, most, least = _TILES_IDLE.get((form, gateup), (1, 1, 0, 0))
+    if splits == 1 and least <= K <= 8192 and -(-M // rows) * -(-N * (1 + gateup) // cols) <= most:
+        # small tiles: where nothing of what costs the library a quarter and more is in the sizes
+        if form < 8 or K % 128 == 0 and (gateup or M > 256 or M % 32 and (form == 8 or M > 224)):
+            return None
     return plan
 
 
@@ -483,12 +486,17 @@ def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = Fa
     and more slower, 1.05 times on average, and one in 25 faster (12288 x 4096, 514 61 / 68, 640 63 /
     70, 486 57 / 58; 11072 x 5760, 517 87 / 92; 16640 x 3648, 315 61 / 66). With 193 tiles and more
     they are ahead again, by 5 per cent, and on rows of 12000 columns the library is up to 1.5 times
-    slower (17856 x 12736, 279 293 / 191). Above 256 rows tiles of 128 x 64 with as many idle and of 96 x
-    128 with two in five go there too, where rows are whole steps of 128 columns (6144 x 4096, 262
-    30.1 / 33.9, 283 30.4 / 35.2; 2048 x 2816, 514 17.1 / 18.5, 661 17.3 / 19.0; 2048 x 2048, 521 13.4 /
-    14.6, 752 14.1 / 15.0; of 330 on two cards three in four 3 per cent and more slower, 1.06 times on
-    average, one in 25 faster): half a step over costs the library a quarter (6144 x
-    3136, 268 31.4 / 27.9).
+    slower (17856 x 12736, 279 293 / 191). Tiles of 128 x 64 with as many idle and of 96 x 128 with two
+    in five go there too, where rows are whole steps of 128 columns (6144 x 4096, 262 30.1 / 33.9, 283 30.4
+    / 35.2; 2048 x 2816, 514 17.1 / 18.5, 661 17.3 / 19.0; 2048 x 2048, 521 13.4 / 14.6, 752 14.1 / 15.0; of 330
+    above 256 rows on two cards three in four 3 per cent and more slower, 1.06 times on average, one in 25
+    faster): half a step over costs the library a quarter (6144 x 3136, 268 31.4 / 27.9). Up to 256 rows
+    whole 32s of them do, and 128 x 64 is ahead up to 224 (6144 x 4096, 250 27.7 / 29.7, 255 27.6 / 30.0, 256
+    40.9 / 30.0; 4608 x 2560, 199 24.8 / 19.4; 9088 x 4096, 191 32.7 / 36.9, 192 40.5 / 36.6; of 128 on a
+    third card 122 were 3 per cent and more slower, 1.1 times on average, none faster). Gate-up in 88 tiles
+    of 128 x 64 and fewer (library and activation / tiles: 2 x 1024 x 2048, 209 12.1 / 14.1; 2 x 896 x 2560,
+    255 13.7 / 16.8; 81 of them, on three cards, 1.09 on average), and from 4224 columns on in 160 of 96 x
+    128 (2 x 5120 x 5888, 190 50.3 / 55.1; 2 x 3072 x 5888, 278 44.9 / 50.6; 101 of them 1.09).
     Of gate-up the largest of more than 4000 rows go there where columns are many (library and
     activation / tiles: 8000 rows of 4096 x 14336 1281 / 1371, 8192 of 7168 x 8192 1315 / 1385, 16000 of
     28672 x 8192 10213 / 10959, 9395 of 16848 x 13952 6023 / 6735; smaller ones not, 5500 of 4096 x 14336

@@ -114,20 +114,28 @@ def test_light_weights():
 
 
 def test_idle_units():
-    """Plain products in 192 unsplit tiles and fewer of 160 x 256, 256 x 128 or, with whole steps of the
-    library's above 256 rows, 128 x 64 (153 and fewer of 96 x 128) are the library's, but for rows
-    out of 2048 to 8192 columns."""
+    """Products in few unsplit tiles are the library's, out of 2048 to 8192 columns: plain ones of 160 x
+    256 and 256 x 128; those of 96 x 128 and 128 x 64 and gate-up on whole steps of its columns only, and
+    plain ones of up to 256 rows not on whole 32s, nor of 128 x 64 on 224 and fewer."""
     plan = ops._lib()[0].oa_tile_gemm_plan
     for M, N, K, form, tiles, taken in ((640, 12288, 4096, 3, 192, False), (514, 12288, 4096, 3, 192, False),
                                         (486, 12288, 4096, 4, 192, False), (517, 11072, 5760, 3, 176, False),
                                         (640, 13056, 4096, 3, 204, True), (514, 12288, 1984, 3, 192, True),
                                         (279, 17856, 12736, 3, 140, True), (283, 6144, 4096, 8, 144, False),
                                         (268, 6144, 3136, 8, 144, True), (283, 6656, 4096, 8, 156, True),
+                                        (191, 9088, 4096, 8, 142, False), (192, 9088, 4096, 8, 142, True),
                                         (700, 2048, 2816, 9, 192, False), (700, 2048, 2752, 9, 192, True),
-                                        (250, 6144, 4096, 9, 192, True), (800, 2048, 2816, 9, 224, True)):
+                                        (250, 6144, 4096, 9, 192, False), (256, 6144, 4096, 9, 192, True),
+                                        (199, 4608, 2560, 9, 144, True), (800, 2048, 2816, 9, 224, True)):
         rows, cols = {3: (160, 256), 4: (256, 128), 8: (96, 128), 9: (128, 64)}[form]
         assert plan(M, N, K, 0, 0) == form * 256 + 1 and -(-M // rows) * -(-N // cols) == tiles
         assert (ops._tile_choice(M, N, K) is not None) == taken
+    for M, N, K, form, tiles, taken in ((209, 1024, 2048, 9, 64, False), (256, 896, 2560, 9, 56, False),
+                                        (209, 1024, 2112, 9, 64, True), (200, 1472, 2560, 9, 92, True),
+                                        (190, 5120, 5888, 8, 160, False), (150, 4928, 3840, 8, 154, True)):
+        rows, cols = {8: (96, 128), 9: (128, 64)}[form]
+        assert plan(M, N, K, 1, 0) == form * 256 + 1 and -(-M // rows) * -(-2 * N // cols) == tiles
+        assert (ops._tile_choice(M, N, K, gateup=True) is not None) == taken
     assert ops._tile_choice(514, 6144, 4096, gateup=True) is not None
 
 
