@@ -390,8 +390,10 @@ def _ring_fastest(M: int, N: int, K: int, gateup: bool):
     us, *form = min(forms)
     plan = _ring_choice(M, N, K, gateup)
     if plan:
-        full = gateup and plan[0] == 128 and form == [64, 1, False] and N > 64 * 112
-        return tuple(form) if us < (0.9 if full else 0.97) * _ring_us(M, N, K, gateup, *plan) else plan
+        full = plan[0] == 128 and form == [64, 1, False] and N > 64 * 112
+        short = plan[2] and form[0] == 64 and not form[2] and min(plan[1], form[1]) > 1 and K <= 2048
+        ahead = 0.9 if gateup and (full or short) else 0.97
+        return tuple(form) if us < ahead * _ring_us(M, N, K, gateup, *plan) else plan
     stream = N * (1 + gateup) * K * 2 / 6.2e6 + 3.0
     near = 1.3 if M > 32 and not form[2] else 1.2
     return tuple(form) if K >= (1536 if M <= 16 else 1024) and us < near * stream else None
@@ -415,7 +417,10 @@ def _ring_form(M: int, N: int, K: int, gateup: bool = False):
     says; against splits of 128-row tiles, as full, they have to be 10 per cent ahead (us, splits
     / two tiles: 2 x 7552 x 3648, M = 103 34.4 / 37.7, 2 x 8128 x 4160, 128 39.3 / 44.7, 2 x 8192 x
     4032, 112 37.0 / 41.7; on fewer CUs 2 x 6720 x 3264, 128 35.2 / 32.7, 2 x 7040 x 3264 35.7 /
-    33.3; far ahead 2 x 8192 x 2048, 128 23.0 / 20.9)."""
+    33.3; far ahead 2 x 8192 x 2048, 128 23.0 / 20.9). So do splits of 128-row strips against those of 64,
+    where rows have 2048 columns and fewer (strips of 64 / 128: 2 x 2816 x 2048, 47 12.8 / 13.8, 34 12.4 /
+    12.8; 2 x 2816 x 1664, 46 11.8 / 13.7; 2 x 3008 x 1344, 34 11.3 / 11.7; but 2 x 2880 x 2240, 40 14.4 /
+    13.4, 2 x 3008 x 3136, 38 17.2 / 14.8)."""
     return _ring_choice(M, N, K, gateup) if M == 2 else _ring_fastest(M, N, K, gateup)
 
 

@@ -61,3 +61,10 @@ def test_full_rounds():
         assert ops._ring_form(M, N, K, True) == ops._ring_choice(M, N, K, True) == (128, 2, False)
     for M, N, K in ((128, 6720, 3264), (128, 7040, 3264), (128, 8192, 2048)):
         assert ops._ring_form(M, N, K, True) == (64, 1, False)
+
+
+def test_short_rows():
+    """Gate-up of 33 to 64 short rows stays in splits of 64-row strips."""
+    for M, N, K in ((47, 2816, 2048), (33, 2816, 2048), (46, 2816, 1664), (34, 3008, 1344)):
+        assert ops._ring_form(M, N, K, True) == ops._ring_choice(M, N, K, True) == (64, 2, True)
+    assert ops._ring_form(38, 3008, 3136, True) == (64, 5, False)
