@@ -448,7 +448,7 @@ def _ring(x: torch.Tensor, w: torch.Tensor, plan: Tuple[int, ...], act: int = 0,
 # a tile, up to how many tiles, from how many columns on
 _TILES_IDLE = {(3, False): (160, 256, 192, 2048), (4, False): (256, 128, 192, 2048),
                (8, False): (96, 128, 153, 2048), (9, False): (128, 64, 192, 2048),
-               (8, True): (96, 128, 160, 4224), (9, True): (128, 64, 88, 2048)}
+               (8, True): (96, 128, 160, 4224)}
 
 
 @functools.lru_cache(maxsize=4096)
@@ -456,7 +456,7 @@ def _tile_sizes(M: int, N: int, K: int, gateup: bool, summed: bool) -> Optional[
     weights = N * K * (2 if gateup else 1)
     if summed and K < 2 * N:             # deep products split, others hardly
         return None
-    if weights < (2 ** 22 if gateup or summed or M > 512 else 9e6) or (
+    if weights < (2 ** 22 if gateup or summed or M >= 500 else 9e6) or (
             M >= 3500 and not gateup):
         return None
     if gateup and M > 4000 and M * weights >= 7.2e11:
@@ -470,7 +470,8 @@ def _tile_sizes(M: int, N: int, K: int, gateup: bool, summed: bool) -> Optional[
     rows, cols, most, least = _TILES_IDLE.get((form, gateup), (1, 1, 0, 0))
     if splits == 1 and least <= K <= 8192 and -(-M // rows) * -(-N * (1 + gateup) // cols) <= most:
         # small tiles: where nothing of what costs the library a quarter and more is in the sizes
-        if form < 8 or K % 128 == 0 and (gateup or M > 256 or M % 32 and (form == 8 or M > 224)):
+        ahead = M > 256 and weights >= 9e6 if form == 9 else gateup or M > 256 or M % 32
+        if form < 8 or K % 128 == 0 and ahead:
             return None
     return plan
 
@@ -478,11 +479,12 @@ def _tile_sizes(M: int, N: int, K: int, gateup: bool, summed: bool) -> Optional[
 def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = False) -> Optional[int]:
     """Form and column splits of the tile product (tile_gemm.hip; figures and the rule by sizes
     there) of more than 128 rows, None where the library is faster: light weights at few rows (us,
-    library / tiles: 2048 x 2048, 256 rows 10.1 / 13.0, 512 11.4 / 13.9, 599 13.6 / 14.0, 800 15.3 / 14.5;
-    2816 x 1664, 512 12.8 / 13.2, 550, where the library needs a tile of rows more, 16.7 / 12.8; 3072 x
-    2048, 512 15.3 / 16.2, 550 16.7 / 15.1; 2560 x 2560, 512 18.6 / 21.1, 599 20.8 / 19.9; deep ones with a norm behind
-    them split, 1024 x 4096, 338 16.9 / 15.0), and from some thousand rows on, where power bounds
-    both (4096 x 4096, 4067 92 / 103, 2900 79 / 78), but for gate-up, whose activation rides along.
+    library / tiles: 2048 x 2048, 256 rows 10.1 / 13.0, 800 15.3 / 14.5; between 500 and 800 level to 2.5 us
+    ahead, 512 11.4 / 13.9, 599 13.6 / 14.0, 2816 x 1664, 550 16.7 / 12.8, which its first call of a number
+    of rows, 76 us of the host where the tiles take 9, outweighs in a model of a few dozen layers; deep
+    ones with a norm behind them split, 1024 x 4096, 338 16.9 / 15.0), and from some thousand rows on,
+    where power bounds both (4096 x 4096, 4067 92 / 103, 2900 79 / 78), but for gate-up, whose activation
+    rides along.
     So do products that would run in whole tiles of 256 x 256, the library's own form and faster
     there (8192 x 4096, 2048 rows 93 / 101; 16384 x 2048, 922 53 / 53, 1966 99 / 105, 2987 156 / 170; 14336 x
     4096, 1024 89 / 94, 2092 180 / 194; 10240 x 8192, 3072 337 / 358), but for short rows, where it is
@@ -491,17 +493,14 @@ def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = Fa
     and more slower, 1.05 times on average, and one in 25 faster (12288 x 4096, 514 61 / 68, 640 63 /
     70, 486 57 / 58; 11072 x 5760, 517 87 / 92; 16640 x 3648, 315 61 / 66). With 193 tiles and more
     they are ahead again, by 5 per cent, and on rows of 12000 columns the library is up to 1.5 times
-    slower (17856 x 12736, 279 293 / 191). Tiles of 128 x 64 with as many idle and of 96 x 128 with two
-    in five go there too, where rows are whole steps of 128 columns (6144 x 4096, 262 30.1 / 33.9, 283 30.4
-    / 35.2; 2048 x 2816, 514 17.1 / 18.5, 661 17.3 / 19.0; 2048 x 2048, 521 13.4 / 14.6, 752 14.1 / 15.0; of 330
-    above 256 rows on two cards three in four 3 per cent and more slower, 1.06 times on average, one in 25
-    faster): half a step over costs the library a quarter (6144 x 3136, 268 31.4 / 27.9). Up to 256 rows
-    whole 32s of them do, and 128 x 64 is ahead up to 224 (6144 x 4096, 250 27.7 / 29.7, 255 27.6 / 30.0, 256
-    40.9 / 30.0; 4608 x 2560, 199 24.8 / 19.4; 9088 x 4096, 191 32.7 / 36.9, 192 40.5 / 36.6; of 128 on a
-    third card 122 were 3 per cent and more slower, 1.1 times on average, none faster). Gate-up in 88 tiles
-    of 128 x 64 and fewer (library and activation / tiles: 2 x 1024 x 2048, 209 12.1 / 14.1; 2 x 896 x 2560,
-    255 13.7 / 16.8; 81 of them, on three cards, 1.09 on average), and from 4224 columns on in 160 of 96 x
-    128 (2 x 5120 x 5888, 190 50.3 / 55.1; 2 x 3072 x 5888, 278 44.9 / 50.6; 101 of them 1.09).
+    slower (17856 x 12736, 279 293 / 191). Tiles of 96 x 128 with two in five idle go there too, where
+    rows are whole steps of 128 columns (6144 x 4096, 262 30.1 / 33.9, 283 30.4 / 35.2; 9088 x 4096, 191
+    32.7 / 36.9; of 141 on two cards 128 were 3 per cent and more slower, 1.1 times on average): half a
+    step over costs the library a quarter (6144 x 3136, 268 31.4 / 27.9), and so do whole 32s of up to
+    256 rows (9088 x 4096, 192 40.5 / 36.6). So do, above 256 rows and but for light weights, those of 128 x
+    64 with a quarter idle (2880 x 4352, 512 26.7 / 31.3; 4032 x 3328, 382 21.9 / 24.9; 3072 x 5120, 497 32 /
+    36), and gate-up of 4224 columns on in 160 of 96 x 128 (library and activation / tiles: 2 x 5120 x 5888,
+    190 50.3 / 55.1; 2 x 3072 x 5888, 278 44.9 / 50.6; 101 of them 1.09 on average).
     Of gate-up the largest of more than 4000 rows go there where columns are many (library and
     activation / tiles: 8000 rows of 4096 x 14336 1281 / 1371, 8192 of 7168 x 8192 1315 / 1385, 16000 of
     28672 x 8192 10213 / 10959, 9395 of 16848 x 13952 6023 / 6735; smaller ones not, 5500 of 4096 x 14336
@@ -511,9 +510,9 @@ def _tile_choice(M: int, N: int, K: int, gateup: bool = False, summed: bool = Fa
     13195 of 13824 x 5120, 16 of 5632 short, 3038 / 2680). Over 113 products of 3000 to 16384 rows, 52 of
     them drawn, the choice is 0.5 per cent from the better of the two on average; many columns in
     part of a round lose up to 6 (5084 rows of 8424 x 9984, 1346 / 1266).
-    Of 33110 plain products at 129 to 3500 rows, 3000 weights but 19 of them drawn, 22300 are taken, 1.2
+    Of 33110 plain products at 129 to 3500 rows, 3000 weights but 19 of them drawn, 23000 are taken, 1.2
     times as fast as the library on average (1.16 on whole steps of 128 columns), 4 in 100 of them 3 per
-    cent and more slower, 6 in 1000 more than 10 (16704 x 5120, 283 rows 81 / 98: three row tiles of
+    cent and more slower, 7 in 1000 more than 10 (16704 x 5120, 283 rows 81 / 98: three row tiles of
     96 in a round and a half); gate-up 1.2 times, hardly one slower. summed: for linear_parts, where a
     norm adds up the splits."""
     return _tile_sizes(M, N, K, gateup, summed) if M > 128 else None

@@ -105,18 +105,16 @@ def test_whole_tiles_of_the_library():
 
 
 def test_light_weights():
-    for N, K in ((2560, 2560), (3072, 2048)):
-        assert ops._tile_choice(512, N, K) is None and ops._tile_choice(513, N, K) is not None
-    for N, K in ((2048, 2048), (2048, 2816)):          # 192 tiles up to 768 rows (test_idle_units)
-        assert ops._tile_choice(768, N, K) is None and ops._tile_choice(769, N, K) is not None
+    for N, K in ((2048, 2048), (2560, 2560), (3072, 2048), (2048, 2816)):
+        assert ops._tile_choice(499, N, K) is None and ops._tile_choice(500, N, K) is not None
     assert ops._tile_choice(512, 2816, 2048, gateup=True) is not None
     assert ops._tile_choice(512, 2048, 8192) is not None
 
 
 def test_idle_units():
     """Products in few unsplit tiles are the library's, out of 2048 to 8192 columns: plain ones of 160 x
-    256 and 256 x 128; those of 96 x 128 and 128 x 64 and gate-up on whole steps of its columns only, and
-    plain ones of up to 256 rows not on whole 32s, nor of 128 x 64 on 224 and fewer."""
+    256 and 256 x 128; on whole steps of its columns those of 96 x 128, but for whole 32s of up to 256
+    plain rows, and of heavy weights and more rows those of 128 x 64."""
     plan = ops._lib()[0].oa_tile_gemm_plan
     for M, N, K, form, tiles, taken in ((640, 12288, 4096, 3, 192, False), (514, 12288, 4096, 3, 192, False),
                                         (486, 12288, 4096, 4, 192, False), (517, 11072, 5760, 3, 176, False),
@@ -124,15 +122,13 @@ def test_idle_units():
                                         (279, 17856, 12736, 3, 140, True), (283, 6144, 4096, 8, 144, False),
                                         (268, 6144, 3136, 8, 144, True), (283, 6656, 4096, 8, 156, True),
                                         (191, 9088, 4096, 8, 142, False), (192, 9088, 4096, 8, 142, True),
-                                        (700, 2048, 2816, 9, 192, False), (700, 2048, 2752, 9, 192, True),
-                                        (250, 6144, 4096, 9, 192, False), (256, 6144, 4096, 9, 192, True),
-                                        (199, 4608, 2560, 9, 144, True), (800, 2048, 2816, 9, 224, True)):
+                                        (512, 2880, 4352, 9, 180, False), (382, 4032, 3328, 9, 189, False),
+                                        (700, 2048, 2816, 9, 192, True), (250, 6144, 4096, 9, 192, True)):
         rows, cols = {3: (160, 256), 4: (256, 128), 8: (96, 128), 9: (128, 64)}[form]
         assert plan(M, N, K, 0, 0) == form * 256 + 1 and -(-M // rows) * -(-N // cols) == tiles
         assert (ops._tile_choice(M, N, K) is not None) == taken
-    for M, N, K, form, tiles, taken in ((209, 1024, 2048, 9, 64, False), (256, 896, 2560, 9, 56, False),
-                                        (209, 1024, 2112, 9, 64, True), (200, 1472, 2560, 9, 92, True),
-                                        (190, 5120, 5888, 8, 160, False), (150, 4928, 3840, 8, 154, True)):
+    for M, N, K, form, tiles, taken in ((190, 5120, 5888, 8, 160, False), (192, 5120, 5888, 8, 160, False),
+                                        (150, 4928, 3840, 8, 154, True), (209, 1024, 2048, 9, 64, True)):
         rows, cols = {8: (96, 128), 9: (128, 64)}[form]
         assert plan(M, N, K, 1, 0) == form * 256 + 1 and -(-M // rows) * -(-2 * N // cols) == tiles
         assert (ops._tile_choice(M, N, K, gateup=True) is not None) == taken
