@@ -66,7 +66,8 @@ def test_queued_steps():
                             {"id": "b", "tokens": b[:11], "want": [0, 10]}], []))
         for t in range(39):
             if t == 9 and not wait:                  # captured by now, which waits by itself
-                for _ in range(200):                 # about 0.8 ms each
+                # 0.4 s and more for thirty steps of 1 ms of the host, which may be held up once
+                for _ in range(800):                 # 0.5 to 0.8 ms each
                     torch.mm(work, work)
                 busy = torch.cuda.Event()
                 busy.record()
