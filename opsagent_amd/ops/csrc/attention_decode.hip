@@ -14,9 +14,10 @@
 //   o_part   [B*Hk*NSPLIT, G, 128] f32, ml_part [B*Hk*NSPLIT, G, 2] f32
 //   out      [B, Hq, 128] bf16
 //
-// A split is `chunk` keys, a multiple of 64 (decode_chunk), and at most nsplit
-// splits cover a sequence; blocks past its last key end at once and the combine
-// reads the splits that exist.
+// Small launches: a split is `chunk` keys, a multiple of 64 (decode_chunk), and blocks past a
+// sequence's last key end at once. Larger ones: the tiles of 64 keys of all sequences are cut in
+// equal runs, one a CU (DecodeRuns). Either way at most nsplit splits cover a sequence, a mark
+// stands behind its last one, and the combine reads those before it.
 
 #include "common.h"
 
@@ -60,7 +61,12 @@ __device__ __forceinline__ float swap_add(float a, float b) {
 // partial results in its place. Both launches, us: 47 rows of up to 3000 tokens in a step
 // of 64 100.2 -> 88.9, 33 of up to 1500 54.3 -> 42.7, 24 of up to 2000 in 32 40.7 -> 38.8;
 // a full step pays for the look: 64 of up to 3000 112.3 -> 112.8, of up to 300 22.1 -> 22.5.
-#define COPY_MARK -1.0f                // where a sum of weights would be
+// (With splits of each sequence; runs leave such rows out and look at them in blocks of their own.)
+//
+// Marks stand where a sum of weights would be: of a copy's first split, of the place behind a
+// row's last one.
+#define COPY_MARK -1.0f
+#define END_MARK -2.0f
 template <int G>
 __device__ __forceinline__ bool copy_of_first(const uint32_t* q, int qs2, const uint32_t* kin, int ks2,
                                               const uint32_t* vin, int vs2, const int* block_table,
@@ -74,6 +80,130 @@ __device__ __forceinline__ bool copy_of_first(const uint32_t* q, int qs2, const 
     for (int i = lane; i < pages; i += WAVE)
         diff |= block_table[(size_t)b * max_blocks + i] ^ block_table[i];
     return !__any(diff != 0);
+}
+
+// 16 bytes of a value row. NT: in a busy step it is read once, and all of it by one load: without
+// being kept. 47 sequences of up to 3000 tokens 79.0 -> 74.5 us, 64 of 300 20.8 -> 20.6. The loads of
+// key rows take a quarter of each at a time, from a line that has to stay meanwhile: with nt 5%
+// slower. The rows of few sequences stay in the last cache from step to step: an agent's turn of an 8B
+// model 59.1 -> 60.9 ms with nt.
+template <bool NT>
+__device__ __forceinline__ uint4 load_value(const uint32_t* p) {
+    typedef __attribute__((ext_vector_type(4))) uint32_t u4;
+    const u4* at = reinterpret_cast<const u4*>(p);
+    return __builtin_bit_cast(uint4, NT ? __builtin_nontemporal_load(at) : *at);
+}
+
+// inclusive sums over the wave's lanes, by row shifts and row broadcasts
+__device__ __forceinline__ int wave_sums(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+
+// Whether row b may be a copy of the first one. (All loads at once: each wait for memory would
+// add to every launch.)
+__device__ __forceinline__ bool maybe_copy(const int* slots, const int* seq_lens, int b, int copies) {
+    if (!copies) return false;
+    const int n = seq_lens[b], n0 = seq_lens[0], slot = slots[b], slot0 = slots[0];
+    return (b > 0) & (slot == slot0) & (n == n0);
+}
+// keys of row b in the runs
+__device__ __forceinline__ int run_keys(const int* seq_lens, const int* slots, int b, int copies) {
+    const int n = seq_lens[b];
+    return maybe_copy(slots, seq_lens, b, copies) ? 0 : max(n, 0);
+}
+__device__ __forceinline__ int in_tiles(int keys) { return (keys + 63) >> 6; }
+
+// Runs. Blocks that end at a sequence's end are unequal, and beyond one a CU they wait for memory
+// that is busy anyway: what bounds a busy step's attention is the cache's rows (256 bytes each, pages
+// in any order: loads alone run at 5.6 TB/s, 6.1 with value rows read without being kept), and
+// prologues and uneven ends on top. So each of `runs` blocks of a key head takes `per` tiles of 64 keys, sequence after
+// sequence; a row of t tiles lies in (t + per - 2) / per + 1 runs at the most, which `per` keeps to
+// nsplit. Key heads go in step, head h on die h % 8.
+//
+// Each row that a run begins costs it a prologue and a merge. Where rows are short, a run is one
+// unit of `size` tiles of a row instead (chunk_base keys, or as many as nsplit asks for; `per` is 1),
+// the rows' first units before what is left. The line: tiles for each of runs and rows, 3.5, or 8
+// where rows are more than the runs by a quarter. Both launches, us, splits of each sequence / runs
+// / units, 4 heads a key head: 47 of up to 3000 tokens in a step of 64, 8 key heads 88.4 / 74.5, 64 of 2500 94.4 /
+// 82.2, 20 of 8000 in 32 102 / 79, 47 of 3000 on 4 52.8 / 43.7, 32 of 3000 62.8 / 55.6, 33 of 1500 42.2 / 37.7,
+// 33 of 800 29.9 / 28.5 / 31, 24 of 1000 25.4 / 25.9, 64 of 1200 52.8 / 51.8, 64 of 700 35.8 / 38 / 34.5, 64 of 300
+// 22.5 / 26 / 20.6; 8 heads a key head, 64 of 500 on 4 21.1 / 30 / 21.0. Runs for 384 or 768 blocks
+// are slower (89, 89), for 512 level (79.5), and so are two tiles ahead (79). Rows that
+// share most of their pages lose what splits in step got from the die's L2: 32 of up to 3000
+// with 2000 in common 39.2 -> 42.1 (47 with 1000 71.5 -> 61.5).
+struct DecodeRuns {
+    int size, per, total;
+    int b, n;               // row (-1: none) and keys of it
+    int before;             // tiles of the rows before it; units: `which` less the unit within the row
+};
+
+__device__ __forceinline__ int in_units(int t, int size) {
+    return size & (size - 1) ? CEIL_DIV(t, size) : (t + size - 1) >> __builtin_ctz(size);
+}
+
+// The row that run `which` begins with. Every wave works it out for itself, a lane per sequence,
+// 64 sequences at a time.
+__device__ __forceinline__ DecodeRuns decode_runs(const int* seq_lens, const int* slots, int B, int copies,
+                                                  int runs, int nsplit, int chunk_base, int which) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    auto keys = [&](int b) {
+        const int n = run_keys(seq_lens, slots, min(b, B - 1), copies);
+        return b < B ? n : 0;
+    };
+    DecodeRuns r;
+    const int n0 = keys(lane);
+    int most = n0, rows = __builtin_popcountll(__ballot(n0 > 0));
+    r.total = __builtin_amdgcn_readlane(wave_sums(in_tiles(n0)), 63);
+#pragma unroll 1
+    for (int b0 = WAVE; b0 < B; b0 += WAVE) {
+        const int n = keys(b0 + lane);
+        most = max(most, n);
+        rows += __builtin_popcountll(__ballot(n > 0));
+        r.total += __builtin_amdgcn_readlane(wave_sums(in_tiles(n)), 63);
+    }
+    most = in_tiles(most);
+    // (divisions only where they are needed: every launch waits for this)
+    const bool units = 2 * r.total < (4 * rows > 5 * runs ? 16 : 7) * (runs + rows);
+    int cut = units ? chunk_base / 64 : __builtin_amdgcn_readfirstlane(CEIL_DIV(r.total, runs));
+    const int over = units ? 0 : 1;
+    while (const uint64_t more = __ballot(most - over > cut * (nsplit - over)))
+        cut = CEIL_DIV(__builtin_amdgcn_readlane(most, __builtin_ctzll(more)) - over, nsplit - over);
+    r.size = units ? cut : 1;
+    r.per = units ? 1 : cut;
+    r.b = -1;
+    // units: the first ones of all rows, then what is left of them
+    const int at = units ? which - B : which * r.per;
+    int before = 0;
+#pragma unroll 1
+    for (int b0 = 0; b0 < B; b0 += WAVE) {
+        const int n = b0 ? keys(b0 + lane) : n0, t = in_tiles(n);
+        uint64_t past;
+        int u = t, sums = 0;
+        if (units && at < 0) {
+            past = which < b0 + WAVE ? 1ull << (which - b0) : 0;
+        } else {
+            if (units) u = max(in_units(t, r.size) - 1, 0);
+            sums = before + wave_sums(u);
+            past = __ballot(sums > at);
+            before = __builtin_amdgcn_readlane(sums, 63);
+        }
+        if (past) {
+            const int row = __builtin_ctzll(past);
+            r.n = __builtin_amdgcn_readlane(n, row);
+            if (r.n == 0) break;
+            r.b = b0 + row;
+            r.before = __builtin_amdgcn_readlane(sums, row) - __builtin_amdgcn_readlane(u, row);
+            if (units) r.before = at < 0 ? which : r.before + B - 1;
+            break;
+        }
+    }
+    return r;
 }
 
 // Scores on the matrix cores, values on the vector units, all in 32 bits.
@@ -101,14 +231,14 @@ __device__ __forceinline__ bool copy_of_first(const uint32_t* q, int qs2, const 
 // [0, n-1), and the split that owns key n-1 rotates the new key, stores it and its
 // value in the cache and starts its softmax with them. kin/vin/cs/sn/slots/kcw/vcw
 // are only read when ROPE.
-template <int G, bool FUSED, bool ROPE>
-__global__ __launch_bounds__(256) void decode_attn_kernel(
+template <int G, bool FUSED, bool ROPE, bool RUNS>
+__global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kernel(
     const uint32_t* __restrict__ q, const uint32_t* __restrict__ kc,
     const uint32_t* __restrict__ vc, const int* __restrict__ block_table,
     const int* __restrict__ seq_lens, float* __restrict__ o_part,
     float* __restrict__ ml_part, unsigned* __restrict__ cnt,
     uint32_t* __restrict__ out, int B, int Hk, int max_blocks,
-    int block_shift /* log2(block_size) */, int nsplit, int chunk_base, float scale,
+    int block_shift /* log2(block_size) */, int nsplit, int chunk_base, int runs, float scale,
     int qs2 /* q batch-row stride in words */,
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
     const float* __restrict__ cs, const float* __restrict__ sn,
@@ -116,46 +246,91 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
     uint32_t* __restrict__ vcw, int ks2, int vs2, int copies) {
     constexpr int GP = G > 4 ? 8 : 4;            // columns of one part of the queries
     constexpr int KL = GP / 4;                   // keys per lane and tile
-    const int bh = blockIdx.x;
-    const int b = bh / Hk;
-    const int h = bh % Hk;
-    const int split = blockIdx.y;
-    const int Hq = Hk * G;
-
-    const int n = seq_lens[b];
-    const int chunk = decode_chunk(n, nsplit, chunk_base);
-    const int kstart = split * chunk;
-    if (!FUSED && kstart >= n) return;
-    if (ROPE && copies && b > 0 && slots[b] == slots[0] && n == seq_lens[0] &&
-        copy_of_first<G>(q, qs2, kin, ks2, vin, vs2, block_table, max_blocks, b, h,
-                         CEIL_DIV(n, 1 << block_shift))) {
-        if (split == 0 && threadIdx.x < G)
-            ml_part[((size_t)bh * nsplit * G + threadIdx.x) * 2 + 1] = COPY_MARK;
-        return;
+    // the (row, key head) in work and its keys; RUNS: tiles of the row, the first of them that
+    // the block takes, and how many it still has to take
+    int b, h, split, n, kstart, kend, own = 0, from = 0, left = 0;
+    bool once = false;                               // value rows are read without being kept
+    if (RUNS) {
+        const int at = blockIdx.y, whole = gridDim.y - copies * (B - 1);
+        h = blockIdx.x;
+        split = 0;
+        if (at < whole) {
+            const DecodeRuns r = decode_runs(seq_lens, slots, B, copies, runs, nsplit, chunk_base, at);
+            if (r.b < 0) return;
+            b = r.b;
+            n = r.n;
+            own = in_tiles(n);
+            once = r.per > 1;
+            if (once) {
+                from = at * r.per - r.before;
+                left = min(r.per, r.total - at * r.per);
+                split = __builtin_amdgcn_readfirstlane(at - r.before / r.per);
+            } else {
+                split = at - r.before;
+                from = split * r.size;
+                left = min(r.size, own - from);
+            }
+        } else {                                     // a row that may be a copy, by itself if it is none
+            b = 1 + at - whole;
+            n = seq_lens[b];
+            if (!maybe_copy(slots, seq_lens, b, copies) || n <= 0) return;
+            left = own = in_tiles(n);
+            if (copy_of_first<G>(q, qs2, kin, ks2, vin, vs2, block_table, max_blocks, b, h,
+                                 (n + (1 << block_shift) - 1) >> block_shift)) {
+                if (threadIdx.x < G) ml_part[((size_t)(b * Hk + h) * nsplit * G + threadIdx.x) * 2 + 1] = COPY_MARK;
+                return;
+            }
+        }
+    } else {
+        b = blockIdx.x / Hk;
+        h = blockIdx.x % Hk;
+        split = blockIdx.y;
+        n = seq_lens[b];
+        const int chunk = decode_chunk(n, nsplit, chunk_base);
+        kstart = split * chunk;
+        if (!FUSED && kstart >= n) return;
+        if (ROPE && maybe_copy(slots, seq_lens, b, copies) &&
+            copy_of_first<G>(q, qs2, kin, ks2, vin, vs2, block_table, max_blocks, b, h,
+                             CEIL_DIV(n, 1 << block_shift))) {
+            if (split == 0 && threadIdx.x < G)
+                ml_part[((size_t)blockIdx.x * nsplit * G + threadIdx.x) * 2 + 1] = COPY_MARK;
+            return;
+        }
+        kend = min(n, kstart + chunk);
     }
-    const int kend = min(n, kstart + chunk);
-    // ROPE: the new key (index n-1) is handled from registers, not cache
-    const int n_cached = ROPE ? (n - 1) : n;
-    const int kend_c = min(kend, n_cached);
 
-    const int lane = threadIdx.x & (WAVE - 1);
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int bmask = (1 << block_shift) - 1;
+    __shared__ __attribute__((aligned(16))) float lds_o_[RUNS ? 2 : 1][4][G][DHEAD];
+    __shared__ float lds_ml_[RUNS ? 2 : 1][4][G][2];
+
+    // of a wave: its own range (of CACHED keys only; ROPE: the new key, index n - 1, is handled from
+    // registers), whole tiles of 16
+    int kend_c, wstart, wend, nt, page = 0;
+    const int* btrow;
+    auto range = [&]() {
+        if (RUNS) {
+            kstart = from * 64;
+            kend = min(n, kstart + min(left, own - from) * 64);
+        }
+        kend_c = min(kend, ROPE ? n - 1 : n);
+        const int span = max(kend_c - kstart, 0);
+        const int wchunk = ((span + 63) >> 6) << 4;
+        wstart = kstart + wid * wchunk;
+        wend = min(kend_c, wstart + wchunk);
+        nt = wend > wstart ? (wend - wstart + 15) >> 4 : 0;
+        btrow = block_table + (size_t)b * max_blocks;
+    };
+    range();
+    uint4 kr_[2][4], vr_[2][4];
+#pragma unroll 1
+    for (int row = 0;; ++row) {
+    const int turn = row & 1;
+    // (RUNS: what hangs on the lane alone is worked out for each row: kept, it costs a wave a SIMD)
+    int lane = threadIdx.x & (WAVE - 1);
+    if (RUNS) asm volatile("" : "+v"(lane));
     const int g16 = lane >> 4;   // row of 16 lanes: keys g16 * 4 .. + 3 of a tile
     const int dl = lane & 15;    // column; owns value channels dl*8 .. dl*8+7
-
-    const int part_idx = (bh * nsplit + split);
-    float* opart_row = o_part + ((size_t)part_idx * G) * DHEAD;
-    float* mlpart_row = ml_part + ((size_t)part_idx * G) * 2;
-
-    // per-wave sub-range (over CACHED keys only), whole tiles of 16
-    const int span = max(kend_c - kstart, 0);
-    const int wchunk = ((span + 63) >> 6) << 4;
-    const int wstart = kstart + wid * wchunk;
-    const int wend = min(kend_c, wstart + wchunk);
-    const int nt = wend > wstart ? (wend - wstart + 15) >> 4 : 0;
-
-    const int* btrow = block_table + (size_t)b * max_blocks;
-    const int bmask = (1 << block_shift) - 1;
     auto slot_of = [&](int kk) {
         return (int64_t)btrow[kk >> block_shift] << block_shift | (kk & bmask);
     };
@@ -165,7 +340,6 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
     // before its loads, 85.7; 8 of up to 1500 21.0, 20.1). Two tiles ahead cost a wave
     // per SIMD: 92.
     auto page_of = [&](int t) { return btrow[(wstart + min(t, nt - 1) * 16) >> block_shift]; };
-    uint4 kr_[2][4], vr_[2][4];
     auto load_tile = [&](int t, int page, uint4 (&kw)[4], uint4 (&vw)[4]) {
         const int k0 = wstart + t * 16;
         // keys past the end repeat the last one; their weights are zero
@@ -184,9 +358,11 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
         const uint32_t* kp = kc + ((size_t)ks * Hk + h) * (DHEAD / 2) + g16 * 4;
 #pragma unroll
         for (int s = 0; s < 4; ++s) kw[s] = *reinterpret_cast<const uint4*>(kp + s * 16);
+        const uint32_t* vp[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            vw[i] = *reinterpret_cast<const uint4*>(vc + ((size_t)vs[i] * Hk + h) * (DHEAD / 2) + dl * 4);
+        for (int i = 0; i < 4; ++i) vp[i] = vc + ((size_t)vs[i] * Hk + h) * (DHEAD / 2) + dl * 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vw[i] = load_value<RUNS>(vp[i]);
     };
     // Loads return in order: the queries and their angles are asked for first, so that they
     // are rotated and split while the first keys, values and the new key are under way
@@ -212,11 +388,12 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    int page = 0;
-    if (nt > 0) {
+    auto load_first = [&]() {
+        if (nt <= 0) return;
         load_tile(0, page_of(0), kr_[0], vr_[0]);
         page = page_of(1);
-    }
+    };
+    if (!RUNS || row == 0) load_first();
     const bool owner = ROPE && n - 1 >= kstart && n - 1 < kend && wid == 3;   // of the new key
     uint4 nk[4], nv;
     if (owner) {
@@ -432,6 +609,22 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
         }
     }
 
+    const int bh = b * Hk + h;
+    float* opart_row = o_part + ((size_t)(bh * nsplit + split) * G) * DHEAD;
+    float* mlpart_row = ml_part + ((size_t)(bh * nsplit + split) * G) * 2;
+    const bool last = !FUSED && kend == n && split + 1 < nsplit;    // of a row's splits, and not of all places
+    auto next = [&]() {
+        left -= own - from;
+        if (left <= 0) return;
+        do n = run_keys(seq_lens, slots, ++b, copies);
+        while (n == 0);
+        own = in_tiles(n);
+        from = split = 0;
+        range();
+        load_first();
+    };
+    if (RUNS) next();
+
     // sums and maxima of every head to all lanes of a row
     if (GP == 4) lsum += row_ror<4>(lsum);
     lsum += row_ror<8>(lsum);
@@ -460,8 +653,9 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
     for (int i = 0; i < NO / 4; ++i) os[i] = swap_add<16>(os[i], os[i + NO / 4]);
 
     // cross-wave combine through LDS: row g16 now holds sums g16 * NO / 4 ... of its channels
-    __shared__ __attribute__((aligned(16))) float lds_o[4][G][DHEAD];
-    __shared__ float lds_ml[4][G][2];
+    // (RUNS: two buffers in turn, as a wave may be a row ahead)
+    auto& lds_o = lds_o_[RUNS ? turn : 0];
+    auto& lds_ml = lds_ml_[RUNS ? turn : 0];
 #pragma unroll
     for (int i = 0; i < NO / 4; ++i) {
         const int at = g16 * (NO / 4) + i;
@@ -496,9 +690,11 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
         if (d == 0) {
             mlpart_row[gh * 2 + 0] = mt;
             mlpart_row[gh * 2 + 1] = lt;
+            if (last) mlpart_row[(G + gh) * 2 + 1] = END_MARK;
         }
     }
 
+    if (RUNS && left > 0) continue;
     if (!FUSED) return;
 
     // ---- G16 publish + reducer election (plain-store recipe) --------------
@@ -546,19 +742,22 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
         reinterpret_cast<uint16_t*>(out)[(size_t)(b * Hq2 + h * G + gh) * DHEAD + d] =
             f32_to_bf16(res);
     }
+    return;
+    }
 }
 
 // Combine split partials -> final output. Grid: B*Hq blocks of NG groups of 32 lanes; a
 // group takes the splits s, s + NG, ..., a lane four channels. A small launch like this is
-// its chain of loads, so a group's first two splits and all statistics are asked for
-// together, and where the chip has room to spare (EARLY) even before the length says
-// which of them exist: what a split past the end left is not looked at. Every wave works
-// the common maximum and sum out for itself.
+// its chain of loads, so statistics and a group's first two splits (EARLY) or the first one of
+// two groups, which nearly always are there, are asked for together, before a mark says how many
+// there are: what lies behind it is not looked at. Every wave works the common maximum and
+// sum out for itself. Both launches, us, the splits counted from the lengths / by the mark: 64 of
+// up to 300 tokens 22.9 / 20.8, 33 of up to 1500 39.9 / 38.5, 47 of up to 3000 76.7 / 74.5.
 template <int G, bool EARLY>
 __global__ __launch_bounds__(EARLY ? 512 : 256) void decode_combine_kernel(
     const float* __restrict__ o_part, const float* __restrict__ ml_part,
     const int* __restrict__ seq_lens, uint32_t* __restrict__ out, int B, int Hk, int nsplit,
-    int chunk_base, const int* __restrict__ slots) {
+    int copies) {
     constexpr int NG = EARLY ? 16 : 8;
     const int bq = blockIdx.x;
     const int Hq = Hk * G;
@@ -568,26 +767,42 @@ __global__ __launch_bounds__(EARLY ? 512 : 256) void decode_combine_kernel(
     const int gh = qh % G;
     const int lane = threadIdx.x & (WAVE - 1);
     const int grp = threadIdx.x >> 5, ch = (threadIdx.x & 31) * 4;
-    size_t first = (size_t)(b * Hk + h) * nsplit * G + gh;
     const int n = seq_lens[b];
-    if (!EARLY && slots && b > 0 && slots[b] == slots[0] && n == seq_lens[0] && n > 0 &&
-        ml_part[first * 2 + 1] == COPY_MARK)
-        first = (size_t)h * nsplit * G + gh;
-    const float2* ml = reinterpret_cast<const float2*>(ml_part) + first;
-    const float* op = o_part + first * DHEAD + ch;
-
-    const int ns = CEIL_DIV(n, decode_chunk(n, nsplit, chunk_base));
-    // EARLY repeats the last split instead of a branch for each load
-    const float2 none = {0.0f, 0.0f};
-    const float2 mine = EARLY || lane < ns ? ml[(EARLY ? min(lane, nsplit - 1) : lane) * G] : none;
-    float2 mo[2];
+    const float2* ml = nullptr;
+    const float* op = nullptr;
+    float2 mine, mo[2];
     float4 ov[2];
+    // asked for before it is known whether they are there: EARLY all, otherwise each wave's first
+    auto look = [&](int pair) {
+        const size_t first = (size_t)pair * nsplit * G + gh;
+        ml = reinterpret_cast<const float2*>(ml_part) + first;
+        op = o_part + first * DHEAD + ch;
+        mine = ml[min(lane, nsplit - 1) * G];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int s = EARLY ? min(grp + NG * i, nsplit - 1) : grp + NG * i;
-        mo[i] = EARLY || s < ns ? ml[s * G] : none;
-        ov[i] = EARLY || s < ns ? *reinterpret_cast<const float4*>(op + (size_t)s * G * DHEAD)
-                                : float4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int i = 0; i < 2; ++i) {
+            const int s = min(grp + NG * i, nsplit - 1);
+            if (!EARLY && !(i == 0 && grp < 2)) continue;
+            mo[i] = ml[s * G];
+            ov[i] = *reinterpret_cast<const float4*>(op + (size_t)s * G * DHEAD);
+        }
+    };
+    look(b * Hk + h);
+    if (!EARLY && copies && __any(lane == 0 && mine.y == COPY_MARK)) look(h);
+    int ns = 0;                                      // the splits end at a mark or with the places
+    for (int s0 = 0; n > 0 && s0 < nsplit; s0 += WAVE) {
+        const bool end = s0 + lane >= nsplit || (s0 ? ml[(s0 + lane) * G] : mine).y == END_MARK;
+        const uint64_t ends = __ballot(end);
+        ns = s0 + (ends ? __builtin_ctzll(ends) : WAVE);
+        if (ends) break;
+    }
+    if (!EARLY) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int s = grp + NG * i;
+            if ((i == 0 && grp < 2) || s >= ns) continue;
+            mo[i] = ml[s * G];
+            ov[i] = *reinterpret_cast<const float4*>(op + (size_t)s * G * DHEAD);
+        }
     }
 
     float mt = lane < ns && mine.y > 0.0f ? mine.x : -INFINITY;
@@ -638,21 +853,32 @@ static int decode_chunk_base(int pairs) {
     return pairs <= 8 ? 64 : pairs <= 32 ? 128 : pairs <= 128 ? 256 : 512;
 }
 
+// Runs of a key head, 0 for splits of each sequence: up to 64 (sequence, key head) pairs what a launch
+// works out first is more than runs gain (us, splits / runs: 12 of up to 900 tokens, 4 key heads 12.5 /
+// 13.3, 8 of 1500, 8 key heads 17.0 / 18.3; but 8 of 6000 37.6 / 34.5, which the host cannot know).
+static int decode_run_count(int B, int Hk, int nsplit) {
+    return B * Hk <= 64 || B > 4096 || nsplit < 2 ? 0 : max(1, 256 / Hk);
+}
+
+// Blocks of a key head: its runs, or the units that fewer than 8 * (runs + B) tiles make
+static int decode_run_blocks(int runs, int cb, int B) {
+    return max(runs, 8 * (runs + B) * 64 / cb + B);
+}
+
 // Early loads pay while the launch is a few blocks (both launches, us: one sequence of 1151
 // tokens 10.4 -> 9.9, 8 of up to 1500 16.9 -> 16.5) and cost where 2048 of them ask for
 // splits that do not exist (64 of up to 300: 24.1 -> 25.0).
 template <int G>
 static void launch_combine(hipStream_t s, const void* o_part, const void* ml_part,
-                           const void* seq_lens, void* out, int B, int Hk, int nsplit, int cb,
-                           const void* slots) {
-    if (B * Hk <= 64)
+                           const void* seq_lens, void* out, int B, int Hk, int nsplit, int copies) {
+    if (B * Hk <= 64 && !copies)
         hipLaunchKernelGGL((decode_combine_kernel<G, true>), dim3(B * Hk * G), dim3(512), 0, s,
                            (const float*)o_part, (const float*)ml_part, (const int*)seq_lens,
-                           (uint32_t*)out, B, Hk, nsplit, cb, (const int*)slots);
+                           (uint32_t*)out, B, Hk, nsplit, 0);
     else
         hipLaunchKernelGGL((decode_combine_kernel<G, false>), dim3(B * Hk * G), dim3(256), 0, s,
                            (const float*)o_part, (const float*)ml_part, (const int*)seq_lens,
-                           (uint32_t*)out, B, Hk, nsplit, cb, (const int*)slots);
+                           (uint32_t*)out, B, Hk, nsplit, copies);
 }
 
 // fused: cnt_ws is zeroed here on each call (hipMemsetAsync). fused = 0: two kernels.
@@ -678,36 +904,28 @@ extern "C" int oa_attention_decode(void* stream, const void* q, const void* kc,
     }
 
     const int cb = decode_chunk_base(B * Hk);
-#define LAUNCH_G(GV)                                                                \
-    do {                                                                            \
-        if (fused) {                                                                \
-            hipLaunchKernelGGL((decode_attn_kernel<GV, true, false>), grid, block,         \
-                               0, (hipStream_t)stream, (const uint32_t*)q,          \
-                               (const uint32_t*)kc, (const uint32_t*)vc,            \
-                               (const int*)block_table, (const int*)seq_lens,       \
-                               (float*)o_part, (float*)ml_part, (unsigned*)cnt_ws,  \
-                               (uint32_t*)out, B, Hk, max_blocks, block_shift,      \
-                               nsplit, cb, scale, qs2, (const uint32_t*)nullptr,        \
-                               (const uint32_t*)nullptr, (const float*)nullptr,     \
-                               (const float*)nullptr, (const int*)nullptr,          \
-                               (uint32_t*)nullptr, (uint32_t*)nullptr, 0, 0, 0);    \
-            HIP_CHECK_LAUNCH();                                                     \
-        } else {                                                                    \
-            hipLaunchKernelGGL((decode_attn_kernel<GV, false, false>), grid, block,        \
-                               0, (hipStream_t)stream, (const uint32_t*)q,          \
-                               (const uint32_t*)kc, (const uint32_t*)vc,            \
-                               (const int*)block_table, (const int*)seq_lens,       \
-                               (float*)o_part, (float*)ml_part, (unsigned*)cnt_ws,  \
-                               (uint32_t*)out, B, Hk, max_blocks, block_shift,      \
-                               nsplit, cb, scale, qs2, (const uint32_t*)nullptr,        \
-                               (const uint32_t*)nullptr, (const float*)nullptr,     \
-                               (const float*)nullptr, (const int*)nullptr,          \
-                               (uint32_t*)nullptr, (uint32_t*)nullptr, 0, 0, 0);    \
-            HIP_CHECK_LAUNCH();                                                     \
-            launch_combine<GV>((hipStream_t)stream, o_part, ml_part, seq_lens, out, B, Hk, \
-                               nsplit, cb, nullptr);                                \
-            HIP_CHECK_LAUNCH();                                                     \
-        }                                                                           \
+    const int runs = fused ? 0 : decode_run_count(B, Hk, nsplit);
+    if (runs) grid = dim3(Hk, decode_run_blocks(runs, cb, B));
+#define LAUNCH_FORM(GV, FUSED, RUNS)                                                           \
+    hipLaunchKernelGGL((decode_attn_kernel<GV, FUSED, false, RUNS>), grid, block, 0,           \
+                       (hipStream_t)stream, (const uint32_t*)q, (const uint32_t*)kc,           \
+                       (const uint32_t*)vc, (const int*)block_table, (const int*)seq_lens,     \
+                       (float*)o_part, (float*)ml_part, (unsigned*)cnt_ws, (uint32_t*)out, B,  \
+                       Hk, max_blocks, block_shift, nsplit, cb, runs, scale, qs2,              \
+                       (const uint32_t*)nullptr, (const uint32_t*)nullptr,                     \
+                       (const float*)nullptr, (const float*)nullptr, (const int*)nullptr,      \
+                       (uint32_t*)nullptr, (uint32_t*)nullptr, 0, 0, 0)
+#define LAUNCH_G(GV)                                                                           \
+    do {                                                                                       \
+        if (fused) LAUNCH_FORM(GV, true, false);                                               \
+        else if (runs) LAUNCH_FORM(GV, false, true);                                           \
+        else LAUNCH_FORM(GV, false, false);                                                    \
+        HIP_CHECK_LAUNCH();                                                                    \
+        if (!fused) {                                                                          \
+            launch_combine<GV>((hipStream_t)stream, o_part, ml_part, seq_lens, out, B, Hk,     \
+                               nsplit, 0);                                                     \
+            HIP_CHECK_LAUNCH();                                                                \
+        }                                                                                      \
     } while (0)
 
     switch (G) {
@@ -718,6 +936,7 @@ extern "C" int oa_attention_decode(void* stream, const void* q, const void* kc,
         default: return -102;
     }
 #undef LAUNCH_G
+#undef LAUNCH_FORM
     return 0;
 }
 
@@ -742,22 +961,26 @@ extern "C" int oa_attention_decode_rope(
     const int cb = decode_chunk_base(B * Hk);
     // few blocks wait for their slowest, which is then a copy looked at twice
     const int copies = B * Hk > 64;
-#define LAUNCH_GR(GV)                                                              \
-    do {                                                                            \
-        hipLaunchKernelGGL((decode_attn_kernel<GV, false, true>), grid, block, 0,   \
-                           (hipStream_t)stream, (const uint32_t*)q,                 \
-                           (const uint32_t*)kc, (const uint32_t*)vc,                \
-                           (const int*)block_table, (const int*)seq_lens,           \
-                           (float*)o_part, (float*)ml_part, (unsigned*)nullptr,     \
-                           (uint32_t*)out, B, Hk, max_blocks, block_shift, nsplit,  \
-                           cb, scale, q_stride / 2, (const uint32_t*)kin,               \
-                           (const uint32_t*)vin, (const float*)cos_t,               \
-                           (const float*)sin_t, (const int*)slots, (uint32_t*)kc,   \
-                           (uint32_t*)vc, k_stride / 2, v_stride / 2, copies);      \
-        HIP_CHECK_LAUNCH();                                                         \
-        launch_combine<GV>((hipStream_t)stream, o_part, ml_part, seq_lens, out, B, Hk,     \
-                           nsplit, cb, copies ? slots : nullptr);                   \
-        HIP_CHECK_LAUNCH();                                                         \
+    const int runs = decode_run_count(B, Hk, nsplit);
+    // rows that may be copies follow the runs
+    if (runs) grid = dim3(Hk, decode_run_blocks(runs, cb, B) + copies * (B - 1));
+#define LAUNCH_FORM(GV, RUNS)                                                                  \
+    hipLaunchKernelGGL((decode_attn_kernel<GV, false, true, RUNS>), grid, block, 0,            \
+                       (hipStream_t)stream, (const uint32_t*)q, (const uint32_t*)kc,           \
+                       (const uint32_t*)vc, (const int*)block_table, (const int*)seq_lens,     \
+                       (float*)o_part, (float*)ml_part, (unsigned*)nullptr, (uint32_t*)out, B, \
+                       Hk, max_blocks, block_shift, nsplit, cb, runs, scale, q_stride / 2,     \
+                       (const uint32_t*)kin, (const uint32_t*)vin, (const float*)cos_t,        \
+                       (const float*)sin_t, (const int*)slots, (uint32_t*)kc, (uint32_t*)vc,   \
+                       k_stride / 2, v_stride / 2, copies)
+#define LAUNCH_GR(GV)                                                                          \
+    do {                                                                                       \
+        if (runs) LAUNCH_FORM(GV, true);                                                       \
+        else LAUNCH_FORM(GV, false);                                                           \
+        HIP_CHECK_LAUNCH();                                                                    \
+        launch_combine<GV>((hipStream_t)stream, o_part, ml_part, seq_lens, out, B, Hk, nsplit, \
+                           copies);                                                            \
+        HIP_CHECK_LAUNCH();                                                                    \
     } while (0)
 
     switch (G) {
@@ -768,5 +991,6 @@ extern "C" int oa_attention_decode_rope(
         default: return -102;
     }
 #undef LAUNCH_GR
+#undef LAUNCH_FORM
     return 0;
 }

@@ -227,3 +227,45 @@ def test_rows_that_are_nearly_copies(G, Hk):
         own = ~copied[b]                              # splits of other sizes: one bf16 rounding apart
         diff = (by_head[b] - want)[own].float().norm() / want[own].float().norm()
         assert diff < 2e-3 and not torch.equal(by_head[b][own], by_head[0][own])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("G", [1, 4, 8])
+@pytest.mark.parametrize("lens,Hk,bs,nsplit", [
+    ([3000, 1, 63, 64, 65, 2111, 128, 129, 1500, 16, 17, 900, 2500, 700, 31, 1023, 1024, 1025, 2048,
+      5, 640], 4, 32, 32),                           # runs that end in, at and across rows
+    ([2000 - 27 * i for i in range(70)], 2, 16, 32),  # more rows than lanes
+    ([4000] + [900 + 7 * i for i in range(16)], 4, 8, 2),     # two places a row
+    ([1 + 9 * i for i in range(66)], 2, 32, 32),     # short rows: units, more rows than lanes
+    ([5000] + [5, 64, 65, 513, 1100] * 13, 4, 64, 3),         # units larger for one long row
+    ([200] * 3 + [4000], 100, 32, 32),               # more key heads than runs for them
+])
+def test_runs_over_sequences(G, lens, Hk, bs, nsplit):
+    """More than 64 (sequence, key head) pairs: blocks go over the tiles of all sequences."""
+    q, k, v, kc, vc, table, lens_t, slots = _case(lens, Hk, G, bs, seed=len(lens) + G)
+    cos, sin = (t.cuda() for t in ops.rope_cos_sin(8192, D))
+    flat_k, flat_v = kc.view(-1, Hk, D), vc.view(-1, Hk, D)
+    plain, roped = [], []
+    for b, n in enumerate(lens):
+        at = torch.arange(n, device="cuda")
+        r = table[b, at // bs].long() * bs + at % bs
+        ks, vs = flat_k[r].double(), flat_v[r].double()
+        plain.append(_attend(q[b].double(), ks, vs, G))
+        new = _rotate(k[b].double(), n - 1, cos, sin)
+        ks, vs = torch.cat([ks[:-1], new[None]]), torch.cat([vs[:-1], v[b].double()[None]])
+        roped.append(_attend(_rotate(q[b].double(), n - 1, cos, sin), ks, vs, G))
+    # every row by itself: a bf16 rounding is 2^-9 at the most of each value, 0.0017 over a row
+    for got, want in [(ops.attention_decode_paged(q, kc, vc, table, lens_t, nsplit=nsplit), plain),
+                      (ops.attention_decode_rope(q, k, v, kc.clone(), vc.clone(), table, lens_t, cos,
+                                                 sin, slots, nsplit=nsplit), roped)]:
+        for b, w in enumerate(want):
+            assert float((got[b].double() - w).norm() / w.norm()) < 2.0 ** -9 + 1e-4, (b, lens[b])
+
+    empty = lens_t.clone()                           # a row without keys is answered by zeros
+    empty[1::3] = 0
+    got = ops.attention_decode_paged(q, kc, vc, table, empty, nsplit=nsplit)
+    for b, w in enumerate(plain):
+        if b % 3 == 1:
+            assert not got[b].any()
+        else:
+            assert float((got[b].double() - w).norm() / w.norm()) < 2.0 ** -9 + 1e-4, (b, lens[b])
