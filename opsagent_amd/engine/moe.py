@@ -20,7 +20,7 @@ from torch import nn
 
 from opsagent_amd import ops
 from opsagent_amd.engine.config import ModelSpec
-from opsagent_amd.engine.model import _init_linear, _shard  # noqa: F401
+from opsagent_amd.engine.model import _init_linear, _shard, _sums_parts  # noqa: F401
 from opsagent_amd.parallel import get_tp_rank, get_tp_size, tp_all_reduce
 
 
@@ -107,13 +107,26 @@ class MoEMLP(nn.Module):
             few = T <= 64 or (decode and P <= 2048)      # the pair kernels' range
             tiles = ops.moe_sorted_ok(x, w13, w2)
             if few or tiles:
-                idx, wts, tok = ops.moe_route(x, self.router_w, self.top_k)
                 local = self.shared is not None and get_tp_size() == 1
-                shared = self.shared(x) if local else None
                 if tiles and not (few and not ops.moe_sorted_wins(P, self.num_experts, self.fp8,
                                                                     self.i_local * H)):
-                    out = ops.moe_sorted_mlp(x, w13, s13, w2, s2, idx, wts, more=shared, parts=parts)
+                    # the shared expert as it is, and nothing that looks at its rows
+                    beside = local and not self.shared.fp8 and _sums_parts(self.shared)
+                    front = ops.moe_front(
+                        x, self.router_w, self.top_k, self.i_local * H, self.fp8,
+                        *((self.shared.gate_up_w, self.shared.down_w) if beside else ()))
+                    if front is None:
+                        idx, wts, _ = ops.moe_route(x, self.router_w, self.top_k)
+                        lists = shared = None
+                    else:
+                        idx, wts, lists, shared = front
+                    if local and shared is None:
+                        shared = self.shared(x)
+                    out = ops.moe_sorted_mlp(x, w13, s13, w2, s2, idx, wts, more=shared, parts=parts,
+                                             lists=lists)
                 else:
+                    idx, wts, tok = ops.moe_route(x, self.router_w, self.top_k)
+                    shared = self.shared(x) if local else None
                     y = ops.moe_grouped_mlp(x, w13, s13, w2, s2, idx.view(-1), tok.view(-1),
                                             wts.view(-1), self.i_local, self.fp8,
                                             num_experts=self.num_experts)

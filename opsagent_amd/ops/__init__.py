@@ -1123,6 +1123,55 @@ def _moe_ring_rows(pairs: int, experts: int, weights: int, fp8: bool) -> int:
     return 64 if small or fp8 or pairs < 64 * experts else 128
 
 
+def _moe_lists(pairs: int, experts: int, weights: int, fp8: bool) -> Tuple[int, int, int]:
+    """Rows of a tile, the most tiles, and the int32s of the sorted pairs' lists."""
+    bm = _moe_ring_rows(pairs, experts, weights, fp8)
+    max_tiles = pairs // bm + min(experts, pairs)
+    return bm, max_tiles, 2 * experts + 2 + max_tiles + pairs
+
+
+def _moe_list_ptrs(ints: torch.Tensor, experts: int, max_tiles: int) -> Tuple[int, int, int, int]:
+    """Addresses of offsets and tile counts [E + 1], tiles' experts and the order in _moe_lists' ints."""
+    at = ints.data_ptr()
+    return (at, at + 4 * (experts + 1), at + 8 * (experts + 1), at + 4 * (2 * experts + 2 + max_tiles))
+
+
+def moe_front(x: torch.Tensor, router_w: torch.Tensor, top: int, weights: int, fp8: bool,
+              gate_up_w: Optional[torch.Tensor] = None, down_w: Optional[torch.Tensor] = None):
+    """Routing of up to 16 tokens x [T, K] with its pairs sorted for moe_sorted_mlp, and a shared
+    expert down(silu(gate x) * up x) beside it where its products are strips: (experts and weights as of
+    moe_route, lists, the shared expert's rows or None), None where the kernels do not take it.
+    weights: size of one expert matrix. Choice and sort are one block's launch, and with the shared
+    expert two launches do for five (moe_grouped.hip; figures there)."""
+    T, K = x.shape
+    E = router_w.shape[0]
+    if not (T <= 16 and E <= 256 and moe_route_ok(x, router_w, top)):
+        return None
+    lib, hip = _lib()
+    stream, dev = hip.current_stream_ptr(), x.device
+    beside = False
+    if gate_up_w is not None and K == gate_up_w.shape[1]:
+        H, I = down_w.shape
+        if gate_up_w.shape[0] == 2 * I and _gateup_form(x, gate_up_w, I) == ("skinny", 1):
+            mid = torch.empty(T, I, dtype=x.dtype, device=dev)
+            beside = (_skinny_ok(mid, down_w) and not _ring_form(T, H, I)
+                      and _skinny_form(T, H, I) == 1)
+    idx = torch.empty(T, top, dtype=torch.int32, device=dev)
+    wts = torch.empty(T, top, dtype=torch.float32, device=dev)
+    scratch = torch.empty(lib.oa_moe_route_scratch(T, E, K), dtype=torch.float32, device=dev)
+    bm, max_tiles, size = _moe_lists(T * top, E, weights, fp8)
+    lists = torch.empty(size, dtype=torch.int32, device=dev)
+    shared = torch.empty(T, H, dtype=x.dtype, device=dev) if beside else None
+    up = (gate_up_w.data_ptr(), mid.data_ptr(), I) if beside else (None, None, 0)
+    down = (mid.data_ptr(), down_w.data_ptr(), shared.data_ptr(), H, I) if beside else (None,) * 3 + (0, 0)
+    hip.check(lib.oa_moe_front_up(stream, x.data_ptr(), router_w.data_ptr(), scratch.data_ptr(), T, E, K,
+                                  *up), "oa_moe_front_up")
+    hip.check(lib.oa_moe_front_down(stream, scratch.data_ptr(), idx.data_ptr(), wts.data_ptr(), T, E, K,
+                                    top, bm, *_moe_list_ptrs(lists, E, max_tiles), *down),
+              "oa_moe_front_down")
+    return idx, wts, lists, shared
+
+
 def moe_sorted_ok(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, act=None) -> bool:
     """Whether moe_sorted_mlp takes these experts: both products run over
     128-column steps, a gate strip holds 64 rows."""
@@ -1147,13 +1196,15 @@ def moe_sorted_mlp(
     act=None,
     more: Optional[torch.Tensor] = None,
     parts: bool = False,
+    lists: Optional[torch.Tensor] = None,
 ) -> Union[torch.Tensor, PairSum]:
     """Routed experts of a prompt-sized batch (GPU): out[t] = sum over token t's
     choices j of weight_tj * W2[e_tj] act(W13[e_tj] x_t), plus more[t] if given.
     x [T, H] bf16; expert_ids int32 and pair_weights float32 [T, top]; experts as
     in moe_grouped_mlp, bf16 or fp8 with row scales. Pairs are sorted by expert
     on the GPU and every expert's rows run as matrix-core tiles: no host sync,
-    static shapes. With `parts` the sum may be left to the norm that follows."""
+    static shapes. With `parts` the sum may be left to the norm that follows. lists: the pairs
+    sorted already (moe_front)."""
     T, H = x.shape
     top = expert_ids.shape[1]
     E, I = w13.shape[0], w2.shape[2]
@@ -1164,21 +1215,23 @@ def moe_sorted_mlp(
     assert expert_ids.shape == pair_weights.shape == (T, top)
     assert (w13.dtype == torch.uint8) == (w13_scale is not None) == (w2_scale is not None)
     P = T * top
-    bm = _moe_ring_rows(P, E, I * H, w13_scale is not None)
-    max_tiles = P // bm + min(E, P)
+    bm, max_tiles, size = _moe_lists(P, E, I * H, w13_scale is not None)
     lib, hip = _lib()
     stream, dev = hip.current_stream_ptr(), x.device
-    ints = torch.empty(2 * E + 2 + max_tiles + P, dtype=torch.int32, device=dev)
-    off, pre, tile_e, perm = ints.split([E + 1, E + 1, max_tiles, P])
-    lists = (off.data_ptr(), pre.data_ptr(), tile_e.data_ptr(), perm.data_ptr())
-    hip.check(lib.oa_moe_sort(stream, expert_ids.data_ptr(), P, E, bm, *lists), "oa_moe_sort")
+    if lists is None:
+        ints = torch.empty(size, dtype=torch.int32, device=dev)
+        ptrs = _moe_list_ptrs(ints, E, max_tiles)
+        hip.check(lib.oa_moe_sort(stream, expert_ids.data_ptr(), P, E, bm, *ptrs), "oa_moe_sort")
+    else:
+        assert lists.shape == (size,) and lists.dtype == torch.int32 and lists.device == dev
+        ptrs = _moe_list_ptrs(lists, E, max_tiles)
     mid = torch.empty(P, I, dtype=x.dtype, device=dev)
     y = torch.empty(P, H, dtype=x.dtype, device=dev)
     ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
-    hip.check(lib.oa_moe_grouped(stream, x.data_ptr(), w13.data_ptr(), ptr(w13_scale), *lists, None,
+    hip.check(lib.oa_moe_grouped(stream, x.data_ptr(), w13.data_ptr(), ptr(w13_scale), *ptrs, None,
                                  mid.data_ptr(), E, I, H, top, bm, max_tiles,
                                  2 if actk == 3 else 1, actk, limit, alpha), "oa_moe_grouped(up)")
-    hip.check(lib.oa_moe_grouped(stream, mid.data_ptr(), w2.data_ptr(), ptr(w2_scale), *lists,
+    hip.check(lib.oa_moe_grouped(stream, mid.data_ptr(), w2.data_ptr(), ptr(w2_scale), *ptrs,
                                  pair_weights.data_ptr(), y.data_ptr(), E, H, I, top, bm, max_tiles,
                                  0, 0, 0.0, 0.0), "oa_moe_grouped(down)")
     return moe_combine(y, top, more, parts)

@@ -64,6 +64,7 @@ def needs_rebuild(out: str = OUT, sources=None) -> bool:
     deps = [os.path.join(CSRC, s) for s in (sources or SOURCES)]
     deps.append(os.path.join(CSRC, "common.h"))
     deps.append(os.path.join(CSRC, "mixer_util.h"))
+    deps.append(os.path.join(CSRC, "skinny_strip.h"))
     return any(_mtime(d) > out_t for d in deps)
 
 

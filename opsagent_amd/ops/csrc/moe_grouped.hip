@@ -17,7 +17,7 @@
 // one order: the output does not depend on how pairs are placed in an expert.
 // Activations are bf16; weights bf16, or fp8 (e4m3, one float32 scale per row)
 // widened exactly to bf16 in registers. Sums are float32.
-#include "common.h"
+#include "skinny_strip.h"
 
 typedef __attribute__((ext_vector_type(4))) unsigned int mgu4;
 typedef __attribute__((ext_vector_type(8))) short mgs8;
@@ -37,19 +37,18 @@ typedef __attribute__((ext_vector_type(4))) float mgf4;
 // launches, 13 tokens x 64 experts x 2048: 9.9, 512 tokens 11.0 (22.2); before, logits and choice in one
 // launch with a token per block, which drew the whole matrix through every block's CU:
 // 20.9 (11.3 with it in cache), as unrolled vector code over the blocks 16.3.
-__global__ __launch_bounds__(256) void moe_logits_kernel(const uint16_t* __restrict__ x,
-                                                         const float* __restrict__ rw,
-                                                         float* __restrict__ part, int T, int E,
-                                                         int K) {
-    __shared__ mgf4 red[4][64];
+__device__ __forceinline__ void moe_logits_part(const uint16_t* __restrict__ x, const float* __restrict__ rw,
+                                                float* __restrict__ part, int T, int E, int K, int bt, int be,
+                                                int bs, int splits, mgf4 (&red)[4][64]) {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
-    const int t0 = blockIdx.x * 16, e0 = blockIdx.y * 16;
+    const int t0 = bt * 16, e0 = be * 16;
     const float* wr = rw + (size_t)min(e0 + r, E - 1) * K;
     const uint16_t* xr = x + (size_t)min(t0 + r, T - 1) * K;
-    const int stride = gridDim.z * 64;  // columns between two steps of a wave
+    const int stride = splits * 64;     // columns between two steps of a wave
     mgf4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    // (blocks of more than four waves: the first four)
 #pragma unroll 1
-    for (int k0 = (blockIdx.z * 4 + wid) * 16 + q * 4; k0 < K; k0 += 4 * stride) {
+    for (int k0 = (bs * 4 + wid) * 16 + q * 4; k0 < K && wid < 4; k0 += 4 * stride) {
         mgf4 w[4];
         uint2 v[4];
 #pragma unroll
@@ -68,7 +67,7 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(const uint16_t* __restr
                                                            acc, 0, 0, 0);
         }
     }
-    red[wid][lane] = acc;
+    if (wid < 4) red[wid][lane] = acc;
     __syncthreads();
     if (wid) return;
     acc = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
@@ -77,7 +76,15 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(const uint16_t* __restr
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (e0 + q * 4 + j < E)
-                part[((size_t)blockIdx.z * T + t0 + r) * E + e0 + q * 4 + j] = acc[j];
+                part[((size_t)bs * T + t0 + r) * E + e0 + q * 4 + j] = acc[j];
+}
+
+__global__ __launch_bounds__(256) void moe_logits_kernel(const uint16_t* __restrict__ x,
+                                                         const float* __restrict__ rw,
+                                                         float* __restrict__ part, int T, int E,
+                                                         int K) {
+    __shared__ mgf4 red[4][64];
+    moe_logits_part(x, rw, part, T, E, K, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, red);
 }
 
 // a op (a of the lane that DPP names); lanes without a source keep their value
@@ -104,17 +111,11 @@ __device__ __forceinline__ float mg_wave_max(float v) {
 
 // Softmax and the `top` best experts, a wave per token; weights normalised over the
 // chosen, ties go to the lower expert.
-__global__ __launch_bounds__(256) void moe_choose_kernel(const float* __restrict__ part,
-                                                         int* __restrict__ idx,
-                                                         float* __restrict__ wout,
-                                                         int* __restrict__ tok, int T, int E,
-                                                         int top, int splits) {
-    __shared__ float zs[4][MG_MAX_E];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int t = blockIdx.x * 4 + wid;
-    if (t >= T) return;
-    float* z = zs[wid];                 // a lane touches its own columns only
-    const size_t o = (size_t)t * top;
+// z: E floats of the wave's own (a lane touches its own columns only). Lane r has the r-th choice and
+// its weight.
+__device__ __forceinline__ void moe_choose_token(const float* __restrict__ part, int t, int T, int E,
+                                                 int top, int splits, float* z, int& who, float& weight) {
+    const int lane = threadIdx.x & 63;
     float mx = -INFINITY;
     for (int e = lane; e < E; e += 64) {
         float a = 0.0f;
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(256) void moe_choose_kernel(const float* __restrict
     sum = wave_reduce_sum(sum);
     for (int e = lane; e < E; e += 64) z[e] = z[e] / sum;
     float mine = 0.0f, total = 0.0f;    // lane r keeps the r-th choice's score
-    int who = 0;
+    who = 0;
 #pragma unroll 1
     for (int r = 0; r < top; ++r) {
         float bv = -INFINITY;
@@ -153,9 +154,25 @@ __global__ __launch_bounds__(256) void moe_choose_kernel(const float* __restrict
         }
         if (lane == (bi & 63)) z[bi] = -INFINITY;   // the lane that reads it next
     }
+    weight = mine / (total + 1e-20f);
+}
+
+__global__ __launch_bounds__(256) void moe_choose_kernel(const float* __restrict__ part,
+                                                         int* __restrict__ idx,
+                                                         float* __restrict__ wout,
+                                                         int* __restrict__ tok, int T, int E,
+                                                         int top, int splits) {
+    __shared__ float zs[4][MG_MAX_E];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int t = blockIdx.x * 4 + wid;
+    if (t >= T) return;
+    int who;
+    float weight;
+    moe_choose_token(part, t, T, E, top, splits, zs[wid], who, weight);
+    const size_t o = (size_t)t * top;
     if (lane < top) {
         idx[o + lane] = who;
-        wout[o + lane] = mine / (total + 1e-20f);
+        wout[o + lane] = weight;
         tok[o + lane] = t;
     }
 }
@@ -164,21 +181,27 @@ __global__ __launch_bounds__(256) void moe_choose_kernel(const float* __restrict
 // One block: counts per expert, offsets, tiles of `bm` rows, then the places.
 // off [E + 1]; pre [E + 1]: first tile of every expert; tile_e: expert of every
 // tile; perm [P]: pair at every sorted place.
-__global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ expert_ids, int P,
-                                                        int E, int bm, int* __restrict__ off,
-                                                        int* __restrict__ pre,
-                                                        int* __restrict__ tile_e,
-                                                        int* __restrict__ perm) {
-    __shared__ int cnt[MG_MAX_E], cur[MG_MAX_E], wsum[2][16];
+// NT threads, no fewer than experts.
+template <int NT, int MAXE>
+struct SortRoom {
+    int cnt[MAXE], cur[MAXE], wsum[2][NT / 64];
+};
+template <int NT, int MAXE>
+__device__ __forceinline__ void moe_sort_pairs(const int* expert_ids, int P, int E, int bm,
+                                               int* __restrict__ off, int* __restrict__ pre,
+                                               int* __restrict__ tile_e, int* __restrict__ perm,
+                                               SortRoom<NT, MAXE>& room) {
+    auto &cnt = room.cnt, &cur = room.cur;
+    auto& wsum = room.wsum;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    for (int e = tid; e < E; e += 1024) cnt[e] = 0;
+    for (int e = tid; e < E; e += NT) cnt[e] = 0;
     __syncthreads();
-    for (int p = tid; p < P; p += 1024) {
+    for (int p = tid; p < P; p += NT) {
         const int e = expert_ids[p];
         if ((unsigned)e < (unsigned)E) atomicAdd(&cnt[e], 1);
     }
     __syncthreads();
-    // inclusive scans of rows and tiles, one expert per thread (E <= 1024)
+    // inclusive scans of rows and tiles, one expert per thread
     const int c = tid < E ? cnt[tid] : 0;
     const int nt = (c + bm - 1) / bm;
     int a = c, b = nt;
@@ -207,10 +230,98 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ 
     }
     if (tid == 0) off[0] = pre[0] = 0;
     __syncthreads();
-    for (int p = tid; p < P; p += 1024) {
+    for (int p = tid; p < P; p += NT) {
         const int e = expert_ids[p];
         if ((unsigned)e < (unsigned)E) perm[atomicAdd(&cur[e], 1)] = p;
     }
+}
+
+__global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ expert_ids, int P,
+                                                        int E, int bm, int* __restrict__ off,
+                                                        int* __restrict__ pre,
+                                                        int* __restrict__ tile_e,
+                                                        int* __restrict__ perm) {
+    __shared__ SortRoom<1024, MG_MAX_E> room;
+    moe_sort_pairs(expert_ids, P, E, bm, off, pre, tile_e, perm, room);
+}
+
+// ---- routing beside the shared expert -------------------------------------------
+// For a few tokens the routing is three launches on one to 64 blocks, one after the other, while the
+// shared expert's two products could run: their strips (skinny.hip) and the logits share a launch,
+// and so do the strips of the second product and one block that chooses and sorts for all tokens.
+// The first blocks are the routing's. Each does what its own launch does, in the same order.
+// Us inside a step, 64 experts of 1408 x 2048, top 6, a shared one of 2816, 13 tokens: five launches 29.2,
+// two 17.6 (8.4 + 9.2: the second waits for its first block, two tokens a wave one after the other, the
+// strips take 6.8). Code that runs once waits for its own fetch: with the logits of a wave's tokens
+// asked for together, in straight lines, the second launch took 14.3. For more than 16 tokens one
+// block is slow (four layers, 50 tokens 743 us, 785 with it), and with the sort apart nothing is won
+// (24 tokens 941 / 928, 32 684 / 688).
+#define MG_FRONT_E 256
+#define MG_FRONT_T 16
+
+template <int WV, int D>
+__global__ __launch_bounds__(WV * 64) void moe_front_up_kernel(
+    const uint16_t* __restrict__ x, const float* __restrict__ rw, float* __restrict__ part, int T, int E,
+    int K, int splits, const uint16_t* __restrict__ w, uint16_t* __restrict__ mid, int I) {
+    __shared__ __attribute__((aligned(16))) union {
+        mgf4 logits[4][64];
+        SkinnyRed<1, true, WV> strip;
+    } room;
+    const int te = CEIL_DIV(E, 16), logits = CEIL_DIV(T, 16) * te * splits;
+    const int at = blockIdx.x;
+    if (at < logits) moe_logits_part(x, rw, part, T, E, K, at / (te * splits), at / splits % te, at % splits, splits,
+                                     room.logits);
+    else skinny_strip<1, true, WV, D>(x, K, w, mid, T, I, K, 0, at - logits, room.strip);
+}
+
+// choice and sort of all tokens by one block of WV waves
+template <int WV>
+struct ChooseRoom {
+    float z[WV][MG_FRONT_E];
+    int ids[MG_FRONT_T * 64];
+    SortRoom<WV * 64, MG_FRONT_E> sort;
+};
+template <int WV>
+__device__ __forceinline__ void moe_choose_all(const float* __restrict__ part, int* __restrict__ idx,
+                                               float* __restrict__ wout, int T, int E, int top, int splits,
+                                               int bm, int* __restrict__ off, int* __restrict__ pre,
+                                               int* __restrict__ tile_e, int* __restrict__ perm,
+                                               ChooseRoom<WV>& room) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll 1
+    for (int t = wid; t < T; t += WV) {
+        int who;
+        float weight;
+        moe_choose_token(part, t, T, E, top, splits, room.z[wid], who, weight);
+        if (lane < top) {
+            room.ids[t * top + lane] = idx[t * top + lane] = who;
+            wout[t * top + lane] = weight;
+        }
+    }
+    __syncthreads();
+    moe_sort_pairs(room.ids, T * top, E, bm, off, pre, tile_e, perm, room.sort);
+}
+
+__global__ __launch_bounds__(1024) void moe_choose_sort_kernel(
+    const float* __restrict__ part, int* __restrict__ idx, float* __restrict__ wout, int T, int E, int top,
+    int splits, int bm, int* __restrict__ off, int* __restrict__ pre, int* __restrict__ tile_e,
+    int* __restrict__ perm) {
+    __shared__ ChooseRoom<16> room;
+    moe_choose_all(part, idx, wout, T, E, top, splits, bm, off, pre, tile_e, perm, room);
+}
+
+template <int WV, int D>
+__global__ __launch_bounds__(WV * 64) void moe_front_down_kernel(
+    const float* __restrict__ part, int* __restrict__ idx, float* __restrict__ wout, int T, int E, int top,
+    int splits, int bm, int* __restrict__ off, int* __restrict__ pre, int* __restrict__ tile_e,
+    int* __restrict__ perm, const uint16_t* __restrict__ mid, const uint16_t* __restrict__ w,
+    uint16_t* __restrict__ out, int H, int I) {
+    __shared__ __attribute__((aligned(16))) union {
+        ChooseRoom<WV> choose;
+        SkinnyRed<1, false, WV> strip;
+    } room;
+    if (blockIdx.x == 0) moe_choose_all(part, idx, wout, T, E, top, splits, bm, off, pre, tile_e, perm, room.choose);
+    else skinny_strip<1, false, WV, D>(mid, I, w, out, T, H, I, 0, blockIdx.x - 1, room.strip);
 }
 
 // ---- grouped products ---------------------------------------------------------
@@ -488,6 +599,62 @@ extern "C" int oa_moe_route(void* stream, const void* x, const void* rw, void* s
                        (float*)scratch, T, E, K);
     hipLaunchKernelGGL(moe_choose_kernel, dim3(CEIL_DIV(T, 4)), dim3(256), 0, (hipStream_t)stream,
                        (const float*)scratch, (int*)idx, (float*)w, (int*)tok, T, E, top, splits);
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
+// Router logits' parts into scratch (oa_moe_route_scratch) and, with gate_up [2I, K], beside them
+// mid [T, I] = silu(x gate^T) * (x up^T): two of the four steps of a layer's routing and shared expert.
+extern "C" int oa_moe_front_up(void* stream, const void* x, const void* rw, void* scratch, int T, int E, int K,
+                               const void* gate_up, void* mid, int I) {
+    if (T < 1 || E < 1 || E > MG_MAX_E || K < 4 || K % 4 != 0) return -100;
+    const int splits = moe_route_splits(T, E, K);
+    const int logits = CEIL_DIV(T, 16) * CEIL_DIV(E, 16) * splits;
+    hipStream_t st = (hipStream_t)stream;
+    if (!gate_up) {
+        hipLaunchKernelGGL(moe_logits_kernel, dim3(CEIL_DIV(T, 16), CEIL_DIV(E, 16), splits), dim3(256), 0, st,
+                           (const uint16_t*)x, (const float*)rw, (float*)scratch, T, E, K);
+        HIP_CHECK_LAUNCH();
+        return 0;
+    }
+    if (T > MG_FRONT_T || I < 1 || K < 32 || K % 32 != 0) return -101;
+#define MFU(WV)                                                                                        \
+    hipLaunchKernelGGL((moe_front_up_kernel<WV, 8>), dim3(logits + CEIL_DIV(I, 16)), dim3((WV) * 64), 0, \
+                       st, (const uint16_t*)x, (const float*)rw, (float*)scratch, T, E, K, splits,     \
+                       (const uint16_t*)gate_up, (uint16_t*)mid, I)
+    // the forms of oa_skinny
+    if (K <= 2048) MFU(4);
+    else MFU(8);
+#undef MFU
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
+// Choice and sort from the logits' parts (idx, w [T, top], lists as of oa_moe_sort) and, with down
+// [H, I], beside them out [T, H] = mid down^T.
+extern "C" int oa_moe_front_down(void* stream, const void* scratch, void* idx, void* w, int T, int E, int K,
+                                 int top, int bm, void* off, void* pre, void* tile_e, void* perm,
+                                 const void* mid, const void* down, void* out, int H, int I) {
+    if (T < 1 || T > MG_FRONT_T || E < 1 || E > MG_FRONT_E || top < 1 || top > E || top > 64 ||
+        (bm != 16 && bm != 32 && bm != 64 && bm != 128))
+        return -100;
+    const int splits = moe_route_splits(T, E, K);
+    hipStream_t st = (hipStream_t)stream;
+    if (!down) {
+        hipLaunchKernelGGL(moe_choose_sort_kernel, dim3(1), dim3(1024), 0, st, (const float*)scratch, (int*)idx,
+                           (float*)w, T, E, top, splits, bm, (int*)off, (int*)pre, (int*)tile_e, (int*)perm);
+        HIP_CHECK_LAUNCH();
+        return 0;
+    }
+    if (H < 1 || I < 32 || I % 32 != 0) return -101;
+#define MFD(WV)                                                                                          \
+    hipLaunchKernelGGL((moe_front_down_kernel<WV, 8>), dim3(1 + CEIL_DIV(H, 16)), dim3((WV) * 64), 0, st, \
+                       (const float*)scratch, (int*)idx, (float*)w, T, E, top, splits, bm, (int*)off,    \
+                       (int*)pre, (int*)tile_e, (int*)perm, (const uint16_t*)mid, (const uint16_t*)down, \
+                       (uint16_t*)out, H, I)
+    if (I >= 2 * H) MFD(4);
+    else MFD(8);
+#undef MFD
     HIP_CHECK_LAUNCH();
     return 0;
 }

@@ -122,6 +122,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_moe_route.restype = i
     lib.oa_moe_route_scratch.argtypes = [i, i, i]
     lib.oa_moe_route_scratch.restype = i64
+    lib.oa_moe_front_up.argtypes = [p, p, p, p, i, i, i, p, p, i]
+    lib.oa_moe_front_up.restype = i
+    lib.oa_moe_front_down.argtypes = [p, p, p, p, i, i, i, i, i, p, p, p, p, p, p, p, i, i]
+    lib.oa_moe_front_down.restype = i
     lib.oa_moe_sort.argtypes = [p, p, i, i, i, p, p, p, p]
     lib.oa_moe_sort.restype = i
     lib.oa_moe_grouped.argtypes = [p] * 10 + [i] * 8 + [f, f]

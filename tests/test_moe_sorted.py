@@ -237,3 +237,55 @@ def test_tiles_agree(monkeypatch, fp8, tiles, T, E, top, H, I):
     want = _reference(x, d13, d2, idx, wts, None, None)
     # the roundings of test_sorted_experts
     assert float((outs[0].double() - want).norm() / want.norm()) < 4e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E,top,H,I,beside", [
+    (3, 64, 6, 2048, 2816, True), (13, 64, 6, 2048, 2816, True),
+    (16, 5, 5, 512, 768, True),      # fewer experts than a block of the logits
+    (16, 100, 64, 1024, 1408, True),     # as many pairs as there are places
+    (7, 256, 8, 2048, 512, True),    # as many experts as there are places
+    (9, 8, 1, 512, 2048, True),      # long rows: four waves a strip
+    (2, 64, 6, 2048, 2816, False), (1, 40, 40, 264, 0, False), (16, 64, 6, 512, 0, False),
+])
+def test_front(T, E, top, H, I, beside):
+    """Routing, sort and the shared expert in shared launches: the bits of the separate ones, and
+    lists that name every pair once, in its expert's place."""
+    gen = torch.Generator(device="cuda").manual_seed(T + E)
+    rn = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    x, rw = rn(T, H).bfloat16(), rn(E, H) * (2.0 * H ** -0.5)
+    gate_up = (rn(2 * I, H) * H ** -0.5).bfloat16() if I else None
+    down = (rn(H, I) * I ** -0.5).bfloat16() if I else None
+    idx, wts, lists, shared = ops.moe_front(x, rw, top, 1408 * 2048, False, gate_up, down)
+    ref_idx, ref_wts, _ = ops.moe_route(x, rw, top)
+    assert torch.equal(idx, ref_idx) and torch.equal(wts, ref_wts)
+    assert (shared is not None) == beside
+    if beside:
+        act = ops._skinny(x, gate_up, 1, gateup=True)
+        assert torch.equal(shared, ops._skinny(act, down, 1))
+    P = T * top
+    bm, max_tiles, size = ops._moe_lists(P, E, 1408 * 2048, False)
+    off, pre, tile_e, perm = (t.cpu() for t in lists.split([E + 1, E + 1, max_tiles, P]))
+    count = torch.bincount(idx.flatten().cpu().long(), minlength=E)
+    tiles = (count + bm - 1) // bm
+    assert torch.equal(off[1:].long(), count.cumsum(0)) and off[0] == pre[0] == 0
+    assert torch.equal(pre[1:].long(), tiles.cumsum(0))
+    assert torch.equal(tile_e[: pre[-1]].long(), torch.arange(E).repeat_interleave(tiles))
+    assert torch.equal(perm.sort().values.long(), torch.arange(P))
+    assert torch.equal(idx.flatten().cpu()[perm.long()].long(), torch.arange(E).repeat_interleave(count))
+
+
+@pytest.mark.gpu
+def test_front_refuses():
+    """What the shared launches do not hold goes through the separate ones."""
+    x = torch.zeros(4, 512, dtype=torch.bfloat16, device="cuda")
+    rw = torch.zeros(257, 512, device="cuda")
+    assert ops.moe_front(x, rw, 2, 0, False) is None and ops.moe_front(x, rw[:256], 2, 0, False)
+    assert ops.moe_front(x.repeat(5, 1)[:17], rw[:16], 2, 0, False) is None
+    assert ops.moe_front(x[:, ::2], rw[:16, :256].contiguous(), 2, 0, False) is None
+    w = torch.zeros(2048, 512, dtype=torch.bfloat16, device="cuda")
+    down = torch.zeros(512, 1024, dtype=torch.bfloat16, device="cuda")
+    assert ops.moe_front(x, rw[:16], 2, 0, False, w, down)[3] is not None
+    for a, b in ((w.float(), down), (w, down.float()), (w, down.t().contiguous().t()),
+                 (torch.nn.Parameter(w), down)):      # other types, strides, gradients asked for
+        assert ops.moe_front(x, rw[:16], 2, 0, False, a, b)[3] is None
