@@ -265,14 +265,21 @@ class DecoderLayer(nn.Module):
             residual = x
             h = ops.rms_norm(x, self.input_norm_w, self.eps) if normed is None else normed
         else:
-            h, residual = ops.fused_add_rms_norm(x, residual, self.input_norm_w, self.eps)
+            # rows that the fp8 products would quantize next come quantized from the norm
+            low = (self.attn.fp8 and _sums_parts(self.attn) and residual.is_cuda
+                   and ops.fp8_rows_ok(*residual.shape))
+            norm = ops.fused_add_rms_norm_fp8 if low else ops.fused_add_rms_norm
+            h, residual = norm(x, residual, self.input_norm_w, self.eps)
         # the norm after a sublayer adds up its last product's parts (not what ranks add up)
         one, attn, mlp = get_tp_size() == 1, self.attn, self.mlp
         if one and _sums_parts(attn):
             a = attn(h, cos, sin, k_cache, v_cache, fb, True)
         else:
             a = attn(h, cos, sin, k_cache, v_cache, fb)
-        h, residual = ops.fused_add_rms_norm(a, residual, self.post_norm_w, self.eps)
+        low = (not self.is_moe_layer and mlp.fp8 and _sums_parts(mlp) and residual.is_cuda
+               and ops.mlp_fp8_rows_ok(*residual.shape, mlp.i_local, mlp.gate_up_q))
+        norm = ops.fused_add_rms_norm_fp8 if low else ops.fused_add_rms_norm
+        h, residual = norm(a, residual, self.post_norm_w, self.eps)
         parts = parts and one and _sums_parts(mlp)
         if self.is_moe_layer:
             decode = fb.kind == "decode"

@@ -734,6 +734,47 @@ def fused_add_rms_norm(
     return out, residual
 
 
+class QuantRows(NamedTuple):
+    """Hidden rows for fp8 products: 8-bit numbers [T, K] and a float32 scale a row."""
+
+    rows: torch.Tensor
+    scales: torch.Tensor
+
+    @property
+    def shape(self):
+        return self.rows.shape
+
+    @property
+    def is_cuda(self) -> bool:
+        return self.rows.is_cuda
+
+
+def fp8_rows_ok(rows: int, K: int) -> bool:
+    """Whether linear_fp8 of as many rows of K columns quantizes them first."""
+    return rows > 8 and K % 128 == 0 and not _fp8_mfma_ok(rows, K)
+
+
+def fused_add_rms_norm_fp8(
+    x: Union[torch.Tensor, PlaneSum, PairSum], residual: torch.Tensor, weight: torch.Tensor,
+    eps: float = 1e-5
+) -> Tuple[Union[torch.Tensor, QuantRows], torch.Tensor]:
+    """fused_add_rms_norm for fp8 products that quantize their rows (fp8_rows_ok): its first result
+    quantized, the bits of quant_fp8, in the same launch; as it is where the kernel does not take it."""
+    rows, dim = residual.shape
+    if not (isinstance(x, torch.Tensor) and x.is_cuda and x.shape == residual.shape and rows
+            and weight.numel() == dim and dim % 8 == 0 and dim <= 8192
+            and all(t.dtype == torch.bfloat16 and t.device == x.device and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 for t in (x, residual, weight))):
+        return fused_add_rms_norm(x, residual, weight, eps)
+    lib, hip = _lib()
+    q = torch.empty(rows, dim, dtype=torch.uint8, device=x.device)
+    scales = torch.empty(rows, dtype=torch.float32, device=x.device)
+    hip.check(lib.oa_fused_add_rmsnorm_fp8(
+        hip.current_stream_ptr(), x.data_ptr(), residual.data_ptr(), weight.data_ptr(), q.data_ptr(),
+        scales.data_ptr(), rows, dim, eps), "oa_fused_add_rmsnorm_fp8")
+    return QuantRows(q, scales), residual
+
+
 def rope_apply_(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -805,7 +846,7 @@ def quant_fp8(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
 
 
 def linear_fp8(
-    x: torch.Tensor, w8: torch.Tensor, w_scale: torch.Tensor
+    x: Union[torch.Tensor, QuantRows], w8: torch.Tensor, w_scale: torch.Tensor
 ) -> torch.Tensor:
     """out = (x @ dequant(w8)^T) with per-row weight scales.
 
@@ -816,7 +857,10 @@ def linear_fp8(
     variant was measured and REVERTED: 70B fp8 turn 723 ms vs 573 with the
     tile GEMM — the per-call dequant round-trip costs more than the GEMM's
     tile-pipeline inefficiency.)
-    CPU: dequantized torch reference."""
+    CPU: dequantized torch reference. x may be quantized already (fused_add_rms_norm_fp8)."""
+    if isinstance(x, QuantRows):
+        assert x.shape[1] == w8.shape[1]
+        return _gemm_fp8(x.rows, x.scales, w8, w_scale)
     M = x.numel() // x.shape[-1]
     K = x.shape[-1]
     N = w8.shape[0]
@@ -922,24 +966,31 @@ def _gemm_fp8(a8: torch.Tensor, a_scale: torch.Tensor, w8: torch.Tensor,
     return out
 
 
+def mlp_fp8_rows_ok(rows: int, K: int, i_local: int, gate_up_q: torch.Tensor) -> bool:
+    """Whether mlp_fp8 runs both products on quantized rows."""
+    return (fp8_rows_ok(rows, K) and i_local % 128 == 0 and gate_up_q.shape[0] == 2 * i_local
+            and not _fp8_mfma_ok(rows, i_local))
+
+
 def mlp_fp8(
-    x: torch.Tensor, gate_up_q: torch.Tensor, gate_up_s: torch.Tensor, i_local: int,
+    x: Union[torch.Tensor, QuantRows], gate_up_q: torch.Tensor, gate_up_s: torch.Tensor, i_local: int,
     down_q: torch.Tensor, down_s: torch.Tensor,
 ) -> torch.Tensor:
     """(silu(x @ gate8^T) * (x @ up8^T)) @ down8^T. Where both products are tile
     products (prefill rows), the activation is quantized as it is made: the same bf16
-    values, rows and scales as quantizing it afterwards."""
-    M, K = x.numel() // x.shape[-1], x.shape[-1]
-    if not (
-        _is_gpu(x) and M > 8 and K % 128 == 0 and i_local % 128 == 0
-        and gate_up_q.shape[0] == 2 * i_local
-        and not _fp8_mfma_ok(M, K) and not _fp8_mfma_ok(M, i_local)
-    ):
+    values, rows and scales as quantizing it afterwards. x may be quantized already, where
+    mlp_fp8_rows_ok says so."""
+    if isinstance(x, QuantRows):
+        M, tiles = x.shape[0], True
+    else:
+        M = x.numel() // x.shape[-1]
+        tiles = _is_gpu(x) and mlp_fp8_rows_ok(M, x.shape[-1], i_local, gate_up_q)
+    if not tiles:
         return linear_fp8(gateup_silu_fp8(x, gate_up_q, gate_up_s, i_local), down_q, down_s)
     gu = linear_fp8(x, gate_up_q, gate_up_s)
     lib, hip = _lib()
-    a8 = torch.empty(M, i_local, dtype=torch.uint8, device=x.device)
-    a_scale = torch.empty(M, dtype=torch.float32, device=x.device)
+    a8 = torch.empty(M, i_local, dtype=torch.uint8, device=gu.device)
+    a_scale = torch.empty(M, dtype=torch.float32, device=gu.device)
     hip.check(lib.oa_silu_quant_fp8(hip.current_stream_ptr(), gu.data_ptr(), a8.data_ptr(),
                                     a_scale.data_ptr(), M, i_local), "oa_silu_quant_fp8")
     return _gemm_fp8(a8, a_scale, down_q, down_s).view(*x.shape[:-1], down_q.shape[0])

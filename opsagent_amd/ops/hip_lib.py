@@ -41,6 +41,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_add_rmsnorm_parts.restype = i
     lib.oa_fused_add_rmsnorm.argtypes = [p, p, p, p, p, i, i, f]
     lib.oa_fused_add_rmsnorm.restype = i
+    lib.oa_fused_add_rmsnorm_fp8.argtypes = [p, p, p, p, p, p, i, i, f]
+    lib.oa_fused_add_rmsnorm_fp8.restype = i
     lib.oa_rope.argtypes = [p, p, p, p, p, p, i, i, i, i]
     lib.oa_rope.restype = i
     lib.oa_silu_mul.argtypes = [p, p, p, p, i64]

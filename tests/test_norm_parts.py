@@ -149,3 +149,58 @@ def test_planes_on_the_cpu():
     for got, want in zip(ops.fused_add_rms_norm(ops.PlaneSum(x), residual, w),
                          ops.fused_add_rms_norm(total, residual, w)):
         assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,D", [(1, 8), (3, 2048), (17, 2056), (70, 4096), (5, 8192)])
+def test_norm_in_8_bits(T, D):
+    """The bits of the norm and of quant_fp8 behind it; rows of zeros and of infinities among them."""
+    g = torch.Generator(device="cuda").manual_seed(D + T)
+    x, residual = (torch.randn(T, D, generator=g, device="cuda").bfloat16() for _ in range(2))
+    w = (1 + 0.1 * torch.randn(D, generator=g, device="cuda")).bfloat16()
+    x[-1], residual[-1] = 0, 0
+    if T > 2:
+        x[1, D // 2] = float("inf")
+    h, want_r = ops.fused_add_rms_norm(x, residual.clone(), w, 1e-5)
+    want, scales = ops.quant_fp8(h)
+    got, got_r = ops.fused_add_rms_norm_fp8(x, residual, w, 1e-5)
+    assert isinstance(got, ops.QuantRows) and got_r.data_ptr() == residual.data_ptr()
+    assert torch.equal(got_r, want_r) and torch.equal(got.rows, want)
+    assert torch.equal(got.scales.view(torch.int32), scales.view(torch.int32))
+
+
+@pytest.mark.gpu
+def test_norm_in_8_bits_refuses():
+    """Sums that the kernel does not take are normed as they were."""
+    x = torch.randn(4, 64, device="cuda").bfloat16()
+    w = torch.ones(64, device="cuda").bfloat16()
+    parts = ops.PlaneSum(x.float()[None])
+    got, _ = ops.fused_add_rms_norm_fp8(parts, x.clone(), w, 1e-5)
+    want, _ = ops.fused_add_rms_norm(parts, x.clone(), w, 1e-5)
+    assert isinstance(got, torch.Tensor) and torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [9, 24, 150])
+def test_fp8_layers_with_rows_in_8_bits(tokens):
+    """A model's hidden rows are the bits of those where a hook has every norm write bf16 rows."""
+    from opsagent_amd.engine.config import ModelSpec
+    from opsagent_amd.engine.model import ForwardBatch, LlamaForCausalLM
+
+    spec = ModelSpec(name="fp8", max_seq_len=512, hidden_size=1024, num_heads=8, num_kv_heads=2,
+                     head_dim=128, intermediate_size=2048, num_layers=3, vocab_size=512)
+    model = LlamaForCausalLM(spec, torch.bfloat16, "cuda", seed=1).eval()
+    model.quantize_fp8_()
+    pos = torch.arange(tokens, dtype=torch.int32, device="cuda")
+    fb = ForwardBatch(kind="prefill", input_ids=pos.long() + 3, positions=pos, slot_mapping=pos)
+    cache = [tuple(torch.zeros(16, 32, 2, 128, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+             for _ in range(3)]
+    with torch.inference_mode():
+        got = model(fb, cache)
+        seen = []
+        for layer in model.layers:
+            for m in (layer.attn, layer.mlp):
+                m.register_forward_pre_hook(lambda m, args: seen.append(args[0]))
+        want = model(fb, cache)
+    assert all(isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 for x in seen) and len(seen) == 6
+    assert torch.equal(got, want)
