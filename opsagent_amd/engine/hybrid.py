@@ -151,12 +151,10 @@ class BiasedAttentionMixer(nn.Module):
 
     def forward(self, h, sb: mx.SeqBatch, kv, state) -> torch.Tensor:
         k_cache, v_cache = kv
-        proj = ops.linear(h, self.proj_w)                     # [T, q|k|v|gate]
-        q = mx.attn_qkv_prepare(proj, self.proj_b, self.q_norm_w, self.k_norm_w,
-                                self.H, self.G, self.D, self.Dv, self.eps,
-                                k_cache, v_cache, sb)
-        ctx = mx.attention_biased_paged(q, proj[:, self.n_qkv:], k_cache, v_cache, sb,
-                                        self.scale, self.slopes)
+        q, gate = mx.attn_proj_prepare(h, self.proj_w, self.proj_b, self.q_norm_w, self.k_norm_w,
+                                       self.H, self.G, self.D, self.Dv, self.eps,
+                                       k_cache, v_cache, sb)
+        ctx = mx.attention_biased_paged(q, gate, k_cache, v_cache, sb, self.scale, self.slopes)
         return ops.linear(ctx, self.o_w)
 
 
@@ -994,6 +992,8 @@ class PlainMLP(nn.Module):
 
 
 class HybridLayer(nn.Module):
+    sums_parts = True           # see _sums_parts
+
     def __init__(self, spec: HybridSpec, ls: HybridLayerSpec, dtype, gen):
         super().__init__()
         C = spec.hidden_size
@@ -1011,19 +1011,23 @@ class HybridLayer(nn.Module):
         shapes["canon"] = (self.canon_w.shape[1] - 1, self.canon_w.shape[0])
         return shapes
 
-    def forward(self, x: torch.Tensor, sb: mx.SeqBatch, kv, state) -> torch.Tensor:
-        """x: float32 residual [T, C], updated in place and returned."""
-        h = mx.causal_conv_seq(x, self.canon_w, state["canon"], sb,
-                               add_input=True, act_silu=False)
+    def forward(self, x: torch.Tensor, sb: mx.SeqBatch, kv, state, h=None, nxt=None):
+        """x: float32 residual [T, C], updated in place and returned. h: the convolution of x that
+        the layer starts with, where the last norm before it had that (nxt, the following layer's
+        weight and carried inputs, returned beside x)."""
+        if h is None:
+            h = mx.causal_conv_seq(x, self.canon_w, state["canon"], sb,
+                                   add_input=True, act_silu=False)
         y = self.mixer(h, sb, kv, state)
         narrow = self.mlp is not None and self.norm1_w.dtype != torch.float32
-        x, copy = mx.group_rms_norm(y, self.norm1_w, self.groups, self.eps,
-                                    residual=x, want_copy=narrow)
+        x, copy, h = mx.group_norm_step(y, self.norm1_w, self.groups, self.eps, x, narrow,
+                                        nxt if self.mlp is None else None, sb)
         if self.mlp is not None:
-            m = self.mlp(copy if narrow else x)
-            x, _ = mx.group_rms_norm(m, self.norm2_w, self.groups, self.eps,
-                                     residual=x, want_copy=False)
-        return x
+            m = copy if narrow else x
+            m = (ops.linear_parts(self.mlp.inner(m), self.mlp.down_w) if _sums_parts(self.mlp)
+                 else self.mlp(m))
+            x, _, h = mx.group_norm_step(m, self.norm2_w, self.groups, self.eps, x, False, nxt, sb)
+        return x if nxt is None else (x, h)
 
 
 class DyTNorm(nn.Module):
@@ -1494,8 +1498,15 @@ class HybridForCausalLM(nn.Module):
                 if self.trace_layers is not None:
                     self.trace_layers.append(x.clone())
             return x
-        for i, layer in enumerate(self.layers):
-            x = layer(x, sb, kv_caches[i], state[i])
+        layers, h = list(self.layers), None
+        # what goes into a layer that is looked at may change on the way: it starts by itself then
+        joined = all(map(_sums_parts, layers))
+        for i, layer in enumerate(layers):
+            if joined and i + 1 < len(layers):
+                nxt = (layers[i + 1].canon_w, state[i + 1]["canon"])
+                x, h = layer(x, sb, kv_caches[i], state[i], h, nxt)
+            else:
+                x, h = layer(x, sb, kv_caches[i], state[i], h), None
             if self.trace_layers is not None:
                 self.trace_layers.append(x.clone())
         return x  # float32 residual [T, C]; compute_logits norms the rows it needs

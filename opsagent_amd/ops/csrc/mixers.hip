@@ -252,6 +252,99 @@ __global__ __launch_bounds__(256) void group_rmsnorm_vec_kernel(
     }
 }
 
+// The form for decode steps and split products, every element held by a thread of its own (8 columns each;
+// parts of whole waves, at most 8192 columns): y may be the ny float32 planes of a product (yp elements
+// apart), added up in order and rounded as the product alone would be. TP > 0, for steps of one token per
+// sequence: behind it goes what causal_conv_small_kernel would do with the new residual, h = residual +
+// conv(residual), TP taps, and the carried inputs move on. A launch of four rows is its chain of loads, so
+// all are asked for before the first sum; padding rows of a captured launch leave h and the carried
+// inputs alone.
+// us, launches apart / here: 4 rows of 4096, parts of a product, norm, convolution 14.6 / 5.0 (a wave for
+// each part of 1024: 8.3); parts and norm of 1434 rows 23.8 / 16.7.
+template <typename TY, int TP>
+__global__ __launch_bounds__(1024) void group_norm_step_kernel(
+    const TY* __restrict__ y, int64_t ys, int ny, int64_t yp, const bf16s* __restrict__ w,
+    float* __restrict__ residual, bf16s* __restrict__ copy, int C, int gs, float eps,
+    const bf16s* __restrict__ cw, float* __restrict__ state, bf16s* __restrict__ h,
+    const int* __restrict__ seq_of, const int* __restrict__ cu, const int* __restrict__ past,
+    const int* __restrict__ slots, int B) {
+    __shared__ float red[16];
+    constexpr int KEPT = TP > 1 ? TP - 1 : 1;
+    const int t = blockIdx.x, c = threadIdx.x * 8;
+    const int wave = threadIdx.x >> 6, per = gs >> 9;       // waves of a part
+    const int64_t at = (int64_t)t * C + c;
+    float v[8], rv[8], wv[8], kept[KEPT][8];
+    raw8 tap[TP > 0 ? TP : 1];
+    ld8(y, (int64_t)t * ys + c, v);
+    ld8(residual, at, rv);
+    ld8(w, c, wv);
+    if constexpr (sizeof(TY) == 4) {
+#pragma unroll 4
+        for (int k = 1; k < ny; ++k) {
+            float a[8];
+            ld8(y, k * yp + (int64_t)t * ys + c, a);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] += a[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = bf16_to_f32(f32_to_bf16(v[e]));
+    }
+    bool live = false;
+    int before = 0;
+    float* st = nullptr;
+    if constexpr (TP > 0) {
+#pragma unroll
+        for (int j = 0; j < TP; ++j) ldraw8(cw, (int64_t)c * TP + j * 8, tap[j]);
+        live = t < cu[B];
+        if (live) {
+            const int b = seq_of[t];
+            before = past[b];
+            st = state + (int64_t)slots[b] * (TP - 1) * C + c;
+#pragma unroll
+            for (int j = 0; j < TP - 1; ++j) ld8(st, (int64_t)j * C, kept[j]);
+        }
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+    ss = wave_reduce_sum(ss);
+    if (per > 1) {
+        if ((threadIdx.x & 63) == 0) red[wave] = ss;
+        __syncthreads();
+        const int first = wave / per * per;
+        ss = 0.0f;
+        for (int i = 0; i < per; ++i) ss += red[first + i];
+    }
+    const float r = 1.0f / sqrtf(ss / (float)gs + eps);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = v[e] * r * wv[e] + rv[e];
+    st8(residual, at, v);
+    if (copy) st8(copy, at, v);
+    if constexpr (TP > 0) {
+        if (!live) return;
+        float f[TP][8], o[8];
+#pragma unroll
+        for (int j = 0; j < TP; ++j) unraw8(cw, tap[j], f[j]);
+        // inputs before the first token are zero
+#pragma unroll
+        for (int j = 0; j < TP - 1; ++j)
+            if (before + j < TP - 1)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) kept[j][e] = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float acc = 0.0f;
+#pragma unroll
+            for (int j = 0; j < TP; ++j)              // the taps of a channel lie together
+                acc += f[(e * TP + j) / 8][(e * TP + j) % 8] * (j < TP - 1 ? kept[j][e] : v[e]);
+            o[e] = acc + v[e];
+        }
+        st8(h, at, o);
+#pragma unroll
+        for (int j = 0; j < TP - 1; ++j) st8(st, (int64_t)j * C, j < TP - 2 ? kept[j + 1 < KEPT ? j + 1 : j] : v);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Attention input preparation, one block per token: the projection biases
 // are added (bias over q | k | v columns, may be null), then weighted RMS
@@ -397,6 +490,85 @@ __global__ __launch_bounds__(256) void attn_prepare_vec_kernel(
             for (int e = 0; e < 8; ++e) x[e] *= rv;
             st8(v_cache, slot * (int64_t)(G * Dv) + g * Dv + i, x);
         }
+    }
+}
+
+// The same with every element held by a thread of its own, 8 columns each (at most 8192 in all): the
+// row is read once, and rows, biases and weights are asked for together. A value head is Dv / 8 lanes
+// next to each other (a power of two; q and k end on a whole head). PARTS: the row is the sum of a
+// product's float32 planes, rounded as the product alone would be, and its columns behind q | k | v
+// are written to `rest`.
+// us, attn_prepare_vec_kernel / here: 4 rows of 6176 columns with the launch that added the planes up
+// 16.3 / 5.4, 1434 rows of 6144 15.9 / 14.2.
+template <typename TC, bool PARTS>
+__global__ __launch_bounds__(1024) void attn_prepare_row_kernel(
+    const TC* __restrict__ qkv, int64_t qs, const float* __restrict__ part, int splits, int64_t plane,
+    const TC* __restrict__ bias, const TC* __restrict__ qw, const TC* __restrict__ kw,
+    TC* __restrict__ q_out, TC* __restrict__ k_cache, TC* __restrict__ v_cache, TC* __restrict__ rest,
+    const int* __restrict__ slot_mapping, const int* __restrict__ cu, int B, int nq, int nk, int Dv,
+    int n, int N, float eps) {
+    __shared__ float red[2][16];
+    const int t = blockIdx.x, i = threadIdx.x * 8;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int64_t slot = slot_mapping[t];
+    const int end = cu[B];
+    float x[8], bv[8], wv[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = bv[e] = wv[e] = 0.0f;
+    if (i < N) {
+        if (i < nq) ld8(qw, i, wv);
+        else if (i < nq + nk) ld8(kw, i - nq, wv);
+        if (bias && i < n) ld8(bias, i, bv);
+        if constexpr (PARTS) {
+            const float* p = part + (int64_t)t * N + i;
+            ld8(p, 0, x);
+#pragma unroll 4
+            for (int s = 1; s < splits; ++s) {
+                float a[8];
+                ld8(p, s * plane, a);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] += a[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = bf16_to_f32(f32_to_bf16(x[e]));
+        } else {
+            ld8(qkv, t * qs + i, x);
+        }
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        x[e] += bv[e];
+        ss += x[e] * x[e];
+    }
+    const float sq = wave_reduce_sum(i < nq ? ss : 0.0f);
+    const float sk = wave_reduce_sum(i >= nq && i < nq + nk ? ss : 0.0f);
+    for (int m = Dv / 16; m > 0; m >>= 1) ss += __shfl_xor(ss, m, WAVE);
+    if (lane == 0) {
+        red[0][wave] = sq;
+        red[1][wave] = sk;
+    }
+    __syncthreads();
+    if (i >= N) return;
+    if (i >= n) {
+        st8(rest, (int64_t)t * (N - n) + i - n, x);
+        return;
+    }
+    if (t >= end) return;                            // padding row of a captured launch
+    if (i < nq + nk) {
+        const bool key = i >= nq;
+        float sum = 0.0f;
+        for (int j = 0; j < nw; ++j) sum += red[key][j];
+        const float r = 1.0f / sqrtf(sum / (float)(key ? nk : nq) + eps);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] *= r * wv[e];
+        if (key) st8(k_cache, slot * nk + i - nq, x);
+        else st8(q_out, (int64_t)t * nq + i, x);
+    } else {
+        const float r = 1.0f / sqrtf(ss / (float)Dv + eps);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] *= r;
+        st8(v_cache, slot * (n - nq - nk) + i - nq - nk, x);
     }
 }
 
@@ -2114,6 +2286,73 @@ extern "C" int oa_group_rmsnorm(void* stream, const void* y, int64_t ys, int y_d
     return 0;
 }
 
+// residual += norm(y) * w in bf16, as above; y: ny float32 planes yp elements apart, or (ny 0) bf16 rows.
+// taps > 0, for steps of one token per sequence: then h = residual + conv(residual; cw), state carried on.
+extern "C" int oa_group_norm_step(void* stream, const void* y, int64_t ys, int ny, int64_t yp, const void* w,
+                                  void* residual, void* copy, int T, int C, int groups, float eps, const void* cw,
+                                  void* state, void* h, const void* seq_of, const void* cu, const void* past,
+                                  const void* slots, int B, int taps) {
+    if (T <= 0) return 0;
+    if (groups < 1 || C % groups != 0 || C / groups % 512 != 0 || C > 8192) return -100;
+    if (!y || !w || !residual || ny < 0 || ys % 8 != 0 || yp % 8 != 0) return -101;
+    if (taps != 0 && (taps < 2 || taps > 4 || !cw || !state || !h)) return -103;
+    if (((uintptr_t)y | (uintptr_t)w | (uintptr_t)residual | (uintptr_t)copy | (uintptr_t)cw | (uintptr_t)state |
+         (uintptr_t)h) % 16 != 0)
+        return -102;
+#define GS(TY, TP)                                                                                                  \
+    hipLaunchKernelGGL((group_norm_step_kernel<TY, TP>), dim3(T), dim3(C / 8), 0, (hipStream_t)stream,              \
+                       (const TY*)y, ys, ny, yp, (const bf16s*)w, (float*)residual, (bf16s*)copy, C, C / groups,    \
+                       eps,                                                                                         \
+                       (const bf16s*)cw, (float*)state, (bf16s*)h, (const int*)seq_of, (const int*)cu,              \
+                       (const int*)past, (const int*)slots, B)
+#define GST(TY)                            \
+    do {                                   \
+        if (taps == 0) GS(TY, 0);          \
+        else if (taps == 2) GS(TY, 2);     \
+        else if (taps == 3) GS(TY, 3);     \
+        else GS(TY, 4);                    \
+    } while (0)
+    if (ny > 0) GST(float);
+    else GST(bf16s);
+#undef GST
+#undef GS
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
+// what attn_prepare_row_kernel takes: N columns in all
+static bool prepare_row_ok(int H, int G, int D, int Dv, int N) {
+    return D % 8 == 0 && Dv % 8 == 0 && Dv <= 512 && (Dv & (Dv - 1)) == 0 && (H + G) * D % Dv == 0 &&
+           N % 8 == 0 && N <= 8192;
+}
+
+template <typename TC, bool PARTS>
+static int prepare_row(hipStream_t s, const void* qkv, int64_t qs, const void* part, int splits, const void* bias,
+                       const void* qw, const void* kw, void* q_out, void* k_cache, void* v_cache, void* rest,
+                       const void* slot_mapping, const void* cu, int B, int T, int H, int G, int D, int Dv, int N,
+                       float eps) {
+    hipLaunchKernelGGL((attn_prepare_row_kernel<TC, PARTS>), dim3(T), dim3(CEIL_DIV(N / 8, 64) * 64), 0, s,
+                       (const TC*)qkv, qs, (const float*)part, splits, (int64_t)T * N, (const TC*)bias, (const TC*)qw,
+                       (const TC*)kw, (TC*)q_out, (TC*)k_cache, (TC*)v_cache, (TC*)rest, (const int*)slot_mapping,
+                       (const int*)cu, B, H * D, G * D, Dv, (H + G) * D + G * Dv, N, eps);
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
+// oa_attn_prepare in bf16 of a product that is still its float32 planes part [splits, T, N]; its columns
+// behind q | k | v go to rest [T, N - ...]
+extern "C" int oa_attn_prepare_parts(void* stream, const void* part, int splits, const void* bias, const void* qw,
+                                     const void* kw, void* q_out, void* k_cache, void* v_cache, void* rest,
+                                     const void* slot_mapping, const void* cu, int B, int T, int H, int G, int D,
+                                     int Dv, int N, float eps) {
+    if (T <= 0) return 0;
+    const int n = (H + G) * D + G * Dv;
+    if (!prepare_row_ok(H, G, D, Dv, N) || n % 8 != 0 || N < n || splits < 1 || (N > n && !rest)) return -100;
+    if (((uintptr_t)part | (uintptr_t)bias | (uintptr_t)qw | (uintptr_t)kw | (uintptr_t)rest) % 16 != 0) return -102;
+    return prepare_row<bf16s, true>((hipStream_t)stream, nullptr, 0, part, splits, bias, qw, kw, q_out, k_cache,
+                                    v_cache, rest, slot_mapping, cu, B, T, H, G, D, Dv, N, eps);
+}
+
 extern "C" int oa_attn_prepare(void* stream, const void* qkv, int64_t qs, const void* bias, const void* qw,
                                const void* kw, void* q_out, void* k_cache, void* v_cache,
                                const void* slot_mapping, const void* cu, int B, int T, int H,
@@ -2122,6 +2361,13 @@ extern "C" int oa_attn_prepare(void* stream, const void* qkv, int64_t qs, const 
     hipStream_t s = (hipStream_t)stream;
     if (D % 8 == 0 && Dv % 8 == 0 && qs % 8 == 0 && (uintptr_t)qkv % 32 == 0 &&
         (!bias || (uintptr_t)bias % 32 == 0)) {
+        if (prepare_row_ok(H, G, D, Dv, (H + G) * D + G * Dv)) {
+            if (dt == 1) return prepare_row<float, false>(s, qkv, qs, nullptr, 0, bias, qw, kw, q_out, k_cache,
+                                                          v_cache, nullptr, slot_mapping, cu, B, T, H, G, D, Dv,
+                                                          (H + G) * D + G * Dv, eps);
+            return prepare_row<bf16s, false>(s, qkv, qs, nullptr, 0, bias, qw, kw, q_out, k_cache, v_cache, nullptr,
+                                             slot_mapping, cu, B, T, H, G, D, Dv, (H + G) * D + G * Dv, eps);
+        }
         if (dt == 1)
             hipLaunchKernelGGL((attn_prepare_vec_kernel<float>), dim3(T), dim3(256), 0, s, (const float*)qkv,
                                qs, (const float*)bias, (const float*)qw, (const float*)kw, (float*)q_out,

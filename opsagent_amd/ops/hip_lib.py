@@ -172,6 +172,8 @@ def _declare_mixers(lib: ctypes.CDLL) -> None:
     f = ctypes.c_float
     ip = ctypes.POINTER(ctypes.c_int)
     sigs = {
+        "oa_group_norm_step": [p, p, i64, i, i64, p, p, p, i, i, i, f, p, p, p, p, p, p, p, i, i],
+        "oa_attn_prepare_parts": [p, p, i, p, p, p, p, p, p, p, p, p, i, i, i, i, i, i, i, f],
         "oa_causal_conv_seq": [p, p, i64, i, p, p, p, i64, p, p, p, p, i, i, i, i, i, i, i, i],
         "oa_group_rmsnorm": [p, p, i64, i, p, p, p, i, i, i, f, i],
         "oa_attn_prepare": [p, p, i64, p, p, p, p, p, p, p, p, i, i, i, i, i, i, f, i],

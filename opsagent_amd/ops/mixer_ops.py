@@ -14,7 +14,7 @@ from __future__ import annotations
 import ctypes
 import dataclasses
 import os
-from typing import List, Optional, Tuple
+from typing import List, Optional, Tuple, Union
 
 import numpy as np
 import torch
@@ -190,6 +190,57 @@ def group_rms_norm(y: torch.Tensor, w: torch.Tensor, groups: int, eps: float,
     return residual, copy
 
 
+def group_norm_step(y: Union[torch.Tensor, "ops.PlaneSum"], w: torch.Tensor, groups: int, eps: float,
+                    residual: torch.Tensor, want_copy: bool = True,
+                    conv: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
+                    sb: Optional[SeqBatch] = None) -> Tuple[torch.Tensor, Optional[torch.Tensor],
+                                                            Optional[torch.Tensor]]:
+    """group_rms_norm onto `residual`, and with conv = (weight, carried inputs) what
+    causal_conv_seq(residual, weight, inputs, sb, add_input=True, act_silu=False) gives: (residual,
+    copy, that or None). y may be a product's parts (ops.linear_parts). In bf16 parts are added up in
+    the norm's launch, and steps of one token per sequence take the convolution along."""
+    from opsagent_amd import ops
+
+    T, C = residual.shape
+    planes = y.planes if isinstance(y, ops.PlaneSum) else None
+    join = conv is not None and sb.max_chunk == 1 and _conv_joins(*conv, C)
+    data = y if planes is None else planes
+    if (residual.is_cuda and (join or planes is not None) and w.dtype == torch.bfloat16
+            and data.dtype == (torch.bfloat16 if planes is None else torch.float32)
+            and residual.dtype == torch.float32 and residual.is_contiguous() and w.is_contiguous()
+            and C % groups == 0 and C // groups % 512 == 0 and C <= 8192
+            and data.shape[-2:] == (T, C) and data.stride(-1) == 1 and data.stride(-2) % 8 == 0
+            and (planes is None or planes.is_contiguous())
+            and (data.data_ptr() | w.data_ptr() | residual.data_ptr()) % 16 == 0):
+        lib, hip = _lib()
+        copy, h = (torch.empty(T, C, dtype=w.dtype, device=w.device) if wanted else None
+                   for wanted in (want_copy, join))
+        geometry = (sb.seq_of_t, sb.cu_t, sb.past_t, sb.slots_t) if join else (None,) * 4
+        hip.check(lib.oa_group_norm_step(
+            hip.current_stream_ptr(), data.data_ptr(), data.stride(-2),
+            0 if planes is None else planes.shape[0], T * C, w.data_ptr(), residual.data_ptr(),
+            copy.data_ptr() if want_copy else None, T, C, groups, eps,
+            *(t.data_ptr() if t is not None else None
+              for t in ((*conv, h) if join else (None,) * 3) + geometry),
+            sb.num_seqs if join else 0, conv[0].shape[1] if join else 0), "oa_group_norm_step")
+    else:
+        join = False
+        if planes is not None:
+            y = ops._added_up(y)
+        residual, copy = group_rms_norm(y, w, groups, eps, residual, want_copy)
+    if conv is not None and not join:
+        h = causal_conv_seq(residual, *conv, sb, add_input=True, act_silu=False)
+    return residual, copy, h if conv is not None else None
+
+
+def _conv_joins(w: torch.Tensor, state: torch.Tensor, C: int) -> bool:
+    """Whether the norm before a convolution of one token per sequence takes it along."""
+    return (w.is_cuda and w.dtype == torch.bfloat16 and w.shape[0] == C and 2 <= w.shape[1] <= 4
+            and state.dtype == torch.float32 and state.shape[1:] == (w.shape[1] - 1, C)
+            and w.is_contiguous() and state.is_contiguous()
+            and (w.data_ptr() | state.data_ptr()) % 16 == 0)
+
+
 def attn_qkv_prepare(qkv: torch.Tensor, bias: Optional[torch.Tensor], q_norm_w: torch.Tensor, k_norm_w: torch.Tensor,
                      H: int, G: int, D: int, Dv: int, eps: float, k_cache: torch.Tensor,
                      v_cache: torch.Tensor, sb: SeqBatch) -> torch.Tensor:
@@ -213,6 +264,37 @@ def attn_qkv_prepare(qkv: torch.Tensor, bias: Optional[torch.Tensor], q_norm_w: 
         _dt(qkv))
     hip.check(rc, "oa_attn_prepare")
     return q
+
+
+def attn_proj_prepare(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor, q_norm_w: torch.Tensor,
+                      k_norm_w: torch.Tensor, H: int, G: int, D: int, Dv: int, eps: float,
+                      k_cache: torch.Tensor, v_cache: torch.Tensor,
+                      sb: SeqBatch) -> Tuple[torch.Tensor, torch.Tensor]:
+    """attn_qkv_prepare of x @ w^T: (q, the product's columns behind q | k | v). Up to 128 rows of
+    bf16 the preparation adds up the product's parts where it is split (ops.linear_parts)."""
+    from opsagent_amd import ops
+
+    T, n, N = x.shape[0], (H + G) * D + G * Dv, w.shape[0]
+    if (x.is_cuda and T <= 128 and x.dtype == torch.bfloat16 and D % 8 == 0 and Dv % 8 == 0
+            and Dv <= 512 and Dv & (Dv - 1) == 0 and (H + G) * D % Dv == 0 and N % 8 == 0 and n < N <= 8192
+            and k_cache.dtype == v_cache.dtype == x.dtype and k_cache.is_contiguous() and v_cache.is_contiguous()
+            and all(t.dtype == x.dtype and t.is_contiguous() and t.data_ptr() % 16 == 0
+                    for t in (bias, q_norm_w, k_norm_w))):
+        p = ops.linear_parts(x, w)
+    else:
+        p = ops.linear(x, w)
+    if isinstance(p, torch.Tensor):
+        return attn_qkv_prepare(p, bias, q_norm_w, k_norm_w, H, G, D, Dv, eps, k_cache, v_cache, sb), p[:, n:]
+    assert k_cache.shape[2:] == (G, D) and v_cache.shape[2:] == (G, Dv)
+    lib, hip = _lib()
+    q = torch.empty(T, H, D, dtype=x.dtype, device=x.device)
+    rest = torch.empty(T, N - n, dtype=x.dtype, device=x.device)
+    hip.check(lib.oa_attn_prepare_parts(
+        hip.current_stream_ptr(), p.planes.data_ptr(), p.planes.shape[0], bias.data_ptr(),
+        q_norm_w.data_ptr(), k_norm_w.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+        rest.data_ptr(), sb.slot_mapping.data_ptr(), sb.cu_t.data_ptr(), sb.num_seqs, T, H, G, D, Dv,
+        N, eps), "oa_attn_prepare_parts")
+    return q, rest
 
 
 _GEOM = {}
