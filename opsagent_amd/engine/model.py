@@ -17,7 +17,7 @@ from __future__ import annotations
 
 import dataclasses
 import math
-from typing import List, Optional, Tuple
+from typing import List, Optional, Tuple, Union
 
 import torch
 import torch.nn.functional as F
@@ -120,9 +120,15 @@ class Attention(nn.Module):
         self.o_w = nn.Parameter(_shard(o_w, 1, rank, tp), requires_grad=False)
         self.fp8 = False  # set by LlamaForCausalLM.quantize_fp8_
 
-    def _qkv(self, x: torch.Tensor) -> torch.Tensor:
+    def _qkv(self, x: torch.Tensor, fused: bool) -> Union[torch.Tensor, ops.PlaneSum]:
+        """The q | k | v rows, or, up to 128 of them, the parts of a split product where what reads
+        them next adds them up (fused: the decode attention, else the rotation)."""
         if self.fp8:
             return ops.linear_fp8(x, self.qkv_q, self.qkv_s)
+        T, D = x.shape[0], self.hd
+        if (1 < T <= 128 and x.is_cuda and D % 16 == 0 and (
+                not fused or ops.decode_takes_parts(T, self.hq, self.hk, D))):
+            return ops.linear_parts(x, self.qkv_w)
         return ops.linear(x, self.qkv_w)
 
     def _o(self, x: torch.Tensor, parts: bool = False) -> torch.Tensor:
@@ -141,7 +147,18 @@ class Attention(nn.Module):
         parts: bool = False,      # the output may be a product's parts (ops.linear_parts)
     ) -> torch.Tensor:
         T = x.shape[0]
-        qkv = self._qkv(x)  # hipBLASLt / HIP gemv / fp8 at decode
+        fused = fb.kind == "decode" and x.is_cuda and _rope_attn_fused()
+        qkv = self._qkv(x, fused)  # hipBLASLt / HIP gemv / fp8 at decode
+        if isinstance(qkv, ops.PlaneSum):
+            if fused:
+                out = ops.attention_decode_parts(
+                    qkv, self.hq, self.hk, self.hd, k_cache, v_cache, fb.block_table, fb.seq_lens,
+                    cos, sin, fb.slot_mapping, self.scale, fb.decode_workspace, fb.nsplit,
+                ).view(T, self.hq * self.hd)
+                return tp_all_reduce(self._o(out, parts))
+            q, k, v = ops.rope_kv_parts(qkv, self.hq, self.hk, self.hd, k_cache, v_cache,
+                                        cos, sin, fb.positions, fb.slot_mapping)
+            return self._attend(q, k, v, k_cache, v_cache, fb, parts)
         q, k, v = qkv.split(
             [self.hq * self.hd, self.hk * self.hd, self.hk * self.hd], dim=-1
         )
@@ -152,7 +169,7 @@ class Attention(nn.Module):
         v = v.view(T, self.hk, self.hd)
         if not x.is_cuda:
             q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-        if fb.kind == "decode" and x.is_cuda and _rope_attn_fused():
+        if fused:
             # fully-fused decode attention (RoPE + KV scatter in-kernel)
             out = ops.attention_decode_rope(
                 q, k, v, k_cache, v_cache, fb.block_table, fb.seq_lens,
@@ -164,7 +181,11 @@ class Attention(nn.Module):
         q, k, v = ops.rope_kv_fused(
             q, k, v, k_cache, v_cache, cos, sin, fb.positions, fb.slot_mapping
         )
+        return self._attend(q, k, v, k_cache, v_cache, fb, parts)
 
+    def _attend(self, q, k, v, k_cache, v_cache, fb: ForwardBatch, parts: bool) -> torch.Tensor:
+        """Attention of rotated rows whose keys and values are in the cache, and the output product."""
+        T = q.shape[0]
         if fb.kind == "prefill":
             slots = None
             if fb.prefill_past_len > 0:

@@ -1408,6 +1408,26 @@ def rope_kv_fused(
     return q, k, v
 
 
+def rope_kv_parts(parts: PlaneSum, Hq: int, Hk: int, D: int, k_cache: torch.Tensor,
+                  v_cache: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+                  positions: torch.Tensor, slot_mapping: torch.Tensor
+                  ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """rope_kv_fused of a q | k | v product that is not added up yet (linear_parts)."""
+    planes = parts.planes
+    n, T, width = planes.shape
+    assert width == (Hq + 2 * Hk) * D and planes.is_contiguous() and planes.dtype == torch.float32
+    assert cos.dtype == torch.float32 and k_cache.dtype == v_cache.dtype == torch.bfloat16
+    assert positions.dtype == torch.int32 and slot_mapping.dtype == torch.int32
+    lib, hip = _lib()
+    qkv = torch.empty(T, width, dtype=k_cache.dtype, device=planes.device)
+    hip.check(lib.oa_rope_kv_parts(
+        hip.current_stream_ptr(), planes.data_ptr(), n, qkv.data_ptr(), k_cache.data_ptr(),
+        v_cache.data_ptr(), cos.data_ptr(), sin.data_ptr(), positions.data_ptr(),
+        slot_mapping.data_ptr(), T, Hq, Hk, D), "oa_rope_kv_parts")
+    q, k, v = qkv.split([Hq * D, Hk * D, Hk * D], dim=-1)
+    return q.view(T, Hq, D), k.view(T, Hk, D), v.view(T, Hk, D)
+
+
 def gateup_silu(x: torch.Tensor, gate_up_w: torch.Tensor, i_local: int) -> torch.Tensor:
     """silu(x @ gate^T) * (x @ up^T) with gate_up_w = [gate; up] rows.
 
@@ -1862,6 +1882,42 @@ def attention_decode_rope(
         k.stride(0), v.stride(0),
     )
     hip.check(rc, "oa_attention_decode_rope")
+    return out
+
+
+def decode_takes_parts(batch: int, Hq: int, Hk: int, D: int) -> bool:
+    """Whether attention_decode_parts takes the step: up to 64 (sequence, key head) pairs."""
+    return bool(_lib()[0].oa_attention_decode_takes_parts(batch, Hq, Hk, D))
+
+
+def attention_decode_parts(
+    parts: PlaneSum, Hq: int, Hk: int, D: int, k_cache: torch.Tensor, v_cache: torch.Tensor,
+    block_table: torch.Tensor, seq_lens: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+    slots: torch.Tensor, scale: float,
+    workspace: Optional[Tuple[torch.Tensor, ...]] = None, nsplit: Optional[int] = None,
+) -> torch.Tensor:
+    """attention_decode_rope of a q | k | v product that is not added up yet (linear_parts), where
+    decode_takes_parts says so."""
+    planes = parts.planes
+    n, B, width = planes.shape
+    block_size, G = k_cache.shape[1], Hq // Hk
+    assert width == (Hq + 2 * Hk) * D and planes.is_contiguous() and planes.dtype == torch.float32
+    assert k_cache.shape[2:] == v_cache.shape[2:] == (Hk, D) and cos.dtype == torch.float32
+    assert block_table.dtype == seq_lens.dtype == slots.dtype == torch.int32
+    if nsplit is None:
+        nsplit = decode_nsplit(B, Hk, int(block_table.shape[1] * block_size))
+    if workspace is None:
+        o_part = torch.empty(B * Hk * nsplit, G, D, dtype=torch.float32, device=planes.device)
+        ml_part = torch.empty(B * Hk * nsplit, G, 2, dtype=torch.float32, device=planes.device)
+    else:
+        o_part, ml_part = workspace[0], workspace[1]
+    lib, hip = _lib()
+    out = torch.empty(B, Hq, D, dtype=k_cache.dtype, device=planes.device)
+    hip.check(lib.oa_attention_decode_parts(
+        hip.current_stream_ptr(), planes.data_ptr(), n, k_cache.data_ptr(), v_cache.data_ptr(),
+        block_table.data_ptr(), seq_lens.data_ptr(), cos.data_ptr(), sin.data_ptr(), slots.data_ptr(),
+        o_part.data_ptr(), ml_part.data_ptr(), out.data_ptr(), B, Hq, Hk, D, block_table.shape[1],
+        block_size, nsplit, scale), "oa_attention_decode_parts")
     return out
 
 

@@ -231,7 +231,13 @@ __device__ __forceinline__ DecodeRuns decode_runs(const int* seq_lens, const int
 // [0, n-1), and the split that owns key n-1 rotates the new key, stores it and its
 // value in the cache and starts its softmax with them. kin/vin/cs/sn/slots/kcw/vcw
 // are only read when ROPE.
-template <int G, bool FUSED, bool ROPE, bool RUNS>
+//
+// PARTS (with ROPE, without runs): the projection is still its `splits` float32 planes [B, (Hq + 2 Hk) * 128],
+// `plane` elements apart. A block adds up the columns of its heads, rounds them as the product alone
+// would, and has them in LDS while its first keys and values are under way: what a launch for the sum took
+// goes but for a barrier. us, that launch, this one and the combine / here: 8 sequences of up to 1500
+// tokens, five planes 22.1 / 18.3 (traced one by one; a step of four layers 481.6 / 475.2).
+template <int G, bool FUSED, bool ROPE, bool RUNS, bool PARTS = false>
 __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kernel(
     const uint32_t* __restrict__ q, const uint32_t* __restrict__ kc,
     const uint32_t* __restrict__ vc, const int* __restrict__ block_table,
@@ -243,7 +249,9 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
     const float* __restrict__ cs, const float* __restrict__ sn,
     const int* __restrict__ slots, uint32_t* __restrict__ kcw,
-    uint32_t* __restrict__ vcw, int ks2, int vs2, int copies) {
+    uint32_t* __restrict__ vcw, int ks2, int vs2, int copies, const float* __restrict__ part_sums,
+    int splits, int64_t plane) {
+    static_assert(!PARTS || (ROPE && !RUNS && !FUSED), "parts of a projection: plain launches only");
     constexpr int GP = G > 4 ? 8 : 4;            // columns of one part of the queries
     constexpr int KL = GP / 4;                   // keys per lane and tile
     // the (row, key head) in work and its keys; RUNS: tiles of the row, the first of them that
@@ -368,7 +376,23 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
     // are rotated and split while the first keys, values and the new key are under way
     const int head = dl % GP, part = dl / GP;
     const bool have = head < G;
+    __shared__ __attribute__((aligned(16))) uint32_t lds_in[PARTS ? (G + 2) * DHEAD / 2 : 4];
+    constexpr int NIN = PARTS ? ((G + 2) * DHEAD / 4 + 255) / 256 : 1;    // four columns a thread and turn
+    constexpr int NP = PARTS ? 8 : 1;            // planes asked for at once
+    da_f4 in[NIN][NP];
+    const da_f4* ip[NIN];
+    if (PARTS) {
+#pragma unroll
+        for (int i = 0; i < NIN; ++i) {
+            const int c = min((int)(i * 256 + threadIdx.x) * 4, (G + 2) * DHEAD - 4), at = c / DHEAD;
+            const int col = (at < G ? h * G + at : Hk * G + (at - G) * Hk + h) * DHEAD + c % DHEAD;
+            ip[i] = reinterpret_cast<const da_f4*>(part_sums + (int64_t)b * (Hk * (G + 2) * DHEAD) + col);
+#pragma unroll
+            for (int k = 0; k < NP; ++k) in[i][k] = ip[i][min(k, splits - 1) * (plane / 4)];
+        }
+    }
     uint4 qw[4];
+    if (!PARTS)
 #pragma unroll
     for (int s = 0; s < 4; ++s)     // lane (column dl, channels s*32 + g16*8 .. + 7 of step s)
         qw[s] = *reinterpret_cast<const uint4*>(
@@ -394,9 +418,32 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
         page = page_of(1);
     };
     if (!RUNS || row == 0) load_first();
+    if (PARTS) {
+#pragma unroll
+        for (int i = 0; i < NIN; ++i) {
+            const int c = (i * 256 + threadIdx.x) * 4;
+            da_f4 sum = in[i][0];
+#pragma unroll
+            for (int k = 1; k < NP; ++k)
+                if (k < splits) sum += in[i][k];
+            for (int k = NP; k < splits; ++k) sum += ip[i][k * (plane / 4)];
+            if (c < (G + 2) * DHEAD)
+                *reinterpret_cast<uint2*>(&lds_in[c / 2]) =
+                    make_uint2(pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3]));
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            qw[s] = *reinterpret_cast<const uint4*>(&lds_in[((have ? head : 0) * DHEAD + s * 32 + g16 * 8) / 2]);
+    }
     const bool owner = ROPE && n - 1 >= kstart && n - 1 < kend && wid == 3;   // of the new key
     uint4 nk[4], nv;
-    if (owner) {
+    if (PARTS && owner) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            nk[s] = *reinterpret_cast<const uint4*>(&lds_in[(G * DHEAD + s * 32 + g16 * 8) / 2]);
+        nv = *reinterpret_cast<const uint4*>(&lds_in[((G + 1) * DHEAD + dl * 8) / 2]);
+    } else if (owner) {
 #pragma unroll
         for (int s = 0; s < 4; ++s)
             nk[s] = *reinterpret_cast<const uint4*>(
@@ -914,7 +961,7 @@ extern "C" int oa_attention_decode(void* stream, const void* q, const void* kc,
                        Hk, max_blocks, block_shift, nsplit, cb, runs, scale, qs2,              \
                        (const uint32_t*)nullptr, (const uint32_t*)nullptr,                     \
                        (const float*)nullptr, (const float*)nullptr, (const int*)nullptr,      \
-                       (uint32_t*)nullptr, (uint32_t*)nullptr, 0, 0, 0)
+                       (uint32_t*)nullptr, (uint32_t*)nullptr, 0, 0, 0, (const float*)nullptr, 0, 0)
 #define LAUNCH_G(GV)                                                                           \
     do {                                                                                       \
         if (fused) LAUNCH_FORM(GV, true, false);                                               \
@@ -972,7 +1019,7 @@ extern "C" int oa_attention_decode_rope(
                        Hk, max_blocks, block_shift, nsplit, cb, runs, scale, q_stride / 2,     \
                        (const uint32_t*)kin, (const uint32_t*)vin, (const float*)cos_t,        \
                        (const float*)sin_t, (const int*)slots, (uint32_t*)kc, (uint32_t*)vc,   \
-                       k_stride / 2, v_stride / 2, copies)
+                       k_stride / 2, v_stride / 2, copies, (const float*)nullptr, 0, 0)
 #define LAUNCH_GR(GV)                                                                          \
     do {                                                                                       \
         if (runs) LAUNCH_FORM(GV, true);                                                       \
@@ -992,5 +1039,45 @@ extern "C" int oa_attention_decode_rope(
     }
 #undef LAUNCH_GR
 #undef LAUNCH_FORM
+    return 0;
+}
+
+// Whether a launch of as many (sequence, key head) pairs takes the projection's planes: one without runs
+extern "C" int oa_attention_decode_takes_parts(int B, int Hq, int Hk, int D) {
+    const int G = Hk > 0 && Hq % Hk == 0 ? Hq / Hk : 0;
+    return D == DHEAD && (G == 1 || G == 2 || G == 4 || G == 8) && decode_run_count(B, Hk, 2) == 0;
+}
+
+// oa_attention_decode_rope of a projection that is still its planes part [splits, B, (Hq + 2 Hk) * D]
+extern "C" int oa_attention_decode_parts(
+    void* stream, const void* part, int splits, void* kc, void* vc, const void* block_table, const void* seq_lens,
+    const void* cos_t, const void* sin_t, const void* slots, void* o_part, void* ml_part, void* out, int B, int Hq,
+    int Hk, int D, int max_blocks, int block_size, int nsplit, float scale) {
+    if (B < 1 || splits < 1 || nsplit < 1 || !oa_attention_decode_takes_parts(B, Hq, Hk, D)) return -100;
+    if ((block_size & (block_size - 1)) != 0) return -101;
+    if ((uintptr_t)part % 16 != 0) return -103;
+    int block_shift = 0;
+    while ((1 << block_shift) < block_size) ++block_shift;
+#define LAUNCH_P(GV)                                                                                              \
+    do {                                                                                                          \
+        hipLaunchKernelGGL((decode_attn_kernel<GV, false, true, false, true>), dim3(B * Hk, nsplit), dim3(256), 0, \
+                           (hipStream_t)stream, (const uint32_t*)nullptr, (const uint32_t*)kc,                    \
+                           (const uint32_t*)vc, (const int*)block_table, (const int*)seq_lens, (float*)o_part,    \
+                           (float*)ml_part, (unsigned*)nullptr, (uint32_t*)out, B, Hk, max_blocks, block_shift,   \
+                           nsplit, decode_chunk_base(B * Hk), 0, scale, 0, (const uint32_t*)nullptr,              \
+                           (const uint32_t*)nullptr, (const float*)cos_t, (const float*)sin_t, (const int*)slots, \
+                           (uint32_t*)kc, (uint32_t*)vc, 0, 0, 0, (const float*)part, splits,                     \
+                           (int64_t)B * (Hq + 2 * Hk) * DHEAD);                                                   \
+        HIP_CHECK_LAUNCH();                                                                                       \
+        launch_combine<GV>((hipStream_t)stream, o_part, ml_part, seq_lens, out, B, Hk, nsplit, 0);                \
+        HIP_CHECK_LAUNCH();                                                                                       \
+    } while (0)
+    switch (Hq / Hk) {
+        case 1: LAUNCH_P(1); break;
+        case 2: LAUNCH_P(2); break;
+        case 4: LAUNCH_P(4); break;
+        default: LAUNCH_P(8); break;
+    }
+#undef LAUNCH_P
     return 0;
 }

@@ -53,6 +53,12 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_kv_write.restype = i
     lib.oa_rope_kv.argtypes = [p, p, p, p, p, p, p, p, p, p, i, i, i, i, i, i, i]
     lib.oa_rope_kv.restype = i
+    lib.oa_rope_kv_parts.argtypes = [p, p, i, p, p, p, p, p, p, p, i, i, i, i]
+    lib.oa_rope_kv_parts.restype = i
+    lib.oa_attention_decode_takes_parts.argtypes = [i, i, i, i]
+    lib.oa_attention_decode_takes_parts.restype = i
+    lib.oa_attention_decode_parts.argtypes = [p, p, i, p, p, p, p, p, p, p, p, p, p, i, i, i, i, i, i, i, f]
+    lib.oa_attention_decode_parts.restype = i
     lib.oa_gemv_gateup_act.argtypes = [p, p, p, p, i, i, i, i]
     lib.oa_gemv_gateup_act.restype = i
     lib.oa_gemv.argtypes = [p, p, p, p, i, i, i]
