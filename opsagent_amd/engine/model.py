@@ -287,7 +287,7 @@ class DecoderLayer(nn.Module):
             h = ops.rms_norm(x, self.input_norm_w, self.eps) if normed is None else normed
         else:
             # rows that the fp8 products would quantize next come quantized from the norm
-            low = (self.attn.fp8 and _sums_parts(self.attn) and residual.is_cuda
+            low = (_sums_parts(self.attn) and self.attn.fp8 and residual.is_cuda
                    and ops.fp8_rows_ok(*residual.shape))
             norm = ops.fused_add_rms_norm_fp8 if low else ops.fused_add_rms_norm
             h, residual = norm(x, residual, self.input_norm_w, self.eps)
@@ -297,7 +297,7 @@ class DecoderLayer(nn.Module):
             a = attn(h, cos, sin, k_cache, v_cache, fb, True)
         else:
             a = attn(h, cos, sin, k_cache, v_cache, fb)
-        low = (not self.is_moe_layer and mlp.fp8 and _sums_parts(mlp) and residual.is_cuda
+        low = (not self.is_moe_layer and _sums_parts(mlp) and mlp.fp8 and residual.is_cuda
                and ops.mlp_fp8_rows_ok(*residual.shape, mlp.i_local, mlp.gate_up_q))
         norm = ops.fused_add_rms_norm_fp8 if low else ops.fused_add_rms_norm
         h, residual = norm(a, residual, self.post_norm_w, self.eps)
