@@ -200,13 +200,13 @@ class RotaryWindowAttentionMixer(nn.Module):
     def forward(self, h, sb: mx.SeqBatch, kv, state) -> torch.Tensor:
         return ops.linear(self.context(h, sb, kv), self.o_w)
 
-    def context(self, h, sb: mx.SeqBatch, kv) -> torch.Tensor:
-        """What the output product reads."""
+    def context(self, h, sb: mx.SeqBatch, kv, merges: bool = False):
+        """What the output product reads (merges: see attn_rope_rows)."""
         k_cache, v_cache = kv
         proj = ops.linear(h, self.proj_w)                     # [T, q|k|v]
         return mx.attn_rope_rows(proj, self.q_norm_w, self.k_norm_w, self.inv_freq,
                                  self.H, self.G, self.D, self.Dv, self.eps, k_cache, v_cache, sb,
-                                 self.scale, window=self.window, sinks=self.sinks)
+                                 self.scale, window=self.window, sinks=self.sinks, merges=merges)
 
     def load(self, get, put, p: str) -> None:
         put(self.proj_w, [get(p + "q"), get(p + "k"), get(p + "v")])
@@ -1086,8 +1086,9 @@ class SandwichLayer(nn.Module):
         post, nxt = self.post1.params(), self.pre2.params() if self.mlp is not None else next_norm
         # one row: the add and the norm ride along with the sublayer's last product
         if x.shape[0] == 1 and _sums_parts(self.mixer):
-            h2 = mx.linear_dyt_norm(self.mixer.context(h, sb, kv), self.mixer.o_w, x, nxt,
-                                    self.dtype, post)
+            o_w = self.mixer.o_w
+            ctx = self.mixer.context(h, sb, kv, mx.merges_split_row(o_w, x, self.dtype))
+            h2 = mx.linear_dyt_norm(ctx, o_w, x, nxt, self.dtype, post)
         else:
             h2 = mx.dyt_norm(x, nxt, self.dtype, y=self.mixer(h, sb, kv, state), post=post)
         if self.mlp is None:

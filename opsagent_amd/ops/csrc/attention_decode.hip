@@ -19,6 +19,8 @@
 // equal runs, one a CU (DecodeRuns). Either way at most nsplit splits cover a sequence, a mark
 // stands behind its last one, and the combine reads those before it.
 
+#include <type_traits>
+
 #include "common.h"
 
 #define DHEAD 128
@@ -237,6 +239,13 @@ __device__ __forceinline__ DecodeRuns decode_runs(const int* seq_lens, const int
 // would, and has them in LDS while its first keys and values are under way: what a launch for the sum took
 // goes but for a barrier. us, that launch, this one and the combine / here: 8 sequences of up to 1500
 // tokens, five planes 22.1 / 18.3 (traced one by one; a step of four layers 481.6 / 475.2).
+struct Planes {
+    const float* sums;
+    int splits;
+    int64_t plane;
+};
+struct NoPlanes {};
+
 template <int G, bool FUSED, bool ROPE, bool RUNS, bool PARTS = false>
 __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kernel(
     const uint32_t* __restrict__ q, const uint32_t* __restrict__ kc,
@@ -249,8 +258,8 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
     const float* __restrict__ cs, const float* __restrict__ sn,
     const int* __restrict__ slots, uint32_t* __restrict__ kcw,
-    uint32_t* __restrict__ vcw, int ks2, int vs2, int copies, const float* __restrict__ part_sums,
-    int splits, int64_t plane) {
+    uint32_t* __restrict__ vcw, int ks2, int vs2, int copies,
+    std::conditional_t<PARTS, Planes, NoPlanes> planes) {
     static_assert(!PARTS || (ROPE && !RUNS && !FUSED), "parts of a projection: plain launches only");
     constexpr int GP = G > 4 ? 8 : 4;            // columns of one part of the queries
     constexpr int KL = GP / 4;                   // keys per lane and tile
@@ -381,14 +390,14 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
     constexpr int NP = PARTS ? 8 : 1;            // planes asked for at once
     da_f4 in[NIN][NP];
     const da_f4* ip[NIN];
-    if (PARTS) {
+    if constexpr (PARTS) {
 #pragma unroll
         for (int i = 0; i < NIN; ++i) {
             const int c = min((int)(i * 256 + threadIdx.x) * 4, (G + 2) * DHEAD - 4), at = c / DHEAD;
             const int col = (at < G ? h * G + at : Hk * G + (at - G) * Hk + h) * DHEAD + c % DHEAD;
-            ip[i] = reinterpret_cast<const da_f4*>(part_sums + (int64_t)b * (Hk * (G + 2) * DHEAD) + col);
+            ip[i] = reinterpret_cast<const da_f4*>(planes.sums + (int64_t)b * (Hk * (G + 2) * DHEAD) + col);
 #pragma unroll
-            for (int k = 0; k < NP; ++k) in[i][k] = ip[i][min(k, splits - 1) * (plane / 4)];
+            for (int k = 0; k < NP; ++k) in[i][k] = ip[i][min(k, planes.splits - 1) * (planes.plane / 4)];
         }
     }
     uint4 qw[4];
@@ -418,15 +427,15 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
         page = page_of(1);
     };
     if (!RUNS || row == 0) load_first();
-    if (PARTS) {
+    if constexpr (PARTS) {
 #pragma unroll
         for (int i = 0; i < NIN; ++i) {
             const int c = (i * 256 + threadIdx.x) * 4;
             da_f4 sum = in[i][0];
 #pragma unroll
             for (int k = 1; k < NP; ++k)
-                if (k < splits) sum += in[i][k];
-            for (int k = NP; k < splits; ++k) sum += ip[i][k * (plane / 4)];
+                if (k < planes.splits) sum += in[i][k];
+            for (int k = NP; k < planes.splits; ++k) sum += ip[i][k * (planes.plane / 4)];
             if (c < (G + 2) * DHEAD)
                 *reinterpret_cast<uint2*>(&lds_in[c / 2]) =
                     make_uint2(pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3]));
@@ -961,7 +970,7 @@ extern "C" int oa_attention_decode(void* stream, const void* q, const void* kc,
                        Hk, max_blocks, block_shift, nsplit, cb, runs, scale, qs2,              \
                        (const uint32_t*)nullptr, (const uint32_t*)nullptr,                     \
                        (const float*)nullptr, (const float*)nullptr, (const int*)nullptr,      \
-                       (uint32_t*)nullptr, (uint32_t*)nullptr, 0, 0, 0, (const float*)nullptr, 0, 0)
+                       (uint32_t*)nullptr, (uint32_t*)nullptr, 0, 0, 0, NoPlanes())
 #define LAUNCH_G(GV)                                                                           \
     do {                                                                                       \
         if (fused) LAUNCH_FORM(GV, true, false);                                               \
@@ -1019,7 +1028,7 @@ extern "C" int oa_attention_decode_rope(
                        Hk, max_blocks, block_shift, nsplit, cb, runs, scale, q_stride / 2,     \
                        (const uint32_t*)kin, (const uint32_t*)vin, (const float*)cos_t,        \
                        (const float*)sin_t, (const int*)slots, (uint32_t*)kc, (uint32_t*)vc,   \
-                       k_stride / 2, v_stride / 2, copies, (const float*)nullptr, 0, 0)
+                       k_stride / 2, v_stride / 2, copies, NoPlanes())
 #define LAUNCH_GR(GV)                                                                          \
     do {                                                                                       \
         if (runs) LAUNCH_FORM(GV, true);                                                       \
@@ -1066,8 +1075,8 @@ extern "C" int oa_attention_decode_parts(
                            (float*)ml_part, (unsigned*)nullptr, (uint32_t*)out, B, Hk, max_blocks, block_shift,   \
                            nsplit, decode_chunk_base(B * Hk), 0, scale, 0, (const uint32_t*)nullptr,              \
                            (const uint32_t*)nullptr, (const float*)cos_t, (const float*)sin_t, (const int*)slots, \
-                           (uint32_t*)kc, (uint32_t*)vc, 0, 0, 0, (const float*)part, splits,                     \
-                           (int64_t)B * (Hq + 2 * Hk) * DHEAD);                                                   \
+                           (uint32_t*)kc, (uint32_t*)vc, 0, 0, 0,                                                 \
+                           Planes{(const float*)part, splits, (int64_t)B * (Hq + 2 * Hk) * DHEAD});               \
         HIP_CHECK_LAUNCH();                                                                                       \
         launch_combine<GV>((hipStream_t)stream, o_part, ml_part, seq_lens, out, B, Hk, nsplit, 0);                \
         HIP_CHECK_LAUNCH();                                                                                       \

@@ -14,6 +14,8 @@
 // Requires K % 512 == 0 (64 lanes x 8 bf16); callers fall back to hipBLASLt
 // otherwise (and for M > 8, where the MFMA path wins).
 
+#include <type_traits>
+
 #include "mixer_util.h"
 
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
@@ -213,14 +215,27 @@ struct DytEpilogue {
     float* residual;
 };
 
-template <bool NORM, int EPI, int RT, int GR, int XV, int WV>
+// MERGE: the activations are an attention row of heads of D that is still its 2 to 6 key splits (sums o
+// [H, splits, D] and maximum and sum of weights ml [H, splits, 2], float32; attn_rows_kernel), which the image
+// merges as attn_combine_kernel would: that is a launch of 4.6 us before this one, and every block reads
+// all splits, 48 KB of 16 heads of 128, from the L2 while its weights are under way. us, the three launches
+// of attention and output product / these two, traced one by one, one row, window 512, 16 heads in 4, 2048 x
+// 2048: 16.4 / 13.5; a step of four layers 10 us less.
+struct MergeRow {
+    const float *o, *ml, *sinks;
+    int splits, D;
+};
+struct NoMerge {};
+
+template <bool NORM, int EPI, int RT, int GR, int XV, int WV, bool MERGE = false>
 __global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restrict__ x,
                                                     const uint32_t* __restrict__ w,
                                                     uint16_t* __restrict__ out,
                                                     const uint32_t* __restrict__ wn,
                                                     const uint16_t* __restrict__ res, int N, int K,
                                                     int waves, int full, int extra, float eps,
-                                                    int act, DytEpilogue dy) {
+                                                    int act, DytEpilogue dy,
+                                                    std::conditional_t<MERGE, MergeRow, NoMerge> mr) {
     extern __shared__ __attribute__((aligned(16))) float xl[];   // [2][K / 2]
     __shared__ float part[8];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -249,9 +264,26 @@ __global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restri
     // i's residual of the wave's row i (at most 64) are asked for before the weights, so
     // that the image below waits for them alone.
     uint4 xv[XV], nv[XV];
+    constexpr int MS = 6, MX = MERGE ? XV : 1;
+    float4 mo[MX][MS][2];
+    float2 ms[MX][MS];
+    float sink[MX];
 #pragma unroll
     for (int j = 0; j < XV; ++j) {
         const int i = min(j * WV * 64 + tid, K / 8 - 1);
+        if constexpr (MERGE) {
+            const int h = i * 8 / mr.D, c = i * 8 - h * mr.D;
+#pragma unroll
+            for (int s = 0; s < MS; ++s) {
+                const int at = h * mr.splits + min(s, mr.splits - 1);
+                ms[j][s] = reinterpret_cast<const float2*>(mr.ml)[at];
+                const float4* o = reinterpret_cast<const float4*>(mr.o + (size_t)at * mr.D + c);
+                mo[j][s][0] = o[0];
+                mo[j][s][1] = o[1];
+            }
+            sink[j] = mr.sinks ? mr.sinks[h] : 0.0f;
+            continue;
+        }
         xv[j] = reinterpret_cast<const uint4*>(x)[i];
         if (NORM) nv[j] = reinterpret_cast<const uint4*>(wn)[i];
     }
@@ -296,6 +328,26 @@ __global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restri
         const int i = j * WV * 64 + tid;
         if (i >= K / 8) continue;
         float f[8];
+        if constexpr (MERGE) {
+            float mx = -INFINITY, l = 0.0f;
+#pragma unroll
+            for (int s = 0; s < MS; ++s)
+                if (s < mr.splits) mx = fmaxf(mx, ms[j][s].x);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] = 0.0f;
+#pragma unroll
+            for (int s = 0; s < MS; ++s) {
+                // (a split without a key has no maximum)
+                const float wt = s < mr.splits && ms[j][s].x != -INFINITY ? expf(ms[j][s].x - mx) : 0.0f;
+                l += ms[j][s].y * wt;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) f[e] += (&mo[j][s][e / 4].x)[e % 4] * wt;
+            }
+            if (mr.sinks) l += expf(sink[j] - mx);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] = bf16_to_f32(f32_to_bf16(f[e] / l));
+        }
+        if constexpr (!MERGE)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             f[2 * e] = bf16_lo((&xv[j].x)[e]);
@@ -374,7 +426,7 @@ __global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restri
 // mode as in oa_gemv_ex, 4: dy; gateup > 0: N gate and N up rows, activation gateup - 1
 static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const void* wn,
                  const void* res, int N, int K, float eps, int mode, int gateup,
-                 const DytEpilogue& dy = {}) {
+                 const DytEpilogue& dy = {}, const MergeRow& mr = {}) {
     // Rows of 4096, and many of 2048: blocks of four waves, of two rows a wave (gate-up one
     // pair), so that CUs even out; the image of a block is quickly made. No more than 32
     // blocks per CU. Us, blocks of eight waves and up to 64 rows a wave / this: 6144 x 4096
@@ -407,17 +459,23 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
     const int blocks = CEIL_DIV(CEIL_DIV(N, per), wv);
     const int waves = blocks * wv;
     const size_t lds = (size_t)K * 4;
-#define G1X(NV, RV, RT, GR, XV, WV)                                                                   \
-    hipLaunchKernelGGL((gemv1_kernel<NV, RV, RT, GR, XV, WV>), dim3(blocks), dim3(WV * 64), lds, st,  \
-                       (const uint32_t*)x, (const uint32_t*)w, (uint16_t*)out, (const uint32_t*)wn,   \
-                       (const uint16_t*)res, N, K, waves, N / waves, N % waves, eps, gateup - 1, dy)
+#define G1X(NV, RV, RT, GR, XV, WV, ...) G1Y(NV, RV, RT, GR, XV, WV, NoMerge(), ##__VA_ARGS__)
+#define G1Y(NV, RV, RT, GR, XV, WV, MR, ...)                                                              \
+    hipLaunchKernelGGL((gemv1_kernel<NV, RV, RT, GR, XV, WV, ##__VA_ARGS__>), dim3(blocks), dim3(WV * 64), \
+                       lds, st, (const uint32_t*)x, (const uint32_t*)w, (uint16_t*)out,               \
+                       (const uint32_t*)wn, (const uint16_t*)res, N, K, waves, N / waves, N % waves,  \
+                       eps, gateup - 1, dy, MR)
 #define G1(NV, RV, RT, GR)                   \
     do {                                     \
         if (wv == 4) G1X(NV, RV, RT, GR, 2, 4);         \
         else if (K <= 4096) G1X(NV, RV, RT, GR, 1, 8);  \
         else G1X(NV, RV, RT, GR, 4, 8);                 \
     } while (0)
-    if (gateup) {
+    if (mr.o) {                          // K = 2048 or 4096
+        if (K == 4096) G1Y(false, 2, 1, 8, 2, 4, mr, true);
+        else if (wv == 4) G1Y(false, 2, 1, 4, 2, 4, mr, true);
+        else G1Y(false, 2, 1, 4, 1, 8, mr, true);
+    } else if (gateup) {
         if (mode & 1) G1(true, 0, 2, 4);
         else G1(false, 0, 2, 4);
     } else if (K % 4096 == 0) {
@@ -439,6 +497,7 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
     }
 #undef G1
 #undef G1X
+#undef G1Y
     HIP_CHECK_LAUNCH();
     return 0;
 }
@@ -520,6 +579,20 @@ extern "C" int oa_gemv_gateup_act(void* stream, const void* x, const void* w,
 }
 
 // mode: 0 plain, 1 norm-prologue, 2 residual-add epilogue, 3 both
+// The same of a row that is still its key splits (MergeRow): K = 2048 or 4096, heads of 64 or 128
+extern "C" int oa_gemv_dyt_merge(void* stream, const void* o, const void* ml, const void* sinks, int splits, int D,
+                                 const void* w, void* residual, const void* pw, const void* pb, const void* pa,
+                                 const void* nw, const void* nb, const void* na, void* out, int N, int K) {
+    if (N < 1 || (K != 2048 && K != 4096) || N > 256 * 64 * 8) return -100;
+    if (splits < 2 || splits > 6 || (D != 64 && D != 128)) return -103;
+    if (!o || !ml || !w || !residual || !pw || !pb || !pa || (out && (!nw || !nb || !na))) return -101;
+    if (((uintptr_t)o | (uintptr_t)w) % 16 != 0 || (uintptr_t)ml % 8 != 0) return -102;
+    const DytEpilogue dy = {(const float*)pw, (const float*)pb, (const float*)pa, (const float*)nw,
+                            (const float*)nb, (const float*)na, (float*)residual};
+    const MergeRow mr = {(const float*)o, (const float*)ml, (const float*)sinks, splits, D};
+    return gemv1((hipStream_t)stream, nullptr, w, out, nullptr, nullptr, N, K, 0.0f, 4, 0, dy, mr);
+}
+
 extern "C" int oa_gemv_ex(void* stream, const void* x, const void* w, void* out,
                           const void* wn, const void* res, int M, int N, int K,
                           float eps, int mode) {

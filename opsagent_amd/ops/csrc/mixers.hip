@@ -2520,7 +2520,7 @@ extern "C" int oa_attn_rows_rope(void* stream, const void* qkv, int64_t qs, cons
     if (qs % 8 != 0 || qs < (int64_t)(H + G + Gv) * D || window < 0 || os < (int64_t)H * D) return -105;
     if (((uintptr_t)qkv | (uintptr_t)qw | (uintptr_t)kw | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 != 0)
         return -102;
-    if (nsplit < 1 || (nsplit > 1 && (!part_o || !part_ml))) return -104;
+    if (nsplit < 1 || (nsplit > 1 ? !part_o || !part_ml : !out)) return -104;
     hipStream_t s = (hipStream_t)stream;
     const int R = H / G, hb = rows_hb(R, ntiles * G, nsplit);
     const dim3 grid(ntiles, G * (R / hb), nsplit);
@@ -2536,7 +2536,7 @@ extern "C" int oa_attn_rows_rope(void* stream, const void* qkv, int64_t qs, cons
     else launch_attn_rows<1, true>(ROPE_ARGS);
 #undef ROPE_ARGS
     HIP_CHECK_LAUNCH();
-    if (nsplit > 1) {
+    if (nsplit > 1 && out) {
         hipLaunchKernelGGL((attn_combine_kernel<bf16s>), dim3((unsigned)((int64_t)T * H)), dim3(256), 0, s,
                            (const float*)part_o, (const float*)part_ml, (const bf16s*)nullptr, (int64_t)0,
                            (const float*)sinks, (bf16s*)out, H, D, nsplit, os, 1.0f, 0);

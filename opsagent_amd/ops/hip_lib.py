@@ -65,6 +65,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_gemv.restype = i
     lib.oa_gemv_ex.argtypes = [p, p, p, p, p, p, i, i, i, f, i]
     lib.oa_gemv_ex.restype = i
+    lib.oa_gemv_dyt_merge.argtypes = [p, p, p, p, i, i, p, p, p, p, p, p, p, p, p, i, i]
+    lib.oa_gemv_dyt_merge.restype = i
     lib.oa_gemv_dyt.argtypes = [p, p, p, p, p, p, p, p, p, p, p, i, i]
     lib.oa_gemv_dyt.restype = i
     lib.oa_gemv_grouped.argtypes = [p, p, p, i, i, i, i, p, p, p, p, p, i]

@@ -14,7 +14,7 @@ from __future__ import annotations
 import ctypes
 import dataclasses
 import os
-from typing import List, Optional, Tuple, Union
+from typing import List, NamedTuple, Optional, Tuple, Union
 
 import numpy as np
 import torch
@@ -499,15 +499,41 @@ def dyt_norm(residual: torch.Tensor, nxt: Optional[Tuple[torch.Tensor, ...]], ou
     return out
 
 
-def linear_dyt_norm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
+class SplitRow(NamedTuple):
+    """An attention row of heads of D that is still its key splits: sums [H * splits, D], maximum and
+    sum of weights [H * splits, 2], float32, and the heads' sinks."""
+
+    o: torch.Tensor
+    ml: torch.Tensor
+    sinks: Optional[torch.Tensor]
+    splits: int
+    D: int
+
+
+def merges_split_row(w: torch.Tensor, residual: torch.Tensor, out_dtype) -> bool:
+    """Whether linear_dyt_norm takes a SplitRow against w."""
+    from opsagent_amd import ops
+
+    return (w.is_cuda and w.dim() == 2 and w.shape[1] in (2048, 4096) and w.shape[0] <= 131072
+            and w.dtype == out_dtype == torch.bfloat16 and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and residual.shape == (1, w.shape[0]) and residual.dtype == torch.float32
+            and residual.is_contiguous() and residual.device == w.device
+            and ops._gemv_m_ok(1) and ops._plain_call(residual, w))
+
+
+def linear_dyt_norm(x: Union[torch.Tensor, SplitRow], w: torch.Tensor, residual: torch.Tensor,
                     nxt: Optional[Tuple[torch.Tensor, ...]], out_dtype,
                     post: Tuple[torch.Tensor, ...]) -> Optional[torch.Tensor]:
     """dyt_norm with y = x @ w^T: for one row of bf16 in one launch, the epilogue of the one-row
     product (gemv.hip), where that takes the row."""
     from opsagent_amd import ops
 
-    K = x.shape[-1]
-    if not (x.is_cuda and x.shape[0] == 1 and x.dtype == w.dtype == out_dtype == torch.bfloat16
+    split = isinstance(x, SplitRow)
+    if split:
+        assert merges_split_row(w, residual, out_dtype) and x.o.numel() == w.shape[1] * x.splits
+        assert x.o.device == w.device and x.o.is_contiguous() and x.ml.is_contiguous()
+    K = w.shape[1] if split else x.shape[-1]
+    if not split and not (x.is_cuda and x.shape[0] == 1 and x.dtype == w.dtype == out_dtype == torch.bfloat16
             and x.dim() == w.dim() == 2 and w.shape[1] == K and residual.shape == (1, w.shape[0])
             and K % 2048 == 0 and K <= 16384 and w.shape[0] <= 131072 and ops._gemv_m_ok(1)
             and x.is_contiguous() and w.is_contiguous() and ops._plain_call(x, w)
@@ -520,10 +546,15 @@ def linear_dyt_norm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
         for t, n in zip(norm, (N, N, 1)):
             assert t.dtype == torch.float32 and t.is_contiguous() and t.numel() == n
     lib, hip = _lib()
-    out = torch.empty(1, N, dtype=out_dtype, device=x.device) if nxt is not None else None
+    out = torch.empty(1, N, dtype=out_dtype, device=w.device) if nxt is not None else None
     kernels = hip.get_lib()
-    hip.check(kernels.oa_gemv_dyt(
-        hip.current_stream_ptr(), x.data_ptr(), w.data_ptr(), residual.data_ptr(),
+    entry, row = kernels.oa_gemv_dyt, (() if split else (x.data_ptr(),))
+    if split:
+        entry = kernels.oa_gemv_dyt_merge
+        row = (x.o.data_ptr(), x.ml.data_ptr(), x.sinks.data_ptr() if x.sinks is not None else None,
+               x.splits, x.D)
+    hip.check(entry(
+        hip.current_stream_ptr(), *row, w.data_ptr(), residual.data_ptr(),
         *(t.data_ptr() for t in post),
         *((t.data_ptr() for t in nxt) if nxt is not None else (None, None, None)),
         out.data_ptr() if out is not None else None, N, K), "oa_gemv_dyt")
@@ -644,9 +675,11 @@ def attn_rope_rows(qkv: torch.Tensor, q_norm_w: torch.Tensor, k_norm_w: torch.Te
                    inv_freq: torch.Tensor, H: int, G: int, D: int, Dv: int, eps: float,
                    k_cache: torch.Tensor, v_cache: torch.Tensor, sb: SeqBatch, scale: float,
                    window: Optional[int] = None,
-                   sinks: Optional[torch.Tensor] = None) -> torch.Tensor:
+                   sinks: Optional[torch.Tensor] = None,
+                   merges: bool = False) -> Union[torch.Tensor, "SplitRow"]:
     """attn_rope_prepare and attention_paged of its queries, [T, H*Dv]; decode steps in one launch
-    (two with key splits) where the kernel for them takes the heads (mixers.hip). There a row's new
+    (two with key splits, whose merge is left to the product behind it where that `merges` and no wave
+    of six splits has more than one piece of keys) where the kernel for them takes the heads (mixers.hip). There a row's new
     key is its own alone: no sequence of a step reads a slot that another one writes in it (pages are
     shared when they are full)."""
     splits = 0
@@ -665,6 +698,11 @@ def attn_rope_rows(qkv: torch.Tensor, q_norm_w: torch.Tensor, k_norm_w: torch.Te
         KT = attn_geometry(H, G, D, Dv, 0, 1)[1]
         reach = min(sb.max_total, window + 1 + KT) if window else sb.max_total
         splits = lib.oa_attn_rows_splits(H, G, D, Dv, 0, 1, tokens, reach) if tokens > 0 else 0
+        # six splits of eight waves with a piece of 32 keys each (us, one prompt of 2000 and eight steps of
+        # four layers, 16 heads, window 512, 3 / 4 / 5 / 6 splits 2943 / 2931 / 2903 / 2895; nine and the
+        # launch that merges them 3003)
+        merges = merges and qkv.shape[0] == tokens == 1 and splits > 1 and reach <= 6 * 8 * 32
+        splits = 6 if merges else splits
     if not splits:
         q = attn_rope_prepare(qkv, q_norm_w, k_norm_w, inv_freq, H, G, D, Dv, eps, k_cache,
                               v_cache, sb)
@@ -672,7 +710,8 @@ def attn_rope_rows(qkv: torch.Tensor, q_norm_w: torch.Tensor, k_norm_w: torch.Te
     assert sinks is None or (sinks.dtype == torch.float32 and sinks.numel() == H
                              and sinks.is_contiguous())
     T = qkv.shape[0]
-    out = torch.empty(T, H * D, dtype=qkv.dtype, device=qkv.device)
+    merges = merges and splits > 1
+    out = None if merges else torch.empty(T, H * D, dtype=qkv.dtype, device=qkv.device)
     part_o = part_ml = None
     if splits > 1:
         part_o = torch.empty(T * H * splits, D, dtype=torch.float32, device=qkv.device)
@@ -680,14 +719,15 @@ def attn_rope_rows(qkv: torch.Tensor, q_norm_w: torch.Tensor, k_norm_w: torch.Te
     hip.check(lib.oa_attn_rows_rope(
         hip.current_stream_ptr(), qkv.data_ptr(), qkv.stride(0), q_norm_w.data_ptr(),
         k_norm_w.data_ptr(), inv_freq.data_ptr(), inv_freq.numel(), eps,
-        sb.slot_mapping.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
+        sb.slot_mapping.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+        None if merges else out.data_ptr(),
         part_o.data_ptr() if part_o is not None else None,
         part_ml.data_ptr() if part_ml is not None else None,
         sb.cu_t.data_ptr(), sb.past_t.data_ptr(), sb.block_table.data_ptr(),
         sb.block_table.shape[1], k_cache.shape[1],
         sinks.data_ptr() if sinks is not None else None, T, sb.num_seqs, tokens, H, G, G, D,
         float(scale), splits, int(window) if window else 0, H * D), "oa_attn_rows_rope")
-    return out
+    return SplitRow(part_o, part_ml, sinks, splits, D) if merges else out
 
 
 ACTS = {"silu": 0, "gelu_tanh": 1, "clamp_swish": 2, "relu2": 3}
