@@ -1090,14 +1090,25 @@ class SandwichLayer(nn.Module):
             ctx = self.mixer.context(h, sb, kv, mx.merges_split_row(o_w, x, self.dtype))
             h2 = mx.linear_dyt_norm(ctx, o_w, x, nxt, self.dtype, post)
         else:
-            h2 = mx.dyt_norm(x, nxt, self.dtype, y=self.mixer(h, sb, kv, state), post=post)
+            h2 = mx.dyt_norm(x, nxt, self.dtype, y=self._product(self.mixer, h, sb, kv, state), post=post)
         if self.mlp is None:
             return x, h2
         if x.shape[0] == 1 and _sums_parts(self.mlp):
             return x, mx.linear_dyt_norm(self.mlp.inner(h2), self.mlp.down_w, x, next_norm,
                                          self.dtype, self.post2.params())
-        m = self.mlp(h2, decode=sb.max_chunk == 1) if self.routed else self.mlp(h2)
+        m = self.mlp(h2, decode=sb.max_chunk == 1) if self.routed else self._product(self.mlp, h2)
         return x, mx.dyt_norm(x, next_norm, self.dtype, y=m, post=self.post2.params())
+
+    @staticmethod
+    def _product(sublayer, h, *more) -> torch.Tensor:
+        """What a sublayer gives, or the float32 planes of its last product, which the norm adds up."""
+        if not _sums_parts(sublayer):
+            return sublayer(h, *more)
+        mixes = isinstance(sublayer, RotaryWindowAttentionMixer)
+        row, w = ((sublayer.context(h, *more[:2]), sublayer.o_w) if mixes
+                  else (sublayer.inner(h), sublayer.down_w))
+        y = ops.linear_parts(row, w)
+        return y.planes if isinstance(y, ops.PlaneSum) else y
 
     def load(self, get, put, p: str) -> None:
         self.pre1.load(get, put, p + "norm1")
@@ -1454,6 +1465,9 @@ class HybridForCausalLM(nn.Module):
         if self.embed_norm_w is not None:
             x = mx.embed_norm_rows(self.embed, fb.input_ids, self.embed_norm_w,
                                    self.spec.norm_eps, offset=1.0)
+        elif self.sandwich and self.pos_freq is None:
+            x, h = mx.embed_dyt_norm(self.embed, fb.input_ids, self.spec.embed_scale,
+                                     self.layers[0].first_norm(), self.dtype)
         else:
             x = mx.embed_rows(self.embed, fb.input_ids, self.spec.embed_scale, self.pos_freq, sb)
         if self.parallel:
@@ -1487,9 +1501,9 @@ class HybridForCausalLM(nn.Module):
             return xs.sum(1) if S > 1 else xs.squeeze(1)
         if self.sandwich or self.pre_norm:
             n = len(self.layers)
-            if self.sandwich:
+            if self.sandwich and self.pos_freq is not None:
                 h = mx.dyt_norm(x, self.layers[0].first_norm(), self.dtype)
-            else:
+            elif not self.sandwich:
                 h = mx.add_layer_norm(x, self.layers[0].first_norm(), self.spec.norm_eps,
                                       self.dtype)
             for i, layer in enumerate(self.layers):
@@ -1537,12 +1551,11 @@ class HybridForCausalLM(nn.Module):
         else:
             _, normed = mx.group_rms_norm(hidden, self.final_norm_w, self.spec.norm_groups,
                                           self.spec.norm_eps, residual=None)
-        logits = ops.linear(normed, self.lm_head)
         if self.spec.logit_scale != 1.0:
-            return logits.float() * self.spec.logit_scale
+            return ops.linear_float(normed, self.lm_head) * self.spec.logit_scale
         if self.spec.logit_softcap is None:
-            return logits.float()
-        return mx.softcap(logits, self.spec.logit_softcap)
+            return ops.linear_float(normed, self.lm_head)
+        return mx.softcap(ops.linear(normed, self.lm_head), self.spec.logit_softcap)
 
     # -- checkpoint names ----------------------------------------------------
     @torch.no_grad()

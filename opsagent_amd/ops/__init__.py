@@ -601,6 +601,21 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x, w)
 
 
+def linear_float(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """linear(x, w).float(), of one bf16 row in the product's own launch where gemv.hip takes it."""
+    N, K = w.shape
+    if not (x.is_cuda and x.dim() == 2 and x.shape == (1, K) and K % 2048 == 0 and K <= 16384
+            and x.dtype == w.dtype == torch.bfloat16 and x.device == w.device
+            and _gemv_m_ok(1) and _plain_call(x, w) and x.is_contiguous() and w.is_contiguous()
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0):
+        return linear(x, w).float()
+    lib, hip = _lib()
+    out = torch.empty(1, N, dtype=torch.float32, device=x.device)
+    hip.check(lib.oa_gemv_float(hip.current_stream_ptr(), x.data_ptr(), w.data_ptr(), out.data_ptr(),
+                                N, K), "oa_gemv_float")
+    return out
+
+
 def _is_gpu(t: torch.Tensor) -> bool:
     return t.is_cuda
 

@@ -215,6 +215,9 @@ struct DytEpilogue {
     float* residual;
 };
 
+// EPI 3 writes the bf16 result as float32 (the logits of a step, us for 32000 x 2048 with the launch that
+// would convert them 25.5 / 21.8).
+//
 // MERGE: the activations are an attention row of heads of D that is still its 2 to 6 key splits (sums o
 // [H, splits, D] and maximum and sum of weights ml [H, splits, 2], float32; attn_rows_kernel), which the image
 // merges as attn_combine_kernel would: that is a launch of 4.6 us before this one, and every block reads
@@ -391,6 +394,7 @@ __global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restri
             if (EPI == 1)
                 v0 += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rs), un));
             if (EPI == 2) mine = lane == un ? v0 : mine;
+            else if (EPI == 3 && lane == 0) reinterpret_cast<float*>(out)[ur] = bf16_to_f32(f32_to_bf16(v0));
             else if (lane == 0) out[ur] = f32_to_bf16(v0);
 #pragma unroll
             for (int t = 0; t < RT; ++t) acc[t] = 0.0f;
@@ -423,7 +427,7 @@ __global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restri
     }
 }
 
-// mode as in oa_gemv_ex, 4: dy; gateup > 0: N gate and N up rows, activation gateup - 1
+// mode as in oa_gemv_ex, 4: dy; 5: out float32; gateup > 0: N gate and N up rows, activation gateup - 1
 static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const void* wn,
                  const void* res, int N, int K, float eps, int mode, int gateup,
                  const DytEpilogue& dy = {}, const MergeRow& mr = {}) {
@@ -484,6 +488,7 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
             case 1: G1(true, 0, 1, 8); break;
             case 2: G1(false, 1, 1, 8); break;
             case 3: G1(true, 1, 1, 8); break;
+            case 5: G1(false, 3, 1, 8); break;
             default: G1(false, 2, 1, 8); break;
         }
     } else {
@@ -492,6 +497,7 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
             case 1: G1(true, 0, 1, 4); break;
             case 2: G1(false, 1, 1, 4); break;
             case 3: G1(true, 1, 1, 4); break;
+            case 5: G1(false, 3, 1, 4); break;
             default: G1(false, 2, 1, 4); break;
         }
     }
@@ -579,7 +585,15 @@ extern "C" int oa_gemv_gateup_act(void* stream, const void* x, const void* w,
 }
 
 // mode: 0 plain, 1 norm-prologue, 2 residual-add epilogue, 3 both
-// The same of a row that is still its key splits (MergeRow): K = 2048 or 4096, heads of 64 or 128
+// out [N] float32 = bf16(x W^T), one row
+extern "C" int oa_gemv_float(void* stream, const void* x, const void* w, void* out, int N, int K) {
+    if (N < 1 || !gemv1_ok(1, K)) return -100;
+    if (!x || !w || !out) return -101;
+    if (((uintptr_t)x | (uintptr_t)w) % 16 != 0) return -102;
+    return gemv1((hipStream_t)stream, x, w, out, nullptr, nullptr, N, K, 0.0f, 5, 0);
+}
+
+// oa_gemv_dyt of a row that is still its key splits (MergeRow): K = 2048 or 4096, heads of 64 or 128
 extern "C" int oa_gemv_dyt_merge(void* stream, const void* o, const void* ml, const void* sinks, int splits, int D,
                                  const void* w, void* residual, const void* pw, const void* pb, const void* pa,
                                  const void* nw, const void* nb, const void* na, void* out, int N, int K) {

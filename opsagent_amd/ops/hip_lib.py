@@ -67,6 +67,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_gemv_ex.restype = i
     lib.oa_gemv_dyt_merge.argtypes = [p, p, p, p, i, i, p, p, p, p, p, p, p, p, p, i, i]
     lib.oa_gemv_dyt_merge.restype = i
+    lib.oa_gemv_float.argtypes = [p, p, p, p, i, i]
+    lib.oa_gemv_float.restype = i
     lib.oa_gemv_dyt.argtypes = [p, p, p, p, p, p, p, p, p, p, p, i, i]
     lib.oa_gemv_dyt.restype = i
     lib.oa_gemv_grouped.argtypes = [p, p, p, i, i, i, i, p, p, p, p, p, i]
@@ -180,6 +182,7 @@ def _declare_mixers(lib: ctypes.CDLL) -> None:
     f = ctypes.c_float
     ip = ctypes.POINTER(ctypes.c_int)
     sigs = {
+        "oa_embed_dyt": [p, p, p, f, p, p, p, p, p, i, i, i],
         "oa_group_norm_step": [p, p, i64, i, i64, p, p, p, i, i, i, f, p, p, p, p, p, p, p, i, i],
         "oa_attn_prepare_parts": [p, p, i, p, p, p, p, p, p, p, p, p, i, i, i, i, i, i, i, f],
         "oa_causal_conv_seq": [p, p, i64, i, p, p, p, i64, p, p, p, p, i, i, i, i, i, i, i, i],

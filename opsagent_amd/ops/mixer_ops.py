@@ -143,6 +143,24 @@ def embed_rows(table: torch.Tensor, ids: torch.Tensor, scale: float = 1.0,
     return out
 
 
+def embed_dyt_norm(table: torch.Tensor, ids: torch.Tensor, scale: float,
+                   nxt: Tuple[torch.Tensor, ...], out_dtype) -> Tuple[torch.Tensor, torch.Tensor]:
+    """embed_rows and the first norm, (x, dyt_norm(x, nxt, out_dtype)), in one launch on the GPU."""
+    if not (table.is_cuda and table.dtype == out_dtype and out_dtype in (torch.bfloat16, torch.float32)
+            and table.is_contiguous() and ids.dtype == torch.int64 and ids.is_contiguous()
+            and all(t.dtype == torch.float32 and t.is_contiguous() for t in nxt)):
+        x = embed_rows(table, ids, scale)
+        return x, dyt_norm(x, nxt, out_dtype)
+    lib, hip = _lib()
+    T, C = ids.shape[0], table.shape[1]
+    x = torch.empty(T, C, dtype=torch.float32, device=table.device)
+    h = torch.empty(T, C, dtype=out_dtype, device=table.device)
+    hip.check(lib.oa_embed_dyt(hip.current_stream_ptr(), table.data_ptr(), ids.data_ptr(), float(scale),
+                               x.data_ptr(), *(t.data_ptr() for t in nxt), h.data_ptr(), T, C,
+                               _dt(table)), "oa_embed_dyt")
+    return x, h
+
+
 def causal_conv_seq(x: torch.Tensor, w: torch.Tensor, state: torch.Tensor, sb: SeqBatch,
                     add_input: bool, act_silu: bool) -> torch.Tensor:
     """(x +) causal per-channel convolution over time (-> silu), continued
