@@ -854,7 +854,7 @@ extern "C" int oa_gemv_gateup_fp8(void* stream, const void* x, const void* w8,
 // ---- fp8 MFMA tile GEMM (prefill path) -------------------------------------
 // C[M, N] = (A8[M, K] @ B8[N, K]^T) * a_scale[m] * b_scale[n], bf16 out.
 //
-// A tile of BM x BN, sixteen waves (4 x 4), K-steps of 128 fp8 bytes, A and B staged by
+// A tile of BM x BN, sixteen waves (4 x 4; 96 rows: fourteen, 3 x 4 and two), K-steps of 128 fp8 bytes, A and B staged by
 // 16-byte global_load_lds. 16-byte chunk c of row r lies at c ^ (r >> 1 & 7): LDS has 64
 // banks, and 16 rows of 128 bytes at one chunk touch each of them once (c ^ (r & 7) touches
 // half of them twice: 11 M conflict cycles of 22 M on 28672 x 4096, M = 700, none here). The
@@ -895,13 +895,16 @@ __device__ __forceinline__ void g8_wait() {
 // 331 / 290 / 271 / 251; 4096 x 14336, 700 76 / 61 / 101 / 94 / 162, 2048 132 / 146 / 139 / 112 /
 // 173; 6144 x 4096, 700 34.5 / 40.5 / 30.1 / 31.8 / 49; 2048 x 8192, 700 45.9 / 33.7 / 43 / 49 /
 // 81; 16384 x 2048, 700 52.9 / 43.5 / 42.9 / 44.2 / 37.9.
+#define G8_WAVES(BM) ((BM) == 96 ? 14 : 16)
 template <int BM, int BN, int ST, int BLOCKS>
-__global__ __launch_bounds__(1024, 4 * BLOCKS) void gemm_fp8_tile_kernel(
+__global__ __launch_bounds__(64 * G8_WAVES(BM), 4 * BLOCKS) void gemm_fp8_tile_kernel(
     const char* __restrict__ a8, const char* __restrict__ b8,
     const float* __restrict__ ascale, const float* __restrict__ bscale,
     uint16_t* __restrict__ c, int M, int N, int K, int mtiles, int items) {
-    constexpr int FI = BM / 128, FJ = BN / 128;                        // fragments of a wave
-    constexpr int STEP = (BM + BN) * GK2, LPW = (BM + BN) / 128;       // transfers of a wave
+    constexpr int FI = BM == 96 ? 1 : BM / 128, FJ = BN / 128;         // fragments of a wave
+    constexpr int WAVES = G8_WAVES(BM);
+    constexpr int STEP = (BM + BN) * GK2, LPW = (BM + BN) / (8 * WAVES);     // transfers of a wave
+    static_assert(LPW * WAVES * 8 == BM + BN, "every wave transfers as much");
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int per = gridDim.x >> 3;
     const int item = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
@@ -915,7 +918,7 @@ __global__ __launch_bounds__(1024, 4 * BLOCKS) void gemm_fp8_tile_kernel(
     const char* src[LPW];
 #pragma unroll
     for (int p = 0; p < LPW; ++p) {
-        const int r = (p * 16 + wid) * 8 + (lane >> 3);      // row of A, then of B
+        const int r = (p * WAVES + wid) * 8 + (lane >> 3);   // row of A, then of B
         const int64_t at = r < BM ? (int64_t)min(tm + r, M - 1) * K : (int64_t)min(tn + r - BM, N - 1) * K;
         src[p] = (r < BM ? a8 : b8) + at + ((lane & 7) ^ (r >> 1 & 7)) * 16;
     }
@@ -923,7 +926,7 @@ __global__ __launch_bounds__(1024, 4 * BLOCKS) void gemm_fp8_tile_kernel(
     auto stage = [&](int buf) {
 #pragma unroll
         for (int p = 0; p < LPW; ++p) {
-            lds_transfer16(lds0 + buf * STEP + p * 16 * 1024, src[p]);
+            lds_transfer16(lds0 + buf * STEP + p * WAVES * 1024, src[p]);
             src[p] += GK2;
         }
     };
@@ -951,6 +954,7 @@ __global__ __launch_bounds__(1024, 4 * BLOCKS) void gemm_fp8_tile_kernel(
         const char* ab = smem + buf * STEP + wr * FI * 32 * GK2;
         const char* bb = smem + buf * STEP + (BM + wc * FJ * 32) * GK2;
         if (t + ST - 1 < ns) stage(buf == 0 ? ST - 1 : buf - 1);
+        if (wr * FI * 32 < BM)                               // (96 rows: two waves transfer alone)
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             i32x8_f8 fa[FI], fb[FJ];
@@ -968,6 +972,7 @@ __global__ __launch_bounds__(1024, 4 * BLOCKS) void gemm_fp8_tile_kernel(
         buf = buf + 1 == ST ? 0 : buf + 1;
     }
 
+    if (wr * FI * 32 >= BM) return;
     // 32x32 C/D map: col = lane & 31, row = (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5).
     // Row scales are read together (rows past the end repeat the last), not one by one
     // behind a branch each.
@@ -995,17 +1000,23 @@ __global__ __launch_bounds__(1024, 4 * BLOCKS) void gemm_fp8_tile_kernel(
 // above): one block of 128 x 128 a CU 0.62 (0.65 over several rounds, which start and end
 // bare), two of them 1.27 and less where the second ones are few, 128 x 256 1.12, 256 x 256
 // 1.9. It names the fastest for 39 of 40 sizes (12288 x 4096, M = 512: 42.1, 38.2).
+//
+// Tiles of 96 x 128, twelve waves at work and two that only transfer, take 0.54: the form where they fit one
+// round, which 128 rows leave a quarter empty or filled with rows past the end. us, 128 / 96 rows a tile: 4096 x
+// 14336, M = 300 55.6 / 49.6, 512 66.7 / 56.6, 700 68.9 / 59.4, 768 67.4 / 60.7; 4096 x 4096, 700 22.8 / 20.4;
+// 2048 x 8192, 1400 38.5 / 33.6; but in two rounds 4096 x 14336, 1000 70.5 / 103.9, 2048 112 / 167.
 static int gemm_fp8_tile(int64_t M, int64_t N, double* us = nullptr, int64_t* rounds = nullptr) {
     const int64_t n1 = CEIL_DIV(M, 128) * CEIL_DIV(N, 128), rest = n1 % 512;
     const int64_t n2 = CEIL_DIV(M, 128) * CEIL_DIV(N, 256), n3 = CEIL_DIV(M, 256) * CEIL_DIV(N, 256);
-    const double t[4] = {n1 <= 256 ? 0.62 : CEIL_DIV(n1, 256) * 0.65,
+    const int64_t n4 = CEIL_DIV(M, 96) * CEIL_DIV(N, 128);
+    const double t[5] = {n1 <= 256 ? 0.62 : CEIL_DIV(n1, 256) * 0.65,
                          n1 / 512 * 1.27 + (rest > 256 ? 0.86 + (rest - 256) * 0.0015 : rest > 0 ? 0.75 : 0.0),
-                         CEIL_DIV(n2, 256) * 1.12, CEIL_DIV(n3, 256) * 1.9};
+                         CEIL_DIV(n2, 256) * 1.12, CEIL_DIV(n3, 256) * 1.9, n4 <= 256 ? 0.54 : 1e9};
     int best = 0;
-    for (int i = 1; i < 4; ++i)
+    for (int i = 1; i < 5; ++i)
         if (t[i] < t[best]) best = i;
     if (us) *us = t[best];
-    if (rounds) *rounds = best == 1 ? CEIL_DIV(n1, 512) : CEIL_DIV(best == 0 ? n1 : best == 2 ? n2 : n3, 256);
+    if (rounds) *rounds = best == 1 ? CEIL_DIV(n1, 512) : CEIL_DIV(best == 0 ? n1 : best == 2 ? n2 : best == 3 ? n3 : n4, 256);
     return best;
 }
 
@@ -1027,12 +1038,13 @@ extern "C" int oa_gemm_fp8(void* stream, const void* a8, const void* b8,
         const int64_t items = (int64_t)CEIL_DIV(N, BN) * mt;                                       \
         if (items > (1 << 28)) return -101;                                                        \
         hipLaunchKernelGGL((gemm_fp8_tile_kernel<BM, BN, ST, BLOCKS>),                             \
-                           dim3((unsigned)(CEIL_DIV(items, 8) * 8)), dim3(1024),                   \
+                           dim3((unsigned)(CEIL_DIV(items, 8) * 8)), dim3(64 * G8_WAVES(BM)),      \
                            (ST) * (BM + BN) * GK2, (hipStream_t)stream, (const char*)a8,           \
                            (const char*)b8, (const float*)ascale, (const float*)bscale,            \
                            (uint16_t*)c, M, N, K, mt, (int)items);                                 \
     } while (0)
     switch (gemm_fp8_tile(M, N)) {
+        case 4: G8(96, 128, 4, 1); break;
         case 0: G8(128, 128, 4, 1); break;
         case 1: G8(128, 128, 2, 2); break;
         case 2: G8(128, 256, 3, 1); break;
