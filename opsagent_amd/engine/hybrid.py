@@ -268,8 +268,7 @@ class ChannelDeltaMixer(nn.Module):
         b_logits = proj[:, o0 : o0 + H]
         a1 = proj[:, o0 + H : o0 + H + self.ra]
         g1 = proj[:, o0 + H + self.ra :]
-        a = ops.linear(a1, self.a2_w)                         # [T, H*D]
-        gate = ops.linear(g1, self.g2_w)                      # [T, H*Dv]
+        a, gate = ops.linear_pair(a1, self.a2_w, g1, self.g2_w)    # [T, H*D], [T, H*Dv]
         y = mx.channel_delta_rule(
             qkv[:, : G * D], qkv[:, G * D : 2 * G * D], qkv[:, 2 * G * D :],
             b_logits, a, self.dt_bias, self.a_log, self.norm_w, gate, state["S"], sb,

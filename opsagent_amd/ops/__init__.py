@@ -601,6 +601,23 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x, w)
 
 
+def linear_pair(x0: torch.Tensor, w0: torch.Tensor, x1: torch.Tensor,
+                w1: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    """linear(x0, w0) and linear(x1, w1): in one launch where both are skinny strips of one size."""
+    M, (N, K) = x0.numel() // x0.shape[-1], w0.shape
+    if not (1 < M <= 16 and x0.shape == x1.shape and w0.shape == w1.shape and x0.dim() == 2
+            and x0.stride() == x1.stride() and x0.device == x1.device
+            and _skinny_ok(x0, w0) and _skinny_ok(x1, w1) and not _ring_form(M, N, K)
+            and _skinny_form(M, N, K, strided=not x0.is_contiguous()) == 1):
+        return linear(x0, w0), linear(x1, w1)
+    lib, hip = _lib()
+    out = torch.empty(2, M, N, dtype=x0.dtype, device=x0.device)
+    hip.check(lib.oa_skinny_pair(
+        hip.current_stream_ptr(), x0.data_ptr(), x1.data_ptr(), K if x0.is_contiguous() else x0.stride(0),
+        w0.data_ptr(), w1.data_ptr(), out[0].data_ptr(), out[1].data_ptr(), M, N, K), "oa_skinny_pair")
+    return out[0], out[1]
+
+
 def linear_float(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """linear(x, w).float(), of one bf16 row in the product's own launch where gemv.hip takes it."""
     N, K = w.shape

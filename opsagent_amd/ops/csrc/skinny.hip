@@ -31,6 +31,20 @@ __global__ __launch_bounds__(WV * 64) void skinny_strip_kernel(
     skinny_strip<MF, GU, WV, D>(x, xs, w, out, M, N, K, act, blockIdx.x, red);
 }
 
+// Two products of equal sizes in one launch (strips, up to 16 rows): one after the other they are a launch of
+// 5 us each, whose strips of short rows end before the chip is full. us, 3 rows of 256 columns against 4096
+// weight rows twice, traced one by one: 10.0 / 5.5.
+template <int WV>
+__global__ __launch_bounds__(WV * 64) void skinny_pair_kernel(
+    const uint16_t* __restrict__ x0, const uint16_t* __restrict__ x1, int64_t xs, const uint16_t* __restrict__ w0,
+    const uint16_t* __restrict__ w1, uint16_t* __restrict__ out0, uint16_t* __restrict__ out1, int M, int N, int K,
+    int units) {
+    __shared__ __attribute__((aligned(16))) SkinnyRed<1, false, WV> red;
+    const bool second = (int)blockIdx.x >= units;
+    skinny_strip<1, false, WV, 8>(second ? x1 : x0, xs, second ? w1 : w0, second ? out1 : out0, M, N, K, 0,
+                                  second ? blockIdx.x - units : blockIdx.x, red);
+}
+
 // Strips go gate, up, gate, up; a register of the ring is refilled with the next
 // strip's columns as soon as it is used, so a wave always has SW loads of 1 KiB in
 // flight, across the barrier of the partial sums too (two LDS buffers, one barrier
@@ -138,6 +152,24 @@ extern "C" int oa_skinny(void* stream, const void* x, int64_t xs, const void* w,
     } else {
         return -102;
     }
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
+// out0 = x0 w0^T and out1 = x1 w1^T, [M, N] of up to 16 rows xs elements apart, the strips of oa_skinny
+extern "C" int oa_skinny_pair(void* stream, const void* x0, const void* x1, int64_t xs, const void* w0, const void* w1,
+                              void* out0, void* out1, int M, int N, int K) {
+    if (M < 1 || M > 16 || N < 1 || K < 32 || K % 32 != 0 || xs % 8 != 0 || xs < K) return -100;
+    if (!x0 || !x1 || !w0 || !w1 || !out0 || !out1) return -101;
+    if (((uintptr_t)x0 | (uintptr_t)x1 | (uintptr_t)w0 | (uintptr_t)w1) % 16 != 0) return -102;
+    const int units = CEIL_DIV(N, 16);
+#define SKT(WV)                                                                                                 \
+    hipLaunchKernelGGL((skinny_pair_kernel<WV>), dim3(2 * units), dim3((WV) * 64), 0, (hipStream_t)stream,      \
+                       (const uint16_t*)x0, (const uint16_t*)x1, xs, (const uint16_t*)w0, (const uint16_t*)w1,  \
+                       (uint16_t*)out0, (uint16_t*)out1, M, N, K, units)
+    if (K >= 2 * N) SKT(4);                          // as oa_skinny
+    else SKT(8);
+#undef SKT
     HIP_CHECK_LAUNCH();
     return 0;
 }

@@ -69,6 +69,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_gemv_dyt_merge.restype = i
     lib.oa_gemv_float.argtypes = [p, p, p, p, i, i]
     lib.oa_gemv_float.restype = i
+    lib.oa_skinny_pair.argtypes = [p, p, p, i64, p, p, p, p, i, i, i]
+    lib.oa_skinny_pair.restype = i
     lib.oa_gemv_dyt.argtypes = [p, p, p, p, p, p, p, p, p, p, p, i, i]
     lib.oa_gemv_dyt.restype = i
     lib.oa_gemv_grouped.argtypes = [p, p, p, i, i, i, i, p, p, p, p, p, i]

@@ -223,7 +223,7 @@ def group_norm_step(y: Union[torch.Tensor, "ops.PlaneSum"], w: torch.Tensor, gro
     planes = y.planes if isinstance(y, ops.PlaneSum) else None
     join = conv is not None and sb.max_chunk == 1 and _conv_joins(*conv, C)
     data = y if planes is None else planes
-    if (residual.is_cuda and (join or planes is not None) and w.dtype == torch.bfloat16
+    if (residual.is_cuda and w.dtype == torch.bfloat16
             and data.dtype == (torch.bfloat16 if planes is None else torch.float32)
             and residual.dtype == torch.float32 and residual.is_contiguous() and w.is_contiguous()
             and C % groups == 0 and C // groups % 512 == 0 and C <= 8192
