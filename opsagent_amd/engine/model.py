@@ -134,7 +134,7 @@ class Attention(nn.Module):
     def _o(self, x: torch.Tensor, parts: bool = False) -> torch.Tensor:
         if self.fp8:
             return ops.linear_fp8(x, self.o_q, self.o_s)
-        return (ops.linear_parts if parts else ops.linear)(x, self.o_w)
+        return ops.linear_parts(x, self.o_w, True) if parts else ops.linear(x, self.o_w)
 
     def forward(
         self,
@@ -243,7 +243,8 @@ class DenseMLP(nn.Module):
                 x, self.gate_up_q, self.gate_up_s, self.i_local, self.down_q, self.down_s
             ))
         act = ops.gateup_silu(x, self.gate_up_w, self.i_local)
-        return tp_all_reduce((ops.linear_parts if parts else ops.linear)(act, self.down_w))
+        return tp_all_reduce(ops.linear_parts(act, self.down_w, True) if parts
+                             else ops.linear(act, self.down_w))
 
 
 _every_module = torch.nn.modules.module        # holds the hooks that are common to all

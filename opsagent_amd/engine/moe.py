@@ -121,7 +121,8 @@ class MoEMLP(nn.Module):
                     else:
                         idx, wts, lists, shared = front
                     if local and shared is None:
-                        shared = self.shared(x)
+                        # its last product's parts go on to the norm with the pairs
+                        shared = self.shared(x, True) if beside and parts else self.shared(x)
                     out = ops.moe_sorted_mlp(x, w13, s13, w2, s2, idx, wts, more=shared, parts=parts,
                                              lists=lists)
                 else:

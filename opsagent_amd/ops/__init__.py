@@ -542,13 +542,31 @@ def _tile(x: torch.Tensor, w: torch.Tensor, plan: int, act: int = 0,
     return part if parts else out
 
 
-def linear_parts(x: torch.Tensor, w: torch.Tensor) -> Union[torch.Tensor, PlaneSum]:
+@functools.lru_cache(maxsize=4096)
+def _shallow_parts(M: int, N: int, K: int) -> Optional[int]:
+    """The tile product's plan of more than 128 rows whose parts a norm adds up, for products of K < 2 N
+    that would be tiles anyway: where splits of more than one are the faster way by the same estimate.
+    They save the launch that would add them up, or fill CUs that one split leaves idle. us a prompt of
+    four layers, without / with: 4096 x 4096 in all, 130 rows 659 / 647, 256 797 / 779, 300 826 / 810,
+    512 1044 / 1038; 2048 x 2048, 512 516 / 498, and with 2048 x 2816 behind 64 experts 1330 / 1312. Larger
+    results cost as much to write in parts as splits gain (4096 x 4096, 600 1273 / 1276, 800 1555 / 1555)."""
+    if K >= 2 * N or M * N > 2200000 or _tile_sizes(M, N, K, False, False) is None:
+        return None
+    plan = _lib()[0].oa_tile_gemm_plan(M, N, K, 0, 1)
+    return plan if plan & 255 > 1 else None
+
+
+def linear_parts(x: torch.Tensor, w: torch.Tensor,
+                 shallow: bool = False) -> Union[torch.Tensor, PlaneSum]:
     """x @ w^T for rows x [T, K] that go through fused_add_rms_norm next: bf16 [T, N], or the
-    product's float32 column parts, which the norm adds up, where the transfer ring splits it."""
+    product's float32 column parts, which the norm adds up, where the transfer ring or the tile
+    product splits it (shallow: also above 128 rows of less than 2 N columns)."""
     M = x.numel() // x.shape[-1]
     if M > 1 and x.dim() == 2 and w.shape[0] <= 8192 and _skinny_ok(x, w):
         if M > 128:
             tile = _tile_choice(M, w.shape[0], w.shape[1], summed=True) if _near_rows(x) else None
+            if tile is None and shallow and _near_rows(x):
+                tile = _shallow_parts(M, w.shape[0], w.shape[1])
             return PlaneSum(_tile(x, w, tile, parts=True)) if tile and tile & 255 > 1 else linear(x, w)
         plan = _ring_form(M, w.shape[0], w.shape[1])
         if plan and plan[1] > 1:
@@ -694,11 +712,11 @@ class PlaneSum(NamedTuple):
 
 class PairSum(NamedTuple):
     """A sum that the norm behind it takes: for each token its `top` rows of y
-    [T * top, H], bf16, plus its row of `more`."""
+    [T * top, H], bf16, plus its row of `more`, which may be a product's parts."""
 
     y: torch.Tensor
     top: int
-    more: Optional[torch.Tensor]
+    more: Union[torch.Tensor, PlaneSum, None]
 
 
 def _added_up(x: Union[PlaneSum, PairSum]) -> torch.Tensor:
@@ -732,6 +750,13 @@ def _add_norm_parts(x: Union[PlaneSum, PairSum], residual: torch.Tensor, weight:
         hip.check(lib.oa_add_rmsnorm_parts(
             hip.current_stream_ptr(), data.data_ptr(), n, at, w, out.data_ptr(), rows, dim, eps),
             "oa_add_rmsnorm_parts")
+    elif isinstance(x.more, PlaneSum):
+        more = x.more.planes
+        assert more.shape[1:] == (rows, dim) and more.dtype == torch.float32
+        assert more.is_contiguous() and more.get_device() == residual.get_device()
+        hip.check(lib.oa_add_rmsnorm_pairs_parts(
+            hip.current_stream_ptr(), data.data_ptr(), n, more.data_ptr(), more.shape[0], at, w,
+            out.data_ptr(), rows, dim, eps), "oa_add_rmsnorm_pairs_parts")
     else:
         hip.check(lib.oa_add_rmsnorm_pairs(
             hip.current_stream_ptr(), data.data_ptr(), n,
@@ -1150,12 +1175,16 @@ def moe_route(x: torch.Tensor, router_w: torch.Tensor, top: int):
     return idx, wts, tok
 
 
-def moe_combine(y: torch.Tensor, top: int, more: Optional[torch.Tensor] = None,
+def moe_combine(y: torch.Tensor, top: int, more: Union[torch.Tensor, PlaneSum, None] = None,
                 parts: bool = False) -> Union[torch.Tensor, PairSum]:
     """out[t] = sum of rows t * top .. + top of y [T * top, H] (+ more[t]), bf16
     with float32 sums in one order. With `parts` it may be left to the norm that follows."""
     T, H = y.shape[0] // top, y.shape[1]
     assert y.is_cuda and y.dtype == torch.bfloat16 and y.is_contiguous()
+    if isinstance(more, PlaneSum):
+        if parts and H % 8 == 0 and H <= 8192 and more.planes.shape[1:] == (T, H):
+            return PairSum(y, top, more)
+        more = _added_up(more)
     assert more is None or (more.shape == (T, H) and more.dtype == y.dtype
                             and more.is_contiguous())
     if parts and H % 8 == 0 and H <= 8192 and (more is None or more.data_ptr() % 16 == 0):
@@ -1277,7 +1306,7 @@ def moe_sorted_mlp(
     expert_ids: torch.Tensor,
     pair_weights: torch.Tensor,
     act=None,
-    more: Optional[torch.Tensor] = None,
+    more: Union[torch.Tensor, PlaneSum, None] = None,
     parts: bool = False,
     lists: Optional[torch.Tensor] = None,
 ) -> Union[torch.Tensor, PairSum]:

@@ -210,8 +210,11 @@ extern "C" int oa_add_rmsnorm_parts(void* stream, const void* x, int parts, void
 // bf16, and its row of `more` if there is one, in that order in float32, rounded to bf16 as
 // the sum by itself would be. One launch and one pass less: a decode step of 13 tokens over 4
 // layers of 64 experts 599 -> 586 us, a prompt of 512 1427 -> 1418.
+// PARTS: `more` is still the n float32 planes [rows, 8 * D8] of its product, added up and rounded as the
+// product alone would be: a prompt of 512 over those layers 1313 -> 1305.
+template <bool PARTS>
 __global__ __launch_bounds__(1024) void rmsnorm_pairs_kernel(
-    const uint4* __restrict__ y, int top, const uint4* __restrict__ more,
+    const uint4* __restrict__ y, int top, const uint4* __restrict__ more, int n,
     uint4* __restrict__ residual, const uint4* __restrict__ w, uint4* __restrict__ out, int D8,
     float inv_d, float eps) {
     __shared__ float red[16];
@@ -222,7 +225,24 @@ __global__ __launch_bounds__(1024) void rmsnorm_pairs_kernel(
     if (c < D8) {
         const uint4 r = residual[at];
         g = w[c];
-        const uint4 m = more ? more[at] : make_uint4(0, 0, 0, 0);
+        uint4 m = make_uint4(0, 0, 0, 0);
+        if (PARTS) {
+            float p[8] = {};
+#pragma unroll 4
+            for (int k = 0; k < n; ++k)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const float4 u = reinterpret_cast<const float4*>(more)[((int64_t)k * gridDim.x * D8 + at) * 2 + h];
+                    p[4 * h] += u.x;
+                    p[4 * h + 1] += u.y;
+                    p[4 * h + 2] += u.z;
+                    p[4 * h + 3] += u.w;
+                }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) (&m.x)[j] = pack_bf16x2(p[2 * j], p[2 * j + 1]);
+        } else if (more) {
+            m = more[at];
+        }
         const uint4* row = y + (int64_t)blockIdx.x * top * D8 + c;
         float a[8] = {};
 #pragma unroll 8
@@ -265,8 +285,21 @@ extern "C" int oa_add_rmsnorm_pairs(void* stream, const void* y, int top, const 
     if (dim % 8 != 0 || dim > 8192 || top < 1 || rows < 1) return -100;
     if (((uintptr_t)y | (uintptr_t)more | (uintptr_t)residual | (uintptr_t)w | (uintptr_t)out) % 16 != 0)
         return -101;
-    hipLaunchKernelGGL(rmsnorm_pairs_kernel, dim3(rows), dim3(CEIL_DIV(dim / 8, WAVE) * WAVE), 0,
-                       (hipStream_t)stream, (const uint4*)y, top, (const uint4*)more,
+    hipLaunchKernelGGL((rmsnorm_pairs_kernel<false>), dim3(rows), dim3(CEIL_DIV(dim / 8, WAVE) * WAVE), 0,
+                       (hipStream_t)stream, (const uint4*)y, top, (const uint4*)more, 0,
+                       (uint4*)residual, (const uint4*)w, (uint4*)out, dim / 8, 1.0f / dim, eps);
+    HIP_CHECK_LAUNCH();
+    return 0;
+}
+
+// more: n float32 planes [rows, dim]
+extern "C" int oa_add_rmsnorm_pairs_parts(void* stream, const void* y, int top, const void* more, int n,
+                                          void* residual, const void* w, void* out, int rows, int dim, float eps) {
+    if (dim % 8 != 0 || dim > 8192 || top < 1 || rows < 1 || n < 1 || !more) return -100;
+    if (((uintptr_t)y | (uintptr_t)more | (uintptr_t)residual | (uintptr_t)w | (uintptr_t)out) % 16 != 0)
+        return -101;
+    hipLaunchKernelGGL((rmsnorm_pairs_kernel<true>), dim3(rows), dim3(CEIL_DIV(dim / 8, WAVE) * WAVE), 0,
+                       (hipStream_t)stream, (const uint4*)y, top, (const uint4*)more, n,
                        (uint4*)residual, (const uint4*)w, (uint4*)out, dim / 8, 1.0f / dim, eps);
     HIP_CHECK_LAUNCH();
     return 0;

@@ -37,6 +37,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_embed_rmsnorm.restype = i
     lib.oa_add_rmsnorm_pairs.argtypes = [p, p, i, p, p, p, p, i, i, f]
     lib.oa_add_rmsnorm_pairs.restype = i
+    lib.oa_add_rmsnorm_pairs_parts.argtypes = [p, p, i, p, i, p, p, p, i, i, f]
+    lib.oa_add_rmsnorm_pairs_parts.restype = i
     lib.oa_add_rmsnorm_parts.argtypes = [p, p, i, p, p, p, i, i, f]
     lib.oa_add_rmsnorm_parts.restype = i
     lib.oa_fused_add_rmsnorm.argtypes = [p, p, p, p, p, i, i, f]
