@@ -1034,9 +1034,9 @@ def mlp_fp8(
     down_q: torch.Tensor, down_s: torch.Tensor,
 ) -> torch.Tensor:
     """(silu(x @ gate8^T) * (x @ up8^T)) @ down8^T. Where both products are tile
-    products (prefill rows), the activation is quantized as it is made: the same bf16
-    values, rows and scales as quantizing it afterwards. x may be quantized already, where
-    mlp_fp8_rows_ok says so."""
+    products (prefill rows), the activation is made by the wide tiles of the first one or
+    quantized as it is made: the same bf16 values, rows and scales as quantizing it afterwards.
+    x may be quantized already, where mlp_fp8_rows_ok says so."""
     if isinstance(x, QuantRows):
         M, tiles = x.shape[0], True
     else:
@@ -1044,13 +1044,27 @@ def mlp_fp8(
         tiles = _is_gpu(x) and mlp_fp8_rows_ok(M, x.shape[-1], i_local, gate_up_q)
     if not tiles:
         return linear_fp8(gateup_silu_fp8(x, gate_up_q, gate_up_s, i_local), down_q, down_s)
-    gu = linear_fp8(x, gate_up_q, gate_up_s)
     lib, hip = _lib()
-    a8 = torch.empty(M, i_local, dtype=torch.uint8, device=gu.device)
-    a_scale = torch.empty(M, dtype=torch.float32, device=gu.device)
-    hip.check(lib.oa_silu_quant_fp8(hip.current_stream_ptr(), gu.data_ptr(), a8.data_ptr(),
-                                    a_scale.data_ptr(), M, i_local), "oa_silu_quant_fp8")
-    return _gemm_fp8(a8, a_scale, down_q, down_s).view(*x.shape[:-1], down_q.shape[0])
+    lead, K = x.shape[:-1], x.shape[-1]
+    if not isinstance(x, QuantRows):
+        assert x.dtype == torch.bfloat16 and x.is_contiguous()
+        x = QuantRows(*quant_fp8(x.reshape(M, K)))
+    form = -1
+    if M > 128 and not _ring_choice_fp8(M, 2 * i_local, K) and (i_local + 256) * K < 2 ** 32:
+        form = _tile_form_fp8(M, 2 * i_local, K)
+    if 0 <= form <= 2 and (x.rows.data_ptr() | gate_up_q.data_ptr()) % 16 == 0:
+        act = torch.empty(M, i_local, dtype=torch.bfloat16, device=x.rows.device)
+        hip.check(lib.oa_tile_gemm_fp8_silu(
+            hip.current_stream_ptr(), x.rows.data_ptr(), x.scales.data_ptr(), gate_up_q.data_ptr(),
+            gate_up_s.data_ptr(), act.data_ptr(), M, i_local, K, form), "oa_tile_gemm_fp8_silu")
+        a8, a_scale = quant_fp8(act)
+    else:
+        gu = linear_fp8(x, gate_up_q, gate_up_s)
+        a8 = torch.empty(M, i_local, dtype=torch.uint8, device=gu.device)
+        a_scale = torch.empty(M, dtype=torch.float32, device=gu.device)
+        hip.check(lib.oa_silu_quant_fp8(hip.current_stream_ptr(), gu.data_ptr(), a8.data_ptr(),
+                                        a_scale.data_ptr(), M, i_local), "oa_silu_quant_fp8")
+    return _gemm_fp8(a8, a_scale, down_q, down_s).view(*lead, down_q.shape[0])
 
 
 def linear_norm(

@@ -89,6 +89,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.oa_tile_gemm.restype = i
     lib.oa_tile_gemm_fp8_form.argtypes = [i, i, i]
     lib.oa_tile_gemm_fp8_form.restype = i
+    lib.oa_tile_gemm_fp8_silu.argtypes = [p, p, p, p, p, p, i, i, i, i]
+    lib.oa_tile_gemm_fp8_silu.restype = i
     lib.oa_tile_gemm_fp8.argtypes = [p, p, p, p, p, p, i, i, i, i]
     lib.oa_tile_gemm_fp8.restype = i
     lib.oa_skinny.argtypes = [p, p, i64, p, p, i, i, i, i, i, i]
