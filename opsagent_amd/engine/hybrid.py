@@ -1516,11 +1516,13 @@ class HybridForCausalLM(nn.Module):
         # what goes into a layer that is looked at may change on the way: it starts by itself then
         joined = all(map(_sums_parts, layers))
         for i, layer in enumerate(layers):
-            if joined and i + 1 < len(layers):
+            if not joined:
+                x = layer(x, sb, kv_caches[i], state[i])
+            elif i + 1 < len(layers):
                 nxt = (layers[i + 1].canon_w, state[i + 1]["canon"])
                 x, h = layer(x, sb, kv_caches[i], state[i], h, nxt)
             else:
-                x, h = layer(x, sb, kv_caches[i], state[i], h), None
+                x = layer(x, sb, kv_caches[i], state[i], h)
             if self.trace_layers is not None:
                 self.trace_layers.append(x.clone())
         return x  # float32 residual [T, C]; compute_logits norms the rows it needs

@@ -82,3 +82,49 @@ def test_attention_preparation(H, G, D, Dv, extra, parts, monkeypatch):
     # one rounding to bf16, and float32 before it
     for got, ref in ((q[:B], want), *zip(caches, far)):
         assert torch.allclose(got.double().cpu(), ref.double(), rtol=2.0 ** -8 + 2.0 ** -18, atol=2.0 ** -18)
+
+
+class Plain(torch.nn.Module):
+    """A layer of another class, as a user's program may put around one: it takes what layers take."""
+
+    def __init__(self, layer):
+        super().__init__()
+        self.layer = layer
+        self.canon_w = layer.canon_w
+
+    def forward(self, x, sb, kv, state):
+        return self.layer(x, sb, kv, state)
+
+
+@pytest.mark.parametrize("device", [pytest.param("cpu", id="cpu"), pytest.param("cuda", id="gpu", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("way", ["class", "hook"])
+def test_layers_that_are_looked_at(device, way):
+    """Each then starts with its own convolution, and a hook's rows are what the next one reads."""
+    import test_povazen as P
+
+    P._skip_if_wrong_device(device)
+    cfg = P.make_cfg(pattern="DaA")
+    W = P.other_ranks(cfg, P.O.random_weights(cfg, seed=3))
+    toks = P.tokens_for(cfg, 9, 4)
+    schedule = [(toks[:6], [5])] + [([t], [0]) for t in toks[6:]]
+
+    def logits(change):
+        eng = P.build_engine(cfg, W)
+        change(eng.model)
+        rp = P.TraceReplayer(eng)
+        return torch.cat([rp.step([{"id": "a", "tokens": t, "want": w}], []).cpu() for t, w in schedule])
+
+    want = logits(lambda m: None)
+
+    def wrap(m):
+        m.layers[1] = Plain(m.layers[1])
+
+    if way == "class":
+        assert torch.allclose(logits(wrap), want, rtol=1e-5, atol=1e-5)
+        return
+    seen = []
+    look = lambda mod, args, out: seen.append(out.shape)  # noqa: E731
+    assert torch.allclose(logits(lambda m: m.layers[0].register_forward_hook(look)), want, rtol=1e-5, atol=1e-5)
+    assert seen
+    double = logits(lambda m: m.layers[0].register_forward_hook(lambda mod, args, out: 2 * out))
+    assert not torch.allclose(double, want, rtol=1e-3)
