@@ -87,6 +87,12 @@ def _init_linear(gen: torch.Generator, out_f: int, in_f: int, dtype) -> torch.Te
     return (w * std).to(dtype)
 
 
+def _product_parts(x: torch.Tensor, w: torch.Tensor) -> Union[torch.Tensor, ops.PlaneSum]:
+    """x @ w^T for the norm behind it, which adds up the parts of a split product."""
+    parts = ops.shallow_parts(x, w)
+    return ops.linear_parts(x, w) if parts is None else parts
+
+
 class Attention(nn.Module):
     sums_parts = True           # see _sums_parts
 
@@ -134,7 +140,7 @@ class Attention(nn.Module):
     def _o(self, x: torch.Tensor, parts: bool = False) -> torch.Tensor:
         if self.fp8:
             return ops.linear_fp8(x, self.o_q, self.o_s)
-        return ops.linear_parts(x, self.o_w, True) if parts else ops.linear(x, self.o_w)
+        return _product_parts(x, self.o_w) if parts else ops.linear(x, self.o_w)
 
     def forward(
         self,
@@ -243,8 +249,7 @@ class DenseMLP(nn.Module):
                 x, self.gate_up_q, self.gate_up_s, self.i_local, self.down_q, self.down_s
             ))
         act = ops.gateup_silu(x, self.gate_up_w, self.i_local)
-        return tp_all_reduce(ops.linear_parts(act, self.down_w, True) if parts
-                             else ops.linear(act, self.down_w))
+        return tp_all_reduce((_product_parts if parts else ops.linear)(act, self.down_w))
 
 
 _every_module = torch.nn.modules.module        # holds the hooks that are common to all
