@@ -1461,6 +1461,7 @@ class HybridForCausalLM(nn.Module):
     def forward(self, fb: ForwardBatch, kv_caches, state=None) -> torch.Tensor:
         sb = fb.seq_batch
         assert sb is not None and state is not None, "hybrid models run flat multi-sequence steps"
+        h = None                    # the first norm's rows, where the embedding's launch made them
         if self.embed_norm_w is not None:
             x = mx.embed_norm_rows(self.embed, fb.input_ids, self.embed_norm_w,
                                    self.spec.norm_eps, offset=1.0)
@@ -1500,9 +1501,9 @@ class HybridForCausalLM(nn.Module):
             return xs.sum(1) if S > 1 else xs.squeeze(1)
         if self.sandwich or self.pre_norm:
             n = len(self.layers)
-            if self.sandwich and self.pos_freq is not None:
+            if self.sandwich and h is None:
                 h = mx.dyt_norm(x, self.layers[0].first_norm(), self.dtype)
-            elif not self.sandwich:
+            elif self.pre_norm:
                 h = mx.add_layer_norm(x, self.layers[0].first_norm(), self.spec.norm_eps,
                                       self.dtype)
             for i, layer in enumerate(self.layers):
@@ -1512,7 +1513,7 @@ class HybridForCausalLM(nn.Module):
                 if self.trace_layers is not None:
                     self.trace_layers.append(x.clone())
             return x
-        layers, h = list(self.layers), None
+        layers = list(self.layers)
         # what goes into a layer that is looked at may change on the way: it starts by itself then
         joined = all(map(_sums_parts, layers))
         for i, layer in enumerate(layers):
