@@ -16,8 +16,8 @@
 //
 // Small launches: a split is `chunk` keys, a multiple of 64 (decode_chunk), and blocks past a
 // sequence's last key end at once. Larger ones: the tiles of 64 keys of all sequences are cut in
-// equal runs, one a CU (DecodeRuns). Either way at most nsplit splits cover a sequence, a mark
-// stands behind its last one, and the combine reads those before it.
+// equal runs, one a CU (DecodeRuns). Either way at most nsplit splits cover a sequence, and the
+// combine reads those that exist: plain splits it counts, behind a sequence's last run stands a mark.
 
 #include <type_traits>
 
@@ -65,8 +65,8 @@ __device__ __forceinline__ float swap_add(float a, float b) {
 // a full step pays for the look: 64 of up to 3000 112.3 -> 112.8, of up to 300 22.1 -> 22.5.
 // (With splits of each sequence; runs leave such rows out and look at them in blocks of their own.)
 //
-// Marks stand where a sum of weights would be: of a copy's first split, of the place behind a
-// row's last one.
+// Marks stand where a sum of weights would be: of a copy's first split, with runs of the place behind
+// a row's last one.
 #define COPY_MARK -1.0f
 #define END_MARK -2.0f
 template <int G>
@@ -244,22 +244,27 @@ struct Planes {
     int splits;
     int64_t plane;
 };
-struct NoPlanes {};
+struct Runs {
+    int count;
+};
 
-template <int G, bool FUSED, bool ROPE, bool RUNS, bool PARTS = false>
+// MORE: Runs with RUNS, otherwise Planes or nothing. (What a form has no use for is no argument: with a
+// few bytes of such arguments here and in gemv1_kernel, decode steps of an 8B model took 2916 us, 2910 without.)
+template <int G, bool FUSED, bool ROPE, bool RUNS, typename... MORE>
 __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kernel(
     const uint32_t* __restrict__ q, const uint32_t* __restrict__ kc,
     const uint32_t* __restrict__ vc, const int* __restrict__ block_table,
     const int* __restrict__ seq_lens, float* __restrict__ o_part,
     float* __restrict__ ml_part, unsigned* __restrict__ cnt,
     uint32_t* __restrict__ out, int B, int Hk, int max_blocks,
-    int block_shift /* log2(block_size) */, int nsplit, int chunk_base, int runs, float scale,
+    int block_shift /* log2(block_size) */, int nsplit, int chunk_base, float scale,
     int qs2 /* q batch-row stride in words */,
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
     const float* __restrict__ cs, const float* __restrict__ sn,
     const int* __restrict__ slots, uint32_t* __restrict__ kcw,
-    uint32_t* __restrict__ vcw, int ks2, int vs2, int copies,
-    std::conditional_t<PARTS, Planes, NoPlanes> planes) {
+    uint32_t* __restrict__ vcw, int ks2, int vs2, int copies, MORE... more) {
+    constexpr bool PARTS = std::is_same_v<void(MORE...), void(Planes)>;
+    static_assert(RUNS ? std::is_same_v<void(MORE...), void(Runs)> : PARTS || sizeof...(MORE) == 0, "one form");
     static_assert(!PARTS || (ROPE && !RUNS && !FUSED), "parts of a projection: plain launches only");
     constexpr int GP = G > 4 ? 8 : 4;            // columns of one part of the queries
     constexpr int KL = GP / 4;                   // keys per lane and tile
@@ -267,12 +272,12 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
     // the block takes, and how many it still has to take
     int b, h, split, n, kstart, kend, own = 0, from = 0, left = 0;
     bool once = false;                               // value rows are read without being kept
-    if (RUNS) {
+    if constexpr (RUNS) {
         const int at = blockIdx.y, whole = gridDim.y - copies * (B - 1);
         h = blockIdx.x;
         split = 0;
         if (at < whole) {
-            const DecodeRuns r = decode_runs(seq_lens, slots, B, copies, runs, nsplit, chunk_base, at);
+            const DecodeRuns r = decode_runs(seq_lens, slots, B, copies, more.count..., nsplit, chunk_base, at);
             if (r.b < 0) return;
             b = r.b;
             n = r.n;
@@ -306,7 +311,7 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
         const int chunk = decode_chunk(n, nsplit, chunk_base);
         kstart = split * chunk;
         if (!FUSED && kstart >= n) return;
-        if (ROPE && maybe_copy(slots, seq_lens, b, copies) &&
+        if (ROPE && copies && b > 0 && slots[b] == slots[0] && n == seq_lens[0] &&
             copy_of_first<G>(q, qs2, kin, ks2, vin, vs2, block_table, max_blocks, b, h,
                              CEIL_DIV(n, 1 << block_shift))) {
             if (split == 0 && threadIdx.x < G)
@@ -391,6 +396,7 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
     da_f4 in[NIN][NP];
     const da_f4* ip[NIN];
     if constexpr (PARTS) {
+        const Planes planes(more...);
 #pragma unroll
         for (int i = 0; i < NIN; ++i) {
             const int c = min((int)(i * 256 + threadIdx.x) * 4, (G + 2) * DHEAD - 4), at = c / DHEAD;
@@ -428,6 +434,7 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
     };
     if (!RUNS || row == 0) load_first();
     if constexpr (PARTS) {
+        const Planes planes(more...);
 #pragma unroll
         for (int i = 0; i < NIN; ++i) {
             const int c = (i * 256 + threadIdx.x) * 4;
@@ -668,7 +675,7 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
     const int bh = b * Hk + h;
     float* opart_row = o_part + ((size_t)(bh * nsplit + split) * G) * DHEAD;
     float* mlpart_row = ml_part + ((size_t)(bh * nsplit + split) * G) * 2;
-    const bool last = !FUSED && kend == n && split + 1 < nsplit;    // of a row's splits, and not of all places
+    const bool last = RUNS && kend == n && split + 1 < nsplit;    // of a row's splits, and not of all places
     auto next = [&]() {
         left -= own - from;
         if (left <= 0) return;
@@ -804,16 +811,19 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
 
 // Combine split partials -> final output. Grid: B*Hq blocks of NG groups of 32 lanes; a
 // group takes the splits s, s + NG, ..., a lane four channels. A small launch like this is
-// its chain of loads, so statistics and a group's first two splits (EARLY) or the first one of
-// two groups, which nearly always are there, are asked for together, before a mark says how many
-// there are: what lies behind it is not looked at. Every wave works the common maximum and
-// sum out for itself. Both launches, us, the splits counted from the lengths / by the mark: 64 of
-// up to 300 tokens 22.9 / 20.8, 33 of up to 1500 39.9 / 38.5, 47 of up to 3000 76.7 / 74.5.
-template <int G, bool EARLY>
+// its chain of loads, so a group's first two splits and all statistics are asked for
+// together, and where the chip has room to spare (EARLY) even before the length says
+// which of them exist: what a split past the end left is not looked at. Every wave works
+// the common maximum and sum out for itself.
+// RUNS: statistics and the first splits of two groups, which nearly always are there, are asked for
+// before a mark says how many there are. Both launches, us, the splits counted from the lengths / by
+// the mark: 64 of up to 300 tokens 22.9 / 20.8, 33 of up to 1500 39.9 / 38.5, 47 of up to 3000 76.7 /
+// 74.5. Small launches would wait for it: decode steps of an 8B model, one sequence, 2926 us by marks, 2916 counted.
+template <int G, bool EARLY, bool RUNS>
 __global__ __launch_bounds__(EARLY ? 512 : 256) void decode_combine_kernel(
     const float* __restrict__ o_part, const float* __restrict__ ml_part,
     const int* __restrict__ seq_lens, uint32_t* __restrict__ out, int B, int Hk, int nsplit,
-    int copies) {
+    int chunk_base, const int* __restrict__ slots) {
     constexpr int NG = EARLY ? 16 : 8;
     const int bq = blockIdx.x;
     const int Hq = Hk * G;
@@ -823,41 +833,57 @@ __global__ __launch_bounds__(EARLY ? 512 : 256) void decode_combine_kernel(
     const int gh = qh % G;
     const int lane = threadIdx.x & (WAVE - 1);
     const int grp = threadIdx.x >> 5, ch = (threadIdx.x & 31) * 4;
+    size_t first = (size_t)(b * Hk + h) * nsplit * G + gh;
     const int n = seq_lens[b];
-    const float2* ml = nullptr;
-    const float* op = nullptr;
+    if (!EARLY && !RUNS && slots && b > 0 && slots[b] == slots[0] && n == seq_lens[0] && n > 0 &&
+        ml_part[first * 2 + 1] == COPY_MARK)
+        first = (size_t)h * nsplit * G + gh;
+    const float2* ml = reinterpret_cast<const float2*>(ml_part) + first;
+    const float* op = o_part + first * DHEAD + ch;
+
+    // the statistics of split `lane`, the first two splits of the own group, and how many exist
+    const float2 none = {0.0f, 0.0f};
     float2 mine, mo[2];
     float4 ov[2];
-    // asked for before it is known whether they are there: EARLY all, otherwise each wave's first
-    auto look = [&](int pair) {
-        const size_t first = (size_t)pair * nsplit * G + gh;
-        ml = reinterpret_cast<const float2*>(ml_part) + first;
-        op = o_part + first * DHEAD + ch;
-        mine = ml[min(lane, nsplit - 1) * G];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int s = min(grp + NG * i, nsplit - 1);
-            if (!EARLY && !(i == 0 && grp < 2)) continue;
-            mo[i] = ml[s * G];
-            ov[i] = *reinterpret_cast<const float4*>(op + (size_t)s * G * DHEAD);
-        }
+    auto ask = [&](int i, int s) {
+        mo[i] = ml[s * G];
+        ov[i] = *reinterpret_cast<const float4*>(op + (size_t)s * G * DHEAD);
     };
-    look(b * Hk + h);
-    if (!EARLY && copies && __any(lane == 0 && mine.y == COPY_MARK)) look(h);
-    int ns = 0;                                      // the splits end at a mark or with the places
-    for (int s0 = 0; n > 0 && s0 < nsplit; s0 += WAVE) {
-        const bool end = s0 + lane >= nsplit || (s0 ? ml[(s0 + lane) * G] : mine).y == END_MARK;
-        const uint64_t ends = __ballot(end);
-        ns = s0 + (ends ? __builtin_ctzll(ends) : WAVE);
-        if (ends) break;
-    }
-    if (!EARLY) {
+    int ns = 0;
+    if constexpr (RUNS) {
+        auto look = [&]() {
+            mine = ml[min(lane, nsplit - 1) * G];
+            if (grp < 2) ask(0, min(grp, nsplit - 1));
+        };
+        look();
+        if (slots && __any(lane == 0 && mine.y == COPY_MARK)) {
+            first = (size_t)h * nsplit * G + gh;
+            ml = reinterpret_cast<const float2*>(ml_part) + first;
+            op = o_part + first * DHEAD + ch;
+            look();
+        }
+        // the splits end at a mark or with the places
+        for (int s0 = 0; n > 0 && s0 < nsplit; s0 += WAVE) {
+            const bool end = s0 + lane >= nsplit || (s0 ? ml[(s0 + lane) * G] : mine).y == END_MARK;
+            const uint64_t ends = __ballot(end);
+            ns = s0 + (ends ? __builtin_ctzll(ends) : WAVE);
+            if (ends) break;
+        }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int s = grp + NG * i;
-            if ((i == 0 && grp < 2) || s >= ns) continue;
-            mo[i] = ml[s * G];
-            ov[i] = *reinterpret_cast<const float4*>(op + (size_t)s * G * DHEAD);
+            if (!(i == 0 && grp < 2) && s < ns) ask(i, s);
+        }
+    } else {
+        ns = CEIL_DIV(n, decode_chunk(n, nsplit, chunk_base));
+        // EARLY repeats the last split instead of a branch for each load
+        mine = EARLY || lane < ns ? ml[(EARLY ? min(lane, nsplit - 1) : lane) * G] : none;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int s = EARLY ? min(grp + NG * i, nsplit - 1) : grp + NG * i;
+            mo[i] = EARLY || s < ns ? ml[s * G] : none;
+            ov[i] = EARLY || s < ns ? *reinterpret_cast<const float4*>(op + (size_t)s * G * DHEAD)
+                                    : float4{0.0f, 0.0f, 0.0f, 0.0f};
         }
     }
 
@@ -926,15 +952,16 @@ static int decode_run_blocks(int runs, int cb, int B) {
 // splits that do not exist (64 of up to 300: 24.1 -> 25.0).
 template <int G>
 static void launch_combine(hipStream_t s, const void* o_part, const void* ml_part,
-                           const void* seq_lens, void* out, int B, int Hk, int nsplit, int copies) {
-    if (B * Hk <= 64 && !copies)
-        hipLaunchKernelGGL((decode_combine_kernel<G, true>), dim3(B * Hk * G), dim3(512), 0, s,
-                           (const float*)o_part, (const float*)ml_part, (const int*)seq_lens,
-                           (uint32_t*)out, B, Hk, nsplit, 0);
-    else
-        hipLaunchKernelGGL((decode_combine_kernel<G, false>), dim3(B * Hk * G), dim3(256), 0, s,
-                           (const float*)o_part, (const float*)ml_part, (const int*)seq_lens,
-                           (uint32_t*)out, B, Hk, nsplit, copies);
+                           const void* seq_lens, void* out, int B, int Hk, int nsplit, int cb,
+                           const void* slots, bool runs) {
+#define LAUNCH_C(EARLY, RUNS)                                                                      \
+    hipLaunchKernelGGL((decode_combine_kernel<G, EARLY, RUNS>), dim3(B * Hk * G),                  \
+                       dim3((EARLY) ? 512 : 256), 0, s, (const float*)o_part, (const float*)ml_part, \
+                       (const int*)seq_lens, (uint32_t*)out, B, Hk, nsplit, cb, (const int*)slots)
+    if (runs) LAUNCH_C(false, true);
+    else if (B * Hk <= 64) LAUNCH_C(true, false);
+    else LAUNCH_C(false, false);
+#undef LAUNCH_C
 }
 
 // fused: cnt_ws is zeroed here on each call (hipMemsetAsync). fused = 0: two kernels.
@@ -962,24 +989,24 @@ extern "C" int oa_attention_decode(void* stream, const void* q, const void* kc,
     const int cb = decode_chunk_base(B * Hk);
     const int runs = fused ? 0 : decode_run_count(B, Hk, nsplit);
     if (runs) grid = dim3(Hk, decode_run_blocks(runs, cb, B));
-#define LAUNCH_FORM(GV, FUSED, RUNS)                                                           \
+#define LAUNCH_FORM(GV, FUSED, RUNS, ...)                                                      \
     hipLaunchKernelGGL((decode_attn_kernel<GV, FUSED, false, RUNS>), grid, block, 0,           \
                        (hipStream_t)stream, (const uint32_t*)q, (const uint32_t*)kc,           \
                        (const uint32_t*)vc, (const int*)block_table, (const int*)seq_lens,     \
                        (float*)o_part, (float*)ml_part, (unsigned*)cnt_ws, (uint32_t*)out, B,  \
-                       Hk, max_blocks, block_shift, nsplit, cb, runs, scale, qs2,              \
+                       Hk, max_blocks, block_shift, nsplit, cb, scale, qs2,                    \
                        (const uint32_t*)nullptr, (const uint32_t*)nullptr,                     \
                        (const float*)nullptr, (const float*)nullptr, (const int*)nullptr,      \
-                       (uint32_t*)nullptr, (uint32_t*)nullptr, 0, 0, 0, NoPlanes())
+                       (uint32_t*)nullptr, (uint32_t*)nullptr, 0, 0, 0, ##__VA_ARGS__)
 #define LAUNCH_G(GV)                                                                           \
     do {                                                                                       \
         if (fused) LAUNCH_FORM(GV, true, false);                                               \
-        else if (runs) LAUNCH_FORM(GV, false, true);                                           \
+        else if (runs) LAUNCH_FORM(GV, false, true, Runs{runs});                               \
         else LAUNCH_FORM(GV, false, false);                                                    \
         HIP_CHECK_LAUNCH();                                                                    \
         if (!fused) {                                                                          \
             launch_combine<GV>((hipStream_t)stream, o_part, ml_part, seq_lens, out, B, Hk,     \
-                               nsplit, 0);                                                     \
+                               nsplit, cb, nullptr, runs);                                     \
             HIP_CHECK_LAUNCH();                                                                \
         }                                                                                      \
     } while (0)
@@ -1020,22 +1047,22 @@ extern "C" int oa_attention_decode_rope(
     const int runs = decode_run_count(B, Hk, nsplit);
     // rows that may be copies follow the runs
     if (runs) grid = dim3(Hk, decode_run_blocks(runs, cb, B) + copies * (B - 1));
-#define LAUNCH_FORM(GV, RUNS)                                                                  \
+#define LAUNCH_FORM(GV, RUNS, ...)                                                             \
     hipLaunchKernelGGL((decode_attn_kernel<GV, false, true, RUNS>), grid, block, 0,            \
                        (hipStream_t)stream, (const uint32_t*)q, (const uint32_t*)kc,           \
                        (const uint32_t*)vc, (const int*)block_table, (const int*)seq_lens,     \
                        (float*)o_part, (float*)ml_part, (unsigned*)nullptr, (uint32_t*)out, B, \
-                       Hk, max_blocks, block_shift, nsplit, cb, runs, scale, q_stride / 2,     \
+                       Hk, max_blocks, block_shift, nsplit, cb, scale, q_stride / 2,           \
                        (const uint32_t*)kin, (const uint32_t*)vin, (const float*)cos_t,        \
                        (const float*)sin_t, (const int*)slots, (uint32_t*)kc, (uint32_t*)vc,   \
-                       k_stride / 2, v_stride / 2, copies, NoPlanes())
+                       k_stride / 2, v_stride / 2, copies, ##__VA_ARGS__)
 #define LAUNCH_GR(GV)                                                                          \
     do {                                                                                       \
-        if (runs) LAUNCH_FORM(GV, true);                                                       \
+        if (runs) LAUNCH_FORM(GV, true, Runs{runs});                                           \
         else LAUNCH_FORM(GV, false);                                                           \
         HIP_CHECK_LAUNCH();                                                                    \
         launch_combine<GV>((hipStream_t)stream, o_part, ml_part, seq_lens, out, B, Hk, nsplit, \
-                           copies);                                                            \
+                           cb, copies ? slots : nullptr, runs);                                \
         HIP_CHECK_LAUNCH();                                                                    \
     } while (0)
 
@@ -1069,16 +1096,17 @@ extern "C" int oa_attention_decode_parts(
     while ((1 << block_shift) < block_size) ++block_shift;
 #define LAUNCH_P(GV)                                                                                              \
     do {                                                                                                          \
-        hipLaunchKernelGGL((decode_attn_kernel<GV, false, true, false, true>), dim3(B * Hk, nsplit), dim3(256), 0, \
+        hipLaunchKernelGGL((decode_attn_kernel<GV, false, true, false>), dim3(B * Hk, nsplit), dim3(256), 0,       \
                            (hipStream_t)stream, (const uint32_t*)nullptr, (const uint32_t*)kc,                    \
                            (const uint32_t*)vc, (const int*)block_table, (const int*)seq_lens, (float*)o_part,    \
                            (float*)ml_part, (unsigned*)nullptr, (uint32_t*)out, B, Hk, max_blocks, block_shift,   \
-                           nsplit, decode_chunk_base(B * Hk), 0, scale, 0, (const uint32_t*)nullptr,              \
+                           nsplit, decode_chunk_base(B * Hk), scale, 0, (const uint32_t*)nullptr,                 \
                            (const uint32_t*)nullptr, (const float*)cos_t, (const float*)sin_t, (const int*)slots, \
                            (uint32_t*)kc, (uint32_t*)vc, 0, 0, 0,                                                 \
-                           Planes{(const float*)part, splits, (int64_t)B * (Hq + 2 * Hk) * DHEAD});               \
+                           (Planes{(const float*)part, splits, (int64_t)B * (Hq + 2 * Hk) * DHEAD}));             \
         HIP_CHECK_LAUNCH();                                                                                       \
-        launch_combine<GV>((hipStream_t)stream, o_part, ml_part, seq_lens, out, B, Hk, nsplit, 0);                \
+        launch_combine<GV>((hipStream_t)stream, o_part, ml_part, seq_lens, out, B, Hk, nsplit,                    \
+                           decode_chunk_base(B * Hk), nullptr, false);                                            \
         HIP_CHECK_LAUNCH();                                                                                       \
     } while (0)
     switch (Hq / Hk) {

@@ -228,17 +228,18 @@ struct MergeRow {
     const float *o, *ml, *sinks;
     int splits, D;
 };
-struct NoMerge {};
 
-template <bool NORM, int EPI, int RT, int GR, int XV, int WV, bool MERGE = false>
+// MORE: MergeRow or nothing, which is no argument (see decode_attn_kernel)
+template <bool NORM, int EPI, int RT, int GR, int XV, int WV, typename... MORE>
 __global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restrict__ x,
                                                     const uint32_t* __restrict__ w,
                                                     uint16_t* __restrict__ out,
                                                     const uint32_t* __restrict__ wn,
                                                     const uint16_t* __restrict__ res, int N, int K,
                                                     int waves, int full, int extra, float eps,
-                                                    int act, DytEpilogue dy,
-                                                    std::conditional_t<MERGE, MergeRow, NoMerge> mr) {
+                                                    int act, DytEpilogue dy, MORE... more) {
+    constexpr bool MERGE = std::is_same_v<void(MORE...), void(MergeRow)>;
+    static_assert(MERGE || sizeof...(MORE) == 0, "a row that is merged, or nothing more");
     extern __shared__ __attribute__((aligned(16))) float xl[];   // [2][K / 2]
     __shared__ float part[8];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -275,6 +276,7 @@ __global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restri
     for (int j = 0; j < XV; ++j) {
         const int i = min(j * WV * 64 + tid, K / 8 - 1);
         if constexpr (MERGE) {
+            const MergeRow mr(more...);
             const int h = i * 8 / mr.D, c = i * 8 - h * mr.D;
 #pragma unroll
             for (int s = 0; s < MS; ++s) {
@@ -332,6 +334,7 @@ __global__ __launch_bounds__(WV * 64) void gemv1_kernel(const uint32_t* __restri
         if (i >= K / 8) continue;
         float f[8];
         if constexpr (MERGE) {
+            const MergeRow mr(more...);
             float mx = -INFINITY, l = 0.0f;
 #pragma unroll
             for (int s = 0; s < MS; ++s)
@@ -463,12 +466,11 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
     const int blocks = CEIL_DIV(CEIL_DIV(N, per), wv);
     const int waves = blocks * wv;
     const size_t lds = (size_t)K * 4;
-#define G1X(NV, RV, RT, GR, XV, WV, ...) G1Y(NV, RV, RT, GR, XV, WV, NoMerge(), ##__VA_ARGS__)
-#define G1Y(NV, RV, RT, GR, XV, WV, MR, ...)                                                              \
-    hipLaunchKernelGGL((gemv1_kernel<NV, RV, RT, GR, XV, WV, ##__VA_ARGS__>), dim3(blocks), dim3(WV * 64), \
-                       lds, st, (const uint32_t*)x, (const uint32_t*)w, (uint16_t*)out,               \
-                       (const uint32_t*)wn, (const uint16_t*)res, N, K, waves, N / waves, N % waves,  \
-                       eps, gateup - 1, dy, MR)
+#define G1X(NV, RV, RT, GR, XV, WV, ...)                                                              \
+    hipLaunchKernelGGL((gemv1_kernel<NV, RV, RT, GR, XV, WV>), dim3(blocks), dim3(WV * 64), lds, st,  \
+                       (const uint32_t*)x, (const uint32_t*)w, (uint16_t*)out, (const uint32_t*)wn,   \
+                       (const uint16_t*)res, N, K, waves, N / waves, N % waves, eps, gateup - 1, dy,  \
+                       ##__VA_ARGS__)
 #define G1(NV, RV, RT, GR)                   \
     do {                                     \
         if (wv == 4) G1X(NV, RV, RT, GR, 2, 4);         \
@@ -476,9 +478,9 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
         else G1X(NV, RV, RT, GR, 4, 8);                 \
     } while (0)
     if (mr.o) {                          // K = 2048 or 4096
-        if (K == 4096) G1Y(false, 2, 1, 8, 2, 4, mr, true);
-        else if (wv == 4) G1Y(false, 2, 1, 4, 2, 4, mr, true);
-        else G1Y(false, 2, 1, 4, 1, 8, mr, true);
+        if (K == 4096) G1X(false, 2, 1, 8, 2, 4, mr);
+        else if (wv == 4) G1X(false, 2, 1, 4, 2, 4, mr);
+        else G1X(false, 2, 1, 4, 1, 8, mr);
     } else if (gateup) {
         if (mode & 1) G1(true, 0, 2, 4);
         else G1(false, 0, 2, 4);
@@ -503,7 +505,6 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
     }
 #undef G1
 #undef G1X
-#undef G1Y
     HIP_CHECK_LAUNCH();
     return 0;
 }

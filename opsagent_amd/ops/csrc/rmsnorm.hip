@@ -13,16 +13,17 @@
 // norm in a step of 8 rows of 4096: 7.7 + 4.4, of 16 of 2048 10.8 + 4.8; a step of 13
 // tokens through experts 590 -> 580, of 8 sequences 505 -> 502, of 47 885 -> 866). An id
 // outside the table, which the engine refuses before, gets a row of NaN.
-// QUANT: out is the normed row as quant_fp8 (fp8_moe.hip) would leave it, of the same bf16 values: 8-bit
+// SCALES (float): out is the normed row as quant_fp8 (fp8_moe.hip) would leave it, of the same bf16 values: 8-bit
 // numbers [rows, D] and a scale a row. One launch, 8 KB a row of 4096 out and in again less: us of a
 // layer's norm and quantization in a run of products, 700 rows of 4096 11.3 -> 6.6, 20 rows 9.3 -> 4.9.
 enum { RN_PLAIN, RN_ADD, RN_EMBED };
-template <int MODE, typename ID, bool QUANT = false>
+template <int MODE, typename ID, typename... SCALES>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(
     const uint4* __restrict__ x,      // [rows, D / 8] packed bf16
     uint4* __restrict__ residual,     // [rows, D / 8] in/out (ADD), out (EMBED)
     const uint4* __restrict__ w, uint4* __restrict__ out, const ID* __restrict__ ids, int64_t vocab,
-    int D8, float inv_d, float eps, float* __restrict__ scales) {
+    int D8, float inv_d, float eps, SCALES*... scales) {
+    constexpr bool QUANT = sizeof...(SCALES) > 0;
     __shared__ float red[16];
     const int64_t row = blockIdx.x;
     int64_t from = row;
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
     __syncthreads();
     amax = fmaxf(fmaxf(most[0], most[1]), fmaxf(most[2], most[3]));
     const float inv = 448.0f / amax;                 // the largest e4m3 number
-    if (threadIdx.x == 0) scales[row] = amax / 448.0f;
+    if (threadIdx.x == 0) ((scales[row] = amax / 448.0f), ...);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const int c = k * 256 + threadIdx.x;
@@ -106,7 +107,7 @@ static int launch_rmsnorm(void* stream, const void* x, void* residual, const voi
     if (dim % 8 != 0 || dim > 8192) return -100;
     hipLaunchKernelGGL((rmsnorm_kernel<MODE, ID>), dim3(rows), dim3(256), 0, (hipStream_t)stream,
                        (const uint4*)x, (uint4*)residual, (const uint4*)w, (uint4*)out,
-                       (const ID*)ids, vocab, dim / 8, 1.0f / dim, eps, (float*)nullptr);
+                       (const ID*)ids, vocab, dim / 8, 1.0f / dim, eps);
     HIP_CHECK_LAUNCH();
     return 0;
 }
@@ -127,7 +128,7 @@ extern "C" int oa_fused_add_rmsnorm_fp8(void* stream, const void* x, void* resid
                                         void* scales, int rows, int dim, float eps) {
     if (rows < 1 || dim % 8 != 0 || dim > 8192) return -100;
     if (((uintptr_t)x | (uintptr_t)residual | (uintptr_t)w) % 16 != 0 || (uintptr_t)q % 8 != 0) return -101;
-    hipLaunchKernelGGL((rmsnorm_kernel<RN_ADD, int64_t, true>), dim3(rows), dim3(256), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL((rmsnorm_kernel<RN_ADD, int64_t, float>), dim3(rows), dim3(256), 0, (hipStream_t)stream,
                        (const uint4*)x, (uint4*)residual, (const uint4*)w, (uint4*)q, (const int64_t*)nullptr,
                        (int64_t)0, dim / 8, 1.0f / dim, eps, (float*)scales);
     HIP_CHECK_LAUNCH();

@@ -6,10 +6,15 @@
 
 #include "common.h"
 
-// PARTS: the projection is still its `splits` float32 planes [T, (Hq + 2 Hk) * D], added up here and rounded
-// as the product alone would be; q, k and v are then only written. us, the launch for the sum and this one
+// With RopePlanes the projection is still its `splits` float32 planes [T, (Hq + 2 Hk) * D], added up here and
+// rounded as the product alone would be; q, k and v are then only written. us, the launch for the sum and this one
 // / here: 77 rows of 6144, five planes 7.4 / 4.1.
-template <bool PARTS>
+struct RopePlanes {
+    const float* sums;
+    int splits;
+};
+
+template <typename... PLANES>
 __global__ __launch_bounds__(256) void rope_kv_kernel(
     uint32_t* __restrict__ q,        // [T, Hq, D/2] words
     uint32_t* __restrict__ k,        // [T, Hk, D/2]
@@ -21,9 +26,13 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(
     const int* __restrict__ slots,      // [T]
     int T, int Hq, int Hk, int d2 /* D/2 */,
     int qts2, int kts2, int vts2 /* per-tensor token strides in words */,
-    const float* __restrict__ part, int splits) {
+    PLANES... planes) {
+    constexpr bool PARTS = sizeof...(PLANES) > 0;
     const int width = (Hq + 2 * Hk) * d2 * 2;
     auto sum4 = [&](int64_t at) {
+        const RopePlanes p{planes...};
+        const float* const part = p.sums;
+        const int splits = p.splits;
         float4 a = *reinterpret_cast<const float4*>(part + at);
 #pragma unroll 4
         for (int s = 1; s < splits; ++s) {
@@ -111,13 +120,13 @@ static int rope_kv(hipStream_t stream, void* q, void* k, void* v, void* k_cache,
     const int d2 = D / 2;
     const int64_t total = (int64_t)T * (Hq + 2 * Hk) * (d2 / 4);
     const int grid = (int)min((int64_t)2048, CEIL_DIV(total, 256));
-#define RK(P)                                                                                       \
-    hipLaunchKernelGGL((rope_kv_kernel<P>), dim3(grid), dim3(256), 0, stream, (uint32_t*)q, (uint32_t*)k, \
+#define RK(...)                                                                                     \
+    hipLaunchKernelGGL(rope_kv_kernel, dim3(grid), dim3(256), 0, stream, (uint32_t*)q, (uint32_t*)k, \
                        (uint32_t*)v, (uint32_t*)k_cache, (uint32_t*)v_cache, (const float*)cos_t,   \
                        (const float*)sin_t, (const int*)positions, (const int*)slots, T, Hq, Hk, d2, \
-                       q_stride / 2, k_stride / 2, v_stride / 2, (const float*)part, splits)
-    if (part) RK(true);
-    else RK(false);
+                       q_stride / 2, k_stride / 2, v_stride / 2, ##__VA_ARGS__)
+    if (part) RK((RopePlanes{(const float*)part, splits}));
+    else RK();
 #undef RK
     HIP_CHECK_LAUNCH();
     return 0;

@@ -154,6 +154,38 @@ def test_combine_of_many_splits(lens, nsplit, Hk):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("lens,nsplit", [([1], 32), ([331], 32), ([64, 700, 129], 8)])
+@pytest.mark.parametrize("G", [1, 4])
+def test_plain_splits_leave_no_marks(lens, nsplit, G):
+    """Up to 64 (sequence, key head) pairs the combine counts the splits: a launch writes the places
+    that it has and no others, and what stood in those is not looked at."""
+    Hk, bs, B = 4, 32, len(lens)
+    q, k, v, kc, vc, table, lens_t, slots = _case(lens, Hk, G, bs, seed=sum(lens))
+    cos, sin = (t.cuda() for t in ops.rope_cos_sin(1024, D))
+    planes = torch.stack([torch.cat([t.reshape(B, -1) for t in (q, k, v)], -1).float()] * 2)
+    planes[1] = 0.0
+    chunk = 64 if B * Hk <= 8 else 128               # keys of a split at these sizes
+
+    def check(call):
+        got = []
+        for mark in (7.0, -2.0):
+            ws = (torch.full((B * Hk * nsplit, G, D), mark, device="cuda"),
+                  torch.full((B * Hk * nsplit, G, 2), mark, device="cuda"))
+            got.append(call(kc.clone(), vc.clone(), ws))
+            for b, n in enumerate(lens):
+                used = -(-n // max(chunk, -(-n // nsplit)))
+                rest = [w.view(B, Hk, nsplit, -1)[b, :, used:] for w in ws]
+                assert all((r == mark).all() for r in rest), (b, used)
+        assert torch.equal(*got)
+
+    check(lambda kc, vc, ws: ops.attention_decode_rope(q, k, v, kc, vc, table, lens_t, cos, sin, slots,
+                                                       workspace=ws, nsplit=nsplit))
+    check(lambda kc, vc, ws: ops.attention_decode_parts(
+        ops.PlaneSum(planes), Hk * G, Hk, D, kc, vc, table, lens_t, cos, sin, slots, D ** -0.5,
+        workspace=ws, nsplit=nsplit))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("G,Hk,lens", [(4, 8, [700, 65, 130]), (8, 4, [513, 64]), (1, 33, [1, 90])])
 def test_copies_of_the_first_row(G, Hk, lens):
     """Rows that repeat the first are answered by its results; rows that write its slot but differ
