@@ -140,6 +140,7 @@ __device__ __forceinline__ int in_tiles(int keys) { return (keys + 63) >> 6; }
 // share most of their pages lose what splits in step got from the die's L2: 32 of up to 3000
 // with 2000 in common 39.2 -> 42.1 (47 with 1000 71.5 -> 61.5).
 struct DecodeRuns {
+    bool units;
     int size, per, total;
     int b, n;               // row (-1: none) and keys of it
     int before;             // tiles of the rows before it; units: `which` less the unit within the row
@@ -176,6 +177,7 @@ __device__ __forceinline__ DecodeRuns decode_runs(const int* seq_lens, const int
     const int over = units ? 0 : 1;
     while (const uint64_t more = __ballot(most - over > cut * (nsplit - over)))
         cut = CEIL_DIV(__builtin_amdgcn_readlane(most, __builtin_ctzll(more)) - over, nsplit - over);
+    r.units = units;
     r.size = units ? cut : 1;
     r.per = units ? 1 : cut;
     r.b = -1;
@@ -271,7 +273,6 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
     // the (row, key head) in work and its keys; RUNS: tiles of the row, the first of them that
     // the block takes, and how many it still has to take
     int b, h, split, n, kstart, kend, own = 0, from = 0, left = 0;
-    bool once = false;                               // value rows are read without being kept
     if constexpr (RUNS) {
         const int at = blockIdx.y, whole = gridDim.y - copies * (B - 1);
         h = blockIdx.x;
@@ -282,15 +283,14 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
             b = r.b;
             n = r.n;
             own = in_tiles(n);
-            once = r.per > 1;
-            if (once) {
-                from = at * r.per - r.before;
-                left = min(r.per, r.total - at * r.per);
-                split = __builtin_amdgcn_readfirstlane(at - r.before / r.per);
-            } else {
+            if (r.units) {
                 split = at - r.before;
                 from = split * r.size;
                 left = min(r.size, own - from);
+            } else {
+                from = at * r.per - r.before;
+                left = min(r.per, r.total - at * r.per);
+                split = __builtin_amdgcn_readfirstlane(at - r.before / r.per);
             }
         } else {                                     // a row that may be a copy, by itself if it is none
             b = 1 + at - whole;
