@@ -1078,10 +1078,11 @@ extern "C" int oa_attention_decode_rope(
     return 0;
 }
 
-// Whether a launch of as many (sequence, key head) pairs takes the projection's planes: one without runs
+// Whether a launch of as many (sequence, key head) pairs takes the projection's planes: up to 64 of them,
+// where there are neither runs nor copies of the first row
 extern "C" int oa_attention_decode_takes_parts(int B, int Hq, int Hk, int D) {
     const int G = Hk > 0 && Hq % Hk == 0 ? Hq / Hk : 0;
-    return D == DHEAD && (G == 1 || G == 2 || G == 4 || G == 8) && decode_run_count(B, Hk, 2) == 0;
+    return D == DHEAD && (G == 1 || G == 2 || G == 4 || G == 8) && (int64_t)B * Hk <= 64;
 }
 
 // oa_attention_decode_rope of a projection that is still its planes part [splits, B, (Hq + 2 Hk) * D]

@@ -48,6 +48,13 @@ def test_decode_attention(B, Hq, Hk, block, parts):
     assert all(torch.equal(a, b) for a, b in zip(caches, other))
 
 
+@pytest.mark.parametrize("B,Hk,takes", [(1, 8, True), (8, 8, True), (64, 1, True), (9, 8, False), (65, 1, False),
+                                        (4096, 8, False), (4097, 8, False), (5000, 1, False)])
+def test_steps_that_add_up_parts(B, Hk, takes):
+    assert ops.decode_takes_parts(B, 4 * Hk, Hk, HEAD) == takes
+    assert not ops.decode_takes_parts(B, 4 * Hk, Hk, 64) and not ops.decode_takes_parts(B, 3 * Hk, Hk, HEAD)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,Hq,Hk,D,parts", [(1, 1, 1, 16, 1), (3, 4, 2, 64, 2), (77, 32, 8, 128, 5), (128, 16, 4, 128, 16)])
 def test_rotation(T, Hq, Hk, D, parts):
