@@ -14,7 +14,7 @@
 //   o_part   [B*Hk*NSPLIT, G, 128] f32, ml_part [B*Hk*NSPLIT, G, 2] f32
 //   out      [B, Hq, 128] bf16
 //
-// Small launches: a split is `chunk` keys, a multiple of 64 (decode_chunk), and blocks past a
+// Launches of under 512 (sequence, key head) pairs: a split is `chunk` keys, a multiple of 64 (decode_chunk), and blocks past a
 // sequence's last key end at once. Larger ones: the tiles of 64 keys of all sequences are cut in
 // equal runs, one a CU (DecodeRuns). Either way at most nsplit splits cover a sequence, and the
 // combine reads those that exist: plain splits it counts, behind a sequence's last run stands a mark.
@@ -935,11 +935,13 @@ static int decode_chunk_base(int pairs) {
     return pairs <= 8 ? 64 : pairs <= 32 ? 128 : pairs <= 128 ? 256 : 512;
 }
 
-// Runs of a key head, 0 for splits of each sequence: up to 64 (sequence, key head) pairs what a launch
-// works out first is more than runs gain (us, splits / runs: 12 of up to 900 tokens, 4 key heads 12.5 /
-// 13.3, 8 of 1500, 8 key heads 17.0 / 18.3; but 8 of 6000 37.6 / 34.5, which the host cannot know).
+// Runs of a key head, 0 for splits of each sequence: under 512 (sequence, key head) pairs the host, which does
+// not know the lengths, cannot tell where runs gain from where they and what a launch works out first cost
+// more (both launches, us, splits / runs, 8 key heads, caches that no cache holds: 32 of up to 3000 tokens 66 /
+// 57, 24 of 1500 in 32 35 / 32, but 32 of 700 21.8 / 26.6, 32 of 1000 28.4 / 30.5, 16 of 1000 18.8 / 20.4, 12 of 500
+// 12.8 / 13.6).
 static int decode_run_count(int B, int Hk, int nsplit) {
-    return B * Hk <= 64 || B > 4096 || nsplit < 2 ? 0 : max(1, 256 / Hk);
+    return B * Hk < 512 || B > 4096 || nsplit < 2 ? 0 : max(1, 256 / Hk);
 }
 
 // Blocks of a key head: its runs, or the units that fewer than 8 * (runs + B) tiles make

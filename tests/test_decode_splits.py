@@ -154,17 +154,18 @@ def test_combine_of_many_splits(lens, nsplit, Hk):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("lens,nsplit", [([1], 32), ([331], 32), ([64, 700, 129], 8)])
+@pytest.mark.parametrize("lens,nsplit,Hk", [([1], 32, 4), ([331], 32, 4), ([64, 700, 129], 8, 4), ([700, 20, 513] * 8, 4, 4),
+                                            ([700, 1000, 30, 512] * 8, 32, 8), ([65, 600, 900] * 21, 32, 8)])
 @pytest.mark.parametrize("G", [1, 4])
-def test_plain_splits_leave_no_marks(lens, nsplit, G):
-    """Up to 64 (sequence, key head) pairs the combine counts the splits: a launch writes the places
-    that it has and no others, and what stood in those is not looked at."""
-    Hk, bs, B = 4, 32, len(lens)
+def test_plain_splits_leave_no_marks(lens, nsplit, Hk, G):
+    """Under 512 (sequence, key head) pairs sequences are split one by one and the combine counts the
+    splits: a launch writes the places that it has and no others, and what stood in those is not
+    looked at."""
+    bs, B = 32, len(lens)
     q, k, v, kc, vc, table, lens_t, slots = _case(lens, Hk, G, bs, seed=sum(lens))
     cos, sin = (t.cuda() for t in ops.rope_cos_sin(1024, D))
-    planes = torch.stack([torch.cat([t.reshape(B, -1) for t in (q, k, v)], -1).float()] * 2)
-    planes[1] = 0.0
-    chunk = 64 if B * Hk <= 8 else 128               # keys of a split at these sizes
+    pairs = B * Hk                                   # keys of a split at these sizes: by the pairs
+    least = 64 if pairs <= 8 else 128 if pairs <= 32 else 256 if pairs <= 128 else 512
 
     def check(call):
         got = []
@@ -173,20 +174,23 @@ def test_plain_splits_leave_no_marks(lens, nsplit, G):
                   torch.full((B * Hk * nsplit, G, 2), mark, device="cuda"))
             got.append(call(kc.clone(), vc.clone(), ws))
             for b, n in enumerate(lens):
-                used = -(-n // max(chunk, -(-n // nsplit)))
+                used = -(-n // max(least, -(-n // nsplit // 64) * 64))
                 rest = [w.view(B, Hk, nsplit, -1)[b, :, used:] for w in ws]
                 assert all((r == mark).all() for r in rest), (b, used)
         assert torch.equal(*got)
 
     check(lambda kc, vc, ws: ops.attention_decode_rope(q, k, v, kc, vc, table, lens_t, cos, sin, slots,
                                                        workspace=ws, nsplit=nsplit))
-    check(lambda kc, vc, ws: ops.attention_decode_parts(
-        ops.PlaneSum(planes), Hk * G, Hk, D, kc, vc, table, lens_t, cos, sin, slots, D ** -0.5,
-        workspace=ws, nsplit=nsplit))
+    if ops.decode_takes_parts(B, Hk * G, Hk, D):
+        planes = torch.stack([torch.cat([t.reshape(B, -1) for t in (q, k, v)], -1).float()] * 2)
+        planes[1] = 0.0
+        check(lambda kc, vc, ws: ops.attention_decode_parts(
+            ops.PlaneSum(planes), Hk * G, Hk, D, kc, vc, table, lens_t, cos, sin, slots, D ** -0.5,
+            workspace=ws, nsplit=nsplit))
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("G,Hk,lens", [(4, 8, [700, 65, 130]), (8, 4, [513, 64]), (1, 33, [1, 90])])
+@pytest.mark.parametrize("G,Hk,lens", [(4, 8, [700, 65, 130]), (8, 4, [513, 64]), (1, 33, [1, 90]), (4, 25, [700, 65, 130])])
 def test_copies_of_the_first_row(G, Hk, lens):
     """Rows that repeat the first are answered by its results; rows that write its slot but differ
     in a query or an earlier page are answered by themselves."""
@@ -220,7 +224,7 @@ def test_copies_of_the_first_row(G, Hk, lens):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("G,Hk", [(4, 8), (8, 4), (1, 33)])
+@pytest.mark.parametrize("G,Hk", [(4, 8), (8, 4), (1, 33), (4, 25)])
 def test_rows_that_are_nearly_copies(G, Hk):
     """Rows with the first row's slot that differ from it in one thing alone (a query, the new key
     or value of one key head, the length, the last page) are answered by themselves. The marks in
@@ -271,9 +275,16 @@ def test_rows_that_are_nearly_copies(G, Hk):
     ([1 + 9 * i for i in range(66)], 2, 32, 32),     # short rows: units, more rows than lanes
     ([5000] + [5, 64, 65, 513, 1100] * 13, 4, 64, 3),         # units larger for one long row
     ([200] * 3 + [4000], 100, 32, 32),               # more key heads than runs for them
+    ([3000, 1, 63, 64, 65, 2111, 128, 129, 1500, 16, 17, 900, 2500, 700, 31, 1023, 1024, 1025, 2048,
+      5, 640], 25, 32, 32),                          # 512 pairs and more: the rows of before
+    ([2000 - 27 * i for i in range(70)], 8, 16, 32),
+    ([4000] + [900 + 7 * i for i in range(16)], 33, 8, 2),
+    ([1 + 9 * i for i in range(66)], 8, 32, 32),
+    ([3000] + [5, 64, 65, 513, 1100] * 13, 8, 64, 3),
+    ([200] * 3 + [4000], 130, 32, 32),
 ])
 def test_runs_over_sequences(G, lens, Hk, bs, nsplit):
-    """More than 64 (sequence, key head) pairs: blocks go over the tiles of all sequences."""
+    """512 (sequence, key head) pairs and more: blocks go over the tiles of all sequences."""
     q, k, v, kc, vc, table, lens_t, slots = _case(lens, Hk, G, bs, seed=len(lens) + G)
     cos, sin = (t.cuda() for t in ops.rope_cos_sin(8192, D))
     flat_k, flat_v = kc.view(-1, Hk, D), vc.view(-1, Hk, D)
