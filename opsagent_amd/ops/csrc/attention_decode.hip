@@ -130,20 +130,23 @@ __device__ __forceinline__ int in_tiles(int keys) { return (keys + 63) >> 6; }
 //
 // Each row that a run begins costs it a prologue and a merge. Where rows are short, a run is one
 // unit of `size` tiles of a row instead (chunk_base keys, or as many as nsplit asks for; `per` is 1),
-// the rows' first units before what is left. The line: tiles for each of runs and rows, 3.5, or 8
-// where rows are more than the runs by a quarter. Both launches, us, splits of each sequence / runs
-// / units, 4 heads a key head: 47 of up to 3000 tokens in a step of 64, 8 key heads 88.4 / 74.5, 64 of 2500 94.4 /
-// 82.2, 20 of 8000 in 32 102 / 79, 47 of 3000 on 4 52.8 / 43.7, 32 of 3000 62.8 / 55.6, 33 of 1500 42.2 / 37.7,
-// 33 of 800 29.9 / 28.5 / 31, 24 of 1000 25.4 / 25.9, 64 of 1200 52.8 / 51.8, 64 of 700 35.8 / 38 / 34.5, 64 of 300
-// 22.5 / 26 / 20.6; 8 heads a key head, 64 of 500 on 4 21.1 / 30 / 21.0. Runs for 384 or 768 blocks
-// are slower (89, 89), for 512 level (79.5), and so are two tiles ahead (79). Rows that
-// share most of their pages lose what splits in step got from the die's L2: 32 of up to 3000
-// with 2000 in common 39.2 -> 42.1 (47 with 1000 71.5 -> 61.5).
+// in step: the rows' first units, then what is left of them. The line: tiles for each of runs and rows, 3.5, or 8
+// where rows are more than the runs by a quarter. Both launches, us, caches that no cache holds, splits of each
+// sequence / here, steps of 64, 4 heads a key head on 8: 47 of up to 3000 tokens 91.5 / 77.9, 33 of 1500 43.2 /
+// 39.6, 64 of 3000 113 / 100; units: 64 of 300 22.7 / 21.1, of 700 36.8 / 35.7, 47 of 700 31.5 / 30.4, of 1000 39.4 / 39.4.
+// What a launch works out first shows where neither gains: 40 of 700 30.2 / 31.0, 47 of 500 25.8 / 26.1, and in
+// steps of 32 on 16 key heads 24 of 1000 with 256 in common 32.6 / 34.9. Runs for 384 or 768 blocks are slower (47
+// of 3000 89, 89; 74.5 for 256), for 512 level (79.5), and so are two tiles ahead (79).
+//
+// Rows that share most of their pages (a prompt's common beginning) are read from the die's L2 by blocks that
+// go in step, and runs would not: units, then, where the page at the mean length is the same. Splits of each
+// sequence / runs / units, us: 64 of up to 1500 with 1024 in common 41.0 / 46.0 / 42.8, of 2200 with 2016 50.1 / 55.7 /
+// 51.1, 56 of 1500 with 1024 39.6 / 42.6 / 39.5. With less in common runs stay ahead: 47 of 3000 with 256 83.3 / 72.1.
 struct DecodeRuns {
     bool units;
     int size, per, total;
     int b, n;               // row (-1: none) and keys of it
-    int before;             // tiles of the rows before it; units: `which` less the unit within the row
+    int before;             // tiles of the rows before it; units: `which` less the unit's number in its row
 };
 
 __device__ __forceinline__ int in_units(int t, int size) {
@@ -152,8 +155,9 @@ __device__ __forceinline__ int in_units(int t, int size) {
 
 // The row that run `which` begins with. Every wave works it out for itself, a lane per sequence,
 // 64 sequences at a time.
-__device__ __forceinline__ DecodeRuns decode_runs(const int* seq_lens, const int* slots, int B, int copies,
-                                                  int runs, int nsplit, int chunk_base, int which) {
+__device__ __forceinline__ DecodeRuns decode_runs(const int* seq_lens, const int* slots, const int* block_table,
+                                                  int max_blocks, int block_shift, int B, int copies, int runs,
+                                                  int nsplit, int chunk_base, int which, int whole) {
     const int lane = threadIdx.x & (WAVE - 1);
     auto keys = [&](int b) {
         const int n = run_keys(seq_lens, slots, min(b, B - 1), copies);
@@ -172,8 +176,19 @@ __device__ __forceinline__ DecodeRuns decode_runs(const int* seq_lens, const int
     }
     most = in_tiles(most);
     // (divisions only where they are needed: every launch waits for this)
-    const bool units = 2 * r.total < (4 * rows > 5 * runs ? 16 : 7) * (runs + rows);
-    int cut = units ? chunk_base / 64 : __builtin_amdgcn_readfirstlane(CEIL_DIV(r.total, runs));
+    bool units = 2 * r.total < (4 * rows > 5 * runs ? 16 : 7) * (runs + rows);
+    int cut = chunk_base / 64;
+    if (!units) {
+        // the page at the mean length: do half and more of the rows that are longer (of 64) have the same one?
+        const int depth = (int)((float)(r.total * 64) * __builtin_amdgcn_rcpf((float)rows));
+        const int page = block_table[(size_t)min(lane, B - 1) * max_blocks + min(depth >> block_shift, max_blocks - 1)];
+        const uint64_t longer = __ballot(n0 > depth);
+        const int first = __builtin_amdgcn_readlane(page, longer ? __builtin_ctzll(longer) : 0);
+        const int same = __builtin_popcountll(longer & __ballot(page == first));
+        units = same > 1 && 2 * same >= __builtin_popcountll(longer);
+        const int fit = __builtin_amdgcn_readfirstlane(CEIL_DIV(r.total, units ? whole - B : runs));
+        cut = units ? max(cut, fit) : fit;
+    }
     const int over = units ? 0 : 1;
     while (const uint64_t more = __ballot(most - over > cut * (nsplit - over)))
         cut = CEIL_DIV(__builtin_amdgcn_readlane(most, __builtin_ctzll(more)) - over, nsplit - over);
@@ -181,31 +196,34 @@ __device__ __forceinline__ DecodeRuns decode_runs(const int* seq_lens, const int
     r.size = units ? cut : 1;
     r.per = units ? 1 : cut;
     r.b = -1;
-    // units: the first ones of all rows, then what is left of them
-    const int at = units ? which - B : which * r.per;
+    // units in step: the first ones of all rows, then, 64 rows at a time, the second ones and so on.
+    // (Rows without keys have no place among them: blocks go to the CUs in turn, and such places would
+    // leave some of them with less: 47 rows of up to 700 tokens in a step of 64 32.6 -> 30.3 us.)
+    const bool firsts = units && which < rows;
+    const int at = units ? which - (firsts ? 0 : rows) : which * r.per;
     int before = 0;
 #pragma unroll 1
     for (int b0 = 0; b0 < B; b0 += WAVE) {
         const int n = b0 ? keys(b0 + lane) : n0, t = in_tiles(n);
-        uint64_t past;
-        int u = t, sums = 0;
-        if (units && at < 0) {
-            past = which < b0 + WAVE ? 1ull << (which - b0) : 0;
-        } else {
-            if (units) u = max(in_units(t, r.size) - 1, 0);
-            sums = before + wave_sums(u);
-            past = __ballot(sums > at);
-            before = __builtin_amdgcn_readlane(sums, 63);
-        }
-        if (past) {
-            const int row = __builtin_ctzll(past);
+        const int u = !units ? t : firsts ? min(t, 1) : max(in_units(t, r.size) - 1, 0);
+        uint64_t some = __ballot(u > 0);
+        const int sums = before + (firsts ? 0 : wave_sums(u));
+        const int end = firsts ? before + __builtin_popcountll(some) : __builtin_amdgcn_readlane(sums, 63);
+        if (end > at) {
+            int unit = firsts ? 0 : 1, place = at - before;
+            while (units && place >= __builtin_popcountll(some)) {
+                place -= __builtin_popcountll(some);
+                some = __ballot(u > unit++);
+            }
+            const uint64_t found = __ballot(units ? (some >> lane & 1) && __builtin_popcountll(some & ((1ull << lane) - 1)) == place
+                                                  : sums > at);
+            const int row = __builtin_ctzll(found);
             r.n = __builtin_amdgcn_readlane(n, row);
-            if (r.n == 0) break;
             r.b = b0 + row;
-            r.before = __builtin_amdgcn_readlane(sums, row) - __builtin_amdgcn_readlane(u, row);
-            if (units) r.before = at < 0 ? which : r.before + B - 1;
+            r.before = units ? which - unit : __builtin_amdgcn_readlane(sums, row) - __builtin_amdgcn_readlane(u, row);
             break;
         }
+        before = end;
     }
     return r;
 }
@@ -278,7 +296,8 @@ __global__ __launch_bounds__(256, RUNS && G <= 4 ? 3 : 1) void decode_attn_kerne
         h = blockIdx.x;
         split = 0;
         if (at < whole) {
-            const DecodeRuns r = decode_runs(seq_lens, slots, B, copies, more.count..., nsplit, chunk_base, at);
+            const DecodeRuns r = decode_runs(seq_lens, slots, block_table, max_blocks, block_shift, B, copies,
+                                             more.count..., nsplit, chunk_base, at, whole);
             if (r.b < 0) return;
             b = r.b;
             n = r.n;
@@ -944,9 +963,10 @@ static int decode_run_count(int B, int Hk, int nsplit) {
     return B * Hk < 512 || B > 4096 || nsplit < 2 ? 0 : max(1, 256 / Hk);
 }
 
-// Blocks of a key head: its runs, or the units that fewer than 8 * (runs + B) tiles make
+// Blocks of a key head: its runs, or the units that fewer than 8 * (runs + B) tiles make; rows that share
+// pages take units that fit in
 static int decode_run_blocks(int runs, int cb, int B) {
-    return max(runs, 8 * (runs + B) * 64 / cb + B);
+    return max(max(runs, 4 * B), 8 * (runs + B) * 64 / cb + B);
 }
 
 // Early loads pay while the launch is a few blocks (both launches, us: one sequence of 1151

@@ -312,3 +312,38 @@ def test_runs_over_sequences(G, lens, Hk, bs, nsplit):
             assert not got[b].any()
         else:
             assert float((got[b].double() - w).norm() / w.norm()) < 2.0 ** -9 + 1e-4, (b, lens[b])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Hk,G,longest,common", [(64, 8, 4, 1500, 1024), (56, 16, 1, 1500, 1024), (100, 6, 2, 900, 640),
+                                                   (64, 8, 4, 1500, 96), (16, 32, 1, 2500, 2016)])
+def test_runs_over_shared_pages(B, Hk, G, longest, common):
+    """Rows that share the page at their mean length are split in units that go in step, others in runs:
+    the marks in the workspace say how many places a row has."""
+    bs, nsplit = 32, 32
+    lens = [max(1, round(longest * (1 - 0.75 * ((0.618034 * b) % 1.0)))) for b in range(B)]
+    q, k, v, kc, vc, table, lens_t, slots = _case(lens, Hk, G, bs, seed=B + Hk)
+    cos, sin = (t.cuda() for t in ops.rope_cos_sin(4096, D))
+    for b, n in enumerate(lens):
+        own = (n - 1) // bs                          # the page that the new key goes to
+        table[b, : min(common // bs, own)] = table[0, : min(common // bs, own)]
+    ws = (torch.full((B * Hk * nsplit, G, D), 7.0, device="cuda"),
+          torch.full((B * Hk * nsplit, G, 2), 7.0, device="cuda"))
+    got = ops.attention_decode_rope(q, k, v, kc.clone(), vc.clone(), table, lens_t, cos, sin, slots, workspace=ws,
+                                    nsplit=nsplit)
+    flat_k, flat_v = kc.view(-1, Hk, D), vc.view(-1, Hk, D)
+    for b, n in enumerate(lens):
+        at = torch.arange(n, device="cuda")
+        r = table[b, at // bs].long() * bs + at % bs
+        ks, vs = flat_k[r].double(), flat_v[r].double()
+        new = _rotate(k[b].double(), n - 1, cos, sin)
+        ks, vs = torch.cat([ks[:-1], new[None]]), torch.cat([vs[:-1], v[b].double()[None]])
+        want = _attend(_rotate(q[b].double(), n - 1, cos, sin), ks, vs, G)
+        # as above: one bf16 rounding of every row
+        assert float((got[b].double() - want).norm() / want.norm()) < 2.0 ** -9 + 1e-4, (b, n)
+    tiles = [(n + 63) // 64 for n in lens]
+    size = max(8, -(-sum(tiles) // (3 * B)))         # 512 keys, or what the launch's blocks ask for
+    units = [-(-n // size) for n in tiles]
+    sums = ws[1].view(B, Hk, nsplit, G, 2)[..., 1]
+    marked = [bool((sums[b, :, u] == -2.0).all()) and not bool((sums[b, :, :u] == -2.0).any()) for b, u in enumerate(units)]
+    assert all(marked) == (common > sum(tiles) * 64 / B)
