@@ -223,7 +223,11 @@ struct DytEpilogue {
 // merges as attn_combine_kernel would: that is a launch of 4.6 us before this one, and every block reads
 // all splits, 48 KB of 16 heads of 128, from the L2 while its weights are under way. us, the three launches
 // of attention and output product / these two, traced one by one, one row, window 512, 16 heads in 4, 2048 x
-// 2048: 16.4 / 13.5; a step of four layers 10 us less.
+// 2048: 16.4 / 13.5; a step of four layers 10 us less. Up to 4096 columns: wider rows have more splits to read than
+// the launch takes. Attention and product, us, windows of 512 and contexts of 1400: 16 heads of 128, 2048 x 2048
+// 15.1 / 12.9 and 15.7 / 14.6; 32 of 64 13.7 / 11.7 and 15.0 / 12.9; 32 of 128, 4096 x 4096 19.4 / 19.1 and 21.8 / 21.2;
+// but 48 of 128, 4096 x 6144 22.6 / 23.9 and 24.5 / 25.7 (6144 x 6144 26.4 / 25.2), 64 of 128, 8192 x 8192 38.0 / 38.4 and
+// 39.2 / 40.7.
 struct MergeRow {
     const float *o, *ml, *sinks;
     int splits, D;
@@ -477,7 +481,7 @@ static int gemv1(hipStream_t st, const void* x, const void* w, void* out, const 
         else if (K <= 4096) G1X(NV, RV, RT, GR, 1, 8);  \
         else G1X(NV, RV, RT, GR, 4, 8);                 \
     } while (0)
-    if (mr.o) {                          // K = 2048 or 4096
+    if (mr.o) {                          // K up to 4096
         if (K == 4096) G1X(false, 2, 1, 8, 2, 4, mr);
         else if (wv == 4) G1X(false, 2, 1, 4, 2, 4, mr);
         else G1X(false, 2, 1, 4, 1, 8, mr);
@@ -594,11 +598,11 @@ extern "C" int oa_gemv_float(void* stream, const void* x, const void* w, void* o
     return gemv1((hipStream_t)stream, x, w, out, nullptr, nullptr, N, K, 0.0f, 5, 0);
 }
 
-// oa_gemv_dyt of a row that is still its key splits (MergeRow): K = 2048 or 4096, heads of 64 or 128
+// oa_gemv_dyt of a row that is still its key splits (MergeRow): K up to 4096, heads of 64 or 128
 extern "C" int oa_gemv_dyt_merge(void* stream, const void* o, const void* ml, const void* sinks, int splits, int D,
                                  const void* w, void* residual, const void* pw, const void* pb, const void* pa,
                                  const void* nw, const void* nb, const void* na, void* out, int N, int K) {
-    if (N < 1 || (K != 2048 && K != 4096) || N > 256 * 64 * 8) return -100;
+    if (N < 1 || K < 2048 || K % 2048 != 0 || K > 4096 || N > 256 * 64 * 8) return -100;
     if (splits < 2 || splits > 6 || (D != 64 && D != 128)) return -103;
     if (!o || !ml || !w || !residual || !pw || !pb || !pa || (out && (!nw || !nb || !na))) return -101;
     if (((uintptr_t)o | (uintptr_t)w) % 16 != 0 || (uintptr_t)ml % 8 != 0) return -102;

@@ -529,10 +529,11 @@ class SplitRow(NamedTuple):
 
 
 def merges_split_row(w: torch.Tensor, residual: torch.Tensor, out_dtype) -> bool:
-    """Whether linear_dyt_norm takes a SplitRow against w."""
+    """Whether linear_dyt_norm takes a SplitRow against w: rows that the one-row product takes, of up to
+    4096 columns (wider ones gain nothing by it: figures in gemv.hip)."""
     from opsagent_amd import ops
 
-    return (w.is_cuda and w.dim() == 2 and w.shape[1] in (2048, 4096) and w.shape[0] <= 131072
+    return (w.is_cuda and w.dim() == 2 and w.shape[1] % 2048 == 0 and 2048 <= w.shape[1] <= 4096 and w.shape[0] <= 131072
             and w.dtype == out_dtype == torch.bfloat16 and w.is_contiguous() and w.data_ptr() % 16 == 0
             and residual.shape == (1, w.shape[0]) and residual.dtype == torch.float32
             and residual.is_contiguous() and residual.device == w.device
@@ -718,7 +719,7 @@ def attn_rope_rows(qkv: torch.Tensor, q_norm_w: torch.Tensor, k_norm_w: torch.Te
         splits = lib.oa_attn_rows_splits(H, G, D, Dv, 0, 1, tokens, reach) if tokens > 0 else 0
         # six splits of eight waves with a piece of 32 keys each (us, one prompt of 2000 and eight steps of
         # four layers, 16 heads, window 512, 3 / 4 / 5 / 6 splits 2943 / 2931 / 2903 / 2895; nine and the
-        # launch that merges them 3003)
+        # launch that merges them 3003; of 32 and more heads the figures stand in gemv.hip)
         merges = merges and qkv.shape[0] == tokens == 1 and splits > 1 and reach <= 6 * 8 * 32
         splits = 6 if merges else splits
     if not splits:
