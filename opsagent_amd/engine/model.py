@@ -89,8 +89,7 @@ def _init_linear(gen: torch.Generator, out_f: int, in_f: int, dtype) -> torch.Te
 
 def _product_parts(x: torch.Tensor, w: torch.Tensor) -> Union[torch.Tensor, ops.PlaneSum]:
     """x @ w^T for the norm behind it, which adds up the parts of a split product."""
-    parts = ops.shallow_parts(x, w)
-    return ops.linear_parts(x, w) if parts is None else parts
+    return ops.linear_parts(x, w, shallow=True)
 
 
 class Attention(nn.Module):

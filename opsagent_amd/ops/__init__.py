@@ -556,25 +556,17 @@ def _shallow_parts(M: int, N: int, K: int) -> Optional[int]:
     return plan if plan & 255 > 1 else None
 
 
-def shallow_parts(x: torch.Tensor, w: torch.Tensor) -> Optional[PlaneSum]:
-    """linear_parts' parts for more than 128 rows of less than 2 N columns, None where the product is
-    not split for the norm."""
-    M = x.numel() // x.shape[-1]
-    if M > 128 and x.dim() == 2 and w.shape[0] <= 8192 and _skinny_ok(x, w) and _near_rows(x):
-        tile = _shallow_parts(M, *w.shape)
-        if tile:
-            return PlaneSum(_tile(x, w, tile, parts=True))
-    return None
-
-
-def linear_parts(x: torch.Tensor, w: torch.Tensor) -> Union[torch.Tensor, PlaneSum]:
+def linear_parts(x: torch.Tensor, w: torch.Tensor,
+                 shallow: bool = False) -> Union[torch.Tensor, PlaneSum]:
     """x @ w^T for rows x [T, K] that go through fused_add_rms_norm next: bf16 [T, N], or the
     product's float32 column parts, which the norm adds up, where the transfer ring or, of deep
-    products, the tiles split it."""
+    products (shallow: of those of fewer columns too, _shallow_parts), the tiles split it."""
     M = x.numel() // x.shape[-1]
     if M > 1 and x.dim() == 2 and w.shape[0] <= 8192 and _skinny_ok(x, w):
         if M > 128:
-            tile = _tile_choice(M, w.shape[0], w.shape[1], summed=True) if _near_rows(x) else None
+            tile = None
+            if _near_rows(x):
+                tile = shallow and _shallow_parts(M, *w.shape) or _tile_choice(M, *w.shape, summed=True)
             return PlaneSum(_tile(x, w, tile, parts=True)) if tile and tile & 255 > 1 else linear(x, w)
         plan = _ring_form(M, w.shape[0], w.shape[1])
         if plan and plan[1] > 1:

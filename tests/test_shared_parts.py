@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from opsagent_amd import ops
+from opsagent_amd.engine.model import _product_parts
 
 
 def added(planes):
@@ -36,9 +37,19 @@ def test_shallow_products(T, N, K):
     g = torch.Generator(device="cuda").manual_seed(T + K)
     x = torch.randn(T, K, generator=g, device="cuda").bfloat16()
     w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).bfloat16()
-    y = ops.shallow_parts(x, w)
-    assert (y is not None) == (T < 2000)
-    got = added(y.planes) if y is not None else ops.linear_parts(x, w)
+    y = ops.linear_parts(x, w, shallow=True)
+    assert isinstance(y, ops.PlaneSum) == (T < 2000)
+    got = added(y.planes) if isinstance(y, ops.PlaneSum) else y
     want = x.double() @ w.double().T
     # one rounding of sums of K products, whose own float32 error is far below it
     assert torch.allclose(got.double(), want, rtol=2.0 ** -8, atol=2.0 ** -12)
+
+
+def test_asked_once(monkeypatch):
+    """A product for a norm looks its operands over once before it goes to the plain product."""
+    x, w, asked = torch.randn(130, 64), torch.randn(32, 64), []
+    look = ops._skinny_ok
+    monkeypatch.setattr(ops, "_skinny_ok", lambda x, w: asked.append(1) or look(x, w))
+    want = ops.linear(x, w)
+    plain = len(asked)
+    assert torch.equal(_product_parts(x, w), want) and len(asked) == 2 * plain + 1
