@@ -25,8 +25,6 @@ def step_batch(past, rows, device):
 @pytest.mark.parametrize("parts", [0, 1, 5])
 @pytest.mark.parametrize("C,groups", [(120, 5), (512, 1), (2048, 1), (4096, 4), (6144, 3), (8192, 1)])
 def test_norm_and_convolution(C, groups, parts, taps):
-    if not parts and not taps:
-        return                                   # the plain norm
     past, T = [0, 1, 2, 3, 900], 8
     g = torch.Generator(device="cuda").manual_seed(C + taps)
     rand = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
