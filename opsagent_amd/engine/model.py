@@ -89,7 +89,7 @@ def _init_linear(gen: torch.Generator, out_f: int, in_f: int, dtype) -> torch.Te
 
 def _product_parts(x: torch.Tensor, w: torch.Tensor) -> Union[torch.Tensor, ops.PlaneSum]:
     """x @ w^T for the norm behind it, which adds up the parts of a split product."""
-    return ops.linear_parts(x, w, shallow=True)
+    return ops.linear_parts(x, w, shallow=True) if x.shape[0] > 128 else ops.linear_parts(x, w)
 
 
 class Attention(nn.Module):
@@ -287,26 +287,27 @@ class DecoderLayer(nn.Module):
     def forward(self, x, residual, cos, sin, k_cache, v_cache, fb, normed=None, parts=False):
         """normed: the input norm of x, where the first layer's caller has it. parts: the first
         result may be left for the norm that follows to add up (ops.PlaneSum, ops.PairSum)."""
+        one, attn, mlp = get_tp_size() == 1, self.attn, self.mlp
+        plain = _sums_parts(attn)
         if residual is None:
             residual = x
             h = ops.rms_norm(x, self.input_norm_w, self.eps) if normed is None else normed
         else:
             # rows that the fp8 products would quantize next come quantized from the norm
-            low = (_sums_parts(self.attn) and self.attn.fp8 and residual.is_cuda
-                   and ops.fp8_rows_ok(*residual.shape))
+            low = plain and attn.fp8 and residual.is_cuda and ops.fp8_rows_ok(*residual.shape)
             norm = ops.fused_add_rms_norm_fp8 if low else ops.fused_add_rms_norm
             h, residual = norm(x, residual, self.input_norm_w, self.eps)
         # the norm after a sublayer adds up its last product's parts (not what ranks add up)
-        one, attn, mlp = get_tp_size() == 1, self.attn, self.mlp
-        if one and _sums_parts(attn):
+        if one and plain:
             a = attn(h, cos, sin, k_cache, v_cache, fb, True)
         else:
             a = attn(h, cos, sin, k_cache, v_cache, fb)
-        low = (not self.is_moe_layer and _sums_parts(mlp) and mlp.fp8 and residual.is_cuda
+        plain = _sums_parts(mlp)
+        low = (plain and not self.is_moe_layer and mlp.fp8 and residual.is_cuda
                and ops.mlp_fp8_rows_ok(*residual.shape, mlp.i_local, mlp.gate_up_q))
         norm = ops.fused_add_rms_norm_fp8 if low else ops.fused_add_rms_norm
         h, residual = norm(a, residual, self.post_norm_w, self.eps)
-        parts = parts and one and _sums_parts(mlp)
+        parts = parts and one and plain
         if self.is_moe_layer:
             decode = fb.kind == "decode"
             m = mlp(h, decode, True) if parts else mlp(h, decode=decode)

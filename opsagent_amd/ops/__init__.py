@@ -556,22 +556,38 @@ def _shallow_parts(M: int, N: int, K: int) -> Optional[int]:
     return plan if plan & 255 > 1 else None
 
 
+def _rows_product(x: torch.Tensor, w: torch.Tensor, M: int, parts: bool = False,
+                  shallow: bool = False) -> Union[torch.Tensor, PlaneSum, None]:
+    """x @ w^T of M > 1 rows on the ring, in strips or in tiles, None where none of them takes it;
+    parts, shallow: see linear_parts."""
+    if not _skinny_ok(x, w):
+        return None
+    N, K = w.shape
+    if M <= 128:
+        plan = _ring_form(M, N, K)
+        if plan:
+            y = _ring(x, w, plan, parts=parts and plan[1] > 1)
+            return PlaneSum(y) if parts and plan[1] > 1 else y
+        form = _skinny_form(M, N, K, strided=not x.is_contiguous())
+        return _skinny(x, w, form) if form else None
+    if not _near_rows(x):
+        return None
+    if parts:
+        plan = shallow and _shallow_parts(M, N, K) or _tile_choice(M, N, K, summed=True)
+        if plan and plan & 255 > 1:
+            return PlaneSum(_tile(x, w, plan, parts=True))
+    plan = _tile_choice(M, N, K)
+    return None if plan is None else _tile(x, w, plan)
+
+
 def linear_parts(x: torch.Tensor, w: torch.Tensor,
                  shallow: bool = False) -> Union[torch.Tensor, PlaneSum]:
     """x @ w^T for rows x [T, K] that go through fused_add_rms_norm next: bf16 [T, N], or the
     product's float32 column parts, which the norm adds up, where the transfer ring or, of deep
     products (shallow: of those of fewer columns too, _shallow_parts), the tiles split it."""
     M = x.numel() // x.shape[-1]
-    if M > 1 and x.dim() == 2 and w.shape[0] <= 8192 and _skinny_ok(x, w):
-        if M > 128:
-            tile = None
-            if _near_rows(x):
-                tile = shallow and _shallow_parts(M, *w.shape) or _tile_choice(M, *w.shape, summed=True)
-            return PlaneSum(_tile(x, w, tile, parts=True)) if tile and tile & 255 > 1 else linear(x, w)
-        plan = _ring_form(M, w.shape[0], w.shape[1])
-        if plan and plan[1] > 1:
-            return PlaneSum(_ring(x, w, plan, parts=True))
-    return linear(x, w)
+    y = _rows_product(x, w, M, x.dim() == 2 and w.shape[0] <= 8192, shallow) if M > 1 else None
+    return _other_product(x, w, M) if y is None else y
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -582,17 +598,12 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     matrix-core GEMV for what 3 to 8 are, the tile product for more than 128 (_tile_choice);
     everything else goes to hipBLASLt."""
     M = x.numel() // x.shape[-1]
-    if 1 < M <= 128 and _skinny_ok(x, w):
-        plan = _ring_form(M, w.shape[0], w.shape[1])
-        if plan:
-            return _ring(x, w, plan)
-        form = _skinny_form(M, w.shape[0], w.shape[1], strided=not x.is_contiguous())
-        if form:
-            return _skinny(x, w, form)
-    if M > 128 and _skinny_ok(x, w) and _near_rows(x):
-        plan = _tile_choice(M, w.shape[0], w.shape[1])
-        if plan is not None:
-            return _tile(x, w, plan)
+    y = _rows_product(x, w, M) if M > 1 else None
+    return _other_product(x, w, M) if y is None else y
+
+
+def _other_product(x: torch.Tensor, w: torch.Tensor, M: int) -> torch.Tensor:
+    """What _rows_product leaves: the VALU and staged GEMVs or the library."""
     if (
         x.is_cuda
         and x.dtype == torch.bfloat16
