@@ -294,7 +294,9 @@ class DecoderLayer(nn.Module):
             h = ops.rms_norm(x, self.input_norm_w, self.eps) if normed is None else normed
         else:
             # rows that the fp8 products would quantize next come quantized from the norm
-            low = plain and attn.fp8 and residual.is_cuda and ops.fp8_rows_ok(*residual.shape)
+            # (the number of rows first: few ones wait for the host)
+            low = (plain and attn.fp8 and residual.shape[0] > 8 and residual.is_cuda
+                   and ops.fp8_rows_ok(*residual.shape))
             norm = ops.fused_add_rms_norm_fp8 if low else ops.fused_add_rms_norm
             h, residual = norm(x, residual, self.input_norm_w, self.eps)
         # the norm after a sublayer adds up its last product's parts (not what ranks add up)
@@ -303,7 +305,7 @@ class DecoderLayer(nn.Module):
         else:
             a = attn(h, cos, sin, k_cache, v_cache, fb)
         plain = _sums_parts(mlp)
-        low = (plain and not self.is_moe_layer and mlp.fp8 and residual.is_cuda
+        low = (plain and not self.is_moe_layer and mlp.fp8 and residual.shape[0] > 8 and residual.is_cuda
                and ops.mlp_fp8_rows_ok(*residual.shape, mlp.i_local, mlp.gate_up_q))
         norm = ops.fused_add_rms_norm_fp8 if low else ops.fused_add_rms_norm
         h, residual = norm(a, residual, self.post_norm_w, self.eps)

@@ -1052,7 +1052,7 @@ def mlp_fp8(
         M, tiles = x.shape[0], True
     else:
         M = x.numel() // x.shape[-1]
-        tiles = _is_gpu(x) and mlp_fp8_rows_ok(M, x.shape[-1], i_local, gate_up_q)
+        tiles = M > 8 and _is_gpu(x) and mlp_fp8_rows_ok(M, x.shape[-1], i_local, gate_up_q)
     if not tiles:
         return linear_fp8(gateup_silu_fp8(x, gate_up_q, gate_up_s, i_local), down_q, down_s)
     lib, hip = _lib()
