@@ -556,6 +556,18 @@ def _shallow_parts(M: int, N: int, K: int) -> Optional[int]:
     return plan if plan & 255 > 1 else None
 
 
+def shallow_parts(x: torch.Tensor, w: torch.Tensor) -> Optional[PlaneSum]:
+    """linear_parts' parts for more than 128 rows of less than 2 N columns, None where the product is
+    not split for the norm. (A caller who wants the product then, too, asks linear_parts with `shallow`:
+    it looks the operands over once.)"""
+    M = x.numel() // x.shape[-1]
+    if M > 128 and x.dim() == 2 and w.shape[0] <= 8192 and _skinny_ok(x, w) and _near_rows(x):
+        tile = _shallow_parts(M, *w.shape)
+        if tile:
+            return PlaneSum(_tile(x, w, tile, parts=True))
+    return None
+
+
 def _rows_product(x: torch.Tensor, w: torch.Tensor, M: int, parts: bool = False,
                   shallow: bool = False) -> Union[torch.Tensor, PlaneSum, None]:
     """x @ w^T of M > 1 rows on the ring, in strips or in tiles, None where none of them takes it;

@@ -37,12 +37,15 @@ def test_shallow_products(T, N, K):
     g = torch.Generator(device="cuda").manual_seed(T + K)
     x = torch.randn(T, K, generator=g, device="cuda").bfloat16()
     w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).bfloat16()
-    y = ops.linear_parts(x, w, shallow=True)
-    assert isinstance(y, ops.PlaneSum) == (T < 2000)
-    got = added(y.planes) if isinstance(y, ops.PlaneSum) else y
+    y = ops.shallow_parts(x, w)
+    assert (y is not None) == (T < 2000)
+    got = added(y.planes) if y is not None else ops.linear_parts(x, w)
     want = x.double() @ w.double().T
     # one rounding of sums of K products, whose own float32 error is far below it
     assert torch.allclose(got.double(), want, rtol=2.0 ** -8, atol=2.0 ** -12)
+    one = ops.linear_parts(x, w, shallow=True)
+    assert isinstance(one, ops.PlaneSum) == (y is not None)
+    assert torch.equal(one.planes, y.planes) if y is not None else torch.equal(one, got)
 
 
 def test_asked_once(monkeypatch):
