@@ -1146,7 +1146,7 @@ __global__ __launch_bounds__(256, FULL && MAXD <= 8 ? 3 : 1) void attn_bias_mfma
 //
 // ROPE: q is the projection itself, rows of q | k | v: what attn_rope_prepare (blocks.hip; norm and
 // rotation of the heads, the new key and value to their slot) does in a launch of 4 us before this one,
-// every block does for its own heads while its first keys are on their way, each sum of squares
+// every block does for its own heads before it asks for its first keys, each sum of squares
 // over four lanes. The slot of the new key is written by one block of its kv head and read by none: its key
 // and value go from registers into the pieces that hold it. Keys past it count for nothing and repeat it.
 struct RowsRope {
