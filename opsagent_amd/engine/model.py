@@ -288,16 +288,16 @@ class DecoderLayer(nn.Module):
         """normed: the input norm of x, where the first layer's caller has it. parts: the first
         result may be left for the norm that follows to add up (ops.PlaneSum, ops.PairSum)."""
         one, attn, mlp = get_tp_size() == 1, self.attn, self.mlp
-        plain = _sums_parts(attn)
+        plain, quant = _sums_parts(attn), None
         if residual is None:
             residual = x
             h = ops.rms_norm(x, self.input_norm_w, self.eps) if normed is None else normed
         else:
             # rows that the fp8 products would quantize next come quantized from the norm
-            # (the number of rows first: few ones wait for the host)
-            low = (plain and attn.fp8 and residual.shape[0] > 8 and residual.is_cuda
-                   and ops.fp8_rows_ok(*residual.shape))
-            norm = ops.fused_add_rms_norm_fp8 if low else ops.fused_add_rms_norm
+            # (the number of rows first: few ones wait for the host; and asked once where they do not)
+            if plain and attn.fp8 and residual.shape[0] > 8 and residual.is_cuda:
+                quant = ops.fp8_rows_ok(*residual.shape)
+            norm = ops.fused_add_rms_norm_fp8 if quant else ops.fused_add_rms_norm
             h, residual = norm(x, residual, self.input_norm_w, self.eps)
         # the norm after a sublayer adds up its last product's parts (not what ranks add up)
         if one and plain:
@@ -305,9 +305,10 @@ class DecoderLayer(nn.Module):
         else:
             a = attn(h, cos, sin, k_cache, v_cache, fb)
         plain = _sums_parts(mlp)
-        low = (plain and not self.is_moe_layer and mlp.fp8 and residual.shape[0] > 8 and residual.is_cuda
-               and ops.mlp_fp8_rows_ok(*residual.shape, mlp.i_local, mlp.gate_up_q))
-        norm = ops.fused_add_rms_norm_fp8 if low else ops.fused_add_rms_norm
+        quant = (quant is not False and plain and not self.is_moe_layer and mlp.fp8
+                 and residual.shape[0] > 8 and residual.is_cuda
+                 and ops.mlp_fp8_rows_ok(*residual.shape, mlp.i_local, mlp.gate_up_q))
+        norm = ops.fused_add_rms_norm_fp8 if quant else ops.fused_add_rms_norm
         h, residual = norm(a, residual, self.post_norm_w, self.eps)
         parts = parts and one and plain
         if self.is_moe_layer:

@@ -955,13 +955,13 @@ def linear_fp8(
     # are VALU-bound (16 dots/lane) and measured 276 us/call on the 70B
     # jump-ahead catch-up passes vs ~80-150 us through the tile GEMM.
     if (M <= 8 or _fp8_mfma_ok(M, K)) and K % 16 == 0:
-        out = torch.empty(M, N, dtype=x.dtype, device=x.device)
+        out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
         rc = lib.oa_gemv_fp8(
-            hip.current_stream_ptr(), x.reshape(M, K).data_ptr(), w8.data_ptr(),
+            hip.current_stream_ptr(), x.data_ptr(), w8.data_ptr(),
             w_scale.data_ptr(), out.data_ptr(), M, N, K,
         )
         hip.check(rc, "oa_gemv_fp8")
-        return out.reshape(*x.shape[:-1], N)
+        return out
     if K % 128 != 0:
         # the pipelined tile GEMM unrolls K in 128-byte steps; shapes below
         # that (tiny test experts) chunk through the skinny-M gemv instead
@@ -1821,15 +1821,14 @@ def _fp8_mfma_ok(M: int, K: int, gateup: bool = False) -> bool:
     """Mirror of fp8_moe.hip's gemv_fp8_use_mfma for the M 9..16 range
     (the VALU kernels have no 9-11/13-15 instantiations — those batch
     sizes are only reachable through the MFMA stream)."""
-    if os.environ.get("OPSAGENT_FP8_GEMV_MFMA", "") == "0":
-        return False
     # unlike bf16 (whose M>8 alternative is a decent hipBLASLt skinny
     # kernel), fp8's M 9..16 alternative is the 128-row tile GEMM on an
     # underfilled grid — in-engine c16 fp8: MFMA gemv 8.93 t/s vs 7.40
     # through the GEMM. Keep the full M 2..16 range here.
-    if K % 512 != 0 or (K // 512) % (4 if gateup else 8) != 0:
+    # (The sizes first: a look at the environment is a microsecond of the host.)
+    if not 2 <= M <= 16 or M * K > 131072 or K % 512 != 0 or (K // 512) % (4 if gateup else 8) != 0:
         return False
-    return 2 <= M <= 16 and M * K <= 131072
+    return os.environ.get("OPSAGENT_FP8_GEMV_MFMA", "") != "0"
 
 
 def _fp8_gemv_ok(x: torch.Tensor) -> bool:

@@ -1,6 +1,8 @@
 """A norm that adds up the parts of the product before it, against the product by itself and
 the norm: one plane and many, widths of one wave to two rounds of a block."""
 
+import types
+
 import pytest
 import torch
 
@@ -204,3 +206,45 @@ def test_fp8_layers_with_rows_in_8_bits(tokens):
         want = model(fb, cache)
     assert all(isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 for x in seen) and len(seen) == 6
     assert torch.equal(got, want)
+
+
+def test_fp8_sizes_before_the_environment(monkeypatch):
+    """Which form an fp8 product takes is read off its sizes where they say so: the host looks at the
+    environment for the others alone."""
+    looks = []
+
+    class Environment(dict):
+        def get(self, *args):
+            looks.append(args[0])
+            return super().get(*args)
+
+    environment = Environment()
+    monkeypatch.setattr(ops, "os", types.SimpleNamespace(environ=environment))
+    for M, K in [(1, 4096), (17, 4096), (40, 4096), (700, 14336), (14, 14336), (9, 1024), (4, 768)]:
+        assert not ops._fp8_mfma_ok(M, K)
+    assert not looks
+    assert ops._fp8_mfma_ok(9, 4096) and ops._fp8_mfma_ok(16, 8192) and looks
+    environment["OPSAGENT_FP8_GEMV_MFMA"] = "0"
+    assert not ops._fp8_mfma_ok(9, 4096) and not ops._fp8_mfma_ok(17, 4096)
+
+
+@pytest.mark.gpu
+def test_fp8_layers_ask_once(monkeypatch):
+    """A layer whose rows no product quantizes asks that once for its norms, and its products on their own."""
+    from opsagent_amd.engine.config import ModelSpec
+    from opsagent_amd.engine.model import ForwardBatch, LlamaForCausalLM
+
+    layers, tokens = 3, 9
+    spec = ModelSpec(name="fp8", max_seq_len=512, hidden_size=4096, num_heads=4, num_kv_heads=2,
+                     head_dim=128, intermediate_size=512, num_layers=layers, vocab_size=512)
+    model = LlamaForCausalLM(spec, torch.bfloat16, "cuda", seed=1).eval()
+    model.quantize_fp8_()
+    pos = torch.arange(tokens, dtype=torch.int32, device="cuda")
+    fb = ForwardBatch(kind="prefill", input_ids=pos.long() + 3, positions=pos, slot_mapping=pos)
+    cache = [tuple(torch.zeros(16, 32, 2, 128, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+             for _ in range(layers)]
+    asked, ok = [], ops.fp8_rows_ok
+    monkeypatch.setattr(ops, "fp8_rows_ok", lambda rows, K: asked.append(ok(rows, K)) or asked[-1])
+    with torch.inference_mode():
+        model(fb, cache)
+    assert asked == [False] * 2 * layers
