@@ -112,9 +112,9 @@ class MoEMLP(nn.Module):
                                                                     self.i_local * H)):
                     # the shared expert as it is, and nothing that looks at its rows
                     beside = local and not self.shared.fp8 and _sums_parts(self.shared)
-                    front = ops.moe_front(
+                    front = ops.moe_front(                  # up to 16 tokens
                         x, self.router_w, self.top_k, self.i_local * H, self.fp8,
-                        *((self.shared.gate_up_w, self.shared.down_w) if beside else ()))
+                        *((self.shared.gate_up_w, self.shared.down_w) if beside else ())) if T <= 16 else None
                     if front is None:
                         idx, wts, _ = ops.moe_route(x, self.router_w, self.top_k)
                         lists = shared = None
