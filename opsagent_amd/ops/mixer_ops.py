@@ -208,6 +208,9 @@ def group_rms_norm(y: torch.Tensor, w: torch.Tensor, groups: int, eps: float,
     return residual, copy
 
 
+_NO_CONV = (None,) * 7 + (0, 0)
+
+
 def group_norm_step(y: Union[torch.Tensor, "ops.PlaneSum"], w: torch.Tensor, groups: int, eps: float,
                     residual: torch.Tensor, want_copy: bool = True,
                     conv: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
@@ -231,16 +234,17 @@ def group_norm_step(y: Union[torch.Tensor, "ops.PlaneSum"], w: torch.Tensor, gro
             and (planes is None or planes.is_contiguous())
             and (data.data_ptr() | w.data_ptr() | residual.data_ptr()) % 16 == 0):
         lib, hip = _lib()
-        copy, h = (torch.empty(T, C, dtype=w.dtype, device=w.device) if wanted else None
-                   for wanted in (want_copy, join))
-        geometry = (sb.seq_of_t, sb.cu_t, sb.past_t, sb.slots_t) if join else (None,) * 4
+        copy = torch.empty(T, C, dtype=w.dtype, device=w.device) if want_copy else None
+        behind = _NO_CONV
+        if join:
+            h = torch.empty(T, C, dtype=w.dtype, device=w.device)
+            behind = (conv[0].data_ptr(), conv[1].data_ptr(), h.data_ptr(), sb.seq_of_t.data_ptr(),
+                      sb.cu_t.data_ptr(), sb.past_t.data_ptr(), sb.slots_t.data_ptr(), sb.num_seqs,
+                      conv[0].shape[1])
         hip.check(lib.oa_group_norm_step(
             hip.current_stream_ptr(), data.data_ptr(), data.stride(-2),
             0 if planes is None else planes.shape[0], T * C, w.data_ptr(), residual.data_ptr(),
-            copy.data_ptr() if want_copy else None, T, C, groups, eps,
-            *(t.data_ptr() if t is not None else None
-              for t in ((*conv, h) if join else (None,) * 3) + geometry),
-            sb.num_seqs if join else 0, conv[0].shape[1] if join else 0), "oa_group_norm_step")
+            copy.data_ptr() if want_copy else None, T, C, groups, eps, *behind), "oa_group_norm_step")
     else:
         join = False
         if planes is not None:
