@@ -170,6 +170,35 @@ def test_layer_without_host_waits(E, top, T, form):
     assert float((got.double() - want).norm() / want.norm()) < 4e-3
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [17, 70])
+def test_layer_asks_the_front_for_few_tokens(monkeypatch, T):
+    """Routing beside the shared expert takes up to 16 tokens: more go to the routing launches at once."""
+    from opsagent_amd.engine.config import ModelSpec
+    from opsagent_amd.engine.moe import MoEMLP
+    from opsagent_amd.parallel import state
+
+    state.set_tp_state(0, 1, None)
+    H, E, top = 256, 16, 4
+    spec = ModelSpec(name="moe", max_seq_len=64, hidden_size=H, num_heads=2, num_kv_heads=2,
+                     head_dim=128, intermediate_size=256, num_layers=1, vocab_size=64,
+                     moe_num_experts=E, moe_top_k=top, moe_intermediate_size=128,
+                     moe_shared_experts=1, moe_dtype="bf16")
+    moe = MoEMLP(spec, torch.bfloat16, torch.Generator(device="cuda").manual_seed(E)).to("cuda")
+    x = torch.randn(T, H, generator=torch.Generator(device="cuda").manual_seed(T), device="cuda").bfloat16()
+    asked, front = [], ops.moe_front
+    monkeypatch.setattr(ops, "moe_front", lambda x, *a: asked.append(x.shape[0]) or front(x, *a))
+    monkeypatch.setattr(ops, "moe_sorted_wins", lambda *a: True)
+    got = moe(x)
+    assert not asked
+    moe(x[:16])
+    assert asked == [16]
+    score, idx = torch.softmax(x.double() @ moe.router_w.double().T, -1).topk(top, -1)
+    want = _reference(x, moe.w13, moe.w2, idx, score / score.sum(-1, keepdim=True), None, moe.shared(x))
+    # the roundings of test_sorted_experts
+    assert float((got.double() - want).norm() / want.norm()) < 4e-3
+
+
 def test_sorted_experts_refuse():
     """CPU tensors and activations that the kernels do not have stay on the
     general path."""
